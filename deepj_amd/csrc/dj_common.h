@@ -74,6 +74,13 @@ void launch_scatter_add(hipStream_t s, float *target, const float *idx, const fl
                         int cols, int n_idx);
 void launch_fill(hipStream_t s, uint32_t *dst, uint32_t bits, int64_t n);
 void launch_copy(hipStream_t s, const float *src, float *dst, int64_t n);
+// host <-> device traffic through pinned memory (runtime.cpp): up to kUploadPieces uploads in one launch, and a download
+// whose chunks (of chunk_floats, a multiple of 4) announce themselves one by one in flags[]
+constexpr int kUploadPieces = 24;
+struct UploadPiece { const float *src; float *dst; int64_t n; };
+struct UploadPieces { UploadPiece p[kUploadPieces]; };
+void launch_upload_pieces(hipStream_t s, const UploadPieces &pieces, int count);
+void launch_download(hipStream_t s, const float *src, float *dst, int64_t n, int64_t chunk_floats, uint32_t *flags, uint32_t tag);
 // measurement floors: a pure streaming read of n floats (nothing kept), and an empty kernel of `grid` workgroups
 void launch_stream_read(hipStream_t s, const float *src, float *sink, int64_t n);
 void launch_nop(hipStream_t s, int grid);

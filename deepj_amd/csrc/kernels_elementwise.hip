@@ -232,6 +232,44 @@ __global__ void __launch_bounds__(kThreads) k_copy(const float *__restrict__ src
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
 }
 
+// Uploads that were staged in pinned memory since the last launch, one grid row each.  Bound by the link (57 GB/s for
+// 1 MiB and more) and below that by the launch: one launch costs the host 2.4 us, so eight uploads of a flush cost 2.4
+// instead of the 8 x (sync + copy) = 75 us that a copy call per upload took.
+__global__ void __launch_bounds__(kThreads) k_upload_pieces(const UploadPieces pieces) {
+    const UploadPiece p = pieces.p[blockIdx.y];
+    const int64_t n4 = p.n >> 2;
+    const int64_t stride = (int64_t)gridDim.x * kThreads, tid = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    for (int64_t i = tid; i < n4; i += stride) reinterpret_cast<float4 *>(p.dst)[i] = reinterpret_cast<const float4 *>(p.src)[i];
+    if (tid < p.n - (n4 << 2)) p.dst[(n4 << 2) + tid] = p.src[(n4 << 2) + tid];
+}
+
+// dst (pinned host memory) = src, in chunks dealt to the workgroups in order; a chunk's workgroup stores `tag` in
+// flags[chunk] once the chunk is there, so the host takes the chunks out while later ones are still on the link and never
+// waits for a queue to drain (flag and spin 9 us after a launch, hipStreamSynchronize 11, a copy call into pageable
+// memory 23 before it and 250 for 4 MiB, of which 86 are the link's).
+__global__ void __launch_bounds__(kThreads) k_download(const float *__restrict__ src, float *__restrict__ dst, int64_t n,
+                                                       int64_t chunk_floats, uint32_t *__restrict__ flags, uint32_t tag) {
+    const int64_t chunks = (n + chunk_floats - 1) / chunk_floats;
+    for (int64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+        const int64_t from = c * chunk_floats, len = n - from < chunk_floats ? n - from : chunk_floats, n4 = len >> 2;
+        const float4 *s4 = reinterpret_cast<const float4 *>(src + from);
+        float4 *d4 = reinterpret_cast<float4 *>(dst + from);
+        for (int64_t i = threadIdx.x; i < n4; i += 4 * kThreads) {
+            float4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (i + u * kThreads < n4) v[u] = s4[i + u * kThreads];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (i + u * kThreads < n4) d4[i + u * kThreads] = v[u];
+        }
+        if (threadIdx.x < len - (n4 << 2)) dst[from + (n4 << 2) + threadIdx.x] = src[from + (n4 << 2) + threadIdx.x];
+        __threadfence_system();              // every thread's stores are in host memory ...
+        __syncthreads();
+        if (threadIdx.x == 0) __hip_atomic_store(flags + c, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);   // ... before the flag is
+    }
+}
+
 // SiLU.java:20-24 then SwiGLULayer.java:69: (g * sigmoid(g)) * up
 __global__ void __launch_bounds__(kThreads) k_silu_mul(const float *__restrict__ gate, const float *__restrict__ up,
                                                        float *__restrict__ out, int64_t n) {
@@ -426,6 +464,20 @@ void launch_nop(hipStream_t s, int grid) {
 void launch_copy(hipStream_t s, const float *src, float *dst, int64_t n) {
     if (n <= 0) return;
     DJ_LAUNCH(k_copy, grid_for(n), kThreads, s, src, dst, n);
+}
+
+void launch_upload_pieces(hipStream_t s, const UploadPieces &pieces, int count) {
+    int64_t most = 0;
+    for (int i = 0; i < count; i++) most = pieces.p[i].n > most ? pieces.p[i].n : most;
+    int64_t blocks = (most / 4 + kThreads - 1) / kThreads;       // one 128-bit word a thread up to 64 workgroups a piece
+    blocks = blocks < 1 ? 1 : blocks > 64 ? 64 : blocks;
+    launch_kernel(k_upload_pieces, dim3((int)blocks, count), dim3(kThreads), 0, s, pieces);
+}
+
+void launch_download(hipStream_t s, const float *src, float *dst, int64_t n, int64_t chunk_floats, uint32_t *flags, uint32_t tag) {
+    // 64 workgroups keep the link busy; a chunk each up to there, then in turn (so that the first chunks arrive first)
+    const int64_t chunks = (n + chunk_floats - 1) / chunk_floats;
+    launch_kernel(k_download, dim3((int)(chunks < 64 ? chunks : 64)), dim3(kThreads), 0, s, src, dst, n, chunk_floats, flags, tag);
 }
 
 void launch_silu_mul(hipStream_t s, const float *gate, const float *up, float *out, int64_t n) {

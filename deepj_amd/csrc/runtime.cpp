@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <unordered_map>
 #include <vector>
 
@@ -47,6 +48,13 @@ struct Graph {
     std::vector<std::pair<int32_t, int32_t>> prepared, self_prepared;
 };
 
+constexpr int kRingSegments = 8;
+constexpr size_t kRingSegmentBytes = (size_t)1 << 20;
+constexpr size_t kStageBytes = (size_t)4 << 20;
+constexpr int64_t kMaxFlags = 16384;
+constexpr size_t kStageAt = kRingSegments * kRingSegmentBytes, kFlagsAt = kStageAt + kStageBytes;
+constexpr size_t kPinnedBytes = kFlagsAt + (size_t)kMaxFlags * sizeof(uint32_t);
+
 struct Runtime {
     bool ready = false;
     int device = 0;
@@ -57,8 +65,16 @@ struct Runtime {
     size_t cache_limit = (size_t)16 << 30;
     float *workspace = nullptr;
     int64_t workspace_floats = 0;
-    void *staging = nullptr;                       // pinned, for small uploads/downloads
-    size_t staging_bytes = 0;
+    // Host <-> device traffic (section "transfers"): one pinned block holds the upload ring, the download stage and the
+    // flags that a download's chunks set.
+    unsigned char *pinned = nullptr;
+    size_t ring_at = 0;                            // next free byte of the ring
+    int ring_segment = 0;
+    hipEvent_t ring_done[kRingSegments] = {};      // recorded behind the last launch that read the segment
+    bool ring_used[kRingSegments] = {};
+    UploadPieces pieces;                           // staged uploads that no launch has taken over yet
+    int n_pieces = 0;
+    uint32_t tag = 0;                              // of the last download
     bool capturing = false;
     std::unordered_map<int32_t, Graph> graphs;
     int32_t next_graph = 1;
@@ -93,8 +109,13 @@ void ensure_init(int device = 0) {
     if (device < 0 || device >= count) fail("deepj_hip: bad device index " + std::to_string(device));
     DJ_HIP(hipSetDevice(device));
     DJ_HIP(hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking));
-    g.staging_bytes = (size_t)1 << 20;
-    DJ_HIP(hipHostMalloc(&g.staging, g.staging_bytes, hipHostMallocDefault));
+    DJ_HIP(hipHostMalloc((void **)&g.pinned, kPinnedBytes, hipHostMallocDefault));
+    std::memset(g.pinned + kFlagsAt, 0, (size_t)kMaxFlags * sizeof(uint32_t));
+    g.ring_at = 0; g.ring_segment = 0; g.n_pieces = 0; g.tag = 0;
+    for (int i = 0; i < kRingSegments; i++) {
+        DJ_HIP(hipEventCreateWithFlags(&g.ring_done[i], hipEventDisableTiming));
+        g.ring_used[i] = false;
+    }
     DJ_HIP(hipMalloc((void **)&g.attn_counters, kAttnCounterHeads * sizeof(unsigned)));
     DJ_HIP(hipMemset(g.attn_counters, 0, kAttnCounterHeads * sizeof(unsigned)));
     g.static_scratch = nullptr;
@@ -104,6 +125,148 @@ void ensure_init(int device = 0) {
     q8_gemm_f16_configure();
     g.device = device;
     g.ready = true;
+}
+
+// ── transfers ───────────────────────────────────────────────────────────────
+// Uploads are copied into a pinned ring and leave it in one launch per flush (k_upload_pieces); downloads arrive chunk by
+// chunk in a pinned stage, or straight in the caller's memory where that came from deepj_hip_host_alloc.  Nothing here
+// waits for the stream except a full ring and a download for its own chunks.  Measured for one tensor operation on a
+// 64 x 32 matrix (two uploads, a product, a download): 57 us with a synchronisation per upload and copy calls.
+
+// Launches what is staged.  Every path that enqueues work or hands a block to another buffer calls it first.
+void launch_uploads() {
+    if (!g.n_pieces) return;
+    const int n = g.n_pieces;
+    g.n_pieces = 0;
+    launch_upload_pieces(g.stream, g.pieces, n);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) fail(std::string("upload failed: ") + hipGetErrorString(e));
+}
+
+// `bytes` (at most a segment) of the ring; waits for the device only where the ring comes round to a segment in use.
+unsigned char *ring_take(size_t bytes) {
+    bytes = (bytes + 255) & ~(size_t)255;
+    if (g.ring_at + bytes > kRingSegmentBytes) {
+        launch_uploads();
+        DJ_HIP(hipEventRecord(g.ring_done[g.ring_segment], g.stream));
+        g.ring_used[g.ring_segment] = true;
+        g.ring_segment = (g.ring_segment + 1) % kRingSegments;
+        g.ring_at = 0;
+        if (g.ring_used[g.ring_segment]) DJ_HIP(hipEventSynchronize(g.ring_done[g.ring_segment]));
+    }
+    unsigned char *p = g.pinned + g.ring_segment * kRingSegmentBytes + g.ring_at;
+    g.ring_at += bytes;
+    return p;
+}
+
+void stage_upload(float *dst, const float *src, int64_t n) {
+    // pieces of a quarter segment: the first is on the link while the next is copied
+    constexpr int64_t kPiece = (int64_t)(kRingSegmentBytes / 4 / 4);
+    for (int i = 0; i < g.n_pieces; i++)                      // pieces of one launch run side by side: no two into the same words
+        if (g.pieces.p[i].dst < dst + n && dst < g.pieces.p[i].dst + g.pieces.p[i].n) { launch_uploads(); break; }
+    for (int64_t at = 0; at < n; at += kPiece) {
+        const int64_t len = std::min(kPiece, n - at);
+        unsigned char *p = ring_take((size_t)len * 4);
+        std::memcpy(p, src + at, (size_t)len * 4);
+        g.pieces.p[g.n_pieces++] = UploadPiece{reinterpret_cast<const float *>(p), dst + at, len};
+        if (g.n_pieces == kUploadPieces || n > kPiece) launch_uploads();
+    }
+}
+
+// Until flags[0..n) hold `tag`, in order; done(i) runs as each arrives.  A short wait spins (the chunk is a launch away);
+// a longer one lets the runtime block, and a stream that ended without setting its flags is an error, not a hang.
+template <class Done> void wait_flags(volatile uint32_t *flags, int64_t n, uint32_t tag, Done &&done) {
+    for (int64_t i = 0; i < n; i++) {
+        for (int spins = 0; __atomic_load_n(flags + i, __ATOMIC_ACQUIRE) != tag; spins++) {
+            __builtin_ia32_pause();
+            if (spins < 20000) continue;                      // about 0.5 ms
+            DJ_HIP(hipStreamSynchronize(g.stream));
+            if (__atomic_load_n(flags + i, __ATOMIC_ACQUIRE) != tag) fail("download: the stream ended without delivering the buffer");
+        }
+        done(i);
+    }
+}
+
+// Host memory the caller may have results put into without a copy: pinned blocks, handed out again after they come back.
+// Bounded: at most kHostLive bytes are out at a time and kHostCached kept for reuse; beyond that the caller uses ordinary
+// memory.  Locked: finalisers of the arrays over them run on any thread.
+struct HostPool {
+    std::mutex lock;
+    std::map<uintptr_t, size_t> out;               // blocks in use: address -> class
+    std::map<size_t, std::vector<void *>> free;
+    size_t live = 0, cached = 0;
+};
+constexpr size_t kHostLive = (size_t)1 << 30, kHostCached = (size_t)512 << 20;
+HostPool g_host;
+
+size_t size_class(size_t bytes);
+
+void *host_take(size_t bytes) {
+    const size_t cls = size_class(std::max<size_t>(bytes, 4096));
+    std::lock_guard<std::mutex> hold(g_host.lock);
+    if (g_host.live + cls > kHostLive) return nullptr;
+    void *p = nullptr;
+    auto it = g_host.free.find(cls);
+    if (it != g_host.free.end() && !it->second.empty()) {
+        p = it->second.back();
+        it->second.pop_back();
+        g_host.cached -= cls;
+    } else if (hipHostMalloc(&p, cls, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    g_host.out.emplace((uintptr_t)p, cls);
+    g_host.live += cls;
+    return p;
+}
+
+void host_give_back(void *p) {
+    std::lock_guard<std::mutex> hold(g_host.lock);
+    auto it = g_host.out.find((uintptr_t)p);
+    if (it == g_host.out.end()) return;
+    const size_t cls = it->second;
+    g_host.out.erase(it);
+    g_host.live -= cls;
+    if (g_host.cached + cls > kHostCached) { (void)hipHostFree(p); return; }
+    g_host.free[cls].push_back(p);
+    g_host.cached += cls;
+}
+
+void host_trim() {
+    std::lock_guard<std::mutex> hold(g_host.lock);
+    for (auto &kv : g_host.free)
+        for (void *p : kv.second) (void)hipHostFree(p);
+    g_host.free.clear();
+    g_host.cached = 0;
+}
+
+bool host_owned(const void *p, size_t bytes) {
+    std::lock_guard<std::mutex> hold(g_host.lock);
+    auto it = g_host.out.upper_bound((uintptr_t)p);
+    if (it == g_host.out.begin()) return false;
+    --it;
+    return (uintptr_t)p + bytes <= it->first + it->second;
+}
+
+void download(const float *src, float *dst, int64_t n) {
+    uint32_t *flags = reinterpret_cast<uint32_t *>(g.pinned + kFlagsAt);
+    float *stage = reinterpret_cast<float *>(g.pinned + kStageAt);
+    // straight into the caller's block where the device can write there in 128-bit words
+    const bool direct = ((uintptr_t)dst & 15) == 0 && host_owned(dst, (size_t)n * 4);
+    for (int64_t at = 0; at < n;) {
+        // chunks of 8 KiB where few of them would otherwise leave a workgroup the whole transfer, 64 KiB from 512 KiB on
+        const int64_t chunk = (n - at) * 4 <= (512 << 10) ? 2048 : 16384;
+        const int64_t len = std::min(n - at, direct ? kMaxFlags * chunk : (int64_t)(kStageBytes / 4));
+        const int64_t chunks = (len + chunk - 1) / chunk;
+        if (++g.tag == 0) g.tag = 1;
+        launch_download(g.stream, src + at, direct ? dst + at : stage, len, chunk, flags, g.tag);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) fail(std::string("download failed: ") + hipGetErrorString(e));
+        wait_flags(flags, chunks, g.tag, [&](int64_t c) {
+            if (!direct) std::memcpy(dst + at + c * chunk, stage + c * chunk, (size_t)std::min(chunk, len - c * chunk) * 4);
+        });
+        at += len;
+    }
 }
 
 // A prepared copy stops standing for its Q8 buffer as soon as either is released or written.
@@ -834,6 +997,7 @@ void run_stream(const int32_t *cmd, int32_t len) {
     if (len > 0 && !cmd) fail("flushOps: null command stream");
     int64_t ws = 0;
     walk(cmd, len, true, &ws);      // validate everything first
+    launch_uploads();
     ensure_workspace(ws);
     walk(cmd, len, false, nullptr);
     hipError_t e = hipGetLastError();
@@ -937,16 +1101,7 @@ int deepj_hip_upload(int32_t id, const float *src, int64_t n) {
         if (n == 0) return;
         if (!src) fail("uploadBuffer: null source");
         forget_prepared(id);
-        size_t bytes = (size_t)n * 4;
-        // The caller's array is only borrowed: the copy out of it has finished on return.
-        if (bytes <= g.staging_bytes) {
-            DJ_HIP(hipStreamSynchronize(g.stream));      // staging block may still be in flight
-            std::memcpy(g.staging, src, bytes);
-            DJ_HIP(hipMemcpyAsync(it->second.ptr, g.staging, bytes, hipMemcpyHostToDevice, g.stream));
-        } else {
-            DJ_HIP(hipMemcpyAsync(it->second.ptr, src, bytes, hipMemcpyHostToDevice, g.stream));
-            DJ_HIP(hipStreamSynchronize(g.stream));
-        }
+        stage_upload(static_cast<float *>(it->second.ptr), src, n);      // the caller's array is only borrowed
     });
 }
 
@@ -959,8 +1114,9 @@ int deepj_hip_download(int32_t id, float *dst, int64_t n) {
             fail("downloadBuffer: " + std::to_string(n) + " floats exceed buffer id=" + std::to_string(id) + " of " +
                  std::to_string(it->second.floats));
         if (n > 0 && !dst) fail("downloadBuffer: null destination");
-        if (n > 0) DJ_HIP(hipMemcpyAsync(dst, it->second.ptr, (size_t)n * 4, hipMemcpyDeviceToHost, g.stream));
-        DJ_HIP(hipStreamSynchronize(g.stream));
+        launch_uploads();
+        if (n > 0) download(static_cast<const float *>(it->second.ptr), dst, n);
+        else DJ_HIP(hipStreamSynchronize(g.stream));
     });
 }
 
@@ -968,6 +1124,7 @@ int deepj_hip_release(const int32_t *ids, int32_t count) {
     return guarded([&] {
         if (!g.ready) return;
         if (count > 0 && !ids) fail("releaseBuffers: null array");
+        launch_uploads();                                // a released block goes to the next buffer of its size
         for (int i = 0; i < count; i++) {
             auto it = g.live.find(ids[i]);
             if (it == g.live.end()) continue;            // unknown id: silent no-op
@@ -1007,6 +1164,7 @@ int deepj_hip_flush_ops_noalloc(const int32_t *cmd, int32_t len) {
         if (len > 0 && !cmd) fail("flushOps: null command stream");
         int64_t ws = 0;
         walk(cmd, len, true, &ws);
+        launch_uploads();
         ensure_workspace(ws);           // only checks the need against the static size here
         launch_fill(g.stream, reinterpret_cast<uint32_t *>(g.attn_counters), 0u, kAttnCounterHeads);
         walk(cmd, len, false, nullptr);
@@ -1019,14 +1177,18 @@ const char *deepj_hip_last_error(void) { return g_error.c_str(); }
 
 int deepj_hip_synchronize(void) {
     return guarded([&] {
-        if (g.ready) DJ_HIP(hipStreamSynchronize(g.stream));
+        if (!g.ready) return;
+        launch_uploads();
+        DJ_HIP(hipStreamSynchronize(g.stream));
     });
 }
 
 int deepj_hip_trim(void) {
     return guarded([&] {
         if (!g.ready) return;
+        launch_uploads();
         DJ_HIP(hipStreamSynchronize(g.stream));
+        host_trim();
         for (auto &kv : g.cache) {
             for (void *p : kv.second) DJ_HIP(hipFree(p));
             kv.second.clear();
@@ -1054,8 +1216,11 @@ int deepj_hip_shutdown(void) {
         if (g.attn_counters) (void)hipFree(g.attn_counters);
         g.attn_counters = nullptr;
         g.prepared.clear();      // the association names buffer ids; a later session may reuse them for other things
-        if (g.staging) (void)hipHostFree(g.staging);
-        g.staging = nullptr;
+        g.n_pieces = 0;
+        for (auto &ev : g.ring_done) { if (ev) (void)hipEventDestroy(ev); ev = nullptr; }
+        if (g.pinned) (void)hipHostFree(g.pinned);
+        g.pinned = nullptr;
+        host_trim();
         (void)hipStreamDestroy(g.stream);
         g.stream = nullptr;
         g.live_bytes = g.cached_bytes = 0;
@@ -1071,6 +1236,20 @@ int deepj_hip_pool_stats(int64_t out[4]) {
         out[2] = g.cached_bytes;
         out[3] = g.driver_allocs;
     });
+}
+
+void *deepj_hip_host_alloc(int64_t bytes) {
+    void *p = nullptr;
+    guarded([&] {
+        if (bytes <= 0) fail("host_alloc: bad size");
+        ensure_init();
+        p = host_take((size_t)bytes);
+    });
+    return p;
+}
+
+void deepj_hip_host_free(void *p) {
+    if (p) guarded([&] { host_give_back(p); });
 }
 
 void *deepj_hip_stream(void) { return g.ready ? (void *)g.stream : nullptr; }
@@ -1132,6 +1311,7 @@ int deepj_hip_time_ops(const int32_t *cmd, int32_t len, int32_t iters, float *ms
         if (iters <= 0 || !ms_total) fail("time_ops: bad arguments");
         int64_t ws = 0;
         walk(cmd, len, true, &ws);
+        launch_uploads();
         ensure_workspace(ws);
         hipEvent_t e0, e1;
         DJ_HIP(hipEventCreate(&e0));
@@ -1160,6 +1340,7 @@ int deepj_hip_clock_probe(const int32_t *cmd, int32_t len, int32_t iters, int32_
             fail("clock_probe: bad arguments");
         int64_t ws = 0;
         if (len > 0) walk(cmd, len, true, &ws);
+        launch_uploads();
         ensure_workspace(ws);
         hipStream_t side = nullptr;
         unsigned long long *d = nullptr;
@@ -1195,6 +1376,7 @@ int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float 
         if (iters <= 0 || !us_per_op || capacity < 0) fail("profile_ops: bad arguments");
         int64_t ws = 0;
         walk(cmd, len, true, &ws);
+        launch_uploads();
         ensure_workspace(ws);
         std::vector<int32_t> starts;                 // word offset of every op
         for (int32_t pos = 0; pos < len; pos += stride_of(cmd[pos])) starts.push_back(pos);
@@ -1269,6 +1451,7 @@ int deepj_hip_graph_capture(const int32_t *cmd, int32_t len, int32_t *handle) {
         g.track = nullptr;
         std::sort(gr.refs.begin(), gr.refs.end());
         gr.refs.erase(std::unique(gr.refs.begin(), gr.refs.end()), gr.refs.end());
+        launch_uploads();
         ensure_workspace(ws);
         if (ws > 0) gr.workspace = g.workspace;
         DJ_HIP(hipStreamSynchronize(g.stream));
@@ -1320,6 +1503,7 @@ int deepj_hip_graph_launch(int32_t handle, int32_t times) {
                 fail("graph_launch: Q8 weights id=" + std::to_string(pr.first) + " were written after graph " + std::to_string(handle) +
                      " was captured with their prepared copy id=" + std::to_string(pr.second) + "; capture the stream again");
         }
+        launch_uploads();
         // Bounded run-ahead: at most kRing windows of kWindow replays are queued behind the one the
         // device is executing, so a long run never piles tens of thousands of dispatches (and their
         // kernel-argument blocks) into the queue; the device is never left idle by this.

@@ -81,6 +81,11 @@ int deepj_hip_shutdown(void);              /* frees every buffer and the cache *
 int deepj_hip_trim(void);                  /* returns cached (released) memory to the driver */
 /* out[0]=live buffers, out[1]=live bytes, out[2]=cached bytes, out[3]=driver allocations so far */
 int deepj_hip_pool_stats(int64_t out[4]);
+/* Host memory that deepj_hip_download fills without a copy in between (pinned; blocks given back are handed out again).
+ * NULL when the bound on such memory (1 GiB at a time) is reached: ordinary memory works everywhere.  These two may be
+ * called from any thread. */
+void *deepj_hip_host_alloc(int64_t bytes);
+void deepj_hip_host_free(void *block);
 /* The HIP stream all work is queued on, as a hipStream_t, for callers that time with HIP events. */
 void *deepj_hip_stream(void);
 
