@@ -7,6 +7,7 @@ point raises; there is no CPU fallback.
 """
 from __future__ import annotations
 
+import array
 import ctypes as C
 import os
 
@@ -28,11 +29,16 @@ _load_error: Exception | None = None
 
 def _bind(lib: C.CDLL) -> None:
     lib.deepj_hip_init.argtypes = [C.c_int32]
-    lib.deepj_hip_alloc_buffers.argtypes = [_i32p, _i32p, C.c_int32]
+    # addresses travel as plain integers: a typed pointer costs more to make than some of these calls take
+    lib.deepj_hip_alloc_buffers.argtypes = [C.c_void_p, C.c_void_p, C.c_int32]
     lib.deepj_hip_upload.argtypes = [C.c_int32, C.c_void_p, C.c_int64]
     lib.deepj_hip_download.argtypes = [C.c_int32, C.c_void_p, C.c_int64]
-    lib.deepj_hip_release.argtypes = [_i32p, C.c_int32]
-    lib.deepj_hip_flush_ops.argtypes = [_i32p, C.c_int32]
+    lib.deepj_hip_release.argtypes = [C.c_void_p, C.c_int32]
+    lib.deepj_hip_flush_ops.argtypes = [C.c_void_p, C.c_int32]
+    lib.deepj_hip_host_alloc.argtypes = [C.c_int64]
+    lib.deepj_hip_host_alloc.restype = C.c_void_p
+    lib.deepj_hip_host_free.argtypes = [C.c_void_p]
+    lib.deepj_hip_host_free.restype = None
     lib.deepj_hip_flush_ops_noalloc.argtypes = [_i32p, C.c_int32]
     lib.deepj_hip_last_error.restype = C.c_char_p
     lib.deepj_hip_pool_stats.argtypes = [C.POINTER(C.c_int64)]
@@ -95,6 +101,39 @@ def _ids(a) -> np.ndarray:
     return np.ascontiguousarray(np.asarray(a, dtype=np.int32))
 
 
+def _words(a):
+    """(object that owns them, address) of int32 words given as an array.array, a numpy array or any sequence."""
+    if type(a) is not array.array:
+        if isinstance(a, np.ndarray):
+            a = np.ascontiguousarray(a, dtype=np.int32)
+            return a, a.ctypes.data
+        a = array.array("i", a)
+    return a, a.buffer_info()[0]
+
+
+class _HostBlock:
+    """A pinned block of the library under a numpy array; goes back when the array (and every view of it) is gone."""
+    __slots__ = ("address", "__array_interface__", "_free")
+
+    def __init__(self, address: int, count: int, free):
+        self.address, self._free = address, free
+        self.__array_interface__ = {"shape": (count,), "typestr": "<f4", "data": (address, False), "version": 3}
+
+    def __del__(self):
+        self._free(self.address)
+
+
+def host_array(count: int) -> np.ndarray:
+    """Uninitialised fp32 array for a download.  From 64 KiB on it is pinned memory that the device writes straight into:
+    no stage, no copy out of it and no page faults of a fresh allocation (80 MB: 1.5 ms instead of 6.5)."""
+    if count * 4 >= 65536:
+        lib = library()
+        address = lib.deepj_hip_host_alloc(count * 4)
+        if address:
+            return np.asarray(_HostBlock(address, count, lib.deepj_hip_host_free))
+    return np.empty(count, dtype=np.float32)
+
+
 class HipNative:
     """Static facade, one method per native entry point (names as in MetalNative)."""
 
@@ -108,29 +147,30 @@ class HipNative:
 
     @staticmethod
     def nativeAllocBuffers(ids, sizes, count: int) -> None:
-        ids, sizes = _ids(ids), _ids(sizes)
-        _check(library().deepj_hip_alloc_buffers(ids.ctypes.data_as(_i32p), sizes.ctypes.data_as(_i32p), count))
+        ids, p = _words(ids)
+        sizes, q = _words(sizes)
+        _check((_lib or library()).deepj_hip_alloc_buffers(p, q, count))
 
     @staticmethod
     def nativeUploadBuffer(buf_id: int, data: np.ndarray) -> None:
         data = np.ascontiguousarray(data)
-        assert data.dtype.itemsize == 4, "buffers hold 32-bit words"
-        _check(library().deepj_hip_upload(buf_id, data.ctypes.data, data.size))
+        assert data.itemsize == 4, "buffers hold 32-bit words"
+        _check((_lib or library()).deepj_hip_upload(buf_id, data.ctypes.data, data.size))
 
     @staticmethod
     def nativeDownloadBuffer(buf_id: int, out: np.ndarray) -> None:
-        assert out.flags["C_CONTIGUOUS"] and out.dtype.itemsize == 4
-        _check(library().deepj_hip_download(buf_id, out.ctypes.data, out.size))
+        assert out.flags.c_contiguous and out.itemsize == 4
+        _check((_lib or library()).deepj_hip_download(buf_id, out.ctypes.data, out.size))
 
     @staticmethod
     def nativeReleaseBuffers(ids, count: int) -> None:
-        ids = _ids(ids)
-        _check(library().deepj_hip_release(ids.ctypes.data_as(_i32p), count))
+        ids, p = _words(ids)
+        _check((_lib or library()).deepj_hip_release(p, count))
 
     @staticmethod
     def nativeFlushOps(cmd_stream, length: int) -> None:
-        cmd = _ids(cmd_stream)
-        _check(library().deepj_hip_flush_ops(cmd.ctypes.data_as(_i32p), length))
+        cmd, p = _words(cmd_stream)
+        _check((_lib or library()).deepj_hip_flush_ops(p, length))
 
     @staticmethod
     def flushOpsNoAlloc(cmd_stream, length: int) -> None:

@@ -10,6 +10,7 @@ protocol the Java class speaks (same encodings, same call order).
 """
 from __future__ import annotations
 
+import array
 import struct
 import weakref
 from typing import Protocol
@@ -32,21 +33,33 @@ class GpuRuntime(Protocol):
 class GpuBuffer:
     """GpuBuffer.java:9-32."""
 
-    __slots__ = ("id", "rows", "cols", "needsUpload", "cpuStale", "allocatedOnGpu")
+    __slots__ = ("id", "rows", "cols", "needsUpload", "cpuStale", "allocatedOnGpu", "graph")
 
-    def __init__(self, id: int, rows: int, cols: int, needs_upload: bool):
+    def __init__(self, id: int, rows: int, cols: int, needs_upload: bool, graph=None):
         self.id, self.rows, self.cols = id, rows, cols
         self.needsUpload = needs_upload
         self.cpuStale = False
         self.allocatedOnGpu = True
+        self.graph = graph          # the graph that tracks it: told when a tensor lets go of this buffer
 
     def floatCount(self) -> int:
         return self.rows * self.cols
 
 
+_pack_float, _unpack_int = struct.Struct("<f").pack, struct.Struct("<i").unpack
+
+
 def float_bits(value: float) -> int:
     """Float.floatToRawIntBits as a signed int32."""
-    return struct.unpack("<i", struct.pack("<f", np.float32(value)))[0]
+    try:
+        return _unpack_int(_pack_float(value))[0]
+    except OverflowError:                       # beyond fp32: infinity, as a cast gives
+        return _unpack_int(_pack_float(np.float32(value)))[0]
+
+
+class _TensorRef(weakref.ref):
+    """A weak reference that remembers which buffer its tensor stood for."""
+    __slots__ = ("id",)
 
 
 # stride and buffer-id slots per opcode (ComputeGraph.java:89-147)
@@ -72,69 +85,78 @@ _OP_META[op.OP_ADAMW_UPDATE] = (13, (1, 2, 3, 4))
 
 
 class ComputeGraph:
+    """Recording one op costs a few microseconds of host time, as much as its launch, so nothing here walks all tracked
+    tensors: buffers that may have lost their tensor announce themselves (a dead weak reference, a replaced tag) and only
+    those are looked at when a flush releases orphans."""
+
     def __init__(self, runtime: GpuRuntime):
         if runtime is None:
             raise TypeError("runtime")          # Objects.requireNonNull
         self.runtime = runtime
         self._next_buf_id = 0
-        self._cmd = np.zeros(4096, dtype=np.int32)
-        self._pos = 0
+        self._cmd = array.array("i")
         self._op_count = 0
-        self._pending_allocs: list[tuple[int, int]] = []
+        self._pending_allocs: list[GpuBuffer] = []
         self._pending_uploads: list[tuple[int, np.ndarray]] = []
-        self._buf_to_tensor: dict[int, weakref.ReferenceType] = {}
+        self._buf_to_tensor: dict[int, _TensorRef] = {}
+        self._maybe_orphans: list[int] = []
+        self._host_array = getattr(runtime, "hostArray", None) or (lambda n: np.zeros(n, dtype=np.float32))
 
     # ── buffer management (ComputeGraph.java:172-234) ───────────────────────
     def ensureGpuBuffer(self, t) -> GpuBuffer:
-        existing = t.getGpuTag()
+        existing = t._gpu_tag
         if isinstance(existing, GpuBuffer):
-            self._track(existing.id, t)
+            ref = self._buf_to_tensor.get(existing.id)
+            if ref is None or ref() is not t:
+                self._track(existing, t)
             if existing.needsUpload:
                 self._pending_uploads.append((existing.id, pack_f32(t)))
                 existing.needsUpload = False
                 existing.cpuStale = False
             return existing
-        buf_id = self._next_buf_id
+        buf = GpuBuffer(self._next_buf_id, t.rows, t.cols, True, self)
         self._next_buf_id += 1
-        buf = GpuBuffer(buf_id, t.rows, t.cols, True)
         buf.allocatedOnGpu = False
-        self._pending_allocs.append((buf_id, buf.floatCount()))
-        self._pending_uploads.append((buf_id, pack_f32(t)))
+        self._pending_allocs.append(buf)
+        self._pending_uploads.append((buf.id, pack_f32(t)))
         t.setGpuTag(buf)
-        self._track(buf_id, t)
+        self._track(buf, t)
         return buf
 
-    def _track(self, buf_id: int, t) -> None:
-        self._buf_to_tensor[buf_id] = weakref.ref(t)
+    def _track(self, buf: GpuBuffer, t) -> None:
+        ref = _TensorRef(t, self._tensor_died)
+        ref.id = buf.id
+        self._buf_to_tensor[buf.id] = ref
+        buf.graph = self
+
+    def _tensor_died(self, ref) -> None:
+        self._maybe_orphans.append(ref.id)
+
+    def tensorLetGo(self, buf: GpuBuffer) -> None:
+        """Tensor.setGpuTag: `buf` is no longer the tag of a tensor that had it."""
+        self._maybe_orphans.append(buf.id)
 
     def newOutputBuffer(self, rows: int, cols: int) -> GpuBuffer:
-        buf_id = self._next_buf_id
+        buf = GpuBuffer(self._next_buf_id, rows, cols, False, self)
         self._next_buf_id += 1
-        buf = GpuBuffer(buf_id, rows, cols, False)
         buf.cpuStale = True
         buf.allocatedOnGpu = False
-        self._pending_allocs.append((buf_id, buf.floatCount()))
+        self._pending_allocs.append(buf)
         return buf
 
     def createOutputTensor(self, buf: GpuBuffer):
-        from .tensor import Tensor
-        t = Tensor(buf.rows, buf.cols)
-        self.bindTensorToBuffer(t, buf)
+        t = _tensor_class()(buf.rows, buf.cols)
+        t._gpu_tag = buf
+        self._track(buf, t)
         return t
 
     def bindTensorToBuffer(self, t, buf: GpuBuffer) -> None:
         t.setGpuTag(buf)
-        self._track(buf.id, t)
+        self._track(buf, t)
 
     # ── op recording (ComputeGraph.java:238-518) ────────────────────────────
     def _emit(self, *words: int) -> None:
-        n = len(words)
-        if self._pos + n > self._cmd.size:
-            grown = np.zeros(max(self._cmd.size * 2, self._pos + n), dtype=np.int32)
-            grown[: self._pos] = self._cmd[: self._pos]
-            self._cmd = grown
-        self._cmd[self._pos: self._pos + n] = words
-        self._pos += n
+        self._cmd.extend(words)
         self._op_count += 1
 
     def recordBinary(self, opcode, a, b, out): self._emit(opcode, a.id, b.id, out.id, out.floatCount())
@@ -203,16 +225,13 @@ class ComputeGraph:
         self._release_orphans()
 
     def _allocate_pending(self) -> None:
-        if not self._pending_allocs:
+        pending = self._pending_allocs
+        if not pending:
             return
-        ids = np.array([a[0] for a in self._pending_allocs], dtype=np.int32)
-        sizes = np.array([a[1] for a in self._pending_allocs], dtype=np.int32)
-        self.runtime.allocBuffers(ids, sizes, len(ids))
-        for ref in self._buf_to_tensor.values():
-            t = ref()
-            if t is not None and isinstance(t.getGpuTag(), GpuBuffer):
-                t.getGpuTag().allocatedOnGpu = True
-        self._pending_allocs.clear()
+        self.runtime.allocBuffers(array.array("i", [b.id for b in pending]), array.array("i", [b.rows * b.cols for b in pending]), len(pending))
+        for b in pending:
+            b.allocatedOnGpu = True
+        self._pending_allocs = []
 
     def _upload_pending(self) -> None:
         for buf_id, data in self._pending_uploads:
@@ -220,51 +239,72 @@ class ComputeGraph:
         self._pending_uploads.clear()
 
     def _execute_pending(self) -> None:
-        if self._op_count > 0:
-            self.runtime.flushOps(self._cmd, self._pos)
-        self._pos = 0
-        self._op_count = 0
+        cmd, count = self._cmd, self._op_count
+        self._cmd, self._op_count = array.array("i"), 0
+        if count > 0:
+            self.runtime.flushOps(cmd, len(cmd))
 
     def _release_orphans(self) -> None:
-        if not self._buf_to_tensor:
+        if not self._maybe_orphans:
             return
+        candidates, self._maybe_orphans = self._maybe_orphans, []
         orphans = []
-        for buf_id, ref in self._buf_to_tensor.items():
+        for buf_id in dict.fromkeys(candidates):
+            ref = self._buf_to_tensor.get(buf_id)
+            if ref is None:
+                continue
             t = ref()
-            orphaned = t is None or not isinstance(t.getGpuTag(), GpuBuffer) or t.getGpuTag().id != buf_id
-            if orphaned and not self._referenced_by_pending_ops(buf_id):
-                orphans.append(buf_id)
+            if t is not None and isinstance(t._gpu_tag, GpuBuffer) and t._gpu_tag.id == buf_id:
+                continue
+            if self._op_count > 0 and self._referenced_by_pending_ops(buf_id):
+                self._maybe_orphans.append(buf_id)
+                continue
+            orphans.append(buf_id)
+            del self._buf_to_tensor[buf_id]
         if not orphans:
             return
-        for buf_id in orphans:
-            self._pending_allocs = [a for a in self._pending_allocs if a[0] != buf_id]
-            self._pending_uploads = [u for u in self._pending_uploads if u[0] != buf_id]
-            del self._buf_to_tensor[buf_id]
-        ids = np.array(orphans, dtype=np.int32)
-        self.runtime.releaseBuffers(ids, len(ids))
+        if self._pending_allocs or self._pending_uploads:
+            gone = set(orphans)
+            self._pending_allocs = [b for b in self._pending_allocs if b.id not in gone]
+            self._pending_uploads = [u for u in self._pending_uploads if u[0] not in gone]
+        self.runtime.releaseBuffers(array.array("i", orphans), len(orphans))
 
     def _referenced_by_pending_ops(self, buf_id: int) -> bool:
         pos = 0
-        while pos < self._pos:
-            meta = _OP_META.get(int(self._cmd[pos]))
+        while pos < len(self._cmd):
+            meta = _OP_META.get(self._cmd[pos])
             if meta is None:
                 return True                     # unknown op: be conservative
             stride, slots = meta
-            if any(int(self._cmd[pos + s]) == buf_id for s in slots):
+            if any(self._cmd[pos + s] == buf_id for s in slots):
                 return True
             pos += stride
         return False
 
     # ── materialize / release (ComputeGraph.java:676-740) ───────────────────
     def materialize(self, t) -> None:
-        buf = t.getGpuTag()
+        buf = t._gpu_tag
         if not isinstance(buf, GpuBuffer) or not buf.cpuStale:
             return
         self.flush()
-        flat = np.zeros(buf.floatCount(), dtype=np.float32)
-        self.runtime.downloadBuffer(buf.id, flat)
-        unpack_f32_into(flat, t)
+        self._download(buf, t)
         buf.cpuStale = False
+
+    def _download(self, buf: GpuBuffer, t) -> None:
+        """The buffer's values in the tensor's host array: written there directly, and into an array of the runtime's
+        own kind where the tensor has none yet."""
+        data = t._data
+        if data is None or not data.flags.c_contiguous or data.dtype != np.float32:
+            flat = self._host_array(buf.rows * buf.cols)
+            self.runtime.downloadBuffer(buf.id, flat)
+            if data is None and flat.size == t.rows * t.cols:
+                t._data = flat.reshape(t.rows, t.cols)
+            else:
+                unpack_f32_into(flat, t)
+            return
+        if data.size != buf.rows * buf.cols:
+            raise ValueError(f"Size mismatch: src has {buf.rows * buf.cols} floats but tensor is {t.rows}x{t.cols}")
+        self.runtime.downloadBuffer(buf.id, data.reshape(-1))
 
     def releaseAll(self) -> None:
         self.flush()
@@ -272,12 +312,10 @@ class ComputeGraph:
             t = ref()
             if t is None:
                 continue
-            gb = t.getGpuTag()
+            gb = t._gpu_tag
             if not isinstance(gb, GpuBuffer) or not gb.cpuStale:
                 continue
-            flat = np.zeros(gb.floatCount(), dtype=np.float32)
-            self.runtime.downloadBuffer(gb.id, flat)
-            unpack_f32_into(flat, t)
+            self._download(gb, t)
             gb.cpuStale = False
             gb.needsUpload = False
         for ref in self._buf_to_tensor.values():
@@ -285,23 +323,34 @@ class ComputeGraph:
             if t is not None:
                 t.setGpuTag(None)
         if self._buf_to_tensor:
-            ids = np.array(list(self._buf_to_tensor.keys()), dtype=np.int32)
+            ids = array.array("i", self._buf_to_tensor.keys())
             self.runtime.releaseBuffers(ids, len(ids))
         self._buf_to_tensor.clear()
-        self._pending_allocs.clear()
+        self._maybe_orphans.clear()
+        self._pending_allocs = []
         self._pending_uploads.clear()
-        self._pos = 0
-        self._op_count = 0
+        self._cmd, self._op_count = array.array("i"), 0
         self._next_buf_id = 0
+
+
+_tensor_type = None
+
+
+def _tensor_class():
+    global _tensor_type
+    if _tensor_type is None:
+        from .tensor import Tensor
+        _tensor_type = Tensor
+    return _tensor_type
 
 
 # TensorAdapters.java:9-47
 def pack_f32(t) -> np.ndarray:
-    return np.array(t.data, dtype=np.float32, copy=True).reshape(-1)
+    return t.data.astype(np.float32, order="C").reshape(-1)          # a copy: the tensor may change before the flush
 
 
 def unpack_f32_into(src: np.ndarray, dst) -> None:
-    if src.size != dst.data.size:
+    if src.size != dst.rows * dst.cols:
         raise ValueError(f"Size mismatch: src has {src.size} floats but tensor is {dst.rows}x{dst.cols}")
     dst.data.reshape(-1)[:] = src
 

@@ -8,10 +8,12 @@ emits exactly the same words.
 """
 from __future__ import annotations
 
+import math
+
 import numpy as np
 
 from . import opcodes as op
-from ._native import HipNative
+from ._native import HipNative, host_array
 
 FUSED_ID_BASE = 1 << 28
 
@@ -43,9 +45,10 @@ class DeviceBuffers:
         HipNative.nativeUploadBuffer(buf_id, a.reshape(-1))
 
     def download(self, buf_id: int, shape, dtype=np.float32) -> np.ndarray:
-        out = np.empty(int(np.prod(shape)), dtype=dtype)
+        count = math.prod(shape) if isinstance(shape, (tuple, list)) else int(np.prod(shape))
+        out = host_array(count)
         HipNative.nativeDownloadBuffer(buf_id, out)
-        return out.reshape(shape)
+        return out.view(dtype).reshape(shape)
 
     def size(self, buf_id: int) -> int:
         return self._sizes[buf_id]
@@ -159,8 +162,7 @@ class Stream:
         return np.asarray(self.words, dtype=np.int32)
 
     def run(self) -> None:
-        a = self.array()
-        HipNative.nativeFlushOps(a, a.size)
+        HipNative.nativeFlushOps(self.words, len(self.words))
 
     def profile(self, iters: int) -> np.ndarray:
         """Mean kernel duration of every op in microseconds (events on each op's own dispatch)."""

@@ -13,7 +13,7 @@ from __future__ import annotations
 import numpy as np
 
 from . import opcodes as op
-from ._native import HipNative
+from ._native import HipNative, host_array
 from .compute_graph import ComputeGraph, GpuBuffer
 from .tensor import Tensor
 
@@ -23,7 +23,8 @@ class HipGpuRuntime:
     def uploadBuffer(self, buf_id, data): HipNative.nativeUploadBuffer(buf_id, data)
     def downloadBuffer(self, buf_id, out): HipNative.nativeDownloadBuffer(buf_id, out)
     def releaseBuffers(self, ids, count): HipNative.nativeReleaseBuffers(ids, count)
-    def flushOps(self, cmd_stream, length): HipNative.nativeFlushOps(cmd_stream[:length], length)
+    def flushOps(self, cmd_stream, length): HipNative.nativeFlushOps(cmd_stream if len(cmd_stream) == length else cmd_stream[:length], length)
+    def hostArray(self, n): return host_array(n)
 
 
 def _require_row_vector(v, target):

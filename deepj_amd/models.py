@@ -15,7 +15,7 @@ from dataclasses import dataclass
 
 import numpy as np
 
-from ._native import library
+from ._native import host_array, library
 
 _i32p = C.POINTER(C.c_int32)
 _f32p = C.POINTER(C.c_float)
@@ -224,7 +224,7 @@ class _DecoderOnlyModel:
         """Logits [len(ids) x vocab] of a fresh sequence (DecoderOnlyModel.forward)."""
         ids = np.ascontiguousarray(np.asarray(ids, dtype=np.int32))
         self.reset()
-        out = np.empty((len(ids), self.cfg.vocabSize), dtype=np.float32)
+        out = host_array(len(ids) * self.cfg.vocabSize).reshape(len(ids), self.cfg.vocabSize)
         self._check(_lib().deepj_runner_prefill(self._h, ids.ctypes.data_as(_i32p), len(ids), out.ctypes.data, 0))
         return out
 
@@ -245,7 +245,7 @@ class _DecoderOnlyModel:
         self._check(_lib().deepj_runner_step(self._h, int(token)))
 
     def lastLogits(self) -> np.ndarray:
-        out = np.empty(self.cfg.vocabSize, dtype=np.float32)
+        out = host_array(self.cfg.vocabSize)
         self._check(_lib().deepj_runner_last_logits(self._h, out.ctypes.data))
         return out
 

@@ -16,15 +16,28 @@ class Tensor:
     _backend = None
 
     def __init__(self, rows: int, cols: int | None = None):
+        self._gpu_tag = None
+        self._data = None                                 # the host copy: made when it is first asked for
         if isinstance(rows, Tensor):                      # copy constructor (Tensor.java:50-59)
             src = rows
             src.materialize()
             self.rows, self.cols = src.rows, src.cols
-            self.data = src.data.copy()
+            self._data = src.data.copy()
         else:
             self.rows, self.cols = int(rows), int(cols)
-            self.data = np.zeros((self.rows, self.cols), dtype=np.float32)
-        self._gpu_tag = None
+            if self.rows < 0 or self.cols < 0:
+                raise ValueError("negative dimensions are not allowed")
+
+    @property
+    def data(self) -> np.ndarray:
+        """The host copy as it is (zeros before anything was put there); numpy() brings it up to date first."""
+        if self._data is None:
+            self._data = np.zeros((self.rows, self.cols), dtype=np.float32)
+        return self._data
+
+    @data.setter
+    def data(self, value) -> None:
+        self._data = value
 
     # ── backend switch (Tensor.java:24-41) ──────────────────────────────────
     @staticmethod
@@ -40,7 +53,11 @@ class Tensor:
         return Tensor._backend
 
     def getGpuTag(self): return self._gpu_tag
-    def setGpuTag(self, tag): self._gpu_tag = tag
+
+    def setGpuTag(self, tag):
+        old, self._gpu_tag = self._gpu_tag, tag
+        if old is not None and old is not tag and isinstance(old, GpuBuffer) and old.graph is not None:
+            old.graph.tensorLetGo(old)
 
     def materialize(self) -> "Tensor":
         if self._gpu_tag is not None:
@@ -55,11 +72,11 @@ class Tensor:
     # ── factories ───────────────────────────────────────────────────────────
     @staticmethod
     def from2D(values) -> "Tensor":
-        a = np.asarray(values, dtype=np.float32)
+        a = np.array(values, dtype=np.float32, order="C")
         if a.ndim != 2:
             raise ValueError("All rows must have the same length")
         t = Tensor(a.shape[0], a.shape[1])
-        t.data[:] = a
+        t._data = a
         return t
 
     @staticmethod
@@ -194,7 +211,11 @@ class Tensor:
     def sliceRows(t, row_indices, cols):
         t.materialize()
         out = Tensor(len(row_indices), cols)
-        out.data[:] = t.data[np.asarray(row_indices, dtype=np.int64), :cols]
+        rows = t.data[np.asarray(row_indices, dtype=np.int64)]         # a copy
+        if rows.shape == (out.rows, out.cols):
+            out._data = rows
+        else:
+            out.data[:] = rows[:, :cols]
         return out
 
     def numpy(self) -> np.ndarray:
