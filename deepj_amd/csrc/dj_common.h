@@ -199,6 +199,9 @@ void launch_attn_decode_records(hipStream_t s, const float *qkv, float *k_cache,
                                 int max_seq);
 void launch_decode_next(hipStream_t s, const float *logits, int32_t *state, int32_t *tokens, int capacity,
                         const float *table, float *x, int vocab, int d, int n_positions);
+constexpr int kSampleTopK = 512;         // the most candidates the device samples among
+void launch_decode_sample(hipStream_t s, const float *logits, int32_t *state, int32_t *tokens, int capacity,
+                          const float *table, float *x, int vocab, int d, int n_positions, uint32_t *params);
 int64_t attention_scratch_floats(int S, int H, int hd, int max_seq);
 
 }  // namespace dj

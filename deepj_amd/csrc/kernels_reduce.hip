@@ -394,6 +394,174 @@ __global__ void __launch_bounds__(1024) k_decode_next(const float *__restrict__ 
     for (int c = threadIdx.x; c < d; c += 1024) x[c] = ok ? src[c] : __builtin_nanf("");
 }
 
+// ── sampled decode step ─────────────────────────────────────────────────────
+// End of a decode step that samples (temperature, 1 < topK <= kSampleTopK): what TextGenerator.java:104-151 does with the
+// logits, on the device, so that a sampled run replays graphs like a greedy one.  In order: the topK largest logits, ties
+// by lowest index (stable descending sort); soft-max of value / temperature with a float64 exp and fp32 sums in that
+// order; one draw of java.util.Random; the first candidate whose cumulative sum reaches it; then record, advance and
+// gather as k_decode_next does.
+// Selection: the topK-th largest of the 1024 threads' own maxima bounds the topK-th largest logit from below, so one more
+// pass collects a few more than topK candidates, which are sorted in LDS.  Logits so full of ties that more than kPool
+// candidates pass are cut exactly by a search over the key's bits first.  Bound by the latency of two passes of one
+// workgroup over the logits; the host's sort it replaces took 3.3 ms for 50257 logits.
+constexpr int kPool = 2048;
+
+// Float.compare's order as unsigned integers: -0 below +0, NaN above everything.
+__device__ __forceinline__ uint32_t order_key(float v) {
+    uint32_t b = __builtin_bit_cast(uint32_t, v);
+    if (v != v) b = 0x7fc00000u;
+    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+}
+
+// Descending bitonic sort of n (a power of two, at most 2 * 1024) values in LDS by 1024 threads.
+template <class T> __device__ __forceinline__ void sort_descending(T *v, int n) {
+    for (int size = 2; size <= n; size <<= 1)
+        for (int step = size >> 1; step > 0; step >>= 1) {
+            __syncthreads();
+            const int t = threadIdx.x;
+            if (t < n / 2) {
+                const int i = 2 * t - (t & (step - 1)), j = i + step;
+                const T a = v[i], b = v[j];
+                const bool down = (i & size) == 0;
+                if (down ? a < b : a > b) { v[i] = b; v[j] = a; }
+            }
+        }
+    __syncthreads();
+}
+
+template <class F> __device__ __forceinline__ void each_logit(const float *logits, int vocab, F &&f) {
+    const int v4 = vocab >> 2;
+    const float4 *l4 = reinterpret_cast<const float4 *>(logits);
+    for (int base = 0; base < v4; base += 1024 * 8) {
+        float4 t[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int i = base + u * 1024 + threadIdx.x;
+            if (i < v4) t[u] = l4[i];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int i = base + u * 1024 + threadIdx.x;
+            if (i < v4) { f(order_key(t[u].x), 4 * i); f(order_key(t[u].y), 4 * i + 1); f(order_key(t[u].z), 4 * i + 2); f(order_key(t[u].w), 4 * i + 3); }
+        }
+    }
+    for (int c = (v4 << 2) + threadIdx.x; c < vocab; c += 1024) f(order_key(logits[c]), c);
+}
+
+__global__ void __launch_bounds__(1024) k_decode_sample(const float *__restrict__ logits, int32_t *__restrict__ state,
+                                                        int32_t *__restrict__ tokens, int capacity,
+                                                        const float *__restrict__ table, float *__restrict__ x, int vocab,
+                                                        int d, int n_positions, uint32_t *__restrict__ params) {
+    __shared__ uint64_t pool[kPool];                     // (key, ~index): larger = earlier in the stable descending order
+    __shared__ uint32_t most[1024];
+    __shared__ float probs[kSampleTopK];
+    __shared__ int s_count, s_tok;
+    const int t = threadIdx.x;
+    const float temperature = __builtin_bit_cast(float, params[2]);
+    int k = (int)params[3];
+    k = k < 1 ? 1 : k > kSampleTopK ? kSampleTopK : k;
+    if (k > vocab) k = vocab;
+
+    uint32_t bound = 0;                                  // candidates: key >= bound
+    if (vocab > kPool) {
+        uint32_t m = 0;
+        each_logit(logits, vocab, [&](uint32_t key, int) { m = key > m ? key : m; });
+        most[t] = m;
+        sort_descending(most, 1024);
+        bound = most[k - 1];
+    }
+    auto count_if = [&](auto &&pred) {                   // how many logits satisfy pred(key, index); every thread gets it
+        if (t == 0) s_count = 0;
+        __syncthreads();
+        int c = 0;
+        each_logit(logits, vocab, [&](uint32_t key, int i) { c += pred(key, i) ? 1 : 0; });
+        atomicAdd(&s_count, c);
+        __syncthreads();
+        const int r = s_count;
+        __syncthreads();
+        return r;
+    };
+    auto collect = [&](auto &&pred) {
+        if (t == 0) s_count = 0;
+        __syncthreads();
+        each_logit(logits, vocab, [&](uint32_t key, int i) {
+            if (!pred(key, i)) return;
+            const int at = atomicAdd(&s_count, 1);
+            if (at < kPool) pool[at] = ((uint64_t)key << 32) | (uint32_t)~i;
+        });
+        __syncthreads();
+        const int r = s_count;
+        __syncthreads();
+        return r;
+    };
+    int n = collect([&](uint32_t key, int) { return key >= bound; });
+    if (n > kPool) {
+        uint32_t kth = 0;                                // the k-th largest key ...
+        for (int bit = 31; bit >= 0; bit--) {
+            const uint32_t c = kth | (1u << bit);
+            if (count_if([&](uint32_t key, int) { return key >= c; }) >= k) kth = c;
+        }
+        const int ties = k - count_if([&](uint32_t key, int) { return key > kth; });
+        int lo = 0, hi = vocab - 1;                      // ... and the index of the last of its equals that belongs
+        while (lo < hi) {
+            const int mid = lo + (hi - lo) / 2;
+            if (count_if([&](uint32_t key, int i) { return key == kth && i <= mid; }) >= ties) hi = mid;
+            else lo = mid + 1;
+        }
+        n = collect([&](uint32_t key, int i) { return key > kth || (key == kth && i <= lo); });
+    }
+    int size = 2;
+    while (size < n) size <<= 1;
+    for (int i = n + t; i < size; i += 1024) pool[i] = 0;
+    sort_descending(pool, size);
+
+    auto index_of = [&](int i) { return (int)~(uint32_t)pool[i]; };
+    float v = t < k ? logits[index_of(t)] / temperature : -INFINITY;
+    float mx = (v != v) ? -INFINITY : v;                 // std::max(-inf, NaN) keeps -inf
+    mx = wave_max(mx);
+    if ((t & 63) == 0) most[t >> 6] = __builtin_bit_cast(uint32_t, mx);
+    __syncthreads();
+    mx = __builtin_bit_cast(float, most[0]);
+#pragma unroll
+    for (int w = 1; w < 16; w++) mx = fmaxf(mx, __builtin_bit_cast(float, most[w]));
+    if (t < k) probs[t] = d_exp(v - mx);
+    __syncthreads();
+    __shared__ float s_sum;
+    if (t == 0) {
+        float sum = 0.0f;
+#pragma unroll 8
+        for (int i = 0; i < k; i++) sum += probs[i];     // in order, as the host adds them
+        s_sum = sum;
+    }
+    __syncthreads();
+    if (t < k) probs[t] = probs[t] / s_sum;
+    __syncthreads();
+    if (t == 0) {
+        uint64_t seed = ((uint64_t)params[1] << 32) | params[0];       // java.util.Random.next(24)
+        seed = (seed * 0x5DEECE66DULL + 0xBULL) & ((1ULL << 48) - 1);
+        params[0] = (uint32_t)seed;
+        params[1] = (uint32_t)(seed >> 32);
+        const float u = (float)(seed >> 24) / 16777216.0f;
+        float cum = 0.0f;
+        int chosen = -1;
+#pragma unroll 8
+        for (int i = 0; i < k; i++) {
+            cum += probs[i];
+            if (chosen < 0 && u <= cum) chosen = i;
+        }
+        if (chosen < 0) chosen = k - 1;
+        const int tok = index_of(chosen), g = state[2];
+        if (g < capacity) tokens[g] = tok;
+        state[1] = tok;
+        state[0] += n_positions;
+        state[2] = g + 1;
+        s_tok = tok;
+    }
+    __syncthreads();
+    const float *src = table + (int64_t)s_tok * d;
+    for (int c = t; c < d; c += 1024) x[c] = src[c];
+}
+
 inline int row_grid(int rows) { return rows < 256 * 16 ? (rows < 1 ? 1 : rows) : 256 * 16; }
 
 }  // namespace
@@ -478,6 +646,12 @@ void launch_decode_next(hipStream_t s, const float *logits, int32_t *state, int3
                         const float *table, float *x, int vocab, int d, int n_positions) {
     launch_kernel(k_decode_next, dim3(1), dim3(1024), 0, s, logits, state, tokens, capacity, table, x, vocab, d,
                        n_positions);
+}
+
+void launch_decode_sample(hipStream_t s, const float *logits, int32_t *state, int32_t *tokens, int capacity,
+                          const float *table, float *x, int vocab, int d, int n_positions, uint32_t *params) {
+    launch_kernel(k_decode_sample, dim3(1), dim3(1024), 0, s, logits, state, tokens, capacity, table, x, vocab, d, n_positions,
+                  params);
 }
 
 void launch_argmax_rows(hipStream_t s, const float *a, int32_t *out, int rows, int cols) {

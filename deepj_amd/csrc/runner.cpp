@@ -86,10 +86,14 @@ struct Runner {
     int64_t prepared_budget = -1;                          // bytes such copies may take in all; -1: no limit
     int64_t prepared_bytes = 0;
     Acts dec, pre;
-    int32_t graph = 0, graph_unrolled = 0;                 // one token per replay / kGraphUnroll tokens per replay
+    int32_t sampler = -1;                                  // DECODE_SAMPLE's parameters
+    // Captured per-token streams by how the token is chosen (Choose): one token per replay / kGraphUnroll per replay.
+    int32_t graph[3] = {}, graph_unrolled[3] = {};
     bool finalized = false;
     int32_t pos = 0;          // host mirror of state[0]
     int32_t generated = 0;    // host mirror of state[2]
+    bool state_stale = false; // state[0] on the device is behind `pos` (a step was taken); see settle_state
+    int32_t stepped = 0;      // the token of that step
     std::string error;
 
     int hd() const { return cfg.d / cfg.heads; }
@@ -117,6 +121,8 @@ struct Runner {
 };
 
 using Stream = std::vector<int32_t>;
+// How a stream ends: with the logits, or with the next token chosen on the device.
+enum Choose { kNone = 0, kGreedy = 1, kSample = 2 };
 template <class... A> void emit(Stream &s, A... words) { (s.push_back((int32_t)words), ...); }
 
 void q8_linear(Stream &s, int32_t x, int32_t w, int32_t out, int m, int k, int n, int flags, int32_t gamma = -1,
@@ -449,19 +455,26 @@ void positions(Runner &r, Stream &s, int32_t x, int rows) {
     if (c.kind == 2) emit(s, DJ_OP_ADD_POSITIONS, x, r.pos_table, r.state, rows, c.d, c.max_seq);
 }
 
-Stream decode_stream(Runner &r, bool sample_on_device) {
+// The next token, its record and its embedding row in dec.x, n positions further on.
+void choose_next(Runner &r, Stream &s, Choose how, int n) {
+    const Config &c = r.cfg;
+    if (how == kGreedy) emit(s, DJ_OP_DECODE_NEXT, r.logits, r.state, r.tokens, c.max_seq, r.emb, r.dec.x, c.vocab, c.d, n);
+    if (how == kSample) emit(s, DJ_OP_DECODE_SAMPLE, r.logits, r.state, r.tokens, c.max_seq, r.emb, r.dec.x, c.vocab, c.d, n, r.sampler);
+}
+
+Stream decode_stream(Runner &r, Choose how) {
     const Config &c = r.cfg;
     Stream s;
-    // Greedy on the device: the previous step (or the prefill) already left the embedding of
-    // the token to process in dec.x.  Host sampling: gather it from state[1] first.
-    if (!sample_on_device) {
+    // A token chosen on the device: the previous step (or the prefill) already left its embedding in dec.x.  One chosen by
+    // the host: gather it from state[1] first.
+    if (how == kNone) {
         emit(s, DJ_OP_EMBED_GATHER, r.emb, r.state, r.dec.x, 1, c.d, c.vocab, 1);
         positions(r, s, r.dec.x, 1);
     }
     for (int l = 0; l < c.layers; l++) block_stream(r, s, r.dec, l, 1);
     head_stream(r, s, r.dec.x);
-    if (sample_on_device) {
-        emit(s, DJ_OP_DECODE_NEXT, r.logits, r.state, r.tokens, c.max_seq, r.emb, r.dec.x, c.vocab, c.d, 1);
+    if (how != kNone) {
+        choose_next(r, s, how, 1);
         positions(r, s, r.dec.x, 1);        // state[0] is already the position of the token just chosen
     }
     return s;
@@ -512,7 +525,7 @@ void check_ids(const Config &c, const int32_t *ids, int n) {
 }
 
 // The command stream that takes the n token ids in r.pre.ids through the model at the current position.
-Stream prompt_stream(Runner &r, int n, bool choose) {
+Stream prompt_stream(Runner &r, int n, Choose how) {
     const Config &c = r.cfg;
     alloc_acts(r, r.pre, n);
     ensure_prepared(r, n);
@@ -522,23 +535,36 @@ Stream prompt_stream(Runner &r, int n, bool choose) {
     for (int l = 0; l < c.layers; l++) block_stream(r, s, r.pre, l, n);
     emit(s, DJ_OP_COPY, r.pre.x, r.last_x, c.d, (int64_t)(n - 1) * c.d, 0);
     head_stream(r, s, r.last_x);
-    if (choose) {
-        emit(s, DJ_OP_DECODE_NEXT, r.logits, r.state, r.tokens, c.max_seq, r.emb, r.dec.x, c.vocab, c.d, n);
+    if (how != kNone) {
+        choose_next(r, s, how, n);
         if (r.pos + n < c.max_seq) positions(r, s, r.dec.x, 1);     // a full cache takes no further token
     }
     return s;
 }
 
+// The device's state words as the host knows them: {positions, token, tokens generated}.
+void upload_state(Runner &r, int32_t token) {
+    const int32_t st[4] = {r.pos, token, r.generated, 0};
+    hip(deepj_hip_upload(r.state, reinterpret_cast<const float *>(st), 4));
+    r.state_stale = false;
+}
+// A caller-chosen step leaves the device's position one behind (the next one uploads its own); whatever else reads the
+// state brings it up to date first.
+void settle_state(Runner &r) {
+    if (r.state_stale) upload_state(r, r.stepped);
+}
+
 // Runs the prompt rows through the model, filling the cache.  Leaves the last row's
-// logits in r.logits; with choose != 0 also picks the next token greedily on the device.
-void prefill(Runner &r, const int32_t *ids, int n, float *all_logits, bool choose) {
+// logits in r.logits; unless `how` is kNone the next token is chosen on the device as well.
+void prefill(Runner &r, const int32_t *ids, int n, float *all_logits, Choose how) {
     const Config &c = r.cfg;
     if (!r.finalized) finalize(r);
     if (n <= 0) throw Error("prefill: empty prompt");
     check_ids(c, ids, n);
     if (r.pos + n > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + n) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
-    Stream s = prompt_stream(r, n, choose);
+    settle_state(r);
+    Stream s = prompt_stream(r, n, how);
     hip(deepj_hip_upload(r.pre.ids, reinterpret_cast<const float *>(ids), n));   // (prompt_stream sized r.pre for n rows)
     r.run(s);
     if (all_logits) {
@@ -550,21 +576,16 @@ void prefill(Runner &r, const int32_t *ids, int n, float *all_logits, bool choos
         hip(deepj_hip_download(full, all_logits, (int64_t)n * c.vocab));
         r.release(full);
     }
-    if (choose) { r.pos += n; r.generated += 1; }
-    else {
-        // advance the position without choosing a token
-        int32_t st[4] = {r.pos + n, 0, r.generated, 0};
-        hip(deepj_hip_upload(r.state, reinterpret_cast<const float *>(st), 4));
-        r.pos += n;
-    }
+    r.pos += n;
+    if (how != kNone) r.generated += 1;
+    else upload_state(r, 0);            // advance the position without choosing a token
 }
 
 void reset(Runner &r) {
     if (!r.finalized) finalize(r);
-    int32_t st[4] = {0, 0, 0, 0};
-    hip(deepj_hip_upload(r.state, reinterpret_cast<const float *>(st), 4));
     r.pos = 0;
     r.generated = 0;
+    upload_state(r, 0);
 }
 
 // The runtime builds a kernel's function object on its first launch (a few hundred microseconds each), and the
@@ -572,7 +593,7 @@ void reset(Runner &r) {
 // attention variants, and a few graph-replayed tokens, move those costs from the first request to finalize();
 // the sequence state is cleared afterwards (the cache rows written here are never read: every row is rewritten
 // before the position counter reaches it).
-void decode_greedy(Runner &r, int steps, int mode);
+void decode(Runner &r, int steps, int mode, Choose how);
 void warm_up(Runner &r) {
     const Config &c = r.cfg;
     const char *env = getenv("DEEPJ_HIP_WARMUP");           // "0": skip (profiling runs that want only the request's launches)
@@ -581,46 +602,44 @@ void warm_up(Runner &r) {
     for (int n : {2048, 1024, 512, 256, 128, 64, 32, 16, 4}) {
         if (n > (int)ids.size()) continue;
         reset(r);
-        prefill(r, ids.data(), n, nullptr, true);
+        prefill(r, ids.data(), n, nullptr, kGreedy);
     }
     reset(r);
     const int steps = kGraphUnroll + 1;
     if (c.max_seq >= steps + 2) {
-        prefill(r, ids.data(), 1, nullptr, true);
-        decode_greedy(r, steps, 1);
+        prefill(r, ids.data(), 1, nullptr, kGreedy);
+        decode(r, steps, 1, kGreedy);
     }
     reset(r);
 }
 
-// Greedy steps on the device: each consumes state[1] at position state[0] and appends the argmax.
+// `times` replays of the graph of `tokens` consecutive per-token streams, captured on first use and again where the runtime
+// refuses it (the workspace it used has been replaced by a larger one since).
+void replay(Runner &r, int32_t &graph, Choose how, int tokens, int times) {
+    if (graph && deepj_hip_graph_launch(graph, times) == 0) return;
+    if (graph) hip(deepj_hip_graph_destroy(graph));
+    graph = 0;
+    Stream one = decode_stream(r, how), s;
+    for (int i = 0; i < tokens; i++) s.insert(s.end(), one.begin(), one.end());
+    hip(deepj_hip_graph_capture(s.data(), (int32_t)s.size(), &graph));
+    hip(deepj_hip_graph_launch(graph, times));
+}
+
+// Steps on the device: each consumes state[1] at position state[0] and appends the token chosen as `how` says.
 // mode 0: the per-token stream, eagerly; 1: the same stream as a replayed HIP graph.
-void decode_greedy(Runner &r, int steps, int mode) {
+void decode(Runner &r, int steps, int mode, Choose how) {
     const Config &c = r.cfg;
     if (steps <= 0) return;
     if (r.pos + steps > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + steps) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
-    const bool use_graph = mode == 1;
-    if (use_graph) {
+    settle_state(r);
+    if (mode == 1) {
         // A replay costs a few microseconds of its own on top of its kernels: long runs go through a graph
         // that holds kGraphUnroll consecutive tokens, the remainder through the one-token graph.
-        const int runs = steps / kGraphUnroll, rest = steps % kGraphUnroll;
-        if (runs > 0) {
-            if (!r.graph_unrolled) {
-                Stream one = decode_stream(r, true), s;
-                for (int i = 0; i < kGraphUnroll; i++) s.insert(s.end(), one.begin(), one.end());
-                hip(deepj_hip_graph_capture(s.data(), (int32_t)s.size(), &r.graph_unrolled));
-            }
-            hip(deepj_hip_graph_launch(r.graph_unrolled, runs));
-        }
-        if (rest > 0) {
-            if (!r.graph) {
-                Stream s = decode_stream(r, true);
-                hip(deepj_hip_graph_capture(s.data(), (int32_t)s.size(), &r.graph));
-            }
-            hip(deepj_hip_graph_launch(r.graph, rest));
-        }
+        if (steps >= kGraphUnroll) replay(r, r.graph_unrolled[how], how, kGraphUnroll, steps / kGraphUnroll);
+        if (steps % kGraphUnroll) replay(r, r.graph[how], how, 1, steps % kGraphUnroll);
     } else {
-        Stream s = decode_stream(r, true);
+        Stream s = decode_stream(r, how);
         for (int i = 0; i < steps; i++) r.run(s);
     }
     r.pos += steps;
@@ -629,40 +648,54 @@ void decode_greedy(Runner &r, int steps, int mode) {
 
 // One token through the single-row path with the token chosen by the caller: logits of the
 // new position end up in r.logits.  (Incremental decode with sampling done elsewhere.)
-void step_token(Runner &r, int32_t token) {
+void step_token(Runner &r, int32_t token, int mode) {
     const Config &c = r.cfg;
     if (!r.finalized) finalize(r);
     check_ids(c, &token, 1);
     if (r.pos + 1 > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + 1) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
-    int32_t st[4] = {r.pos, token, r.generated, 0};
-    hip(deepj_hip_upload(r.state, reinterpret_cast<const float *>(st), 4));
-    Stream fwd = decode_stream(r, false);
-    r.run(fwd);
+    upload_state(r, token);
+    // Replayed like a greedy token: the launches of a token one by one cost the host 2.4 us each (43 of them: 190 us a
+    // step of 8 layers, 130 as a graph).
+    if (mode == 1) replay(r, r.graph[kNone], kNone, 1, 1);
+    else r.run(decode_stream(r, kNone));
+    r.stepped = token;
     r.pos += 1;
-    st[0] = r.pos;
-    hip(deepj_hip_upload(r.state, reinterpret_cast<const float *>(st), 4));
+    r.state_stale = true;
 }
 
 // ── TextGenerator.sampleFromLogits on the host (temperature / top-k > 1) ────
 
-int java_float_compare(float x, float y) {
-    if (x < y) return -1;
-    if (x > y) return 1;
-    int32_t bx, by;
-    std::memcpy(&bx, &x, 4); std::memcpy(&by, &y, 4);
-    if (x != x) bx = 0x7fc00000;
-    if (y != y) by = 0x7fc00000;
-    return bx == by ? 0 : (bx < by ? -1 : 1);
+// The stable descending order of the logits (TextGenerator.java:163-170) by a radix sort: 11 bits a pass over keys that
+// order like Float.compare, least significant first, so equal logits keep their index order.
+void descending_order(const std::vector<float> &logits, std::vector<int32_t> &order) {
+    const size_t n = logits.size();
+    struct Item { uint32_t key; int32_t index; };
+    std::vector<Item> a(n), b(n);
+    constexpr int kBits = 11, kBuckets = 1 << kBits;
+    std::vector<uint32_t> count(3 * kBuckets, 0);
+    for (size_t i = 0; i < n; i++) {
+        uint32_t u;
+        std::memcpy(&u, &logits[i], 4);
+        if (logits[i] != logits[i]) u = 0x7fc00000u;
+        u = (u & 0x80000000u) ? u : ~u & 0x7fffffffu;         // descending: positive values by falling magnitude, then negative by rising
+        a[i] = {u, (int32_t)i};
+        for (int pass = 0; pass < 3; pass++) count[pass * kBuckets + ((u >> (pass * kBits)) & (kBuckets - 1))]++;
+    }
+    for (int pass = 0; pass < 3; pass++) {
+        uint32_t *c = count.data() + pass * kBuckets, at = 0;
+        for (int k = 0; k < kBuckets; k++) { const uint32_t here = c[k]; c[k] = at; at += here; }
+        for (const Item &it : a) b[c[(it.key >> (pass * kBits)) & (kBuckets - 1)]++] = it;
+        a.swap(b);
+    }
+    order.resize(n);
+    for (size_t i = 0; i < n; i++) order[i] = a[i].index;
 }
 
 int32_t sample_from_logits(const std::vector<float> &logits, float temperature, int top_k, void *rng) {
     int n = (int)logits.size();
-    std::vector<int32_t> order(n);
-    for (int i = 0; i < n; i++) order[i] = i;
-    // stable sort, descending (TextGenerator.java:163-170)
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int32_t i, int32_t j) { return java_float_compare(logits[j], logits[i]) < 0; });
+    std::vector<int32_t> order;
+    descending_order(logits, order);
     int k = top_k == 0 ? n : std::min(top_k, n);
     float mx = -INFINITY;
     for (int i = 0; i < k; i++) mx = std::max(mx, logits[order[i]] / temperature);
@@ -700,37 +733,41 @@ void generate(Runner &r, const int32_t *prompt, int n_prompt, int max_new, float
     if (max_new == 0) return;
     // tokens 0 .. cached-1 see a context that fits the window (n_prompt + t <= maxSeqLen)
     const int cached = n_prompt > c.max_seq ? 0 : std::min(max_new, c.max_seq - n_prompt + 1);
-    const bool greedy = top_k == 1;       // argmax needs no random draw to pick, and greedy output is seed independent
-    void *rng = greedy ? nullptr : deepj_host_random_create(seed);
+    // argmax needs no random draw to pick, and greedy output is seed independent; a moderate top-k is sampled on the
+    // device, so that those runs replay graphs too; the rest (whole vocabulary) is sorted and drawn from on the host
+    const Choose how = top_k == 1 ? kGreedy : top_k > 0 && top_k <= DEEPJ_HIP_SAMPLE_TOP_K ? kSample : kNone;
+    void *rng = how == kNone ? deepj_host_random_create(seed) : nullptr;
     try {
-        std::vector<float> logits(greedy ? 0 : (size_t)c.vocab);
+        std::vector<float> logits(how == kNone ? (size_t)c.vocab : 0);
         auto sample = [&](int t) {
             hip(deepj_hip_download(r.logits, logits.data(), c.vocab));
             out[n_prompt + t] = sample_from_logits(logits, temperature, top_k, rng);
         };
         reset(r);
-        if (cached > 0 && greedy) {
-            prefill(r, prompt, n_prompt, nullptr, true);
-            decode_greedy(r, cached - 1, mode);
+        if (how == kSample) {
+            if (r.sampler < 0) r.sampler = r.alloc(4);
+            const uint64_t start = ((uint64_t)seed ^ 0x5DEECE66DULL) & ((1ULL << 48) - 1);      // java.util.Random(seed)
+            int32_t params[4] = {(int32_t)(uint32_t)start, (int32_t)(start >> 32), 0, top_k};
+            std::memcpy(&params[2], &temperature, 4);
+            hip(deepj_hip_upload(r.sampler, reinterpret_cast<const float *>(params), 4));
+        }
+        if (cached > 0 && how != kNone) {
+            prefill(r, prompt, n_prompt, nullptr, how);
+            decode(r, cached - 1, mode, how);
             hip(deepj_hip_download(r.tokens, reinterpret_cast<float *>(out + n_prompt), cached));
         } else if (cached > 0) {
-            Stream fwd = decode_stream(r, false);
-            prefill(r, prompt, n_prompt, nullptr, false);
+            prefill(r, prompt, n_prompt, nullptr, kNone);
             for (int t = 0; t < cached; t++) {
-                if (t > 0) {
-                    r.run(fwd);          // consumes the token in state[1] at position state[0]
-                    r.pos += 1;
-                }
+                if (t > 0) step_token(r, out[n_prompt + t - 1], mode);
                 sample(t);
-                int32_t st[4] = {r.pos, out[n_prompt + t], t + 1, 0};
-                hip(deepj_hip_upload(r.state, reinterpret_cast<const float *>(st), 4));
                 r.generated = t + 1;
             }
+            upload_state(r, out[n_prompt + cached - 1]);
         }
         for (int t = cached; t < max_new; t++) {
             reset(r);
-            prefill(r, out + n_prompt + t - c.max_seq, c.max_seq, nullptr, greedy);
-            if (greedy) hip(deepj_hip_download(r.tokens, reinterpret_cast<float *>(out + n_prompt + t), 1));
+            prefill(r, out + n_prompt + t - c.max_seq, c.max_seq, nullptr, how);
+            if (how != kNone) hip(deepj_hip_download(r.tokens, reinterpret_cast<float *>(out + n_prompt + t), 1));
             else sample(t);
         }
     } catch (...) {
@@ -777,8 +814,9 @@ void *deepj_runner_create(const int32_t cfg[9], int32_t id_base) {
 void deepj_runner_destroy(void *h) {
     auto *r = static_cast<Runner *>(h);
     if (!r) return;
-    if (r->graph) deepj_hip_graph_destroy(r->graph);
-    if (r->graph_unrolled) deepj_hip_graph_destroy(r->graph_unrolled);
+    for (int how = 0; how < 3; how++)
+        for (int32_t g : {r->graph[how], r->graph_unrolled[how]})
+            if (g) deepj_hip_graph_destroy(g);
     deepj_hip_synchronize();
     // every id in [id_base, next_id) that is still live belongs to this runner
     std::vector<int32_t> ids;
@@ -789,7 +827,7 @@ void deepj_runner_destroy(void *h) {
             add(id);
     for (int32_t id : {r->emb, r->gf, r->wlm, r->blm, r->cos_t, r->sin_t, r->kc, r->vc, r->state,
                        r->tokens, r->scratch, r->records, r->logits, r->last_x,
-                       r->pos_table, r->bf, r->latent, r->kv_all})
+                       r->pos_table, r->bf, r->latent, r->kv_all, r->sampler})
         add(id);
     for (Acts *a : {&r->dec, &r->pre})
         for (int32_t id : {a->x, a->x2, a->qkv, a->q, a->att, a->ff, a->ids, a->cq, a->ckv}) add(id);
@@ -850,20 +888,20 @@ int deepj_runner_reset(void *h) {
 // all_logits: null, or room for n*vocab floats (logits of every prompt row, as DecoderOnlyModel.forward returns)
 int deepj_runner_prefill(void *h, const int32_t *ids, int32_t n, float *all_logits, int32_t choose_next) {
     auto *r = static_cast<Runner *>(h);
-    return guarded(r, [&] { prefill(*r, ids, n, all_logits, choose_next != 0); });
+    return guarded(r, [&] { prefill(*r, ids, n, all_logits, choose_next != 0 ? kGreedy : kNone); });
 }
 
 int deepj_runner_decode(void *h, int32_t steps, int32_t mode) {
     auto *r = static_cast<Runner *>(h);
     return guarded(r, [&] {
         if (mode < 0 || mode > 1) throw Error("decode: mode must be 0 (eager) or 1 (graph)");
-        decode_greedy(*r, steps, mode);
+        decode(*r, steps, mode, kGreedy);
     });
 }
 
 int deepj_runner_step(void *h, int32_t token) {
     auto *r = static_cast<Runner *>(h);
-    return guarded(r, [&] { step_token(*r, token); });
+    return guarded(r, [&] { step_token(*r, token, 1); });
 }
 
 int deepj_runner_last_logits(void *h, float *out) {
@@ -900,7 +938,7 @@ int deepj_runner_prefill_stream(void *h, int32_t n, int32_t *out, int32_t capaci
     return guarded(r, [&] {
         if (!r->finalized) finalize(*r);
         if (n <= 0 || r->pos + n > r->cfg.max_seq) throw Error("prefill_stream: row count outside the context window");
-        Stream s = prompt_stream(*r, n, false);
+        Stream s = prompt_stream(*r, n, kNone);
         if (len) *len = (int32_t)s.size();
         if (out && capacity >= (int32_t)s.size()) std::memcpy(out, s.data(), s.size() * sizeof(int32_t));
     });
@@ -911,7 +949,7 @@ int deepj_runner_decode_stream(void *h, int32_t *out, int32_t capacity, int32_t 
     auto *r = static_cast<Runner *>(h);
     return guarded(r, [&] {
         if (!r->finalized) finalize(*r);
-        Stream s = decode_stream(*r, true);
+        Stream s = decode_stream(*r, kGreedy);
         if (len) *len = (int32_t)s.size();
         if (out && capacity >= (int32_t)s.size()) std::memcpy(out, s.data(), s.size() * sizeof(int32_t));
     });

@@ -404,6 +404,7 @@ int stride_of(int op) {
         case DJ_OP_NOP: return 2;
         case DJ_OP_Q8_PREPARE: return 5;
         case DJ_OP_Q8_LINEAR_ROPE: return 20;
+        case DJ_OP_DECODE_SAMPLE: return 11;
         default: return -1;
     }
 }
@@ -850,16 +851,20 @@ void exec_one(Cursor &c) {
                                       reinterpret_cast<int32_t *>(out), (int)cap, w[5]);
             break;
         }
-        case DJ_OP_DECODE_NEXT: {
-            // [op, logits, state, tokens, capacity, table, x, vocab, d, nPos]
+        case DJ_OP_DECODE_NEXT: case DJ_OP_DECODE_SAMPLE: {
+            // [op, logits, state, tokens, capacity, table, x, vocab, d, nPos(, params)]
             int64_t cap = w[4], vocab = w[7], d = w[8];
-            if (cap < 0 || vocab <= 0 || d <= 0 || w[9] < 0) fail("OP_DECODE_NEXT: bad shape");
+            if (cap < 0 || vocab <= 0 || d <= 0 || w[9] < 0) fail(std::string(op_name(op)) + ": bad shape");
             const float *lg = buf(w[1], vocab, op, "logits");
             float *st = buf(w[2], 4, op, "state");
             float *tk = buf(w[3], std::max<int64_t>(cap, 1), op, "tokens");
             const float *tb = buf(w[5], vocab * d, op, "table");
             float *x = buf(w[6], d, op, "x");
-            if (run)
+            float *params = op == DJ_OP_DECODE_SAMPLE ? buf(w[10], 4, op, "params") : nullptr;
+            if (run && params)
+                launch_decode_sample(s, lg, reinterpret_cast<int32_t *>(st), reinterpret_cast<int32_t *>(tk), (int)cap, tb, x,
+                                     (int)vocab, (int)d, w[9], reinterpret_cast<uint32_t *>(params));
+            else if (run)
                 launch_decode_next(s, lg, reinterpret_cast<int32_t *>(st), reinterpret_cast<int32_t *>(tk), (int)cap,
                                    tb, x, (int)vocab, (int)d, w[9]);
             break;
@@ -1035,6 +1040,7 @@ const char *op_name(int op) {
         case DJ_OP_ROPE_ROWS: return "OP_ROPE_ROWS";
         case DJ_OP_ATTENTION_KV: return "OP_ATTENTION_KV";
         case DJ_OP_DECODE_NEXT: return "OP_DECODE_NEXT";
+        case DJ_OP_DECODE_SAMPLE: return "OP_DECODE_SAMPLE";
         case DJ_OP_ATTN_DECODE: return "OP_ATTN_DECODE";
         case DJ_OP_APPEND_ROWS: return "OP_APPEND_ROWS";
         case DJ_OP_Q8_LINEAR_DYN: return "OP_Q8_LINEAR_DYN";

@@ -129,6 +129,9 @@ class Stream:
     def decode_next(self, logits, state, tokens, capacity, table, x, vocab, d, n_pos=1):
         return self.emit(op.OP_DECODE_NEXT, logits, state, tokens, capacity, table, x, vocab, d, n_pos)
 
+    def decode_sample(self, logits, state, tokens, capacity, table, x, vocab, d, params, n_pos=1):
+        return self.emit(op.OP_DECODE_SAMPLE, logits, state, tokens, capacity, table, x, vocab, d, n_pos, params)
+
     def attn_decode(self, qkv, k_cache, v_cache, out, state, scratch, cos, sin, H, hd, max_seq, layer):
         return self.emit(op.OP_ATTN_DECODE, qkv, k_cache, v_cache, out, state, scratch, cos, sin, H, hd, max_seq, layer)
 

@@ -214,6 +214,10 @@ enum {
      *     and one pass over the [M x 3 d] product less than Q8_LINEAR followed by ROPE_KV_STORE, same results to the
      *     last bit or two of the rotation.  Only for shapes the fp16 GEMM takes with an unshared K
      *     (deepj_hip_q8_linear_rope_ok(M, K, d) != 0) and not through deepj_hip_flush_ops_noalloc; refused otherwise.
+     * DECODE_SAMPLE [op, logits, state, tokens, capacity, table, x, vocab, d, nPos, params]
+     *     DECODE_NEXT with the token drawn as J/models/TextGenerator.java:104-151 draws it.  params (4 int32 words): [0..1]
+     *     the 48-bit state of the java.util.Random (low word first), advanced by one draw; [2] the temperature's bits;
+     *     [3] top_k, 1 .. DEEPJ_HIP_SAMPLE_TOP_K (clamped to that and to the vocabulary)
      */
     DJ_OP_Q8_QUANTIZE = 64, DJ_OP_Q8_DEQUANTIZE = 65, DJ_OP_Q8_LINEAR = 66, DJ_OP_RMSNORM = 67,
     DJ_OP_SILU_MUL = 68, DJ_OP_EMBED_GATHER = 69, DJ_OP_ROPE_KV_STORE = 70, DJ_OP_ATTENTION = 71,
@@ -221,8 +225,11 @@ enum {
     DJ_OP_ROPE_ROWS = 76, DJ_OP_ATTENTION_KV = 77, DJ_OP_DECODE_NEXT = 78, DJ_OP_ATTN_DECODE = 79,
     DJ_OP_APPEND_ROWS = 80, DJ_OP_Q8_LINEAR_DYN = 81, /* 82 unused */ DJ_OP_LAYERNORM = 83,
     DJ_OP_ADD_POSITIONS = 84, DJ_OP_ATTN_DECODE_RECORDS = 85, DJ_OP_STREAM_READ = 86, DJ_OP_NOP = 87, DJ_OP_Q8_PREPARE = 88,
-    DJ_OP_Q8_LINEAR_ROPE = 89
+    DJ_OP_Q8_LINEAR_ROPE = 89, DJ_OP_DECODE_SAMPLE = 90
 };
+
+/* Largest top_k that DECODE_SAMPLE takes. */
+#define DEEPJ_HIP_SAMPLE_TOP_K 512
 
 enum { DJ_LIN_RMSNORM = 1, DJ_LIN_BIAS = 2, DJ_LIN_RESIDUAL = 4, DJ_LIN_SWIGLU = 8, DJ_LIN_LAYERNORM = 16,
        DJ_LIN_GELU = 32, DJ_LIN_ATTN_MERGE = 64 };

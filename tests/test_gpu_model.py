@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from deepj_amd import DeepSeekConfig, DeepSeekModel, HipNative, LlamaConfig, LlamaModel, TextGenerator
+from deepj_amd.fused import DeviceBuffers, Stream
 from deepj_amd.models import _DecoderOnlyModel
 from oracle import cpu_ref as ref
 
@@ -408,3 +409,37 @@ def test_short_and_chunked_prompts_on_prepared_weights_against_the_oracle():
     finally:
         gpu.close()
         ref.set_threads(1)
+
+
+@pytest.mark.parametrize("vocab,kind", [(1, "normal"), (3, "normal"), (513, "normal"), (2048, "normal"), (2049, "ties"), (5000, "equal"),
+                                        (4097, "nan"), (50257, "normal"), (50257, "ties")])
+@pytest.mark.parametrize("top_k,temperature", [(2, 1.0), (40, 0.7), (512, 1.6)])
+def test_sampling_on_the_device_draws_what_the_oracle_draws(vocab, kind, top_k, temperature):
+    """DECODE_SAMPLE at the sizes where its selection changes: fewer logits than candidates, one more than its pool, a pool
+    overflowing with ties (cut by index).  Token ids are whole numbers: they have to be the oracle's.  8 draws in a row, so
+    that the generator's state on the device is checked too."""
+    rng = np.random.default_rng(vocab + top_k)
+    logits = rng.standard_normal(vocab).astype(np.float32) * 3
+    if kind == "ties":
+        logits = np.round(logits)
+    if kind == "equal":
+        logits[:] = np.float32(-0.25)
+    if kind == "nan":
+        logits[[5, vocab // 2]] = np.nan
+        logits[7] = -np.inf
+    d, rnd = 36, ref.JavaRandom(99)
+    start = (99 ^ 0x5DEECE66D) & ((1 << 48) - 1)
+    dev = DeviceBuffers()
+    try:
+        table = rng.standard_normal((vocab, d)).astype(np.float32)
+        params = np.array([start & 0xFFFFFFFF, start >> 32, np.float32(temperature).view(np.uint32), top_k], np.uint32).view(np.int32)
+        lb, tb, pb = dev.upload(logits), dev.upload(table), dev.upload(params)
+        state, tokens, x = dev.upload(np.array([4, 0, 0, 0], np.int32)), dev.alloc(8), dev.alloc(d)
+        for _ in range(8):
+            Stream().decode_sample(lb, state, tokens, 8, tb, x, vocab, d, pb).run()
+        exp = [ref.sample_from_logits(logits, temperature, top_k, rnd) for _ in range(8)]
+        assert list(dev.download(tokens, (8,), np.int32)) == exp
+        assert list(dev.download(state, (4,), np.int32)) == [12, exp[-1], 8, 0]
+        assert np.array_equal(dev.download(x, (d,)), table[exp[-1]])
+    finally:
+        dev.release_all()
