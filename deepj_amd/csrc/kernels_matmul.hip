@@ -2,10 +2,8 @@
 //
 //   C[M x N] = A[M x K] . B      A fp32 row-major, fp32 accumulate
 //
-// fp32 B [K x N] row-major (OP_MATMUL; CpuBackend.java:168-188 in the reference): v_mfma_f32_32x32x2_f32.
-// 256 threads = 4 wavefronts; workgroup tile 64 x 64 (one 32 x 32 accumulator per wavefront) or 128 x 128 (four),
-// K advances 32 per step.  Both operand tiles sit k-major in LDS so the 64 lanes of an MFMA operand read 32
-// consecutive floats per half-wave (no bank conflicts).
+// fp32 B [K x N] row-major (OP_MATMUL; CpuBackend.java:168-188 in the reference): v_mfma_f32_32x32x2_f32 in k_matmul,
+// whose wavefronts share a tile's K and feed the matrix cores straight from the caches.
 //
 // Q8 B [N x Kp] int8 + one fp32 scale per 32-group (prefill-time Q8 GEMM; the M = 1 decode case is the HBM-bound
 // kernel in kernels_q8.hip): v_mfma_f32_32x32x16_bf16 at full fp32 accuracy.  An int8 weight is exact in bf16,
@@ -25,236 +23,164 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 namespace {
 
-constexpr int BM = 64, BN = 64, BK = 32;
-constexpr int PAD = 4;
-
-__global__ void __launch_bounds__(256) k_gemm(const float *__restrict__ A, const float *__restrict__ Bf,
-                                              float *__restrict__ C, int M, const int N, const int K,
-                                              GemmEpilogue ep) {
-    __shared__ float As[BK][BM + PAD];
-    __shared__ float Bl[BK][BN + PAD];
-
-    const int t = threadIdx.x;
-    const int lane = t & 63, wave = t >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    if (ep.m_dev) {
-        int live = ep.m_dev[0] + ep.m_extra;
-        if (live < M) M = live;
-        if (m0 >= M) return;                 // workgroup-uniform
-    }
-
-    floatx16 acc;
-#pragma unroll
-    for (int j = 0; j < 16; j++) acc[j] = 0.0f;
-
-    const int a_row = t >> 2;            // 0..63
-    const int a_k = (t & 3) * 8;         // 0,8,16,24
-    const bool a_vec = (K & 3) == 0;
-
-    // Register-staged software pipeline: the global loads of K-step i+1 are issued before the MFMAs of
-    // step i, so their latency hides behind the matrix work instead of adding to every step.
-    float va[8];                 // A: 8 consecutive k of one row
-    float wb[8];                 // B: 8 consecutive columns of one k
-    auto fetch = [&](int k0) {
-        {
-            int gr = m0 + a_row;
-            if (gr < M && a_vec && k0 + a_k + 8 <= K) {
-                const float4 *p = reinterpret_cast<const float4 *>(A + (int64_t)gr * K + k0 + a_k);
-                float4 x = p[0], y = p[1];
-                va[0] = x.x; va[1] = x.y; va[2] = x.z; va[3] = x.w; va[4] = y.x; va[5] = y.y; va[6] = y.z; va[7] = y.w;
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    int gk = k0 + a_k + j;
-                    va[j] = (gr < M && gk < K) ? A[(int64_t)gr * K + gk] : 0.0f;
-                }
-            }
-        }
-        {
-            int bk = t >> 3, bn = (t & 7) * 8;       // 8 consecutive columns per thread
-            int gk = k0 + bk;
-            if (gk < K && (N & 3) == 0 && n0 + bn + 8 <= N) {
-                const float4 *p = reinterpret_cast<const float4 *>(Bf + (int64_t)gk * N + n0 + bn);
-                float4 x = p[0], y = p[1];
-                wb[0] = x.x; wb[1] = x.y; wb[2] = x.z; wb[3] = x.w; wb[4] = y.x; wb[5] = y.y; wb[6] = y.z; wb[7] = y.w;
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    int gn = n0 + bn + j;
-                    wb[j] = (gk < K && gn < N) ? Bf[(int64_t)gk * N + gn] : 0.0f;
-                }
-            }
-        }
-    };
-    auto stage = [&]() {
-#pragma unroll
-        for (int j = 0; j < 8; j++) As[a_k + j][a_row] = va[j];
-        {
-            int bk = t >> 3, bn = (t & 7) * 8;
-#pragma unroll
-            for (int j = 0; j < 8; j++) Bl[bk][bn + j] = wb[j];
-        }
-    };
-
-    if (K > 0) fetch(0);
-    for (int k0 = 0; k0 < K; k0 += BK) {
-        stage();
-        __syncthreads();
-        if (k0 + BK < K) fetch(k0 + BK);
-
-        // ── 16 MFMA steps of K = 2 ─────────────────────────────────────────
-        const int half = lane >> 5, l32 = lane & 31;
-#pragma unroll
-        for (int kk = 0; kk < BK / 2; kk++) {
-            float a = As[2 * kk + half][wm * 32 + l32];
-            float b = Bl[2 * kk + half][wn * 32 + l32];
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
-        }
-        __syncthreads();
-    }
-
-    // ── epilogue: acc[j] is C[8*(j/4) + 4*(lane/32) + j%4][lane%32] of the wave tile ──
-    const int col = n0 + wn * 32 + (lane & 31);
-    if (col < N) {
-        float badd = 0.0f;
-        if (ep.bias) badd = ep.interleaved_bias ? ((col & 1) ? ep.bias2[col >> 1] : ep.bias[col >> 1]) : ep.bias[col];
-#pragma unroll
-        for (int j = 0; j < 16; j++) {
-            int row = m0 + wm * 32 + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
-            if (row < M) {
-                float v = acc[j];
-                if (ep.bias) v = v + badd;
-                if (ep.gelu) v = gemm_gelu(v);
-                if (ep.residual) v = ep.residual[(int64_t)row * N + col] + v;
-                C[(int64_t)row * N + col] = v;
-            }
-        }
-    }
-}
-
-// ── 128 x 128 workgroup tile ────────────────────────────────────────────────
-// Same data flow with each wavefront owning a 64 x 64 block (four 32 x 32 accumulators): every operand
-// value read from LDS feeds two MFMAs instead of one, which is what the 64 x 64 kernel is bound by.
+constexpr int BM = 64, BN = 64;            // Q8 tiles
 constexpr int BM2 = 128, BN2 = 128;
 
-__global__ void __launch_bounds__(256) k_gemm128(const float *__restrict__ A, const float *__restrict__ Bf,
-                                                 float *__restrict__ C, int M, const int N, const int K,
-                                                 GemmEpilogue ep) {
-    __shared__ float As[BK][BM2 + PAD];
-    __shared__ float Bl[BK][BN2 + PAD];
+// ── fp32 x fp32 ─────────────────────────────────────────────────────────────
+// One workgroup computes a tile of 32 TM x 32 TN; its KW wavefronts each multiply the WHOLE tile over their own share of K
+// (stages of 8 U consecutive k dealt in turn) and are added through LDS at the end, in a fixed order.  As no two
+// wavefronts want the same operand values there is nothing to stage: every lane loads what the matrix instruction takes
+// from it (row or column lane % 32, half of the stage's k by lane / 32, so A comes as 128-bit words) into registers,
+// D - 1 stages ahead, and the loop has no barrier.
+// Bound: the fp32 matrix rate at the large end (157 TFLOP/s: 64 cycles a 32 x 32 x 2 product), one trip to memory and the
+// launch at the small one.  What limits the stages in flight is the L1: a compute unit has 256 lines, and once more than
+// that are outstanding they evict one another (1 x 2752 x 1024 with twice the wavefronts: 11.4 us instead of 7.8).
+// Before (64 x 64 or 128 x 128 tiles staged through LDS, two barriers per 32 k) -> now: 64 x 256 x 256 10.3 -> 3.7 us,
+// 256 x 768 x 192 8.9 -> 3.9, 500 x 2752 x 1024 61 -> 32, 500 x 1024 x 2752 114 -> 33, 1024 x 7000 x 2048 326 -> 295
+// (100 TFLOP/s), 1000 x 2048 x 7000 391 -> 222 (129).
+__device__ __forceinline__ float at_bytes(const float *base, uint32_t bytes) {
+    return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + bytes);
+}
 
-    const int t = threadIdx.x;
-    const int lane = t & 63, wave = t >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.y * BM2, n0 = blockIdx.x * BN2;
-    if (ep.m_dev) {
-        int live = ep.m_dev[0] + ep.m_extra;
-        if (live < M) M = live;
-        if (m0 >= M) return;                 // workgroup-uniform
+template <int TM, int TN, int KW, int U, int D, bool VEC>
+__global__ void __launch_bounds__(64 * KW) k_matmul(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C,
+                                                    const int M, const int N, const int K, const int tiles_m, const int tiles_n) {
+    constexpr int SK = 8 * U;
+    constexpr int kStride = 36;                     // LDS row of a 32-column block (16-byte aligned, spreads the two halves)
+    __shared__ __align__(16) float red[KW][32 * kStride];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = lane >> 5, l32 = lane & 31;
+    // Workgroups go to the eight XCDs in turn: give each XCD a run of neighbouring tiles, along the larger operand, so
+    // that its L2 holds an eighth of that one.
+    const int total = tiles_m * tiles_n, xcd = blockIdx.x & 7, q = total >> 3, r = total & 7;
+    const int idx = xcd * q + (xcd < r ? xcd : r) + (int)(blockIdx.x >> 3);
+    const bool by_cols = N >= M;
+    const int tile_n = by_cols ? idx / tiles_m : idx % tiles_n, tile_m = by_cols ? idx % tiles_m : idx / tiles_n;
+    const int m0 = tile_m * 32 * TM, n0 = tile_n * 32 * TN;
+
+    // rows and columns past the matrix repeat its last one: their products are not stored
+    const float *Am = A + (int64_t)m0 * K;
+    uint32_t a_off[TM], b_off[TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        const int row = 32 * i + l32 < M - m0 ? 32 * i + l32 : M - 1 - m0;
+        a_off[i] = ((uint32_t)row * (uint32_t)K + 4u * U * half) * 4u;
+    }
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        const int col = n0 + 32 * j + l32 < N ? n0 + 32 * j + l32 : N - 1;
+        b_off[j] = (4u * U * half * (uint32_t)N + (uint32_t)col) * 4u;
     }
 
-    floatx16 acc[2][2];
+    floatx16 acc[TM][TN];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
 
-    const int a_row = t >> 1;            // 0..127
-    const int a_k = (t & 1) * 16;        // 0,16
-    const bool a_vec = (K & 3) == 0;
-
-    float va[16];                // A: 16 consecutive k of one row
-    float wb[16];                // B: 16 consecutive columns of one k
-    auto fetch = [&](int k0) {
-        {
-            int gr = m0 + a_row;
-            if (gr < M && a_vec && k0 + a_k + 16 <= K) {
-                const float4 *p = reinterpret_cast<const float4 *>(A + (int64_t)gr * K + k0 + a_k);
+    struct Stage { float a[U][TM][4], b[U][TN][4]; };
+    auto load = [&](Stage &st, int k0) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    float4 x = p[q];
-                    va[4 * q] = x.x; va[4 * q + 1] = x.y; va[4 * q + 2] = x.z; va[4 * q + 3] = x.w;
-                }
-            } else {
+        for (int u = 0; u < U; u++) {
 #pragma unroll
-                for (int j = 0; j < 16; j++) {
-                    int gk = k0 + a_k + j;
-                    va[j] = (gr < M && gk < K) ? A[(int64_t)gr * K + gk] : 0.0f;
+            for (int i = 0; i < TM; i++) {
+                const char *p = reinterpret_cast<const char *>(Am + k0 + 4 * u) + a_off[i];
+                if constexpr (VEC) {
+                    const float4 v = *reinterpret_cast<const float4 *>(p);
+                    st.a[u][i][0] = v.x; st.a[u][i][1] = v.y; st.a[u][i][2] = v.z; st.a[u][i][3] = v.w;
+                } else {
+#pragma unroll
+                    for (int x = 0; x < 4; x++) st.a[u][i][x] = reinterpret_cast<const float *>(p)[x];
                 }
             }
-        }
-        {
-            int bk = t >> 3, bn = (t & 7) * 16;      // 16 consecutive columns per thread
-            int gk = k0 + bk;
-            if (gk < K && (N & 3) == 0 && n0 + bn + 16 <= N) {
-                const float4 *p = reinterpret_cast<const float4 *>(Bf + (int64_t)gk * N + n0 + bn);
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    float4 x = p[q];
-                    wb[4 * q] = x.x; wb[4 * q + 1] = x.y; wb[4 * q + 2] = x.z; wb[4 * q + 3] = x.w;
-                }
-            } else {
+            for (int x = 0; x < 4; x++) {
+                const float *row = B + (int64_t)(k0 + 4 * u + x) * N;
 #pragma unroll
-                for (int j = 0; j < 16; j++) {
-                    int gn = n0 + bn + j;
-                    wb[j] = (gk < K && gn < N) ? Bf[(int64_t)gk * N + gn] : 0.0f;
-                }
+                for (int j = 0; j < TN; j++) st.b[u][j][x] = at_bytes(row, b_off[j]);
             }
         }
     };
-    auto stage = [&]() {
+    auto multiply = [&](const Stage &st) {
 #pragma unroll
-        for (int j = 0; j < 16; j++) As[a_k + j][a_row] = va[j];
-        {
-            int bk = t >> 3, bn = (t & 7) * 16;
+        for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int j = 0; j < 16; j++) Bl[bk][bn + j] = wb[j];
-        }
+            for (int x = 0; x < 4; x++)
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(st.a[u][i][x], st.b[u][j][x], acc[i][j], 0, 0, 0);
     };
 
-    if (K > 0) fetch(0);
-    for (int k0 = 0; k0 < K; k0 += BK) {
-        stage();
-        __syncthreads();
-        if (k0 + BK < K) fetch(k0 + BK);
-        const int half = lane >> 5, l32 = lane & 31;
+    // No load of the loop sits under a branch (the last one is repeated instead): the number in flight is then known at
+    // compile time, and a stage's products wait for that stage's loads alone.
+    const int stages = K / SK, mine = (stages - wave + KW - 1) / KW;
+    if (mine > 0) {
+        Stage st[D];
+        auto stage_k = [&](int i) { return (wave + (i < mine ? i : mine - 1) * KW) * SK; };
 #pragma unroll
-        for (int kk = 0; kk < BK / 2; kk++) {
-            float a0 = As[2 * kk + half][wm * 64 + l32], a1 = As[2 * kk + half][wm * 64 + 32 + l32];
-            float b0 = Bl[2 * kk + half][wn * 64 + l32], b1 = Bl[2 * kk + half][wn * 64 + 32 + l32];
-            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc[0][1], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc[1][1], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-
-    // epilogue: acc[i][jn][e] is C[32*i + 8*(e/4) + 4*(lane/32) + e%4][32*jn + lane%32] of the wave's 64 x 64 block
+        for (int d = 0; d < D - 1; d++) load(st[d], stage_k(d));
+        int i = 0;
+        for (; i + D <= mine; i += D) {
 #pragma unroll
-    for (int jn = 0; jn < 2; jn++) {
-        const int col = n0 + wn * 64 + 32 * jn + (lane & 31);
-        if (col >= N) continue;
-        float badd = 0.0f;
-        if (ep.bias) badd = ep.interleaved_bias ? ((col & 1) ? ep.bias2[col >> 1] : ep.bias[col >> 1]) : ep.bias[col];
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                int row = m0 + wm * 64 + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-                if (row < M) {
-                    float v = acc[i][jn][e];
-                    if (ep.bias) v = v + badd;
-                    if (ep.gelu) v = gemm_gelu(v);
-                    if (ep.residual) v = ep.residual[(int64_t)row * N + col] + v;
-                    C[(int64_t)row * N + col] = v;
-                }
+            for (int d = 0; d < D; d++) {
+                load(st[(d + D - 1) % D], stage_k(i + d + D - 1));
+                __builtin_amdgcn_sched_barrier(0);      // (the scheduler would move the loads down to their use)
+                multiply(st[d]);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
+#pragma unroll
+        for (int d = 0; d < D - 1; d++)
+            if (i + d < mine) multiply(st[d]);
     }
+    if (stages * SK < K && wave == stages % KW) {   // what is left of K, 8 at a time: zeros past its end, in both operands
+        const uint32_t back = 4u * (U - 1) * half;
+#pragma unroll
+        for (int i = 0; i < TM; i++) a_off[i] -= back * 4u;
+#pragma unroll
+        for (int j = 0; j < TN; j++) b_off[j] -= back * (uint32_t)N * 4u;
+        for (int k0 = stages * SK; k0 < K; k0 += 8) {
+            float a[TM][4], b[TN][4];
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                const int k = k0 + 4 * half + x;
+                const bool ok = k < K;
+#pragma unroll
+                for (int i = 0; i < TM; i++) a[i][x] = ok ? at_bytes(Am + k0 + x, a_off[i]) : 0.0f;
+#pragma unroll
+                for (int j = 0; j < TN; j++) b[j][x] = ok ? at_bytes(B + (int64_t)(k0 + x) * N, b_off[j]) : 0.0f;
+            }
+#pragma unroll
+            for (int x = 0; x < 4; x++)
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][x], b[j][x], acc[i][j], 0, 0, 0);
+        }
+    }
+
+    // acc[i][j][e] is C[32 i + 8 (e / 4) + 4 half + e % 4][32 j + l32] of the tile; 32 x 32 blocks leave one by one
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            if (i + j > 0) __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 16; e++) red[wave][(8 * (e >> 2) + 4 * half + (e & 3)) * kStride + l32] = acc[i][j][e];
+            __syncthreads();
+            for (int o = threadIdx.x; o < 1024; o += 64 * KW) {
+                const int row = o >> 5, col = o & 31;
+                float v = red[0][row * kStride + col];
+#pragma unroll
+                for (int w = 1; w < KW; w++) v += red[w][row * kStride + col];
+                if (m0 + 32 * i + row < M && n0 + 32 * j + col < N) C[(int64_t)(m0 + 32 * i + row) * N + n0 + 32 * j + col] = v;
+            }
+        }
 }
 
 // ── Q8 weights: three-way bf16 split of the activations ────────────────────
@@ -556,17 +482,44 @@ inline bool use_big_tile(int m, int n) {
 
 }  // namespace
 
+namespace {
+template <int TM, int TN, int KW, int U, int D>
+void launch_matmul(hipStream_t s, const float *a, const float *b, float *out, int m, int n, int k) {
+    const int tm = (m + 32 * TM - 1) / (32 * TM), tn = (n + 32 * TN - 1) / (32 * TN);
+    if ((k & 3) == 0) launch_kernel((k_matmul<TM, TN, KW, U, D, true>), dim3(tm * tn), dim3(64 * KW), 0, s, a, b, out, m, n, k, tm, tn);
+    else launch_kernel((k_matmul<TM, TN, KW, U, D, false>), dim3(tm * tn), dim3(64 * KW), 0, s, a, b, out, m, n, k, tm, tn);
+}
+}  // namespace
+
 void launch_matmul_f32(hipStream_t s, const float *a, const float *b, float *out, int m, int n, int k) {
     if (m <= 0 || n <= 0) return;
     if (k <= 0) { launch_fill(s, reinterpret_cast<uint32_t *>(out), 0u, (int64_t)m * n); return; }
-    GemmEpilogue ep{nullptr, nullptr, nullptr, 0, nullptr, 0, 0, 0};
-    if (use_big_tile(m, n)) {
-        dim3 grid2((n + BN2 - 1) / BN2, (m + BM2 - 1) / BM2);
-        launch_kernel(k_gemm128, grid2, dim3(256), 0, s, a, b, out, m, n, k, ep);
-        return;
+    // The tile with the least time on the busiest compute unit: rounds of 256 tiles times the 32 x 32 blocks of one times
+    // what a block's products take with this tile, relative to the best (measured at K = 1024 and 2752; a small tile loads
+    // more per product, and the rows of A that a tall one walks may share a cache set).
+    struct Shape { int tm, tn; double weight; };
+    static const Shape shapes[] = {{1, 1, 2.0}, {1, 2, 1.35}, {2, 2, 1.3}, {2, 3, 1.05}, {4, 2, 1.1}, {2, 4, 1.0}};
+    int best = 0;
+    double least = 0;
+    for (int i = 0; i < (int)(sizeof(shapes) / sizeof(shapes[0])); i++) {
+        const int64_t tiles = (int64_t)((m + 32 * shapes[i].tm - 1) / (32 * shapes[i].tm)) * ((n + 32 * shapes[i].tn - 1) / (32 * shapes[i].tn));
+        const double cost = (double)((tiles + 255) / 256) * shapes[i].tm * shapes[i].tn * shapes[i].weight;
+        if (i == 0 || cost < least) { least = cost; best = i; }
     }
-    dim3 grid((n + BN - 1) / BN, (m + BM - 1) / BM);
-    launch_kernel(k_gemm, grid, dim3(256), 0, s, a, b, out, m, n, k, ep);
+    const int64_t blocks = (int64_t)((m + 31) / 32) * ((n + 31) / 32);
+    switch (best) {
+        case 0:
+            // a tile per compute unit at most: more wavefronts share its K, with shorter stages so that their lines fit
+            if (blocks <= 256 && k > 256) launch_matmul<1, 1, 16, 1, 2>(s, a, b, out, m, n, k);
+            else if (blocks <= 256) launch_matmul<1, 1, 8, 4, 2>(s, a, b, out, m, n, k);
+            else launch_matmul<1, 1, 4, 4, 2>(s, a, b, out, m, n, k);
+            break;
+        case 1: launch_matmul<1, 2, 4, 1, 4>(s, a, b, out, m, n, k); break;
+        case 2: launch_matmul<2, 2, 4, 1, 2>(s, a, b, out, m, n, k); break;
+        case 3: launch_matmul<2, 3, 4, 1, 2>(s, a, b, out, m, n, k); break;
+        case 4: launch_matmul<4, 2, 4, 1, 2>(s, a, b, out, m, n, k); break;
+        default: launch_matmul<2, 4, 4, 1, 4>(s, a, b, out, m, n, k); break;
+    }
 }
 
 // Few tiles over a long K: how many workgroups share a tile's K (1: none).  A 64 x 64 tile's workgroup (1024 threads,

@@ -33,6 +33,21 @@ def test_matmul_matches_cpu(m, k, n):                                 # :70-78 (
         assert_close(ref.matmul(a, b), be.matmul(tensor(a), tensor(b)), 1e-4, 1e-4, f"matmul {m}x{k}x{n}")
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 33, 7), (31, 32, 8), (33, 65, 31), (32, 64, 256), (64, 96, 257), (40, 300, 515),
+                                   (97, 2000, 40), (256, 1003, 129), (320, 2752, 36), (500, 2700, 260), (1030, 1100, 130), (900, 4100, 68),
+                                   (2100, 1000, 37)])
+def test_matmul_tiles_and_remainders(m, n, k):
+    """Every tile of the dispatch with rows, columns and K that do not fill it, and K below, at and past a stage of its
+    loop.  Bound: a sum of k products in any order is off by at most k * 2^-24 * sum |a||b| (first order; the 2 covers the
+    second)."""
+    rng = np.random.default_rng(m * n + k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    with backend() as be:
+        got = be.matmul(tensor(a), tensor(b)).numpy().astype(np.float64)
+    bound = 2 * k * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
+    assert np.all(np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= bound)
+
+
 def test_matmul_rejects_shape_mismatch():                             # :80-86
     with backend() as be:
         with pytest.raises(ValueError, match="Shape mismatch"):
