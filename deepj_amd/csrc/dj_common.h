@@ -68,8 +68,11 @@ void launch_unary(hipStream_t s, int op, const float *a, float *out, int64_t n);
 void launch_scalar(hipStream_t s, int op, const float *a, float *out, float s0, float s1, int64_t n);
 void launch_broadcast(hipStream_t s, int op, const float *a, const float *v, float *out, int rows, int cols);
 void launch_transpose(hipStream_t s, const float *a, float *out, int rows, int cols);
-void launch_adamw(hipStream_t s, float *w, const float *g, float *mt, float *vt, int64_t n, float lr,
-                  float beta1, float beta2, float eps, float wd, float bc1, float bc2);
+// AdamW on up to kAdamTensors tensors in one launch (none of them shares memory with another)
+constexpr int kAdamTensors = 16;
+struct AdamTensor { float *w; const float *g; float *mt, *vt; int64_t n; float lr, beta1, beta2, eps, wd, bc1, bc2; };
+struct AdamTensors { AdamTensor t[kAdamTensors]; };
+void launch_adamw(hipStream_t s, const AdamTensors &tensors, int count);
 void launch_scatter_add(hipStream_t s, float *target, const float *idx, const float *grad, int target_rows,
                         int cols, int n_idx);
 void launch_fill(hipStream_t s, uint32_t *dst, uint32_t bits, int64_t n);

@@ -356,6 +356,8 @@ struct Cursor {
     int32_t pos;
     bool dry;          // validate only
     int64_t ws_need;   // workspace floats the stream needs (collected in the dry pass)
+    int32_t skip = 0;  // words behind this op whose ops its launch has taken along
+    bool alone = false; // every op by itself (per-op timing)
 };
 
 const char *op_name(int op);
@@ -543,13 +545,31 @@ void exec_one(Cursor &c) {
             break;
         }
         case DJ_OP_ADAMW_UPDATE: {
-            int64_t n = w[12]; need_positive(op, "n", n);
-            float *wt = buf(w[1], n, op, "w");
-            const float *gr = buf(w[2], n, op, "g");
-            float *mt = buf(w[3], n, op, "mt"), *vt = buf(w[4], n, op, "vt");
-            if (run)
-                launch_adamw(s, wt, gr, mt, vt, n, bits_to_float(w[5]), bits_to_float(w[6]), bits_to_float(w[7]),
-                             bits_to_float(w[8]), bits_to_float(w[9]), bits_to_float(w[10]), bits_to_float(w[11]));
+            // an optimiser steps its parameters one behind the other: those that share no buffer go out together
+            AdamTensors batch;
+            int count = 0;
+            auto shares = [&](const int32_t *v) {
+                for (const int32_t *u = w; u < v; u += 13)
+                    for (int i = 1; i <= 4; i++)
+                        for (int j = 1; j <= 4; j++)
+                            if (u[i] == v[j]) return true;
+                return false;
+            };
+            const int32_t *v = w;
+            do {
+                int64_t n = v[12]; need_positive(op, "n", n);
+                AdamTensor &t = batch.t[count++];
+                t.w = buf(v[1], n, op, "w"); t.g = buf(v[2], n, op, "g");
+                t.mt = buf(v[3], n, op, "mt"); t.vt = buf(v[4], n, op, "vt");
+                t.n = n;
+                t.lr = bits_to_float(v[5]); t.beta1 = bits_to_float(v[6]); t.beta2 = bits_to_float(v[7]); t.eps = bits_to_float(v[8]);
+                t.wd = bits_to_float(v[9]); t.bc1 = bits_to_float(v[10]); t.bc2 = bits_to_float(v[11]);
+                v += 13;
+            } while (run && !c.alone && count < kAdamTensors && v + 13 <= c.cmd + c.len && v[0] == DJ_OP_ADAMW_UPDATE && !shares(v));
+            if (run) {
+                launch_adamw(s, batch, count);
+                c.skip = (int32_t)(v - w) - 13;
+            }
             break;
         }
         case DJ_OP_SCATTER_ADD_ROWS: case DJ_OP_SCATTER_ADD_ROWS_ATOMIC: {
@@ -992,7 +1012,8 @@ void walk(const int32_t *cmd, int32_t len, bool dry, int64_t *ws_need) {
         if (c.pos + stride > len)
             fail(std::string(op_name(op)) + ": command stream truncated at word " + std::to_string(c.pos));
         exec_one(c);
-        c.pos += stride;
+        c.pos += stride + c.skip;
+        c.skip = 0;
     }
     if (ws_need) *ws_need = c.ws_need;
 }
@@ -1403,6 +1424,7 @@ int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float 
                 g.chain.valid = false;
                 for (int i = 0; i < n; i++) {
                     Cursor c{cmd, len, starts[(size_t)i], false, 0};
+                    c.alone = true;
                     g_launch_timing.pairs = ev.data() + (size_t)per_op * i;
                     g_launch_timing.used = 0;
                     g_launch_timing.armed = true;

@@ -322,3 +322,39 @@ def test_released_buffers_are_recycled_without_new_driver_allocations():
             t.materialize()
         after = HipNative.poolStats()
         assert after["driver_allocs"] == before, "in-place rebinding must reuse pooled blocks"
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 5), (33, 4), (127, 32), (129, 36), (300, 1003), (1025, 192), (5, 2752)])
+def test_column_sums_and_broadcasts_at_ragged_sizes(rows, cols):
+    """sumRows with rows and columns that do not fill its 32 x 128 (or 32 x 32) passes: bound rows * 2^-24 * sum |a|.  The
+    broadcasts give every value its own row's or column's operand: bit for bit."""
+    rng = np.random.default_rng(rows * cols)
+    a = rng.standard_normal((rows, cols)).astype(np.float32)
+    row, col = rng.standard_normal((1, cols)).astype(np.float32), rng.standard_normal((rows, 1)).astype(np.float32)
+    with backend() as be:
+        t = tensor(a)
+        got = be.sumRows(t).numpy()
+        assert np.all(np.abs(got - a.sum(0, dtype=np.float64)) <= 2 * rows * 2.0 ** -24 * np.abs(a).sum(0, dtype=np.float64))
+        assert np.array_equal(be.addRowVector(t, tensor(row)).numpy(), a + row)
+        assert np.array_equal(be.multiplyBroadcastRows(t, tensor(row)).numpy(), a * row)
+        assert np.array_equal(be.subtractBroadcastCols(t, tensor(col)).numpy(), a - col)
+        assert np.array_equal(be.divideBroadcastCols(t, tensor(col)).numpy(), a / col)
+
+
+def test_adamw_steps_recorded_together_match_steps_one_by_one():
+    """More tensors than one launch takes, odd sizes, and a parameter stepped twice in the same flush (which must see its
+    first step)."""
+    rng = np.random.default_rng(3)
+    shapes = [(1, n) for n in (1, 2, 3, 5, 7, 64, 255, 1001)] + [(33, 17)] * 11
+    hyper = (1e-2, 0.9, 0.999, 1e-8, 0.01, 0.1, 0.001)
+    results = []
+    for flush_each in (False, True):
+        rng = np.random.default_rng(3)
+        with backend() as be:
+            sets = [[tensor(np.abs(rng.standard_normal(s)).astype(np.float32)) for _ in range(4)] for s in shapes]
+            for k in list(range(len(sets))) + [2]:
+                be.adamWUpdate(*sets[k], *hyper)
+                if flush_each:
+                    be.graph.flush()
+            results.append([t.numpy().copy() for four in sets for t in four])
+    assert all(np.array_equal(x, y) for x, y in zip(*results))
