@@ -97,9 +97,10 @@ class ComputeGraph:
         self._cmd = array.array("i")
         self._op_count = 0
         self._pending_allocs: list[GpuBuffer] = []
-        self._pending_uploads: list[tuple[int, np.ndarray]] = []
+        self._pending_uploads: list[tuple[int, np.ndarray | int]] = []      # values, or how many zeros
         self._buf_to_tensor: dict[int, _TensorRef] = {}
         self._maybe_orphans: list[int] = []
+        self._zero_buffers = getattr(runtime, "zeroBuffers", None)
         self._host_array = getattr(runtime, "hostArray", None) or (lambda n: np.zeros(n, dtype=np.float32))
 
     # ── buffer management (ComputeGraph.java:172-234) ───────────────────────
@@ -118,7 +119,9 @@ class ComputeGraph:
         self._next_buf_id += 1
         buf.allocatedOnGpu = False
         self._pending_allocs.append(buf)
-        self._pending_uploads.append((buf.id, pack_f32(t)))
+        # a tensor nothing was ever written to is cleared on the device, where the runtime can, instead of sending zeros
+        zeros = t._data is None and self._zero_buffers is not None
+        self._pending_uploads.append((buf.id, buf.rows * buf.cols if zeros else pack_f32(t)))
         t.setGpuTag(buf)
         self._track(buf, t)
         return buf
@@ -234,8 +237,12 @@ class ComputeGraph:
         self._pending_allocs = []
 
     def _upload_pending(self) -> None:
+        zeros = [u for u in self._pending_uploads if type(u[1]) is int]
+        if zeros:                               # first: a buffer's zeros come before whatever else is sent to it
+            self._zero_buffers(zeros)
         for buf_id, data in self._pending_uploads:
-            self.runtime.uploadBuffer(buf_id, data)
+            if type(data) is not int:
+                self.runtime.uploadBuffer(buf_id, data)
         self._pending_uploads.clear()
 
     def _execute_pending(self) -> None:

@@ -26,6 +26,10 @@ class HipGpuRuntime:
     def flushOps(self, cmd_stream, length): HipNative.nativeFlushOps(cmd_stream if len(cmd_stream) == length else cmd_stream[:length], length)
     def hostArray(self, n): return host_array(n)
 
+    def zeroBuffers(self, buffers):
+        cmd = [w for buf_id, n in buffers for w in (op.OP_FILL, buf_id, 0, n)]
+        HipNative.nativeFlushOps(cmd, len(cmd))
+
 
 def _require_row_vector(v, target):
     if v.rows != 1 or v.cols != target.cols:
