@@ -42,6 +42,7 @@ SOURCES = {
     "kernels_matmul.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_gemm_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_q8.hip": [],
+    "kernels_decode.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "runner.cpp": [],
     "host_random.cpp": [],

@@ -207,4 +207,44 @@ void launch_decode_sample(hipStream_t s, const float *logits, int32_t *state, in
                           const float *table, float *x, int vocab, int d, int n_positions, uint32_t *params);
 int64_t attention_scratch_floats(int S, int H, int hd, int max_seq);
 
+// kernels_decode.hip: a block of a narrow model for one token in two launches.  Each leaves partial sums of its row to the
+// next, which starts from x + (their sum + bias), writes that to out and normalises it.
+struct DecodeRow {
+    const float *x;            // [d] the row two launches back (or the token's embedding)
+    const float *part;         // [n_part][d] partial sums to add to it
+    int n_part;
+    const int32_t *at_state;   // set: part is a table of `table_rows` rows, row state[0] of it the one partial sum (learned positions)
+    int table_rows;
+    const float *bias;         // [d] or null, added to the partial sums (if there are any)
+    float *out;                // [d] the finished row; not x, not part
+    const float *gamma, *beta; // the norm: gamma alone RMSNorm, both LayerNorm
+    int d;
+};
+struct DecodeAttn {
+    DecodeRow in;
+    const int8_t *wqkv; const float *s_qkv;     // [3 d] rows over d
+    const int8_t *wo; const float *s_wo;        // [d] rows over d
+    float *k_cache, *v_cache;                   // the layer's [H][max_seq][hd]
+    const int32_t *state;
+    const float *cos_t, *sin_t;
+    float *part;                                // [H][d]
+    int hd, max_seq;
+    float scale;
+};
+struct DecodeFfn {
+    DecodeRow in;
+    const int8_t *wgu; const float *s_gu;       // SwiGLU: rows 2 n gate, 2 n + 1 up; GELU: row n
+    const float *bg, *bu;                       // [dff] or null
+    const int8_t *wd; const float *s_d;         // [d] rows over dff
+    float *part;                                // [decode_ffn_parts(dff)][d]
+    int dff;
+    bool swiglu;
+};
+bool decode_block_ok(int d, int hd, int dff);
+int decode_block_positions(int hd);             // cached positions up to which this is the faster way
+int decode_ffn_parts(int dff);
+void launch_decode_attn(hipStream_t s, const DecodeAttn &a);
+void launch_decode_ffn(hipStream_t s, const DecodeFfn &a);
+void launch_decode_row(hipStream_t s, const DecodeRow &r);
+
 }  // namespace dj

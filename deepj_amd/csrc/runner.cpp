@@ -49,7 +49,10 @@ struct Config {
 
 struct Error : std::runtime_error { using std::runtime_error::runtime_error; };
 
-constexpr int kGraphUnroll = 4;     // tokens per replay of the unrolled decode graph
+// Tokens per replay of a decode graph.  A replay costs 13 us of its own, so long runs go through graphs of consecutive tokens;
+// 16 of them only where a token is short enough for that to be seen (kShortStream launches, 2.6 us each: 5 % at 11 of them).
+constexpr int kReplayTokens[] = {16, 4, 1};
+constexpr int kShortStream = 32;
 
 void hip(int rc) {
     if (rc != 0) throw Error(deepj_hip_last_error());
@@ -68,6 +71,7 @@ struct Acts {          // activation buffers for S rows
     int32_t x = -1, x2 = -1, qkv = -1, q = -1, att = -1, ff = -1, ids = -1;
     int32_t cq = -1;                                                 // MLA: [cQ | pad | cKV] rows (latent cache: cQ rows)
     int32_t ckv = -1;                                                // MLA with the latent cache: cKV rows
+    int32_t part_a = -1, part_f = -1;                                // DECODE_ATTN's / DECODE_FFN's partial sums (one row only)
 };
 
 struct Runner {
@@ -87,8 +91,8 @@ struct Runner {
     int64_t prepared_bytes = 0;
     Acts dec, pre;
     int32_t sampler = -1;                                  // DECODE_SAMPLE's parameters
-    // Captured per-token streams by how the token is chosen (Choose): one token per replay / kGraphUnroll per replay.
-    int32_t graph[3] = {}, graph_unrolled[3] = {};
+    // Captured per-token streams by how the token is chosen (Choose), whether the blocks are narrow, and kReplayTokens.
+    int32_t graph[3][2][3] = {};
     bool finalized = false;
     int32_t pos = 0;          // host mirror of state[0]
     int32_t generated = 0;    // host mirror of state[2]
@@ -97,6 +101,8 @@ struct Runner {
     std::string error;
 
     int hd() const { return cfg.d / cfg.heads; }
+    // up to this many positions a token's block takes two launches (DECODE_ATTN, DECODE_FFN), from there on five
+    int narrow_positions() const { return cfg.kind == 1 ? 0 : deepj_hip_decode_block_positions(cfg.d, hd(), cfg.dff); }
     // MLA: width of [cQ | pad | cKV]; cKV starts at a multiple of 32 so that the Q8 groups of Wuk and Wuv
     // (32 consecutive inputs) are the ones each matrix would get on its own
     int q_rank_padded() const { return (cfg.q_rank + 31) / 32 * 32; }
@@ -370,6 +376,10 @@ void finalize(Runner &r) {
     emit(s, DJ_OP_FILL, r.state, 0, 4);
     r.run(s);
     alloc_acts(r, r.dec, 1);
+    if (r.narrow_positions()) {
+        r.dec.part_a = r.alloc((int64_t)c.heads * c.d);
+        r.dec.part_f = r.alloc((int64_t)deepj_hip_decode_ffn_parts(c.dff) * c.d);
+    }
     // the prompt-sized buffers for the longest prompt the cache can take, so that no request pays for allocation
     alloc_acts(r, r.pre, c.max_seq);
     r.finalized = true;
@@ -440,6 +450,23 @@ void block_stream(Runner &r, Stream &s, Acts &a, int l, int S) {
     q8_linear(s, a.ff, L.wd, a.x, S, c.dff, d, DJ_LIN_BIAS | DJ_LIN_RESIDUAL, -1, L.bd, -1, a.x2);
 }
 
+// The blocks of one token whose embedding row is in dec.x (without its position row), two launches each; result in dec.x.
+void narrow_blocks_stream(Runner &r, Stream &s) {
+    const Config &c = r.cfg;
+    const Acts &a = r.dec;
+    const int parts = deepj_hip_decode_ffn_parts(c.dff), hd = r.hd();
+    const bool gpt = c.kind == 2;
+    for (int l = 0; l < c.layers; l++) {
+        const Layer &L = r.layers[l];
+        if (l == 0) emit(s, DJ_OP_DECODE_ATTN, a.x, gpt ? r.pos_table : -1, gpt ? -1 : 0, -1);
+        else emit(s, DJ_OP_DECODE_ATTN, a.q, a.part_f, parts, r.layers[l - 1].bd);
+        emit(s, a.x2, L.g1, L.be1, c.d, L.wqkv, L.wo, r.kc, r.vc, r.state, r.cos_t, r.sin_t, a.part_a, hd, c.max_seq, l);
+        emit(s, DJ_OP_DECODE_FFN, a.x2, a.part_a, c.heads, -1, a.q, L.g2, L.be2, c.d, L.wgu, L.bg, L.bu, L.wd, a.part_f, c.dff,
+             gpt ? DJ_LIN_GELU : DJ_LIN_SWIGLU);
+    }
+    emit(s, DJ_OP_DECODE_ROW, a.q, a.part_f, parts, r.layers[c.layers - 1].bd, a.x, c.d);
+}
+
 // logits = lmHead(normF(x)) on `rows` rows                                   DecoderOnlyModel.java:62-63
 void head_rows(Runner &r, Stream &s, int32_t x, int32_t out, int rows) {
     const Config &c = r.cfg;
@@ -462,21 +489,20 @@ void choose_next(Runner &r, Stream &s, Choose how, int n) {
     if (how == kSample) emit(s, DJ_OP_DECODE_SAMPLE, r.logits, r.state, r.tokens, c.max_seq, r.emb, r.dec.x, c.vocab, c.d, n, r.sampler);
 }
 
-Stream decode_stream(Runner &r, Choose how) {
+// narrow: the blocks in two launches each (only where narrow_positions() says that the model takes them)
+Stream decode_stream(Runner &r, Choose how, bool narrow) {
     const Config &c = r.cfg;
     Stream s;
     // A token chosen on the device: the previous step (or the prefill) already left its embedding in dec.x.  One chosen by
     // the host: gather it from state[1] first.
-    if (how == kNone) {
-        emit(s, DJ_OP_EMBED_GATHER, r.emb, r.state, r.dec.x, 1, c.d, c.vocab, 1);
+    if (how == kNone) emit(s, DJ_OP_EMBED_GATHER, r.emb, r.state, r.dec.x, 1, c.d, c.vocab, 1);
+    if (narrow) narrow_blocks_stream(r, s);
+    else {
         positions(r, s, r.dec.x, 1);
+        for (int l = 0; l < c.layers; l++) block_stream(r, s, r.dec, l, 1);
     }
-    for (int l = 0; l < c.layers; l++) block_stream(r, s, r.dec, l, 1);
     head_stream(r, s, r.dec.x);
-    if (how != kNone) {
-        choose_next(r, s, how, 1);
-        positions(r, s, r.dec.x, 1);        // state[0] is already the position of the token just chosen
-    }
+    choose_next(r, s, how, 1);
     return s;
 }
 
@@ -535,10 +561,7 @@ Stream prompt_stream(Runner &r, int n, Choose how) {
     for (int l = 0; l < c.layers; l++) block_stream(r, s, r.pre, l, n);
     emit(s, DJ_OP_COPY, r.pre.x, r.last_x, c.d, (int64_t)(n - 1) * c.d, 0);
     head_stream(r, s, r.last_x);
-    if (how != kNone) {
-        choose_next(r, s, how, n);
-        if (r.pos + n < c.max_seq) positions(r, s, r.dec.x, 1);     // a full cache takes no further token
-    }
+    choose_next(r, s, how, n);
     return s;
 }
 
@@ -593,7 +616,8 @@ void reset(Runner &r) {
 // attention variants, and a few graph-replayed tokens, move those costs from the first request to finalize();
 // the sequence state is cleared afterwards (the cache rows written here are never read: every row is rewritten
 // before the position counter reaches it).
-void decode(Runner &r, int steps, int mode, Choose how);
+int token_launches(const Config &c, bool narrow);
+void decode_steps(Runner &r, int steps, int mode, Choose how, bool narrow);
 void warm_up(Runner &r) {
     const Config &c = r.cfg;
     const char *env = getenv("DEEPJ_HIP_WARMUP");           // "0": skip (profiling runs that want only the request's launches)
@@ -604,25 +628,44 @@ void warm_up(Runner &r) {
         reset(r);
         prefill(r, ids.data(), n, nullptr, kGreedy);
     }
-    reset(r);
-    const int steps = kGraphUnroll + 1;
-    if (c.max_seq >= steps + 2) {
+    for (const bool narrow : {true, false}) {
+        if (narrow ? r.narrow_positions() == 0 : r.narrow_positions() >= c.max_seq) continue;
+        // every size of graph, or as many tokens as there is room for
+        const int steps = std::min(c.max_seq - 2, token_launches(c, narrow) <= kShortStream ? 16 + 4 + 1 : 4 + 1);
+        if (steps < 1) continue;
+        reset(r);
         prefill(r, ids.data(), 1, nullptr, kGreedy);
-        decode(r, steps, 1, kGreedy);
+        decode_steps(r, steps, 1, kGreedy, narrow);
     }
     reset(r);
 }
 
-// `times` replays of the graph of `tokens` consecutive per-token streams, captured on first use and again where the runtime
-// refuses it (the workspace it used has been replaced by a larger one since).
-void replay(Runner &r, int32_t &graph, Choose how, int tokens, int times) {
+// `times` replays of the graph of kReplayTokens[size] consecutive per-token streams, captured on first use and again where the
+// runtime refuses it (the workspace it used has been replaced by a larger one since).
+void replay(Runner &r, Choose how, bool narrow, int size, int times) {
+    int32_t &graph = r.graph[how][narrow][size];
     if (graph && deepj_hip_graph_launch(graph, times) == 0) return;
     if (graph) hip(deepj_hip_graph_destroy(graph));
     graph = 0;
-    Stream one = decode_stream(r, how), s;
-    for (int i = 0; i < tokens; i++) s.insert(s.end(), one.begin(), one.end());
+    Stream one = decode_stream(r, how, narrow), s;
+    for (int i = 0; i < kReplayTokens[size]; i++) s.insert(s.end(), one.begin(), one.end());
     hip(deepj_hip_graph_capture(s.data(), (int32_t)s.size(), &graph));
     hip(deepj_hip_graph_launch(graph, times));
+}
+
+// The launches of a token, roughly: blocks of 2 or 5, the row behind the narrow ones, the head and the choice.
+int token_launches(const Config &c, bool narrow) { return narrow ? 2 * c.layers + 3 : 5 * c.layers + 2; }
+
+void decode_steps(Runner &r, int steps, int mode, Choose how, bool narrow) {
+    if (mode != 1) {
+        Stream s = decode_stream(r, how, narrow);
+        for (int i = 0; i < steps; i++) r.run(s);
+        return;
+    }
+    for (int size = token_launches(r.cfg, narrow) <= kShortStream ? 0 : 1; size < 3; size++) {
+        if (steps >= kReplayTokens[size]) replay(r, how, narrow, size, steps / kReplayTokens[size]);
+        steps %= kReplayTokens[size];
+    }
 }
 
 // Steps on the device: each consumes state[1] at position state[0] and appends the token chosen as `how` says.
@@ -633,15 +676,9 @@ void decode(Runner &r, int steps, int mode, Choose how) {
     if (r.pos + steps > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + steps) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
     settle_state(r);
-    if (mode == 1) {
-        // A replay costs a few microseconds of its own on top of its kernels: long runs go through a graph
-        // that holds kGraphUnroll consecutive tokens, the remainder through the one-token graph.
-        if (steps >= kGraphUnroll) replay(r, r.graph_unrolled[how], how, kGraphUnroll, steps / kGraphUnroll);
-        if (steps % kGraphUnroll) replay(r, r.graph[how], how, 1, steps % kGraphUnroll);
-    } else {
-        Stream s = decode_stream(r, how);
-        for (int i = 0; i < steps; i++) r.run(s);
-    }
+    const int narrow = std::min(steps, std::max(0, r.narrow_positions() - r.pos));
+    if (narrow) decode_steps(r, narrow, mode, how, true);
+    if (steps > narrow) decode_steps(r, steps - narrow, mode, how, false);
     r.pos += steps;
     r.generated += steps;
 }
@@ -657,8 +694,9 @@ void step_token(Runner &r, int32_t token, int mode) {
     upload_state(r, token);
     // Replayed like a greedy token: the launches of a token one by one cost the host 2.4 us each (43 of them: 190 us a
     // step of 8 layers, 130 as a graph).
-    if (mode == 1) replay(r, r.graph[kNone], kNone, 1, 1);
-    else r.run(decode_stream(r, kNone));
+    const bool narrow = r.pos < r.narrow_positions();
+    if (mode == 1) replay(r, kNone, narrow, 2, 1);
+    else r.run(decode_stream(r, kNone, narrow));
     r.stepped = token;
     r.pos += 1;
     r.state_stale = true;
@@ -815,8 +853,9 @@ void deepj_runner_destroy(void *h) {
     auto *r = static_cast<Runner *>(h);
     if (!r) return;
     for (int how = 0; how < 3; how++)
-        for (int32_t g : {r->graph[how], r->graph_unrolled[how]})
-            if (g) deepj_hip_graph_destroy(g);
+        for (auto &sizes : r->graph[how])
+            for (int32_t g : sizes)
+                if (g) deepj_hip_graph_destroy(g);
     deepj_hip_synchronize();
     // every id in [id_base, next_id) that is still live belongs to this runner
     std::vector<int32_t> ids;
@@ -830,7 +869,7 @@ void deepj_runner_destroy(void *h) {
                        r->pos_table, r->bf, r->latent, r->kv_all, r->sampler})
         add(id);
     for (Acts *a : {&r->dec, &r->pre})
-        for (int32_t id : {a->x, a->x2, a->qkv, a->q, a->att, a->ff, a->ids, a->cq, a->ckv}) add(id);
+        for (int32_t id : {a->x, a->x2, a->qkv, a->q, a->att, a->ff, a->ids, a->cq, a->ckv, a->part_a, a->part_f}) add(id);
     for (int32_t id : r->prepared) add(id);
     if (!ids.empty()) deepj_hip_release(ids.data(), (int32_t)ids.size());
     delete r;
@@ -949,7 +988,7 @@ int deepj_runner_decode_stream(void *h, int32_t *out, int32_t capacity, int32_t 
     auto *r = static_cast<Runner *>(h);
     return guarded(r, [&] {
         if (!r->finalized) finalize(*r);
-        Stream s = decode_stream(*r, kGreedy);
+        Stream s = decode_stream(*r, kGreedy, r->pos < r->narrow_positions());
         if (len) *len = (int32_t)s.size();
         if (out && capacity >= (int32_t)s.size()) std::memcpy(out, s.data(), s.size() * sizeof(int32_t));
     });

@@ -407,8 +407,37 @@ int stride_of(int op) {
         case DJ_OP_Q8_PREPARE: return 5;
         case DJ_OP_Q8_LINEAR_ROPE: return 20;
         case DJ_OP_DECODE_SAMPLE: return 11;
+        case DJ_OP_DECODE_ATTN: return 20;
+        case DJ_OP_DECODE_FFN: return 16;
+        case DJ_OP_DECODE_ROW: return 7;
         default: return -1;
     }
+}
+
+float *buf(int32_t id, int64_t floats, int op, const char *role);
+
+// Words 1 .. 5 (and gamma, beta behind them) of the DECODE_* ops: the row they start from.
+DecodeRow decode_row(const int32_t *w, int op, int64_t d, bool norm, const int32_t *state, int64_t table_rows) {
+    DecodeRow r{};
+    const int64_t parts = w[3];
+    if (parts < (state ? -1 : 0)) fail(std::string(op_name(op)) + ": bad part count");
+    r.d = (int)d;
+    r.x = buf(w[1], d, op, "x");
+    if (parts == -1) { r.part = buf(w[2], table_rows * d, op, "part"); r.n_part = 1; r.at_state = state; r.table_rows = (int)table_rows; }
+    else if (parts > 0) { r.part = buf(w[2], parts * d, op, "part"); r.n_part = (int)parts; }
+    if (w[4] >= 0) r.bias = buf(w[4], d, op, "bias");
+    r.out = buf(w[5], d, op, "out");
+    if (r.out == r.x || r.out == r.part) fail(std::string(op_name(op)) + ": out needs a buffer of its own");
+    if (norm) {
+        r.gamma = buf(w[6], d, op, "gamma");
+        if (w[7] >= 0) r.beta = buf(w[7], d, op, "beta");
+    }
+    return r;
+}
+
+void q8_weight(int32_t id, int64_t k, int64_t rows, int op, const char *role, const int8_t *&wq, const float *&scales) {
+    wq = reinterpret_cast<const int8_t *>(buf(id, (q8_bytes((int)k, (int)rows) + 3) / 4, op, role));
+    scales = reinterpret_cast<const float *>(wq + q8_scale_offset_bytes((int)k, (int)rows));
 }
 
 float bits_to_float(int32_t b) { float f; std::memcpy(&f, &b, 4); return f; }
@@ -926,6 +955,51 @@ void exec_one(Cursor &c) {
                                            reinterpret_cast<const int32_t *>(st), ct, sn, (int)H, (int)hd, (int)max_seq);
             break;
         }
+        case DJ_OP_DECODE_ATTN: {
+            const int64_t d = w[8], hd = w[17], max_seq = w[18], layer = w[19];
+            if (max_seq <= 0 || layer < 0 || !decode_block_ok((int)d, (int)hd, 1)) fail("OP_DECODE_ATTN: bad shape");
+            const int64_t H = d / hd, per_layer = max_seq * d;
+            DecodeAttn a;
+            const int32_t *st = reinterpret_cast<const int32_t *>(buf(w[13], 4, op, "state"));
+            a.in = decode_row(w, op, d, true, st, max_seq);
+            q8_weight(w[9], d, 3 * d, op, "wqkv", a.wqkv, a.s_qkv);
+            q8_weight(w[10], d, d, op, "wo", a.wo, a.s_wo);
+            a.k_cache = buf(w[11], (layer + 1) * per_layer, op, "kCache") + layer * per_layer;
+            a.v_cache = buf(w[12], (layer + 1) * per_layer, op, "vCache") + layer * per_layer;
+            a.state = st;
+            a.cos_t = buf(w[14], max_seq * (hd / 2), op, "cos"); a.sin_t = buf(w[15], max_seq * (hd / 2), op, "sin");
+            a.part = buf(w[16], H * d, op, "partOut");
+            a.hd = (int)hd; a.max_seq = (int)max_seq;
+            a.scale = (float)(1.0 / std::sqrt((double)hd));
+            if (a.part == a.in.part || a.part == a.in.x || a.part == a.in.out) fail("OP_DECODE_ATTN: partOut needs a buffer of its own");
+            if (run) launch_decode_attn(s, a);
+            break;
+        }
+        case DJ_OP_DECODE_FFN: {
+            const int64_t d = w[8], dff = w[14];
+            const int flags = w[15];
+            if (dff <= 0 || !decode_block_ok((int)d, 32, (int)std::min<int64_t>(dff, 1 << 30))) fail("OP_DECODE_FFN: bad shape");
+            if (flags != DJ_LIN_SWIGLU && flags != DJ_LIN_GELU) fail("OP_DECODE_FFN: flags must be SWIGLU or GELU");
+            DecodeFfn a;
+            a.in = decode_row(w, op, d, true, nullptr, 0);
+            a.swiglu = flags == DJ_LIN_SWIGLU;
+            q8_weight(w[9], d, a.swiglu ? 2 * dff : dff, op, "wgu", a.wgu, a.s_gu);
+            a.bg = w[10] >= 0 ? buf(w[10], dff, op, "bg") : nullptr;
+            a.bu = w[11] >= 0 && a.swiglu ? buf(w[11], dff, op, "bu") : nullptr;
+            q8_weight(w[12], dff, d, op, "wd", a.wd, a.s_d);
+            a.part = buf(w[13], decode_ffn_parts((int)dff) * d, op, "partOut");
+            a.dff = (int)dff;
+            if (a.part == a.in.part || a.part == a.in.x || a.part == a.in.out) fail("OP_DECODE_FFN: partOut needs a buffer of its own");
+            if (run) launch_decode_ffn(s, a);
+            break;
+        }
+        case DJ_OP_DECODE_ROW: {
+            const int64_t d = w[6];
+            if (d <= 0) fail("OP_DECODE_ROW: bad shape");
+            const DecodeRow r = decode_row(w, op, d, false, nullptr, 0);
+            if (run) launch_decode_row(s, r);
+            break;
+        }
         case DJ_OP_APPEND_ROWS: {
             // [op, src, dst, state, rows, rowFloats, maxRows, dstOff]: dst[dstOff + (state[0]+i)*rowFloats ..] = src row i
             int64_t rows = w[4], rf = w[5], max_rows = w[6], off = w[7];
@@ -1062,6 +1136,9 @@ const char *op_name(int op) {
         case DJ_OP_ATTENTION_KV: return "OP_ATTENTION_KV";
         case DJ_OP_DECODE_NEXT: return "OP_DECODE_NEXT";
         case DJ_OP_DECODE_SAMPLE: return "OP_DECODE_SAMPLE";
+        case DJ_OP_DECODE_ATTN: return "OP_DECODE_ATTN";
+        case DJ_OP_DECODE_FFN: return "OP_DECODE_FFN";
+        case DJ_OP_DECODE_ROW: return "OP_DECODE_ROW";
         case DJ_OP_ATTN_DECODE: return "OP_ATTN_DECODE";
         case DJ_OP_APPEND_ROWS: return "OP_APPEND_ROWS";
         case DJ_OP_Q8_LINEAR_DYN: return "OP_Q8_LINEAR_DYN";
@@ -1282,6 +1359,8 @@ void deepj_hip_host_free(void *p) {
 void *deepj_hip_stream(void) { return g.ready ? (void *)g.stream : nullptr; }
 
 int32_t deepj_hip_attn_record_splits(void) { return kAttnRecordSplits; }
+int32_t deepj_hip_decode_block_positions(int32_t d, int32_t hd, int32_t dff) { return decode_block_ok(d, hd, dff) ? decode_block_positions(hd) : 0; }
+int32_t deepj_hip_decode_ffn_parts(int32_t dff) { return dff > 0 ? decode_ffn_parts(dff) : 0; }
 
 int64_t deepj_hip_attention_scratch_floats(int32_t S, int32_t H, int32_t hd, int32_t max_seq) {
     if (S <= 0 || H <= 0 || hd <= 0) return 0;

@@ -138,6 +138,16 @@ class Stream:
     def attn_decode_records(self, qkv, k_cache, v_cache, records, state, cos, sin, H, hd, max_seq, layer):
         return self.emit(op.OP_ATTN_DECODE_RECORDS, qkv, k_cache, v_cache, records, state, cos, sin, H, hd, max_seq, layer)
 
+    def decode_attn(self, x, part, n_part, bias, out, gamma, beta, d, wqkv, wo, k_cache, v_cache, state, cos, sin, part_out, hd, max_seq, layer):
+        return self.emit(op.OP_DECODE_ATTN, x, part, n_part, bias, out, gamma, beta, d, wqkv, wo, k_cache, v_cache, state, cos, sin, part_out,
+                         hd, max_seq, layer)
+
+    def decode_ffn(self, x, part, n_part, bias, out, gamma, beta, d, wgu, bg, bu, wd, part_out, dff, flags):
+        return self.emit(op.OP_DECODE_FFN, x, part, n_part, bias, out, gamma, beta, d, wgu, bg, bu, wd, part_out, dff, flags)
+
+    def decode_row(self, x, part, n_part, bias, out, d):
+        return self.emit(op.OP_DECODE_ROW, x, part, n_part, bias, out, d)
+
     def append_rows(self, src, dst, state, rows, row_floats, max_rows, dst_off=0):
         return self.emit(op.OP_APPEND_ROWS, src, dst, state, rows, row_floats, max_rows, dst_off)
 

@@ -71,6 +71,9 @@ OP_NOP = 87                # measurement floor: an empty kernel
 OP_Q8_PREPARE = 88         # a Q8 weight in the many-row GEMM's own layout (fp16 rows, transposed scales)
 OP_Q8_LINEAR_ROPE = 89     # the q | k | v projection of a prompt with RoPE and the cache append as its epilogue
 OP_DECODE_SAMPLE = 90      # DECODE_NEXT that samples (temperature, top-k, java.util.Random)
+OP_DECODE_ATTN = 91        # a narrow model's block for one token in two launches: this half and the next
+OP_DECODE_FFN = 92
+OP_DECODE_ROW = 93         # the row behind the last block
 
 LIN_RMSNORM = 1
 LIN_BIAS = 2
@@ -87,4 +90,5 @@ FUSED_STRIDES = {OP_Q8_QUANTIZE: 8, OP_Q8_DEQUANTIZE: 8, OP_Q8_LINEAR: 12, OP_RM
                  OP_EMBED_GATHER: 8, OP_ROPE_KV_STORE: 13, OP_ATTENTION: 12, OP_ARGMAX_ROWS: 5, OP_DECODE_ADVANCE: 6,
                  OP_COPY: 6, OP_FILL: 4, OP_ROPE_ROWS: 13, OP_ATTENTION_KV: 14, OP_DECODE_NEXT: 10, OP_ATTN_DECODE: 13,
                  OP_APPEND_ROWS: 8, OP_Q8_LINEAR_DYN: 10, OP_LAYERNORM: 7, OP_ADD_POSITIONS: 7,
-                 OP_ATTN_DECODE_RECORDS: 12, OP_STREAM_READ: 4, OP_NOP: 2, OP_Q8_PREPARE: 5, OP_Q8_LINEAR_ROPE: 20, OP_DECODE_SAMPLE: 11}
+                 OP_ATTN_DECODE_RECORDS: 12, OP_STREAM_READ: 4, OP_NOP: 2, OP_Q8_PREPARE: 5, OP_Q8_LINEAR_ROPE: 20, OP_DECODE_SAMPLE: 11,
+                 OP_DECODE_ATTN: 20, OP_DECODE_FFN: 16, OP_DECODE_ROW: 7}

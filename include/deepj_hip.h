@@ -218,6 +218,17 @@ enum {
      *     DECODE_NEXT with the token drawn as J/models/TextGenerator.java:104-151 draws it.  params (4 int32 words): [0..1]
      *     the 48-bit state of the java.util.Random (low word first), advanced by one draw; [2] the temperature's bits;
      *     [3] top_k, 1 .. DEEPJ_HIP_SAMPLE_TOP_K (clamped to that and to the vocabulary)
+     * A transformer block for one token in two launches, for narrow models (deepj_hip_decode_block_positions).  Each op starts from
+     * the row r = x + (part[0] + .. + part[nPart - 1] + bias) (part: nPart rows of d floats; nPart 0: r = x; nPart -1: part
+     * is a [maxSeq x d] table, row state[0] of it is added), writes r to `out` (a buffer of its own) and normalises it (beta
+     * -1: RMSNorm, else LayerNorm):
+     * DECODE_ATTN   [op, x, part, nPart, bias, out, gamma, beta, d, wqkv, wo, kCache, vCache, state, cosT, sinT, partOut, hd, maxSeq, layer]
+     *     norm, q | k | v, RoPE, cache append at position state[0], attention, output projection: partOut holds d / hd
+     *     rows of d floats that add up to the block's attention output
+     * DECODE_FFN    [op, x, part, nPart, bias, out, gamma, beta, d, wgu, bg, bu, wd, partOut, dff, flags]
+     *     norm, up projection(s) with bg (and bu; flags DJ_LIN_SWIGLU or DJ_LIN_GELU as in Q8_LINEAR), down projection without
+     *     its bias: partOut holds deepj_hip_decode_ffn_parts(dff) rows of d floats
+     * DECODE_ROW    [op, x, part, nPart, bias, out, d]      out = r
      */
     DJ_OP_Q8_QUANTIZE = 64, DJ_OP_Q8_DEQUANTIZE = 65, DJ_OP_Q8_LINEAR = 66, DJ_OP_RMSNORM = 67,
     DJ_OP_SILU_MUL = 68, DJ_OP_EMBED_GATHER = 69, DJ_OP_ROPE_KV_STORE = 70, DJ_OP_ATTENTION = 71,
@@ -225,7 +236,8 @@ enum {
     DJ_OP_ROPE_ROWS = 76, DJ_OP_ATTENTION_KV = 77, DJ_OP_DECODE_NEXT = 78, DJ_OP_ATTN_DECODE = 79,
     DJ_OP_APPEND_ROWS = 80, DJ_OP_Q8_LINEAR_DYN = 81, /* 82 unused */ DJ_OP_LAYERNORM = 83,
     DJ_OP_ADD_POSITIONS = 84, DJ_OP_ATTN_DECODE_RECORDS = 85, DJ_OP_STREAM_READ = 86, DJ_OP_NOP = 87, DJ_OP_Q8_PREPARE = 88,
-    DJ_OP_Q8_LINEAR_ROPE = 89, DJ_OP_DECODE_SAMPLE = 90
+    DJ_OP_Q8_LINEAR_ROPE = 89, DJ_OP_DECODE_SAMPLE = 90,
+    DJ_OP_DECODE_ATTN = 91, DJ_OP_DECODE_FFN = 92, DJ_OP_DECODE_ROW = 93
 };
 
 /* Largest top_k that DECODE_SAMPLE takes. */
@@ -236,6 +248,11 @@ enum { DJ_LIN_RMSNORM = 1, DJ_LIN_BIAS = 2, DJ_LIN_RESIDUAL = 4, DJ_LIN_SWIGLU =
 
 /* Key splits per head of ATTN_DECODE_RECORDS: its records buffer holds H * splits * (hd + 4) floats. */
 int32_t deepj_hip_attn_record_splits(void);
+
+/* 0 when DECODE_ATTN / DECODE_FFN do not take a model of this width, head width and hidden width, else the number of cached
+ * positions up to which they are the faster way through a block; rows of DECODE_FFN's partOut. */
+int32_t deepj_hip_decode_block_positions(int32_t d, int32_t hd, int32_t dff);
+int32_t deepj_hip_decode_ffn_parts(int32_t dff);
 
 /* Floats the scratch buffer of ATTENTION / ATTENTION_KV must hold for S query rows (0: none needed). */
 int64_t deepj_hip_attention_scratch_floats(int32_t S, int32_t H, int32_t hd, int32_t max_seq);

@@ -443,3 +443,77 @@ def test_sampling_on_the_device_draws_what_the_oracle_draws(vocab, kind, top_k, 
         assert np.array_equal(dev.download(x, (d,)), table[exp[-1]])
     finally:
         dev.release_all()
+
+
+@pytest.mark.parametrize("d,hd,dff,max_seq,pos", [
+    (32, 32, 1, 8, 0), (96, 32, 63, 40, 39), (128, 64, 65, 300, 255), (256, 32, 688, 256, 100), (160, 32, 864, 520, 519),
+    (224, 32, 130, 70, 1), (192, 64, 96, 200, 63), (256, 64, 3072, 1024, 1023), (64, 64, 1376, 65, 64)])
+@pytest.mark.parametrize("gpt", [False, True])
+def test_a_narrow_block_in_two_launches_matches_the_layers(d, hd, dff, max_seq, pos, gpt):
+    """DECODE_ATTN, DECODE_FFN, DECODE_ROW against the layers in float64 (on the dequantised weights): half steps of 64
+    inputs, a hidden width that leaves most of a workgroup idle, rows past the last whole tile, keys at the edges of a round."""
+    rng = np.random.default_rng(d + dff + pos)
+    H = d // hd
+    normal = lambda r, c, s: (rng.standard_normal((r, c)) * s).astype(np.float32)
+    x, g1, g2 = normal(1, d, 1.0), 1 + normal(1, d, 0.2), 1 + normal(1, d, 0.2)
+    be1, be2, table, bias, bd = normal(1, d, 0.2), normal(1, d, 0.2), normal(max_seq, d, 0.3), normal(1, d, 0.3), normal(1, d, 0.3)
+    rows = dff if gpt else 2 * dff
+    wqkv, wo, wgu, wd = normal(d, 3 * d, d ** -0.5), normal(d, d, d ** -0.5), normal(d, rows, d ** -0.5), normal(dff, d, dff ** -0.5)
+    bg, bu = normal(1, dff, 0.3), normal(1, dff, 0.3)
+    kc, vc, part = normal(H * max_seq, hd, 1.0), normal(H * max_seq, hd, 1.0), normal(3, d, 0.5)
+    cos, sin = ref.rope_tables(hd, max_seq)
+    dev = DeviceBuffers()
+    try:
+        def q8(w):
+            k, n = w.shape
+            src, dst = dev.upload(w), dev.alloc(HipNative.q8Floats(k, n))
+            Stream().q8_quantize(src, dst, k, n, 0, 1, n).run()
+            return dst, ref.q8_roundtrip(w).astype(np.float64)
+        (wqkv_b, wqkv), (wo_b, wo), (wgu_b, wgu), (wd_b, wd) = q8(wqkv), q8(wo), q8(wgu), q8(wd)
+        up = {k: dev.upload(v) for k, v in dict(x=x, g1=g1, g2=g2, be1=be1, be2=be2, table=table, bias=bias, bd=bd, bg=bg, bu=bu,
+                                                kc=kc, vc=vc, part=part, cos=cos, sin=sin).items()}
+        state = dev.upload(np.array([pos, 0, 0, 0], np.int32))
+        x1, x2, out, pa, pf = dev.alloc(d), dev.alloc(d), dev.alloc(d), dev.alloc(H * d), dev.alloc((dff + 63) // 64 * d)
+        s = Stream()
+        s.decode_attn(up["x"], up["table"] if gpt else up["part"], -1 if gpt else 3, -1 if gpt else up["bias"], x1, up["g1"],
+                      up["be1"] if gpt else -1, d, wqkv_b, wo_b, up["kc"], up["vc"], state, up["cos"], up["sin"], pa, hd, max_seq, 0)
+        s.decode_ffn(x1, pa, H, -1, x2, up["g2"], up["be2"] if gpt else -1, d, wgu_b, up["bg"], up["bu"], wd_b, pf, dff,
+                     32 if gpt else 8)
+        s.decode_row(x2, pf, (dff + 63) // 64, up["bd"], out, d)
+        s.run()
+        got = [dev.download(b, (d,)) for b in (x1, x2, out)]
+        keys, values = (dev.download(up[n], (H, max_seq, hd)) for n in ("kc", "vc"))
+        s.run()                                                    # the same bits again: sums are taken in a fixed order
+        assert np.array_equal(got[2], dev.download(out, (d,)))
+    finally:
+        dev.release_all()
+
+    def norm(v, g, b):
+        if gpt:
+            return (v - v.mean()) / np.sqrt(v.var() + 1e-5) * g + b
+        return v / np.sqrt(np.mean(v * v) + 1e-6) * g
+    x = x.astype(np.float64)
+    r1 = x + (table[pos] if gpt else part.sum(0) + bias)
+    qkv = norm(r1, g1, be1) @ wqkv
+    q, k = ((lambda t: np.stack([t[..., 0::2] * cos[pos] - t[..., 1::2] * sin[pos], t[..., 0::2] * sin[pos] + t[..., 1::2] * cos[pos]], -1)
+             .reshape(H, hd))(qkv[0, i * d:(i + 1) * d].reshape(H, hd)) for i in (0, 1))
+    K, V = kc.reshape(H, max_seq, hd).astype(np.float64), vc.reshape(H, max_seq, hd).astype(np.float64)
+    K[:, pos], V[:, pos] = k, qkv[0, 2 * d:].reshape(H, hd)
+    p = np.einsum("hd,hkd->hk", q, K[:, :pos + 1]) / np.sqrt(hd)
+    p = np.exp(p - p.max(1, keepdims=True))
+    att = np.einsum("hk,hkd->hd", p / p.sum(1, keepdims=True), V[:, :pos + 1]).reshape(1, d)
+    r2 = r1 + att @ wo
+    h = norm(r2, g2, be2) @ wgu
+    if gpt:
+        h = h + bg
+        h = 0.5 * h * (1 + np.tanh(np.sqrt(2 / np.pi) * (h + 0.044715 * h ** 3)))
+    else:
+        gate, upv = h[:, 0::2] + bg, h[:, 1::2] + bu
+        h = gate / (1 + np.exp(-gate)) * upv
+    # wgu was laid out with gate n in column 2 n; every value here is of order 1 and a sum of at most 3072 products of which no
+    # chain adds more than 64 roundings: a few times 64 * 2^-24 = 4e-6 through the five products in a row
+    exp = [r1, r2, r2 + h @ wd + bd]
+    for name, a, b in zip(("row", "attention", "feed-forward"), got, exp):
+        err = float(np.max(np.abs(a - b)))
+        assert err <= 4e-5, (name, err)
+    assert float(np.max(np.abs(keys - K))) <= 2e-5 and float(np.max(np.abs(values - V))) <= 2e-5
