@@ -70,11 +70,34 @@ __device__ __forceinline__ void rope_store(const RopeStore &r, const RopeColumn 
     else *reinterpret_cast<float4 *>(r.k_cache + at) = o;
 }
 
+// tanh for the GELU below, in double to within 1e-9 absolute (its result is rounded to float and added to 1, where that is a
+// 60th of a unit in the last place): 1 - 2 / (1 + 2^y), y = 2 t log2(e), 2^y from the power series of e^(f ln 2) to the
+// eighth degree for |f| <= 1/2.  The math library's tanh is right to the last bit of a double, in some 2 KB of code that
+// a decode step fetches anew at every launch: the matvec of 768 -> 3072 with GELU took 5.9 us with it and takes 4.2 with this.
+__device__ __forceinline__ double gelu_tanh(float t) {
+    double y = (double)t * 2.88539008177792681472;              // 2 log2(e)
+    y = y > 64.0 ? 64.0 : (y < -64.0 ? -64.0 : y);              // tanh is +-1 in float long before; a NaN stays one
+    const double n = rint(y), f = y - n;
+    double p = 1.3215486790144305e-06;
+    p = fma(p, f, 1.5252733804059838e-05);
+    p = fma(p, f, 0.00015403530393381606);
+    p = fma(p, f, 0.0013333558146428441);
+    p = fma(p, f, 0.009618129107628477);
+    p = fma(p, f, 0.055504108664821576);
+    p = fma(p, f, 0.2402265069591007);
+    p = fma(p, f, 0.6931471805599453);
+    p = fma(p, f, 1.0);
+    const double den = 1.0 + ldexp(p, (int)n);
+    double r = __builtin_amdgcn_rcp(den);
+    r = fma(fma(-den, r, 1.0), r, r);
+    return fma(-2.0, r, 1.0);
+}
+// tensor/cpu/CpuBackend.java:338 (tanh form)
 __device__ __forceinline__ float gemm_gelu(float x) {
     float c = sqrtf(2.0f / 3.14159265358979323846f);
     float x3 = x * x * x;
     float t = c * (x + 0.044715f * x3);
-    return 0.5f * x * (1.0f + (float)tanh((double)t));
+    return 0.5f * x * (1.0f + (float)gelu_tanh(t));
 }
 
 }  // namespace dj

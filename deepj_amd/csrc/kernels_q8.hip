@@ -59,13 +59,6 @@ __device__ __forceinline__ float wave_sum(float v) {
 // The epilogue sits on the critical path of every wavefront: single precision exp (about 1 ulp) instead of the
 // double precision one the element-wise SIGMOID opcode uses; the difference is far inside the 1e-4 per-op bound.
 __device__ __forceinline__ float d_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
-// tensor/cpu/CpuBackend.java:338 (tanh form)
-__device__ __forceinline__ float d_gelu(float x) {
-    float c = sqrtf(2.0f / 3.14159265358979323846f);
-    float x3 = x * x * x;
-    float t = c * (x + 0.044715f * x3);
-    return 0.5f * x * (1.0f + (float)tanh((double)t));
-}
 
 // ── quantise: grid (ceil(N/64), Kp/32); a workgroup takes 64 columns x one group ──
 __global__ void __launch_bounds__(kThreads) k_q8_quantize(const float *__restrict__ w, int8_t *__restrict__ q,
@@ -231,7 +224,7 @@ __device__ __forceinline__ void finish_batch(const RowBatch<NC, B *(SWIGLU ? 2 :
                 } else {
                     v = acc[u];
                     if (p.bias) v = v + eb[u];
-                    if constexpr (GELU) v = d_gelu(v);
+                    if constexpr (GELU) v = gemm_gelu(v);
                 }
                 if (p.residual) v = er[u] + v;
                 p.out[o] = v;
@@ -305,7 +298,7 @@ __device__ __forceinline__ void stage_digits(float *xs, int plane0, int shift_at
 // applies the RMSNorm prologue; after that the next batch is always in flight while
 // the current one is multiplied (two register buffers used in turn).
 // MODE (compile time, so that the other variants do not pay for its registers): 1 = GELU on the biased sum
-// (its double-precision tanh costs some forty registers); 2 = ATTN_MERGE prologue: x is not the activation row
+// (its double-precision tanh costs registers); 2 = ATTN_MERGE prologue: x is not the activation row
 // but the per-split records [head][kAttnRecordSplits][hd + 4] = {max, sum, -, -, o[hd]} the decode attention
 // kernel left, and the row is their merge  x[h*hd + j] = sum_s w_s o_s[j] / sum_s w_s l_s,  w_s = exp(max_s - max).
 // PRO (compile time too: an operand that is not there must not be loaded - a workgroup's activation-sized loads
