@@ -44,6 +44,8 @@ def _bind(lib: C.CDLL) -> None:
     lib.deepj_hip_pool_stats.argtypes = [C.POINTER(C.c_int64)]
     lib.deepj_hip_stream.restype = C.c_void_p
     lib.deepj_hip_attn_record_splits.restype = C.c_int32
+    lib.deepj_hip_latent_decode_splits.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32]
+    lib.deepj_hip_latent_decode_splits.restype = C.c_int32
     lib.deepj_hip_attention_scratch_floats.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32]
     lib.deepj_hip_attention_scratch_floats.restype = C.c_int64
     lib.deepj_hip_q8_floats.argtypes = [C.c_int32, C.c_int32]
@@ -212,6 +214,10 @@ class HipNative:
     @staticmethod
     def attnRecordSplits() -> int:
         return int(library().deepj_hip_attn_record_splits())
+
+    @staticmethod
+    def latentDecodeSplits(H: int, hd: int, rank: int, max_seq: int) -> int:
+        return int(library().deepj_hip_latent_decode_splits(H, hd, rank, max_seq))
 
     @staticmethod
     def q8PreparedFloats(k: int, rows: int) -> int:

@@ -44,6 +44,7 @@ SOURCES = {
     "kernels_q8.hip": [],
     "kernels_decode.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "kernels_latent.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "runner.cpp": [],
     "host_random.cpp": [],
 }

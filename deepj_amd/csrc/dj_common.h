@@ -189,6 +189,8 @@ void launch_rope_rows(hipStream_t s, const float *x, float *out, const int32_t *
                       const float *sin_t, int rows, int H, int hd, int max_seq, int pos_from_row, int row_stride,
                       int live_extra);
 void launch_attention(hipStream_t s, const AttnArgs &a);
+// out [heads][hd] from base-2 records [heads][shares][hd + 4] = {max, sum, -, -, o[hd]} (max -inf: no keys)
+void launch_attention_merge(hipStream_t s, const float *records, float *out, int heads, int hd, int shares);
 void launch_attn_decode(hipStream_t s, const float *qkv, float *k_cache, float *v_cache, float *out,
                         const int32_t *state, float *scratch, const float *cos_t, const float *sin_t, int H, int hd,
                         int max_seq, unsigned *counters);
@@ -246,5 +248,21 @@ int decode_ffn_parts(int dff);
 void launch_decode_attn(hipStream_t s, const DecodeAttn &a);
 void launch_decode_ffn(hipStream_t s, const DecodeFfn &a);
 void launch_decode_row(hipStream_t s, const DecodeRow &r);
+
+// Decode attention over the latent cache (kernels_latent.hip)
+struct LatentDecode {
+    const float *q;                             // [d] the token's queries, not rotated
+    const float *ckv;                           // [rank] its latent row
+    float *latent;                              // the layer's [max_seq][rank]
+    const int8_t *wq; const float *scales;      // [2 d] rows over rank: Wuk, then Wuv
+    const int32_t *state;
+    const float *cos_t, *sin_t;
+    float *records, *out;                       // [heads][splits][hd + 4], [d]
+    int heads, hd, rank, max_seq;
+    float scale;                                // set by the launcher
+};
+int latent_decode_splits(int heads, int hd, int rank, int max_seq);
+void latent_decode_configure();                 // once per device, before the first launch
+void launch_latent_decode(hipStream_t s, LatentDecode a);
 
 }  // namespace dj

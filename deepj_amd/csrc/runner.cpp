@@ -370,6 +370,7 @@ void finalize(Runner &r) {
     // attention scratch: the split records of one row (decode paths) or of a short prompt whose key rounds are shared
     int64_t sf = (int64_t)c.heads * ns * (hd + 4);
     for (int rows = 2; rows <= 32; rows++) sf = std::max(sf, deepj_hip_attention_scratch_floats(rows, c.heads, hd, c.max_seq));
+    if (c.latent) sf = std::max(sf, (int64_t)c.heads * deepj_hip_latent_decode_splits(c.heads, hd, c.kv_rank, c.max_seq) * (hd + 4));
     r.scratch = r.alloc(sf);
     r.records = r.alloc((int64_t)c.heads * deepj_hip_attn_record_splits() * (hd + 4));
     Stream s;
@@ -408,11 +409,16 @@ void block_stream(Runner &r, Stream &s, Acts &a, int l, int S) {
         q8_linear(s, a.x, L.wdq, a.cq, S, d, qr, DJ_LIN_RMSNORM, L.g1);
         q8_linear(s, a.cq, L.wuq, a.qkv, S, qr, d, 0);
         q8_linear(s, a.x, L.wdkv, a.ckv, S, d, kvr, DJ_LIN_RMSNORM, L.g1);
-        emit(s, DJ_OP_APPEND_ROWS, a.ckv, r.latent, r.state, S, kvr, c.max_seq, lat_off);
-        emit(s, DJ_OP_Q8_LINEAR_DYN, r.latent, L.wukv, r.kv_all, c.max_seq, kvr, 2 * d, r.state, S, lat_off);
-        emit(s, DJ_OP_ROPE_ROWS, r.kv_all, r.kv_all, r.state, r.cos_t, r.sin_t, c.max_seq, H, hd, c.max_seq, 1, 2 * d, S);
-        emit(s, DJ_OP_ROPE_ROWS, a.qkv, a.q, r.state, r.cos_t, r.sin_t, S, H, hd, c.max_seq, 0, 0, -1);
-        emit(s, DJ_OP_ATTENTION_KV, a.q, r.kv_all, r.kv_all, a.att, r.state, r.scratch, S, H, hd, c.max_seq, 0, 2 * d, d);
+        const int splits = S == 1 ? deepj_hip_latent_decode_splits(H, hd, kvr, c.max_seq) : 0;
+        if (splits) {        // one row: the cache stays latent (its scratch holds the splits' records)
+            emit(s, DJ_OP_LATENT_DECODE, a.qkv, a.ckv, r.latent, L.wukv, r.state, r.cos_t, r.sin_t, r.scratch, a.att, H, hd, kvr, c.max_seq, l);
+        } else {
+            emit(s, DJ_OP_APPEND_ROWS, a.ckv, r.latent, r.state, S, kvr, c.max_seq, lat_off);
+            emit(s, DJ_OP_Q8_LINEAR_DYN, r.latent, L.wukv, r.kv_all, c.max_seq, kvr, 2 * d, r.state, S, lat_off);
+            emit(s, DJ_OP_ROPE_ROWS, r.kv_all, r.kv_all, r.state, r.cos_t, r.sin_t, c.max_seq, H, hd, c.max_seq, 1, 2 * d, S);
+            emit(s, DJ_OP_ROPE_ROWS, a.qkv, a.q, r.state, r.cos_t, r.sin_t, S, H, hd, c.max_seq, 0, 0, -1);
+            emit(s, DJ_OP_ATTENTION_KV, a.q, r.kv_all, r.kv_all, a.att, r.state, r.scratch, S, H, hd, c.max_seq, 0, 2 * d, d);
+        }
         q8_linear(s, a.att, L.wo, a.x2, S, d, d, DJ_LIN_RESIDUAL, -1, -1, -1, a.x);
         wo_done = true;
     } else if (c.kind == 1) {

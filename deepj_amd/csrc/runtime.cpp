@@ -123,6 +123,7 @@ void ensure_init(int device = 0) {
     if (!g.static_scratch) fail("deepj_hip: the static scratch array has no device address");
     DJ_HIP(hipMemset(g.static_scratch, 0, kStaticCounterBytes));
     q8_gemm_f16_configure();
+    latent_decode_configure();
     g.device = device;
     g.ready = true;
 }
@@ -410,6 +411,7 @@ int stride_of(int op) {
         case DJ_OP_DECODE_ATTN: return 20;
         case DJ_OP_DECODE_FFN: return 16;
         case DJ_OP_DECODE_ROW: return 7;
+        case DJ_OP_LATENT_DECODE: return 15;
         default: return -1;
     }
 }
@@ -1000,6 +1002,25 @@ void exec_one(Cursor &c) {
             if (run) launch_decode_row(s, r);
             break;
         }
+        case DJ_OP_LATENT_DECODE: {
+            // [op, q, ckv, latent, wukv, state, cos, sin, records, out, H, hd, rank, maxSeq, layer]
+            const int64_t H = w[10], hd = w[11], rank = w[12], max_seq = w[13], layer = w[14];
+            const int splits = latent_decode_splits((int)H, (int)hd, (int)rank, (int)max_seq);
+            if (!splits || layer < 0) fail("OP_LATENT_DECODE: bad shape");
+            const int64_t d = H * hd, per_layer = max_seq * rank;
+            LatentDecode a{};
+            a.q = buf(w[1], d, op, "q");
+            a.ckv = buf(w[2], rank, op, "ckv");
+            a.latent = buf(w[3], (layer + 1) * per_layer, op, "latent") + layer * per_layer;
+            q8_weight(w[4], rank, 2 * d, op, "wukv", a.wq, a.scales);
+            a.state = reinterpret_cast<const int32_t *>(buf(w[5], 4, op, "state"));
+            a.cos_t = buf(w[6], max_seq * (hd / 2), op, "cos"); a.sin_t = buf(w[7], max_seq * (hd / 2), op, "sin");
+            a.records = buf(w[8], H * splits * (hd + 4), op, "records");
+            a.out = buf(w[9], d, op, "out");
+            a.heads = (int)H; a.hd = (int)hd; a.rank = (int)rank; a.max_seq = (int)max_seq;
+            if (run) launch_latent_decode(s, a);
+            break;
+        }
         case DJ_OP_APPEND_ROWS: {
             // [op, src, dst, state, rows, rowFloats, maxRows, dstOff]: dst[dstOff + (state[0]+i)*rowFloats ..] = src row i
             int64_t rows = w[4], rf = w[5], max_rows = w[6], off = w[7];
@@ -1139,6 +1160,7 @@ const char *op_name(int op) {
         case DJ_OP_DECODE_ATTN: return "OP_DECODE_ATTN";
         case DJ_OP_DECODE_FFN: return "OP_DECODE_FFN";
         case DJ_OP_DECODE_ROW: return "OP_DECODE_ROW";
+        case DJ_OP_LATENT_DECODE: return "OP_LATENT_DECODE";
         case DJ_OP_ATTN_DECODE: return "OP_ATTN_DECODE";
         case DJ_OP_APPEND_ROWS: return "OP_APPEND_ROWS";
         case DJ_OP_Q8_LINEAR_DYN: return "OP_Q8_LINEAR_DYN";
@@ -1360,6 +1382,7 @@ void *deepj_hip_stream(void) { return g.ready ? (void *)g.stream : nullptr; }
 
 int32_t deepj_hip_attn_record_splits(void) { return kAttnRecordSplits; }
 int32_t deepj_hip_decode_block_positions(int32_t d, int32_t hd, int32_t dff) { return decode_block_ok(d, hd, dff) ? decode_block_positions(hd) : 0; }
+int32_t deepj_hip_latent_decode_splits(int32_t H, int32_t hd, int32_t rank, int32_t max_seq) { return latent_decode_splits(H, hd, rank, max_seq); }
 int32_t deepj_hip_decode_ffn_parts(int32_t dff) { return dff > 0 ? decode_ffn_parts(dff) : 0; }
 
 int64_t deepj_hip_attention_scratch_floats(int32_t S, int32_t H, int32_t hd, int32_t max_seq) {

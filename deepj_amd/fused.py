@@ -145,6 +145,9 @@ class Stream:
     def decode_ffn(self, x, part, n_part, bias, out, gamma, beta, d, wgu, bg, bu, wd, part_out, dff, flags):
         return self.emit(op.OP_DECODE_FFN, x, part, n_part, bias, out, gamma, beta, d, wgu, bg, bu, wd, part_out, dff, flags)
 
+    def latent_decode(self, q, ckv, latent, wukv, state, cos, sin, records, out, H, hd, rank, max_seq, layer):
+        return self.emit(op.OP_LATENT_DECODE, q, ckv, latent, wukv, state, cos, sin, records, out, H, hd, rank, max_seq, layer)
+
     def decode_row(self, x, part, n_part, bias, out, d):
         return self.emit(op.OP_DECODE_ROW, x, part, n_part, bias, out, d)
 

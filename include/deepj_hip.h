@@ -229,6 +229,11 @@ enum {
      *     norm, up projection(s) with bg (and bu; flags DJ_LIN_SWIGLU or DJ_LIN_GELU as in Q8_LINEAR), down projection without
      *     its bias: partOut holds deepj_hip_decode_ffn_parts(dff) rows of d floats
      * DECODE_ROW    [op, x, part, nPart, bias, out, d]      out = r
+     * LATENT_DECODE [op, q, ckv, latent, wukv, state, cosT, sinT, records, out, H, hd, rank, maxSeq, layer]
+     *     one token's attention over latent rows (J/.../MultiHeadLatentAttention.java:98-123): ckv is appended to the layer's
+     *     rows of `latent` [layers][maxSeq][rank] at position state[0]; out [H * hd] = attention of q (not rotated) over
+     *     K = RoPE(rows . Wuk) and V = rows . Wuv, wukv a Q8 weight with the 2 * H * hd output rows Wuk, Wuv.  records: scratch
+     *     of H * deepj_hip_latent_decode_splits(H, hd, rank, maxSeq) * (hd + 4) floats; refused where that is 0.
      */
     DJ_OP_Q8_QUANTIZE = 64, DJ_OP_Q8_DEQUANTIZE = 65, DJ_OP_Q8_LINEAR = 66, DJ_OP_RMSNORM = 67,
     DJ_OP_SILU_MUL = 68, DJ_OP_EMBED_GATHER = 69, DJ_OP_ROPE_KV_STORE = 70, DJ_OP_ATTENTION = 71,
@@ -237,7 +242,7 @@ enum {
     DJ_OP_APPEND_ROWS = 80, DJ_OP_Q8_LINEAR_DYN = 81, /* 82 unused */ DJ_OP_LAYERNORM = 83,
     DJ_OP_ADD_POSITIONS = 84, DJ_OP_ATTN_DECODE_RECORDS = 85, DJ_OP_STREAM_READ = 86, DJ_OP_NOP = 87, DJ_OP_Q8_PREPARE = 88,
     DJ_OP_Q8_LINEAR_ROPE = 89, DJ_OP_DECODE_SAMPLE = 90,
-    DJ_OP_DECODE_ATTN = 91, DJ_OP_DECODE_FFN = 92, DJ_OP_DECODE_ROW = 93
+    DJ_OP_DECODE_ATTN = 91, DJ_OP_DECODE_FFN = 92, DJ_OP_DECODE_ROW = 93, DJ_OP_LATENT_DECODE = 94
 };
 
 /* Largest top_k that DECODE_SAMPLE takes. */
@@ -253,6 +258,10 @@ int32_t deepj_hip_attn_record_splits(void);
  * positions up to which they are the faster way through a block; rows of DECODE_FFN's partOut. */
 int32_t deepj_hip_decode_block_positions(int32_t d, int32_t hd, int32_t dff);
 int32_t deepj_hip_decode_ffn_parts(int32_t dff);
+
+/* Key splits per head of LATENT_DECODE; 0 where it does not take the shape (hd 32, 64 or 128; rank a multiple of 4 up to
+ * 512), and APPEND_ROWS, Q8_LINEAR_DYN, ROPE_ROWS and ATTENTION_KV are the way. */
+int32_t deepj_hip_latent_decode_splits(int32_t H, int32_t hd, int32_t rank, int32_t max_seq);
 
 /* Floats the scratch buffer of ATTENTION / ATTENTION_KV must hold for S query rows (0: none needed). */
 int64_t deepj_hip_attention_scratch_floats(int32_t S, int32_t H, int32_t hd, int32_t max_seq);

@@ -517,3 +517,50 @@ def test_a_narrow_block_in_two_launches_matches_the_layers(d, hd, dff, max_seq, 
         err = float(np.max(np.abs(a - b)))
         assert err <= 4e-5, (name, err)
     assert float(np.max(np.abs(keys - K))) <= 2e-5 and float(np.max(np.abs(values - V))) <= 2e-5
+
+
+@pytest.mark.parametrize("H,hd,rank,max_seq,pos", [
+    (1, 32, 4, 8, 0), (3, 32, 36, 70, 31), (2, 64, 96, 100, 32), (5, 64, 260, 300, 299), (16, 128, 512, 1024, 300),
+    (32, 64, 512, 1100, 1099), (2, 128, 512, 65, 64), (7, 32, 484, 40, 33), (4, 64, 512, 64, 63), (40, 32, 256, 500, 480), (300, 32, 8, 70, 66)])
+def test_decode_attention_over_latent_rows_matches_the_expanded_one(H, hd, rank, max_seq, pos):
+    """LATENT_DECODE against K = RoPE(rows . Wuk), V = rows . Wuv in float64: positions at the edges of a 32-row tile, splits
+    without keys, several tiles a split, latent rows that are no whole scale group, one head and more heads than compute units."""
+    rng = np.random.default_rng(H + rank + pos)
+    d, layers, layer = H * hd, 2, 1
+    q, ckv = (rng.standard_normal(n).astype(np.float32) for n in (d, rank))
+    rows = rng.standard_normal((layers, max_seq, rank)).astype(np.float32)
+    w = (rng.standard_normal((rank, 2 * d)) * rank ** -0.5).astype(np.float32)
+    cos, sin = ref.rope_tables(hd, max_seq)
+    dev = DeviceBuffers()
+    try:
+        src, wq = dev.upload(w), dev.alloc(HipNative.q8Floats(rank, 2 * d))
+        Stream().q8_quantize(src, wq, rank, 2 * d, 0, 1, 2 * d).run()
+        state = dev.upload(np.array([pos, 0, 0, 0], np.int32))
+        lat, out = dev.upload(rows), dev.alloc(d)
+        rec = dev.alloc(H * HipNative.latentDecodeSplits(H, hd, rank, max_seq) * (hd + 4))
+        s = Stream()
+        s.latent_decode(dev.upload(q), dev.upload(ckv), lat, wq, state, dev.upload(cos), dev.upload(sin), rec, out, H, hd, rank, max_seq, layer)
+        s.run()
+        got, cache = dev.download(out, (d,)), dev.download(lat, rows.shape)
+        s.run()
+        assert np.array_equal(got, dev.download(out, (d,)))
+    finally:
+        dev.release_all()
+    rows[layer, pos] = ckv
+    assert np.array_equal(cache, rows)
+    kv = rows[layer, :pos + 1].astype(np.float64) @ ref.q8_roundtrip(w).astype(np.float64)
+
+    def rotate(t, c, s):                                       # [.., H, hd] by [.., hd / 2]
+        c, s = c[..., None, :], s[..., None, :]
+        return np.stack([t[..., 0::2] * c - t[..., 1::2] * s, t[..., 0::2] * s + t[..., 1::2] * c], -1).reshape(t.shape)
+    k = rotate(kv[:, :d].reshape(-1, H, hd), cos[:pos + 1], sin[:pos + 1])
+    p = np.einsum("hd,khd->hk", rotate(q.astype(np.float64).reshape(H, hd), cos[pos], sin[pos]), k) / np.sqrt(hd)
+    p = np.exp(p - p.max(1, keepdims=True))
+    exp = np.einsum("hk,khd->hd", p / p.sum(1, keepdims=True), kv[:, d:].reshape(-1, H, hd)).reshape(d)
+    # sums of at most 512 products of order 1 / sqrt(512) and of at most 1100 keys, in chains of under 100 roundings of 2^-24
+    assert float(np.max(np.abs(got - exp))) <= 1e-5 * max(1.0, float(np.max(np.abs(exp))))
+
+
+def test_latent_decode_refuses_what_it_does_not_take():
+    for shape in ((4, 48, 64, 64), (4, 64, 6, 64), (4, 64, 516, 64), (0, 64, 64, 64), (4, 64, 64, 0)):
+        assert HipNative.latentDecodeSplits(*shape) == 0
