@@ -194,43 +194,34 @@ template <int NC, int B, bool SWIGLU, bool GELU, bool DIGITS>
 __device__ __forceinline__ void finish_batch(const RowBatch<NC, B *(SWIGLU ? 2 : 1)> &b, const XSlice<NC, DIGITS> &xr,
                                              const MatvecArgs &p, int o0, int o_end, int lane, float rms) {
     constexpr int R = B * (SWIGLU ? 2 : 1);
-    float acc[R];
+    float acc[R];                                   // the same in every lane
 #pragma unroll
     for (int u = 0; u < R; u++) {
         float a = 0.0f;
 #pragma unroll
         for (int c = 0; c < NC; c++) a = fmaf(dot_slice<NC>(b.w[u][c], xr, c), b.sc[u][c], a);
-        acc[u] = wave_sum_dpp(a) / rms;        // rms = 1 unless the RMSNorm scale was deferred to here
+        acc[u] = wave_sum_dpp(a);
     }
-    float eb[B], eb2[B], er[B];
+    // Lane u finishes output o0 + u: one division, activation and store for the batch, where one after the other on lane 0
+    // is their code (which every launch fetches anew) B times over.  rms = 1 unless the RMSNorm scale was deferred to here.
+    float v = acc[0], up = SWIGLU ? acc[1] : 0.0f;
 #pragma unroll
-    for (int u = 0; u < B; u++) {
-        eb[u] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, b.ev), u));
-        eb2[u] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, b.ev), B + u));
-        er[u] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, b.ev), 2 * B + u));
+    for (int u = 1; u < B; u++) {
+        v = lane == u ? acc[SWIGLU ? 2 * u : u] : v;
+        if constexpr (SWIGLU) up = lane == u ? acc[2 * u + 1] : up;
     }
-    if (lane == 0) {
-#pragma unroll
-        for (int u = 0; u < B; u++) {
-            int o = o0 + u;
-            if (o < o_end) {
-                float v;
-                if constexpr (SWIGLU) {
-                    float gate = acc[2 * u], up = acc[2 * u + 1];
-                    if (p.bias) gate = gate + eb[u];
-                    if (p.bias2) up = up + eb2[u];
-                    float sg = gate * d_sigmoid(gate);     // SiLU.java:20-24
-                    v = sg * up;                            // SwiGLULayer.java:69
-                } else {
-                    v = acc[u];
-                    if (p.bias) v = v + eb[u];
-                    if constexpr (GELU) v = gemm_gelu(v);
-                }
-                if (p.residual) v = er[u] + v;
-                p.out[o] = v;
-            }
-        }
+    v = v / rms;
+    if (p.bias) v = v + b.ev;
+    if constexpr (SWIGLU) {
+        up = up / rms;
+        if (p.bias2) up = up + __shfl(b.ev, lane + B, 64);
+        const float sg = v * d_sigmoid(v);          // SiLU.java:20-24
+        v = sg * up;                                // SwiGLULayer.java:69
+    } else {
+        if constexpr (GELU) v = gemm_gelu(v);
     }
+    if (p.residual) v = __shfl(b.ev, lane + 2 * B, 64) + v;
+    if (lane < B && o0 + lane < o_end) p.out[o0 + lane] = v;
 }
 
 // LDS layout of the staged activation row, float form (rows whose length is not a multiple of 4).  A lane multiplies
@@ -539,13 +530,16 @@ k_q8_matvec(const float *a_x, const int8_t *a_wq, const float *a_scales, float *
     }
 
     DJ_STAMP(3);
-    for (int o0 = o_begin; o0 < o_end; o0 += 2 * o_step) {
-        if (o0 + o_step < o_end) { load_batch<NC, R>(bb, p, (o0 + o_step) * RPO, row_last, lane, groups); load_epilogue<NC, R, B, SWIGLU>(bb, p, o0 + o_step); }
+    // One copy of the loop's code, its registers moved along: a launch fetches its code anew, at some 16 bytes a ns, and two
+    // buffers used in turn are two copies of the batch's loads and products.
+#pragma unroll 1
+    for (int o0 = o_begin;; o0 += o_step) {
+        const bool more = o0 + o_step < o_end;      // wave-uniform
+        if (more) { load_batch<NC, R>(bb, p, (o0 + o_step) * RPO, row_last, lane, groups); load_epilogue<NC, R, B, SWIGLU>(bb, p, o0 + o_step); }
         finish_batch<NC, B, SWIGLU, GELU, VEC>(ba, xr, p, o0, o_end, lane, rms);
         if (o0 == o_begin) DJ_STAMP(4);
-        if (o0 + o_step >= o_end) break;
-        if (o0 + 2 * o_step < o_end) { load_batch<NC, R>(ba, p, (o0 + 2 * o_step) * RPO, row_last, lane, groups); load_epilogue<NC, R, B, SWIGLU>(ba, p, o0 + 2 * o_step); }
-        finish_batch<NC, B, SWIGLU, GELU, VEC>(bb, xr, p, o0 + o_step, o_end, lane, rms);
+        if (!more) break;
+        ba = bb;
     }
     DJ_STAMP(5);
 }
