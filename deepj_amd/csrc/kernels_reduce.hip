@@ -429,10 +429,13 @@ __global__ void __launch_bounds__(1024) k_decode_next(const float *__restrict__ 
 // by lowest index (stable descending sort); soft-max of value / temperature with a float64 exp and fp32 sums in that
 // order; one draw of java.util.Random; the first candidate whose cumulative sum reaches it; then record, advance and
 // gather as k_decode_next does.
-// Selection: the topK-th largest of the 1024 threads' own maxima bounds the topK-th largest logit from below, so one more
-// pass collects a few more than topK candidates, which are sorted in LDS.  Logits so full of ties that more than kPool
-// candidates pass are cut exactly by a search over the key's bits first.  Bound by the latency of two passes of one
-// workgroup over the logits; the host's sort it replaces took 3.3 ms for 50257 logits.
+// Selection: at least topK of the 1024 threads' own maxima lie at or above the least, over the 16 wavefronts, of a wavefront's
+// ceil(topK / 16)-th largest one, so that bounds the topK-th largest logit from below; one more pass collects the
+// candidates (some three times topK), whose places in the order are counted or, when they are many, sorted in LDS.  Logits so
+// full of ties that more than kPool candidates pass are cut exactly by a search over the key's bits first.  Bound by the
+// latency of two passes of one workgroup over the logits (the host's sort took 3.3 ms for 50257 of them) and by its serial
+// steps: with the 1024 maxima sorted through 55 barriers, every candidate sorted, and a branch per logit in the second pass
+// it took 28 us for 50257 logits, now 14.
 constexpr int kPool = 2048;
 
 // Float.compare's order as unsigned integers: -0 below +0, NaN above everything.
@@ -458,23 +461,60 @@ template <class T> __device__ __forceinline__ void sort_descending(T *v, int n) 
     __syncthreads();
 }
 
-template <class F> __device__ __forceinline__ void each_logit(const float *logits, int vocab, F &&f) {
+// f(key, index) for every logit whose key may be `bound` or more (for all of them where bound is 0).  floor_of(bound) is
+// a float below no such logit, so a word of four is passed over with four compares.
+__device__ __forceinline__ float floor_of(uint32_t bound) {
+    return __builtin_bit_cast(float, (bound & 0x80000000u) ? bound ^ 0x80000000u : ~bound);
+}
+template <class F> __device__ __forceinline__ void each_logit(const float *logits, int vocab, uint32_t bound, F &&f) {
     const int v4 = vocab >> 2;
     const float4 *l4 = reinterpret_cast<const float4 *>(logits);
+    const float low = floor_of(bound);                   // (a NaN for a bound of 0 or a NaN's: every compare lets it pass)
     for (int base = 0; base < v4; base += 1024 * 8) {
         float4 t[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const int i = base + u * 1024 + threadIdx.x;
-            if (i < v4) t[u] = l4[i];
+            t[u] = l4[i < v4 ? i : 0];
         }
+        uint32_t pass = 0;
 #pragma unroll
         for (int u = 0; u < 8; u++) {
-            const int i = base + u * 1024 + threadIdx.x;
-            if (i < v4) { f(order_key(t[u].x), 4 * i); f(order_key(t[u].y), 4 * i + 1); f(order_key(t[u].z), 4 * i + 2); f(order_key(t[u].w), 4 * i + 3); }
+            const bool any = !(t[u].x < low) | !(t[u].y < low) | !(t[u].z < low) | !(t[u].w < low);
+            pass |= any && base + u * 1024 + (int)threadIdx.x < v4 ? 1u << u : 0u;
+        }
+        while (pass) {                                   // the few words left are read again
+            const int i = base + __builtin_ctz(pass) * 1024 + threadIdx.x;
+            pass &= pass - 1;
+            const float4 w = l4[i];
+            const float v[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) f(order_key(v[j]), 4 * i + j);
         }
     }
     for (int c = (v4 << 2) + threadIdx.x; c < vocab; c += 1024) f(order_key(logits[c]), c);
+}
+
+// The largest key of this thread's logits: words of four, or single ones where words would leave threads without any.
+__device__ __forceinline__ uint32_t most_of(const float *logits, int vocab) {
+    const int v4 = vocab < 8192 ? 0 : vocab >> 2;
+    const float4 *l4 = reinterpret_cast<const float4 *>(logits);
+    uint32_t m = 0;
+    for (int base = 0; base < v4; base += 1024 * 8) {
+        float4 t[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int i = base + u * 1024 + threadIdx.x;
+            t[u] = l4[i < v4 ? i : 0];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const uint32_t k = max(max(order_key(t[u].x), order_key(t[u].y)), max(order_key(t[u].z), order_key(t[u].w)));
+            if (base + u * 1024 + (int)threadIdx.x < v4) m = max(m, k);
+        }
+    }
+    for (int c = (v4 << 2) + threadIdx.x; c < vocab; c += 1024) m = max(m, order_key(logits[c]));
+    return m;
 }
 
 __global__ void __launch_bounds__(1024) k_decode_sample(const float *__restrict__ logits, int32_t *__restrict__ state,
@@ -482,7 +522,7 @@ __global__ void __launch_bounds__(1024) k_decode_sample(const float *__restrict_
                                                         const float *__restrict__ table, float *__restrict__ x, int vocab,
                                                         int d, int n_positions, uint32_t *__restrict__ params) {
     __shared__ uint64_t pool[kPool];                     // (key, ~index): larger = earlier in the stable descending order
-    __shared__ uint32_t most[1024];
+    __shared__ uint32_t most[16];
     __shared__ float probs[kSampleTopK];
     __shared__ int s_count, s_tok;
     const int t = threadIdx.x;
@@ -493,27 +533,35 @@ __global__ void __launch_bounds__(1024) k_decode_sample(const float *__restrict_
 
     uint32_t bound = 0;                                  // candidates: key >= bound
     if (vocab > kPool) {
-        uint32_t m = 0;
-        each_logit(logits, vocab, [&](uint32_t key, int) { m = key > m ? key : m; });
-        most[t] = m;
-        sort_descending(most, 1024);
-        bound = most[k - 1];
+        const uint32_t m = most_of(logits, vocab);
+        const int q = (k + 15) / 16;                     // 1 .. 32 of a wavefront's 64
+        uint32_t kth = 0;                                // its q-th largest maximum, bit by bit
+#pragma unroll 1
+        for (int bit = 31; bit >= 0; bit--) {
+            const uint32_t c = kth | (1u << bit);
+            if (__popcll(__ballot(m >= c)) >= q) kth = c;
+        }
+        if ((t & 63) == 0) most[t >> 6] = kth;
+        __syncthreads();
+        bound = most[0];
+#pragma unroll
+        for (int w = 1; w < 16; w++) bound = min(bound, most[w]);
     }
     auto count_if = [&](auto &&pred) {                   // how many logits satisfy pred(key, index); every thread gets it
         if (t == 0) s_count = 0;
         __syncthreads();
         int c = 0;
-        each_logit(logits, vocab, [&](uint32_t key, int i) { c += pred(key, i) ? 1 : 0; });
+        each_logit(logits, vocab, 0, [&](uint32_t key, int i) { c += pred(key, i) ? 1 : 0; });
         atomicAdd(&s_count, c);
         __syncthreads();
         const int r = s_count;
         __syncthreads();
         return r;
     };
-    auto collect = [&](auto &&pred) {
+    auto collect = [&](uint32_t from, auto &&pred) {
         if (t == 0) s_count = 0;
         __syncthreads();
-        each_logit(logits, vocab, [&](uint32_t key, int i) {
+        each_logit(logits, vocab, from, [&](uint32_t key, int i) {
             if (!pred(key, i)) return;
             const int at = atomicAdd(&s_count, 1);
             if (at < kPool) pool[at] = ((uint64_t)key << 32) | (uint32_t)~i;
@@ -523,7 +571,7 @@ __global__ void __launch_bounds__(1024) k_decode_sample(const float *__restrict_
         __syncthreads();
         return r;
     };
-    int n = collect([&](uint32_t key, int) { return key >= bound; });
+    int n = collect(bound, [&](uint32_t key, int) { return key >= bound; });
     if (n > kPool) {
         uint32_t kth = 0;                                // the k-th largest key ...
         for (int bit = 31; bit >= 0; bit--) {
@@ -537,12 +585,25 @@ __global__ void __launch_bounds__(1024) k_decode_sample(const float *__restrict_
             if (count_if([&](uint32_t key, int i) { return key == kth && i <= mid; }) >= ties) hi = mid;
             else lo = mid + 1;
         }
-        n = collect([&](uint32_t key, int i) { return key > kth || (key == kth && i <= lo); });
+        n = collect(kth, [&](uint32_t key, int i) { return key > kth || (key == kth && i <= lo); });
     }
-    int size = 2;
-    while (size < n) size <<= 1;
-    for (int i = n + t; i < size; i += 1024) pool[i] = 0;
-    sort_descending(pool, size);
+    if (n <= 256) {
+        // few: a candidate's place is how many lie above it (no two are equal), counted by four threads each
+        const int i = t >> 2, part = t & 3;
+        const uint64_t mine = i < n ? pool[i] : 0;
+        int above = 0;
+        for (int j = part; j < n; j += 4) above += pool[j] > mine ? 1 : 0;
+        above += __shfl_xor(above, 1, 64);
+        above += __shfl_xor(above, 2, 64);
+        __syncthreads();
+        if (i < n && part == 0) pool[above] = mine;
+        __syncthreads();
+    } else {
+        int size = 512;
+        while (size < n) size <<= 1;
+        for (int i = n + t; i < size; i += 1024) pool[i] = 0;
+        sort_descending(pool, size);
+    }
 
     auto index_of = [&](int i) { return (int)~(uint32_t)pool[i]; };
     float v = t < k ? logits[index_of(t)] / temperature : -INFINITY;

@@ -412,7 +412,7 @@ def test_short_and_chunked_prompts_on_prepared_weights_against_the_oracle():
 
 
 @pytest.mark.parametrize("vocab,kind", [(1, "normal"), (3, "normal"), (513, "normal"), (2048, "normal"), (2049, "ties"), (5000, "equal"),
-                                        (4097, "nan"), (50257, "normal"), (50257, "ties")])
+                                        (4097, "nan"), (8191, "normal"), (8194, "rising"), (50257, "normal"), (50257, "ties")])
 @pytest.mark.parametrize("top_k,temperature", [(2, 1.0), (40, 0.7), (512, 1.6)])
 def test_sampling_on_the_device_draws_what_the_oracle_draws(vocab, kind, top_k, temperature):
     """DECODE_SAMPLE at the sizes where its selection changes: fewer logits than candidates, one more than its pool, a pool
@@ -424,6 +424,8 @@ def test_sampling_on_the_device_draws_what_the_oracle_draws(vocab, kind, top_k, 
         logits = np.round(logits)
     if kind == "equal":
         logits[:] = np.float32(-0.25)
+    if kind == "rising":                  # all of the largest in one wavefront's words
+        logits.sort()
     if kind == "nan":
         logits[[5, vocab // 2]] = np.nan
         logits[7] = -np.inf
