@@ -366,7 +366,6 @@ __global__ void __launch_bounds__(1024) k_decode_next(const float *__restrict__ 
                                                       int vocab, int d, int n_positions) {
     __shared__ float sv[16];
     __shared__ int si[16];
-    __shared__ int s_tok;
     float bv = -INFINITY;
     int bi = 0x7fffffff;
     // the counters the last phase updates: requested now, used after the reduction
@@ -406,18 +405,22 @@ __global__ void __launch_bounds__(1024) k_decode_next(const float *__restrict__ 
     int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0) { sv[wave] = bv; si[wave] = bi; }
     __syncthreads();
+    // every wavefront picks among the sixteen for itself: nobody waits for one thread's walk over them
+    bv = sv[lane & 15]; bi = si[lane & 15];
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) {
+        float ov = __shfl_xor(bv, off, 64);
+        int oi = __shfl_xor(bi, off, 64);
+        if (better(ov, oi, bv, bi)) { bv = ov; bi = oi; }
+    }
+    const int tok = bi;
     if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; w++)
-            if (better(sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
         const int g = st_gen;
-        if (g < capacity) tokens[g] = bi;
-        state[1] = bi;
+        if (g < capacity) tokens[g] = tok;
+        state[1] = tok;
         state[0] = st_pos + n_positions;
         state[2] = g + 1;
-        s_tok = bi;
     }
-    __syncthreads();
-    int tok = s_tok;
     bool ok = tok >= 0 && tok < vocab;
     const float *src = table + (int64_t)(ok ? tok : 0) * d;
     for (int c = threadIdx.x; c < d; c += 1024) x[c] = ok ? src[c] : __builtin_nanf("");
