@@ -81,30 +81,7 @@ __global__ void __launch_bounds__(kThreads) k_latent_decode(const float *__restr
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), half = lane >> 5, l32 = lane & 31;
     const int h = blockIdx.x, split_i = blockIdx.y, splits = gridDim.y;
     float *rec = records + ((int64_t)h * splits + split_i) * (HD + 4);
-    int pos = state[0];
-    pos = pos < 0 ? 0 : (pos >= max_seq ? max_seq - 1 : pos);
-    const int tiles = pos / kTile + 1;
-    if (split_i >= tiles) {                                     // no keys for this split
-        if (t == 0) { rec[0] = -INFINITY; rec[1] = 0.0f; }
-        return;
-    }
     const int groups = (rank + kQ8Group - 1) / kQ8Group, kp = groups * kQ8Group;
-
-    // the tile rows this thread stages: row t / 16, float4s (t % 16) + 16 m; the new token's row is not in the cache yet
-    const int s_row = t >> 4, s_at = (t & 15) * 4;
-    FloatV<4 * NM> c;
-    auto load_rows = [&](int tile) {
-        const int key = tile * kTile + s_row;
-        int at0 = s_at;
-        asm volatile("" : "+v"(at0));                           // offsets are worked out anew: kept over the tiles they cost registers that are not there
-        const float *src = key >= pos ? ckv : latent + (int64_t)key * rank;
-#pragma unroll
-        for (int m = 0; m < NM; m++) {
-            const float4 v = *reinterpret_cast<const float4 *>(src + (at0 + 64 * m < rank ? at0 + 64 * m : 0));
-            c[4 * m] = v.x; c[4 * m + 1] = v.y; c[4 * m + 2] = v.z; c[4 * m + 3] = v.w;
-        }
-    };
-    load_rows(split_i);
 
     const int ct = wave % NT, kset = wave / NT;
     const int g0 = kset * NG;                                             // this set's first group
@@ -137,6 +114,30 @@ __global__ void __launch_bounds__(kThreads) k_latent_decode(const float *__restr
         }
     };
     load_weights((uint32_t)(h * HD + col), wk, sk);
+    // (the weights are on their way while the position is waited for)
+    int pos = state[0];
+    pos = pos < 0 ? 0 : (pos >= max_seq ? max_seq - 1 : pos);
+    const int tiles = pos / kTile + 1;
+    if (split_i >= tiles) {                                     // no keys for this split
+        if (t == 0) { rec[0] = -INFINITY; rec[1] = 0.0f; }
+        return;
+    }
+    // the tile rows this thread stages: row t / 16, float4s (t % 16) + 16 m; the new token's row is not in the cache yet
+    const int s_row = t >> 4, s_at = (t & 15) * 4;
+    FloatV<4 * NM> c;
+    auto load_rows = [&](int tile) {
+        const int key = tile * kTile + s_row;
+        int at0 = s_at;
+        asm volatile("" : "+v"(at0));                           // offsets are worked out anew: kept over the tiles they cost registers that are not there
+        const float *src = key >= pos ? ckv : latent + (int64_t)key * rank;
+#pragma unroll
+        for (int m = 0; m < NM; m++) {
+            const float4 v = *reinterpret_cast<const float4 *>(src + (at0 + 64 * m < rank ? at0 + 64 * m : 0));
+            c[4 * m] = v.x; c[4 * m + 1] = v.y; c[4 * m + 2] = v.z; c[4 * m + 3] = v.w;
+        }
+    };
+    load_rows(split_i);
+
     // Wuv's rows are multiplied last; beside Wuk's they do not fit the registers, so for now a word of each of their lines
     // is asked for, which brings the lines to this chiplet's L2
     const int v_line = t * 128 < HD * kp ? t * 128 : 0;
