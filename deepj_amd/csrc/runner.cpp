@@ -659,8 +659,9 @@ void replay(Runner &r, Choose how, bool narrow, int size, int times) {
     hip(deepj_hip_graph_launch(graph, times));
 }
 
-// The launches of a token, roughly: blocks of 2 or 5, the row behind the narrow ones, the head and the choice.
-int token_launches(const Config &c, bool narrow) { return narrow ? 2 * c.layers + 3 : 5 * c.layers + 2; }
+// The launches of a token, roughly: blocks of 2 or 5 (8 over a latent cache), the row behind the narrow ones, the head and
+// the choice.
+int token_launches(const Config &c, bool narrow) { return narrow ? 2 * c.layers + 3 : (c.latent ? 8 : 5) * c.layers + 2; }
 
 void decode_steps(Runner &r, int steps, int mode, Choose how, bool narrow) {
     if (mode != 1) {
