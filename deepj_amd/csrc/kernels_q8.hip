@@ -616,7 +616,12 @@ void dispatch_mv(hipStream_t s, const MatvecArgs &a, bool swiglu, bool gelu) {
     }
     constexpr int BMAX = NC == 1 ? 8 : (NC == 2 ? 4 : (NC <= 4 ? 2 : 1));
     int rows = swiglu ? 2 * a.n_out : a.n_out;
-    int want = (rows + mv_target_waves() - 1) / mv_target_waves();      // rows per wavefront per step
+    // Short rows (one chunk): half as many wavefronts.  Staging the activations, normalised, is what a workgroup spends most
+    // of its time on there, and a second row per wavefront costs less than a second workgroup that stages them again (768 ->
+    // 3072 with LayerNorm and GELU 4.0 -> 3.8 us, a token of the 12-layer GPT 232 -> 226).  Rows of two chunks lose by it
+    // (2048 -> 6144: 64 tokens of the 16-layer model 29.2 -> 29.4 ms).
+    const int target = NC == 1 ? mv_target_waves() / 2 : mv_target_waves();
+    int want = (rows + target - 1) / target;                            // rows per wavefront per step
     if (swiglu) {
         constexpr int BS = BMAX >= 2 ? BMAX / 2 : 1;
         if (BS >= 4 && want >= 8) launch_mv<NC, (BS >= 4 ? 4 : 1), true>(s, a);
