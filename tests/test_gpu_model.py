@@ -234,6 +234,23 @@ def test_deepseek_latent_cache_decode_row_equals_prefill_row(ds_latent):
     assert float(np.max(np.abs(gpu.lastLogits() - full[29]))) <= 2e-4
 
 
+@pytest.mark.parametrize("kv_rank", [22, 36, 520])
+def test_latent_rows_of_any_width_decode_to_the_prompt_rows(kv_rank):
+    """Widths LATENT_DECODE takes (36) and widths that go through the expanded cache (no multiple of 4, more than 512)."""
+    gpu = DeepSeekModel(DeepSeekConfig(vocabSize=256, maxSeqLen=96, dModel=128, nHeads=2, nLayers=2, dFF=176, qRank=64, kvRank=kv_rank), 42,
+                        latent_cache=True)
+    try:
+        ids = ref.JavaRandom(12).ints(40, 256)
+        full = gpu.forward(ids)
+        gpu.reset()
+        gpu.prefill(ids[:30], choose_next=False)
+        for t in range(30, 40):
+            gpu.step(int(ids[t]))
+            assert float(np.max(np.abs(gpu.lastLogits() - full[t]))) <= 2e-4, t
+    finally:
+        gpu.close()
+
+
 def test_latent_cache_is_a_deepseek_option_only():
     with pytest.raises(ValueError, match="latent KV cache belongs to the DeepSeek"):
         _DecoderOnlyModel(C1, None, 0, True)
