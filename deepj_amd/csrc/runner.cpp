@@ -96,8 +96,6 @@ struct Runner {
     bool finalized = false;
     int32_t pos = 0;          // host mirror of state[0]
     int32_t generated = 0;    // host mirror of state[2]
-    bool state_stale = false; // state[0] on the device is behind `pos` (a step was taken); see settle_state
-    int32_t stepped = 0;      // the token of that step
     std::string error;
 
     int hd() const { return cfg.d / cfg.heads; }
@@ -575,12 +573,6 @@ Stream prompt_stream(Runner &r, int n, Choose how) {
 void upload_state(Runner &r, int32_t token) {
     const int32_t st[4] = {r.pos, token, r.generated, 0};
     hip(deepj_hip_upload(r.state, reinterpret_cast<const float *>(st), 4));
-    r.state_stale = false;
-}
-// A caller-chosen step leaves the device's position one behind (the next one uploads its own); whatever else reads the
-// state brings it up to date first.
-void settle_state(Runner &r) {
-    if (r.state_stale) upload_state(r, r.stepped);
 }
 
 // Runs the prompt rows through the model, filling the cache.  Leaves the last row's
@@ -592,7 +584,6 @@ void prefill(Runner &r, const int32_t *ids, int n, float *all_logits, Choose how
     check_ids(c, ids, n);
     if (r.pos + n > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + n) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
-    settle_state(r);
     Stream s = prompt_stream(r, n, how);
     hip(deepj_hip_upload(r.pre.ids, reinterpret_cast<const float *>(ids), n));   // (prompt_stream sized r.pre for n rows)
     r.run(s);
@@ -682,7 +673,6 @@ void decode(Runner &r, int steps, int mode, Choose how) {
     if (steps <= 0) return;
     if (r.pos + steps > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + steps) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
-    settle_state(r);
     const int narrow = std::min(steps, std::max(0, r.narrow_positions() - r.pos));
     if (narrow) decode_steps(r, narrow, mode, how, true);
     if (steps > narrow) decode_steps(r, steps - narrow, mode, how, false);
@@ -704,9 +694,8 @@ void step_token(Runner &r, int32_t token, int mode) {
     const bool narrow = r.pos < r.narrow_positions();
     if (mode == 1) replay(r, kNone, narrow, 2, 1);
     else r.run(decode_stream(r, kNone, narrow));
-    r.stepped = token;
     r.pos += 1;
-    r.state_stale = true;
+    upload_state(r, token);             // the next launch takes it along, or the next step's overwrites it where it is staged
 }
 
 // ── TextGenerator.sampleFromLogits on the host (temperature / top-k > 1) ────

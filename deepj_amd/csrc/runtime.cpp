@@ -134,7 +134,8 @@ void ensure_init(int device = 0) {
 // waits for the stream except a full ring and a download for its own chunks.  Measured for one tensor operation on a
 // 64 x 32 matrix (two uploads, a product, a download): 57 us with a synchronisation per upload and copy calls.
 
-// Launches what is staged.  Every path that enqueues work or hands a block to another buffer calls it first.
+// Launches what is staged.  Every path that enqueues work or hands a block to another buffer calls it first; a download
+// only where it would read what is staged.
 void launch_uploads() {
     if (!g.n_pieces) return;
     const int n = g.n_pieces;
@@ -142,6 +143,12 @@ void launch_uploads() {
     launch_upload_pieces(g.stream, g.pieces, n);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) fail(std::string("upload failed: ") + hipGetErrorString(e));
+}
+
+bool staged_for(const float *p, int64_t n) {
+    for (int i = 0; i < g.n_pieces; i++)
+        if (g.pieces.p[i].dst < p + n && p < g.pieces.p[i].dst + g.pieces.p[i].n) return true;
+    return false;
 }
 
 // `bytes` (at most a segment) of the ring; waits for the device only where the ring comes round to a segment in use.
@@ -163,8 +170,14 @@ unsigned char *ring_take(size_t bytes) {
 void stage_upload(float *dst, const float *src, int64_t n) {
     // pieces of a quarter segment: the first is on the link while the next is copied
     constexpr int64_t kPiece = (int64_t)(kRingSegmentBytes / 4 / 4);
-    for (int i = 0; i < g.n_pieces; i++)                      // pieces of one launch run side by side: no two into the same words
-        if (g.pieces.p[i].dst < dst + n && dst < g.pieces.p[i].dst + g.pieces.p[i].n) { launch_uploads(); break; }
+    for (int i = 0; i < g.n_pieces; i++) {
+        const UploadPiece &p = g.pieces.p[i];
+        if (p.dst == dst && p.n == n) {                       // the same words again before anything read them: the later values stand
+            std::memcpy(const_cast<float *>(p.src), src, (size_t)n * 4);
+            return;
+        }
+    }
+    if (staged_for(dst, n)) launch_uploads();                 // pieces of one launch run side by side: no two into the same words
     for (int64_t at = 0; at < n; at += kPiece) {
         const int64_t len = std::min(kPiece, n - at);
         unsigned char *p = ring_take((size_t)len * 4);
@@ -1240,8 +1253,9 @@ int deepj_hip_download(int32_t id, float *dst, int64_t n) {
             fail("downloadBuffer: " + std::to_string(n) + " floats exceed buffer id=" + std::to_string(id) + " of " +
                  std::to_string(it->second.floats));
         if (n > 0 && !dst) fail("downloadBuffer: null destination");
-        launch_uploads();
-        if (n > 0) download(static_cast<const float *>(it->second.ptr), dst, n);
+        const float *src = static_cast<const float *>(it->second.ptr);
+        if (n == 0 || staged_for(src, n)) launch_uploads();      // (others can wait for the next flush)
+        if (n > 0) download(src, dst, n);
         else DJ_HIP(hipStreamSynchronize(g.stream));
     });
 }

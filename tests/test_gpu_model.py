@@ -234,6 +234,23 @@ def test_deepseek_latent_cache_decode_row_equals_prefill_row(ds_latent):
     assert float(np.max(np.abs(gpu.lastLogits() - full[29]))) <= 2e-4
 
 
+@pytest.mark.parametrize("fetched", ["before the step", "after the step"])
+def test_a_stream_run_after_a_step_works_at_the_position_behind_it(c1, fetched):
+    """The device's own position is current after step(): a prompt stream of the caller's appends behind the stepped token."""
+    gpu, _ = c1
+    ids = ref.JavaRandom(21).ints(9, 256)
+    full = gpu.forward(np.concatenate([ids, ids[:5]]))
+    gpu.reset()
+    gpu.prefill(ids[:8], choose_next=False)
+    stream = gpu.prefillStream(5)                  # over the ids of the last prefill: ids[:5]
+    gpu.step(int(ids[8]))
+    if fetched == "after the step":
+        stream = gpu.prefillStream(5)
+    HipNative.nativeFlushOps(stream, len(stream))
+    assert float(np.max(np.abs(gpu.lastLogits() - full[13]))) <= 2e-4
+    gpu.reset()
+
+
 @pytest.mark.parametrize("kv_rank", [22, 36, 520])
 def test_latent_rows_of_any_width_decode_to_the_prompt_rows(kv_rank):
     """Widths LATENT_DECODE takes (36) and widths that go through the expanded cache (no multiple of 4, more than 512)."""
