@@ -497,7 +497,7 @@ k_decode_ffn(const float *x, const float *part, const int8_t *wgu, const float *
     }
 }
 
-// out = x + (sum of the partial rows + bias): the row behind the last block
+// out = x + (sum of the partial rows + bias), x where there are none: the row behind the last block
 __global__ void __launch_bounds__(256) k_decode_row(const float *__restrict__ x, const float *__restrict__ part, int n_part,
                                                     const float *__restrict__ bias, float *__restrict__ out, int d) {
     __shared__ float red[16][16];
@@ -510,7 +510,7 @@ __global__ void __launch_bounds__(256) k_decode_row(const float *__restrict__ x,
     __syncthreads();
     if (threadIdx.x < 16 && col < d) {
         for (int q = 1; q < 16; q++) s += red[q][c];
-        out[col] = x[col] + (s + (bias ? bias[col] : 0.0f));
+        out[col] = n_part > 0 ? x[col] + (s + (bias ? bias[col] : 0.0f)) : x[col];
     }
 }
 

@@ -555,6 +555,27 @@ def test_a_narrow_block_in_two_launches_matches_the_layers(d, hd, dff, max_seq, 
     assert float(np.max(np.abs(keys - K))) <= 2e-5 and float(np.max(np.abs(values - V))) <= 2e-5
 
 
+@pytest.mark.parametrize("d,parts", [(33, 0), (16, 1), (33, 17), (256, 48)])
+def test_decode_row_adds_its_parts_and_their_bias(d, parts):
+    """DECODE_ROW at widths that do not fill its columns and part counts around its sixteen sets; without parts it is x, bit
+    for bit, whatever the bias.  Bound: parts + 2 roundings of the sum's terms."""
+    rng = np.random.default_rng(d + parts)
+    x, bias, part = (rng.standard_normal(n).astype(np.float32) for n in (d, d, max(parts, 1) * d))
+    x[0] = -0.0
+    dev = DeviceBuffers()
+    try:
+        out = dev.alloc(d)
+        Stream().decode_row(dev.upload(x), dev.upload(part), parts, dev.upload(bias), out, d).run()
+        got = dev.download(out, (d,))
+    finally:
+        dev.release_all()
+    if not parts:
+        assert np.array_equal(got.view(np.uint32), x.view(np.uint32))
+        return
+    terms = np.concatenate([x[None], bias[None], part.reshape(parts, d)]).astype(np.float64)
+    assert np.all(np.abs(got - terms.sum(0)) <= (parts + 2) * 2.0 ** -24 * np.abs(terms).sum(0))
+
+
 @pytest.mark.parametrize("H,hd,rank,max_seq,pos", [
     (1, 32, 4, 8, 0), (3, 32, 36, 70, 31), (2, 64, 96, 100, 32), (5, 64, 260, 300, 299), (16, 128, 512, 1024, 300),
     (32, 64, 512, 1100, 1099), (2, 128, 512, 65, 64), (7, 32, 484, 40, 33), (4, 64, 512, 64, 63), (40, 32, 256, 500, 480), (300, 32, 8, 70, 66)])
