@@ -1388,8 +1388,13 @@ void *deepj_hip_host_alloc(int64_t bytes) {
     return p;
 }
 
+// Leaves the thread's last error alone: finalisers call it between a failed call and the reading of its message.
 void deepj_hip_host_free(void *p) {
-    if (p) guarded([&] { host_give_back(p); });
+    if (!p) return;
+    try {
+        host_give_back(p);
+    } catch (...) {            // (no memory for the list of free blocks: the block stays out of use)
+    }
 }
 
 void *deepj_hip_stream(void) { return g.ready ? (void *)g.stream : nullptr; }

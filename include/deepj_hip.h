@@ -83,7 +83,7 @@ int deepj_hip_trim(void);                  /* returns cached (released) memory t
 int deepj_hip_pool_stats(int64_t out[4]);
 /* Host memory that deepj_hip_download fills without a copy in between (pinned; blocks given back are handed out again).
  * NULL when the bound on such memory (1 GiB at a time) is reached: ordinary memory works everywhere.  These two may be
- * called from any thread. */
+ * called from any thread; host_free leaves the thread's last error as it is. */
 void *deepj_hip_host_alloc(int64_t bytes);
 void deepj_hip_host_free(void *block);
 /* The HIP stream all work is queued on, as a hipStream_t, for callers that time with HIP events. */

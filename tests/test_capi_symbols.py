@@ -42,6 +42,21 @@ def test_no_silent_cpu_fallback_without_a_device():
     assert HipNative.q8Floats(64, 2) == (256 + 2 * 2 * 4) // 4      # pure size arithmetic needs no device
 
 
+def test_a_finaliser_keeps_the_message_of_a_failed_call():
+    """Arrays over the library's host memory give their block back whenever they are collected, also between a failed call
+    and the reading of its message."""
+    lib = ctypes.CDLL(LIB_PATH)
+    lib.deepj_hip_last_error.restype = ctypes.c_char_p
+    lib.deepj_hip_host_free.argtypes = [ctypes.c_void_p]
+    lib.deepj_hip_host_free.restype = None
+    other = ctypes.create_string_buffer(64)                          # no block of the library: ignored
+    assert lib.deepj_hip_upload(1 << 30, other, ctypes.c_int64(1)) != 0
+    message = lib.deepj_hip_last_error()
+    assert message
+    lib.deepj_hip_host_free(ctypes.addressof(other))
+    assert lib.deepj_hip_last_error() == message
+
+
 def test_device_code_is_built_for_gfx950_with_the_required_flags():
     """Every HIP source is compiled for gfx950 with packed-FP32 instructions switched off and with the leading
     kernel arguments preloaded into registers (the decode kernels' argument order relies on it)."""
