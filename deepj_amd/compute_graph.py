@@ -246,10 +246,9 @@ class ComputeGraph:
         self._pending_uploads.clear()
 
     def _execute_pending(self) -> None:
-        cmd, count = self._cmd, self._op_count
+        if self._op_count > 0:
+            self.runtime.flushOps(self._cmd, len(self._cmd))        # (fails before its first launch: the ops stay recorded)
         self._cmd, self._op_count = array.array("i"), 0
-        if count > 0:
-            self.runtime.flushOps(cmd, len(cmd))
 
     def _release_orphans(self) -> None:
         if not self._maybe_orphans:

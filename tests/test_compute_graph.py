@@ -112,6 +112,27 @@ def test_second_flush_only_executes_new_ops(graph, rt):               # :233-253
     assert len(rt.allocCalls) == 2 and len(rt.flushCalls) == 2 and len(rt.uploads) == 1
 
 
+def test_ops_of_a_failed_flush_stay_recorded(graph, rt):
+    """A refused stream has run nothing: its results stay stale, and the next attempt runs it instead of handing out what
+    happens to be in their buffers."""
+    b = graph.newOutputBuffer(2, 3)
+    out = graph.createOutputTensor(b)
+    graph.recordUnary(op.OP_EXP, graph.ensureGpuBuffer(Tensor(2, 3)), b)
+    run, attempts = rt.flushOps, []
+
+    def refuse_once(cmd, length):
+        attempts.append(np.array(cmd[:length]).copy())
+        if len(attempts) == 1:
+            raise RuntimeError("workspace")
+        run(cmd, length)
+    rt.flushOps = refuse_once
+    with pytest.raises(RuntimeError, match="workspace"):
+        graph.materialize(out)
+    assert b.cpuStale and not rt.downloads and not graph.isEmpty()
+    graph.materialize(out)
+    assert len(attempts) == 2 and np.array_equal(*attempts) and rt.downloads == [b.id] and graph.isEmpty()
+
+
 def test_cmd_stream_grows_past_4096_ints(graph, rt):                  # :255-270
     a, b = graph.newOutputBuffer(2, 2), graph.newOutputBuffer(2, 2)
     for _ in range(1000):
