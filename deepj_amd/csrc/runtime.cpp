@@ -49,7 +49,7 @@ struct Graph {
 };
 
 constexpr int kRingSegments = 8;
-constexpr size_t kRingSegmentBytes = (size_t)1 << 20;
+constexpr size_t kRingSegmentBytes = (size_t)512 << 10;
 constexpr size_t kStageBytes = (size_t)4 << 20;
 constexpr int64_t kMaxFlags = 16384;
 constexpr size_t kStageAt = kRingSegments * kRingSegmentBytes, kFlagsAt = kStageAt + kStageBytes;
@@ -110,7 +110,7 @@ void ensure_init(int device = 0) {
     DJ_HIP(hipSetDevice(device));
     DJ_HIP(hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking));
     DJ_HIP(hipHostMalloc((void **)&g.pinned, kPinnedBytes, hipHostMallocDefault));
-    std::memset(g.pinned + kFlagsAt, 0, (size_t)kMaxFlags * sizeof(uint32_t));
+    std::memset(g.pinned, 0, kPinnedBytes);       // the flags start at 0; and no transfer pays for a page's first use (1.4 us each)
     g.ring_at = 0; g.ring_segment = 0; g.n_pieces = 0; g.tag = 0;
     for (int i = 0; i < kRingSegments; i++) {
         DJ_HIP(hipEventCreateWithFlags(&g.ring_done[i], hipEventDisableTiming));
@@ -129,10 +129,13 @@ void ensure_init(int device = 0) {
 }
 
 // ── transfers ───────────────────────────────────────────────────────────────
-// Uploads are copied into a pinned ring and leave it in one launch per flush (k_upload_pieces); downloads arrive chunk by
-// chunk in a pinned stage, or straight in the caller's memory where that came from deepj_hip_host_alloc.  Nothing here
-// waits for the stream except a full ring and a download for its own chunks.  Measured for one tensor operation on a
-// 64 x 32 matrix (two uploads, a product, a download): 57 us with a synchronisation per upload and copy calls.
+// Uploads of up to kRingUpload are copied into a pinned ring and leave it in one launch per flush (k_upload_pieces); larger
+// ones go through a copy call, whose own staging keeps the link busier than one thread's copy into the ring does (1 MiB: 40 us
+// through the ring, 51 by copy call; 4 MiB 146 and 132; 128 MiB 5.3 and 4.7 ms).  Downloads arrive chunk by chunk in a pinned
+// stage, or straight in the caller's memory where that came from deepj_hip_host_alloc.  Nothing here waits for the stream
+// except a full ring, a large upload and a download for its own chunks.  Measured for one tensor operation on a 64 x 32
+// matrix (two uploads, a product, a download): 57 us with a synchronisation per upload and copy calls.
+constexpr int64_t kRingUpload = (1 << 20) / 4;
 
 // Launches what is staged.  Every path that enqueues work or hands a block to another buffer calls it first; a download
 // only where it would read what is staged.
@@ -168,8 +171,8 @@ unsigned char *ring_take(size_t bytes) {
 }
 
 void stage_upload(float *dst, const float *src, int64_t n) {
-    // pieces of a quarter segment: the first is on the link while the next is copied
-    constexpr int64_t kPiece = (int64_t)(kRingSegmentBytes / 4 / 4);
+    // pieces of half a segment: the first is on the link while the next is copied
+    constexpr int64_t kPiece = (int64_t)(kRingSegmentBytes / 2 / 4);
     for (int i = 0; i < g.n_pieces; i++) {
         const UploadPiece &p = g.pieces.p[i];
         if (p.dst == dst && p.n == n) {                       // the same words again before anything read them: the later values stand
@@ -178,6 +181,11 @@ void stage_upload(float *dst, const float *src, int64_t n) {
         }
     }
     if (staged_for(dst, n)) launch_uploads();                 // pieces of one launch run side by side: no two into the same words
+    if (n > kRingUpload) {
+        DJ_HIP(hipMemcpyAsync(dst, src, (size_t)n * 4, hipMemcpyHostToDevice, g.stream));
+        DJ_HIP(hipStreamSynchronize(g.stream));               // the caller's array is only borrowed
+        return;
+    }
     for (int64_t at = 0; at < n; at += kPiece) {
         const int64_t len = std::min(kPiece, n - at);
         unsigned char *p = ring_take((size_t)len * 4);

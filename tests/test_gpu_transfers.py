@@ -1,0 +1,104 @@
+"""Host <-> device transfers: the pinned upload ring, staged and direct downloads, host arrays of the library's own.  Values
+travel as they are, so every comparison is of bits."""
+import numpy as np
+import pytest
+
+from deepj_amd import HipNative
+from deepj_amd.fused import DeviceBuffers
+
+pytestmark = pytest.mark.gpu
+
+PIECE = 1 << 16                  # floats of one piece of the upload ring
+RING_UPLOAD = 1 << 18            # largest upload that goes through it
+RING = 1 << 20                   # floats the ring holds
+
+
+@pytest.fixture
+def dev():
+    d = DeviceBuffers()
+    yield d
+    d.release_all()
+
+
+def values(n, seed):
+    return np.random.default_rng(seed).integers(-2 ** 31, 2 ** 31, n, dtype=np.int64).astype(np.int32)
+
+
+def read(dev, buf, n):
+    out = np.empty(n, np.int32)
+    HipNative.nativeDownloadBuffer(buf, out)
+    return out
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 63, 1021, PIECE - 1, PIECE, PIECE + 1, 2 * PIECE + 3, RING_UPLOAD - 1, RING_UPLOAD,
+                               RING_UPLOAD + 1, 3 * RING_UPLOAD + 5])
+def test_an_upload_of_any_size_arrives_whole_and_nothing_behind_it(dev, n):
+    """One piece, several, the largest that goes through the ring and one more; from a source that is not 16-byte aligned."""
+    a, old = values(n + 1, n)[1:], values(n + 7, n + 1)
+    buf = dev.upload(old)
+    dev.write(buf, a)
+    got = read(dev, buf, n + 7)
+    assert np.array_equal(got[:n], a) and np.array_equal(got[n:], old[n:])
+
+
+def test_uploads_of_several_rings_before_anything_waits(dev):
+    """More than the ring holds, three times over, in sizes that leave every segment's end ragged: none may be overwritten in
+    the ring before its launch has read it."""
+    sizes, total, rng = [], 0, np.random.default_rng(5)
+    while total < 3 * RING:
+        sizes.append(int(rng.choice([1, 7, 300, 5000, PIECE - 5, PIECE, 2 * PIECE + 9, RING_UPLOAD])))
+        total += (sizes[-1] + 63) // 64 * 64
+    sent = [values(n, i) for i, n in enumerate(sizes)]
+    bufs = [dev.upload(a) for a in sent]
+    for i in range(0, len(sent), 3):                       # a third of them again, while the first may still be on the link
+        sent[i] = values(sizes[i], 1000 + i)
+        dev.write(bufs[i], sent[i])
+    for a, b in zip(sent, bufs):
+        assert np.array_equal(read(dev, b, a.size), a)
+
+
+@pytest.mark.parametrize("large", [100, RING_UPLOAD + 64])
+def test_uploads_into_the_same_buffer_land_in_their_order(dev, large):
+    """The whole buffer, its beginning, the whole again and a shorter beginning, before anything waits: staged words are replaced,
+    or launched before the later ones are sent, by either way of sending."""
+    whole, first, again, short = values(large, 1), values(large // 2, 2), values(large, 3), values(17, 4)
+    buf = dev.alloc(large)
+    for seq in ([whole, first], [first, whole], [whole, first, again, short], [short, short + 1, first, whole, short]):
+        exp = read(dev, buf, large)
+        for a in seq:
+            dev.write(buf, a)
+            exp[:a.size] = a
+        assert np.array_equal(read(dev, buf, large), exp)
+
+
+def test_a_released_buffer_takes_no_upload_of_its_predecessor(dev):
+    """The block of a released buffer goes to the next one of its size: what was staged for the first is written first."""
+    for n in (40, 5000):
+        for seed in range(4):
+            a = dev.upload(values(n, seed))
+            dev.release(a)
+            b = dev.upload(values(n, 100 + seed))
+            assert np.array_equal(read(dev, b, n), values(n, 100 + seed))
+            dev.release(b)
+
+
+@pytest.mark.parametrize("n", [1, 3, 2047, 2048, 2049, (512 << 10) // 4, (512 << 10) // 4 + 1, (1 << 20) - 1, (1 << 20) + 1, 2 * (1 << 20) + 4099])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_a_download_into_ordinary_memory(dev, n, offset):
+    """Through the stage: parts of a chunk, chunk edges, both chunk sizes, more than the 4 MiB stage; into memory that is not
+    16-byte aligned, of a buffer that holds more; what surrounds the destination stays."""
+    a = values(n + 9, n)
+    buf, out = dev.upload(a), np.full(n + offset + 3, 7, np.int32)
+    HipNative.nativeDownloadBuffer(buf, out[offset:offset + n])
+    assert np.array_equal(out[offset:offset + n], a[:n])
+    assert np.all(out[:offset] == 7) and np.all(out[offset + n:] == 7)
+
+
+def test_a_small_buffer_is_read_while_uploads_to_others_are_staged(dev):
+    """A download launches staged uploads only where it reads them."""
+    a, b = values(33, 1), values(70, 2)
+    ba, bb = dev.upload(a), dev.upload(b)
+    assert np.array_equal(read(dev, ba, 33), a)
+    dev.write(bb, b + 1)
+    assert np.array_equal(read(dev, ba, 33), a)
+    assert np.array_equal(read(dev, bb, 70), b + 1)
