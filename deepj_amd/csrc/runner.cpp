@@ -608,11 +608,21 @@ void reset(Runner &r) {
     upload_state(r, 0);
 }
 
-// The runtime builds a kernel's function object on its first launch (a few hundred microseconds each), and the
-// decode graphs are captured on first use.  One pass over prompts of the lengths that select the different GEMM and
-// attention variants, and a few graph-replayed tokens, move those costs from the first request to finalize();
-// the sequence state is cleared afterwards (the cache rows written here are never read: every row is rewritten
-// before the position counter reaches it).
+// A graph of kReplayTokens[size] consecutive per-token streams.
+void capture(Runner &r, Choose how, bool narrow, int size) {
+    Stream one = decode_stream(r, how, narrow), s;
+    for (int i = 0; i < kReplayTokens[size]; i++) s.insert(s.end(), one.begin(), one.end());
+    hip(deepj_hip_graph_capture(s.data(), (int32_t)s.size(), &r.graph[how][narrow][size]));
+}
+
+// The runtime builds a kernel's function object on its first launch (a few hundred microseconds each).  One pass over
+// prompts of the lengths that select the different GEMM and attention variants, and a few tokens, move that from the first
+// request to finalize(), and with it the capture of the graphs that greedy decoding replays first; the sequence state is
+// cleared afterwards (the cache rows written here are never read: every row is rewritten before the position counter reaches
+// it).  What a program may never use is left to the request that does: graphs of sampled and of caller-chosen tokens (0.5 to
+// 1.3 ms once) and, for a narrow model, those of the blocks in five launches, which it takes late in a long context or never
+// (1.1 ms once, where loading a 4-layer model of width 256 paid 3.3).  The 16-token graph is captured and not run: its first
+// replay costs what every other does.
 int token_launches(const Config &c, bool narrow);
 void decode_steps(Runner &r, int steps, int mode, Choose how, bool narrow);
 void warm_up(Runner &r) {
@@ -625,28 +635,30 @@ void warm_up(Runner &r) {
         reset(r);
         prefill(r, ids.data(), n, nullptr, kGreedy);
     }
-    for (const bool narrow : {true, false}) {
-        if (narrow ? r.narrow_positions() == 0 : r.narrow_positions() >= c.max_seq) continue;
-        // every size of graph, or as many tokens as there is room for
-        const int steps = std::min(c.max_seq - 2, token_launches(c, narrow) <= kShortStream ? 16 + 4 + 1 : 4 + 1);
-        if (steps < 1) continue;
+    const bool narrow_model = r.narrow_positions() > 0;
+    if (c.max_seq >= 3 && narrow_model && r.narrow_positions() < c.max_seq) {
         reset(r);
         prefill(r, ids.data(), 1, nullptr, kGreedy);
-        decode_steps(r, steps, 1, kGreedy, narrow);
+        decode_steps(r, 1, 0, kGreedy, false);
     }
+    const int steps = std::min(c.max_seq - 2, 4 + 1);
+    if (steps >= 1) {
+        reset(r);
+        prefill(r, ids.data(), 1, nullptr, kGreedy);
+        decode_steps(r, steps, 1, kGreedy, narrow_model);
+    }
+    if (c.max_seq > kReplayTokens[0] && token_launches(c, narrow_model) <= kShortStream) capture(r, kGreedy, narrow_model, 0);
     reset(r);
 }
 
-// `times` replays of the graph of kReplayTokens[size] consecutive per-token streams, captured on first use and again where the
-// runtime refuses it (the workspace it used has been replaced by a larger one since).
+// `times` replays of a graph, captured on first use and again where the runtime refuses it (the workspace it used has been
+// replaced by a larger one since).
 void replay(Runner &r, Choose how, bool narrow, int size, int times) {
     int32_t &graph = r.graph[how][narrow][size];
     if (graph && deepj_hip_graph_launch(graph, times) == 0) return;
     if (graph) hip(deepj_hip_graph_destroy(graph));
     graph = 0;
-    Stream one = decode_stream(r, how, narrow), s;
-    for (int i = 0; i < kReplayTokens[size]; i++) s.insert(s.end(), one.begin(), one.end());
-    hip(deepj_hip_graph_capture(s.data(), (int32_t)s.size(), &graph));
+    capture(r, how, narrow, size);
     hip(deepj_hip_graph_launch(graph, times));
 }
 

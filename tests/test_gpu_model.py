@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from deepj_amd import DeepSeekConfig, DeepSeekModel, HipNative, LlamaConfig, LlamaModel, TextGenerator
+from deepj_amd import opcodes as op
 from deepj_amd.fused import DeviceBuffers, Stream
 from deepj_amd.models import _DecoderOnlyModel
 from oracle import cpu_ref as ref
@@ -232,6 +233,23 @@ def test_deepseek_latent_cache_decode_row_equals_prefill_row(ds_latent):
     gpu.prefill(ids[13:29], choose_next=False)
     gpu.step(int(ids[29]))
     assert float(np.max(np.abs(gpu.lastLogits() - full[29]))) <= 2e-4
+
+
+@pytest.mark.parametrize("d,heads,layers,max_seq,graphs", [(64, 2, 1, 1400, 3), (512, 8, 2, 64, 3), (512, 8, 8, 64, 2), (64, 2, 1, 8, 2)])
+def test_loading_a_model_captures_what_its_requests_replay_first(d, heads, layers, max_seq, graphs):
+    """Graphs of 16, 4 and 1 greedy tokens (16 only for short tokens and contexts that hold them), of one way through the
+    blocks: loading must not pay for graphs that most programs never replay."""
+    nop = Stream().emit(op.OP_NOP, 1).array()
+
+    def next_handle():
+        h = HipNative.graphCapture(nop)
+        HipNative.graphDestroy(h)
+        return h
+    before = next_handle()
+    gpu = LlamaModel(LlamaConfig(vocabSize=64, maxSeqLen=max_seq, dModel=d, nHeads=heads, nLayers=layers, dFF=2 * d), 42)
+    after = next_handle()
+    gpu.close()
+    assert after - before - 1 == graphs
 
 
 @pytest.mark.parametrize("fetched", ["before the step", "after the step"])
