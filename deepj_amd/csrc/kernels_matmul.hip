@@ -2,8 +2,9 @@
 //
 //   C[M x N] = A[M x K] . B      A fp32 row-major, fp32 accumulate
 //
-// fp32 B [K x N] row-major (OP_MATMUL; CpuBackend.java:168-188 in the reference): v_mfma_f32_32x32x2_f32 in k_matmul,
-// whose wavefronts share a tile's K and feed the matrix cores straight from the caches.
+// fp32 B [K x N] row-major (OP_MATMUL; CpuBackend.java:168-188 in the reference): v_mfma_f32_32x32x2_f32, in k_matmul, whose
+// wavefronts share a tile's K and feed the matrix cores straight from the caches, where a tile per compute unit covers the
+// product, else in k_matmul_lds, whose tiles go through LDS and run several to a compute unit.
 //
 // Q8 B [N x Kp] int8 + one fp32 scale per 32-group (prefill-time Q8 GEMM; the M = 1 decode case is the HBM-bound
 // kernel in kernels_q8.hip): v_mfma_f32_32x32x16_bf16 at full fp32 accuracy.  An int8 weight is exact in bf16,
@@ -36,8 +37,8 @@ constexpr int BM2 = 128, BN2 = 128;
 // launch at the small one.  What limits the stages in flight is the L1: a compute unit has 256 lines, and once more than
 // that are outstanding they evict one another (1 x 2752 x 1024 with twice the wavefronts: 11.4 us instead of 7.8).
 // Before (64 x 64 or 128 x 128 tiles staged through LDS, two barriers per 32 k) -> now: 64 x 256 x 256 10.3 -> 3.7 us,
-// 256 x 768 x 192 8.9 -> 3.9, 500 x 2752 x 1024 61 -> 32, 500 x 1024 x 2752 114 -> 33, 1024 x 7000 x 2048 326 -> 295
-// (100 TFLOP/s), 1000 x 2048 x 7000 391 -> 222 (129).
+// 256 x 768 x 192 8.9 -> 3.9, 500 x 2752 x 1024 61 -> 32, 500 x 1024 x 2752 114 -> 33, 2048 x 1024 x 2752 125 -> 97
+// (119 TFLOP/s).
 __device__ __forceinline__ float at_bytes(const float *base, uint32_t bytes) {
     return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + bytes);
 }
@@ -181,6 +182,80 @@ __global__ void __launch_bounds__(64 * KW) k_matmul(const float *__restrict__ A,
                 if (m0 + 32 * i + row < M && n0 + 32 * j + col < N) C[(int64_t)(m0 + 32 * i + row) * N + n0 + 32 * j + col] = v;
             }
         }
+}
+
+// Where a tile per compute unit does not cover the product: workgroups of four wavefronts, a 64 x 64 tile (32 x 32 per
+// wavefront), 32 k a step through LDS.  Both operands sit k-major there, so the 64 lanes of an operand read 32 consecutive
+// floats per half (no bank conflicts).  The loads of the next step are issued before this step's products, and a compute unit
+// holds four such workgroups, whose loads and barriers hide behind one another's products - the direct loads of k_matmul
+// evict one another from the L1 as soon as two of its workgroups share a compute unit.
+// Bound: the fp32 matrix rate.  k_matmul -> this: 1024 x 2752 x 1024 100 -> 68 us, 1000 x 7000 x 1024 266 -> 154,
+// 4096 x 4096 x 256 122 -> 87, 4096 x 4096 x 1024 325 -> 313 (110 TFLOP/s; a 128 x 128 tile took 288 with the sum below in
+// one chain, and there is no room in its registers for more).
+// A sum of K products is taken in four parts by k, as there: its error is that of k_matmul at every K (2.9e-7 of the result's
+// rms at 1024 k), half of what one chain has.
+__global__ void __launch_bounds__(256) k_matmul_lds(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C,
+                                                    const int M, const int N, const int K, const int tiles_n) {
+    constexpr int T = 64, BK = 32, E = 8, kPad = 4, kParts = 4;  // E: values of each operand a thread stages per step
+    __shared__ float As[BK][T + kPad];
+    __shared__ float Bl[BK][T + kPad];
+
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, half = lane >> 5, l32 = lane & 31;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int m0 = ((int)blockIdx.x / tiles_n) * T, n0 = ((int)blockIdx.x % tiles_n) * T;
+
+    const int a_row = t >> 2, a_k = (t & 3) * E;                 // E consecutive k of one row of A
+    const int b_k = t >> 3, b_n = (t & 7) * E;                   // E consecutive columns of one k of B
+    const bool a_vec = (K & 3) == 0, b_vec = (N & 3) == 0;
+    float va[E], vb[E];
+    auto fetch = [&](int k0) {
+        const int row = m0 + a_row, k = k0 + b_k;
+        if (row < M && a_vec && k0 + a_k + E <= K) {
+            const float4 *p = reinterpret_cast<const float4 *>(A + (int64_t)row * K + k0 + a_k);
+            const float4 x = p[0], y = p[1];
+            va[0] = x.x; va[1] = x.y; va[2] = x.z; va[3] = x.w; va[4] = y.x; va[5] = y.y; va[6] = y.z; va[7] = y.w;
+        } else {
+#pragma unroll
+            for (int j = 0; j < E; j++) va[j] = row < M && k0 + a_k + j < K ? A[(int64_t)row * K + k0 + a_k + j] : 0.0f;
+        }
+        if (k < K && b_vec && n0 + b_n + E <= N) {
+            const float4 *p = reinterpret_cast<const float4 *>(B + (int64_t)k * N + n0 + b_n);
+            const float4 x = p[0], y = p[1];
+            vb[0] = x.x; vb[1] = x.y; vb[2] = x.z; vb[3] = x.w; vb[4] = y.x; vb[5] = y.y; vb[6] = y.z; vb[7] = y.w;
+        } else {
+#pragma unroll
+            for (int j = 0; j < E; j++) vb[j] = k < K && n0 + b_n + j < N ? B[(int64_t)k * N + n0 + b_n + j] : 0.0f;
+        }
+    };
+
+    floatx16 acc[kParts];
+#pragma unroll
+    for (int p = 0; p < kParts; p++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[p][e] = 0.0f;
+    fetch(0);
+    for (int k0 = 0; k0 < K; k0 += BK) {
+#pragma unroll
+        for (int j = 0; j < E; j++) As[a_k + j][a_row] = va[j];
+#pragma unroll
+        for (int j = 0; j < E; j++) Bl[b_k][b_n + j] = vb[j];
+        __syncthreads();
+        if (k0 + BK < K) fetch(k0 + BK);
+#pragma unroll
+        for (int kk = 0; kk < BK / 2; kk++)
+            acc[kk % kParts] = __builtin_amdgcn_mfma_f32_32x32x2f32(As[2 * kk + half][wm + l32], Bl[2 * kk + half][wn + l32],
+                                                                    acc[kk % kParts], 0, 0, 0);
+        __syncthreads();
+    }
+
+    // acc[..][e] is C[8 (e / 4) + 4 half + e % 4][l32] of the wavefront's block
+    const int col = n0 + wn + l32;
+    if (col >= N) return;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const int row = m0 + wm + 8 * (e >> 2) + 4 * half + (e & 3);
+        if (row < M) C[(int64_t)row * N + col] = (acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]);
+    }
 }
 
 // ── Q8 weights: three-way bf16 split of the activations ────────────────────
@@ -494,17 +569,29 @@ void launch_matmul(hipStream_t s, const float *a, const float *b, float *out, in
 void launch_matmul_f32(hipStream_t s, const float *a, const float *b, float *out, int m, int n, int k) {
     if (m <= 0 || n <= 0) return;
     if (k <= 0) { launch_fill(s, reinterpret_cast<uint32_t *>(out), 0u, (int64_t)m * n); return; }
-    // The tile with the least time on the busiest compute unit: rounds of 256 tiles times the 32 x 32 blocks of one times
-    // what a block's products take with this tile, relative to the best (measured at K = 1024 and 2752; a small tile loads
-    // more per product, and the rows of A that a tall one walks may share a cache set).
-    struct Shape { int tm, tn; double weight; };
-    static const Shape shapes[] = {{1, 1, 2.0}, {1, 2, 1.35}, {2, 2, 1.3}, {2, 3, 1.05}, {4, 2, 1.1}, {2, 4, 1.0}};
-    int best = 0;
-    double least = 0;
-    for (int i = 0; i < (int)(sizeof(shapes) / sizeof(shapes[0])); i++) {
-        const int64_t tiles = (int64_t)((m + 32 * shapes[i].tm - 1) / (32 * shapes[i].tm)) * ((n + 32 * shapes[i].tn - 1) / (32 * shapes[i].tn));
-        const double cost = (double)((tiles + 255) / 256) * shapes[i].tm * shapes[i].tn * shapes[i].weight;
-        if (i == 0 || cost < least) { least = cost; best = i; }
+    // The kernel and tile of least estimated time, in us: fixed + weight of its rounds x (round + k x per_k), a round being a
+    // tile on each of the 256 compute units.  k_matmul: the first round weighs 1 and every further one `more`, about 2, as two
+    // of its workgroups on a compute unit are in each other's way (2 x 4 tiles leave no room for a second).  k_matmul_lds: the
+    // first of every four rounds (a compute unit's workgroups) 1 and the others `more`.  Fitted to 980 shapes of 1 to 12000
+    // rows and columns over 4 to 6000 k, some of them odd: the tile chosen takes 1.01 times the best one's time on average, 1.4 at
+    // worst; with rounds of k_matmul alone and one weight a tile it took 1.09 on average and 2.8 at worst.
+    struct Shape { int rows, cols; double fixed, round, per_k, more; };
+    static const Shape shapes[] = {{32, 32, 2.3, 0.15, 0.0061, 1.95}, {32, 64, 2.9, 0.2, 0.0101, 2.1},   {64, 64, 3.6, 0.6, 0.0178, 1.6},
+                                   {64, 96, 5.1, 0.6, 0.026, 2.0},    {128, 64, 5.6, 1.3, 0.0334, 1.7}, {64, 128, 0.0, 7.3, 0.0346, 0.97},
+                                   {64, 64, 1.8, 1.4, 0.032, 0.5}};
+    constexpr int kLds = 6;
+    const bool aligned = ((k | n) & 3) == 0;                       // k_matmul_lds stages word by word otherwise: 1.6 x
+    // k_matmul addresses a tile's rows of A and a stage's rows of B in 32 bits
+    const bool in_reach = (int64_t)k * 128 * 4 <= UINT32_MAX && (int64_t)n * 17 * 4 <= UINT32_MAX;
+    int best = kLds;
+    double least = -1.0;
+    for (int i = in_reach ? 0 : kLds; i <= kLds; i++) {
+        const Shape &h = shapes[i];
+        const int64_t tiles = (int64_t)((m + h.rows - 1) / h.rows) * ((n + h.cols - 1) / h.cols), rounds = (tiles + 255) / 256;
+        const int64_t firsts = i == kLds ? (rounds + 3) / 4 : 1;
+        const double weight = (double)firsts + (double)(rounds - firsts) * h.more;
+        const double t = h.fixed + weight * (h.round + h.per_k * k * (i == kLds && !aligned ? 1.6 : 1.0));
+        if (least < 0.0 || t < least) { least = t; best = i; }
     }
     const int64_t blocks = (int64_t)((m + 31) / 32) * ((n + 31) / 32);
     switch (best) {
@@ -518,7 +605,11 @@ void launch_matmul_f32(hipStream_t s, const float *a, const float *b, float *out
         case 2: launch_matmul<2, 2, 4, 1, 2>(s, a, b, out, m, n, k); break;
         case 3: launch_matmul<2, 3, 4, 1, 2>(s, a, b, out, m, n, k); break;
         case 4: launch_matmul<4, 2, 4, 1, 2>(s, a, b, out, m, n, k); break;
-        default: launch_matmul<2, 4, 4, 1, 4>(s, a, b, out, m, n, k); break;
+        case 5: launch_matmul<2, 4, 4, 1, 4>(s, a, b, out, m, n, k); break;
+        default: {
+            const int tn = (n + 63) / 64;
+            launch_kernel(k_matmul_lds, dim3((m + 63) / 64 * tn), dim3(256), 0, s, a, b, out, m, n, k, tn);
+        }
     }
 }
 

@@ -8,6 +8,7 @@ import pytest
 
 from deepj_amd import HipNative, Tensor
 from deepj_amd import opcodes as op
+from deepj_amd.fused import DeviceBuffers, Stream
 from oracle import cpu_ref as ref
 from gpu_util import assert_close, backend, rnd, tensor
 
@@ -35,7 +36,8 @@ def test_matmul_matches_cpu(m, k, n):                                 # :70-78 (
 
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 33, 7), (31, 32, 8), (33, 65, 31), (32, 64, 256), (64, 96, 257), (40, 300, 515),
                                    (97, 2000, 40), (256, 1003, 129), (320, 2752, 36), (500, 2700, 260), (1030, 1100, 130), (900, 4100, 68),
-                                   (2100, 1000, 37)])
+                                   (2100, 1000, 37), (1030, 2756, 1), (1024, 2752, 31), (1090, 2760, 36), (1000, 7000, 133),
+                                   (3001, 2047, 65), (4100, 2052, 260)])
 def test_matmul_tiles_and_remainders(m, n, k):
     """Every tile of the dispatch with rows, columns and K that do not fill it, and K below, at and past a stage of its
     loop.  Bound: a sum of k products in any order is off by at most k * 2^-24 * sum |a||b| (first order; the 2 covers the
@@ -46,6 +48,22 @@ def test_matmul_tiles_and_remainders(m, n, k):
         got = be.matmul(tensor(a), tensor(b)).numpy().astype(np.float64)
     bound = 2 * k * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
     assert np.all(np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= bound)
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 1, 8500000), (1, (1 << 26) + 5, 3)])
+def test_matmul_with_rows_beyond_32_bit_offsets(m, n, k):
+    """A tile's rows of A, or a stage's rows of B, more than 4 GiB apart: what the last row and column hold is found there."""
+    dev = DeviceBuffers()
+    try:
+        a, b, out = dev.alloc(m * k), dev.alloc(k * n), dev.alloc(m * n)
+        three, five = dev.upload(np.array([3.0], np.float32)), dev.upload(np.array([5.0], np.float32))
+        s = Stream().fill(a, 0, m * k).fill(b, 0, k * n)
+        s.copy(three, a, 1, 0, m * k - 1).copy(five, b, 1, 0, k * n - 1).matmul(a, b, out, m, n, k).run()
+        got = dev.download(out, (m * n,))
+    finally:
+        dev.release_all()
+        HipNative.trim()
+    assert got[-1] == 15.0 and np.count_nonzero(got) == 1
 
 
 def test_matmul_rejects_shape_mismatch():                             # :80-86
