@@ -126,8 +126,10 @@ class _HostBlock:
 
 
 def host_array(count: int) -> np.ndarray:
-    """Uninitialised fp32 array for a download.  From 64 KiB on it is pinned memory that the device writes straight into:
-    no stage, no copy out of it and no page faults of a fresh allocation (80 MB: 1.5 ms instead of 6.5)."""
+    """Uninitialised fp32 array for a download.  From 64 KiB on, once some arrays of about its size have been asked for, it is
+    pinned memory that the device writes straight into and that is used again when the array is gone: no stage, no copy out
+    of it and no page faults of a fresh allocation (80 MB: 1.5 ms instead of 6.5).  The library says when (it costs 28 ms to
+    make 80 MB of it); otherwise ordinary memory."""
     if count * 4 >= 65536:
         lib = library()
         address = lib.deepj_hip_host_alloc(count * 4)

@@ -82,8 +82,10 @@ int deepj_hip_trim(void);                  /* returns cached (released) memory t
 /* out[0]=live buffers, out[1]=live bytes, out[2]=cached bytes, out[3]=driver allocations so far */
 int deepj_hip_pool_stats(int64_t out[4]);
 /* Host memory that deepj_hip_download fills without a copy in between (pinned; blocks given back are handed out again).
- * NULL when the bound on such memory (1 GiB at a time) is reached: ordinary memory works everywhere.  These two may be
- * called from any thread; host_free leaves the thread's last error as it is. */
+ * NULL where ordinary memory is the better choice: below 64 KiB, for the first requests of about a size (making a block costs
+ * more than several downloads), where the blocks made so far are kept rather than given back, and when the bound on such
+ * memory (1 GiB at a time) is reached.  Ordinary memory works everywhere.  These two may be called from any thread;
+ * host_free leaves the thread's last error as it is. */
 void *deepj_hip_host_alloc(int64_t bytes);
 void deepj_hip_host_free(void *block);
 /* The HIP stream all work is queued on, as a hipStream_t, for callers that time with HIP events. */

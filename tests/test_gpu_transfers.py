@@ -1,9 +1,13 @@
 """Host <-> device transfers: the pinned upload ring, staged and direct downloads, host arrays of the library's own.  Values
 travel as they are, so every comparison is of bits."""
+import gc
+import resource
+
 import numpy as np
 import pytest
 
 from deepj_amd import HipNative
+from deepj_amd._native import host_array, library
 from deepj_amd.fused import DeviceBuffers
 
 pytestmark = pytest.mark.gpu
@@ -102,3 +106,101 @@ def test_a_small_buffer_is_read_while_uploads_to_others_are_staged(dev):
     dev.write(bb, b + 1)
     assert np.array_equal(read(dev, ba, 33), a)
     assert np.array_equal(read(dev, bb, 70), b + 1)
+
+
+@pytest.fixture
+def blocks():
+    """host_alloc on a pool without blocks and without history."""
+    HipNative.init(0)
+    gc.collect()
+    HipNative.trim()
+    lib, taken = library(), []
+
+    def take(size):
+        p = lib.deepj_hip_host_alloc(size)
+        if p:
+            taken.append(p)
+        return p
+
+    def give(p):
+        taken.remove(p)
+        lib.deepj_hip_host_free(p)
+    yield take, give
+    for p in taken:
+        lib.deepj_hip_host_free(p)
+    HipNative.trim()
+
+
+def test_pinned_blocks_are_made_for_sizes_that_are_asked_for_again_and_again(blocks):
+    take, give = blocks
+    size = 3 << 20
+    assert [take(size - 100 * i) for i in range(8)] == [None] * 8      # the first results of about a size: ordinary memory
+    a, b = take(size), take(size)
+    assert a and b and a != b
+    assert take(size) is None                                          # kept, not given back: no more of them
+    give(a)
+    assert take(size - 4096) == a                                      # used again: one more is worth making
+    c = take(size)
+    assert c and take(size) is None
+    give(b)
+    assert take(1 << 20) == b                                          # up to four times what is asked for
+    give(c)
+    assert take(600 << 10) is None and take(65535) is None
+    give(b)
+    HipNative.trim()
+    assert take(size) is None                                          # nothing kept, nothing remembered
+
+
+def test_a_pinned_block_leaves_no_page_to_its_reader(blocks, dev):
+    """Its pages are in use before it is handed out: the first look at a result must not pay for them."""
+    take, _ = blocks
+    n = 1 << 20
+    for _ in range(8):
+        take(4 * n)
+    out = host_array(n)
+    assert library().deepj_hip_host_alloc(0) is None and type(out.base).__name__ == "_HostBlock"
+    buf = dev.upload(np.arange(n, dtype=np.int32))
+    HipNative.nativeDownloadBuffer(buf, out)
+    before = resource.getrusage(resource.RUSAGE_SELF).ru_minflt
+    last = int(out.view(np.int32)[::1024].max())
+    assert resource.getrusage(resource.RUSAGE_SELF).ru_minflt - before < 64 and last == n - 1024
+
+
+def test_the_bound_on_pinned_memory_ends_in_ordinary_memory(blocks):
+    take, give = blocks
+    size = 300 << 20
+    for _ in range(8):
+        assert take(size) is None
+    a, b = take(size), take(size)
+    give(a)
+    a = take(size)
+    c = take(size)                                                     # 900 MiB (and what the size class adds) are out
+    assert a and b and c
+    give(c)
+    c = take(size)
+    assert c and take(size) is None                                    # another block would pass 1 GiB
+
+
+@pytest.mark.parametrize("n", [1 << 14, (1 << 18) + 3, (1 << 20) + 1, 5 * (1 << 20) + 7])
+def test_a_view_keeps_its_pinned_block(blocks, dev, n):
+    """Results land in the block itself; a view that outlives its array keeps the block from the next result."""
+    take, _ = blocks
+    for _ in range(8):
+        take(4 * n)
+    a, b = values(n, 1), values(n, 2)
+    ba, bb = dev.upload(a), dev.upload(b)
+    first = host_array(n)
+    assert type(first.base).__name__ == "_HostBlock"
+    HipNative.nativeDownloadBuffer(ba, first)
+    view = first[5:n - 1].view(np.int32)
+    address = first.ctypes.data
+    del first
+    second = host_array(n)
+    assert second.ctypes.data != address
+    HipNative.nativeDownloadBuffer(bb, second)
+    assert np.array_equal(view, a[5:n - 1]) and np.array_equal(second.view(np.int32), b)
+    HipNative.nativeDownloadBuffer(bb, second[3:])                     # inside the block, where 128-bit words do not fit
+    assert np.array_equal(second.view(np.int32)[3:], b[:n - 3]) and np.array_equal(second.view(np.int32)[:3], b[:3])
+    del view
+    third = host_array(n)
+    assert third.ctypes.data == address
