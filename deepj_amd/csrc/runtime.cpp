@@ -58,6 +58,10 @@ constexpr int64_t kMaxFlags = 16384;
 constexpr size_t kStageAt = kRingSegments * kRingSegmentBytes, kFlagsAt = kStageAt + kStageBytes;
 constexpr size_t kPinnedBytes = kFlagsAt + (size_t)kMaxFlags * sizeof(uint32_t);
 
+// Host memory that kernels and the host read and write while either runs (the ring, the stage, flags, results whose chunks are
+// announced by flags) has to be coherent; the default is so only as long as the environment (HIP_HOST_COHERENT) leaves it.
+constexpr unsigned kPinnedFlags = hipHostMallocCoherent;
+
 struct Runtime {
     bool ready = false;
     int device = 0;
@@ -112,7 +116,7 @@ void ensure_init(int device = 0) {
     if (device < 0 || device >= count) fail("deepj_hip: bad device index " + std::to_string(device));
     DJ_HIP(hipSetDevice(device));
     DJ_HIP(hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking));
-    DJ_HIP(hipHostMalloc((void **)&g.pinned, kPinnedBytes, hipHostMallocDefault));
+    DJ_HIP(hipHostMalloc((void **)&g.pinned, kPinnedBytes, kPinnedFlags));
     std::memset(g.pinned, 0, kPinnedBytes);       // the flags start at 0; and no transfer pays for a page's first use (1.4 us each)
     g.ring_at = 0; g.ring_segment = 0; g.n_pieces = 0; g.tag = 0;
     for (int i = 0; i < kRingSegments; i++) {
@@ -302,7 +306,7 @@ void *host_take(size_t bytes) {
         g_host.live += cls;                        // (the block itself is made outside the lock)
     }
     void *p = nullptr;
-    const bool ok = hipHostMalloc(&p, cls, hipHostMallocDefault) == hipSuccess;
+    const bool ok = hipHostMalloc(&p, cls, kPinnedFlags) == hipSuccess;
     if (ok)
         for (size_t at = 0; at < cls; at += kPage) static_cast<volatile unsigned char *>(p)[at] = 0;
     else (void)hipGetLastError();
