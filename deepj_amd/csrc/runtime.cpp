@@ -25,6 +25,9 @@
 #include <unordered_map>
 #include <vector>
 
+#include <pthread.h>
+#include <sys/mman.h>
+
 #include "dj_common.h"
 
 namespace dj {
@@ -271,8 +274,12 @@ template <class Done> void wait_flags(volatile uint32_t *flags, int64_t n, uint3
 // ordinary memory.
 // Bounded: at most kHostLive bytes are out at a time and kHostCached kept for reuse.  Locked: finalisers of the arrays over
 // them run on any thread.
+// The driver keeps pinned pages out of a forked child, which may hold arrays over them (a worker that reads results): what
+// the blocks in use hold is copied before the fork and moved to the blocks' addresses in the child, as ordinary memory.
 struct HostPool {
     std::mutex lock;
+    std::vector<std::pair<uintptr_t, void *>> saved;  // between fork's handlers: blocks in use, copies of them (null: no memory)
+    bool fork_handled = false, forked = false;        // handlers registered; this process is the child of one that had blocks
     std::map<uintptr_t, size_t> out;               // blocks in use: address -> class
     std::map<size_t, std::vector<void *>> free;
     size_t live = 0, cached = 0;
@@ -284,12 +291,41 @@ HostPool g_host;
 
 size_t size_class(size_t bytes);
 
+void before_fork() {
+    g_host.lock.lock();
+    if (g_host.forked) return;                     // (a child's arrays are its own memory)
+    for (const auto &block : g_host.out) {
+        void *copy = mmap(nullptr, block.second, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+        if (copy == MAP_FAILED) copy = nullptr;
+        else std::memcpy(copy, reinterpret_cast<const void *>(block.first), block.second);
+        g_host.saved.emplace_back(block.first, copy);
+    }
+}
+void after_fork(bool child) {
+    for (const auto &block : g_host.saved) {
+        if (!block.second) continue;
+        const size_t size = g_host.out[block.first];
+        if (child) (void)mremap(block.second, size, size, MREMAP_MAYMOVE | MREMAP_FIXED, reinterpret_cast<void *>(block.first));
+        else (void)munmap(block.second, size);
+    }
+    g_host.saved.clear();
+    if (child && !g_host.forked) {
+        g_host.forked = true;
+        g_host.free.clear();
+        g_host.cached = 0;
+    }
+    g_host.lock.unlock();
+}
+
 void *host_take(size_t bytes) {
     if (bytes < kHostLeast) return nullptr;
     const size_t cls = size_class(bytes);
     HostPool::Octave &octave = g_host.octaves[63 - __builtin_clzll(bytes)];
     {
         std::lock_guard<std::mutex> hold(g_host.lock);
+        if (g_host.forked) return nullptr;
+        if (!g_host.fork_handled) g_host.fork_handled = pthread_atfork(before_fork, [] { after_fork(false); }, [] { after_fork(true); }) == 0;
+        if (!g_host.fork_handled) return nullptr;
         for (auto it = g_host.free.lower_bound(cls); it != g_host.free.end() && it->first <= 4 * cls; ++it) {
             if (it->second.empty() || g_host.live + it->first > kHostLive) continue;
             void *p = it->second.back();
@@ -323,6 +359,7 @@ void host_give_back(void *p) {
     const size_t cls = it->second;
     g_host.out.erase(it);
     g_host.live -= cls;
+    if (g_host.forked) { (void)munmap(p, cls); return; }
     if (g_host.cached + cls > kHostCached) { (void)hipHostFree(p); return; }
     g_host.free[cls].push_back(p);
     g_host.cached += cls;

@@ -1,6 +1,7 @@
 """Host <-> device transfers: the pinned upload ring, staged and direct downloads, host arrays of the library's own.  Values
 travel as they are, so every comparison is of bits."""
 import gc
+import os
 import resource
 
 import numpy as np
@@ -208,3 +209,40 @@ def test_a_view_keeps_its_pinned_block(blocks, dev, n):
     del view
     third = host_array(n)
     assert third.ctypes.data == address
+
+
+def test_a_forked_child_reads_results_in_pinned_memory(blocks, dev):
+    """As a worker process does that was handed results: their values in the child, which changes its copy, gives it back and
+    forks again; the parent's are untouched, and so is what it goes on to do."""
+    take, _ = blocks
+    n = (1 << 20) + 5
+    for _ in range(8):
+        take(4 * n)
+    a, b = values(n, 1), values(n, 2)
+    ba, bb = dev.upload(a), dev.upload(b)
+    kept, dropped = host_array(n).view(np.int32), host_array(n).view(np.int32)
+    assert type(kept.base.base).__name__ == "_HostBlock"
+    HipNative.nativeDownloadBuffer(ba, kept)
+    HipNative.nativeDownloadBuffer(bb, dropped)
+    del dropped                                                        # a free block: the child has none
+    pid = os.fork()
+    if pid == 0:
+        code = 1
+        try:
+            ok = np.array_equal(kept, a)
+            kept[:] = 7
+            grandchild = os.fork()
+            if grandchild == 0:
+                os._exit(0 if ok and int(kept.sum()) == 7 * n else 1)
+            ok = ok and os.waitpid(grandchild, 0)[1] == 0
+            other = host_array(n)
+            ok = ok and type(other.base).__name__ != "_HostBlock"
+            del kept
+            code = 0 if ok else 2
+        finally:
+            os._exit(code)
+    assert os.waitpid(pid, 0)[1] == 0
+    assert np.array_equal(kept, a)
+    again = host_array(n).view(np.int32)
+    HipNative.nativeDownloadBuffer(bb, again)
+    assert np.array_equal(again, b) and np.array_equal(kept, a)
