@@ -243,7 +243,7 @@ struct DecodeFfn {
     bool swiglu;
 };
 bool decode_block_ok(int d, int hd, int dff);
-int decode_block_positions(int hd);             // cached positions up to which this is the faster way
+int decode_block_positions(int d, int hd);      // cached positions up to which this is the faster way
 int decode_ffn_parts(int dff);
 void launch_decode_attn(hipStream_t s, const DecodeAttn &a);
 void launch_decode_ffn(hipStream_t s, const DecodeFfn &a);

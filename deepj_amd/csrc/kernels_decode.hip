@@ -528,9 +528,13 @@ template <bool SWIGLU> void go_ffn(hipStream_t s, const DecodeFfn &a) {
 }  // namespace
 
 bool decode_block_ok(int d, int hd, int dff) { return d > 0 && dff > 0 && (hd == 32 || hd == 64) && d % hd == 0 && d <= kMaxD; }
-// One workgroup reads all of a head's keys (50 bytes a clock), where the five-launch path has four: at 64 floats a key it is the
-// slower one from about 430 positions on, at 32 from 1400 (d = 256).
-int decode_block_positions(int hd) { return hd == 32 ? 1280 : 384; }
+// One workgroup reads all of a head's keys (50 bytes a clock), where the five-launch path has four, so from some position on the
+// latter is the faster one: 4-layer models, us a token here / there, at 16, 300, 700 and 1250 positions: d 64, hd 32, dff 173
+// 43.8 / 56.4, 46.8 / 56.9, 51.1 / 56.8, 56.7 / 59.6; d 256, hd 32, dff 691 47.7 / 58.8, 52.4 / 58.9, 56.1 / 59.3, 62.2 / 62.4; d 64,
+// hd 64, dff 173 44.4 / 55.1, 51.8 / 55.7, 60.4 / 58.4, 73.5 / 61.3; d 256, hd 64, dff 691 50.1 / 58.7, 58.7 / 59.2, 68.0 / 62.2, 81.9 /
+// 65.3.  The line falls with the width; over dff from 86 to 4096, SwiGLU and GELU, it lies between 130 and 540 positions at hd 64
+// and between 650 and 1650 at hd 32, and this rule is within 5 % of the better way everywhere.
+int decode_block_positions(int d, int hd) { return hd == 32 ? 1536 - 11 * d / 4 : 512 - d; }
 int decode_ffn_parts(int dff) { return (dff + kFfnUnits - 1) / kFfnUnits; }
 
 void launch_decode_attn(hipStream_t s, const DecodeAttn &a) {

@@ -1520,7 +1520,7 @@ void deepj_hip_host_free(void *p) {
 void *deepj_hip_stream(void) { return g.ready ? (void *)g.stream : nullptr; }
 
 int32_t deepj_hip_attn_record_splits(void) { return kAttnRecordSplits; }
-int32_t deepj_hip_decode_block_positions(int32_t d, int32_t hd, int32_t dff) { return decode_block_ok(d, hd, dff) ? decode_block_positions(hd) : 0; }
+int32_t deepj_hip_decode_block_positions(int32_t d, int32_t hd, int32_t dff) { return decode_block_ok(d, hd, dff) ? decode_block_positions(d, hd) : 0; }
 int32_t deepj_hip_latent_decode_splits(int32_t H, int32_t hd, int32_t rank, int32_t max_seq) { return latent_decode_splits(H, hd, rank, max_seq); }
 int32_t deepj_hip_decode_ffn_parts(int32_t dff) { return dff > 0 ? decode_ffn_parts(dff) : 0; }
 

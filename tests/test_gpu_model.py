@@ -8,8 +8,9 @@ dFF 688, maxSeq 256, seed 42, prompt = 32 ids from Random(7), 64 greedy tokens."
 import numpy as np
 import pytest
 
-from deepj_amd import DeepSeekConfig, DeepSeekModel, HipNative, LlamaConfig, LlamaModel, TextGenerator
+from deepj_amd import DeepSeekConfig, DeepSeekModel, GPTConfig, GPTModel, HipNative, LlamaConfig, LlamaModel, TextGenerator
 from deepj_amd import opcodes as op
+from deepj_amd._native import library
 from deepj_amd.fused import DeviceBuffers, Stream
 from deepj_amd.models import _DecoderOnlyModel
 from oracle import cpu_ref as ref
@@ -571,6 +572,36 @@ def test_a_narrow_block_in_two_launches_matches_the_layers(d, hd, dff, max_seq, 
         err = float(np.max(np.abs(a - b)))
         assert err <= 4e-5, (name, err)
     assert float(np.max(np.abs(keys - K))) <= 2e-5 and float(np.max(np.abs(values - V))) <= 2e-5
+
+
+@pytest.mark.parametrize("d,hd,dff,gpt", [(256, 64, 300, False), (128, 64, 130, True), (256, 32, 257, True), (64, 64, 512, False), (192, 32, 384, False)])
+def test_one_generation_goes_from_two_launches_a_block_to_five(d, hd, dff, gpt):
+    """Around the position where a narrow model's blocks change: rows of the cached path equal the prompt's on both sides (within
+    the tolerance of the other such tests), and a greedy, a sampled and an eager run that pass it agree with one another and
+    with the prompt's logits."""
+    at = library().deepj_hip_decode_block_positions(d, hd, dff)
+    cls, config = (GPTModel, GPTConfig) if gpt else (LlamaModel, LlamaConfig)
+    gpu = cls(config(vocabSize=97, maxSeqLen=at + 60, dModel=d, nHeads=d // hd, nLayers=2, dFF=dff), 11)
+    try:
+        before = len(gpu.decodeStream())
+        ids = ref.JavaRandom(5).ints(at + 5, 97)
+        full = gpu.forward(ids)
+        gpu.reset()
+        gpu.prefill(ids[:at - 4], choose_next=False)
+        for t in range(at - 4, at + 5):
+            gpu.step(int(ids[t]))
+            assert float(np.max(np.abs(gpu.lastLogits() - full[t]))) <= 2e-4, t
+        assert len(gpu.decodeStream()) > before                       # (five ops a block: the line was crossed)
+        prompt = ids[:at - 21]
+        greedy = TextGenerator.generate(gpu, prompt, 45, top_k=1)
+        assert np.array_equal(greedy, TextGenerator.generate(gpu, prompt, 45, top_k=1, use_graph=False))
+        sampled = [TextGenerator.generate(gpu, prompt, 45, 0.9, 5, 3, use_graph=g) for g in (True, False)]
+        assert np.array_equal(*sampled)
+        logits = gpu.forward(greedy)
+        for t in range(len(prompt), len(greedy)):                     # the largest logit, up to the tolerance of a row
+            assert logits[t - 1].max() - logits[t - 1, greedy[t]] <= 4e-4, t
+    finally:
+        gpu.close()
 
 
 @pytest.mark.parametrize("d,parts", [(33, 0), (16, 1), (33, 17), (256, 48)])
