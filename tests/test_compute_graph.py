@@ -112,6 +112,33 @@ def test_second_flush_only_executes_new_ops(graph, rt):               # :233-253
     assert len(rt.allocCalls) == 2 and len(rt.flushCalls) == 2 and len(rt.uploads) == 1
 
 
+def test_a_runtime_that_clears_buffers_is_sent_no_zeros(rt):
+    """A tensor nothing was written to is cleared by the runtime, before anything else of the flush is sent; one that was
+    written to, with zeros or not, is sent, and so are all of them where the runtime has no such call."""
+    events = []
+    upload = rt.uploadBuffer
+
+    def upload_logged(buf_id, data):
+        events.append(("sent", buf_id))
+        upload(buf_id, data)
+    rt.uploadBuffer = upload_logged
+    rt.zeroBuffers = lambda buffers: events.append(("cleared", list(buffers)))
+    graph = ComputeGraph(rt)
+    empty, touched, other = Tensor(2, 3), Tensor(2, 3), Tensor(4, 1)
+    touched.data.fill(0.0)
+    ids = [graph.ensureGpuBuffer(t).id for t in (touched, empty, other)]
+    graph.flush()
+    assert events == [("cleared", [(ids[1], 6), (ids[2], 4)]), ("sent", ids[0])]
+    graph.flush()
+    assert len(events) == 2
+
+    plain = RecordingRuntime()
+    g = ComputeGraph(plain)
+    b = g.ensureGpuBuffer(Tensor(2, 3))
+    g.flush()
+    assert [u[0] for u in plain.uploads] == [b.id] and np.array_equal(plain.uploads[0][1], np.zeros(6, np.float32))
+
+
 def test_ops_of_a_failed_flush_stay_recorded(graph, rt):
     """A refused stream has run nothing: its results stay stale, and the next attempt runs it instead of handing out what
     happens to be in their buffers."""

@@ -7,9 +7,10 @@ import resource
 import numpy as np
 import pytest
 
-from deepj_amd import HipNative
+from deepj_amd import HipNative, Tensor
 from deepj_amd._native import host_array, library
 from deepj_amd.fused import DeviceBuffers
+from gpu_util import backend, tensor
 
 pytestmark = pytest.mark.gpu
 
@@ -246,3 +247,22 @@ def test_a_forked_child_reads_results_in_pinned_memory(blocks, dev):
     again = host_array(n).view(np.int32)
     HipNative.nativeDownloadBuffer(bb, again)
     assert np.array_equal(again, b) and np.array_equal(kept, a)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (33, 7), (64, 64), (300, 1003)])
+def test_tensors_nothing_was_written_to_are_zeros_on_the_device(rows, cols):
+    """They are cleared there instead of being sent, in blocks that held other values before, next to tensors that are sent."""
+    rng = np.random.default_rng(rows)
+    with backend() as be:
+        for _ in range(3):                                             # blocks of these sizes with something in them
+            be.add(tensor(rng.standard_normal((rows, cols))), tensor(rng.standard_normal((rows, cols)))).numpy()
+        be.graph.releaseAll()
+        a = rng.standard_normal((rows, cols)).astype(np.float32)
+        z1, z2, row = Tensor.zeros(rows, cols), Tensor.zeros(rows, cols), Tensor.zeros(1, cols)
+        t = tensor(a)
+        assert np.array_equal(be.add(be.add(t, z1), z2).numpy(), a)
+        assert np.array_equal(be.addRowVector(t, row).numpy(), a)
+        assert np.array_equal(be.multiply(z1, t).numpy(), np.zeros_like(a))
+        late = Tensor.zeros(rows, cols)
+        late.data[:] = a                                               # written before it was ever used: sent
+        assert np.array_equal(be.add(late, z2).numpy(), a)
