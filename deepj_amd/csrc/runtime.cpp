@@ -269,9 +269,9 @@ template <class Done> void wait_flags(volatile uint32_t *flags, int64_t n, uint3
 // A block is dear: hipHostMalloc takes 15 us to 0.7 ms, and the host's first use of each of its pages 1.4 us (80 MB: 27 ms, ten
 // times what ordinary memory takes), where a download saves 5 us at 256 KiB, 23 at 1 MiB and 5 ms at 80 MB.  So it is made -
 // its pages in use, nothing of that left to whoever reads the result - for sizes (by octaves) that were asked for kHostAsked
-// times without one: two of them, as a loop holds one result while the next arrives, and then one more for every two times
-// that one has come back and been used again, up to two ahead.  A program that keeps its results, or wants a few, is given
-// ordinary memory.
+// times without one: two of them, as a loop holds one result while the next arrives, or kHostAhead bytes where that is more (the
+// arrays of a training step's tensors, which are filled again at every step), and then one more for every two times that one
+// has come back and been used again.  A program that wants a few results, or keeps large ones, is given ordinary memory.
 // Bounded: at most kHostLive bytes are out at a time and kHostCached kept for reuse.  Locked: finalisers of the arrays over
 // them run on any thread.
 // The driver keeps pinned pages out of a forked child, which may hold arrays over them (a worker that reads results): what
@@ -283,10 +283,11 @@ struct HostPool {
     std::map<uintptr_t, size_t> out;               // blocks in use: address -> class
     std::map<size_t, std::vector<void *>> free;
     size_t live = 0, cached = 0;
-    struct Octave { int asked = 0, spent = 0; } octaves[64];        // a block made costs 2, a block used again gives 1
+    struct Octave { int asked = 0; size_t ahead = 0; } octaves[64];  // bytes of blocks made, less half of those used again
 };
 constexpr size_t kHostLive = (size_t)1 << 30, kHostCached = (size_t)512 << 20, kHostLeast = (size_t)64 << 10, kPage = 4096;
-constexpr int kHostAsked = 8, kHostCredit = 4;
+constexpr size_t kHostAhead = (size_t)16 << 20;
+constexpr int kHostAsked = 4;
 HostPool g_host;
 
 size_t size_class(size_t bytes);
@@ -333,12 +334,12 @@ void *host_take(size_t bytes) {
             it->second.pop_back();
             g_host.cached -= it->first;
             g_host.live += it->first;
-            if (octave.spent > 0) octave.spent--;
+            octave.ahead -= std::min(octave.ahead, cls / 2);
             return p;
         }
         if (octave.asked < kHostAsked) { octave.asked++; return nullptr; }
-        if (octave.spent + 2 > kHostCredit || g_host.live + cls > kHostLive) return nullptr;
-        octave.spent += 2;
+        if (octave.ahead + cls > std::max(2 * cls, kHostAhead) || g_host.live + cls > kHostLive) return nullptr;
+        octave.ahead += cls;
         g_host.live += cls;                        // (the block itself is made outside the lock)
     }
     void *p = nullptr;
@@ -348,7 +349,7 @@ void *host_take(size_t bytes) {
     else (void)hipGetLastError();
     std::lock_guard<std::mutex> hold(g_host.lock);
     if (ok) g_host.out.emplace((uintptr_t)p, cls);
-    else { octave.spent -= 2; g_host.live -= cls; }
+    else { octave.ahead -= std::min(octave.ahead, cls); g_host.live -= cls; }
     return ok ? p : nullptr;
 }
 
