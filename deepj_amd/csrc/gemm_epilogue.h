@@ -70,10 +70,12 @@ __device__ __forceinline__ void rope_store(const RopeStore &r, const RopeColumn 
     else *reinterpret_cast<float4 *>(r.k_cache + at) = o;
 }
 
-// tanh for the GELU below, in double to within 1e-9 absolute (its result is rounded to float and added to 1, where that is a
-// 60th of a unit in the last place): 1 - 2 / (1 + 2^y), y = 2 t log2(e), 2^y from the power series of e^(f ln 2) to the
+// tanh for the GELU below, in double to within 1.4e-10 absolute (its result is rounded to float and added to 1, where that is a
+// 400th of a unit in the last place): 1 - 2 / (1 + 2^y), y = 2 t log2(e), 2^y from the power series of e^(f ln 2) to the
 // eighth degree for |f| <= 1/2.  The math library's tanh is right to the last bit of a double, in some 2 KB of code that
 // a decode step fetches anew at every launch: the matvec of 768 -> 3072 with GELU took 5.9 us with it and takes 4.2 with this.
+// Over 2e7 arguments of N(0, 2) the GELU differs from the one with the library's tanh at 5 of 100000, by one unit in the last
+// place, and is as far from float64 (3.4536e-8 of the results' rms either way, 4.33e-7 at most).
 __device__ __forceinline__ double gelu_tanh(float t) {
     double y = (double)t * 2.88539008177792681472;              // 2 log2(e)
     y = y > 64.0 ? 64.0 : (y < -64.0 ? -64.0 : y);              // tanh is +-1 in float long before; a NaN stays one

@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(256) k_transpose(const float *__restrict__ a, 
 }
 
 // One grid row per tensor: the parameters of a model are stepped one behind the other, and a launch for each cost more than
-// the update of most (nine tensors of 0.6 M values in all: 22 us in nine launches, 5 in one).
+// the update of most (nine tensors of 0.6 M values in all: 22 us in nine launches, 6 in one).
 __global__ void __launch_bounds__(kThreads) k_adamw(const AdamTensors tensors) {
     const AdamTensor p = tensors.t[blockIdx.y];
     const int64_t stride = (int64_t)gridDim.x * kThreads, tid = (int64_t)blockIdx.x * kThreads + threadIdx.x, n4 = p.n >> 2;
@@ -262,9 +262,9 @@ __global__ void __launch_bounds__(kThreads) k_copy(const float *__restrict__ src
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
 }
 
-// Uploads that were staged in pinned memory since the last launch, one grid row each.  Bound by the link (57 GB/s for
-// 1 MiB and more) and below that by the launch: one launch costs the host 2.4 us, so eight uploads of a flush cost 2.4
-// instead of the 8 x (sync + copy) = 75 us that a copy call per upload took.
+// Uploads that were staged in pinned memory since the last launch, one grid row each.  Bound by the link (1 MiB in 22 us) and
+// below that by the launch: one launch costs the host 2.4 us, so eight uploads of a flush cost 2.4 instead of the
+// 8 x (sync + copy) = 75 us that a copy call per upload took.
 __global__ void __launch_bounds__(kThreads) k_upload_pieces(const UploadPieces pieces) {
     const UploadPiece p = pieces.p[blockIdx.y];
     const int64_t n4 = p.n >> 2;

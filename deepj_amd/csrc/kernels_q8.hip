@@ -287,9 +287,10 @@ __device__ __forceinline__ void stage_digits(float *xs, int plane0, int shift_at
 // wavefront's first batch are issued before anything else - they do not depend on the activations - so
 // the HBM stream is already running while the workgroup stages x through LDS and
 // applies the RMSNorm prologue; after that the next batch is always in flight while
-// the current one is multiplied (two register buffers used in turn).
+// the current one is multiplied (its registers move along when it is that one's turn: one copy of the loop's code).
+// The outputs of a batch leave together, an output a lane: bias, activation, residual and the store.
 // MODE (compile time, so that the other variants do not pay for its registers): 1 = GELU on the biased sum
-// (its double-precision tanh costs registers); 2 = ATTN_MERGE prologue: x is not the activation row
+// (its tanh is in double); 2 = ATTN_MERGE prologue: x is not the activation row
 // but the per-split records [head][kAttnRecordSplits][hd + 4] = {max, sum, -, -, o[hd]} the decode attention
 // kernel left, and the row is their merge  x[h*hd + j] = sum_s w_s o_s[j] / sum_s w_s l_s,  w_s = exp(max_s - max).
 // PRO (compile time too: an operand that is not there must not be loaded - a workgroup's activation-sized loads

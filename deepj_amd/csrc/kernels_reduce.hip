@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(kThreads) k_row_reduce(const float *__restrict
 // Column sums [rows x cols] -> [1 x cols].  A workgroup of 1024 threads takes 32 columns (one 128-byte line of every row):
 // V = 4 of them a thread and 128 rows at a time, or one (V = 1, widths that are no multiple of 4) and 32; eight rows a
 // thread are on their way at once.  Bound by that latency: 256 x 768 (0.8 MB) 10.0 us with 64 columns and four rows at a
-// time -> 3.1.
+// time -> 2.9.
 template <int V>
 __global__ void __launch_bounds__(1024) k_sum_rows(const float *__restrict__ a, float *__restrict__ out, int rows, int cols) {
     constexpr int kCols = 32 / V, kLanes = 1024 / kCols;             // threads along a row, and rows at a time
