@@ -85,8 +85,8 @@ int deepj_hip_pool_stats(int64_t out[4]);
  * NULL where ordinary memory is the better choice: below 64 KiB, for the first requests of about a size (making a block costs
  * more than several downloads), where the blocks made so far are kept rather than given back, and when the bound on such
  * memory (1 GiB at a time) is reached.  Ordinary memory works everywhere.  These two may be called from any thread
- * (host_alloc once the library is initialised); host_free leaves the thread's last error as it is.  A child made by fork() finds the blocks in use, with what they held,
- * as ordinary memory of its own. */
+ * (host_alloc once the library is initialised); host_free leaves the thread's last error as it is.  A child made by
+ * fork() finds the blocks in use, with what they held, as ordinary memory of its own. */
 void *deepj_hip_host_alloc(int64_t bytes);
 void deepj_hip_host_free(void *block);
 /* The HIP stream all work is queued on, as a hipStream_t, for callers that time with HIP events. */
