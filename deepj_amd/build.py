@@ -41,6 +41,7 @@ SOURCES = {
     # instructions after every few products, and each trip through the accumulator file costs a move per value
     "kernels_matmul.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_gemm_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "kernels_gemm_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_q8.hip": [],
     "kernels_decode.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],

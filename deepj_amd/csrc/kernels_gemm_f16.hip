@@ -44,6 +44,7 @@
 // stores 16 bytes per lane.
 #include "dj_common.h"
 #include "gemm_epilogue.h"
+#include "gemm_rows.h"
 #include <cstdlib>
 #include <type_traits>
 
@@ -70,20 +71,6 @@ struct GemmF16Args {
     int split_steps;            // 64-row kernel only: K steps per share of a tile (0: all of K, no partial sums); gridDim.z shares
     float *partial;             // [gridDim.z][m][n] partial products when split_steps > 0
 };
-
-// 64 lanes x 16 bytes from base + off[lane] into LDS bytes [dst, dst + 1024), lane order.  The statements write M0
-// and say so in their clobber lists, so that the compiler never carries a value of its own in M0 across them (it
-// initialises M0 itself for some LDS and message instructions); clang notes that M0 is a reserved register, which
-// is the point of listing it.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void load_to_lds16(const void *base, uint32_t off, uint32_t dst) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
-}
-__device__ __forceinline__ void load_to_lds4(const void *base, uint32_t off, uint32_t dst) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
-}
-#pragma clang diagnostic pop
 
 // Timeline of one launch, for tuning builds only (-DDJ_TRACE; never in the shipped library): every wavefront leaves
 // 100 MHz time stamps at its start, at its first product, after its K loop and after its epilogue.
@@ -584,13 +571,24 @@ __global__ void __launch_bounds__(256) k_sum_partials(const float *__restrict__ 
 // one each (the sum of the slabs, the split of the rows).  Rows that fit the register path only.
 struct SplitSum { const float *partial; int splits; int64_t slab; const float *bias, *residual; float *sum_out; };
 
-template <int NORM, bool SUM = false>
+template <int NORM, bool SUM = false, bool OPERAND = false>
 __global__ void __launch_bounds__(256) k_split_f16(const float *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta,
                                                    uint16_t *__restrict__ planes, float *__restrict__ unscale, int m, int k, int kp, int pitch,
                                                    int64_t plane_elems, const SplitSum sum) {
 #pragma clang fp contract(off)
     __shared__ float red[4];
-    const int row = blockIdx.x, t = threadIdx.x;
+    int row = blockIdx.x;
+    const int t = threadIdx.x;
+    // operand order: eight consecutive rows share their lines, and an XCD (workgroup index mod 8) writes them all
+    if (OPERAND && (row | 63) < (int)gridDim.x) row = (row & ~63) | ((row & 7) << 3) | ((row >> 3) & 7);
+    if (OPERAND && row >= m) {
+        for (int c = t * 8; c < kp; c += 2048) {
+            uint4 *p = reinterpret_cast<uint4 *>(planes + operand_at(row, c, kp / kQ8Group));
+            p[0] = p[kOperandPiece / 8] = make_uint4(0u, 0u, 0u, 0u);
+        }
+        if (t == 0) unscale[row] = 0.f;
+        return;
+    }
     if (row >= m) {
         uint32_t *hi32 = reinterpret_cast<uint32_t *>(planes + (int64_t)row * pitch), *lo32 = hi32 + plane_elems / 2;
         for (int c = t; c < kp / 2; c += 256) { hi32[c] = 0u; lo32[c] = 0u; }
@@ -625,8 +623,8 @@ __global__ void __launch_bounds__(256) k_split_f16(const float *__restrict__ x, 
         l = __builtin_bit_cast(uint16_t, ll);
     };
     uint16_t *hi = planes + (int64_t)row * pitch, *lo = hi + plane_elems;
-    constexpr int NV = 8;                                            // 128-bit words a thread keeps of one row
-    if (SUM || ((k & 3) == 0 && k == kp && k <= 256 * 4 * NV)) {
+    constexpr int NV = OPERAND ? 12 : 8;                             // 128-bit words a thread keeps of one row
+    if (SUM || ((k & 3) == 0 && (k == kp || OPERAND) && kp <= 256 * 4 * NV)) {
         // the row stays in registers: one pass over memory
         const int n4 = k >> 2;
         const float4 *row4 = reinterpret_cast<const float4 *>(xr);
@@ -698,9 +696,16 @@ __global__ void __launch_bounds__(256) k_split_f16(const float *__restrict__ x, 
 #pragma unroll
         for (int j = 0; j < NV; j++) {
             const int i = t + j * 256;
-            if (i >= n4) continue;
+            if (i >= (OPERAND ? kp >> 2 : n4)) continue;
             uint16_t h[4], l[4];
-            halves(v[j].x * up, h[0], l[0]); halves(v[j].y * up, h[1], l[1]); halves(v[j].z * up, h[2], l[2]); halves(v[j].w * up, h[3], l[3]);
+            const float by = OPERAND && operand_negated(4 * i) ? -up : up;
+            halves(v[j].x * by, h[0], l[0]); halves(v[j].y * by, h[1], l[1]); halves(v[j].z * by, h[2], l[2]); halves(v[j].w * by, h[3], l[3]);
+            if constexpr (OPERAND) {
+                uint16_t *p = planes + operand_at(row, 4 * i, kp / kQ8Group);
+                *reinterpret_cast<uint2 *>(p) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+                *reinterpret_cast<uint2 *>(p + kOperandPiece) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+                continue;
+            }
             reinterpret_cast<uint2 *>(hi)[i] = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
             reinterpret_cast<uint2 *>(lo)[i] = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
         }
@@ -731,9 +736,10 @@ __global__ void __launch_bounds__(256) k_split_f16(const float *__restrict__ x, 
     const float up = scale_of(block_reduce(mx, true));
     for (int c = t; c < kp; c += 256) {
         uint16_t h, l;
-        halves(c < k ? value(c) * up : 0.f, h, l);
-        hi[c] = h;
-        lo[c] = l;
+        halves(c < k ? value(c) * (OPERAND && operand_negated(c) ? -up : up) : 0.f, h, l);
+        const int64_t at = OPERAND ? operand_at(row, c, kp / kQ8Group) : (int64_t)row * pitch + c;
+        planes[at] = h;
+        planes[at + (OPERAND ? kOperandPiece : plane_elems)] = l;
     }
 }
 
@@ -963,6 +969,11 @@ void launch_q8_gemm_f16(hipStream_t s, const float *x, const float *gamma, const
         if (roped) launch_kernel((k_gemm_q8_f16<4, true>), dim3(grid_x), dim3(256), (size_t)kStages * stage128_bytes(4), s, a);
         else launch_kernel((k_gemm_q8_f16<4>), dim3(grid_x), dim3(256), (size_t)kStages * stage128_bytes(4), s, a);
     }
+}
+
+void launch_split_operand(hipStream_t s, const float *x, const float *gamma, const float *beta, uint16_t *planes, float *unscale, int m, int m_pad, int k, int kp) {
+    auto split = !gamma ? k_split_f16<0, false, true> : beta ? k_split_f16<2, false, true> : k_split_f16<1, false, true>;
+    launch_kernel(split, dim3(m_pad), dim3(256), 0, s, x, gamma, beta, planes, unscale, m, k, kp, kp, (int64_t)0, SplitSum{});
 }
 
 #ifdef DJ_TRACE

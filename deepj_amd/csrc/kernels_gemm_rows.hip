@@ -1,0 +1,342 @@
+// Q8 GEMM for a batch of rows straight from the int8 weights: C[M x N] = X[M x K] . dequant(W)^T, W int8 [N x Kp] with one
+// fp32 scale per 32 k.
+//
+// Arithmetic as in kernels_gemm_f16.hip: a row of activations times a power of two, split into two fp16 numbers (22 bits), the
+// weights exact in fp16, two v_mfma_f32_32x32x16_f16 per 16 k, the group scale on the finished 32-k sums.  The split happens
+// once, in a launch in front that also normalises the rows (k_split_f16), where the bf16 kernels (kernels_matmul.hip) turn the
+// activations into three pieces anew for every column tile; the weights stay int8 in memory and become fp16 in registers,
+// where the fp16 GEMM reads a copy of twice their size.
+//
+// A workgroup takes a tile of 32 TMW x 32 TNW and deals its K to four wavefronts in chunks of 128, one line of a weight row:
+// no wavefront waits for another before the end, when their sums meet in LDS.  A wavefront asks for a chunk of its weights one
+// chunk ahead, global -> LDS in whole lines, and for its activations NA groups ahead, straight into registers in operand order;
+// loads return in the order they were asked for, so waiting for activations that were asked for after a chunk is waiting for
+// the chunk.  The matrix cores' 32 cycles a product hide the group before's scaling and the next one's conversion.
+//
+// What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 38 us with the split, 87 on the bf16
+// kernels; 4.6 TB/s in the K loop), then the activations, which every tile reads anew from L2 (8 KB for every 64 x 64 x 32:
+// 64 x 22016 51 us, 86; 200 x 11264 over 2048 41, 67), and on small weights two launches' latency (30 x 2304 over 768 9.7 us,
+// 11.9).  Tried and slower: eight wavefronts a workgroup (two workgroups of four fill a compute unit better: 64 x 22016 54 us
+// against 49), the K loop or the epilogue rolled (3 % and 10 %), a 64 x 64 tile whose wavefronts share the activations through
+// LDS (latency of its reads and barriers: 400 x 768 over 3072 34 us against 22).
+//
+// Error against 64 bits: 0.95e-7 to 1.83e-7 of the result's rms over 768 to 11008 k, 0.96e-7 to 1.87e-7 on the bf16 kernels.  It
+// hangs on the number of sums a row is dealt to (four wavefronts, NS sets in each), on the low pieces' products going first, and
+// on every second chunk's sign (operand_negated).
+#include "dj_common.h"
+#include <algorithm>
+#include "gemm_epilogue.h"
+#include "gemm_rows.h"
+
+namespace dj {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+
+namespace {
+
+constexpr int kWaves = 4;
+constexpr int kChunk = kOperandChunk / kQ8Group;                   // scale groups a wavefront takes at a time: 128 k, one line of a weight row
+constexpr int slot_bytes(int tnw) { return 32 * tnw * 128 + kChunk * 256; }       // a wavefront's chunk in LDS: weights [column][128], scales [group][64]
+
+struct GemmRowsArgs {
+    const uintx4 *planes;        // activations in operand order (rows_plane_at)
+    const int8_t *wq;           // [n][kp]
+    const float *scales;        // [n][groups]
+    const float *unscale;       // [m up to a multiple of 32]
+    float *out;
+    int m, n, groups;
+    int m_tiles, n_tiles;       // tiles of the launched kernel's size
+    GemmEpilogue ep;
+    int share_chunks;           // > 0: gridDim.z workgroups share a tile's K, this many chunks each
+    float *partial;             // [gridDim.z][m][n] when they do
+};
+
+// four int8 of a word as fp16: the byte with its sign bit flipped is b + 128, under the exponent of 1024 it reads 1152 + b
+__device__ __forceinline__ void int8x4_to_half(uint32_t r, uint32_t &lo, uint32_t &hi) {
+    const halfx2 bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    r ^= 0x80808080u;
+    lo = __builtin_bit_cast(uint32_t, __builtin_bit_cast(halfx2, __builtin_amdgcn_perm(0x64646464u, r, 0x04010400u)) + bias);
+    hi = __builtin_bit_cast(uint32_t, __builtin_bit_cast(halfx2, __builtin_amdgcn_perm(0x64646464u, r, 0x04030402u)) + bias);
+}
+
+template <int TMW, int TNW>
+__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) k_gemm_q8_rows(const GemmRowsArgs a) {
+    constexpr int TN = 32 * TNW, NL = TN / 8;          // NL: loads a wavefront makes for a chunk of its TN weight rows
+    constexpr int kSlot = slot_bytes(TNW);
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), half = lane >> 5, l32 = lane & 31;
+    unsigned char *wl = lds + wave * 2 * kSlot;
+    const uint32_t wl_at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)wl);
+    // row tiles of a column tile on one XCD
+    const int per_group = 8 * a.m_tiles, gi = (int)blockIdx.x / per_group, r = (int)blockIdx.x % per_group;
+    const int n_tile = gi * 8 + (r & 7), m_tile = r >> 3;
+    if (n_tile >= a.n_tiles) return;
+    const int n0 = n_tile * TN, m0 = m_tile * 32 * TMW, kp = a.groups * kQ8Group;
+    const int row_tiles = (a.m + 31) >> 5;
+
+    const int chunks = (a.groups + kChunk - 1) / kChunk;
+    const int c_begin = a.share_chunks > 0 ? (int)blockIdx.z * a.share_chunks : 0;
+    const int c_end = a.share_chunks > 0 ? min(chunks, c_begin + a.share_chunks) : chunks;
+
+    // All addresses stay inside: columns past N read the last row's weights, rows past M the zeros behind the last (or its tile
+    // again), pieces past K the row's first again.
+    // This lane's pieces of a chunk: 16 bytes of row 8 i + lane / 8.  Piece p of a row goes to position p ^ (row % 8).
+    const int b_piece = ((lane & 7) ^ (lane >> 3)) * 16;
+    const int8_t *b_base = a.wq + (int64_t)n0 * kp;
+    const float *s_base = a.scales + (int64_t)n0 * a.groups;
+    uint32_t b_off[NL];
+#pragma unroll
+    for (int i = 0; i < NL; i++) b_off[i] = (uint32_t)min(8 * i + (lane >> 3), a.n - 1 - n0) * (uint32_t)kp + b_piece;
+    const uint32_t s_off = (uint32_t)min(min(lane, TN - 1), a.n - 1 - n0) * (uint32_t)a.groups * 4u;
+    const uint32_t q_at = l32 * 128, q_x = l32 & 7;
+    const uintx4 *ap[TMW];
+#pragma unroll
+    for (int i = 0; i < TMW; i++) ap[i] = a.planes + (int64_t)min(m_tile * TMW + i, row_tiles - 1) * chunks * kChunk * 256;
+
+    auto fetch_b = [&](int c, int slot) __attribute__((always_inline)) {
+        const uint32_t back = c * (kChunk * kQ8Group) + b_piece < kp ? 0u : (uint32_t)b_piece;       // past the row's end: a piece that meets activations of zero
+        const uint32_t dst = wl_at + slot * kSlot;
+#pragma unroll
+        for (int i = 0; i < NL; i++) load_to_lds16(b_base + (int64_t)c * (kChunk * kQ8Group), b_off[i] - back, dst + i * 1024);
+#pragma unroll
+        for (int g = 0; g < kChunk; g++) load_to_lds4(s_base + min(c * kChunk + g, a.groups - 1), s_off, dst + TN * 128 + g * 256);
+    };
+    constexpr int NA = TMW == 1 ? 4 : 2;               // groups of activations in flight
+    uintx4 av[NA][TMW][4];                             // [group % NA][row tile]: low pieces of the two k steps, high pieces
+    auto fetch_a = [&](int i, int j, int g) __attribute__((always_inline)) { return (ap[i] + (int64_t)g * 256)[64 * (2 * (j & 1) + (j < 2)) + lane]; };
+    constexpr int NS = 4 / (TMW * TNW);                // sets of sums: a group's goes to set group % NS
+    floatx16 acc[NS][TMW][TNW], p[2];
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+#pragma unroll
+        for (int i = 0; i < TMW; i++)
+#pragma unroll
+            for (int j = 0; j < TNW; j++)
+#pragma unroll
+                for (int z = 0; z < NS; z++) acc[z][i][j][e] = 0.0f;
+        p[0][e] = p[1][e] = 0.0f;
+    }
+    uint32_t bw[2][8];                                 // [stage parity]: the weights of a stage (a column tile of a group) as fp16
+    uintx4 q[2];                                       // ... and as bytes, up to two stages ahead
+    float sc[4] = {0.f, 0.f, 0.f, 0.f};                // their scales: of the stage before, this one and the two next
+    auto read_q = [&](int slot, int g, int tn, int at, int at_sc) __attribute__((always_inline)) {
+        sc[at_sc] = *reinterpret_cast<const float *>(wl + slot * kSlot + TN * 128 + g * 256 + (32 * tn + l32) * 4);
+        q[at] = *reinterpret_cast<const uintx4 *>(wl + slot * kSlot + 4096 * tn + q_at + (((2 * g + half) ^ q_x) << 4));
+    };
+    int c = c_begin + wave, slot = 0;
+    if (c < c_end) {
+        fetch_b(c, 0);
+#pragma unroll
+        for (int g = 0; g < NA; g++)
+#pragma unroll
+            for (int i = 0; i < TMW; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) av[g][i][j] = fetch_a(i, j, c * kChunk + g);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * NA * TMW) : "memory");
+        read_q(0, 0, 0, 0, 1);
+#pragma unroll
+        for (int w = 0; w < 4; w++) int8x4_to_half(q[0][w], bw[0][2 * w], bw[0][2 * w + 1]);
+        read_q(0, 1 / TNW, 1 % TNW, 1, 2);
+        constexpr int S = kChunk * TNW, kAhead = 2 / TNW;     // stages of a chunk; groups in two stages
+#pragma unroll 1
+        for (; c < c_end; c += kWaves, slot ^= 1) {
+            const int next = min(c + kWaves, c_end - 1);
+            fetch_b(next, slot ^ 1);
+#pragma unroll
+            for (int st = 0; st < S; st++) {
+                const int g = st / TNW, tn = st % TNW;
+                // two stages on is the next chunk: its weights were asked for before the activations of the groups since
+                if (st == S - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((4 - kAhead) * 4 * TMW) : "memory");
+                const uintx4 qn = q[(st + 1) & 1];
+                const bool wrap = st + 2 >= S;
+                const int g2 = (g + kAhead) % kChunk;
+                read_q(wrap ? slot ^ 1 : slot, g2, tn, st & 1, (st + 3) & 3);
+#pragma unroll
+                for (int tm = 0; tm < TMW; tm++) {
+                    const int u = st * TMW + tm;
+                    const int ptm = tm > 0 ? tm - 1 : TMW - 1, pst = tm > 0 ? st : (st + S - 1) % S, ptn = pst % TNW, pg = pst / TNW;
+                    const float psc = tm > 0 ? sc[(st + 1) & 3] : sc[st & 3];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const uint32_t *w4 = bw[st & 1] + 4 * (j & 1);
+                        p[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, av[g % NA][tm][j]), __builtin_bit_cast(halfx8, (uintx4){w4[0], w4[1], w4[2], w4[3]}),
+                                                                          j == 0 ? (floatx16){} : p[u & 1], 0, 0, 0);
+                        if (tn == TNW - 1) av[g % NA][tm][j] = fetch_a(tm, j, g + NA < kChunk ? c * kChunk + g + NA : next * kChunk + g + NA - kChunk);
+                        // the sums of the tile before, and a share of the next stage's weights
+#pragma unroll
+                        for (int e = 0; e < 16; e++)
+                            if (j == (e < 6 ? 1 : e < 11 ? 2 : 3)) acc[pg % NS][ptm][ptn][e] = fmaf(p[(u & 1) ^ 1][e], psc, acc[pg % NS][ptm][ptn][e]);
+                        if (TMW == 1 || (j & 1) == 0) {
+                            const int w = TMW == 1 ? j : 2 * tm + j / 2;
+                            int8x4_to_half(qn[w], bw[(st + 1) & 1][2 * w], bw[(st + 1) & 1][2 * w + 1]);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[3 % NS][TMW - 1][TNW - 1][e] = fmaf(p[1][e], sc[0], acc[3 % NS][TMW - 1][TNW - 1][e]);
+        if constexpr (NS > 1) {
+#pragma unroll
+            for (int i = 0; i < TMW; i++)
+#pragma unroll
+                for (int j = 0; j < TNW; j++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) {
+                        acc[0][i][j][e] += acc[1][i][j][e];
+                        if constexpr (NS == 4) acc[0][i][j][e] += acc[2][i][j][e] + acc[3][i][j][e];
+                    }
+        }
+    }
+
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the loads ahead of the last chunk have landed before LDS is used again
+    // the wavefronts' sums, in a fixed order
+    __syncthreads();
+    float4 *red = reinterpret_cast<float4 *>(lds);
+    constexpr int Q = TMW * TNW * 4;                   // runs of four rows of a lane
+#pragma unroll
+    for (int i = 0; i < TMW; i++)
+#pragma unroll
+        for (int j = 0; j < TNW; j++)
+#pragma unroll
+            for (int eq = 0; eq < 4; eq++)
+                red[(wave * Q + (i * TNW + j) * 4 + eq) * 64 + lane] = make_float4(acc[0][i][j][4 * eq], acc[0][i][j][4 * eq + 1], acc[0][i][j][4 * eq + 2], acc[0][i][j][4 * eq + 3]);
+    __syncthreads();
+    const GemmEpilogue &ep = a.ep;
+#pragma unroll 1
+    for (int q = wave; q < Q; q += kWaves) {
+        const int tile = q >> 2, eq = q & 3, tm = tile / TNW, tn = tile % TNW;
+        const int row0 = m0 + 32 * tm + 8 * eq + 4 * half, col = n0 + 32 * tn + l32;
+        if (m0 + 32 * tm + 8 * eq >= a.m) continue;    // wavefront-uniform
+        float4 s = red[q * 64 + lane];
+#pragma unroll
+        for (int v = 1; v < kWaves; v++) {
+            const float4 o = red[(v * Q + q) * 64 + lane];
+            if ((v & 1) == 0) { s.x += o.x; s.y += o.y; s.z += o.z; s.w += o.w; }
+            else { s.x -= o.x; s.y -= o.y; s.z -= o.z; s.w -= o.w; }
+        }
+        const float4 us = *reinterpret_cast<const float4 *>(a.unscale + row0);
+        const float turn = c_begin & 1 ? -1.0f : 1.0f;
+        s.x *= us.x * turn; s.y *= us.y * turn; s.z *= us.z * turn; s.w *= us.w * turn;
+        const bool in = col < a.n;
+        float badd = 0.0f;
+        if (a.share_chunks == 0 && ep.bias && in) badd = ep.interleaved_bias ? ((col & 1) ? ep.bias2[col >> 1] : ep.bias[col >> 1]) : ep.bias[col];
+#pragma unroll
+        for (int row = row0; row < row0 + 4; row++) {  // (rolled: the steps below are most of a short launch's code)
+            float v = s.x;
+            s.x = s.y; s.y = s.z; s.z = s.w;
+            const bool live = in && row < a.m;
+            if (a.share_chunks > 0) {
+                if (live) a.partial[((int64_t)blockIdx.z * a.m + row) * a.n + col] = v;
+                continue;
+            }
+            if (ep.bias) v = v + badd;
+            if (ep.swiglu) {
+                // (gate, up) pairs in neighbouring lanes (SiLU.java:20-24, SwiGLULayer.java:69)
+                const float other = __shfl_xor(v, 1, 64);
+                if (live && (col & 1) == 0) a.out[(int64_t)row * (a.n >> 1) + (col >> 1)] = v * (1.0f / (1.0f + expf(-v))) * other;
+                continue;
+            }
+            if (!live) continue;
+            if (ep.gelu) v = gemm_gelu(v);
+            if (ep.residual) v = ep.residual[(int64_t)row * a.n + col] + v;
+            a.out[(int64_t)row * a.n + col] = v;
+        }
+    }
+}
+
+constexpr int lds_bytes(int tmw, int tnw) {
+    const int stage = kWaves * 2 * slot_bytes(tnw), red = kWaves * tmw * tnw * 4096;
+    return stage > red ? stage : red;
+}
+
+template <typename F> void each_kernel(F f) {
+    f(k_gemm_q8_rows<1, 1>, 1, 1); f(k_gemm_q8_rows<1, 2>, 1, 2); f(k_gemm_q8_rows<2, 1>, 2, 1); f(k_gemm_q8_rows<2, 2>, 2, 2);
+}
+
+int chunks_of(int k) { return (q8_padded_k(k) / kQ8Group + kChunk - 1) / kChunk; }
+
+// A tile's rows and columns in units of 32 and the workgroups that share its K: those of least estimated time, in us.  With x
+// tiles a compute unit and kk thousand k a wavefront, a launch takes
+//   fixed + per_x x + kk (per_k + again (rounds - 1) + per_kx x) + slabs m n shares / 10^6,
+// rounds being 1 up to one tile a compute unit, 2 up to two (two workgroups fit one) and x beyond.  Fitted to 155 shapes of 4 to
+// 512 rows, 768 to 50257 columns and 256 to 11008 k: the choice takes 1.01 times the best one's time on average.  (200 x 2304
+// over 768: 32 x 32 13.4 us, 32 x 64 15.8, 64 x 32 15.3, 64 x 64 15.6; 200 x 11008 over 4096: 53, 44, 48, 41; 4 x 4096 over
+// 11008: 32 x 32 31, K shared by two 25, by four 27.)
+struct RowsPlan { int tmw, tnw, shares; };
+RowsPlan rows_plan(int m, int n_rows, int k, bool may_share) {
+    struct Shape { int tmw, tnw, shares; double fixed, per_x, per_k, again, per_kx, slabs; };
+    static const Shape shapes[] = {{1, 1, 1, 8.29, 0.27, 1.63, 1.29, 0.91, 0.0}, {1, 2, 1, 8.65, 0.87, 2.59, 1.63, 1.5, 0.0},
+                                   {2, 1, 1, 8.12, 0.31, 2.51, 1.72, 1.63, 0.0}, {2, 2, 1, 9.76, 1.37, 3.49, 2.53, 2.2, 0.0},
+                                   {1, 1, 2, 10.39, 0.6, 1.49, 1.12, 0.8, 2.24}, {1, 1, 4, 9.63, 1.19, 2.91, 1.57, -0.04, 1.12}};
+    RowsPlan best{};
+    double least = -1.0;
+    for (const Shape &h : shapes) {
+        if (h.shares > 1 && (!may_share || (n_rows & 1) || chunks_of(k) < 2 * h.shares)) continue;      // k_sum_partials_q8 takes columns in pairs
+        const double x = (double)((m + 32 * h.tmw - 1) / (32 * h.tmw)) * (double)((n_rows + 32 * h.tnw - 1) / (32 * h.tnw)) * h.shares / 256.0;
+        const double rounds = x <= 1.0 ? 1.0 : x <= 2.0 ? 2.0 : x;
+        const int turns = ((chunks_of(k) + kWaves - 1) / kWaves + h.shares - 1) / h.shares;
+        const double kk = turns * kWaves * kChunk * kQ8Group * 1e-3;
+        const double t = h.fixed + h.per_x * x + kk * (h.per_k + h.again * (rounds - 1.0) + h.per_kx * x) + h.slabs * m * n_rows * h.shares * 1e-6;
+        if (least < 0.0 || t < least) { least = t; best = {h.tmw, h.tnw, h.shares}; }
+    }
+    return best;
+}
+
+}  // namespace
+
+void q8_gemm_rows_configure() {
+    each_kernel([](auto kernel, int tmw, int tnw) {
+        hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes(tmw, tnw)), "hipFuncSetAttribute(k_gemm_q8_rows)");
+    });
+}
+
+// What the fp16 GEMM does not take: fewer than 256 rows without a copy of the weights in its layout (64 x 22016 over 4096 50 us,
+// 86 on the bf16 kernels), or few tiles, or a short K.  The rows' split into planes costs a launch.  Where they are normalised
+// first it takes that launch's place: 128 x 2048 over 2048 13.3 us against 17.9 on the bf16 kernels, 16 x 256 over 256 8.6, 9.6,
+// and only a multitude of rows against a small weight is better off there (700 x 768 over 256: 13.2, 11.8; 700 x 1536 over 512
+// 18.9, 20.9).  Where they are not, the weight has to be large enough to make up for it: 128 x 2048 over 2048 12.4, 14.1 and 30 x
+// 6144 over 2048 11.5, 16.1, but 16 x 2048 over 2048 11.8, 11.0 and 128 x 768 over 3072 14.6, 13.2.  A lane's offset into a
+// column tile's weights is 32 bits.
+bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared) {
+    if (k > (1 << 24) || q8_gemm_f16_shape_ok(m, n_rows, k, prepared)) return false;
+    const int64_t weights = (int64_t)n_rows * k;
+    return norm ? m <= 512 || weights >= 3 << 18 : weights >= (m > 32 ? 4 << 20 : 8 << 20);
+}
+
+// floats of workspace: planes, row factors, the partial products where K is shared
+int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, bool may_share) {
+    const int64_t m_pad = round_up(m, 32), ka = round_up(q8_padded_k(k), kOperandChunk);
+    const int shares = rows_plan(m, n_rows, k, may_share).shares;
+    return round_up(m_pad * ka, 64) + round_up(m_pad, 64) + (shares > 1 ? (int64_t)shares * m * n_rows : 0);
+}
+
+void launch_q8_gemm_rows(hipStream_t s, const float *x, const float *gamma, const float *beta, const int8_t *wq, const float *scales, float *out, int m, int k,
+                         int n_rows, const GemmEpilogue &ep, float *workspace, int64_t workspace_floats, bool may_share) {
+    if (workspace_floats < q8_gemm_rows_workspace_floats(m, n_rows, k, may_share)) fail("q8_gemm_rows: workspace too small");
+    if (ep.swiglu && ((n_rows & 1) || ep.residual || ep.gelu)) fail("q8_gemm_rows: the SwiGLU epilogue needs an even row count and takes no residual or GELU");
+    const RowsPlan p = rows_plan(m, n_rows, k, may_share);
+    const int kp = q8_padded_k(k), ka = (int)round_up(kp, kOperandChunk), m_pad = (int)round_up(m, 32);
+    const int m_tiles = (m + 32 * p.tmw - 1) / (32 * p.tmw), n_tiles = (n_rows + 32 * p.tnw - 1) / (32 * p.tnw);
+    float *w = workspace;
+    uint16_t *planes = reinterpret_cast<uint16_t *>(w); w += round_up((int64_t)m_pad * ka, 64);
+    float *unscale = w;                                  w += round_up(m_pad, 64);
+    launch_split_operand(s, x, gamma, beta, planes, unscale, m, m_pad, k, ka);
+    GemmRowsArgs a{reinterpret_cast<const uintx4 *>(planes), wq, scales, unscale, out, m, n_rows, kp / kQ8Group, m_tiles, n_tiles, ep, 0, nullptr};
+    dim3 grid((unsigned)((n_tiles + 7) / 8 * 8 * m_tiles));
+    if (p.shares > 1) {
+        a.share_chunks = (chunks_of(k) + p.shares - 1) / p.shares;
+        grid.z = (chunks_of(k) + a.share_chunks - 1) / a.share_chunks;
+        a.partial = w;
+    }
+    each_kernel([&](auto kernel, int tmw, int tnw) {
+        if (tmw == p.tmw && tnw == p.tnw) launch_kernel(kernel, grid, dim3(64 * kWaves), (size_t)lds_bytes(tmw, tnw), s, a);
+    });
+    if (p.shares > 1) launch_q8_sum_partials(s, w, out, (int)grid.z, m, n_rows, ep);
+}
+
+}  // namespace dj

@@ -17,6 +17,7 @@
 #include <cstdlib>
 #include "dj_common.h"
 #include "gemm_epilogue.h"
+#include "gemm_rows.h"
 
 namespace dj {
 
@@ -514,7 +515,7 @@ __global__ void __launch_bounds__(256 * KS) k_gemm_q8(const float *__restrict__ 
     }
 }
 
-// C = epilogue(sum over the splits of partial[z]) for the K-sharing launches of k_gemm_q8: the same bias / GELU /
+// C = epilogue(sum over the splits of partial[z]) for the K-sharing launches of k_gemm_q8 and k_gemm_q8_rows: the same bias / GELU /
 // residual / SwiGLU steps, in the same order, as the kernel's own epilogue (a fixed order of additions, so a run
 // repeats bit for bit - which adding into C with atomics would not).  One thread per column pair of a row.
 __global__ void __launch_bounds__(256) k_sum_partials_q8(const float *__restrict__ partial, float *__restrict__ C, int splits,
@@ -635,6 +636,11 @@ int64_t q8_gemm_workspace_floats(int m, int n_rows, int k) {
     return shares > 1 ? (int64_t)shares * m * n_rows : 0;
 }
 
+void launch_q8_sum_partials(hipStream_t s, const float *partial, float *out, int splits, int m, int n_rows, const GemmEpilogue &ep) {
+    const int64_t pairs = (int64_t)m * (n_rows / 2);
+    launch_kernel(k_sum_partials_q8, dim3((unsigned)std::min<int64_t>((pairs + 255) / 256, 4096)), dim3(256), 0, s, partial, out, splits, m, n_rows, ep);
+}
+
 // Q8 GEMM used by launch_q8_linear for M > 1.  n_rows is the number of Q8 rows
 // (= output columns of this launch; 2N for an interleaved gate/up weight).  workspace: room for the partial products
 // of a K-sharing launch (q8_gemm_workspace_floats), or less - then no K is shared.
@@ -667,9 +673,7 @@ void launch_q8_gemm(hipStream_t s, const float *x, const int8_t *wq, const float
         grid.z = shares;
         launch_kernel((k_gemm_q8<1, 1, kGroupsFew, kSetsFew>), grid, dim3(256 * kSetsFew), 0, s, x, wq, scales, out, m, n_rows, k, q8_padded_k(k), ep,
                       per * step, workspace);
-        const int64_t pairs = (int64_t)m * (n_rows / 2);
-        launch_kernel(k_sum_partials_q8, dim3((unsigned)std::min<int64_t>((pairs + 255) / 256, 4096)), dim3(256), 0, s, (const float *)workspace, out,
-                      shares, m, n_rows, ep);
+        launch_q8_sum_partials(s, workspace, out, shares, m, n_rows, ep);
         return;
     }
     // few tiles (about one per CU): a workgroup brings its own second wavefront per SIMD

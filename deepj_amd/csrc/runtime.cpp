@@ -29,6 +29,7 @@
 #include <sys/mman.h>
 
 #include "dj_common.h"
+#include "gemm_rows.h"
 
 namespace dj {
 
@@ -133,6 +134,7 @@ void ensure_init(int device = 0) {
     if (!g.static_scratch) fail("deepj_hip: the static scratch array has no device address");
     DJ_HIP(hipMemset(g.static_scratch, 0, kStaticCounterBytes));
     q8_gemm_f16_configure();
+    q8_gemm_rows_configure();
     latent_decode_configure();
     g.device = device;
     g.ready = true;

@@ -1,0 +1,110 @@
+"""The Q8 GEMM that multiplies a batch of rows straight from the int8 weights, through the C ABI against float64 on the
+oracle's dequantised weights, at the edges of its tiles (32 or 64 rows and columns), of its 128-k chunks and of the ways it
+deals them: one to four wavefronts with work, K shared by several workgroups, odd and ragged everything.
+
+Gate on the rms error of the whole product: an activation is held to 2^-23, and an output is at most four sums (one a
+wavefront) of G = K / 128 scaled group sums, whose n-th rounding is 2^-24 of a partial sum of n groups: 2^-23 (1 + sqrt(G / 2))
+of the product's rms covers both."""
+import numpy as np
+import pytest
+
+from deepj_amd import HipNative, JavaRandom
+from deepj_amd.fused import DeviceBuffers, Stream
+from oracle import cpu_ref as ref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = DeviceBuffers()
+    yield d
+    d.release_all()
+
+
+def check(got, exp, k, what, times=1):
+    size = np.sqrt(np.mean(exp ** 2, axis=1, keepdims=True))
+    assert not got[size[:, 0] == 0].any(), f"{what}: a row of zeros"
+    err = float(np.sqrt(np.mean(((got - exp) / np.where(size == 0, 1, size)) ** 2)))
+    assert err <= times * 2.0 ** -23 * (1 + np.sqrt(k / 256)), f"{what}: rms error {err:.2e}"
+
+
+def rms_normalised(x, gamma):
+    return x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-6) * gamma
+
+
+# (a small weight without a normalisation stays on the bf16 kernels.)  The last seven: K shared (few rows against a narrow
+# weight, long K), columns in pairs or not, and each of the wider tiles
+@pytest.mark.parametrize("m,k,n,norm", [(2, 32, 2, 1), (7, 31, 33, 1), (32, 128, 32, 1), (33, 129, 31, 1), (64, 160, 65, 1), (65, 416, 64, 1), (96, 512, 97, 1),
+                                        (31, 640, 127, 1), (30, 11008, 1024, 0), (30, 11008, 1023, 0), (5, 5600, 2050, 0), (200, 12300, 500, 0),
+                                        (40, 96, 50001, 0), (250, 288, 20002, 0), (200, 1028, 5002, 0)])
+def test_product_at_the_edges(dev, m, k, n, norm):
+    w, x, gamma = JavaRandom(5).tensor(k, n, k ** -0.5), JavaRandom(6).tensor(m, k, 1.0), JavaRandom(7).tensor(1, k, 1.0)
+    if m > 4:
+        x[1] = 0.0                                       # a row without a largest value
+        x[2] *= 1e-18                                    # rows far from one, which leave the others as they are
+        x[3] *= 1e15
+    src, wq, xb, ob, gb = dev.upload(w), dev.alloc(HipNative.q8Floats(k, n)), dev.upload(x), dev.alloc(m * n), dev.upload(gamma)
+    Stream().q8_quantize(src, wq, k, n).run()
+    op = Stream().q8_linear(xb, wq, ob, m, k, n, gamma=gb if norm else -1)
+    op.run()
+    got = dev.download(ob, (m, n)).copy()
+    op.run()
+    assert np.array_equal(got, dev.download(ob, (m, n)))                 # the same bits again
+    dev.release(src, wq, xb, ob, gb)
+    a = rms_normalised(x.astype(np.float64), gamma) if norm else x.astype(np.float64)
+    check(got, a @ ref.q8_roundtrip(w).astype(np.float64), k, f"{m} x {k} x {n}", times=1 + norm)
+
+
+@pytest.mark.parametrize("m,k,n", [(9, 200, 46), (64, 2052, 2100), (30, 8224, 1026)])
+@pytest.mark.parametrize("epilogue", ["bias_gelu_residual", "swiglu", "rms", "layernorm"])
+def test_prologues_and_epilogues(dev, m, k, n, epilogue):
+    sw = epilogue == "swiglu"
+    w, x = [JavaRandom(7 + i).tensor(k, n, k ** -0.5) for i in range(1 + sw)], JavaRandom(9).tensor(m, k, 1.0)
+    vec = [JavaRandom(10 + i).tensor(1, k if i > 1 else n, 0.5) for i in range(4)]
+    res = JavaRandom(15).tensor(m, n, 1.0)
+    wq, xb, ob, rb = dev.alloc(HipNative.q8Floats(k, n * (1 + sw))), dev.upload(x), dev.alloc(m * n), dev.upload(res)
+    vb = [dev.upload(v) for v in vec]
+    for i, wi in enumerate(w):
+        src = dev.upload(wi)
+        Stream().q8_quantize(src, wq, k, n, i, 1 + sw, n * (1 + sw)).run()
+        dev.release(src)
+    kw = {"bias_gelu_residual": dict(bias=vb[0], gelu=True, residual=rb), "swiglu": dict(swiglu=True, bias=vb[0], bias2=vb[1]),
+          "rms": dict(gamma=vb[2]), "layernorm": dict(gamma=vb[2], beta=vb[3], bias=vb[0])}[epilogue]
+    Stream().q8_linear(xb, wq, ob, m, k, n, **kw).run()
+    got = dev.download(ob, (m, n)).copy()
+    dev.release(wq, xb, ob, rb, *vb)
+    a, v, deq = x.astype(np.float64), [t.astype(np.float64) for t in vec], [ref.q8_roundtrip(wi).astype(np.float64) for wi in w]
+    if epilogue == "rms":
+        a = rms_normalised(a, v[2])
+    if epilogue == "layernorm":
+        c = a - a.mean(1, keepdims=True)
+        a = c / np.sqrt((c * c).mean(1, keepdims=True) + 1e-5) * v[2] + v[3]
+    y = a @ deq[0]
+    if epilogue == "bias_gelu_residual":
+        y = y + v[0]
+        y = res + 0.5 * y * (1 + np.tanh(0.7978845608 * (y + 0.044715 * y ** 3)))
+    if sw:
+        gate, up = y + v[0], a @ deq[1] + v[1]
+        y = gate / (1 + np.exp(-gate)) * up
+    if epilogue == "layernorm":
+        y = y + v[0]
+    # (the normalisations and activations add some roundings of their own: as much again)
+    check(got, y, k, epilogue, times=2)
+
+
+def test_a_row_that_is_not_finite_stays_alone(dev):
+    m, k, n = 40, 600, 8000
+    w, x = JavaRandom(5).tensor(k, n, 0.05), JavaRandom(6).tensor(m, k, 1.0)
+    src, wq, xb, ob = dev.upload(w), dev.alloc(HipNative.q8Floats(k, n)), dev.upload(x), dev.alloc(m * n)
+    op = Stream().q8_quantize(src, wq, k, n).q8_linear(xb, wq, ob, m, k, n)
+    op.run()
+    clean = dev.download(ob, (m, n)).copy()
+    x[3, 17], x[35, 599] = np.inf, np.nan
+    dev.write(xb, x)
+    op.run()
+    got = dev.download(ob, (m, n)).copy()
+    dev.release(src, wq, xb, ob)
+    assert not np.isfinite(got[[3, 35]]).any()
+    keep = [r for r in range(m) if r not in (3, 35)]
+    assert np.array_equal(got[keep], clean[keep])
