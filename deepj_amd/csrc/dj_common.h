@@ -144,6 +144,13 @@ void launch_q8_quantize(hipStream_t s, const float *w, int8_t *q, float *scales,
                         int row_step);
 void launch_q8_dequantize(hipStream_t s, const int8_t *q, const float *scales, float *w, int k, int n,
                           int row_off, int row_step);
+struct Q8LinearPair {                  // two weights over one RMS-normalised row
+    const float *x, *gamma;
+    const int8_t *wq[2]; const float *scales[2]; float *out[2];
+    int n[2], k;
+};
+bool q8_linear_pair_ok(int k);
+void launch_q8_linear_pair(hipStream_t s, const Q8LinearPair &p);
 void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_t workspace_floats);
 int64_t q8_linear_workspace_floats(int m, int k, int n, int flags);
 // The size at which launch_q8_linear takes its fastest path (>= the one above); callers that may grow their workspace

@@ -303,24 +303,17 @@ __device__ __forceinline__ void stage_digits(float *xs, int plane0, int shift_at
 // staging paths made the compiler merge their registers with copies placed right behind the first activation
 // load - a wait for it ahead of every weight load.
 template <int NC, int B, bool SWIGLU, int MODE, int PRO, bool VEC>
-__global__ void __launch_bounds__(kThreads)
-k_q8_matvec(const float *a_x, const int8_t *a_wq, const float *a_scales, float *a_out, int a_k, int a_grid, int a_n_out,
-            int a_rec_hd, const float *a_gamma, const float *a_bias, const float *a_bias2, const float *a_residual,
-            const float *a_beta) {
-    // (the grid size comes as an argument: gridDim.x is one more value fetched from the argument buffer)
-    const MatvecArgs p{a_x, a_wq, a_scales, a_out, a_k, (a_k + kQ8Group - 1) / kQ8Group * kQ8Group, a_n_out, a_gamma,
-                       a_bias, a_bias2, a_residual, a_beta, a_rec_hd};
+__device__ __forceinline__ void matvec(const MatvecArgs &p, float *xs, int block, int grid) {   // xs: the activation row, laid out by xs_at()
     constexpr bool GELU = MODE == 1;
     constexpr bool MERGE = MODE == 2;
     constexpr int NS = kAttnRecordSplits;
-    extern __shared__ __align__(16) float xs[];   // the activation row, laid out by xs_at() below
     __shared__ float red[kWaves], red2[kWaves];
     constexpr int RPO = SWIGLU ? 2 : 1;           // Q8 rows per output
     constexpr int R = B * RPO;                    // rows per batch
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int groups = p.kp / kQ8Group;
-    const int wave_global = blockIdx.x * kWaves + wave;
-    const int wave_count = a_grid * kWaves;
+    const int wave_global = block * kWaves + wave;
+    const int wave_count = grid * kWaves;
     // Batches are dealt round-robin: batch j of wave w is batch w + j*wave_count of the
     // matrix, so at any moment the rows in flight across the chip are neighbours in memory.
     const int n_batches = (p.n_out + B - 1) / B;
@@ -547,6 +540,32 @@ k_q8_matvec(const float *a_x, const int8_t *a_wq, const float *a_scales, float *
     DJ_STAMP(5);
 }
 
+template <int NC, int B, bool SWIGLU, int MODE, int PRO, bool VEC>
+__global__ void __launch_bounds__(kThreads)
+k_q8_matvec(const float *a_x, const int8_t *a_wq, const float *a_scales, float *a_out, int a_k, int a_grid, int a_n_out,
+            int a_rec_hd, const float *a_gamma, const float *a_bias, const float *a_bias2, const float *a_residual,
+            const float *a_beta) {
+    extern __shared__ __align__(16) float xs[];
+    // (the grid size comes as an argument: gridDim.x is one more value fetched from the argument buffer)
+    const MatvecArgs p{a_x, a_wq, a_scales, a_out, a_k, (a_k + kQ8Group - 1) / kQ8Group * kQ8Group, a_n_out, a_gamma,
+                       a_bias, a_bias2, a_residual, a_beta, a_rec_hd};
+    matvec<NC, B, SWIGLU, MODE, PRO, VEC>(p, xs, blockIdx.x, a_grid);
+}
+
+// Two weights over the same normalised row in one launch: a small matvec is bound by its launch and the first answer of memory,
+// and the second one's are the first one's here.  The latent models' down projections (d 2048, 1024 and 512 output rows; 4
+// layers): a token 176.5 -> 169.9 us, at d 1024 123.7 -> 115.6, at d 512 108.4 -> 100.3.
+template <int NC, int B>
+__global__ void __launch_bounds__(kThreads)
+k_q8_matvec_pair(const float *a_x, const int8_t *a_wq, const float *a_scales, float *a_out, int a_k, int a_grid, int a_n_out, const float *a_gamma,
+                 const int8_t *b_wq, const float *b_scales, float *b_out, int b_grid, int b_n_out) {
+    extern __shared__ __align__(16) float xs[];
+    const bool second = (int)blockIdx.x >= a_grid;
+    const MatvecArgs p{a_x, second ? b_wq : a_wq, second ? b_scales : a_scales, second ? b_out : a_out, a_k, (a_k + kQ8Group - 1) / kQ8Group * kQ8Group,
+                       second ? b_n_out : a_n_out, a_gamma, nullptr, nullptr, nullptr, nullptr, 0};
+    matvec<NC, B, false, 0, 1, true>(p, xs, second ? blockIdx.x - a_grid : blockIdx.x, second ? b_grid : a_grid);
+}
+
 constexpr int kMvGridCap = 768;          // three workgroups per CU
 constexpr int kMvGridCapWide = 1024;     // four for the widest matrices (the LM head: two batches per wavefront instead of three, 14.7 -> 14.0 us)
 inline int mv_grid_cap() { return kMvGridCap; }
@@ -681,6 +700,33 @@ int64_t q8_linear_preferred_workspace_floats(int m, int k, int n, int flags, boo
     if (!mv && q8_gemm_f16_shape_ok(m, n_rows, k, prepared)) return std::max(ws, q8_gemm_f16_workspace_floats(m, n_rows, k, prepared));
     if (!mv) return ws + q8_gemm_workspace_floats(m, n_rows, k);      // the partial products of a K-sharing launch
     return ws;
+}
+
+bool q8_linear_pair_ok(int k) { return k > 0 && (k & 3) == 0 && k <= 4096; }
+
+void launch_q8_linear_pair(hipStream_t s, const Q8LinearPair &p) {
+    if (!q8_linear_pair_ok(p.k)) fail("q8_linear_pair: shape outside this kernel's range");
+    auto go = [&](auto nc, auto b) {
+        constexpr int NC = decltype(nc)::value, B = decltype(b)::value;
+        int grid[2];
+        const int per = B * kWaves, all = (p.n[0] + per - 1) / per + (p.n[1] + per - 1) / per, rounds = (all + mv_grid_cap() - 1) / mv_grid_cap();
+        for (int i = 0; i < 2; i++) grid[i] = (p.n[i] + per * rounds - 1) / (per * rounds);
+        launch_kernel(k_q8_matvec_pair<NC, B>, dim3(grid[0] + grid[1]), dim3(kThreads), (size_t)xs_floats(q8_padded_k(p.k)) * sizeof(float), s, p.x, p.wq[0],
+                      p.scales[0], p.out[0], p.k, grid[0], p.n[0], p.gamma, p.wq[1], p.scales[1], p.out[1], grid[1], p.n[1]);
+    };
+    // Two rows a wavefront once one a wavefront is more than a workgroup per compute unit: a token of the 4-layer model below 171.6
+    // us with one (384 workgroups), 169.9 with two.
+    const int nc = (q8_padded_k(p.k) + 1023) / 1024;
+    auto rows = [&](auto c) {
+        if (p.n[0] + p.n[1] > 256 * kWaves) go(c, std::integral_constant<int, 2>{});
+        else go(c, std::integral_constant<int, 1>{});
+    };
+    switch (nc) {
+        case 1: rows(std::integral_constant<int, 1>{}); break;
+        case 2: rows(std::integral_constant<int, 2>{}); break;
+        case 3: rows(std::integral_constant<int, 3>{}); break;
+        default: rows(std::integral_constant<int, 4>{}); break;
+    }
 }
 
 void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_t workspace_floats) {

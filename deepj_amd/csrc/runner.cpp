@@ -404,9 +404,12 @@ void block_stream(Runner &r, Stream &s, Acts &a, int l, int S) {
         // on Q, attention over the token-major rows (MultiHeadLatentAttention.java:92-123).
         const int qr = c.q_rank, kvr = c.kv_rank;
         const int64_t lat_off = (int64_t)l * c.max_seq * kvr;
-        q8_linear(s, a.x, L.wdq, a.cq, S, d, qr, DJ_LIN_RMSNORM, L.g1);
+        if (S == 1 && (d & 3) == 0 && d <= 4096) emit(s, DJ_OP_Q8_LINEAR_PAIR, a.x, L.g1, d, L.wdq, a.cq, qr, L.wdkv, a.ckv, kvr);
+        else {
+            q8_linear(s, a.x, L.wdq, a.cq, S, d, qr, DJ_LIN_RMSNORM, L.g1);
+            q8_linear(s, a.x, L.wdkv, a.ckv, S, d, kvr, DJ_LIN_RMSNORM, L.g1);
+        }
         q8_linear(s, a.cq, L.wuq, a.qkv, S, qr, d, 0);
-        q8_linear(s, a.x, L.wdkv, a.ckv, S, d, kvr, DJ_LIN_RMSNORM, L.g1);
         const int splits = S == 1 ? deepj_hip_latent_decode_splits(H, hd, kvr, c.max_seq) : 0;
         if (splits) {        // one row: the cache stays latent (its scratch holds the splits' records)
             emit(s, DJ_OP_LATENT_DECODE, a.qkv, a.ckv, r.latent, L.wukv, r.state, r.cos_t, r.sin_t, r.scratch, a.att, H, hd, kvr, c.max_seq, l);

@@ -548,6 +548,7 @@ int stride_of(int op) {
         case DJ_OP_DECODE_FFN: return 16;
         case DJ_OP_DECODE_ROW: return 7;
         case DJ_OP_LATENT_DECODE: return 15;
+        case DJ_OP_Q8_LINEAR_PAIR: return 10;
         default: return -1;
     }
 }
@@ -1157,6 +1158,21 @@ void exec_one(Cursor &c) {
             if (run) launch_latent_decode(s, a);
             break;
         }
+        case DJ_OP_Q8_LINEAR_PAIR: {
+            // [op, x, gamma, K, weightA, outA, nA, weightB, outB, nB]
+            const int64_t k = w[3];
+            if (k > (1 << 20) || !q8_linear_pair_ok((int)k) || w[6] <= 0 || w[9] <= 0) fail("OP_Q8_LINEAR_PAIR: bad shape");
+            Q8LinearPair p{};
+            p.x = buf(w[1], k, op, "x"); p.gamma = buf(w[2], k, op, "gamma"); p.k = (int)k;
+            for (int i = 0; i < 2; i++) {
+                p.n[i] = w[6 + 3 * i];
+                q8_weight(w[4 + 3 * i], k, p.n[i], op, "weight", p.wq[i], p.scales[i]);
+                p.out[i] = buf(w[5 + 3 * i], p.n[i], op, "out");
+            }
+            if (p.out[0] == p.out[1] || p.out[0] == p.x || p.out[1] == p.x) fail("OP_Q8_LINEAR_PAIR: every out needs a buffer of its own");
+            if (run) launch_q8_linear_pair(s, p);
+            break;
+        }
         case DJ_OP_APPEND_ROWS: {
             // [op, src, dst, state, rows, rowFloats, maxRows, dstOff]: dst[dstOff + (state[0]+i)*rowFloats ..] = src row i
             int64_t rows = w[4], rf = w[5], max_rows = w[6], off = w[7];
@@ -1297,6 +1313,7 @@ const char *op_name(int op) {
         case DJ_OP_DECODE_FFN: return "OP_DECODE_FFN";
         case DJ_OP_DECODE_ROW: return "OP_DECODE_ROW";
         case DJ_OP_LATENT_DECODE: return "OP_LATENT_DECODE";
+        case DJ_OP_Q8_LINEAR_PAIR: return "OP_Q8_LINEAR_PAIR";
         case DJ_OP_ATTN_DECODE: return "OP_ATTN_DECODE";
         case DJ_OP_APPEND_ROWS: return "OP_APPEND_ROWS";
         case DJ_OP_Q8_LINEAR_DYN: return "OP_Q8_LINEAR_DYN";

@@ -148,6 +148,9 @@ class Stream:
     def latent_decode(self, q, ckv, latent, wukv, state, cos, sin, records, out, H, hd, rank, max_seq, layer):
         return self.emit(op.OP_LATENT_DECODE, q, ckv, latent, wukv, state, cos, sin, records, out, H, hd, rank, max_seq, layer)
 
+    def q8_linear_pair(self, x, gamma, k, w_a, out_a, n_a, w_b, out_b, n_b):
+        return self.emit(op.OP_Q8_LINEAR_PAIR, x, gamma, k, w_a, out_a, n_a, w_b, out_b, n_b)
+
     def decode_row(self, x, part, n_part, bias, out, d):
         return self.emit(op.OP_DECODE_ROW, x, part, n_part, bias, out, d)
 

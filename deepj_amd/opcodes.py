@@ -75,6 +75,7 @@ OP_DECODE_ATTN = 91        # a narrow model's block for one token in two launche
 OP_DECODE_FFN = 92
 OP_DECODE_ROW = 93         # the row behind the last block
 OP_LATENT_DECODE = 94      # one token's attention over a latent KV cache that stays latent
+OP_Q8_LINEAR_PAIR = 95     # two weights over one normalised row
 
 LIN_RMSNORM = 1
 LIN_BIAS = 2
@@ -92,4 +93,4 @@ FUSED_STRIDES = {OP_Q8_QUANTIZE: 8, OP_Q8_DEQUANTIZE: 8, OP_Q8_LINEAR: 12, OP_RM
                  OP_COPY: 6, OP_FILL: 4, OP_ROPE_ROWS: 13, OP_ATTENTION_KV: 14, OP_DECODE_NEXT: 10, OP_ATTN_DECODE: 13,
                  OP_APPEND_ROWS: 8, OP_Q8_LINEAR_DYN: 10, OP_LAYERNORM: 7, OP_ADD_POSITIONS: 7,
                  OP_ATTN_DECODE_RECORDS: 12, OP_STREAM_READ: 4, OP_NOP: 2, OP_Q8_PREPARE: 5, OP_Q8_LINEAR_ROPE: 20, OP_DECODE_SAMPLE: 11,
-                 OP_DECODE_ATTN: 20, OP_DECODE_FFN: 16, OP_DECODE_ROW: 7, OP_LATENT_DECODE: 15}
+                 OP_DECODE_ATTN: 20, OP_DECODE_FFN: 16, OP_DECODE_ROW: 7, OP_LATENT_DECODE: 15, OP_Q8_LINEAR_PAIR: 10}

@@ -238,6 +238,8 @@ enum {
      *     rows of `latent` [layers][maxSeq][rank] at position state[0]; out [H * hd] = attention of q (not rotated) over
      *     K = RoPE(rows . Wuk) and V = rows . Wuv, wukv a Q8 weight with the 2 * H * hd output rows Wuk, Wuv.  records: scratch
      *     of H * deepj_hip_latent_decode_splits(H, hd, rank, maxSeq) * (hd + 4) floats; refused where that is 0.
+     * Q8_LINEAR_PAIR [op, x, gamma, K, weightA, outA, nA, weightB, outB, nB]
+     *     two Q8_LINEARs of one row with the same x and RMSNorm gain in one launch, the same bits; K a multiple of 4 up to 4096
      */
     DJ_OP_Q8_QUANTIZE = 64, DJ_OP_Q8_DEQUANTIZE = 65, DJ_OP_Q8_LINEAR = 66, DJ_OP_RMSNORM = 67,
     DJ_OP_SILU_MUL = 68, DJ_OP_EMBED_GATHER = 69, DJ_OP_ROPE_KV_STORE = 70, DJ_OP_ATTENTION = 71,
@@ -246,7 +248,7 @@ enum {
     DJ_OP_APPEND_ROWS = 80, DJ_OP_Q8_LINEAR_DYN = 81, /* 82 unused */ DJ_OP_LAYERNORM = 83,
     DJ_OP_ADD_POSITIONS = 84, DJ_OP_ATTN_DECODE_RECORDS = 85, DJ_OP_STREAM_READ = 86, DJ_OP_NOP = 87, DJ_OP_Q8_PREPARE = 88,
     DJ_OP_Q8_LINEAR_ROPE = 89, DJ_OP_DECODE_SAMPLE = 90,
-    DJ_OP_DECODE_ATTN = 91, DJ_OP_DECODE_FFN = 92, DJ_OP_DECODE_ROW = 93, DJ_OP_LATENT_DECODE = 94
+    DJ_OP_DECODE_ATTN = 91, DJ_OP_DECODE_FFN = 92, DJ_OP_DECODE_ROW = 93, DJ_OP_LATENT_DECODE = 94, DJ_OP_Q8_LINEAR_PAIR = 95
 };
 
 /* Largest top_k that DECODE_SAMPLE takes. */

@@ -235,3 +235,29 @@ def test_latent_ops_reject_bad_streams(dev):
         Stream().q8_linear_dyn(a, w, a, 4, 32, 4, st, 1, 0).run()         # x holds 64 floats, 4 rows of 32 need 128
     with pytest.raises(RuntimeError, match="bad shape"):
         Stream().q8_linear_dyn(a, w, a, 1, 32, 4, st, -1, 0).run()
+
+
+@pytest.mark.parametrize("k,na,nb", [(4, 1, 3), (1000, 5, 700), (1024, 2000, 1), (2048, 1024, 512), (2052, 3072, 130), (4096, 9, 13000)])
+def test_a_pair_of_weights_in_one_launch_gives_the_bits_of_two(k, na, nb):
+    """One and two rows a wavefront, every chunk count of K, weights that end inside a workgroup."""
+    dev = DeviceBuffers()
+    try:
+        rng = np.random.default_rng(k)
+        x, g = dev.upload(rng.standard_normal(k, dtype=np.float32)), dev.upload(rng.standard_normal(k, dtype=np.float32))
+        w, one, two = [], [dev.alloc(na), dev.alloc(nb)], [dev.alloc(na), dev.alloc(nb)]
+        s = Stream()
+        for n in (na, nb):
+            src = dev.upload(rng.standard_normal((k, n), dtype=np.float32))
+            w.append(dev.alloc(HipNative.q8Floats(k, n)))
+            s.q8_quantize(src, w[-1], k, n)
+        for i, n in enumerate((na, nb)):
+            s.q8_linear(x, w[i], two[i], 1, k, n, gamma=g)
+        s.q8_linear_pair(x, g, k, w[0], one[0], na, w[1], one[1], nb).run()
+        for i, n in enumerate((na, nb)):
+            assert np.array_equal(dev.download(one[i], (n,)).view(np.int32), dev.download(two[i], (n,)).view(np.int32))
+        for bad in (dict(k=k + 1), dict(out_b=one[0]), dict(out_a=x), dict(n_a=0), dict(k=4100)):
+            args = dict(dict(x=x, gamma=g, k=k, w_a=w[0], out_a=one[0], n_a=na, w_b=w[1], out_b=one[1], n_b=nb), **bad)
+            with pytest.raises(Exception, match="OP_Q8_LINEAR_PAIR"):
+                Stream().q8_linear_pair(**args).run()
+    finally:
+        dev.release_all()
