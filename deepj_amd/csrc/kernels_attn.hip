@@ -278,17 +278,39 @@ __global__ void __launch_bounds__(256) k_attention_tiled(AttnKernelArgs a) {
     const int vslot = 16 * (vkp >> 3) + 8 * ((vkp >> 1) & 1) + 4 * ((vkp >> 2) & 1) + 2 * (vkp & 1);
     const int k_first = SHARE ? (int)blockIdx.z * KT * KSETS : 0;
     const int k_stride = SHARE ? (int)gridDim.z * KT * KSETS : KT * KSETS;
+    // One or two key sets: the rows a round stages are requested a round ahead and fly while this one's products run (32 heads
+    // of 128 x 2048 rows 262 -> 241 us, 32 of 64 x 1024 55.6 -> 54.3).  Four sets have too many rows to hold for it (12 heads of
+    // 64 x 400 rows 18.1 -> 19.0, 24 x 200 11.6 -> 12.3).
+    constexpr bool AHEAD = KSETS <= 2;
+    constexpr int PART = HD / 8;
+    typedef float floatx4 __attribute__((ext_vector_type(4)));
+    floatx4 kreg[KSETS][PART / 4], vreg[PVB ? 1 : KSETS][PVB ? 1 : PART / 4];
+    auto request_keys = [&](int k0, int ks) __attribute__((always_inline)) {       // rows past the last key repeat it (masked below)
+        const float *kr = kbase + (int64_t)min(k0 + ks * KT + (t & 31), wg_last) * a.tok_stride + (t >> 5) * PART;
+#pragma unroll
+        for (int j = 0; j < PART; j += 4) kreg[ks][j / 4] = *reinterpret_cast<const floatx4 *>(kr + j);
+    };
+    auto request_values = [&](int k0, int ks) __attribute__((always_inline)) {
+        const float *vr = vbase + (int64_t)min(k0 + ks * KT + (t >> 3), wg_last) * a.tok_stride + (t & 7) * PART;
+#pragma unroll
+        for (int j = 0; j < PART; j += 4) vreg[ks][j / 4] = *reinterpret_cast<const floatx4 *>(vr + j);
+    };
+    auto request = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ks = 0; ks < KSETS; ks++) {
+            request_keys(k0, ks);
+            if constexpr (!PVB) request_values(k0, ks);
+        }
+    };
+    if (AHEAD && k_first <= wg_last) request(k_first);
     for (int k0 = k_first; k0 <= wg_last; k0 += k_stride) {
 #pragma unroll
         for (int ks = 0; ks < KSETS; ks++) {
-            // stage the key tile as bf16 planes and the value tile; rows past the last key repeat it (masked below)
-            constexpr int PART = HD / 8;
-            int key = k0 + ks * KT + (t & 31);
-            if (key > wg_last) key = wg_last;
-            const float *kr = kbase + (int64_t)key * a.tok_stride + (t >> 5) * PART;
+            // stage the key tile as bf16 planes
+            if constexpr (!AHEAD) request_keys(k0, ks);
 #pragma unroll
             for (int j = 0; j < PART; j += 4) {
-                float4 v = *reinterpret_cast<const float4 *>(kr + j);
+                const floatx4 v = kreg[ks][j / 4];
                 const int c = (t >> 5) * PART + j;                                       // first of four elements of the row
                 const int at = ((((c >> 3) ^ (t & 31)) & (CH - 1)) << 3) + (c & 7);       // chunk c / 8 lives at (c / 8) ^ key
                 uint32_t hi[2], mid[2], lo[2];
@@ -303,13 +325,9 @@ __global__ void __launch_bounds__(256) k_attention_tiled(AttnKernelArgs a) {
         if constexpr (!PVB) {
 #pragma unroll
             for (int ks = 0; ks < KSETS; ks++) {
-                constexpr int PART = HD / 8;
-                int vkey = k0 + ks * KT + (t >> 3);
-                if (vkey > wg_last) vkey = wg_last;
-                const float *vr = vbase + (int64_t)vkey * a.tok_stride + (t & 7) * PART;
+                if constexpr (!AHEAD) request_values(k0, ks);
 #pragma unroll
-                for (int j = 0; j < PART; j += 4)
-                    *reinterpret_cast<float4 *>(&Vs[ks][t >> 3][(t & 7) * PART + j]) = *reinterpret_cast<const float4 *>(vr + j);
+                for (int j = 0; j < PART; j += 4) *reinterpret_cast<floatx4 *>(&Vs[ks][t >> 3][(t & 7) * PART + j]) = vreg[ks][j / 4];
             }
         }
 #pragma unroll
@@ -324,7 +342,8 @@ __global__ void __launch_bounds__(256) k_attention_tiled(AttnKernelArgs a) {
                 vb[ks][rep] = *reinterpret_cast<const float4 *>(vbase + (int64_t)key_b * a.tok_stride + j0);
             }
         }
-        __syncthreads();
+        if (AHEAD && k0 + k_stride <= wg_last) request(k0 + k_stride);
+        lds_barrier();                                      // (__syncthreads would wait for what was just requested)
         const int kb0 = k0 + kset * KT;                     // this wavefront's tile of the round
         const bool active = kb0 <= wave_last;               // wave-uniform
         floatx16 st;
@@ -381,7 +400,7 @@ __global__ void __launch_bounds__(256) k_attention_tiled(AttnKernelArgs a) {
                 }
             }
         }
-        __syncthreads();                                    // every wavefront has read its keys (PVB: the bytes now take the values)
+        lds_barrier();                                    // every wavefront has read its keys (PVB: the bytes now take the values)
         if constexpr (!PVB) continue;
 #pragma unroll
         for (int ks = 0; ks < (PVB ? KSETS : 0); ks++) {
@@ -401,7 +420,7 @@ __global__ void __launch_bounds__(256) k_attention_tiled(AttnKernelArgs a) {
                 }
             }
         }
-        __syncthreads();
+        lds_barrier();
         if (active) {
             // O^T += V^T . P: the k slots of product mm are the keys the lane holds in st[8 mm .. 8 mm + 7]
 #pragma unroll
@@ -427,7 +446,7 @@ __global__ void __launch_bounds__(256) k_attention_tiled(AttnKernelArgs a) {
                 }
             }
         }
-        __syncthreads();
+        lds_barrier();
     }
     if constexpr (KSETS > 1) {
         // merge the key sets' states of the same queries: every set but the first parks (m, l, acc) lane by lane,
