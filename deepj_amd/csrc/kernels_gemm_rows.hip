@@ -13,9 +13,9 @@
 // loads return in the order they were asked for, so waiting for activations that were asked for after a chunk is waiting for
 // the chunk.  The matrix cores' 32 cycles a product hide the group before's scaling and the next one's conversion.
 //
-// What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 38 us with the split, 87 on the bf16
+// What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 32 us with the split, 87 on the bf16
 // kernels; 4.6 TB/s in the K loop), then the activations, which every tile reads anew from L2 (8 KB for every 64 x 64 x 32:
-// 64 x 22016 51 us, 86; 200 x 11264 over 2048 41, 67), and on small weights two launches' latency (30 x 2304 over 768 9.7 us,
+// 64 x 22016 43 us, 86; 200 x 11264 over 2048 41, 67), and on small weights two launches' latency (30 x 2304 over 768 9.7 us,
 // 11.9).  Tried and slower: eight wavefronts a workgroup (two workgroups of four fill a compute unit better: 64 x 22016 54 us
 // against 49), the K loop or the epilogue rolled (3 % and 10 %), a 64 x 64 tile whose wavefronts share the activations through
 // LDS (latency of its reads and barriers: 400 x 768 over 3072 34 us against 22).
@@ -39,7 +39,8 @@ namespace {
 
 constexpr int kWaves = 4;
 constexpr int kChunk = kOperandChunk / kQ8Group;                   // scale groups a wavefront takes at a time: 128 k, one line of a weight row
-constexpr int slot_bytes(int tnw) { return 32 * tnw * 128 + kChunk * 256; }       // a wavefront's chunk in LDS: weights [column][128], scales [group][64]
+constexpr int scale_row(int tnw) { return tnw > 2 ? 512 : 256; }
+constexpr int slot_bytes(int tnw) { return 32 * tnw * 128 + kChunk * scale_row(tnw); }       // a wavefront's chunk in LDS: weights [column][128], scales [group][64 or 128]
 
 struct GemmRowsArgs {
     const uintx4 *planes;        // activations in operand order (rows_plane_at)
@@ -63,7 +64,7 @@ __device__ __forceinline__ void int8x4_to_half(uint32_t r, uint32_t &lo, uint32_
 }
 
 template <int TMW, int TNW>
-__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) k_gemm_q8_rows(const GemmRowsArgs a) {
+__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(TMW * TNW > 4 ? 1 : 2, 2))) k_gemm_q8_rows(const GemmRowsArgs a) {
     constexpr int TN = 32 * TNW, NL = TN / 8;          // NL: loads a wavefront makes for a chunk of its TN weight rows
     constexpr int kSlot = slot_bytes(TNW);
     extern __shared__ __align__(16) unsigned char lds[];
@@ -90,7 +91,9 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     uint32_t b_off[NL];
 #pragma unroll
     for (int i = 0; i < NL; i++) b_off[i] = (uint32_t)min(8 * i + (lane >> 3), a.n - 1 - n0) * (uint32_t)kp + b_piece;
+    constexpr int kScaleRow = scale_row(TNW);
     const uint32_t s_off = (uint32_t)min(min(lane, TN - 1), a.n - 1 - n0) * (uint32_t)a.groups * 4u;
+    const uint32_t s_off2 = (uint32_t)min(min(64 + lane, TN - 1), a.n - 1 - n0) * (uint32_t)a.groups * 4u;
     const uint32_t q_at = l32 * 128, q_x = l32 & 7;
     const uintx4 *ap[TMW];
 #pragma unroll
@@ -102,12 +105,16 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
         for (int i = 0; i < NL; i++) load_to_lds16(b_base + (int64_t)c * (kChunk * kQ8Group), b_off[i] - back, dst + i * 1024);
 #pragma unroll
-        for (int g = 0; g < kChunk; g++) load_to_lds4(s_base + min(c * kChunk + g, a.groups - 1), s_off, dst + TN * 128 + g * 256);
+        for (int g = 0; g < kChunk; g++) {
+            const float *at = s_base + min(c * kChunk + g, a.groups - 1);
+            load_to_lds4(at, s_off, dst + TN * 128 + g * kScaleRow);
+            if constexpr (TN > 64) load_to_lds4(at, s_off2, dst + TN * 128 + g * kScaleRow + 256);
+        }
     };
     constexpr int NA = TMW == 1 ? 4 : 2;               // groups of activations in flight
     uintx4 av[NA][TMW][4];                             // [group % NA][row tile]: low pieces of the two k steps, high pieces
     auto fetch_a = [&](int i, int j, int g) __attribute__((always_inline)) { return (ap[i] + (int64_t)g * 256)[64 * (2 * (j & 1) + (j < 2)) + lane]; };
-    constexpr int NS = 4 / (TMW * TNW);                // sets of sums: a group's goes to set group % NS
+    constexpr int NS = TMW * TNW > 4 ? 1 : 4 / (TMW * TNW);       // sets of sums: a group's goes to set group % NS
     floatx16 acc[NS][TMW][TNW], p[2];
 #pragma unroll
     for (int e = 0; e < 16; e++) {
@@ -123,7 +130,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     uintx4 q[2];                                       // ... and as bytes, up to two stages ahead
     float sc[4] = {0.f, 0.f, 0.f, 0.f};                // their scales: of the stage before, this one and the two next
     auto read_q = [&](int slot, int g, int tn, int at, int at_sc) __attribute__((always_inline)) {
-        sc[at_sc] = *reinterpret_cast<const float *>(wl + slot * kSlot + TN * 128 + g * 256 + (32 * tn + l32) * 4);
+        sc[at_sc] = *reinterpret_cast<const float *>(wl + slot * kSlot + TN * 128 + g * kScaleRow + (32 * tn + l32) * 4);
         q[at] = *reinterpret_cast<const uintx4 *>(wl + slot * kSlot + 4096 * tn + q_at + (((2 * g + half) ^ q_x) << 4));
     };
     int c = c_begin + wave, slot = 0;
@@ -140,7 +147,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
         for (int w = 0; w < 4; w++) int8x4_to_half(q[0][w], bw[0][2 * w], bw[0][2 * w + 1]);
         read_q(0, 1 / TNW, 1 % TNW, 1, 2);
-        constexpr int S = kChunk * TNW, kAhead = 2 / TNW;     // stages of a chunk; groups in two stages
+        constexpr int S = kChunk * TNW, kAhead = TNW == 1 ? 2 : 1;      // stages of a chunk; groups two stages reach ahead, whole or begun
 #pragma unroll 1
         for (; c < c_end; c += kWaves, slot ^= 1) {
             const int next = min(c + kWaves, c_end - 1);
@@ -151,9 +158,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
                 // two stages on is the next chunk: its weights were asked for before the activations of the groups since
                 if (st == S - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((4 - kAhead) * 4 * TMW) : "memory");
                 const uintx4 qn = q[(st + 1) & 1];
-                const bool wrap = st + 2 >= S;
-                const int g2 = (g + kAhead) % kChunk;
-                read_q(wrap ? slot ^ 1 : slot, g2, tn, st & 1, (st + 3) & 3);
+                const int st2 = (st + 2) % S;
+                read_q(st + 2 >= S ? slot ^ 1 : slot, st2 / TNW, st2 % TNW, st & 1, (st + 3) & 3);
 #pragma unroll
                 for (int tm = 0; tm < TMW; tm++) {
                     const int u = st * TMW + tm;
@@ -256,6 +262,7 @@ constexpr int lds_bytes(int tmw, int tnw) {
 
 template <typename F> void each_kernel(F f) {
     f(k_gemm_q8_rows<1, 1>, 1, 1); f(k_gemm_q8_rows<1, 2>, 1, 2); f(k_gemm_q8_rows<2, 1>, 2, 1); f(k_gemm_q8_rows<2, 2>, 2, 2);
+    f(k_gemm_q8_rows<1, 3>, 1, 3); f(k_gemm_q8_rows<2, 3>, 2, 3);
 }
 
 int chunks_of(int k) { return (q8_padded_k(k) / kQ8Group + kChunk - 1) / kChunk; }
@@ -263,15 +270,17 @@ int chunks_of(int k) { return (q8_padded_k(k) / kQ8Group + kChunk - 1) / kChunk;
 // A tile's rows and columns in units of 32 and the workgroups that share its K: those of least estimated time, in us.  With x
 // tiles a compute unit and kk thousand k a wavefront, a launch takes
 //   fixed + per_x x + kk (per_k + again (rounds - 1) + per_kx x) + slabs m n shares / 10^6,
-// rounds being 1 up to one tile a compute unit, 2 up to two (two workgroups fit one) and x beyond.  Fitted to 155 shapes of 4 to
+// rounds being 1 up to one tile a compute unit, 2 up to two (two workgroups fit one) and x beyond.  Fitted to 239 shapes of 4 to
 // 512 rows, 768 to 50257 columns and 256 to 11008 k: the choice takes 1.01 times the best one's time on average.  (200 x 2304
-// over 768: 32 x 32 13.4 us, 32 x 64 15.8, 64 x 32 15.3, 64 x 64 15.6; 200 x 11008 over 4096: 53, 44, 48, 41; 4 x 4096 over
-// 11008: 32 x 32 31, K shared by two 25, by four 27.)
+// over 768: 32 x 32 13.4 us, 32 x 64 15.8, 64 x 32 15.3, 64 x 64 15.6; 200 x 11264 over 2048: 53, 44, 48, 41; 64 x 22016 over
+// 4096: 63, 49, 54, 50, and 43 with 64 x 96, whose 230 tiles are one round where 64 x 64 makes 344; 4 x 4096 over 11008:
+// 32 x 32 31, K shared by two 25, by four 27.)
 struct RowsPlan { int tmw, tnw, shares; };
 RowsPlan rows_plan(int m, int n_rows, int k, bool may_share) {
     struct Shape { int tmw, tnw, shares; double fixed, per_x, per_k, again, per_kx, slabs; };
     static const Shape shapes[] = {{1, 1, 1, 8.29, 0.27, 1.63, 1.29, 0.91, 0.0}, {1, 2, 1, 8.65, 0.87, 2.59, 1.63, 1.5, 0.0},
                                    {2, 1, 1, 8.12, 0.31, 2.51, 1.72, 1.63, 0.0}, {2, 2, 1, 9.76, 1.37, 3.49, 2.53, 2.2, 0.0},
+                                   {1, 3, 1, 6.77, 4.03, 4.46, 3.91, 1.01, 0.0}, {2, 3, 1, 6.39, 7.45, 6.26, 6.74, 0.93, 0.0},
                                    {1, 1, 2, 10.39, 0.6, 1.49, 1.12, 0.8, 2.24}, {1, 1, 4, 9.63, 1.19, 2.91, 1.57, -0.04, 1.12}};
     RowsPlan best{};
     double least = -1.0;
@@ -295,7 +304,7 @@ void q8_gemm_rows_configure() {
     });
 }
 
-// What the fp16 GEMM does not take: fewer than 256 rows without a copy of the weights in its layout (64 x 22016 over 4096 50 us,
+// What the fp16 GEMM does not take: fewer than 256 rows without a copy of the weights in its layout (64 x 22016 over 4096 43 us,
 // 86 on the bf16 kernels), or few tiles, or a short K.  The rows' split into planes costs a launch.  Where they are normalised
 // first it takes that launch's place: 128 x 2048 over 2048 13.3 us against 17.9 on the bf16 kernels, 16 x 256 over 256 8.6, 9.6,
 // and only a multitude of rows against a small weight is better off there (700 x 768 over 256: 13.2, 11.8; 700 x 1536 over 512

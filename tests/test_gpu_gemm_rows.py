@@ -33,11 +33,11 @@ def rms_normalised(x, gamma):
     return x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-6) * gamma
 
 
-# (a small weight without a normalisation stays on the bf16 kernels.)  The last seven: K shared (few rows against a narrow
+# (a small weight without a normalisation stays on the bf16 kernels.)  The last nine: K shared (few rows against a narrow
 # weight, long K), columns in pairs or not, and each of the wider tiles
 @pytest.mark.parametrize("m,k,n,norm", [(2, 32, 2, 1), (7, 31, 33, 1), (32, 128, 32, 1), (33, 129, 31, 1), (64, 160, 65, 1), (65, 416, 64, 1), (96, 512, 97, 1),
                                         (31, 640, 127, 1), (30, 11008, 1024, 0), (30, 11008, 1023, 0), (5, 5600, 2050, 0), (200, 12300, 500, 0),
-                                        (40, 96, 50001, 0), (250, 288, 20002, 0), (200, 1028, 5002, 0)])
+                                        (40, 96, 50001, 0), (250, 288, 20002, 0), (200, 1028, 5002, 0), (30, 1100, 24497, 0), (50, 1100, 24497, 0)])
 def test_product_at_the_edges(dev, m, k, n, norm):
     w, x, gamma = JavaRandom(5).tensor(k, n, k ** -0.5), JavaRandom(6).tensor(m, k, 1.0), JavaRandom(7).tensor(1, k, 1.0)
     if m > 4:
