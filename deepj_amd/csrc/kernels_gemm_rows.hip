@@ -13,9 +13,9 @@
 // loads return in the order they were asked for, so waiting for activations that were asked for after a chunk is waiting for
 // the chunk.  The matrix cores' 32 cycles a product hide the group before's scaling and the next one's conversion.
 //
-// What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 32 us with the split, 87 on the bf16
+// What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 29 us with the split, 87 on the bf16
 // kernels; 4.6 TB/s in the K loop), then the activations, which every tile reads anew from L2 (8 KB for every 64 x 64 x 32:
-// 64 x 22016 43 us, 86; 200 x 11264 over 2048 41, 67), and on small weights two launches' latency (30 x 2304 over 768 9.7 us,
+// 64 x 22016 41 us, 86; 200 x 11264 over 2048 41, 67), and on small weights two launches' latency (30 x 2304 over 768 9.2 us,
 // 11.9).  Tried and slower: eight wavefronts a workgroup (two workgroups of four fill a compute unit better: 64 x 22016 54 us
 // against 49), the K loop or the epilogue rolled (3 % and 10 %), a 64 x 64 tile whose wavefronts share the activations through
 // LDS (latency of its reads and barriers: 400 x 768 over 3072 34 us against 22).
@@ -91,7 +91,13 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     uint32_t b_off[NL];
 #pragma unroll
     for (int i = 0; i < NL; i++) b_off[i] = (uint32_t)min(8 * i + (lane >> 3), a.n - 1 - n0) * (uint32_t)kp + b_piece;
+    // A column's scales of a chunk in one load of 16 bytes, to [column][4], where its row of them allows (groups a multiple of
+    // four); else a load per group, to [group][column].  A load takes the address unit a cycle a line, and every column is a
+    // line of its own: a group's scales cost it as much as 4 KB of activations (64 x 22016 over 4096 42.5 -> 41.0 us, 64 x 4096
+    // over 11008 33.1 -> 31.0, 30 x 2048 over 2048 11.8 -> 11.1).
     constexpr int kScaleRow = scale_row(TNW);
+    const bool scales4 = (a.groups & (kChunk - 1)) == 0;
+    const int sc_col = scales4 ? 16 : 4, sc_group = scales4 ? 4 : kScaleRow, sc_at = l32 * sc_col;
     const uint32_t s_off = (uint32_t)min(min(lane, TN - 1), a.n - 1 - n0) * (uint32_t)a.groups * 4u;
     const uint32_t s_off2 = (uint32_t)min(min(64 + lane, TN - 1), a.n - 1 - n0) * (uint32_t)a.groups * 4u;
     const uint32_t q_at = l32 * 128, q_x = l32 & 7;
@@ -104,6 +110,11 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
         const uint32_t dst = wl_at + slot * kSlot;
 #pragma unroll
         for (int i = 0; i < NL; i++) load_to_lds16(b_base + (int64_t)c * (kChunk * kQ8Group), b_off[i] - back, dst + i * 1024);
+        if (scales4) {
+            load_to_lds16(s_base + c * kChunk, s_off, dst + TN * 128);
+            if constexpr (TN > 64) load_to_lds16(s_base + c * kChunk, s_off2, dst + TN * 128 + 1024);
+            return;
+        }
 #pragma unroll
         for (int g = 0; g < kChunk; g++) {
             const float *at = s_base + min(c * kChunk + g, a.groups - 1);
@@ -130,7 +141,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     uintx4 q[2];                                       // ... and as bytes, up to two stages ahead
     float sc[4] = {0.f, 0.f, 0.f, 0.f};                // their scales: of the stage before, this one and the two next
     auto read_q = [&](int slot, int g, int tn, int at, int at_sc) __attribute__((always_inline)) {
-        sc[at_sc] = *reinterpret_cast<const float *>(wl + slot * kSlot + TN * 128 + g * kScaleRow + (32 * tn + l32) * 4);
+        sc[at_sc] = *reinterpret_cast<const float *>(wl + slot * kSlot + TN * 128 + sc_at + (g * sc_group + 32 * tn * sc_col));
         q[at] = *reinterpret_cast<const uintx4 *>(wl + slot * kSlot + 4096 * tn + q_at + (((2 * g + half) ^ q_x) << 4));
     };
     int c = c_begin + wave, slot = 0;
@@ -304,7 +315,7 @@ void q8_gemm_rows_configure() {
     });
 }
 
-// What the fp16 GEMM does not take: fewer than 256 rows without a copy of the weights in its layout (64 x 22016 over 4096 43 us,
+// What the fp16 GEMM does not take: fewer than 256 rows without a copy of the weights in its layout (64 x 22016 over 4096 41 us,
 // 86 on the bf16 kernels), or few tiles, or a short K.  The rows' split into planes costs a launch.  Where they are normalised
 // first it takes that launch's place: 128 x 2048 over 2048 13.3 us against 17.9 on the bf16 kernels, 16 x 256 over 256 8.6, 9.6,
 // and only a multitude of rows against a small weight is better off there (700 x 768 over 256: 13.2, 11.8; 700 x 1536 over 512
