@@ -285,16 +285,20 @@ __global__ void __launch_bounds__(256) k_attention_tiled(AttnKernelArgs a) {
     constexpr int PART = HD / 8;
     typedef float floatx4 __attribute__((ext_vector_type(4)));
     floatx4 kreg[KSETS][PART / 4], vreg[PVB ? 1 : KSETS][PVB ? 1 : PART / 4];
-    auto request_keys = [&](int k0, int ks) __attribute__((always_inline)) {       // rows past the last key repeat it (masked below)
-        const float *kr = kbase + (int64_t)min(k0 + ks * KT + (t & 31), wg_last) * a.tok_stride + (t >> 5) * PART;
+    // Neighbouring lanes take neighbouring 16 bytes of a row: a load takes the address unit a cycle a line, and with a row a lane
+    // it was 64 of them (32 heads of 64 x 512 rows 23.3 -> 21.9 us, 12 x 400 18.2 -> 17.6, 16 of 128 x 1024 73.8 -> 70.1).  One key
+    // set has the products to cover that, and a row a lane is still the better one (32 of 128 x 2048 rows 250 us, 255 so).
+    constexpr bool BY_ROW = KSETS == 1;
+    constexpr int LPR = HD / 4;                              // lanes a row
+    auto piece_row = [&](int j) __attribute__((always_inline)) { return BY_ROW ? t & 31 : t / LPR + 256 / LPR * j; };
+    auto piece_at = [&](int j) __attribute__((always_inline)) { return BY_ROW ? (t >> 5) * PART + 4 * j : t % LPR * 4; };
+    auto request_rows = [&](floatx4 (&to)[PART / 4], const float *base, int k0, int ks) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < PART; j += 4) kreg[ks][j / 4] = *reinterpret_cast<const floatx4 *>(kr + j);
+        for (int j = 0; j < PART / 4; j++)                   // rows past the last key repeat it (masked below)
+            to[j] = *reinterpret_cast<const floatx4 *>(base + (int64_t)min(k0 + ks * KT + piece_row(j), wg_last) * a.tok_stride + piece_at(j));
     };
-    auto request_values = [&](int k0, int ks) __attribute__((always_inline)) {
-        const float *vr = vbase + (int64_t)min(k0 + ks * KT + (t >> 3), wg_last) * a.tok_stride + (t & 7) * PART;
-#pragma unroll
-        for (int j = 0; j < PART; j += 4) vreg[ks][j / 4] = *reinterpret_cast<const floatx4 *>(vr + j);
-    };
+    auto request_keys = [&](int k0, int ks) __attribute__((always_inline)) { request_rows(kreg[ks], kbase, k0, ks); };
+    auto request_values = [&](int k0, int ks) __attribute__((always_inline)) { if constexpr (!PVB) request_rows(vreg[ks], vbase, k0, ks); };
     auto request = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
         for (int ks = 0; ks < KSETS; ks++) {
@@ -309,15 +313,15 @@ __global__ void __launch_bounds__(256) k_attention_tiled(AttnKernelArgs a) {
             // stage the key tile as bf16 planes
             if constexpr (!AHEAD) request_keys(k0, ks);
 #pragma unroll
-            for (int j = 0; j < PART; j += 4) {
-                const floatx4 v = kreg[ks][j / 4];
-                const int c = (t >> 5) * PART + j;                                       // first of four elements of the row
-                const int at = ((((c >> 3) ^ (t & 31)) & (CH - 1)) << 3) + (c & 7);       // chunk c / 8 lives at (c / 8) ^ key
+            for (int j = 0; j < PART / 4; j++) {
+                const floatx4 v = kreg[ks][j];
+                const int row = piece_row(j), c = piece_at(j);
+                const int at = ((((c >> 3) ^ row) & (CH - 1)) << 3) + (c & 7);            // chunk c / 8 lives at (c / 8) ^ key
                 uint32_t hi[2], mid[2], lo[2];
                 split3(v.x, v.y, hi[0], mid[0], lo[0]); split3(v.z, v.w, hi[1], mid[1], lo[1]);
-                *reinterpret_cast<uint2 *>(&Kb[ks][0][t & 31][at]) = make_uint2(hi[0], hi[1]);
-                *reinterpret_cast<uint2 *>(&Kb[ks][1][t & 31][at]) = make_uint2(mid[0], mid[1]);
-                *reinterpret_cast<uint2 *>(&Kb[ks][2][t & 31][at]) = make_uint2(lo[0], lo[1]);
+                *reinterpret_cast<uint2 *>(&Kb[ks][0][row][at]) = make_uint2(hi[0], hi[1]);
+                *reinterpret_cast<uint2 *>(&Kb[ks][1][row][at]) = make_uint2(mid[0], mid[1]);
+                *reinterpret_cast<uint2 *>(&Kb[ks][2][row][at]) = make_uint2(lo[0], lo[1]);
             }
         }
         // PVB: the value rows are requested now and fly while the scores are computed; else the value tile is staged as it is
@@ -327,7 +331,7 @@ __global__ void __launch_bounds__(256) k_attention_tiled(AttnKernelArgs a) {
             for (int ks = 0; ks < KSETS; ks++) {
                 if constexpr (!AHEAD) request_values(k0, ks);
 #pragma unroll
-                for (int j = 0; j < PART; j += 4) *reinterpret_cast<floatx4 *>(&Vs[ks][t >> 3][(t & 7) * PART + j]) = vreg[ks][j / 4];
+                for (int j = 0; j < PART / 4; j++) *reinterpret_cast<floatx4 *>(&Vs[ks][piece_row(j)][piece_at(j)]) = vreg[ks][j];
             }
         }
 #pragma unroll
