@@ -26,6 +26,7 @@
 
 #include "dj_common.h"
 #include "dj_device.h"
+#include <type_traits>
 #include "gemm_rows.h"
 
 namespace dj {
@@ -302,11 +303,30 @@ __device__ __forceinline__ void stage_digits(float *xs, int plane0, int shift_at
 // VEC (compile time): K is a multiple of 4 and the row is loaded as float4s.  A run-time choice between the two
 // staging paths made the compiler merge their registers with copies placed right behind the first activation
 // load - a wait for it ahead of every weight load.
-template <int NC, int B, bool SWIGLU, int MODE, int PRO, bool VEC>
-__device__ __forceinline__ void matvec(const MatvecArgs &p, float *xs, int block, int grid) {   // xs: the activation row, laid out by xs_at()
+// Second: a kernel of two weights over the same row; workgroups from a_grid on take the second one.
+struct SecondWeight { const int8_t *wq; const float *scales; float *out; int grid, n_out; };
+struct NoSecond {};
+
+template <int NC, int B, bool SWIGLU, int MODE, int PRO, bool VEC, typename Second = NoSecond>
+__global__ void __launch_bounds__(kThreads)
+k_q8_matvec(const float *a_x, const int8_t *a_wq, const float *a_scales, float *a_out, int a_k, int a_grid, int a_n_out,
+            int a_rec_hd, const float *a_gamma, const float *a_bias, const float *a_bias2, const float *a_residual,
+            const float *a_beta, const Second a_second) {
+    // (the grid size comes as an argument: gridDim.x is one more value fetched from the argument buffer)
+    constexpr bool PAIR = std::is_same_v<Second, SecondWeight>;
+    int block = blockIdx.x, grid = a_grid;
+    MatvecArgs p{a_x, a_wq, a_scales, a_out, a_k, (a_k + kQ8Group - 1) / kQ8Group * kQ8Group, a_n_out, a_gamma,
+                 a_bias, a_bias2, a_residual, a_beta, a_rec_hd};
+    if constexpr (PAIR) {
+        if (block >= a_grid) {
+            block -= a_grid; grid = a_second.grid;
+            p.wq = a_second.wq; p.scales = a_second.scales; p.out = a_second.out; p.n_out = a_second.n_out;
+        }
+    }
     constexpr bool GELU = MODE == 1;
     constexpr bool MERGE = MODE == 2;
     constexpr int NS = kAttnRecordSplits;
+    extern __shared__ __align__(16) float xs[];   // the activation row, laid out by xs_at() below
     __shared__ float red[kWaves], red2[kWaves];
     constexpr int RPO = SWIGLU ? 2 : 1;           // Q8 rows per output
     constexpr int R = B * RPO;                    // rows per batch
@@ -540,32 +560,6 @@ __device__ __forceinline__ void matvec(const MatvecArgs &p, float *xs, int block
     DJ_STAMP(5);
 }
 
-template <int NC, int B, bool SWIGLU, int MODE, int PRO, bool VEC>
-__global__ void __launch_bounds__(kThreads)
-k_q8_matvec(const float *a_x, const int8_t *a_wq, const float *a_scales, float *a_out, int a_k, int a_grid, int a_n_out,
-            int a_rec_hd, const float *a_gamma, const float *a_bias, const float *a_bias2, const float *a_residual,
-            const float *a_beta) {
-    extern __shared__ __align__(16) float xs[];
-    // (the grid size comes as an argument: gridDim.x is one more value fetched from the argument buffer)
-    const MatvecArgs p{a_x, a_wq, a_scales, a_out, a_k, (a_k + kQ8Group - 1) / kQ8Group * kQ8Group, a_n_out, a_gamma,
-                       a_bias, a_bias2, a_residual, a_beta, a_rec_hd};
-    matvec<NC, B, SWIGLU, MODE, PRO, VEC>(p, xs, blockIdx.x, a_grid);
-}
-
-// Two weights over the same normalised row in one launch: a small matvec is bound by its launch and the first answer of memory,
-// and the second one's are the first one's here.  The latent models' down projections (d 2048, 1024 and 512 output rows; 4
-// layers): a token 176.5 -> 169.9 us, at d 1024 123.7 -> 115.6, at d 512 108.4 -> 100.3.
-template <int NC, int B>
-__global__ void __launch_bounds__(kThreads)
-k_q8_matvec_pair(const float *a_x, const int8_t *a_wq, const float *a_scales, float *a_out, int a_k, int a_grid, int a_n_out, const float *a_gamma,
-                 const int8_t *b_wq, const float *b_scales, float *b_out, int b_grid, int b_n_out) {
-    extern __shared__ __align__(16) float xs[];
-    const bool second = (int)blockIdx.x >= a_grid;
-    const MatvecArgs p{a_x, second ? b_wq : a_wq, second ? b_scales : a_scales, second ? b_out : a_out, a_k, (a_k + kQ8Group - 1) / kQ8Group * kQ8Group,
-                       second ? b_n_out : a_n_out, a_gamma, nullptr, nullptr, nullptr, nullptr, 0};
-    matvec<NC, B, false, 0, 1, true>(p, xs, second ? blockIdx.x - a_grid : blockIdx.x, second ? b_grid : a_grid);
-}
-
 constexpr int kMvGridCap = 768;          // three workgroups per CU
 constexpr int kMvGridCapWide = 1024;     // four for the widest matrices (the LM head: two batches per wavefront instead of three, 14.7 -> 14.0 us)
 inline int mv_grid_cap() { return kMvGridCap; }
@@ -596,10 +590,10 @@ void launch_mv(hipStream_t s, const MatvecArgs &a) {
         constexpr int PRO = decltype(pro_tag)::value;
         if (vec) {
             launch_kernel(k_q8_matvec<NC, B, SW, MODE, PRO, true>, dim3(grid), dim3(kThreads), lds, s, a.x, a.wq,
-                          a.scales, a.out, a.k, grid, a.n_out, a.rec_hd, a.gamma, a.bias, a.bias2, a.residual, a.beta);
+                          a.scales, a.out, a.k, grid, a.n_out, a.rec_hd, a.gamma, a.bias, a.bias2, a.residual, a.beta, NoSecond{});
         } else if constexpr (B == 1 && MODE != 2) {
             launch_kernel(k_q8_matvec<NC, B, SW, MODE, PRO, false>, dim3(grid), dim3(kThreads), lds, s, a.x, a.wq,
-                          a.scales, a.out, a.k, grid, a.n_out, a.rec_hd, a.gamma, a.bias, a.bias2, a.residual, a.beta);
+                          a.scales, a.out, a.k, grid, a.n_out, a.rec_hd, a.gamma, a.bias, a.bias2, a.residual, a.beta, NoSecond{});
         } else {
             fail("q8_linear: no matvec kernel for this shape");     // launch_mv sends ragged K to B = 1
         }
@@ -704,6 +698,9 @@ int64_t q8_linear_preferred_workspace_floats(int m, int k, int n, int flags, boo
 
 bool q8_linear_pair_ok(int k) { return k > 0 && (k & 3) == 0 && k <= 4096; }
 
+// Two weights over the same normalised row in one launch: a small matvec is bound by its launch and the first answer of memory,
+// and the second one's are the first one's here.  The latent models' down projections (d 2048, 1024 and 512 output rows; 4
+// layers): a token 176.5 -> 169.9 us, at d 1024 123.7 -> 115.6, at d 512 108.4 -> 100.3.
 void launch_q8_linear_pair(hipStream_t s, const Q8LinearPair &p) {
     if (!q8_linear_pair_ok(p.k)) fail("q8_linear_pair: shape outside this kernel's range");
     auto go = [&](auto nc, auto b) {
@@ -711,8 +708,9 @@ void launch_q8_linear_pair(hipStream_t s, const Q8LinearPair &p) {
         int grid[2];
         const int per = B * kWaves, all = (p.n[0] + per - 1) / per + (p.n[1] + per - 1) / per, rounds = (all + mv_grid_cap() - 1) / mv_grid_cap();
         for (int i = 0; i < 2; i++) grid[i] = (p.n[i] + per * rounds - 1) / (per * rounds);
-        launch_kernel(k_q8_matvec_pair<NC, B>, dim3(grid[0] + grid[1]), dim3(kThreads), (size_t)xs_floats(q8_padded_k(p.k)) * sizeof(float), s, p.x, p.wq[0],
-                      p.scales[0], p.out[0], p.k, grid[0], p.n[0], p.gamma, p.wq[1], p.scales[1], p.out[1], grid[1], p.n[1]);
+        launch_kernel(k_q8_matvec<NC, B, false, 0, 1, true, SecondWeight>, dim3(grid[0] + grid[1]), dim3(kThreads), (size_t)xs_floats(q8_padded_k(p.k)) * sizeof(float), s,
+                      p.x, p.wq[0], p.scales[0], p.out[0], p.k, grid[0], p.n[0], 0, p.gamma, (const float *)nullptr, (const float *)nullptr,
+                      (const float *)nullptr, (const float *)nullptr, SecondWeight{p.wq[1], p.scales[1], p.out[1], grid[1], p.n[1]});
     };
     // Two rows a wavefront once one a wavefront is more than a workgroup per compute unit: a token of the 4-layer model below 171.6
     // us with one (384 workgroups), 169.9 with two.
