@@ -256,7 +256,7 @@ class HipNative:
     @staticmethod
     def q8GemmPath(m: int, k: int, rows: int) -> int:
         """128 or 64 (rows per workgroup tile) when a Q8_LINEAR of m rows over such a weight runs on the fp16 direct-load
-        GEMM, 0 when it runs on the bf16 kernels or the matvec."""
+        GEMM, 0 when it runs on the kernels that read the int8 weights or the matvec."""
         return int(library().deepj_hip_q8_gemm_path(m, k, rows))
 
     @staticmethod

@@ -565,6 +565,8 @@ __global__ void __launch_bounds__(256) k_sum_partials(const float *__restrict__ 
 // (the weights' padding is zero as well, but 0 x garbage could be a NaN).  The grid covers the rows the GEMM's tiles
 // read, which may go past m: those rows only feed output rows that are never stored, and are written as zeros so that
 // the GEMM never multiplies what an earlier user of the workspace left there.
+// OPERAND: the planes in the order the rows kernel's matrix instructions read them (operand_at), up to a multiple of 128 k, and
+// rows of up to 12288 floats in registers.
 // SUM: the row is not read from x but put together first - the sum over `splits` slabs of partial products of a
 // K-sharing GEMM, plus bias and residual in the order that GEMM's own epilogue uses - and written to sum_out as that
 // GEMM's result; what follows is the next GEMM's prologue on it.  One kernel where the two GEMMs would otherwise launch
@@ -778,10 +780,10 @@ struct GemmF16Plan { int tile_rows, tile_cols, splits; };
 
 constexpr int kNPad = 768;      // weight rows of a prepared buffer are padded to a multiple of both tile widths
 
-constexpr int kMinRowsPrepared = 16;     // fewer rows than this stay on the bf16 kernels even with prepared weights
+constexpr int kMinRowsPrepared = 16;     // fewer rows than this read the int8 weights even where a copy is prepared
 
 GemmF16Plan q8_gemm_f16_plan(int m, int n_rows, int k, bool prepared) {
-    // DEEPJ_HIP_GEMM_F16=0 keeps every GEMM on the bf16 kernels; =128, =128192, =64 or =192 force the 128 x 256,
+    // DEEPJ_HIP_GEMM_F16=0 keeps every GEMM off these kernels; =128, =128192, =64 or =192 force the 128 x 256,
     // 128 x 192, 64 x 256 or 64 x 192 tile (for comparisons)
     static const int forced = [] { const char *e = getenv("DEEPJ_HIP_GEMM_F16"); return e ? atoi(e) : -1; }();
     if (forced == 0) return {0, 0, 1};

@@ -320,12 +320,12 @@ void q8_gemm_rows_configure() {
 // first it takes that launch's place: 128 x 2048 over 2048 13.3 us against 17.9 on the bf16 kernels, 16 x 256 over 256 8.6, 9.6,
 // and only a multitude of rows against a small weight is better off there (700 x 768 over 256: 13.2, 11.8; 700 x 1536 over 512
 // 18.9, 20.9).  Where they are not, the weight has to be large enough to make up for it: 128 x 2048 over 2048 12.4, 14.1 and 30 x
-// 6144 over 2048 11.5, 16.1, but 16 x 2048 over 2048 11.8, 11.0 and 128 x 768 over 3072 14.6, 13.2.  A lane's offset into a
-// column tile's weights is 32 bits.
+// 6144 over 2048 11.5, 16.1, but 16 x 2048 over 2048 11.8, 11.0 and 128 x 768 over 3072 14.6, 13.2.  (Past 4096 rows the bf16
+// kernels, which need no workspace for them.)  A lane's offset into a column tile's weights is 32 bits.
 bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared) {
     if (k > (1 << 24) || q8_gemm_f16_shape_ok(m, n_rows, k, prepared)) return false;
     const int64_t weights = (int64_t)n_rows * k;
-    return norm ? m <= 512 || weights >= 3 << 18 : weights >= (m > 32 ? 4 << 20 : 8 << 20);
+    return norm ? m <= 512 || weights >= 3 << 18 : m <= 4096 && weights >= (m > 32 ? 4 << 20 : 8 << 20);
 }
 
 // floats of workspace: planes, row factors, the partial products where K is shared

@@ -277,7 +277,7 @@ int64_t deepj_hip_q8_floats(int32_t k, int32_t rows);
 
 /* Floats of the buffer Q8_PREPARE fills for such a weight (about 2 bytes per weight), and which kernel a Q8_LINEAR of m
  * rows over it runs on when its workspace may grow: the fp16 direct-load GEMM with 128 or 64 rows per workgroup tile
- * (returns 128 or 64), or the bf16 kernels / the matvec (returns 0).
+ * (returns 128 or 64), or the kernels that read the int8 weights / the matvec (returns 0).
  * No counterpart in the reference, whose weights are fp32 (J/layers/Linear.java:9-24). */
 int64_t deepj_hip_q8_prepared_floats(int32_t k, int32_t rows);
 int32_t deepj_hip_q8_gemm_path(int32_t m, int32_t k, int32_t rows);
@@ -333,7 +333,7 @@ int deepj_runner_init_seeded_gpt(void *runner, int64_t seed, float init_scale, i
  * form: -1 (default) no limit - a copy of every layer, written at the first prompt of 64 rows or more (+ 2 bytes
  * per weight); 0 none - every call converts into the workspace; otherwise layers in order while the budget lasts.
  * Prompts of 256 rows and more give the same bits whatever the budget; shorter ones take the fp16 GEMM only where a
- * copy exists (the bf16 kernels otherwise: same tolerance, other last bits).  deepj_runner_prepared_bytes: what the copies take now. */
+ * copy exists (others otherwise: same tolerance, other last bits).  deepj_runner_prepared_bytes: what the copies take now. */
 int deepj_runner_set_prepared_budget(void *runner, int64_t bytes);
 int64_t deepj_runner_prepared_bytes(void *runner);
 int deepj_runner_finalize(void *runner);
