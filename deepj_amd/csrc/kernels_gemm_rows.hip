@@ -281,18 +281,18 @@ int chunks_of(int k) { return (q8_padded_k(k) / kQ8Group + kChunk - 1) / kChunk;
 // A tile's rows and columns in units of 32 and the workgroups that share its K: those of least estimated time, in us.  With x
 // tiles a compute unit and kk thousand k a wavefront, a launch takes
 //   fixed + per_x x + kk (per_k + again (rounds - 1) + per_kx x) + slabs m n shares / 10^6,
-// rounds being 1 up to one tile a compute unit, 2 up to two (two workgroups fit one) and x beyond.  Fitted to 239 shapes of 4 to
-// 512 rows, 768 to 50257 columns and 256 to 11008 k: the choice takes 1.01 times the best one's time on average.  (200 x 2304
-// over 768: 32 x 32 13.4 us, 32 x 64 15.8, 64 x 32 15.3, 64 x 64 15.6; 200 x 11264 over 2048: 53, 44, 48, 41; 64 x 22016 over
-// 4096: 63, 49, 54, 50, and 43 with 64 x 96, whose 230 tiles are one round where 64 x 64 makes 344; 4 x 4096 over 11008:
-// 32 x 32 31, K shared by two 25, by four 27.)
+// rounds being 1 up to one tile a compute unit, 2 up to two (two workgroups fit one) and x beyond.  Fitted to 200 shapes of 4 to
+// 400 rows, 768 to 50257 columns and 256 to 11008 k: the choice takes 1.006 times the best one's time on average, 1.08 at worst.
+// (200 x 2304 over 768: 32 x 32 12.5 us, 32 x 64 14.6, 64 x 32 14.4, 64 x 64 14.7; 200 x 11264 over 2048: 49, 41, 46, 41; 64 x
+// 22016 over 4096: 55, 48, 49, 46, and 42 with 64 x 96, whose 230 tiles are one round where 64 x 64 makes 344; 4 x 4096 over
+// 11008: 32 x 32 32, K shared by two 27, by four 29.)
 struct RowsPlan { int tmw, tnw, shares; };
 RowsPlan rows_plan(int m, int n_rows, int k, bool may_share) {
     struct Shape { int tmw, tnw, shares; double fixed, per_x, per_k, again, per_kx, slabs; };
-    static const Shape shapes[] = {{1, 1, 1, 8.29, 0.27, 1.63, 1.29, 0.91, 0.0}, {1, 2, 1, 8.65, 0.87, 2.59, 1.63, 1.5, 0.0},
-                                   {2, 1, 1, 8.12, 0.31, 2.51, 1.72, 1.63, 0.0}, {2, 2, 1, 9.76, 1.37, 3.49, 2.53, 2.2, 0.0},
-                                   {1, 3, 1, 6.77, 4.03, 4.46, 3.91, 1.01, 0.0}, {2, 3, 1, 6.39, 7.45, 6.26, 6.74, 0.93, 0.0},
-                                   {1, 1, 2, 10.39, 0.6, 1.49, 1.12, 0.8, 2.24}, {1, 1, 4, 9.63, 1.19, 2.91, 1.57, -0.04, 1.12}};
+    static const Shape shapes[] = {{1, 1, 1, 7.26, 0.42, 1.74, 1.0, 0.93, 0.0}, {1, 2, 1, 8.51, 0.75, 2.48, 1.8, 1.14, 0.0},
+                                   {2, 1, 1, 7.99, 0.25, 2.44, 1.75, 1.49, 0.0}, {2, 2, 1, 9.25, 1.16, 3.35, 2.66, 2.0, 0.0},
+                                   {1, 3, 1, 8.69, 2.87, 3.86, 4.54, 0.45, 0.0}, {2, 3, 1, 9.82, 4.83, 5.42, 7.58, 0.5, 0.0},
+                                   {1, 1, 2, 9.6, 0.42, 1.76, 0.73, 1.0, 6.0}, {1, 1, 4, 9.63, 1.1, 2.41, 0.29, 1.2, 0.52}};
     RowsPlan best{};
     double least = -1.0;
     for (const Shape &h : shapes) {
