@@ -41,7 +41,8 @@ SOURCES = {
     # instructions after every few products, and each trip through the accumulator file costs a move per value
     "kernels_matmul.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_gemm_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-    "kernels_gemm_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    # (its K loop is 24 to 144 products unrolled, past the compiler's bound for a requested unrolling)
+    "kernels_gemm_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-pragma-unroll-threshold=65536"],
     "kernels_q8.hip": [],
     "kernels_decode.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],

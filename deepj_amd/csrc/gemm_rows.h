@@ -6,14 +6,14 @@
 
 namespace dj {
 
-// Where the fp16 pieces of activation (row, c) lie for v_mfma_f32_32x32x16_f16: blocks of 1 KB, one per 32 rows, 32 k, half of
+// Where the bf16 pieces of activation (row, c) lie for v_mfma_f32_32x32x16_bf16: blocks of 1 KB, one per 32 rows, 32 k, half of
 // those k and piece; in a block 8 consecutive k for each lane.  Lane l of step s of a group holds row l % 32 and
 // k = 16 (l / 32) + 8 s + j, as the weights' side does (a lane's 16 k of a weight row are 16 consecutive bytes).  The high
-// piece; the low one is kOperandPiece further on.
-constexpr int kOperandPiece = 512;
+// piece; the middle and the low one are kOperandPiece and twice that further on.
+constexpr int kOperandPiece = 512, kOperandPieces = 3;
 __host__ __device__ inline int64_t operand_at(int row, int c, int groups) {
     const int g = c >> 5, h = (c >> 4) & 1, s = (c >> 3) & 1, j = c & 7;
-    return ((((int64_t)(row >> 5) * groups + g) * 2 + s) * 2 * 64 + h * 32 + (row & 31)) * 8 + j;
+    return ((((int64_t)(row >> 5) * groups + g) * 2 + s) * kOperandPieces * 64 + h * 32 + (row & 31)) * 8 + j;
 }
 // Every second 128 k are stored with their sign turned, and the sums over them are subtracted: the matrix cores cut off the
 // low bits of what they add up, always downwards, and two halves of opposite sign are cut off in opposite directions (4096 x
@@ -38,7 +38,7 @@ __device__ __forceinline__ void load_to_lds4(const void *base, uint32_t off, uin
 #endif
 
 // kernels_gemm_f16.hip: the rows, normalised if gamma (and beta) say so, in that order; rows [m, m_pad) as zeros
-void launch_split_operand(hipStream_t s, const float *x, const float *gamma, const float *beta, uint16_t *planes, float *unscale, int m, int m_pad, int k, int kp);
+void launch_split_operand(hipStream_t s, const float *x, const float *gamma, const float *beta, uint16_t *planes, int m, int m_pad, int k, int kp);
 
 // kernels_matmul.hip: C = epilogue(sum of the slabs of partial products)
 void launch_q8_sum_partials(hipStream_t s, const float *partial, float *out, int splits, int m, int n_rows, const GemmEpilogue &ep);

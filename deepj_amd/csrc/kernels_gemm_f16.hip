@@ -565,8 +565,8 @@ __global__ void __launch_bounds__(256) k_sum_partials(const float *__restrict__ 
 // (the weights' padding is zero as well, but 0 x garbage could be a NaN).  The grid covers the rows the GEMM's tiles
 // read, which may go past m: those rows only feed output rows that are never stored, and are written as zeros so that
 // the GEMM never multiplies what an earlier user of the workspace left there.
-// OPERAND: the planes in the order the rows kernel's matrix instructions read them (operand_at), up to a multiple of 128 k, and
-// rows of up to 12288 floats in registers.
+// OPERAND: instead of the planes, the three bf16 pieces that make up each value exactly, in the order the rows kernel's matrix
+// instructions read them (operand_at), up to a multiple of 128 k; rows of up to 12288 floats in registers.
 // SUM: the row is not read from x but put together first - the sum over `splits` slabs of partial products of a
 // K-sharing GEMM, plus bias and residual in the order that GEMM's own epilogue uses - and written to sum_out as that
 // GEMM's result; what follows is the next GEMM's prologue on it.  One kernel where the two GEMMs would otherwise launch
@@ -586,9 +586,8 @@ __global__ void __launch_bounds__(256) k_split_f16(const float *__restrict__ x, 
     if (OPERAND && row >= m) {
         for (int c = t * 8; c < kp; c += 2048) {
             uint4 *p = reinterpret_cast<uint4 *>(planes + operand_at(row, c, kp / kQ8Group));
-            p[0] = p[kOperandPiece / 8] = make_uint4(0u, 0u, 0u, 0u);
+            p[0] = p[kOperandPiece / 8] = p[kOperandPiece / 4] = make_uint4(0u, 0u, 0u, 0u);
         }
-        if (t == 0) unscale[row] = 0.f;
         return;
     }
     if (row >= m) {
@@ -623,6 +622,13 @@ __global__ void __launch_bounds__(256) k_split_f16(const float *__restrict__ x, 
         const _Float16 ll = (_Float16)(v - (float)hh);
         h = __builtin_bit_cast(uint16_t, hh);
         l = __builtin_bit_cast(uint16_t, ll);
+    };
+    // the leading 8 significant bits, the next 8 and the 8 that are left, each the upper half of a float
+    auto pieces = [](float v, uint32_t &h, uint32_t &c, uint32_t &l) {
+        h = __float_as_uint(v) & 0xffff0000u;
+        const float r = v - __uint_as_float(h);
+        c = __float_as_uint(r) & 0xffff0000u;
+        l = __float_as_uint(r - __uint_as_float(c));
     };
     uint16_t *hi = planes + (int64_t)row * pitch, *lo = hi + plane_elems;
     constexpr int NV = OPERAND ? 12 : 8;                             // 128-bit words a thread keeps of one row
@@ -691,6 +697,23 @@ __global__ void __launch_bounds__(256) k_split_f16(const float *__restrict__ x, 
                                    ((v[j].z - mean) / sd) * g.z + bt.z, ((v[j].w - mean) / sd) * g.w + bt.w);
             }
         }
+        if constexpr (OPERAND) {
+#pragma unroll
+            for (int j = 0; j < NV; j++) {
+                const int i = t + j * 256;
+                if (i >= kp >> 2) continue;
+                const bool turn = operand_negated(4 * i);
+                const float u[4] = {turn ? -v[j].x : v[j].x, turn ? -v[j].y : v[j].y, turn ? -v[j].z : v[j].z, turn ? -v[j].w : v[j].w};
+                uint32_t h[4], c[4], l[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) pieces(u[e], h[e], c[e], l[e]);
+                uint16_t *p = planes + operand_at(row, 4 * i, kp / kQ8Group);
+                *reinterpret_cast<uint2 *>(p) = make_uint2((h[0] >> 16) | h[1], (h[2] >> 16) | h[3]);
+                *reinterpret_cast<uint2 *>(p + kOperandPiece) = make_uint2((c[0] >> 16) | c[1], (c[2] >> 16) | c[3]);
+                *reinterpret_cast<uint2 *>(p + 2 * kOperandPiece) = make_uint2((l[0] >> 16) | (l[1] & 0xffff0000u), (l[2] >> 16) | (l[3] & 0xffff0000u));
+            }
+            return;
+        }
         float mx = 0.f;
 #pragma unroll
         for (int j = 0; j < NV; j++) mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
@@ -698,16 +721,9 @@ __global__ void __launch_bounds__(256) k_split_f16(const float *__restrict__ x, 
 #pragma unroll
         for (int j = 0; j < NV; j++) {
             const int i = t + j * 256;
-            if (i >= (OPERAND ? kp >> 2 : n4)) continue;
+            if (i >= n4) continue;
             uint16_t h[4], l[4];
-            const float by = OPERAND && operand_negated(4 * i) ? -up : up;
-            halves(v[j].x * by, h[0], l[0]); halves(v[j].y * by, h[1], l[1]); halves(v[j].z * by, h[2], l[2]); halves(v[j].w * by, h[3], l[3]);
-            if constexpr (OPERAND) {
-                uint16_t *p = planes + operand_at(row, 4 * i, kp / kQ8Group);
-                *reinterpret_cast<uint2 *>(p) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
-                *reinterpret_cast<uint2 *>(p + kOperandPiece) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
-                continue;
-            }
+            halves(v[j].x * up, h[0], l[0]); halves(v[j].y * up, h[1], l[1]); halves(v[j].z * up, h[2], l[2]); halves(v[j].w * up, h[3], l[3]);
             reinterpret_cast<uint2 *>(hi)[i] = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
             reinterpret_cast<uint2 *>(lo)[i] = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
         }
@@ -733,15 +749,24 @@ __global__ void __launch_bounds__(256) k_split_f16(const float *__restrict__ x, 
         if (NORM == 2) return ((v - mean) / denom) * gamma[c] + beta[c];
         return v;
     };
+    if constexpr (OPERAND) {
+        for (int c = t; c < kp; c += 256) {
+            const float v = c < k ? value(c) : 0.f;
+            uint32_t h, mid, l;
+            pieces(operand_negated(c) ? -v : v, h, mid, l);
+            uint16_t *p = planes + operand_at(row, c, kp / kQ8Group);
+            p[0] = (uint16_t)(h >> 16); p[kOperandPiece] = (uint16_t)(mid >> 16); p[2 * kOperandPiece] = (uint16_t)(l >> 16);
+        }
+        return;
+    }
     float mx = 0.f;
     for (int c = t; c < k; c += 256) mx = fmaxf(mx, fabsf(value(c)));
     const float up = scale_of(block_reduce(mx, true));
     for (int c = t; c < kp; c += 256) {
         uint16_t h, l;
-        halves(c < k ? value(c) * (OPERAND && operand_negated(c) ? -up : up) : 0.f, h, l);
-        const int64_t at = OPERAND ? operand_at(row, c, kp / kQ8Group) : (int64_t)row * pitch + c;
-        planes[at] = h;
-        planes[at + (OPERAND ? kOperandPiece : plane_elems)] = l;
+        halves(c < k ? value(c) * up : 0.f, h, l);
+        hi[c] = h;
+        lo[c] = l;
     }
 }
 
@@ -973,9 +998,9 @@ void launch_q8_gemm_f16(hipStream_t s, const float *x, const float *gamma, const
     }
 }
 
-void launch_split_operand(hipStream_t s, const float *x, const float *gamma, const float *beta, uint16_t *planes, float *unscale, int m, int m_pad, int k, int kp) {
+void launch_split_operand(hipStream_t s, const float *x, const float *gamma, const float *beta, uint16_t *planes, int m, int m_pad, int k, int kp) {
     auto split = !gamma ? k_split_f16<0, false, true> : beta ? k_split_f16<2, false, true> : k_split_f16<1, false, true>;
-    launch_kernel(split, dim3(m_pad), dim3(256), 0, s, x, gamma, beta, planes, unscale, m, k, kp, kp, (int64_t)0, SplitSum{});
+    launch_kernel(split, dim3(m_pad), dim3(256), 0, s, x, gamma, beta, planes, (float *)nullptr, m, k, kp, kp, (int64_t)0, SplitSum{});
 }
 
 #ifdef DJ_TRACE

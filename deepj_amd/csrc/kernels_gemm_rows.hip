@@ -1,28 +1,30 @@
 // Q8 GEMM for a batch of rows straight from the int8 weights: C[M x N] = X[M x K] . dequant(W)^T, W int8 [N x Kp] with one
 // fp32 scale per 32 k.
 //
-// Arithmetic as in kernels_gemm_f16.hip: a row of activations times a power of two, split into two fp16 numbers (22 bits), the
-// weights exact in fp16, two v_mfma_f32_32x32x16_f16 per 16 k, the group scale on the finished 32-k sums.  The split happens
-// once, in a launch in front that also normalises the rows (k_split_f16), where the bf16 kernels (kernels_matmul.hip) turn the
-// activations into three pieces anew for every column tile; the weights stay int8 in memory and become fp16 in registers,
-// where the fp16 GEMM reads a copy of twice their size.
+// Arithmetic as in k_gemm_q8 (kernels_matmul.hip): an activation as three bf16 pieces that make it up exactly, the weights exact in
+// bf16, three v_mfma_f32_32x32x16_bf16 per 16 k, the group scale on the finished 32-k sums.  The split happens once, in a launch
+// in front that also normalises the rows (k_split_f16), where k_gemm_q8 does it anew for every column tile; the weights stay int8
+// in memory and become bf16 in registers.  (Two fp16 pieces under one power of two a row, as the fp16 GEMM takes them, are a third
+// less to read and multiply, 64 x 22016 over 4096 41 us, but 22 bits, and fewer for elements far below their row's largest: with one
+// of 1e8 among values of about 1 that meets zero weights the error against 64 bits was 7e-5 of the result's rms, 9e-8 so.)
 //
 // A workgroup takes a tile of 32 TMW x 32 TNW and deals its K to four wavefronts in chunks of 128, one line of a weight row:
 // no wavefront waits for another before the end, when their sums meet in LDS.  A wavefront asks for a chunk of its weights one
-// chunk ahead, global -> LDS in whole lines, and for its activations NA groups ahead, straight into registers in operand order;
+// chunk ahead, global -> LDS in whole lines, and for its activations NA pieces ahead, straight into registers in operand order;
 // loads return in the order they were asked for, so waiting for activations that were asked for after a chunk is waiting for
 // the chunk.  The matrix cores' 32 cycles a product hide the group before's scaling and the next one's conversion.
 //
-// What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 29 us with the split, 87 on the bf16
-// kernels; 4.6 TB/s in the K loop), then the activations, which every tile reads anew from L2 (8 KB for every 64 x 64 x 32:
-// 64 x 22016 41 us, 86; 200 x 11264 over 2048 41, 67), and on small weights two launches' latency (30 x 2304 over 768 9.2 us,
-// 11.9).  Tried and slower: eight wavefronts a workgroup (two workgroups of four fill a compute unit better: 64 x 22016 54 us
-// against 49), the K loop or the epilogue rolled (3 % and 10 %), a 64 x 64 tile whose wavefronts share the activations through
-// LDS (latency of its reads and barriers: 400 x 768 over 3072 34 us against 22).
+// What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 33 us with the split, 39 where they come from
+// HBM, 87 on the bf16 kernels), then the activations, which every tile reads anew from L2 (12 KB for every 64 x 64 x 32: 64 x
+// 22016 46 us, 86; 200 x 11264 over 2048 47, 67), and on small weights two launches' latency (30 x 2304 over 768 9.0 us, 10.8).
+// Tried and slower, with two pieces: eight wavefronts a workgroup (two workgroups of four fill a compute unit better: 64 x 22016
+// 54 us against 49), the K loop or the epilogue rolled (3 % and 10 %), a 64 x 64 tile whose wavefronts share the activations
+// through LDS (latency of its reads and barriers: 400 x 768 over 3072 34 us against 22).
 //
-// Error against 64 bits: 0.95e-7 to 1.83e-7 of the result's rms over 768 to 11008 k, 0.96e-7 to 1.87e-7 on the bf16 kernels.  It
-// hangs on the number of sums a row is dealt to (four wavefronts, NS sets in each), on the low pieces' products going first, and
-// on every second chunk's sign (operand_negated).
+// Error against 64 bits, as a share of the result's rms: 0.77e-7 over 768 k, 0.81e-7 to 0.94e-7 over 2048, 0.94e-7 to 1.79e-7 over
+// 11008, by the number of sums a row is dealt to (four wavefronts, NS sets in each); 0.96e-7, 1.06e-7 and 1.2e-7 on the bf16
+// kernels where they share K.  It also hangs on the low pieces' products going first and on every second chunk's sign
+// (operand_negated).
 #include "dj_common.h"
 #include <algorithm>
 #include "gemm_epilogue.h"
@@ -31,22 +33,21 @@
 namespace dj {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
 constexpr int kWaves = 4;
+constexpr int NP = 2 * kOperandPieces, kGroupWords = NP * 64;       // products of a 32 x 32 tile and 32 k; 16-byte words of 32 rows' activations
 constexpr int kChunk = kOperandChunk / kQ8Group;                   // scale groups a wavefront takes at a time: 128 k, one line of a weight row
 constexpr int scale_row(int tnw) { return tnw > 2 ? 512 : 256; }
 constexpr int slot_bytes(int tnw) { return 32 * tnw * 128 + kChunk * scale_row(tnw); }       // a wavefront's chunk in LDS: weights [column][128], scales [group][64 or 128]
 
 struct GemmRowsArgs {
-    const uintx4 *planes;        // activations in operand order (rows_plane_at)
+    const uintx4 *planes;        // activations in operand order (operand_at)
     const int8_t *wq;           // [n][kp]
     const float *scales;        // [n][groups]
-    const float *unscale;       // [m up to a multiple of 32]
     float *out;
     int m, n, groups;
     int m_tiles, n_tiles;       // tiles of the launched kernel's size
@@ -55,16 +56,15 @@ struct GemmRowsArgs {
     float *partial;             // [gridDim.z][m][n] when they do
 };
 
-// four int8 of a word as fp16: the byte with its sign bit flipped is b + 128, under the exponent of 1024 it reads 1152 + b
-__device__ __forceinline__ void int8x4_to_half(uint32_t r, uint32_t &lo, uint32_t &hi) {
-    const halfx2 bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    r ^= 0x80808080u;
-    lo = __builtin_bit_cast(uint32_t, __builtin_bit_cast(halfx2, __builtin_amdgcn_perm(0x64646464u, r, 0x04010400u)) + bias);
-    hi = __builtin_bit_cast(uint32_t, __builtin_bit_cast(halfx2, __builtin_amdgcn_perm(0x64646464u, r, 0x04030402u)) + bias);
+// four int8 of a word as bf16, exactly
+__device__ __forceinline__ void int8x4_to_bf16(uint32_t r, uint32_t &lo, uint32_t &hi) {
+    auto pack = [](float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302); };
+    lo = pack((float)(int8_t)r, (float)(int8_t)(r >> 8));
+    hi = pack((float)(int8_t)(r >> 16), (float)(int8_t)(r >> 24));
 }
 
 template <int TMW, int TNW>
-__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(TMW * TNW > 4 ? 1 : 2, 2))) k_gemm_q8_rows(const GemmRowsArgs a) {
+__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(TNW > 2 ? 1 : 2, TNW > 2 ? 1 : 2))) k_gemm_q8_rows(const GemmRowsArgs a) {
     constexpr int TN = 32 * TNW, NL = TN / 8;          // NL: loads a wavefront makes for a chunk of its TN weight rows
     constexpr int kSlot = slot_bytes(TNW);
     extern __shared__ __align__(16) unsigned char lds[];
@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     const uint32_t q_at = l32 * 128, q_x = l32 & 7;
     const uintx4 *ap[TMW];
 #pragma unroll
-    for (int i = 0; i < TMW; i++) ap[i] = a.planes + (int64_t)min(m_tile * TMW + i, row_tiles - 1) * chunks * kChunk * 256;
+    for (int i = 0; i < TMW; i++) ap[i] = a.planes + (int64_t)min(m_tile * TMW + i, row_tiles - 1) * chunks * kChunk * kGroupWords;
 
     auto fetch_b = [&](int c, int slot) __attribute__((always_inline)) {
         const uint32_t back = c * (kChunk * kQ8Group) + b_piece < kp ? 0u : (uint32_t)b_piece;       // past the row's end: a piece that meets activations of zero
@@ -122,9 +122,15 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             if constexpr (TN > 64) load_to_lds4(at, s_off2, dst + TN * 128 + g * kScaleRow + 256);
         }
     };
-    constexpr int NA = TMW == 1 ? 4 : 2;               // groups of activations in flight
-    uintx4 av[NA][TMW][4];                             // [group % NA][row tile]: low pieces of the two k steps, high pieces
-    auto fetch_a = [&](int i, int j, int g) __attribute__((always_inline)) { return (ap[i] + (int64_t)g * 256)[64 * (2 * (j & 1) + (j < 2)) + lane]; };
+    // The activations come as a sequence of pieces, NP a group: low ones of the two k steps, middle ones, high ones.  NA of them
+    // are in registers or on their way: as many as the registers of two wavefronts a SIMD leave room for, or of one where LDS has no
+    // room for a second workgroup (96 columns).  24 instead of 12 where TMW is 1: 30 x 2304 over 768 9.2 us against 9.0; 8 instead
+    // of 6 where it is 2: 128 x 50257 over 768 60 against 53, with registers spilled; 8 instead of 24 at 96 columns: 30 x 22016 over
+    // 4096 37 against 33.
+    constexpr int NA = TNW > 2 ? 24 : TMW == 1 ? 12 : 6;
+    static_assert(kChunk * NP % NA == 0, "a piece's register is known at compile time");
+    uintx4 av[TMW][NA];
+    auto fetch_a = [&](int i, int q, int c) __attribute__((always_inline)) { return (ap[i] + ((int64_t)c * kChunk + q / NP) * kGroupWords)[64 * (kOperandPieces * (q & 1) + 2 - (q % NP >> 1)) + lane]; };
     constexpr int NS = TMW * TNW > 4 ? 1 : 4 / (TMW * TNW);       // sets of sums: a group's goes to set group % NS
     floatx16 acc[NS][TMW][TNW], p[2];
 #pragma unroll
@@ -138,25 +144,23 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
         p[0][e] = p[1][e] = 0.0f;
     }
     uint32_t bw[2][8];                                 // [stage parity]: the weights of a stage (a column tile of a group) as fp16
-    uintx4 q[2];                                       // ... and as bytes, up to two stages ahead
+    uintx4 qw[2];                                      // ... and as bytes, up to two stages ahead
     float sc[4] = {0.f, 0.f, 0.f, 0.f};                // their scales: of the stage before, this one and the two next
     auto read_q = [&](int slot, int g, int tn, int at, int at_sc) __attribute__((always_inline)) {
         sc[at_sc] = *reinterpret_cast<const float *>(wl + slot * kSlot + TN * 128 + sc_at + (g * sc_group + 32 * tn * sc_col));
-        q[at] = *reinterpret_cast<const uintx4 *>(wl + slot * kSlot + 4096 * tn + q_at + (((2 * g + half) ^ q_x) << 4));
+        qw[at] = *reinterpret_cast<const uintx4 *>(wl + slot * kSlot + 4096 * tn + q_at + (((2 * g + half) ^ q_x) << 4));
     };
     int c = c_begin + wave, slot = 0;
     if (c < c_end) {
         fetch_b(c, 0);
 #pragma unroll
-        for (int g = 0; g < NA; g++)
+        for (int q = 0; q < NA; q++)
 #pragma unroll
-            for (int i = 0; i < TMW; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) av[g][i][j] = fetch_a(i, j, c * kChunk + g);
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * NA * TMW) : "memory");
+            for (int i = 0; i < TMW; i++) av[i][q] = fetch_a(i, q, c);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA * TMW) : "memory");
         read_q(0, 0, 0, 0, 1);
 #pragma unroll
-        for (int w = 0; w < 4; w++) int8x4_to_half(q[0][w], bw[0][2 * w], bw[0][2 * w + 1]);
+        for (int w = 0; w < 4; w++) int8x4_to_bf16(qw[0][w], bw[0][2 * w], bw[0][2 * w + 1]);
         read_q(0, 1 / TNW, 1 % TNW, 1, 2);
         constexpr int S = kChunk * TNW, kAhead = TNW == 1 ? 2 : 1;      // stages of a chunk; groups two stages reach ahead, whole or begun
 #pragma unroll 1
@@ -167,8 +171,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             for (int st = 0; st < S; st++) {
                 const int g = st / TNW, tn = st % TNW;
                 // two stages on is the next chunk: its weights were asked for before the activations of the groups since
-                if (st == S - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((4 - kAhead) * 4 * TMW) : "memory");
-                const uintx4 qn = q[(st + 1) & 1];
+                if (st == S - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((4 - kAhead) * NP * TMW) : "memory");
+                const uintx4 qn = qw[(st + 1) & 1];
                 const int st2 = (st + 2) % S;
                 read_q(st + 2 >= S ? slot ^ 1 : slot, st2 / TNW, st2 % TNW, st & 1, (st + 3) & 3);
 #pragma unroll
@@ -177,18 +181,19 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
                     const int ptm = tm > 0 ? tm - 1 : TMW - 1, pst = tm > 0 ? st : (st + S - 1) % S, ptn = pst % TNW, pg = pst / TNW;
                     const float psc = tm > 0 ? sc[(st + 1) & 3] : sc[st & 3];
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
+                    for (int j = 0; j < NP; j++) {
+                        const int q = g * NP + j;
                         const uint32_t *w4 = bw[st & 1] + 4 * (j & 1);
-                        p[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, av[g % NA][tm][j]), __builtin_bit_cast(halfx8, (uintx4){w4[0], w4[1], w4[2], w4[3]}),
-                                                                          j == 0 ? (floatx16){} : p[u & 1], 0, 0, 0);
-                        if (tn == TNW - 1) av[g % NA][tm][j] = fetch_a(tm, j, g + NA < kChunk ? c * kChunk + g + NA : next * kChunk + g + NA - kChunk);
+                        p[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av[tm][q % NA]), __builtin_bit_cast(bf16x8, (uintx4){w4[0], w4[1], w4[2], w4[3]}),
+                                                                           j == 0 ? (floatx16){} : p[u & 1], 0, 0, 0);
+                        if (tn == TNW - 1) av[tm][q % NA] = q + NA < kChunk * NP ? fetch_a(tm, q + NA, c) : fetch_a(tm, q + NA - kChunk * NP, next);
                         // the sums of the tile before, and a share of the next stage's weights
 #pragma unroll
                         for (int e = 0; e < 16; e++)
-                            if (j == (e < 6 ? 1 : e < 11 ? 2 : 3)) acc[pg % NS][ptm][ptn][e] = fmaf(p[(u & 1) ^ 1][e], psc, acc[pg % NS][ptm][ptn][e]);
-                        if (TMW == 1 || (j & 1) == 0) {
+                            if (j == 1 + e / 4) acc[pg % NS][ptm][ptn][e] = fmaf(p[(u & 1) ^ 1][e], psc, acc[pg % NS][ptm][ptn][e]);
+                        if (TMW == 1 ? j < 4 : (j & 1) == 0 && j < 4) {
                             const int w = TMW == 1 ? j : 2 * tm + j / 2;
-                            int8x4_to_half(qn[w], bw[(st + 1) & 1][2 * w], bw[(st + 1) & 1][2 * w + 1]);
+                            int8x4_to_bf16(qn[w], bw[(st + 1) & 1][2 * w], bw[(st + 1) & 1][2 * w + 1]);
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     }
@@ -236,9 +241,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             if ((v & 1) == 0) { s.x += o.x; s.y += o.y; s.z += o.z; s.w += o.w; }
             else { s.x -= o.x; s.y -= o.y; s.z -= o.z; s.w -= o.w; }
         }
-        const float4 us = *reinterpret_cast<const float4 *>(a.unscale + row0);
         const float turn = c_begin & 1 ? -1.0f : 1.0f;
-        s.x *= us.x * turn; s.y *= us.y * turn; s.z *= us.z * turn; s.w *= us.w * turn;
+        s.x *= turn; s.y *= turn; s.z *= turn; s.w *= turn;
         const bool in = col < a.n;
         float badd = 0.0f;
         if (a.share_chunks == 0 && ep.bias && in) badd = ep.interleaved_bias ? ((col & 1) ? ep.bias2[col >> 1] : ep.bias[col >> 1]) : ep.bias[col];
@@ -328,11 +332,11 @@ bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared) {
     return norm ? m <= 512 || weights >= 3 << 18 : m <= 4096 && weights >= (m > 32 ? 4 << 20 : 8 << 20);
 }
 
-// floats of workspace: planes, row factors, the partial products where K is shared
+// floats of workspace: the activations' pieces, the partial products where K is shared
 int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, bool may_share) {
     const int64_t m_pad = round_up(m, 32), ka = round_up(q8_padded_k(k), kOperandChunk);
     const int shares = rows_plan(m, n_rows, k, may_share).shares;
-    return round_up(m_pad * ka, 64) + round_up(m_pad, 64) + (shares > 1 ? (int64_t)shares * m * n_rows : 0);
+    return m_pad * ka / 2 * kOperandPieces + (shares > 1 ? (int64_t)shares * m * n_rows : 0);
 }
 
 void launch_q8_gemm_rows(hipStream_t s, const float *x, const float *gamma, const float *beta, const int8_t *wq, const float *scales, float *out, int m, int k,
@@ -343,10 +347,9 @@ void launch_q8_gemm_rows(hipStream_t s, const float *x, const float *gamma, cons
     const int kp = q8_padded_k(k), ka = (int)round_up(kp, kOperandChunk), m_pad = (int)round_up(m, 32);
     const int m_tiles = (m + 32 * p.tmw - 1) / (32 * p.tmw), n_tiles = (n_rows + 32 * p.tnw - 1) / (32 * p.tnw);
     float *w = workspace;
-    uint16_t *planes = reinterpret_cast<uint16_t *>(w); w += round_up((int64_t)m_pad * ka, 64);
-    float *unscale = w;                                  w += round_up(m_pad, 64);
-    launch_split_operand(s, x, gamma, beta, planes, unscale, m, m_pad, k, ka);
-    GemmRowsArgs a{reinterpret_cast<const uintx4 *>(planes), wq, scales, unscale, out, m, n_rows, kp / kQ8Group, m_tiles, n_tiles, ep, 0, nullptr};
+    uint16_t *planes = reinterpret_cast<uint16_t *>(w); w += (int64_t)m_pad * ka / 2 * kOperandPieces;
+    launch_split_operand(s, x, gamma, beta, planes, m, m_pad, k, ka);
+    GemmRowsArgs a{reinterpret_cast<const uintx4 *>(planes), wq, scales, out, m, n_rows, kp / kQ8Group, m_tiles, n_tiles, ep, 0, nullptr};
     dim3 grid((unsigned)((n_tiles + 7) / 8 * 8 * m_tiles));
     if (p.shares > 1) {
         a.share_chunks = (chunks_of(k) + p.shares - 1) / p.shares;

@@ -2,9 +2,9 @@
 oracle's dequantised weights, at the edges of its tiles (32 or 64 rows and columns), of its 128-k chunks and of the ways it
 deals them: one to four wavefronts with work, K shared by several workgroups, odd and ragged everything.
 
-Gate on the rms error of the whole product: an activation is held to 2^-23, and an output is at most four sums (one a
+Gate on the rms error of the whole product: activations and weights are held exactly, and an output is at most four sums (one a
 wavefront) of G = K / 128 scaled group sums, whose n-th rounding is 2^-24 of a partial sum of n groups: 2^-23 (1 + sqrt(G / 2))
-of the product's rms covers both."""
+of the product's rms covers that and the roundings inside a group."""
 import numpy as np
 import pytest
 
@@ -54,6 +54,33 @@ def test_product_at_the_edges(dev, m, k, n, norm):
     dev.release(src, wq, xb, ob, gb)
     a = rms_normalised(x.astype(np.float64), gamma) if norm else x.astype(np.float64)
     check(got, a @ ref.q8_roundtrip(w).astype(np.float64), k, f"{m} x {k} x {n}", times=1 + norm)
+
+
+@pytest.mark.parametrize("m,k,n,norm", [(30, 2048, 5632, 0), (64, 4096, 3000, 0), (64, 4096, 1500, 1), (40, 11008, 1024, 0), (7, 12320, 1500, 1)])
+@pytest.mark.parametrize("spread", ["outlier", "groups"])
+def test_the_range_within_a_row_costs_no_bits(dev, m, k, n, norm, spread):
+    """A column of 1e4 to 1e8 whose weights are zero, and 32-k groups over twelve decades whose weights run the other way: an
+    activation's bits are its own, whatever the largest of its row is."""
+    rng = np.random.default_rng(k + norm)
+    w, x, gamma = (rng.standard_normal(s).astype(np.float32) for s in ((k, n), (m, k), (1, k)))
+    by = np.ones(k, np.float32)
+    if spread == "outlier":
+        w[33] = 0.0
+        by[33] = 1e8
+        x[: m // 2, 33] *= np.float32(1e-4)
+    else:
+        by[:] = np.repeat(10.0 ** rng.uniform(-6, 6, (k + 31) // 32), 32)[:k]
+        w /= by[:, None]
+    if norm:
+        gamma *= by                                      # (the normalised row has the range)
+    else:
+        x *= by
+    src, wq, xb, ob, gb = dev.upload(w), dev.alloc(HipNative.q8Floats(k, n)), dev.upload(x), dev.alloc(m * n), dev.upload(gamma)
+    Stream().q8_quantize(src, wq, k, n).q8_linear(xb, wq, ob, m, k, n, gamma=gb if norm else -1).run()
+    got = dev.download(ob, (m, n)).copy()
+    dev.release(src, wq, xb, ob, gb)
+    a = rms_normalised(x.astype(np.float64), gamma) if norm else x.astype(np.float64)
+    check(got, a @ ref.q8_roundtrip(w).astype(np.float64), k, f"{m} x {k} x {n} {spread}", times=1 + norm)
 
 
 @pytest.mark.parametrize("m,k,n", [(9, 200, 46), (64, 2052, 2100), (30, 8224, 1026)])
