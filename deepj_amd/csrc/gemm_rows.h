@@ -40,14 +40,29 @@ __device__ __forceinline__ void load_to_lds4(const void *base, uint32_t off, uin
 // kernels_gemm_f16.hip: the rows, normalised if gamma (and beta) say so, in that order; rows [m, m_pad) as zeros
 void launch_split_operand(hipStream_t s, const float *x, const float *gamma, const float *beta, uint16_t *planes, int m, int m_pad, int k, int kp);
 
-// kernels_matmul.hip: C = epilogue(sum of the slabs of partial products)
+// An estimate of a Q8 GEMM's time in us.  With x workgroups a compute unit, in `rounds` rounds, kk thousand k a workgroup and
+// `full` of its rows inside the matrix:
+//   fixed + per_x x + kk (per_k + again (rounds - 1) + per_kx x full) + (slabs m n shares + rows m k + weights n k) / 10^6.
+struct GemmCost {
+    double fixed, per_x, per_k, again, per_kx, slabs, rows, weights;
+    double us(double x, double rounds, double kk, double full, double m, double n, double k, int shares) const {
+        return fixed + per_x * x + kk * (per_k + again * (rounds - 1.0) + per_kx * x * full) + ((shares > 1 ? slabs * m * n * shares : 0.0) + rows * m * k + weights * n * k) * 1e-6;
+    }
+};
+
+// kernels_matmul.hip: what a product takes on k_gemm_q8, and into how many sums it deals an output's K
+struct Q8GemmEstimate { double us; int sums; };
+Q8GemmEstimate q8_gemm_estimate(int m, int n_rows, int k, bool norm, bool may_share);
+// C = epilogue(sum of the slabs of partial products)
 void launch_q8_sum_partials(hipStream_t s, const float *partial, float *out, int splits, int m, int n_rows, const GemmEpilogue &ep);
 
 // kernels_gemm_rows.hip
 void q8_gemm_rows_configure();   // once per device, before the first launch
-bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared);
-int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, bool may_share);   // may_share: a tile's K among several workgroups
+struct RowsPlan { int tmw, tnw, shares; double us; };      // a tile's rows and columns in units of 32, the workgroups that share its K
+// false: not a product for this kernel.  may_share: a tile's K among several workgroups
+bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared, bool may_share, RowsPlan *plan = nullptr);
+int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, const RowsPlan &plan);
 void launch_q8_gemm_rows(hipStream_t s, const float *x, const float *gamma, const float *beta, const int8_t *wq, const float *scales, float *out, int m, int k,
-                         int n_rows, const GemmEpilogue &ep, float *workspace, int64_t workspace_floats, bool may_share);
+                         int n_rows, const GemmEpilogue &ep, const RowsPlan &plan, float *workspace, int64_t workspace_floats);
 
 }  // namespace dj

@@ -16,17 +16,18 @@
 //
 // What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 33 us with the split, 39 where they come from
 // HBM, 87 on the bf16 kernels), then the activations, which every tile reads anew from L2 (12 KB for every 64 x 64 x 32: 64 x
-// 22016 46 us, 86; 200 x 11264 over 2048 47, 67), and on small weights two launches' latency (30 x 2304 over 768 9.0 us, 10.8).
+// 22016 46 us, 86; 200 x 11264 over 2048 47, 67), and on small weights two launches' latency (30 x 2304 over 768 8.9 us, 10.8).
 // Tried and slower, with two pieces: eight wavefronts a workgroup (two workgroups of four fill a compute unit better: 64 x 22016
 // 54 us against 49), the K loop or the epilogue rolled (3 % and 10 %), a 64 x 64 tile whose wavefronts share the activations
 // through LDS (latency of its reads and barriers: 400 x 768 over 3072 34 us against 22).
 //
 // Error against 64 bits, as a share of the result's rms: 0.77e-7 over 768 k, 0.81e-7 to 0.94e-7 over 2048, 0.94e-7 to 1.79e-7 over
-// 11008, by the number of sums a row is dealt to (four wavefronts, NS sets in each); 0.96e-7, 1.06e-7 and 1.2e-7 on the bf16
-// kernels where they share K.  It also hangs on the low pieces' products going first and on every second chunk's sign
-// (operand_negated).
+// 11008, by the number of sums an output is dealt to (four wavefronts, NS sets in each, the workgroups that share K); 0.96e-7 to
+// 1.88e-7 on k_gemm_q8.  No tile is taken that would do worse than k_gemm_q8 on the same product (rows_plan).  The error also
+// hangs on the low pieces' products going first and on every second chunk's sign (operand_negated).
 #include "dj_common.h"
 #include <algorithm>
+#include <cmath>
 #include "gemm_epilogue.h"
 #include "gemm_rows.h"
 
@@ -41,6 +42,7 @@ namespace {
 constexpr int kWaves = 4;
 constexpr int NP = 2 * kOperandPieces, kGroupWords = NP * 64;       // products of a 32 x 32 tile and 32 k; 16-byte words of 32 rows' activations
 constexpr int kChunk = kOperandChunk / kQ8Group;                   // scale groups a wavefront takes at a time: 128 k, one line of a weight row
+constexpr int sum_sets(int tmw, int tnw) { return tmw * tnw > 4 ? 1 : 4 / (tmw * tnw); }       // sums a wavefront deals an output's groups to
 constexpr int scale_row(int tnw) { return tnw > 2 ? 512 : 256; }
 constexpr int slot_bytes(int tnw) { return 32 * tnw * 128 + kChunk * scale_row(tnw); }       // a wavefront's chunk in LDS: weights [column][128], scales [group][64 or 128]
 
@@ -131,7 +133,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     static_assert(kChunk * NP % NA == 0, "a piece's register is known at compile time");
     uintx4 av[TMW][NA];
     auto fetch_a = [&](int i, int q, int c) __attribute__((always_inline)) { return (ap[i] + ((int64_t)c * kChunk + q / NP) * kGroupWords)[64 * (kOperandPieces * (q & 1) + 2 - (q % NP >> 1)) + lane]; };
-    constexpr int NS = TMW * TNW > 4 ? 1 : 4 / (TMW * TNW);       // sets of sums: a group's goes to set group % NS
+    constexpr int NS = sum_sets(TMW, TNW);             // a group's sum goes to set group % NS
     floatx16 acc[NS][TMW][TNW], p[2];
 #pragma unroll
     for (int e = 0; e < 16; e++) {
@@ -282,31 +284,38 @@ template <typename F> void each_kernel(F f) {
 
 int chunks_of(int k) { return (q8_padded_k(k) / kQ8Group + kChunk - 1) / kChunk; }
 
-// A tile's rows and columns in units of 32 and the workgroups that share its K: those of least estimated time, in us.  With x
-// tiles a compute unit and kk thousand k a wavefront, a launch takes
-//   fixed + per_x x + kk (per_k + again (rounds - 1) + per_kx x) + slabs m n shares / 10^6,
-// rounds being 1 up to one tile a compute unit, 2 up to two (two workgroups fit one) and x beyond.  Fitted to 200 shapes of 4 to
-// 400 rows, 768 to 50257 columns and 256 to 11008 k: the choice takes 1.006 times the best one's time on average, 1.08 at worst.
-// (200 x 2304 over 768: 32 x 32 12.5 us, 32 x 64 14.6, 64 x 32 14.4, 64 x 64 14.7; 200 x 11264 over 2048: 49, 41, 46, 41; 64 x
-// 22016 over 4096: 55, 48, 49, 46, and 42 with 64 x 96, whose 230 tiles are one round where 64 x 64 makes 344; 4 x 4096 over
-// 11008: 32 x 32 32, K shared by two 27, by four 29.)
-struct RowsPlan { int tmw, tnw, shares; };
-RowsPlan rows_plan(int m, int n_rows, int k, bool may_share) {
-    struct Shape { int tmw, tnw, shares; double fixed, per_x, per_k, again, per_kx, slabs; };
-    static const Shape shapes[] = {{1, 1, 1, 7.26, 0.42, 1.74, 1.0, 0.93, 0.0}, {1, 2, 1, 8.51, 0.75, 2.48, 1.8, 1.14, 0.0},
-                                   {2, 1, 1, 7.99, 0.25, 2.44, 1.75, 1.49, 0.0}, {2, 2, 1, 9.25, 1.16, 3.35, 2.66, 2.0, 0.0},
-                                   {1, 3, 1, 8.69, 2.87, 3.86, 4.54, 0.45, 0.0}, {2, 3, 1, 9.82, 4.83, 5.42, 7.58, 0.5, 0.0},
-                                   {1, 1, 2, 9.6, 0.42, 1.76, 0.73, 1.0, 6.0}, {1, 1, 4, 9.63, 1.1, 2.41, 0.29, 1.2, 0.52}};
+// The tile and the sharing of K of least estimated time.  A column tile's row tiles lie on one XCD, so what counts is the tiles of
+// the XCD that has most; two workgroups fit a compute unit, one where a tile is 96 columns wide (its lines take 112 KB of LDS).
+// Fitted to the times of 2 to 700 rows, 256 to 50257 columns and 256 to 11008 k, weights from the memory-side cache and from HBM: the
+// choice, k_gemm_q8 among it, takes 1.014 times the best one's time on average.  (200 x 2304 over 768: 32 x 32 12.4 us, 32 x 64
+// 14.6; 64 x 22016 over 4096: 64 x 64 56 us, 64 x 96, whose 230 tiles are one round where 64 x 64 makes 344, 47; 64 x 4096 over 11008:
+// 32 x 32 39, 32 x 64 with K shared by two 34.)
+//
+// No tile whose outputs would be worse than k_gemm_q8's: an output is `sums` sums of groups / sums terms each, and the squared error
+// against 64 bits, in units of 1e-14 of the result's squared rms, was 0.55 + 0.031 a term here (768 to 11008 k, every tile) and 1.07 +
+// 0.025 a term there.
+RowsPlan rows_plan(int m, int n_rows, int k, bool may_share, int sums_there) {
+    struct Shape { int tmw, tnw, shares; GemmCost cost; };
+    static constexpr Shape shapes[] = {
+        {1, 1, 1, {5.65, 0.2, 2.52, 2.03, 0.3, 0.0, 7.0, 0.075}},  {1, 2, 1, {6.46, 0.83, 3.59, 3.04, 0.0, 0.0, 6.5, 0.08}},
+        {2, 1, 1, {6.24, 0.04, 3.76, 3.12, 0.85, 0.0, 8.7, 0.035}}, {2, 2, 1, {7.52, 1.04, 5.37, 4.49, 0.54, 0.0, 9.5, 0.045}},
+        {1, 3, 1, {7.22, 3.37, 5.09, 5.28, 0.0, 0.0, 3.8, 0.03}},   {2, 3, 1, {9.13, 6.03, 6.36, 7.96, 0.0, 0.0, 7.9, 0.01}},
+        {1, 1, 2, {7.39, 0.64, 2.86, 1.6, 0.25, 1.8, 6.7, 0.093}},  {1, 1, 4, {7.9, 0.43, 2.49, 0.34, 1.4, 1.86, 6.4, 0.12}},
+        {2, 2, 2, {8.63, 0.11, 5.86, 4.19, 0.0, 3.25, 6.6, 0.1}},   {1, 2, 2, {7.96, 0.82, 3.95, 2.53, 0.0, 2.12, 5.8, 0.097}},
+        {1, 2, 4, {8.46, 0.61, 4.2, 2.12, 0.0, 2.08, 6.4, 0.137}}};
     RowsPlan best{};
-    double least = -1.0;
+    const int chunks = chunks_of(k), groups = q8_padded_k(k) / kQ8Group;
     for (const Shape &h : shapes) {
-        if (h.shares > 1 && (!may_share || (n_rows & 1) || chunks_of(k) < 2 * h.shares)) continue;      // k_sum_partials_q8 takes columns in pairs
-        const double x = (double)((m + 32 * h.tmw - 1) / (32 * h.tmw)) * (double)((n_rows + 32 * h.tnw - 1) / (32 * h.tnw)) * h.shares / 256.0;
-        const double rounds = x <= 1.0 ? 1.0 : x <= 2.0 ? 2.0 : x;
-        const int turns = ((chunks_of(k) + kWaves - 1) / kWaves + h.shares - 1) / h.shares;
-        const double kk = turns * kWaves * kChunk * kQ8Group * 1e-3;
-        const double t = h.fixed + h.per_x * x + kk * (h.per_k + h.again * (rounds - 1.0) + h.per_kx * x) + h.slabs * m * n_rows * h.shares * 1e-6;
-        if (least < 0.0 || t < least) { least = t; best = {h.tmw, h.tnw, h.shares}; }
+        if (h.shares > 1 && (!may_share || (n_rows & 1) || chunks < 2 * h.shares)) continue;      // k_sum_partials_q8 takes columns in pairs
+        const int sums = kWaves * sum_sets(h.tmw, h.tnw) * h.shares;
+        if ((double)groups / sums > 16.0 + 0.75 * groups / sums_there) continue;
+        const int64_t n_tiles = (n_rows + 32 * h.tnw - 1) / (32 * h.tnw), m_tiles = (m + 32 * h.tmw - 1) / (32 * h.tmw);
+        const double x = (double)((n_tiles + 7) / 8 * m_tiles * h.shares) / 32.0;
+        const int fit = h.tnw > 2 ? 1 : 2;
+        const double rounds = x <= 2 * fit ? ceil(x) : fit * ceil(x / fit);
+        const double kk = (((chunks + kWaves - 1) / kWaves + h.shares - 1) / h.shares) * kWaves * kChunk * kQ8Group * 1e-3;
+        const double us = h.cost.us(x, rounds, kk, 1.0, m, n_rows, k, h.shares);
+        if (!best.tmw || us < best.us) best = {h.tmw, h.tnw, h.shares, us};
     }
     return best;
 }
@@ -319,31 +328,30 @@ void q8_gemm_rows_configure() {
     });
 }
 
-// What the fp16 GEMM does not take: fewer than 256 rows without a copy of the weights in its layout (64 x 22016 over 4096 41 us,
-// 86 on the bf16 kernels), or few tiles, or a short K.  The rows' split into planes costs a launch.  Where they are normalised
-// first it takes that launch's place: 128 x 2048 over 2048 13.3 us against 17.9 on the bf16 kernels, 16 x 256 over 256 8.6, 9.6,
-// and only a multitude of rows against a small weight is better off there (700 x 768 over 256: 13.2, 11.8; 700 x 1536 over 512
-// 18.9, 20.9).  Where they are not, the weight has to be large enough to make up for it: 128 x 2048 over 2048 12.4, 14.1 and 30 x
-// 6144 over 2048 11.5, 16.1, but 16 x 2048 over 2048 11.8, 11.0 and 128 x 768 over 3072 14.6, 13.2.  (Past 4096 rows the bf16
-// kernels, which need no workspace for them.)  A lane's offset into a column tile's weights is 32 bits.
-bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared) {
-    if (k > (1 << 24) || q8_gemm_f16_shape_ok(m, n_rows, k, prepared)) return false;
-    const int64_t weights = (int64_t)n_rows * k;
-    return norm ? m <= 512 || weights >= 3 << 18 : m <= 4096 && weights >= (m > 32 ? 4 << 20 : 8 << 20);
+// What the fp16 GEMM does not take (fewer than 256 rows without a copy of the weights in its layout, few tiles, a short K) and
+// k_gemm_q8 would take longer for, by both estimates: the split of the rows into pieces costs a launch, which takes the place of
+// their normalisation where there is one (30 x 768 over 768 8.9 us against 10.8 on k_gemm_q8) and has to be made up for where there
+// is none (30 x 6144 over 2048 12.1, 16.0, but 8 x 768 over 256 6.7, 6.2 and 128 x 768 over 3072 15.0, 12.1).  Up to 768 rows: long
+// batches belong to k_gemm_q8's larger tiles (1500 x 50257 over 768 655 us, 504; 2048 rows 1058, 647; 1500 x 8001 over 1500 233, 158).  A
+// lane's offset into a column tile's weights is 32 bits.
+bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared, bool may_share, RowsPlan *plan) {
+    if (m > 768 || k > (1 << 24) || q8_gemm_f16_shape_ok(m, n_rows, k, prepared)) return false;
+    const Q8GemmEstimate there = q8_gemm_estimate(m, n_rows, k, norm, may_share);
+    const RowsPlan p = rows_plan(m, n_rows, k, may_share, there.sums);
+    if (plan) *plan = p;
+    return p.tmw && p.us < 0.98 * there.us - 0.2;
 }
 
 // floats of workspace: the activations' pieces, the partial products where K is shared
-int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, bool may_share) {
+int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, const RowsPlan &p) {
     const int64_t m_pad = round_up(m, 32), ka = round_up(q8_padded_k(k), kOperandChunk);
-    const int shares = rows_plan(m, n_rows, k, may_share).shares;
-    return m_pad * ka / 2 * kOperandPieces + (shares > 1 ? (int64_t)shares * m * n_rows : 0);
+    return m_pad * ka / 2 * kOperandPieces + (p.shares > 1 ? (int64_t)p.shares * m * n_rows : 0);
 }
 
 void launch_q8_gemm_rows(hipStream_t s, const float *x, const float *gamma, const float *beta, const int8_t *wq, const float *scales, float *out, int m, int k,
-                         int n_rows, const GemmEpilogue &ep, float *workspace, int64_t workspace_floats, bool may_share) {
-    if (workspace_floats < q8_gemm_rows_workspace_floats(m, n_rows, k, may_share)) fail("q8_gemm_rows: workspace too small");
+                         int n_rows, const GemmEpilogue &ep, const RowsPlan &p, float *workspace, int64_t workspace_floats) {
+    if (workspace_floats < q8_gemm_rows_workspace_floats(m, n_rows, k, p)) fail("q8_gemm_rows: workspace too small");
     if (ep.swiglu && ((n_rows & 1) || ep.residual || ep.gelu)) fail("q8_gemm_rows: the SwiGLU epilogue needs an even row count and takes no residual or GELU");
-    const RowsPlan p = rows_plan(m, n_rows, k, may_share);
     const int kp = q8_padded_k(k), ka = (int)round_up(kp, kOperandChunk), m_pad = (int)round_up(m, 32);
     const int m_tiles = (m + 32 * p.tmw - 1) / (32 * p.tmw), n_tiles = (n_rows + 32 * p.tnw - 1) / (32 * p.tnw);
     float *w = workspace;

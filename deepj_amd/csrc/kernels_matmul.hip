@@ -631,6 +631,33 @@ int q8_gemm_k_shares(int m, int n_rows, int k) {
     return (steps + per - 1) / per;
 }
 
+// Two 128 x 128 workgroups fit a CU, so the tiles run in rounds of 512; when the last round would be mostly
+// empty (352 or 704 tiles), 64 x 128 tiles - twice as many, three to four per CU - finish sooner
+// (512 x 11264 x 2048: 101 against 113 us; 1024 rows: 194 against 229 us).
+static bool last_round_empty(int m, int n_rows) {
+    const int64_t tiles = (int64_t)((n_rows + BN2 - 1) / BN2) * ((m + BM2 - 1) / BM2), rounds = (tiles + 511) / 512;
+    return tiles * 100 < rounds * 512 * 85;
+}
+
+// Fitted to the launches below over 2 to 700 rows, 256 to 50257 columns and 256 to 11008 k, with the weights in the memory-side
+// cache and from HBM: 5 % of the time on average.  A normalisation in front is a launch of its own.
+Q8GemmEstimate q8_gemm_estimate(int m, int n_rows, int k, bool norm, bool may_share) {
+    static constexpr GemmCost shared{5.83, 0.38, 8.95, 0.0, 0.34, 2.08, 0.0, 0.038}, few{5.08, 0.91, 8.37, 8.6, 1.73, 0.0, 0.0, 0.016},
+                              many{0.0, 2.3, 13.4, 4.7, 2.6, 0.0, 0.0, 0.0}, wide{9.0, 0.9, 8.0, 4.6, 10.7, 0.0, 0.0, 0.17}, big{0.0, 9.1, 0.0, 5.9, 16.4, 0.0, 0.0, 0.9};
+    const bool large = use_big_tile(m, n_rows), by64 = large && last_round_empty(m, n_rows);
+    const int tm = large && !by64 ? BM2 : BM, tn = large ? BN2 : BN;
+    const int64_t m_tiles = (m + tm - 1) / tm, tiles = m_tiles * ((n_rows + tn - 1) / tn);
+    const int shares = may_share ? q8_gemm_k_shares(m, n_rows, k) : 1;
+    const bool four_sets = !large && tiles <= kFewTiles;
+    const GemmCost &c = by64 ? wide : large ? big : !four_sets ? many : shares > 1 ? shared : few;
+    const int fit = by64 ? 3 : large ? 2 : !four_sets ? 4 : shares > 1 ? 1 : 2;         // workgroups on a compute unit
+    constexpr int step = kQ8Group * kGroupsFew;
+    const int steps = (q8_padded_k(k) + step - 1) / step;
+    const double x = (double)tiles * shares / 256.0, kk = (steps + shares - 1) / shares * step * 1e-3;
+    const double us = c.us(x, x <= fit ? ceil(x) : x, kk, (double)m / (double)(m_tiles * tm), m, n_rows, k, shares);
+    return {us + (norm ? 2.2 + 4e-6 * m * k : 0.0), (four_sets ? kSetsFew : 1) * shares};
+}
+
 int64_t q8_gemm_workspace_floats(int m, int n_rows, int k) {
     const int shares = q8_gemm_k_shares(m, n_rows, k);
     return shares > 1 ? (int64_t)shares * m * n_rows : 0;
@@ -653,11 +680,7 @@ void launch_q8_gemm(hipStream_t s, const float *x, const int8_t *wq, const float
     GemmEpilogue ep{bias, bias2, residual, interleaved_bias, m_dev, m_extra, gelu, swiglu};
     if (!m_dev && use_big_tile(m, n_rows)) {       // a device-side row count is usually far below m: keep small tiles
         dim3 grid2((n_rows + BN2 - 1) / BN2, (m + BM2 - 1) / BM2);
-        // Two 128 x 128 workgroups fit a CU, so the tiles run in rounds of 512; when the last round would be mostly
-        // empty (352 or 704 tiles), 64 x 128 tiles - twice as many, three to four per CU - finish sooner
-        // (512 x 11264 x 2048: 101 against 113 us; 1024 rows: 194 against 229 us).
-        const int64_t tiles = (int64_t)grid2.x * grid2.y, rounds = (tiles + 511) / 512;
-        if (tiles * 100 < rounds * 512 * 85) {
+        if (last_round_empty(m, n_rows)) {
             dim3 gridw(grid2.x, (m + 63) / 64);
             launch_kernel((k_gemm_q8<1, 2, 2, 1>), gridw, dim3(256), 0, s, x, wq, scales, out, m, n_rows, k, q8_padded_k(k), ep, 0, nullptr);
             return;

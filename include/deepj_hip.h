@@ -289,6 +289,12 @@ void deepj_hip_q8_gemm_tile(int32_t m, int32_t k, int32_t rows, int32_t *tile_ro
 /* the same for a weight that Q8_PREPARE has written in the fp16 GEMM's layout: from 16 rows on instead of 256 (64-row tiles,
  * K shared so that as many workgroups as possible stream weights) */
 void deepj_hip_q8_gemm_tile_prepared(int32_t m, int32_t k, int32_t rows, int32_t *tile_rows, int32_t *tile_cols, int32_t *k_shares);
+/* The same for the kernel that multiplies a batch of rows straight from the int8 weights (32 or 64 rows by 32, 64 or 96
+ * columns a tile): 1 when a Q8_LINEAR of m rows with (norm) or without a normalisation prologue runs on it, 0 when on
+ * another (a single row within the matvec's reach never does).  alloc_free: under deepj_hip_flush_ops_noalloc, as far as its
+ * fixed workspace holds the rows. */
+int32_t deepj_hip_q8_gemm_rows_tile(int32_t m, int32_t k, int32_t rows, int32_t norm, int32_t prepared, int32_t alloc_free, int32_t *tile_rows,
+                                    int32_t *tile_cols, int32_t *k_shares);
 /* Host arithmetic only (no GPU call): the last byte + 1 that the fp16 GEMM's direct global -> LDS loads reach in its three
  * operand buffers {activation planes, fp16 weights, transposed scales} for a tile of tile_rows x tile_cols (128 or 64 rows
  * by 256 or 192 columns; tile_rows 0: the tile the library would choose), and the bytes those buffers hold.  Returns 1

@@ -56,11 +56,42 @@ def test_product_at_the_edges(dev, m, k, n, norm):
     check(got, a @ ref.q8_roundtrip(w).astype(np.float64), k, f"{m} x {k} x {n}", times=1 + norm)
 
 
-@pytest.mark.parametrize("m,k,n,norm", [(30, 2048, 5632, 0), (64, 4096, 3000, 0), (64, 4096, 1500, 1), (40, 11008, 1024, 0), (7, 12320, 1500, 1)])
+# (tile rows, tile columns, workgroups that share its K), every one of them: K of whole chunks, whose scales come in one load, and
+# ragged, whose scales come group by group; columns that end inside a tile
+EVERY_TILE = [((32, 32, 1), (2, 128, 33, 1)), ((32, 32, 1), (2, 40, 33, 1)), ((32, 32, 2), (30, 3072, 2050, 1)), ((32, 32, 2), (30, 3000, 2050, 1)),
+              ((32, 32, 4), (2, 1152, 250, 1)), ((32, 32, 4), (2, 1028, 250, 1)), ((32, 64, 1), (640, 640, 500, 1)), ((32, 64, 1), (640, 600, 500, 1)),
+              ((32, 64, 2), (640, 2048, 1002, 1)), ((32, 64, 2), (640, 3000, 1002, 1)), ((32, 64, 4), (200, 4096, 1500, 1)), ((32, 64, 4), (700, 6004, 500, 1)),
+              ((32, 96, 1), (400, 1152, 1500, 1)), ((32, 96, 1), (400, 1028, 1500, 1)), ((64, 32, 1), (33, 256, 6150, 1)), ((64, 32, 1), (33, 200, 6150, 1)),
+              ((64, 64, 1), (700, 512, 3010, 1)), ((64, 64, 1), (700, 416, 3010, 1)), ((64, 64, 2), (130, 6144, 2050, 1)), ((64, 64, 2), (130, 6004, 2050, 1)),
+              ((64, 96, 1), (640, 1152, 2049, 1)), ((64, 96, 1), (640, 1028, 2049, 1))]
+
+
+@pytest.mark.parametrize("tile,shape", EVERY_TILE)
+def test_product_on_every_tile(dev, tile, shape):
+    assert HipNative.q8GemmRowsTile(*shape) == tile
+    test_product_at_the_edges(dev, *shape)
+
+
+@pytest.mark.parametrize("m,k,n,there", [(128, 6144, 4096, 1.26e-7), (250, 8224, 2050, 1.68e-7), (96, 2048, 6144, 1.12e-7)])
+def test_error_is_no_larger_than_the_kernel_it_stands_in_for(dev, m, k, n, there):
+    """`there`: k_gemm_q8's rms error on the same product, with the numbers of other seeds 1 % apart."""
+    assert HipNative.q8GemmRowsTile(m, k, n)[0]
+    w, x = JavaRandom(5).tensor(k, n, k ** -0.5), JavaRandom(6).tensor(m, k, 1.0)
+    src, wq, xb, ob = dev.upload(w), dev.alloc(HipNative.q8Floats(k, n)), dev.upload(x), dev.alloc(m * n)
+    Stream().q8_quantize(src, wq, k, n).q8_linear(xb, wq, ob, m, k, n).run()
+    got = dev.download(ob, (m, n)).copy()
+    dev.release(src, wq, xb, ob)
+    exp = x.astype(np.float64) @ ref.q8_roundtrip(w).astype(np.float64)
+    err = float(np.sqrt(np.mean((got - exp) ** 2) / np.mean(exp ** 2)))
+    assert err <= 1.01 * there, f"rms error {err:.3e}"
+
+
+@pytest.mark.parametrize("m,k,n,norm", [(30, 2048, 5632, 0), (96, 4096, 4500, 0), (64, 4096, 6000, 1), (30, 11008, 1023, 0), (7, 12320, 1500, 1)])
 @pytest.mark.parametrize("spread", ["outlier", "groups"])
 def test_the_range_within_a_row_costs_no_bits(dev, m, k, n, norm, spread):
     """A column of 1e4 to 1e8 whose weights are zero, and 32-k groups over twelve decades whose weights run the other way: an
     activation's bits are its own, whatever the largest of its row is."""
+    assert HipNative.q8GemmRowsTile(m, k, n, norm)[0]
     rng = np.random.default_rng(k + norm)
     w, x, gamma = (rng.standard_normal(s).astype(np.float32) for s in ((k, n), (m, k), (1, k)))
     by = np.ones(k, np.float32)
@@ -120,8 +151,9 @@ def test_prologues_and_epilogues(dev, m, k, n, epilogue):
     check(got, y, k, epilogue, times=2)
 
 
-def test_a_row_that_is_not_finite_stays_alone(dev):
-    m, k, n = 40, 600, 8000
+@pytest.mark.parametrize("m,k,n,taken", [(40, 600, 8000, False), (40, 2048, 8000, True)])
+def test_a_row_that_is_not_finite_stays_alone(dev, m, k, n, taken):
+    assert (HipNative.q8GemmRowsTile(m, k, n)[0] > 0) == taken           # k_gemm_q8 the other one
     w, x = JavaRandom(5).tensor(k, n, 0.05), JavaRandom(6).tensor(m, k, 1.0)
     src, wq, xb, ob = dev.upload(w), dev.alloc(HipNative.q8Floats(k, n)), dev.upload(x), dev.alloc(m * n)
     op = Stream().q8_quantize(src, wq, k, n).q8_linear(xb, wq, ob, m, k, n)
