@@ -151,7 +151,10 @@ struct Q8LinearPair {                  // two weights over one RMS-normalised ro
 };
 bool q8_linear_pair_ok(int k);
 void launch_q8_linear_pair(hipStream_t s, const Q8LinearPair &p);
-void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_t workspace_floats);
+// pieces: a block for the products that multiply a batch of rows straight from the int8 weights; others are taken where it is
+// smaller than q8_linear_pieces_floats
+void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_t workspace_floats, float *pieces, int64_t pieces_floats);
+int64_t q8_linear_pieces_floats(int m, int k, int n, int flags, bool prepared);
 int64_t q8_linear_workspace_floats(int m, int k, int n, int flags);
 // The size at which launch_q8_linear takes its fastest path (>= the one above); callers that may grow their workspace
 // offer this much, callers that may not offer what they have.

@@ -690,11 +690,17 @@ int64_t q8_linear_preferred_workspace_floats(int m, int k, int n, int flags, boo
     const int64_t ws = q8_linear_workspace_floats(m, k, n, flags);
     const int n_rows = (flags & DJ_LIN_SWIGLU) ? 2 * n : n;
     const bool mv = (m == 1) && matvec_supported(k);
-    RowsPlan plan;
-    if (!mv && q8_gemm_rows_ok(m, n_rows, k, (flags & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM)) != 0, prepared, true, &plan)) return std::max(ws, q8_gemm_rows_workspace_floats(m, n_rows, k, plan));
+    if (q8_linear_pieces_floats(m, k, n, flags, prepared) > 0) return ws;
     if (!mv && q8_gemm_f16_shape_ok(m, n_rows, k, prepared)) return std::max(ws, q8_gemm_f16_workspace_floats(m, n_rows, k, prepared));
     if (!mv) return ws + q8_gemm_workspace_floats(m, n_rows, k);      // the partial products of a K-sharing launch
     return ws;
+}
+
+int64_t q8_linear_pieces_floats(int m, int k, int n, int flags, bool prepared) {
+    const int n_rows = (flags & DJ_LIN_SWIGLU) ? 2 * n : n;
+    RowsPlan plan;
+    if ((m == 1 && matvec_supported(k)) || !q8_gemm_rows_ok(m, n_rows, k, (flags & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM)) != 0, prepared, true, &plan)) return 0;
+    return q8_gemm_rows_workspace_floats(m, n_rows, k, plan);
 }
 
 bool q8_linear_pair_ok(int k) { return k > 0 && (k & 3) == 0 && k <= 4096; }
@@ -728,7 +734,7 @@ void launch_q8_linear_pair(hipStream_t s, const Q8LinearPair &p) {
     }
 }
 
-void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_t workspace_floats) {
+void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_t workspace_floats, float *pieces, int64_t pieces_floats) {
     if (p.m <= 0 || p.n <= 0) return;
     const bool swiglu = (p.flags & DJ_LIN_SWIGLU) != 0;
     const bool layernorm = (p.flags & DJ_LIN_LAYERNORM) != 0;
@@ -769,14 +775,14 @@ void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_
     // normalisation happens on the rows' way into that layout
     const int n_rows = swiglu ? 2 * p.n : p.n;
     const bool rope = p.rope.q != nullptr;
-    // Fewer rows: straight from the int8 weights.  With a workspace that cannot grow where the operands fit it, whatever copies of
+    // Fewer rows: straight from the int8 weights.  With memory that cannot grow where the operands fit it, whatever copies of
     // the weights exist, and without sharing K: one rule for the allocation-free entry point.
     const bool may_share = !p.small_workspace_only;
     RowsPlan plan;
     if (!p.m_dev && !rope && !(p.chain && p.chain->planes_ready) && q8_gemm_rows_ok(p.m, n_rows, p.k, gamma != nullptr, p.prepared && may_share, may_share, &plan) &&
-        workspace_floats >= q8_gemm_rows_workspace_floats(p.m, n_rows, p.k, plan)) {
+        pieces_floats >= q8_gemm_rows_workspace_floats(p.m, n_rows, p.k, plan)) {
         const GemmEpilogue ep{bias, swiglu ? bias2 : nullptr, residual, swiglu, nullptr, 0, swiglu ? 0 : gelu, swiglu, RopeStore{}};
-        launch_q8_gemm_rows(s, p.x, gamma, beta, p.wq, p.scales, p.out, p.m, p.k, n_rows, ep, plan, workspace, workspace_floats);
+        launch_q8_gemm_rows(s, p.x, gamma, beta, p.wq, p.scales, p.out, p.m, p.k, n_rows, ep, plan, pieces, pieces_floats);
         return;
     }
     if (!p.m_dev && !p.small_workspace_only && q8_gemm_f16_shape_ok(p.m, n_rows, p.k, p.prepared != nullptr) && workspace_floats >= q8_gemm_f16_workspace_floats(p.m, n_rows, p.k, p.prepared != nullptr)) {

@@ -43,13 +43,19 @@ struct Buffer {
     int64_t floats = 0;       // size the caller asked for
 };
 
+// Floats of device scratch that a stream needs: the workspace, and the block for the Q8 GEMM that multiplies a batch of rows
+// straight from the int8 weights (the rows in pieces, its partial products).
+struct Scratch { int64_t workspace = 0, row_pieces = 0; };
+
 // A captured graph holds raw device addresses.  The buffers its stream named (id, address at capture time) and
-// the workspace it used are remembered, and a replay is refused once any of them is gone or has moved.
+// the workspace it used are remembered, and a replay is refused once any of them is gone or has moved.  The block of pieces
+// it used is kept for it instead: products that need no workspace stay launchable whatever other streams need.
 struct Graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     std::vector<std::pair<int32_t, void *>> refs;
     float *workspace = nullptr;       // set when the stream needs workspace
+    float *row_pieces = nullptr;      // set when the stream needs it; freed with the last graph once a larger one has replaced it
     // (weight id, prepared id) of every Q8_LINEAR that was captured reading a prepared copy the stream had not written
     // itself: once the copy stops standing for the weights (they were written again) a replay would use stale weights
     std::vector<std::pair<int32_t, int32_t>> prepared, self_prepared;
@@ -76,6 +82,8 @@ struct Runtime {
     size_t cache_limit = (size_t)16 << 30;
     float *workspace = nullptr;
     int64_t workspace_floats = 0;
+    float *row_pieces = nullptr;
+    int64_t row_pieces_floats = 0;
     // Host <-> device traffic (section "transfers"): one pinned block holds the upload ring, the download stage and the
     // flags that a download's chunks set.
     unsigned char *pinned = nullptr;
@@ -485,6 +493,23 @@ void ensure_workspace(int64_t floats) {
     g.workspace_floats = want;
 }
 
+bool graph_holds_pieces(const float *block) {
+    return std::any_of(g.graphs.begin(), g.graphs.end(), [&](const auto &kv) { return kv.second.row_pieces == block; });
+}
+
+void ensure_scratch(const Scratch &need) {
+    ensure_workspace(need.workspace);
+    if (g.no_alloc || need.row_pieces <= g.row_pieces_floats) return;      // (the fixed array: products that it does not hold take another kernel)
+    DJ_HIP(hipStreamSynchronize(g.stream));
+    if (g.row_pieces && !graph_holds_pieces(g.row_pieces)) DJ_HIP(hipFree(g.row_pieces));
+    g.row_pieces = nullptr;
+    g.row_pieces_floats = 0;
+    const int64_t want = std::max<int64_t>(need.row_pieces, (int64_t)1 << 20);
+    DJ_HIP(hipMalloc((void **)&g.row_pieces, (size_t)want * 4));
+    g.driver_allocs++;
+    g.row_pieces_floats = want;
+}
+
 // ── stream interpreter ──────────────────────────────────────────────────────
 
 struct Cursor {
@@ -492,12 +517,24 @@ struct Cursor {
     int32_t len;
     int32_t pos;
     bool dry;          // validate only
-    int64_t ws_need;   // workspace floats the stream needs (collected in the dry pass)
+    Scratch need;      // collected in the dry pass
     int32_t skip = 0;  // words behind this op whose ops its launch has taken along
     bool alone = false; // every op by itself (per-op timing)
 };
 
 const char *op_name(int op);
+
+// An op's device scratch: collected in the dry pass, in a captured graph's run pass noted as what its launches hold (weights that
+// the stream itself writes or prepares may take another kernel there than the dry pass saw, in whatever scratch there is)
+void need_scratch(Cursor &c, int64_t workspace, int64_t pieces) {
+    if (c.dry) {
+        c.need.workspace = std::max(c.need.workspace, workspace);
+        c.need.row_pieces = std::max(c.need.row_pieces, pieces);
+    } else if (g.capture_into) {
+        if (workspace > 0 || pieces > g.row_pieces_floats) g.capture_into->workspace = g.workspace;
+        if (pieces > 0) g.capture_into->row_pieces = g.row_pieces;
+    }
+}
 
 int stride_of(int op) {
     switch (op) {
@@ -831,7 +868,7 @@ void exec_one(Cursor &c) {
             }
             int64_t ws = g.no_alloc ? q8_linear_workspace_floats((int)m, (int)k, (int)n, flags)
                                     : q8_linear_preferred_workspace_floats((int)m, (int)k, (int)n, flags, p.prepared != nullptr);
-            if (c.dry) c.ws_need = std::max(c.ws_need, ws);
+            need_scratch(c, ws, g.no_alloc ? 0 : q8_linear_pieces_floats((int)m, (int)k, (int)n, flags, p.prepared != nullptr));
             // One rule for the allocation-free entry point, whatever happens to fit its fixed array: the many-row
             // fp16 GEMM (whose operands live in a workspace sized by the shape) is never taken there.
             p.small_workspace_only = g.no_alloc;
@@ -856,7 +893,7 @@ void exec_one(Cursor &c) {
                 }
                 p.chain = &chain;
             }
-            if (run) launch_q8_linear(s, p, g.workspace, g.workspace_floats);
+            if (run) launch_q8_linear(s, p, g.workspace, g.workspace_floats, g.row_pieces, g.row_pieces_floats);
             if (chain.left_planes) {
                 g.chain.cmd = c.cmd; g.chain.pos = next_pos; g.chain.x_id = w[3]; g.chain.gamma_id = next_gamma_id;
                 g.chain.m = m; g.chain.k = n; g.chain.valid = true;
@@ -902,11 +939,11 @@ void exec_one(Cursor &c) {
                 if (std::find(own.begin(), own.end(), pr) == own.end()) g.capture_into->prepared.push_back(pr);
             }
             const int64_t ws = q8_linear_preferred_workspace_floats((int)m, (int)k, (int)rows, flags, p.prepared != nullptr);
-            if (c.dry) c.ws_need = std::max(c.ws_need, ws);
+            need_scratch(c, ws, 0);
             GemmChain chain;
             chain.planes_ready = chained(w[1], w[8], flags, m, k);
             p.chain = &chain;
-            if (run) launch_q8_linear(s, p, g.workspace, g.workspace_floats);
+            if (run) launch_q8_linear(s, p, g.workspace, g.workspace_floats, g.row_pieces, g.row_pieces_floats);
             break;
         }
         case DJ_OP_RMSNORM: {
@@ -1197,7 +1234,7 @@ void exec_one(Cursor &c) {
             p.gamma = p.bias = p.bias2 = p.residual = nullptr;
             p.m_dev = reinterpret_cast<const int32_t *>(buf(w[7], 4, op, "state"));
             p.m_extra = (int)extra;
-            if (run) launch_q8_linear(s, p, g.workspace, g.workspace_floats);
+            if (run) launch_q8_linear(s, p, g.workspace, g.workspace_floats, g.row_pieces, g.row_pieces_floats);
             break;
         }
         case DJ_OP_COPY: {
@@ -1249,7 +1286,7 @@ void exec_one(Cursor &c) {
     }
 }
 
-void walk(const int32_t *cmd, int32_t len, bool dry, int64_t *ws_need) {
+void walk(const int32_t *cmd, int32_t len, bool dry, Scratch *need) {
     Cursor c{cmd, len, 0, dry, 0};
     g.chain.valid = false;          // nothing carries over from an earlier stream (or from one that ended in an error)
     while (c.pos < len) {
@@ -1262,16 +1299,16 @@ void walk(const int32_t *cmd, int32_t len, bool dry, int64_t *ws_need) {
         c.pos += stride + c.skip;
         c.skip = 0;
     }
-    if (ws_need) *ws_need = c.ws_need;
+    if (need) *need = c.need;
 }
 
 void run_stream(const int32_t *cmd, int32_t len) {
     if (len < 0) fail("flushOps: negative stream length");
     if (len > 0 && !cmd) fail("flushOps: null command stream");
-    int64_t ws = 0;
-    walk(cmd, len, true, &ws);      // validate everything first
+    Scratch need;
+    walk(cmd, len, true, &need);      // validate everything first
     launch_uploads();
-    ensure_workspace(ws);
+    ensure_scratch(need);
     walk(cmd, len, false, nullptr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) fail(std::string("kernel launch failed: ") + hipGetErrorString(e));
@@ -1431,21 +1468,21 @@ int deepj_hip_flush_ops_noalloc(const int32_t *cmd, int32_t len) {
         if (!g.ready)
             fail("flush_ops_noalloc: the runtime is not initialised (initialisation allocates: call deepj_hip_init first)");
         struct Scope {
-            float *ws = g.workspace; int64_t wsf = g.workspace_floats; unsigned *ctr = g.attn_counters;
+            float *ws = g.workspace, *pieces = g.row_pieces; int64_t wsf = g.workspace_floats, pf = g.row_pieces_floats; unsigned *ctr = g.attn_counters;
             Scope() {
                 g.no_alloc = true;
                 g.attn_counters = reinterpret_cast<unsigned *>(g.static_scratch);
-                g.workspace = reinterpret_cast<float *>(g.static_scratch + kStaticCounterBytes);
-                g.workspace_floats = kStaticWorkspaceFloats;
+                g.workspace = g.row_pieces = reinterpret_cast<float *>(g.static_scratch + kStaticCounterBytes);      // (no op uses both)
+                g.workspace_floats = g.row_pieces_floats = kStaticWorkspaceFloats;
             }
-            ~Scope() { g.no_alloc = false; g.workspace = ws; g.workspace_floats = wsf; g.attn_counters = ctr; }
+            ~Scope() { g.no_alloc = false; g.workspace = ws; g.workspace_floats = wsf; g.row_pieces = pieces; g.row_pieces_floats = pf; g.attn_counters = ctr; }
         } scope;
         if (len < 0) fail("flushOps: negative stream length");
         if (len > 0 && !cmd) fail("flushOps: null command stream");
-        int64_t ws = 0;
-        walk(cmd, len, true, &ws);
+        Scratch need;
+        walk(cmd, len, true, &need);
         launch_uploads();
-        ensure_workspace(ws);           // only checks the need against the static size here
+        ensure_scratch(need);           // only checks the need against the static size here
         launch_fill(g.stream, reinterpret_cast<uint32_t *>(g.attn_counters), 0u, kAttnCounterHeads);
         walk(cmd, len, false, nullptr);
         hipError_t e = hipGetLastError();
@@ -1485,6 +1522,12 @@ int deepj_hip_shutdown(void) {
             if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
             if (kv.second.graph) (void)hipGraphDestroy(kv.second.graph);
         }
+        std::vector<float *> blocks{g.row_pieces};
+        for (auto &kv : g.graphs)
+            if (std::find(blocks.begin(), blocks.end(), kv.second.row_pieces) == blocks.end()) blocks.push_back(kv.second.row_pieces);
+        for (float *b : blocks)
+            if (b) (void)hipFree(b);
+        g.row_pieces = nullptr; g.row_pieces_floats = 0;
         g.graphs.clear();
         for (auto &kv : g.live) (void)hipFree(kv.second.ptr);
         g.live.clear();
@@ -1607,10 +1650,10 @@ int deepj_hip_time_ops(const int32_t *cmd, int32_t len, int32_t iters, float *ms
     return guarded([&] {
         ensure_init();
         if (iters <= 0 || !ms_total) fail("time_ops: bad arguments");
-        int64_t ws = 0;
-        walk(cmd, len, true, &ws);
+        Scratch need;
+        walk(cmd, len, true, &need);
         launch_uploads();
-        ensure_workspace(ws);
+        ensure_scratch(need);
         hipEvent_t e0, e1;
         DJ_HIP(hipEventCreate(&e0));
         DJ_HIP(hipEventCreate(&e1));
@@ -1636,10 +1679,10 @@ int deepj_hip_clock_probe(const int32_t *cmd, int32_t len, int32_t iters, int32_
         ensure_init();
         if (iters < 0 || samples <= 0 || samples > (1 << 20) || sleep_reps < 0 || sleep_reps > 4096 || !pairs || !window)
             fail("clock_probe: bad arguments");
-        int64_t ws = 0;
-        if (len > 0) walk(cmd, len, true, &ws);
+        Scratch need;
+        if (len > 0) walk(cmd, len, true, &need);
         launch_uploads();
-        ensure_workspace(ws);
+        ensure_scratch(need);
         hipStream_t side = nullptr;
         unsigned long long *d = nullptr;
         DJ_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
@@ -1672,10 +1715,10 @@ int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float 
     return guarded([&] {
         ensure_init();
         if (iters <= 0 || !us_per_op || capacity < 0) fail("profile_ops: bad arguments");
-        int64_t ws = 0;
-        walk(cmd, len, true, &ws);
+        Scratch need;
+        walk(cmd, len, true, &need);
         launch_uploads();
-        ensure_workspace(ws);
+        ensure_scratch(need);
         std::vector<int32_t> starts;                 // word offset of every op
         for (int32_t pos = 0; pos < len; pos += stride_of(cmd[pos])) starts.push_back(pos);
         const int n = (int)starts.size();
@@ -1738,11 +1781,11 @@ int deepj_hip_graph_capture(const int32_t *cmd, int32_t len, int32_t *handle) {
     return guarded([&] {
         ensure_init();
         if (!handle) fail("graph_capture: null handle");
-        int64_t ws = 0;
+        Scratch need;
         Graph gr;
         g.track = &gr.refs;
         try {
-            walk(cmd, len, true, &ws);
+            walk(cmd, len, true, &need);
         } catch (...) {
             g.track = nullptr;
             throw;
@@ -1751,8 +1794,7 @@ int deepj_hip_graph_capture(const int32_t *cmd, int32_t len, int32_t *handle) {
         std::sort(gr.refs.begin(), gr.refs.end());
         gr.refs.erase(std::unique(gr.refs.begin(), gr.refs.end()), gr.refs.end());
         launch_uploads();
-        ensure_workspace(ws);
-        if (ws > 0) gr.workspace = g.workspace;
+        ensure_scratch(need);
         DJ_HIP(hipStreamSynchronize(g.stream));
         DJ_HIP(hipStreamBeginCapture(g.stream, hipStreamCaptureModeThreadLocal));
         g.capturing = true;
@@ -1827,7 +1869,9 @@ int deepj_hip_graph_destroy(int32_t handle) {
         DJ_HIP(hipStreamSynchronize(g.stream));
         (void)hipGraphExecDestroy(it->second.exec);
         (void)hipGraphDestroy(it->second.graph);
+        float *pieces = it->second.row_pieces;
         g.graphs.erase(it);
+        if (pieces && pieces != g.row_pieces && !graph_holds_pieces(pieces)) DJ_HIP(hipFree(pieces));
     });
 }
 

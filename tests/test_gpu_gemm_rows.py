@@ -167,3 +167,35 @@ def test_a_row_that_is_not_finite_stays_alone(dev, m, k, n, taken):
     assert not np.isfinite(got[[3, 35]]).any()
     keep = [r for r in range(m) if r not in (3, 35)]
     assert np.array_equal(got[keep], clean[keep])
+
+
+def test_a_captured_product_outlives_a_larger_one(dev):
+    """A product without a normalisation needs no workspace: a graph of it stays launchable whatever other streams need, over the
+    block of pieces that it was captured with, also beside graphs of other blocks and once one of its own block is gone."""
+    m, k, n = 30, 2048, 6144
+    big_m, big_k, big_n = 767, 32768, 2050               # 41 Mi floats of pieces and partial products: more than any other test's
+    assert HipNative.q8GemmRowsTile(m, k, n)[0] and HipNative.q8GemmRowsTile(big_m, big_k, big_n)[0]
+    w, x = JavaRandom(5).tensor(k, n, k ** -0.5), JavaRandom(6).tensor(m, k, 1.0)
+    src, wq, xb, ob = dev.upload(w), dev.alloc(HipNative.q8Floats(k, n)), dev.upload(x), dev.alloc(m * n)
+    Stream().q8_quantize(src, wq, k, n).run()
+    words = Stream().q8_linear(xb, wq, ob, m, k, n)
+    words.run()
+    expected = dev.download(ob, (m, n)).copy()
+    big_x, big_w, big_o = dev.alloc(big_m * big_k), dev.alloc(HipNative.q8Floats(big_k, big_n)), dev.alloc(big_m * big_n)
+    Stream().fill(big_x, 0, big_m * big_k).fill(big_w, 0, HipNative.q8Floats(big_k, big_n)).run()
+    graphs = [HipNative.graphCapture(words.array()) for _ in range(2)]
+
+    def replays(graph):
+        for _ in range(3):
+            dev.write(ob, np.zeros((m, n), np.float32))
+            HipNative.graphLaunch(graph, 2)
+            assert np.array_equal(dev.download(ob, (m, n)), expected)
+
+    allocs = HipNative.poolStats()["driver_allocs"]
+    Stream().q8_linear(big_x, big_w, big_o, big_m, big_k, big_n).run()
+    assert HipNative.poolStats()["driver_allocs"] == allocs + 1
+    graphs.append(HipNative.graphCapture(words.array()))
+    for g in (0, 2, 1):
+        replays(graphs[g])
+        HipNative.graphDestroy(graphs[g])
+    dev.release(src, wq, xb, ob, big_x, big_w, big_o)
