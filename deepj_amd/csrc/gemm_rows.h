@@ -37,7 +37,9 @@ __device__ __forceinline__ void load_to_lds4(const void *base, uint32_t off, uin
 #pragma clang diagnostic pop
 #endif
 
-// kernels_gemm_f16.hip: the rows, normalised if gamma (and beta) say so, in that order; rows [m, m_pad) as zeros
+// kernels_gemm_f16.hip
+int q8_gemm_f16_forced();        // DEEPJ_HIP_GEMM_F16, -1 where it is not set; 0: every GEMM on k_gemm_q8
+// The rows, normalised if gamma (and beta) say so, in that order; rows [m, m_pad) as zeros
 void launch_split_operand(hipStream_t s, const float *x, const float *gamma, const float *beta, uint16_t *planes, int m, int m_pad, int k, int kp);
 
 // An estimate of a Q8 GEMM's time in us.  With x workgroups a compute unit, in `rounds` rounds, kk thousand k a workgroup and

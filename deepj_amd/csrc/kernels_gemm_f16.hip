@@ -807,10 +807,15 @@ constexpr int kNPad = 768;      // weight rows of a prepared buffer are padded t
 
 constexpr int kMinRowsPrepared = 16;     // fewer rows than this read the int8 weights even where a copy is prepared
 
-GemmF16Plan q8_gemm_f16_plan(int m, int n_rows, int k, bool prepared) {
-    // DEEPJ_HIP_GEMM_F16=0 keeps every GEMM off these kernels; =128, =128192, =64 or =192 force the 128 x 256,
-    // 128 x 192, 64 x 256 or 64 x 192 tile (for comparisons)
+// DEEPJ_HIP_GEMM_F16=0 keeps every GEMM on k_gemm_q8; =128, =128192, =64 or =192 force the 128 x 256, 128 x 192, 64 x 256 or
+// 64 x 192 tile of the fp16 GEMM (for comparisons)
+int q8_gemm_f16_forced() {
     static const int forced = [] { const char *e = getenv("DEEPJ_HIP_GEMM_F16"); return e ? atoi(e) : -1; }();
+    return forced;
+}
+
+GemmF16Plan q8_gemm_f16_plan(int m, int n_rows, int k, bool prepared) {
+    const int forced = q8_gemm_f16_forced();
     if (forced == 0) return {0, 0, 1};
     // four columns per lane in the epilogue need n_rows % 4 == 0
     if ((n_rows & 3) != 0 || k < 64) return {0, 0, 1};

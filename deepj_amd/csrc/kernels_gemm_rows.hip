@@ -335,7 +335,7 @@ void q8_gemm_rows_configure() {
 // batches belong to k_gemm_q8's larger tiles (1500 x 50257 over 768 655 us, 504; 2048 rows 1058, 647; 1500 x 8001 over 1500 233, 158).  A
 // lane's offset into a column tile's weights is 32 bits.
 bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared, bool may_share, RowsPlan *plan) {
-    if (m > 768 || k > (1 << 24) || q8_gemm_f16_shape_ok(m, n_rows, k, prepared)) return false;
+    if (m > 768 || k > (1 << 24) || q8_gemm_f16_forced() == 0 || q8_gemm_f16_shape_ok(m, n_rows, k, prepared)) return false;
     const Q8GemmEstimate there = q8_gemm_estimate(m, n_rows, k, norm, may_share);
     const RowsPlan p = rows_plan(m, n_rows, k, may_share, there.sums);
     if (plan) *plan = p;

@@ -1,10 +1,15 @@
 """Which products the kernel that multiplies a batch of rows straight from the int8 weights takes: host arithmetic of the library,
 no GPU call."""
+import os
 import random
+import subprocess
+import sys
 
 import pytest
 
 from deepj_amd import HipNative
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.mark.parametrize("k,n", [(768, 50257), (1500, 8001), (2048, 4001), (4096, 16385), (256, 256), (768, 768)])
@@ -34,3 +39,18 @@ def test_every_choice_is_one_the_kernel_has():
         if not alloc_free:                               # never where the fp16 GEMM is taken
             assert not (HipNative.q8GemmTilePrepared if prepared else HipNative.q8GemmTile)(m, k, n)[0]
     assert len(seen) == 12                               # eleven and none
+
+
+def test_the_switch_that_keeps_every_gemm_on_k_gemm_q8():
+    shapes = [(30, 2048, 6144), (64, 4096, 22016), (200, 2048, 11264), (512, 2048, 6144), (400, 768, 50257)]
+    program = f"""
+from deepj_amd import HipNative as H
+for m, k, n in {shapes}:
+    for norm in (False, True):
+        for alloc_free in (False, True):
+            assert H.q8GemmRowsTile(m, k, n, norm, alloc_free=alloc_free) == (0, 0, 1), (m, k, n)
+    assert H.q8GemmPath(m, k, n) == H.q8GemmTilePrepared(m, k, n)[0] == 0, (m, k, n)
+"""
+    subprocess.run([sys.executable, "-c", program], check=True, timeout=120, cwd=ROOT, env=dict(os.environ, DEEPJ_HIP_GEMM_F16="0"))
+    for m, k, n in shapes:
+        assert HipNative.q8GemmRowsTile(m, k, n, norm=True)[0] or HipNative.q8GemmPath(m, k, n)
