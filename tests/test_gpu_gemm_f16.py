@@ -112,8 +112,8 @@ def test_every_way_the_shares_of_k_are_dealt_to_the_xcds(dev, m, k, n, shares):
 ])
 def test_fewer_than_256_rows_on_prepared_weights(dev, m, k, n, tile, epilogue):
     """With the weights already in the fp16 GEMM's layout the library takes prompts from 16 rows on, where its plan
-    expects enough workgroups (deepj_hip_q8_gemm_tile_prepared); without them the same shapes stay on the bf16 kernels.
-    Both against the oracle."""
+    expects enough workgroups (deepj_hip_q8_gemm_tile_prepared); without them the same shapes run on kernels that read
+    the int8 weights.  Both against the oracle."""
     swiglu = epilogue == "swiglu"
     n_rows = 2 * n if swiglu else n
     assert HipNative.q8GemmTile(m, k, n_rows) == (0, 0, 1)
@@ -147,7 +147,7 @@ def test_fewer_than_256_rows_on_prepared_weights(dev, m, k, n, tile, epilogue):
     op = Stream().q8_linear(xb, wq, ob, m, k, n, **kw)
     op.run()
     unprepared = dev.download(ob, (m, n))
-    assert_close(exp, unprepared, atol=gate(exp), rtol=1e-4, what=f"bf16 kernels M={m} K={k} N={n} {epilogue}")
+    assert_close(exp, unprepared, atol=gate(exp), rtol=1e-4, what=f"int8 weights M={m} K={k} N={n} {epilogue}")
     prep = dev.alloc(HipNative.q8PreparedFloats(k, n_rows))
     Stream().q8_prepare(wq, prep, k, n_rows).run()
     counts = HipNative.profileOps(op.array(), 1, detail=True)[2]

@@ -33,12 +33,15 @@ def rms_normalised(x, gamma):
     return x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-6) * gamma
 
 
-# (a small weight without a normalisation stays on the bf16 kernels.)  The last nine: K shared (few rows against a narrow
-# weight, long K), columns in pairs or not, and each of the wider tiles
+# Products that k_gemm_q8 keeps, under the same gate (its sums are no longer): eight, seven and eight workgroups sharing K, and
+# small weights without a normalisation in front
+ON_K_GEMM_Q8 = [(30, 11008, 1024, 0), (5, 5600, 2050, 0), (200, 12300, 500, 0), (40, 96, 50001, 0), (250, 288, 20002, 0)]
+
+
 @pytest.mark.parametrize("m,k,n,norm", [(2, 32, 2, 1), (7, 31, 33, 1), (32, 128, 32, 1), (33, 129, 31, 1), (64, 160, 65, 1), (65, 416, 64, 1), (96, 512, 97, 1),
-                                        (31, 640, 127, 1), (30, 11008, 1024, 0), (30, 11008, 1023, 0), (5, 5600, 2050, 0), (200, 12300, 500, 0),
-                                        (40, 96, 50001, 0), (250, 288, 20002, 0), (200, 1028, 5002, 0), (30, 1100, 24497, 0), (50, 1100, 24497, 0)])
+                                        (31, 640, 127, 1), (30, 11008, 1023, 0), (200, 1028, 5002, 0), (30, 1100, 24497, 0), (50, 1100, 24497, 0), *ON_K_GEMM_Q8])
 def test_product_at_the_edges(dev, m, k, n, norm):
+    assert (HipNative.q8GemmRowsTile(m, k, n, norm)[0] == 0) == ((m, k, n, norm) in ON_K_GEMM_Q8)
     w, x, gamma = JavaRandom(5).tensor(k, n, k ** -0.5), JavaRandom(6).tensor(m, k, 1.0), JavaRandom(7).tensor(1, k, 1.0)
     if m > 4:
         x[1] = 0.0                                       # a row without a largest value
@@ -114,10 +117,16 @@ def test_the_range_within_a_row_costs_no_bits(dev, m, k, n, norm, spread):
     check(got, a @ ref.q8_roundtrip(w).astype(np.float64), k, f"{m} x {k} x {n} {spread}", times=1 + norm)
 
 
-@pytest.mark.parametrize("m,k,n", [(9, 200, 46), (64, 2052, 2100), (30, 8224, 1026)])
-@pytest.mark.parametrize("epilogue", ["bias_gelu_residual", "swiglu", "rms", "layernorm"])
-def test_prologues_and_epilogues(dev, m, k, n, epilogue):
+# (on: the ones that run here; the others on k_gemm_q8.)  The last but two: K shared, the epilogue in the sum of the shares
+EPILOGUES = ("bias_gelu_residual", "swiglu", "rms", "layernorm")
+
+
+@pytest.mark.parametrize("m,k,n,on", [(9, 200, 46, EPILOGUES[2:]), (64, 2052, 2100, ()), (30, 8224, 1026, EPILOGUES[2:]), (250, 8224, 2050, EPILOGUES),
+                                      (200, 1028, 5002, EPILOGUES), (40, 2056, 4100, EPILOGUES[1:2])])
+@pytest.mark.parametrize("epilogue", EPILOGUES)
+def test_prologues_and_epilogues(dev, m, k, n, on, epilogue):
     sw = epilogue == "swiglu"
+    assert (HipNative.q8GemmRowsTile(m, k, n * (1 + sw), epilogue in EPILOGUES[2:])[0] > 0) == (epilogue in on)
     w, x = [JavaRandom(7 + i).tensor(k, n, k ** -0.5) for i in range(1 + sw)], JavaRandom(9).tensor(m, k, 1.0)
     vec = [JavaRandom(10 + i).tensor(1, k if i > 1 else n, 0.5) for i in range(4)]
     res = JavaRandom(15).tensor(m, n, 1.0)

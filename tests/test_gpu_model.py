@@ -428,9 +428,9 @@ def test_generate_slides_the_window_past_max_seq_len():
 
 def test_short_and_chunked_prompts_on_prepared_weights_against_the_oracle():
     """With prepared (fp16) copies of the weights the prompt GEMM takes prompts from 16 rows on where the projection is
-    wide enough - here q | k | v and gate/up of a d = 2048 model - and the bf16 kernels take the rest.  A 200-token
-    prompt in one piece, the same prompt as chunks of 128 + 40 + 17 + 15 rows, and the one-piece prompt with no copies
-    at all (every GEMM below 256 rows on the bf16 kernels) against the oracle's forward: same logits within the gate,
+    wide enough - here q | k | v and gate/up of a d = 2048 model - and kernels that read the int8 weights take the rest.  A
+    200-token prompt in one piece, the same prompt as chunks of 128 + 40 + 17 + 15 rows, and the one-piece prompt with no
+    copies at all (every GEMM below 256 rows straight from the int8 weights) against the oracle's forward: same logits within the gate,
     same next tokens."""
     cfg = LlamaConfig(vocabSize=512, maxSeqLen=256, dModel=2048, nHeads=16, nLayers=2, dFF=5632)
     assert HipNative.q8GemmTilePrepared(128, 2048, 3 * 2048)[0] == 64 and HipNative.q8GemmTile(128, 2048, 3 * 2048)[0] == 0
@@ -448,7 +448,7 @@ def test_short_and_chunked_prompts_on_prepared_weights_against_the_oracle():
             gpu.prefill(prompt[pos:pos + n], choose_next=False)
             pos += n
         chunked_last = gpu.lastLogits()
-        gpu.setPreparedBudget(0)                                # no copies: the bf16 kernels for every short GEMM
+        gpu.setPreparedBudget(0)                                # no copies: the int8 weights for every short GEMM
         assert gpu.preparedBytes() == 0
         plain = gpu.forward(prompt)
         assert gpu.preparedBytes() == 0

@@ -71,9 +71,11 @@ def test_noalloc_flush_matches_flush_on_two_calls_the_second_smaller():
     try:
         # the second case is smaller in every dimension: its workspace rows and its counters lie inside what
         # the first call used
-        # (GEMM shapes that flush_ops runs as ONE launch of the bf16 kernel, as the allocation-free entry point always
-        # does: 288 tiles of 64 x 64, and a K of three steps - too many tiles, too short a K, for workgroups to share it)
+        # (GEMM shapes that both entry points run on the same tile of the same kernel, K not shared, straight from the int8
+        # weights, with the rows' pieces in the array here)
         cases = [Case(dev, 192, 2048, 6144, 32, 64, 515, 100), Case(dev, 40, 384, 96, 8, 32, 70, 200)]
+        for c, tile in zip(cases, ((64, 96, 1), (32, 32, 1))):
+            assert [HipNative.q8GemmRowsTile(c.m, c.k, c.n, True, alloc_free=a) for a in (False, True)] == [tile, tile]
         expected = [c.run(noalloc=False) for c in cases]
         # the oracle on the first case's GEMM: the comparison below is between two HIP paths, this pins one of them
         c = cases[0]
@@ -96,32 +98,53 @@ def test_noalloc_flush_matches_flush_on_two_calls_the_second_smaller():
         dev.release_all()
 
 
-def test_noalloc_flush_never_shares_k_among_workgroups():
-    """A few-tile, long-K product (64 rows x 2048 x 2048: 32 tiles) runs under flush_ops as eight workgroups per tile
-    with their partial products in the workspace; the allocation-free entry point runs it as one launch.  Both are
-    held to the oracle at the per-op tolerance."""
+# (tile rows, tile columns, workgroups sharing K) of the kernel that multiplies straight from the int8 weights, under flush_ops and
+# here; None: k_gemm_q8.  The last two: its rows' pieces are more than the array holds, and k_gemm_q8 takes them.
+NEVER_SHARED = [(64, 2048, 2048, False, None, (32, 32, 1)), (30, 11008, 1024, False, None, (32, 32, 1)), (690, 396, 32, False, None, None),
+                (627, 2032, 274, False, None, None), (30, 3072, 2050, True, (32, 32, 2), (32, 32, 1)), (2, 1152, 250, True, (32, 32, 4), (32, 32, 1)),
+                (640, 2048, 1002, True, (32, 64, 2), (32, 64, 1)), (250, 8224, 2050, False, (32, 64, 2), None),
+                (500, 4096, 4099, True, (32, 96, 1), None)]
+
+
+@pytest.mark.parametrize("m,k,n,norm,shared,here", NEVER_SHARED)
+def test_noalloc_flush_never_shares_k_among_workgroups(m, k, n, norm, shared, here):
+    """Products that flush_ops has several workgroups a tile share the K of, their partial products beside it, on either
+    kernel (64 rows x 2048 x 2048: eight on k_gemm_q8); the allocation-free entry point runs them as one GEMM.  Both are
+    held to the oracle at the per-op tolerance; they add a sum up in different orders, so some bits differ, and each
+    repeats its own."""
     HipNative.init(0)
     dev = DeviceBuffers()
     try:
-        m, k, n = 64, 2048, 2048
+        pieces = -(-m // 32) * 32 * (-(-k // 128) * 128) * 3 // 2
+        tiles = [HipNative.q8GemmRowsTile(m, k, n, norm, alloc_free=a) for a in (False, True)]
+        if pieces > NOALLOC_WORKSPACE_FLOATS:
+            assert tiles[1][0] and here is None          # (the query knows nothing of the array)
+            tiles[1] = (0, 0, 1)
+        assert tiles == [shared or (0, 0, 1), here or (0, 0, 1)]
+        assert HipNative.q8GemmPath(m, k, n) == 0
         w = gaussian(k, n, 41, 0.02)
         x = gaussian(m, k, 42)
         src = dev.upload(w)
         wq = dev.alloc(HipNative.q8Floats(k, n))
         Stream().q8_quantize(src, wq, k, n).run()
         dev.release(src)
-        xb, out = dev.upload(x), dev.alloc(m * n)
-        exp = ref.matmul(x, ref.q8_roundtrip(w))
+        gamma = 1.0 + gaussian(1, k, 43, 0.02)
+        xb, gb, out = dev.upload(x), dev.upload(gamma), dev.alloc(m * n)
+        exp = ref.matmul(ref.rmsnorm(x, gamma) if norm else x, ref.q8_roundtrip(w))
         scale = float(np.sqrt(np.mean(exp.astype(np.float64) ** 2)))
-        words = Stream().q8_linear(xb, wq, out, m, k, n).array()
-        HipNative.nativeFlushOps(words, words.size)
-        assert_close(exp, dev.download(out, (m, n)), atol=1e-4 * scale, rtol=1e-4, what="flush_ops (K shared) vs oracle")
-        dev.write(out, np.zeros(m * n, np.float32))
-        before = HipNative.poolStats()["driver_allocs"]
-        HipNative.flushOpsNoAlloc(words, words.size)
-        got = dev.download(out, (m, n))
-        assert HipNative.poolStats()["driver_allocs"] == before
-        assert_close(exp, got, atol=1e-4 * scale, rtol=1e-4, what="noalloc (one launch) vs oracle")
+        words = Stream().q8_linear(xb, wq, out, m, k, n, gamma=gb if norm else -1).array()
+        results = []
+        for flush, what in ((HipNative.nativeFlushOps, "flush_ops"), (HipNative.flushOpsNoAlloc, "noalloc")):
+            for again in (False, True):
+                dev.write(out, np.zeros(m * n, np.float32))
+                before = HipNative.poolStats()["driver_allocs"]
+                flush(words, words.size)
+                results.append(dev.download(out, (m, n)).copy())
+                if what == "noalloc" or again:
+                    assert HipNative.poolStats()["driver_allocs"] == before
+            assert_close(exp, results[-1], atol=1e-4 * scale, rtol=1e-4, what=f"{what} vs oracle")
+            assert np.array_equal(results[-1].view(np.int32), results[-2].view(np.int32)), f"{what}: other bits the second time"
+        assert not np.array_equal(results[0], results[2])
     finally:
         dev.release_all()
 
