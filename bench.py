@@ -171,6 +171,15 @@ def matvec_roofline(model, position: int, iters: int = 12):
 MFMA_PEAK_TFLOPS = 2500.0       # MI355X dense fp16 / bf16 matrix-core peak
 
 
+def int8_gemm_name(m, k, rows, norm):
+    """The kernel of a Q8 GEMM that reads the int8 weights: three bf16 pieces an activation on either."""
+    from deepj_amd import HipNative
+    tile_rows, tile_cols, shares = HipNative.q8GemmRowsTile(m, k, rows, norm)
+    if not tile_rows:
+        return "k_gemm_q8 (bf16 x 3)"
+    return f"k_gemm_q8_rows ({tile_rows} x {tile_cols} tiles" + (f", K shared by {shares}" if shares > 1 else "") + ", bf16 x 3) + k_split_f16"
+
+
 def prefill_roofline(model, n: int, iters: int = 6):
     """Per-op durations of the n-token prompt's command stream, measured live like the decode table: a start and a stop
     event on EVERY dispatch of every op, summed per op - so a projection's figure holds its GEMM and the helpers the
@@ -178,7 +187,7 @@ def prefill_roofline(model, n: int, iters: int = 6):
     when workgroups share K; the per-call conversion of the weights when the runner holds no fp16 copy).  `gemm_us` is
     the op's longest dispatch alone.  A projection's algorithmic work is one multiply-add per weight per row,
     2 M K N flops; the fp16 kernels issue two matrix-core products for it (hi and lo halves of the activation), the
-    bf16 kernels three - `issued` counts those against the same peak."""
+    kernels that read the int8 weights three (bf16) - `issued` counts those against the same peak."""
     from deepj_amd import HipNative, opcodes as op
     stream = model.prefillStream(n)
     ops = decode_ops(stream)
@@ -201,7 +210,8 @@ def prefill_roofline(model, n: int, iters: int = 6):
             e = table.setdefault(names.get((k, rows), f"{k}x{rows}") + ("_rope_kv_store" if fused_rope else ""), {
                 "launches": 0, "us": 0.0, "gemm_us": 0.0, "dispatches_per_op": int(c), "flops": f,
                 "kernel": (f"k_gemm_q8_f16 ({tile} x {tile_cols} tiles" + (f", K shared by {shares}" if shares > 1 else "") +
-                           ", fp16 x 2" + (", RoPE + cache append as the epilogue)" if fused_rope else ")")) if tile else "k_gemm_q8 (bf16 x 3)"})
+                           ", fp16 x 2" + (", RoPE + cache append as the epilogue)" if fused_rope else ")")) if tile
+                          else int8_gemm_name(m, k, rows, bool(flags & (op.LIN_RMSNORM | op.LIN_LAYERNORM)))})
             e["launches"] += 1
             e["us"] += float(t)
             e["gemm_us"] += float(t_top)
@@ -316,7 +326,7 @@ def c2_sweep(iters: int = 10, cpu: bool = True):
                     plain.q8_linear(x, q, out, m, k, n)
                 us = period_us(plain, len(use))
                 row.update({"kernel": (f"k_gemm_q8_f16 ({tile} x {tile_cols} tiles" + (f", K shared by {shares}" if shares > 1 else "") +
-                                       ", fp16 x 2) + k_split_f16 + k_q8_to_f16") if tile else "k_gemm_q8 (bf16 x 3)",
+                                       ", fp16 x 2) + k_split_f16 + k_q8_to_f16") if tile else int8_gemm_name(m, k, n, False),
                             "flops": flops, "us": round(us, 2), "TFLOPs": round(flops / us / 1e6, 1),
                             "frac_of_mfma_peak": round(flops / us / 1e6 / MFMA_PEAK_TFLOPS, 4)})
                 ptile, ptile_cols, pshares = HipNative.q8GemmTilePrepared(m, k, n)

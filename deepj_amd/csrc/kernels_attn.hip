@@ -279,15 +279,15 @@ __global__ void __launch_bounds__(256) k_attention_tiled(AttnKernelArgs a) {
     const int k_first = SHARE ? (int)blockIdx.z * KT * KSETS : 0;
     const int k_stride = SHARE ? (int)gridDim.z * KT * KSETS : KT * KSETS;
     // One or two key sets: the rows a round stages are requested a round ahead and fly while this one's products run (32 heads
-    // of 128 x 2048 rows 262 -> 241 us, 32 of 64 x 1024 55.6 -> 54.3).  Four sets have too many rows to hold for it (12 heads of
+    // of 128 x 2048 rows 264 -> 245 us; 32 of 64 x 1024 53 either way).  Four sets have too many rows to hold for it (12 heads of
     // 64 x 400 rows 18.1 -> 19.0, 24 x 200 11.6 -> 12.3).
     constexpr bool AHEAD = KSETS <= 2;
     constexpr int PART = HD / 8;
     typedef float floatx4 __attribute__((ext_vector_type(4)));
     floatx4 kreg[KSETS][PART / 4], vreg[PVB ? 1 : KSETS][PVB ? 1 : PART / 4];
     // Neighbouring lanes take neighbouring 16 bytes of a row: a load takes the address unit a cycle a line, and with a row a lane
-    // it was 64 of them (32 heads of 64 x 512 rows 23.3 -> 21.9 us, 12 x 400 18.2 -> 17.6, 16 of 128 x 1024 73.8 -> 70.1).  One key
-    // set has the products to cover that, and a row a lane is still the better one (32 of 128 x 2048 rows 250 us, 255 so).
+    // it was 64 of them (32 heads of 64 x 512 rows 22.7 -> 21.4 us, 12 x 400 17.7 -> 17.2, 16 of 128 x 1024 75 -> 70).  One key
+    // set has the products to cover that, and a row a lane is still the better one (32 of 128 x 2048 rows 245 us, 250 so).
     constexpr bool BY_ROW = KSETS == 1;
     constexpr int LPR = HD / 4;                              // lanes a row
     auto piece_row = [&](int j) __attribute__((always_inline)) { return BY_ROW ? t & 31 : t / LPR + 256 / LPR * j; };

@@ -14,9 +14,10 @@
 // loads return in the order they were asked for, so waiting for activations that were asked for after a chunk is waiting for
 // the chunk.  The matrix cores' 32 cycles a product hide the group before's scaling and the next one's conversion.
 //
-// What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 33 us with the split, 39 where they come from
-// HBM, 87 on the bf16 kernels), then the activations, which every tile reads anew from L2 (12 KB for every 64 x 64 x 32: 64 x
-// 22016 46 us, 86; 200 x 11264 over 2048 47, 67), and on small weights two launches' latency (30 x 2304 over 768 8.9 us, 10.8).
+// What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 34 us with the rows' normalisation and split, 42
+// where they come from HBM, 87 and 90 on k_gemm_q8), then the activations, which every tile reads anew from L2 (12 KB for every
+// 64 x 64 x 32: 64 x 22016 48 us, 53 from HBM, 86 and 92; 200 x 11264 over 2048 49 and 52, 66 and 67), and on small weights two
+// launches' latency (30 x 2304 over 768 8.7 and 9.7 us, 13 and 12.6).
 // Tried and slower, with two pieces: eight wavefronts a workgroup (two workgroups of four fill a compute unit better: 64 x 22016
 // 54 us against 49), the K loop or the epilogue rolled (3 % and 10 %), a 64 x 64 tile whose wavefronts share the activations
 // through LDS (latency of its reads and barriers: 400 x 768 over 3072 34 us against 22).
@@ -145,7 +146,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
                 for (int z = 0; z < NS; z++) acc[z][i][j][e] = 0.0f;
         p[0][e] = p[1][e] = 0.0f;
     }
-    uint32_t bw[2][8];                                 // [stage parity]: the weights of a stage (a column tile of a group) as fp16
+    uint32_t bw[2][8];                                 // [stage parity]: the weights of a stage (a column tile of a group) as bf16
     uintx4 qw[2];                                      // ... and as bytes, up to two stages ahead
     float sc[4] = {0.f, 0.f, 0.f, 0.f};                // their scales: of the stage before, this one and the two next
     auto read_q = [&](int slot, int g, int tn, int at, int at_sc) __attribute__((always_inline)) {

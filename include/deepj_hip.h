@@ -56,11 +56,11 @@ int deepj_hip_flush_ops(const int32_t *cmd, int32_t len);
  * serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Same streams and
  * the same kernels and bits as deepj_hip_flush_ops, with ONE exception: a Q8_LINEAR of more than one row never
  * runs here on the fp16 GEMM with its own copy of the weights (256 rows and more - 16 and more with prepared weights -
- * and enough tiles), never lets several workgroups share a tile's K (few tiles, long K), and runs as a single launch of
- * k_gemm_q8 where its rows in the pieces that flush_ops multiplies (6 bytes a value) do not fit the fixed workspace; all of these
- * meet the per-op tolerance against the CPU backend, their bits differ.  The
- * device scratch the kernels need - the workspace that Q8_LINEAR with a norm
- * prologue and M > 1 writes its normalised rows to, and the arrival counters of the split decode attention
+ * and enough tiles) but on the kernels that read the int8 weights, never lets several workgroups share a tile's K (few tiles,
+ * long K), and runs as a single launch of k_gemm_q8 where its rows in the pieces that flush_ops multiplies (6 bytes a value) do
+ * not fit the fixed workspace; all of these meet the per-op tolerance against the CPU backend, their bits differ.  The
+ * device scratch the kernels need - the workspace that Q8_LINEAR with M > 1 writes its rows' pieces or, with a norm
+ * prologue, its normalised rows to, and the arrival counters of the split decode attention
  * (ATTENTION / ATTENTION_KV with S = 1, ATTN_DECODE) - is a fixed array inside the library's code object instead
  * of memory the runtime allocates and grows.  The call never calls hipMalloc or hipFree: it fails when the
  * runtime is not initialised yet (deepj_hip_init allocates), when the stream needs more than
