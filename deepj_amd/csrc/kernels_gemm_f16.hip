@@ -844,9 +844,11 @@ GemmF16Plan q8_gemm_f16_plan(int m, int n_rows, int k, bool prepared) {
     // Few tiles: several workgroups per tile, each with a share of K of at least kMinSplitSteps steps, their partial
     // products summed by a second kernel - as many workgroups as that allows, on the tile width that gives more of them
     // (the wider one unless the narrower gives 5 % more).  Worth it when there is enough work to stream: K of 1536 or more
-    // (512 x 2048 over K 1024: 25 us against 17.5 on the bf16 kernels) and 48 narrow tiles or more, or 40 with a long K.  Measured against the bf16 kernels (us, prepared weights): 512 x 2048 over K 5632
-    // 44 / 68; 512 x 2048 over K 2048 29 / 28; 256 x 6144 over K 2048 (two shares) 29 / 49; 320 x 2048 over K 2048 (six
-    // shares) 23 / 26; 64 x 11008 over K 4096 28 / 47; 128 x 11264 over K 2048 27 / 48; 255 x 2048 over K 5632 30 / 45.
+    // (512 x 2048 over K 1024: 25 us against 17.5 on k_gemm_q8) and 48 narrow tiles or more, or 40 with a long K.  Measured
+    // against k_gemm_q8 (us, prepared weights): 512 x 2048 over K 5632 44 / 68; 512 x 2048 over K 2048 29 / 28; 256 x 6144 over
+    // K 2048 (two shares) 29 / 49; 320 x 2048 over K 2048 (six shares) 23 / 26; 64 x 11008 over K 4096 28 / 47; 128 x 11264
+    // over K 2048 27 / 48; 255 x 2048 over K 5632 30 / 45.
+    // (k_gemm_q8_rows, from the int8 weights: 30 and 31 for the 64 and 128 rows, 15.5 against 20 here for 30 x 11264 over 2048.)
     // Below those bounds the partial products cost more than the launch gains (256 x 2048 over K 2048: 23 / 19; 64 x 2048
     // over K 2048, eight shares: 16 / 12).
     const int steps = q8_padded_k(k) / 32;
