@@ -2,9 +2,10 @@
 //
 //   C[M x N] = A[M x K] . B      A fp32 row-major, fp32 accumulate
 //
-// fp32 B [K x N] row-major (OP_MATMUL; CpuBackend.java:168-188 in the reference): v_mfma_f32_32x32x2_f32, in k_matmul, whose
-// wavefronts share a tile's K and feed the matrix cores straight from the caches, where a tile per compute unit covers the
-// product, else in k_matmul_lds, whose tiles go through LDS and run several to a compute unit.
+// fp32 B [K x N] row-major (OP_MATMUL; CpuBackend.java:168-188 in the reference): v_mfma_f32_32x32x2_f32 in k_matmul, whose
+// wavefronts share a tile's K and feed the matrix cores straight from the caches, for products of few tiles;
+// v_mfma_f32_32x32x16_bf16 on the exact pieces of both operands in k_matmul_split for those that the matrix rate bounds;
+// k_matmul_lds (fp32 instructions, tiles through LDS) for large ones over a short K.
 //
 // Q8 B [N x Kp] int8 + one fp32 scale per 32-group (prefill-time Q8 GEMM; the M = 1 decode case is the HBM-bound
 // kernel in kernels_q8.hip): v_mfma_f32_32x32x16_bf16 at full fp32 accuracy.  An int8 weight is exact in bf16,
@@ -16,6 +17,7 @@
 // shape by launch_q8_gemm; the epilogue adds bias / GELU / residual or pairs interleaved gate/up columns (SwiGLU).
 #include <cstdlib>
 #include "dj_common.h"
+#include "dj_device.h"
 #include "gemm_epilogue.h"
 #include "gemm_rows.h"
 
@@ -27,6 +29,16 @@ namespace {
 
 constexpr int BM = 64, BN = 64;            // Q8 tiles
 constexpr int BM2 = 128, BN2 = 128;
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// bf16(a) | bf16(b) << 16, both by truncation
+__device__ __forceinline__ uint32_t pack_bf16_hi(float a, float b) {
+    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302);
+}
+__device__ __forceinline__ float top_bits(float x) {      // the leading 8 significant bits of x: a bf16 value
+    return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u);
+}
 
 // ── fp32 x fp32 ─────────────────────────────────────────────────────────────
 // One workgroup computes a tile of 32 TM x 32 TN; its KW wavefronts each multiply the WHOLE tile over their own share of K
@@ -185,14 +197,219 @@ __global__ void __launch_bounds__(64 * KW) k_matmul(const float *__restrict__ A,
         }
 }
 
+// ── fp32 x fp32 on the bf16 matrix cores ────────────────────────────────────
+// An fp32 value is the exact sum of three bf16 values (itself rounded to bf16, the remainder rounded, the rest), so
+//   a . b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh) + ...       what is left out is about 2^-26 of |a b|
+// and six bf16 products of 16 k take 0.375 of the time of eight fp32 products of 2.  The first product and the five small ones
+// have accumulators of their own, so that the large sum is cut off once per 16 k and set (fp32 instructions: eight times): its
+// error against float64 is 0.99e-7 to 1.3e-7 of the result's rms at 1024 k by tile, where k_matmul has 2.9e-7; 1.5e-7 to
+// 2.2e-7 against 4.7e-7 at 2752; 6e-8 to 7e-8 against 1.1e-7 at 192.
+// Bound: the matrix cores at the clock they run the chip down to (about 27 products of 32 x 32 x 16 a ns over the whole chip; the
+// same rate at every depth of pipelining tried) once the tiles fill it, loads and splits in turn below.  k_matmul or
+// k_matmul_lds -> this: 500 x 2752 x 1024 31.4 -> 25.6 us, 1000 x 2752 x 1024 69 -> 43, 1000 x 7000 x 1024 153 -> 103.
+struct Pieces { bf16x8 h, m, l; };
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+// (a dot product of two with -1 and 0 takes the pieces off their values without unpacking them)
+__device__ __forceinline__ Pieces split8(const float (&v)[8], float &most) {
+    union U { bf16x2 p[4]; bf16x8 b; } h, m, l;
+    uint32_t lo = 0x0000bf80u, hi = 0xbf800000u;     // -1 in one half (in registers: as an inline constant -1.0 is the upper half's)
+    asm("" : "+s"(lo));
+    asm("" : "+s"(hi));
+    const bf16x2 first = __builtin_bit_cast(bf16x2, lo), second = __builtin_bit_cast(bf16x2, hi);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const floatx2 x = {v[2 * j], v[2 * j + 1]};
+        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(v[2 * j]), "v"(v[2 * j + 1]));   // (fmaxf: three instructions)
+        h.p[j] = __builtin_convertvector(x, bf16x2);
+        const floatx2 r = {__builtin_amdgcn_fdot2_f32_bf16(h.p[j], first, x[0], false), __builtin_amdgcn_fdot2_f32_bf16(h.p[j], second, x[1], false)};
+        m.p[j] = __builtin_convertvector(r, bf16x2);
+        const floatx2 t = {__builtin_amdgcn_fdot2_f32_bf16(m.p[j], first, r[0], false), __builtin_amdgcn_fdot2_f32_bf16(m.p[j], second, r[1], false)};
+        l.p[j] = __builtin_convertvector(t, bf16x2);
+    }
+    return {h.b, m.b, l.b};
+}
+__device__ __forceinline__ floatx16 product(bf16x8 a, bf16x8 b, floatx16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+
+// A workgroup computes a tile of 32 TM x 32 WC in WC x KS wavefronts: a wavefront has 32 of its columns and every KS-th 16 k
+// (the sets' sums meet in LDS at the end, in a fixed order).  The columns' values go from memory to the registers of the one
+// wavefront that splits and multiplies them, two steps of 16 KS k ahead; the rows' are split once for the workgroup and shared
+// through LDS (16-byte operands in lane order), one step ahead.
+template <int TM, int WC, int KS, bool VEC>
+__global__ void __launch_bounds__(64 * WC * KS) k_matmul_split(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C,
+                                                               const int M, const int N, const int K, const int tiles_m, const int tiles_n) {
+    constexpr int kWaves = WC * KS, kStep = 16 * KS, kRows = 32 * TM;
+    constexpr int kStages = (TM + WC - 1) / WC;     // groups of 8 values of A that a thread stages a step (some threads: one fewer)
+    constexpr int kStride = 36;                     // LDS row of a 32-column block (16-byte aligned, spreads the two halves)
+    constexpr int kOperands = KS * TM * 3 * 64;     // 16-byte words of a step
+    __shared__ uint32_t row_most[kRows], col_most[32 * WC];
+    __shared__ int any_tiny;
+    auto is_tiny = [](uint32_t most) { return most < (127u - 77u) << 23 && most > 0u; };       // 2^-77
+    __shared__ __align__(16) uint4 lds[2 * kOperands * 16 > kWaves * 32 * kStride * 4 ? 2 * kOperands : kWaves * 32 * kStride / 4];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = lane >> 5, l32 = lane & 31, wc = wave % WC, set = wave / WC;
+    // Workgroups go to the eight XCDs in turn: each XCD gets a run of neighbouring tiles, along the larger operand.
+    const int total = tiles_m * tiles_n, xcd = blockIdx.x & 7, q = total >> 3, r = total & 7;
+    const int idx = xcd * q + (xcd < r ? xcd : r) + (int)(blockIdx.x >> 3);
+    const bool by_cols = N >= M;
+    const int tile_n = by_cols ? idx / tiles_m : idx % tiles_n, tile_m = by_cols ? idx % tiles_m : idx / tiles_n;
+    const int m0 = tile_m * kRows, n0 = tile_n * 32 * WC;
+
+    // rows and columns past the matrix repeat its last one: their products are not stored
+    const float *Am = A + (int64_t)m0 * K;
+    uint32_t a_off[kStages];
+#pragma unroll
+    for (int g = 0; g < kStages; g++) {
+        // wavefront w stages for set w / WC the rows 32 (w % WC) .., 32 (w % WC + WC) ..
+        const int row = 32 * (wc + g * WC) + l32;
+        a_off[g] = ((uint32_t)(row < M - m0 ? row : M - 1 - m0) * (uint32_t)K + 16u * set + 8u * half) * 4u;
+    }
+    const int col = n0 + 32 * wc + l32 < N ? n0 + 32 * wc + l32 : N - 1;
+    const auto b_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B), 0, (int)((uint32_t)K * (uint32_t)N * 4u), 0x00020000);
+    const uint32_t b_off = ((16u * set + 8u * half) * (uint32_t)N + (uint32_t)col) * 4u;
+
+    floatx16 acc[TM], low[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[i][e] = low[i][e] = 0.0f;
+
+    float most_a[kStages] = {}, most_b = 0.0f;       // the largest magnitude seen of the rows staged, of the column
+    struct Eight { float v[8]; };
+    auto load_a = [&](Eight (&a)[kStages], int k0) {
+#pragma unroll
+        for (int g = 0; g < kStages; g++) {
+            if (wc + g * WC >= TM) break;           // wavefront-uniform
+            const char *p = reinterpret_cast<const char *>(Am + k0) + a_off[g];
+            if constexpr (VEC) {
+                const float4 u = reinterpret_cast<const float4 *>(p)[0], v = reinterpret_cast<const float4 *>(p)[1];
+                a[g] = {{u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w}};
+            } else {
+#pragma unroll
+                for (int x = 0; x < 8; x++) a[g].v[x] = reinterpret_cast<const float *>(p)[x];
+            }
+        }
+    };
+    auto load_b = [&](Eight &b, int k0) {
+#pragma unroll
+        for (int x = 0; x < 8; x++) {
+            b.v[x] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b_rsrc, (int)b_off, (int)((uint32_t)(k0 + x) * (uint32_t)N * 4u), 0));
+        }
+    };
+    auto stage = [&](const Eight (&a)[kStages], int buffer) {
+#pragma unroll
+        for (int g = 0; g < kStages; g++) {
+            if (wc + g * WC >= TM) break;
+            const Pieces p = split8(a[g].v, most_a[g]);
+            uint4 *at = lds + buffer * kOperands + (set * TM + wc + g * WC) * 192 + lane;
+            at[0] = __builtin_bit_cast(uint4, p.h); at[64] = __builtin_bit_cast(uint4, p.m); at[128] = __builtin_bit_cast(uint4, p.l);
+        }
+    };
+    auto multiply = [&](const Eight &raw, int buffer) {
+        Pieces a[TM];
+        const uint4 *at = lds + buffer * kOperands + set * TM * 192 + lane;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+            a[i] = {__builtin_bit_cast(bf16x8, at[i * 192]), __builtin_bit_cast(bf16x8, at[i * 192 + 64]), __builtin_bit_cast(bf16x8, at[i * 192 + 128])};
+        const Pieces b = split8(raw.v, most_b);
+#define DJ_EACH(acc, x, y) _Pragma("unroll") for (int i = 0; i < TM; i++) acc[i] = product(a[i].x, b.y, acc[i])
+        DJ_EACH(acc, h, h);
+        DJ_EACH(low, h, m);
+        DJ_EACH(low, m, h);
+        DJ_EACH(low, m, m);
+        DJ_EACH(low, h, l);
+        DJ_EACH(low, l, h);
+#undef DJ_EACH
+    };
+
+    // The loads past the last whole step repeat it: the number in flight is known at compile time.
+    const int steps = K / kStep, tail = K - steps * kStep;
+    if (steps > 0) {
+        Eight a[2][kStages], b[2];
+        auto step_k = [&](int i) { return (i < steps ? i : steps - 1) * kStep; };
+        load_a(a[0], 0);
+        load_b(b[0], 0);
+        load_b(b[1], step_k(1));
+        load_a(a[1], step_k(1));
+        stage(a[0], 0);
+        dev::lds_barrier();
+        int i = 0;
+        for (; i + 2 <= steps; i += 2) {
+#pragma unroll
+            for (int d = 0; d < 2; d++) {
+                load_a(a[d], step_k(i + d + 2));
+                multiply(b[d], d);
+                load_b(b[d], step_k(i + d + 2));
+                stage(a[d ^ 1], d ^ 1);
+                dev::lds_barrier();
+            }
+        }
+        if (i < steps) {
+            multiply(b[0], 0);
+            dev::lds_barrier();
+        }
+    }
+    if (tail > 0) {                                 // zeros past the end of K, in both operands
+        Eight a[kStages], b;
+        const int k0 = steps * kStep, k = k0 + 16 * set + 8 * half;
+#pragma unroll
+        for (int x = 0; x < 8; x++) {
+#pragma unroll
+            for (int g = 0; g < kStages; g++) a[g].v[x] = wc + g * WC < TM && k + x < K ? at_bytes(Am + k0 + x, a_off[g]) : 0.0f;
+            b.v[x] = k + x < K ? at_bytes(B + (int64_t)(k0 + x) * N, b_off) : 0.0f;
+        }
+        __syncthreads();
+        stage(a, 0);
+        __syncthreads();
+        multiply(b, 0);
+    }
+
+    // acc[i][e] is C[32 i + 8 (e / 4) + 4 half + e % 4][l32] of the wavefront's columns
+    float *red = reinterpret_cast<float *>(lds);
+    for (int o = threadIdx.x; o < kRows + 32 * WC; o += 64 * kWaves) (o < kRows ? row_most[o] : col_most[o - kRows]) = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < kStages; g++)
+        if (wc + g * WC < TM) atomicMax(&row_most[32 * (wc + g * WC) + l32], __builtin_bit_cast(uint32_t, most_a[g]));
+    atomicMax(&col_most[32 * wc + l32], __builtin_bit_cast(uint32_t, most_b));
+    if (threadIdx.x == 0) any_tiny = 0;
+    __syncthreads();
+    for (int o = threadIdx.x; o < kRows + 32 * WC; o += 64 * kWaves)
+        if (is_tiny(o < kRows ? row_most[o] : col_most[o - kRows])) any_tiny = 1;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 16; e++) red[(wave * 32 + 8 * (e >> 2) + 4 * half + (e & 3)) * kStride + l32] = acc[i][e] + low[i][e];
+        __syncthreads();
+        for (int o = threadIdx.x; o < 1024 * WC; o += 64 * kWaves) {
+            const int row = o / (32 * WC), c = o % (32 * WC), at = ((c >> 5) * 32 + row) * kStride + (c & 31);
+            float v = red[at];
+#pragma unroll
+            for (int w = 1; w < KS; w++) v += red[w * WC * 32 * kStride + at];
+            const int out_row = m0 + 32 * i + row, out_col = n0 + c;
+            if (out_row < M && out_col < N) {
+                // An operand that is no finite number has no such pieces, and a sum may leave the range in another order; and
+                // where a whole row or column is tiny, pieces below 2^-126 are lost that matter: there the products are
+                // added one by one.
+                if (!(fabsf(v) <= 3.40282347e38f) || (any_tiny && (is_tiny(row_most[32 * i + row]) || is_tiny(col_most[c])))) {
+                    v = 0.0f;
+                    for (int k = 0; k < K; k++) v = fmaf(A[(int64_t)out_row * K + k], B[(int64_t)k * N + out_col], v);
+                }
+                C[(int64_t)out_row * N + out_col] = v;
+            }
+        }
+    }
+}
+
 // Where a tile per compute unit does not cover the product: workgroups of four wavefronts, a 64 x 64 tile (32 x 32 per
 // wavefront), 32 k a step through LDS.  Both operands sit k-major there, so the 64 lanes of an operand read 32 consecutive
 // floats per half (no bank conflicts).  The loads of the next step are issued before this step's products, and a compute unit
 // holds four such workgroups, whose loads and barriers hide behind one another's products - the direct loads of k_matmul
 // evict one another from the L1 as soon as two of its workgroups share a compute unit.
 // Bound: the fp32 matrix rate.  k_matmul -> this: 1024 x 2752 x 1024 100 -> 68 us, 1000 x 7000 x 1024 266 -> 154,
-// 4096 x 4096 x 256 122 -> 87, 4096 x 4096 x 1024 325 -> 313 (110 TFLOP/s; a 128 x 128 tile took 288 with the sum below in
-// one chain, and there is no room in its registers for more).
+// 4096 x 4096 x 256 122 -> 87.  (k_matmul_split has taken over from both over more than some 50 k.)
 // A sum of K products is taken in four parts by k, as there: its error is that of k_matmul at every K (2.9e-7 of the result's
 // rms at 1024 k), half of what one chain has.
 __global__ void __launch_bounds__(256) k_matmul_lds(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C,
@@ -260,15 +477,6 @@ __global__ void __launch_bounds__(256) k_matmul_lds(const float *__restrict__ A,
 }
 
 // ── Q8 weights: three-way bf16 split of the activations ────────────────────
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-// bf16(a) | bf16(b) << 16, both by truncation
-__device__ __forceinline__ uint32_t pack_bf16_hi(float a, float b) {
-    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302);
-}
-__device__ __forceinline__ float top_bits(float x) {      // the leading 8 significant bits of x: a bf16 value
-    return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u);
-}
 
 // Workgroup tile 64 WTM x 64 WTN, WTM x WTN accumulators of 32 x 32 per wavefront (1 x 1: 64 x 64 tile; 2 x 2: 128 x 128).
 // G: scale groups (of 32 k) per step.  A step costs two barriers and an LDS round trip whatever its size, and a
@@ -565,37 +773,55 @@ void launch_matmul(hipStream_t s, const float *a, const float *b, float *out, in
     if ((k & 3) == 0) launch_kernel((k_matmul<TM, TN, KW, U, D, true>), dim3(tm * tn), dim3(64 * KW), 0, s, a, b, out, m, n, k, tm, tn);
     else launch_kernel((k_matmul<TM, TN, KW, U, D, false>), dim3(tm * tn), dim3(64 * KW), 0, s, a, b, out, m, n, k, tm, tn);
 }
+template <int TM, int WC, int KS>
+void launch_matmul_split(hipStream_t s, const float *a, const float *b, float *out, int m, int n, int k) {
+    const int tm = (m + 32 * TM - 1) / (32 * TM), tn = (n + 32 * WC - 1) / (32 * WC);
+    if ((k & 3) == 0) launch_kernel((k_matmul_split<TM, WC, KS, true>), dim3(tm * tn), dim3(64 * WC * KS), 0, s, a, b, out, m, n, k, tm, tn);
+    else launch_kernel((k_matmul_split<TM, WC, KS, false>), dim3(tm * tn), dim3(64 * WC * KS), 0, s, a, b, out, m, n, k, tm, tn);
+}
 }  // namespace
+
+// The kernel and tile of least estimated time, in us: fixed + weight of its rounds x (round + k x per_k), a round being a tile
+// on each of the 256 compute units.  The first of every `fit` rounds (the workgroups that a compute unit holds; k_matmul: of all)
+// weighs 1 and the others `more`: about 2 for k_matmul, two of whose workgroups on a compute unit are in each other's way.
+// `odd`: the factor on per_k where words are loaded one by one (k, or for k_matmul_lds k or n, no multiple of 4).  k_matmul
+// and k_matmul_lds were fitted to 980 shapes of 1 to 12000 rows and columns over 4 to 6000 k, some of them odd, k_matmul_split
+// to 260 of 8 to 8000 over 32 to 6000; the choice takes 1.002 times the best one's time on average over the latter, 1.09 at
+// worst, where the choice without k_matmul_split takes 1.043 and 1.94.
+static int matmul_kernel(int m, int n, int k) {
+    struct Shape { int rows, cols; double fixed, round, per_k, more; int fit; double odd; };
+    static const Shape shapes[] = {{32, 32, 2.3, 0.15, 0.0061, 1.95, 0, 1.0},     // k_matmul
+                                   {32, 64, 2.9, 0.2, 0.0101, 2.1, 0, 1.0},
+                                   {64, 64, 3.6, 0.6, 0.0178, 1.6, 0, 1.0},
+                                   {64, 64, 3.1, 2.0, 0.0177, 0.52, 3, 1.06},     // k_matmul_split
+                                   {64, 96, 0.9, 5.1, 0.0156, 0.81, 1, 1.02},
+                                   {96, 128, 0.0, 7.2, 0.029, 0.8, 1, 1.03},
+                                   {128, 128, 0.0, 9.6, 0.0348, 0.8, 1, 1.06},
+                                   {64, 64, 1.8, 1.4, 0.032, 0.5, 4, 1.6}};       // k_matmul_lds
+    constexpr int kSplit = 3, kLds = 7;
+    // k_matmul and k_matmul_split address a tile's rows of A in 32 bits, k_matmul a stage's rows of B, k_matmul_split all of B
+    const bool in_reach = (int64_t)k * 128 * 4 <= UINT32_MAX && (int64_t)n * 17 * 4 <= UINT32_MAX;
+    const bool split_reach = in_reach && (int64_t)k * n * 4 <= INT32_MAX;
+    int best = kLds;
+    double least = -1.0;
+    for (int i = in_reach ? 0 : kLds; i <= kLds; i++) {
+        if (i >= kSplit && i < kLds && !split_reach) continue;
+        const Shape &h = shapes[i];
+        const int64_t tiles = (int64_t)((m + h.rows - 1) / h.rows) * ((n + h.cols - 1) / h.cols), rounds = (tiles + 255) / 256;
+        const int64_t firsts = h.fit ? (rounds + h.fit - 1) / h.fit : 1;
+        const double weight = (double)firsts + (double)(rounds - firsts) * h.more;
+        const bool odd = i == kLds ? ((k | n) & 3) != 0 : (k & 3) != 0;
+        const double t = h.fixed + weight * (h.round + h.per_k * k * (odd ? h.odd : 1.0));
+        if (least < 0.0 || t < least) { least = t; best = i; }
+    }
+    return best;
+}
 
 void launch_matmul_f32(hipStream_t s, const float *a, const float *b, float *out, int m, int n, int k) {
     if (m <= 0 || n <= 0) return;
     if (k <= 0) { launch_fill(s, reinterpret_cast<uint32_t *>(out), 0u, (int64_t)m * n); return; }
-    // The kernel and tile of least estimated time, in us: fixed + weight of its rounds x (round + k x per_k), a round being a
-    // tile on each of the 256 compute units.  k_matmul: the first round weighs 1 and every further one `more`, about 2, as two
-    // of its workgroups on a compute unit are in each other's way (2 x 4 tiles leave no room for a second).  k_matmul_lds: the
-    // first of every four rounds (a compute unit's workgroups) 1 and the others `more`.  Fitted to 980 shapes of 1 to 12000
-    // rows and columns over 4 to 6000 k, some of them odd: the tile chosen takes 1.01 times the best one's time on average, 1.4 at
-    // worst; with rounds of k_matmul alone and one weight a tile it took 1.09 on average and 2.8 at worst.
-    struct Shape { int rows, cols; double fixed, round, per_k, more; };
-    static const Shape shapes[] = {{32, 32, 2.3, 0.15, 0.0061, 1.95}, {32, 64, 2.9, 0.2, 0.0101, 2.1},   {64, 64, 3.6, 0.6, 0.0178, 1.6},
-                                   {64, 96, 5.1, 0.6, 0.026, 2.0},    {128, 64, 5.6, 1.3, 0.0334, 1.7}, {64, 128, 0.0, 7.3, 0.0346, 0.97},
-                                   {64, 64, 1.8, 1.4, 0.032, 0.5}};
-    constexpr int kLds = 6;
-    const bool aligned = ((k | n) & 3) == 0;                       // k_matmul_lds stages word by word otherwise: 1.6 x
-    // k_matmul addresses a tile's rows of A and a stage's rows of B in 32 bits
-    const bool in_reach = (int64_t)k * 128 * 4 <= UINT32_MAX && (int64_t)n * 17 * 4 <= UINT32_MAX;
-    int best = kLds;
-    double least = -1.0;
-    for (int i = in_reach ? 0 : kLds; i <= kLds; i++) {
-        const Shape &h = shapes[i];
-        const int64_t tiles = (int64_t)((m + h.rows - 1) / h.rows) * ((n + h.cols - 1) / h.cols), rounds = (tiles + 255) / 256;
-        const int64_t firsts = i == kLds ? (rounds + 3) / 4 : 1;
-        const double weight = (double)firsts + (double)(rounds - firsts) * h.more;
-        const double t = h.fixed + weight * (h.round + h.per_k * k * (i == kLds && !aligned ? 1.6 : 1.0));
-        if (least < 0.0 || t < least) { least = t; best = i; }
-    }
     const int64_t blocks = (int64_t)((m + 31) / 32) * ((n + 31) / 32);
-    switch (best) {
+    switch (matmul_kernel(m, n, k)) {
         case 0:
             // a tile per compute unit at most: more wavefronts share its K, with shorter stages so that their lines fit
             if (blocks <= 256 && k > 256) launch_matmul<1, 1, 16, 1, 2>(s, a, b, out, m, n, k);
@@ -604,9 +830,10 @@ void launch_matmul_f32(hipStream_t s, const float *a, const float *b, float *out
             break;
         case 1: launch_matmul<1, 2, 4, 1, 4>(s, a, b, out, m, n, k); break;
         case 2: launch_matmul<2, 2, 4, 1, 2>(s, a, b, out, m, n, k); break;
-        case 3: launch_matmul<2, 3, 4, 1, 2>(s, a, b, out, m, n, k); break;
-        case 4: launch_matmul<4, 2, 4, 1, 2>(s, a, b, out, m, n, k); break;
-        case 5: launch_matmul<2, 4, 4, 1, 4>(s, a, b, out, m, n, k); break;
+        case 3: launch_matmul_split<2, 2, 2>(s, a, b, out, m, n, k); break;
+        case 4: launch_matmul_split<2, 3, 4>(s, a, b, out, m, n, k); break;
+        case 5: launch_matmul_split<3, 4, 2>(s, a, b, out, m, n, k); break;
+        case 6: launch_matmul_split<4, 4, 2>(s, a, b, out, m, n, k); break;
         default: {
             const int tn = (n + 63) / 64;
             launch_kernel(k_matmul_lds, dim3((m + 63) / 64 * tn), dim3(256), 0, s, a, b, out, m, n, k, tn);

@@ -50,6 +50,36 @@ def test_matmul_tiles_and_remainders(m, n, k):
     assert np.all(np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= bound)
 
 
+@pytest.mark.parametrize("m,n,k", [(551, 2878, 52), (743, 2462, 127), (1153, 3201, 321),                     # 64 x 64
+                                   (2003, 515, 66), (500, 2752, 97), (449, 2785, 193), (846, 1233, 200),     # 64 x 96
+                                   (1096, 1943, 39), (961, 2690, 131), (705, 2753, 97), (1000, 2752, 256),   # 96 x 128
+                                   (1000, 3083, 52), (1024, 3329, 129), (897, 3457, 159)])                   # 128 x 128
+def test_matmul_on_bf16_pieces(m, n, k):
+    """The tiles that multiply exact bf16 pieces: an element past a tile in rows and columns, K at and past their steps (32 and
+    64), under the same bound.  Then operands that have no pieces, or whose small ones are lost: infinities and NaN give what
+    the sum of the products gives, a tiny row and column (1e-36, against 1e30 and more) keep the bound."""
+    rng = np.random.default_rng(m + n * k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    a[3] *= np.float32(1e-36)
+    b[:, n - 1] *= np.float32(1e-36)
+    b[:, 5] *= np.float32(1e33)
+    a[m - 1] *= np.float32(1e30)
+    a[7] = 0.0
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    bound = 2 * k * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)) + k * 2.0 ** -149
+    exact[m - 1, 5] = 0.0                                                   # beyond fp32
+    with backend() as be:
+        got = be.matmul(tensor(a), tensor(b)).numpy().astype(np.float64)
+        got[m - 1, 5] = 0.0
+        assert np.all(np.abs(got - exact) <= bound)
+        a[0, 1], a[1, k - 1], b[0, 0] = np.inf, np.nan, -np.inf
+        got = be.matmul(tensor(a), tensor(b)).numpy()
+    assert np.all(np.isinf(got[0, 1:5])) and np.array_equal(np.sign(got[0, 1:5]), np.sign(b[1, 1:5])) and np.all(np.isnan(got[1]))
+    assert np.array_equal(got[8:m - 1, 0], np.where(a[8:m - 1, 0] > 0, -np.inf, np.inf)) and np.isnan(got[7, 0])
+    ok = (slice(8, m - 1), slice(6, n))
+    assert np.all(np.abs(got[ok] - exact[ok]) <= bound[ok])
+
+
 @pytest.mark.parametrize("m,n,k", [(128, 1, 8500000), (1, (1 << 26) + 5, 3)])
 def test_matmul_with_rows_beyond_32_bit_offsets(m, n, k):
     """A tile's rows of A, or a stage's rows of B, more than 4 GiB apart: what the last row and column hold is found there."""
