@@ -115,6 +115,13 @@ def _words(a):
     return a, a.buffer_info()[0]
 
 
+def call_addresses() -> tuple:
+    """Where the five GpuRuntime calls and the error text are: alloc, upload, download, release, flush, error."""
+    lib = library()
+    return tuple(C.cast(getattr(lib, "deepj_hip_" + n), C.c_void_p).value
+                 for n in ("alloc_buffers", "upload", "download", "release", "flush_ops", "last_error"))
+
+
 class _HostBlock:
     """A pinned block of the library under a numpy array; goes back when the array (and every view of it) is gone."""
     __slots__ = ("address", "__array_interface__", "_free")

@@ -103,12 +103,26 @@ def _compile(item):
     return obj, out
 
 
+def build_graph_core() -> str:
+    """The recording half of the tensor backend, a CPython extension (host code only)."""
+    import sysconfig
+    lib = os.path.join(HERE, "_graph_core.so")
+    cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-fvisibility=hidden", "-I", sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "graph_core.cpp"), "-o", lib + f".{os.getpid()}"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on graph_core.cpp:\n" + r.stdout + r.stderr)
+    os.replace(lib + f".{os.getpid()}", lib)        # (this process may have the present one loaded)
+    return lib
+
+
 def build(verbose: bool = False, kernarg_preload: bool = True) -> str:
     obj_dir = OBJ if kernarg_preload else OBJ + "_nopreload"
     lib = LIB if kernarg_preload else LIB_NO_PRELOAD
     common = COMMON if kernarg_preload else BASE
     os.makedirs(obj_dir, exist_ok=True)
     verify_packed_fp32_off()
+    build_graph_core()
     present = [(s, e, common, obj_dir) for s, e in SOURCES.items() if os.path.exists(os.path.join(CSRC, s))]
     with ThreadPoolExecutor(max_workers=min(8, len(present))) as ex:
         results = list(ex.map(_compile, present))

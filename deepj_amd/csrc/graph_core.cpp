@@ -1,0 +1,981 @@
+// The recording half of the tensor backend as a CPython extension: buffers, the lazy graph's bookkeeping and command words,
+// and the tensors' link to their buffers.  deepj_amd/compute_graph.py, tensor.py and hip_backend.py derive from and call these
+// types; what an operation records, the order of a flush and the error texts are theirs.
+//
+// Why native: recording is host time that no kernel hides (a tensor is read, the graph runs, the program goes on recording).
+// In Python an operation took some sixteen calls and objects, 3 to 5 us, and a round trip through ctypes 8 us more.  An attention
+// layer that reads its tensors back 20 times: 870 -> 560 us; six training steps of some 70 operations: 3040 -> 2270; a
+// feed-forward layer of 15 operations: 202 -> 177.
+//
+// A tensor's death is what releases its buffer.  Each tensor knows the (graph, id) pairs under which it is tracked and tells
+// those graphs when it goes; a graph that goes first takes itself out of its tensors.  Neither holds the other alive.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <structmember.h>
+
+#include <algorithm>
+#include <cstdint>
+#include <cstdlib>
+#include <cstring>
+#include <initializer_list>
+#include <new>
+#include <unordered_map>
+#include <utility>
+#include <vector>
+
+namespace {
+
+struct Graph;
+struct Tensor;
+
+PyObject *g_empty, *g_zeros, *g_float32, *g_pack, *g_unpack;       // numpy's and compute_graph.py's (set_helpers)
+PyTypeObject *g_tensor_class;                                      // deepj_amd.Tensor
+std::unordered_map<int, std::pair<int, std::vector<int>>> g_op_meta;     // opcode -> stride, buffer slots
+int g_fill_op;
+
+// ── GpuBuffer ───────────────────────────────────────────────────────────────
+struct Buffer {
+    PyObject_HEAD
+    int id;
+    Py_ssize_t rows, cols;
+    char needs_upload, cpu_stale, allocated;
+    PyObject *graph;                       // the graph that tracks it: told when a tensor lets go of this buffer
+};
+extern PyTypeObject BufferType, GraphType, TensorType;
+inline bool is_buffer(PyObject *o) { return o && PyObject_TypeCheck(o, &BufferType); }
+
+Buffer *new_buffer(int id, Py_ssize_t rows, Py_ssize_t cols, bool needs_upload, bool allocated, PyObject *graph) {
+    Buffer *b = reinterpret_cast<Buffer *>(BufferType.tp_alloc(&BufferType, 0));
+    if (!b) return nullptr;
+    b->id = id; b->rows = rows; b->cols = cols;
+    b->needs_upload = needs_upload; b->cpu_stale = 0; b->allocated = allocated;
+    Py_XINCREF(graph);
+    b->graph = graph;
+    return b;
+}
+int buffer_init(Buffer *self, PyObject *args, PyObject *kw) {
+    static const char *names[] = {"id", "rows", "cols", "needs_upload", "graph", nullptr};
+    int id, needs;
+    Py_ssize_t rows, cols;
+    PyObject *graph = Py_None;
+    if (!PyArg_ParseTupleAndKeywords(args, kw, "innp|O", const_cast<char **>(names), &id, &rows, &cols, &needs, &graph)) return -1;
+    self->id = id; self->rows = rows; self->cols = cols;
+    self->needs_upload = (char)needs; self->cpu_stale = 0; self->allocated = 1;
+    Py_INCREF(graph);
+    Py_XSETREF(self->graph, graph);
+    return 0;
+}
+int buffer_traverse(Buffer *self, visitproc visit, void *arg) { Py_VISIT(self->graph); return 0; }
+int buffer_clear(Buffer *self) { Py_CLEAR(self->graph); return 0; }
+void buffer_dealloc(Buffer *self) {
+    PyObject_GC_UnTrack(self);
+    Py_CLEAR(self->graph);
+    Py_TYPE(self)->tp_free(reinterpret_cast<PyObject *>(self));
+}
+PyObject *buffer_float_count(Buffer *self, PyObject *) { return PyLong_FromSsize_t(self->rows * self->cols); }
+PyMemberDef buffer_members[] = {
+    {"id", T_INT, offsetof(Buffer, id), 0, nullptr},
+    {"rows", T_PYSSIZET, offsetof(Buffer, rows), 0, nullptr},
+    {"cols", T_PYSSIZET, offsetof(Buffer, cols), 0, nullptr},
+    {"needsUpload", T_BOOL, offsetof(Buffer, needs_upload), 0, nullptr},
+    {"cpuStale", T_BOOL, offsetof(Buffer, cpu_stale), 0, nullptr},
+    {"allocatedOnGpu", T_BOOL, offsetof(Buffer, allocated), 0, nullptr},
+    {"graph", T_OBJECT, offsetof(Buffer, graph), 0, nullptr},
+    {nullptr, 0, 0, 0, nullptr}};
+PyMethodDef buffer_methods[] = {{"floatCount", (PyCFunction)buffer_float_count, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+
+// ── tensors ─────────────────────────────────────────────────────────────────
+struct Track { Graph *graph; int id; };
+struct Tensor {
+    PyObject_HEAD
+    Py_ssize_t rows, cols;
+    PyObject *data;                        // the host copy, once there is one (None or null before)
+    PyObject *tag;
+    std::vector<Track> tracks;
+};
+inline bool has_data(const Tensor *t) { return t->data && t->data != Py_None; }
+inline Buffer *tag_of(const Tensor *t) { return is_buffer(t->tag) ? reinterpret_cast<Buffer *>(t->tag) : nullptr; }
+
+// What a flush sends: values (a copy: the tensor may change before), or how many zeros.
+struct Upload {
+    int id;
+    int64_t count;
+    float *values;                         // null: zeros
+};
+
+struct Native {                            // the library's calls
+    int (*alloc)(const int32_t *, const int32_t *, int32_t);
+    int (*upload)(int32_t, const float *, int64_t);
+    int (*download)(int32_t, float *, int64_t);
+    int (*release)(const int32_t *, int32_t);
+    int (*flush)(const int32_t *, int32_t);
+    const char *(*error)();
+};
+
+struct State {
+    std::vector<int32_t> cmd;
+    int64_t ops = 0;
+    std::vector<Buffer *> allocs;          // strong
+    std::vector<Upload> uploads;
+    std::unordered_map<int, Tensor *> tensors;     // null: it has died
+    std::vector<int> maybe_orphans;
+};
+struct Graph {
+    PyObject_HEAD
+    PyObject *runtime, *zero_buffers, *host_array;
+    int next_id;
+    Native native;
+    PyTypeObject *native_type;             // a runtime of exactly this class, with nothing set on it, is spoken to directly
+    State *s;
+};
+
+void track(Graph *g, int id, Tensor *t) {
+    Tensor *&slot = g->s->tensors[id];
+    if (slot == t) return;
+    if (slot)
+        for (Track &k : slot->tracks)
+            if (k.graph == g && k.id == id) { k = slot->tracks.back(); slot->tracks.pop_back(); break; }
+    slot = t;
+    t->tracks.push_back({g, id});
+}
+void forget(Graph *g, int id) {            // the graph no longer tracks this buffer
+    auto it = g->s->tensors.find(id);
+    if (it == g->s->tensors.end()) return;
+    if (Tensor *t = it->second)
+        for (Track &k : t->tracks)
+            if (k.graph == g && k.id == id) { k = t->tracks.back(); t->tracks.pop_back(); break; }
+    g->s->tensors.erase(it);
+}
+
+PyObject *tensor_new(PyTypeObject *type, PyObject *, PyObject *) {
+    Tensor *t = reinterpret_cast<Tensor *>(type->tp_alloc(type, 0));
+    if (t) new (&t->tracks) std::vector<Track>();
+    return reinterpret_cast<PyObject *>(t);
+}
+void tensor_dealloc(Tensor *t) {
+    for (const Track &k : t->tracks) {
+        k.graph->s->tensors[k.id] = nullptr;
+        k.graph->s->maybe_orphans.push_back(k.id);
+    }
+    t->tracks.~vector();
+    Py_CLEAR(t->data);
+    Py_CLEAR(t->tag);
+    Py_TYPE(t)->tp_free(reinterpret_cast<PyObject *>(t));
+}
+// Tensor(rows, cols), or a copy of another tensor (Tensor.java:50-59)
+int tensor_init(Tensor *t, PyObject *args, PyObject *kw) {
+    static const char *names[] = {"rows", "cols", nullptr};
+    PyObject *rows, *cols = Py_None;
+    if (!PyArg_ParseTupleAndKeywords(args, kw, "O|O", const_cast<char **>(names), &rows, &cols)) return -1;
+    if (PyObject_TypeCheck(rows, &TensorType)) {
+        PyObject *r = PyObject_CallMethod(rows, "materialize", nullptr);
+        if (!r) return -1;
+        Py_DECREF(r);
+        Tensor *src = reinterpret_cast<Tensor *>(rows);
+        t->rows = src->rows; t->cols = src->cols;
+        PyObject *data = PyObject_GetAttrString(rows, "data");
+        PyObject *copy = data ? PyObject_CallMethod(data, "copy", nullptr) : nullptr;
+        Py_XDECREF(data);
+        if (!copy) return -1;
+        Py_XSETREF(t->data, copy);
+        return 0;
+    }
+    PyObject *ri = PyNumber_Long(rows), *ci = ri ? PyNumber_Long(cols) : nullptr;
+    if (ci) { t->rows = PyLong_AsSsize_t(ri); t->cols = PyLong_AsSsize_t(ci); }
+    Py_XDECREF(ri);
+    Py_XDECREF(ci);
+    if (PyErr_Occurred()) return -1;
+    if (t->rows < 0 || t->cols < 0) { PyErr_SetString(PyExc_ValueError, "negative dimensions are not allowed"); return -1; }
+    return 0;
+}
+// The host copy as it is (zeros before anything was put there)
+PyObject *tensor_data(Tensor *t, void *) {
+    if (!has_data(t)) {
+        PyObject *a = PyObject_CallFunction(g_zeros, "(nn)O", t->rows, t->cols, g_float32);
+        if (!a) return nullptr;
+        Py_XSETREF(t->data, a);
+    }
+    Py_INCREF(t->data);
+    return t->data;
+}
+int tensor_set_data(Tensor *t, PyObject *v, void *) {
+    if (!v) v = Py_None;
+    Py_INCREF(v);
+    Py_XSETREF(t->data, v);
+    return 0;
+}
+PyObject *tensor_get_tag(Tensor *t, PyObject *) {
+    PyObject *o = t->tag ? t->tag : Py_None;
+    Py_INCREF(o);
+    return o;
+}
+void set_tag(Tensor *t, PyObject *tag) {   // tag: borrowed
+    PyObject *old = t->tag;
+    Py_INCREF(tag);
+    t->tag = tag;
+    if (old && old != tag && is_buffer(old)) {
+        PyObject *g = reinterpret_cast<Buffer *>(old)->graph;
+        if (g && PyObject_TypeCheck(g, &GraphType)) reinterpret_cast<Graph *>(g)->s->maybe_orphans.push_back(reinterpret_cast<Buffer *>(old)->id);
+    }
+    Py_XDECREF(old);
+}
+PyObject *tensor_set_tag(Tensor *t, PyObject *tag) {
+    set_tag(t, tag);
+    Py_RETURN_NONE;
+}
+PyMemberDef tensor_members[] = {
+    {"rows", T_PYSSIZET, offsetof(Tensor, rows), 0, nullptr},
+    {"cols", T_PYSSIZET, offsetof(Tensor, cols), 0, nullptr},
+    {"_data", T_OBJECT, offsetof(Tensor, data), 0, nullptr},
+    {"_gpu_tag", T_OBJECT, offsetof(Tensor, tag), 0, nullptr},
+    {nullptr, 0, 0, 0, nullptr}};
+PyGetSetDef tensor_getset[] = {
+    {"data", (getter)tensor_data, (setter)tensor_set_data, "The host copy as it is (zeros before anything was put there); numpy() brings it up to date first.", nullptr},
+    {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyMethodDef tensor_methods[] = {
+    {"getGpuTag", (PyCFunction)tensor_get_tag, METH_NOARGS, nullptr},
+    {"setGpuTag", (PyCFunction)tensor_set_tag, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+// ── the graph ───────────────────────────────────────────────────────────────
+PyObject *graph_new(PyTypeObject *type, PyObject *, PyObject *) {
+    Graph *g = reinterpret_cast<Graph *>(type->tp_alloc(type, 0));
+    if (g) g->s = new State();
+    return reinterpret_cast<PyObject *>(g);
+}
+void drop_uploads(State *s) {
+    for (Upload &u : s->uploads) free(u.values);
+    s->uploads.clear();
+}
+void drop_allocs(State *s) {
+    std::vector<Buffer *> gone;
+    gone.swap(s->allocs);
+    for (Buffer *b : gone) Py_DECREF(b);
+}
+int graph_traverse(Graph *g, visitproc visit, void *arg) {
+    Py_VISIT(g->runtime); Py_VISIT(g->zero_buffers); Py_VISIT(g->host_array); Py_VISIT(g->native_type);
+    for (Buffer *b : g->s->allocs) Py_VISIT(b);
+    return 0;
+}
+int graph_clear(Graph *g) {
+    Py_CLEAR(g->runtime); Py_CLEAR(g->zero_buffers); Py_CLEAR(g->host_array); Py_CLEAR(g->native_type);
+    drop_allocs(g->s);
+    return 0;
+}
+void graph_dealloc(Graph *g) {
+    PyObject_GC_UnTrack(g);
+    graph_clear(g);
+    for (auto &e : g->s->tensors)
+        if (e.second) {
+            auto &k = e.second->tracks;
+            k.erase(std::remove_if(k.begin(), k.end(), [g](const Track &x) { return x.graph == g; }), k.end());
+        }
+    drop_uploads(g->s);
+    delete g->s;
+    Py_TYPE(g)->tp_free(reinterpret_cast<PyObject *>(g));
+}
+// GraphCore(runtime, zero_buffers or None, host_array, native class or None, addresses of its calls)
+int graph_init(Graph *g, PyObject *args, PyObject *) {
+    PyObject *runtime, *zero, *host, *type, *calls;
+    if (!PyArg_ParseTuple(args, "OOOOO", &runtime, &zero, &host, &type, &calls)) return -1;
+    if (runtime == Py_None) { PyErr_SetString(PyExc_TypeError, "runtime"); return -1; }          // Objects.requireNonNull
+    auto keep = [](PyObject *&slot, PyObject *o) { Py_INCREF(o); Py_XSETREF(slot, o); };
+    keep(g->runtime, runtime); keep(g->zero_buffers, zero); keep(g->host_array, host);
+    if (type != Py_None) {
+        unsigned long long p[6];
+        if (!PyArg_ParseTuple(calls, "KKKKKK", p, p + 1, p + 2, p + 3, p + 4, p + 5)) return -1;
+        static_assert(sizeof(Native) == sizeof(p), "six addresses");
+        memcpy(&g->native, p, sizeof(p));
+        PyObject *t = reinterpret_cast<PyObject *>(g->native_type);
+        keep(t, type);
+        g->native_type = reinterpret_cast<PyTypeObject *>(t);
+    }
+    return 0;
+}
+bool direct(Graph *g) {
+    if (!g->native_type || Py_TYPE(g->runtime) != g->native_type) return false;
+    PyObject **d = _PyObject_GetDictPtr(g->runtime);
+    return !d || !*d || PyDict_GET_SIZE(*d) == 0;
+}
+bool failed(Graph *g, int rc) {
+    if (rc == 0) return false;
+    PyObject *text = PyUnicode_DecodeUTF8(g->native.error(), (Py_ssize_t)strlen(g->native.error()), "replace");
+    if (text) { PyErr_SetObject(PyExc_RuntimeError, text); Py_DECREF(text); }
+    return true;
+}
+
+// A copy of the tensor's host values as fp32 in row order: straight where they are that already, through pack_f32 otherwise.
+bool add_upload(Graph *g, int id, Tensor *t) {
+    Upload u{id, 0, nullptr};
+    if (!has_data(t)) {
+        if (g->zero_buffers != Py_None) {  // cleared on the device, where the runtime can, instead of sending zeros
+            u.count = t->rows * t->cols;
+            g->s->uploads.push_back(u);
+            return true;
+        }
+        PyObject *d = tensor_data(t, nullptr);
+        if (!d) return false;
+        Py_DECREF(d);
+    }
+    Py_buffer v;
+    PyObject *packed = nullptr;
+    bool plain = PyObject_GetBuffer(t->data, &v, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) == 0;
+    if (plain && !(v.itemsize == 4 && v.format && strcmp(v.format, "f") == 0)) { PyBuffer_Release(&v); plain = false; }
+    if (!plain) {
+        PyErr_Clear();
+        packed = PyObject_CallFunctionObjArgs(g_pack, t, nullptr);
+        if (!packed) return false;
+        if (PyObject_GetBuffer(packed, &v, PyBUF_C_CONTIGUOUS) != 0) { Py_DECREF(packed); return false; }
+    }
+    u.count = v.len / 4;
+    u.values = static_cast<float *>(malloc(v.len ? v.len : 1));
+    if (u.values) memcpy(u.values, v.buf, v.len);
+    PyBuffer_Release(&v);
+    Py_XDECREF(packed);
+    if (!u.values) { PyErr_NoMemory(); return false; }
+    g->s->uploads.push_back(u);
+    return true;
+}
+
+bool failed(Graph *g, int rc);
+// The values of a new buffer from 1 MiB on are sent as they are instead of being copied for the flush (three weights of 11 MB:
+// 7.8 ms to their first result with the copies, 1.8 without): nothing recorded refers to the buffer yet, so it does not matter when they arrive.
+// 1: sent, 0: not of that kind, -1: an error.
+int send_now(Graph *g, Buffer *b, Tensor *t) {
+    constexpr Py_ssize_t kLarge = 1 << 20;
+    if (!has_data(t) || t->rows * t->cols * 4 < kLarge || !direct(g)) return 0;
+    Py_buffer v;
+    if (PyObject_GetBuffer(t->data, &v, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) != 0) { PyErr_Clear(); return 0; }
+    int r = 0;
+    if (v.itemsize == 4 && v.format && strcmp(v.format, "f") == 0 && v.len == t->rows * t->cols * 4) {
+        const int32_t id = b->id, size = (int32_t)(t->rows * t->cols);
+        r = failed(g, g->native.alloc(&id, &size, 1)) || failed(g, g->native.upload(id, static_cast<const float *>(v.buf), size)) ? -1 : 1;
+        if (r > 0) b->allocated = 1;
+    }
+    PyBuffer_Release(&v);
+    return r;
+}
+
+Tensor *as_tensor(PyObject *o) {
+    if (PyObject_TypeCheck(o, &TensorType)) return reinterpret_cast<Tensor *>(o);
+    PyErr_Format(PyExc_TypeError, "expected a Tensor, not %.100s", Py_TYPE(o)->tp_name);
+    return nullptr;
+}
+Buffer *ensure(Graph *g, Tensor *t) {      // borrowed
+    if (Buffer *b = tag_of(t)) {
+        auto it = g->s->tensors.find(b->id);
+        if (it == g->s->tensors.end() || it->second != t) {
+            track(g, b->id, t);
+            Py_INCREF(g);
+            Py_XSETREF(b->graph, reinterpret_cast<PyObject *>(g));
+        }
+        if (b->needs_upload) {
+            if (!has_data(t)) { PyObject *d = tensor_data(t, nullptr); if (!d) return nullptr; Py_DECREF(d); }
+            if (!add_upload(g, b->id, t)) return nullptr;
+            b->needs_upload = 0;
+            b->cpu_stale = 0;
+        }
+        return b;
+    }
+    Buffer *b = new_buffer(g->next_id, t->rows, t->cols, true, false, reinterpret_cast<PyObject *>(g));
+    if (!b) return nullptr;
+    Py_INCREF(b);                          // until it is the tag
+    const int sent = send_now(g, b, t);
+    if (sent < 0 || (sent == 0 && !add_upload(g, b->id, t))) { Py_DECREF(b); Py_DECREF(b); return nullptr; }
+    g->next_id++;
+    if (sent) Py_DECREF(b);
+    else g->s->allocs.push_back(b);        // (takes the reference)
+    set_tag(t, reinterpret_cast<PyObject *>(b));
+    track(g, b->id, t);
+    Py_DECREF(b);
+    return b;
+}
+Buffer *new_output(Graph *g, Py_ssize_t rows, Py_ssize_t cols) {       // a reference of the caller's
+    Buffer *b = new_buffer(g->next_id, rows, cols, false, false, reinterpret_cast<PyObject *>(g));
+    if (!b) return nullptr;
+    g->next_id++;
+    b->cpu_stale = 1;
+    Py_INCREF(b);
+    g->s->allocs.push_back(b);
+    return b;
+}
+PyObject *output_tensor(Graph *g, Buffer *b) {
+    PyObject *o = tensor_new(g_tensor_class, nullptr, nullptr);
+    if (!o) return nullptr;
+    Tensor *t = reinterpret_cast<Tensor *>(o);
+    t->rows = b->rows; t->cols = b->cols;
+    Py_INCREF(b);
+    t->tag = reinterpret_cast<PyObject *>(b);
+    track(g, b->id, t);
+    Py_INCREF(g);
+    Py_XSETREF(b->graph, reinterpret_cast<PyObject *>(g));
+    return o;
+}
+void bind(Graph *g, Tensor *t, Buffer *b) {
+    set_tag(t, reinterpret_cast<PyObject *>(b));
+    track(g, b->id, t);
+    Py_INCREF(g);
+    Py_XSETREF(b->graph, reinterpret_cast<PyObject *>(g));
+}
+// The result of a recorded operation: a new tensor, or `into` on its new buffer.  Takes the caller's reference to out.
+PyObject *finish(Graph *g, Buffer *out, PyObject *into) {
+    PyObject *r;
+    if (into) { bind(g, reinterpret_cast<Tensor *>(into), out); r = Py_None; Py_INCREF(r); }
+    else r = output_tensor(g, out);
+    Py_DECREF(out);
+    return r;
+}
+inline void emit(Graph *g, std::initializer_list<int64_t> words) {
+    for (int64_t w : words) g->s->cmd.push_back((int32_t)w);
+    g->s->ops++;
+}
+bool read_float_bits(PyObject *o, int32_t &bits) {
+    const double d = PyFloat_AsDouble(o);
+    if (d == -1.0 && PyErr_Occurred()) return false;
+    const float f = (float)d;
+    memcpy(&bits, &f, 4);
+    return true;
+}
+bool read_int(PyObject *o, int64_t &v) {
+    v = PyLong_AsLongLong(o);
+    return !(v == -1 && PyErr_Occurred());
+}
+bool arity(Py_ssize_t n, Py_ssize_t want) {
+    if (n == want) return true;
+    PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", want, n);
+    return false;
+}
+
+PyObject *graph_ensure(Graph *g, PyObject *o) {
+    Tensor *t = as_tensor(o);
+    Buffer *b = t ? ensure(g, t) : nullptr;
+    Py_XINCREF(b);
+    return reinterpret_cast<PyObject *>(b);
+}
+PyObject *graph_new_output(Graph *g, PyObject *const *a, Py_ssize_t n) {
+    int64_t r, c;
+    if (!arity(n, 2) || !read_int(a[0], r) || !read_int(a[1], c)) return nullptr;
+    return reinterpret_cast<PyObject *>(new_output(g, r, c));
+}
+Buffer *as_buffer(PyObject *o) {
+    if (is_buffer(o)) return reinterpret_cast<Buffer *>(o);
+    PyErr_Format(PyExc_TypeError, "expected a GpuBuffer, not %.100s", Py_TYPE(o)->tp_name);
+    return nullptr;
+}
+PyObject *graph_output_tensor(Graph *g, PyObject *o) {
+    Buffer *b = as_buffer(o);
+    return b ? output_tensor(g, b) : nullptr;
+}
+PyObject *graph_bind(Graph *g, PyObject *const *a, Py_ssize_t n) {
+    if (!arity(n, 2)) return nullptr;
+    Tensor *t = as_tensor(a[0]);
+    Buffer *b = t ? as_buffer(a[1]) : nullptr;
+    if (!b) return nullptr;
+    bind(g, t, b);
+    Py_RETURN_NONE;
+}
+PyObject *graph_let_go(Graph *g, PyObject *o) {
+    Buffer *b = as_buffer(o);
+    if (!b) return nullptr;
+    g->s->maybe_orphans.push_back(b->id);
+    Py_RETURN_NONE;
+}
+PyObject *graph_emit(Graph *g, PyObject *const *a, Py_ssize_t n) {     // one operation's words
+    const size_t at = g->s->cmd.size();
+    for (Py_ssize_t i = 0; i < n; i++) {
+        int64_t w;
+        bool ok = read_int(a[i], w);
+        if (ok && (w < INT32_MIN || w > INT32_MAX)) { PyErr_SetString(PyExc_OverflowError, "a command word is 32 bits"); ok = false; }
+        if (!ok) { g->s->cmd.resize(at); return nullptr; }
+        g->s->cmd.push_back((int32_t)w);
+    }
+    g->s->ops++;
+    Py_RETURN_NONE;
+}
+
+// ── operations of the backend: check, inputs, output, words ─────────────────
+bool same_shape(Tensor *a, Tensor *b, PyObject *name) {
+    if (a->rows == b->rows && a->cols == b->cols) return true;
+    PyErr_Format(PyExc_ValueError, "Shape mismatch for %U: %zdx%zd vs %zdx%zd", name, a->rows, a->cols, b->rows, b->cols);
+    return false;
+}
+// (opcode, name, a, b, in place)
+PyObject *graph_binary(Graph *g, PyObject *const *v, Py_ssize_t n) {
+    int64_t op;
+    if (!arity(n, 5) || !read_int(v[0], op)) return nullptr;
+    Tensor *a = as_tensor(v[2]), *b = a ? as_tensor(v[3]) : nullptr;
+    if (!b || !same_shape(a, b, v[1])) return nullptr;
+    Buffer *ga = ensure(g, a), *gb = ga ? ensure(g, b) : nullptr, *out = gb ? new_output(g, a->rows, a->cols) : nullptr;
+    if (!out) return nullptr;
+    emit(g, {op, ga->id, gb->id, out->id, out->rows * out->cols});
+    return finish(g, out, v[4] == Py_True ? v[2] : nullptr);
+}
+// (opcode, a, in place)
+PyObject *graph_unary(Graph *g, PyObject *const *v, Py_ssize_t n) {
+    int64_t op;
+    if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
+    Tensor *a = as_tensor(v[1]);
+    Buffer *ga = a ? ensure(g, a) : nullptr, *out = ga ? new_output(g, a->rows, a->cols) : nullptr;
+    if (!out) return nullptr;
+    emit(g, {op, ga->id, out->id, out->rows * out->cols});
+    return finish(g, out, v[2] == Py_True ? v[1] : nullptr);
+}
+// (opcode, a, scalar, in place)
+PyObject *graph_scalar(Graph *g, PyObject *const *v, Py_ssize_t n) {
+    int64_t op;
+    int32_t bits;
+    if (!arity(n, 4) || !read_int(v[0], op) || !read_float_bits(v[2], bits)) return nullptr;
+    Tensor *a = as_tensor(v[1]);
+    Buffer *ga = a ? ensure(g, a) : nullptr, *out = ga ? new_output(g, a->rows, a->cols) : nullptr;
+    if (!out) return nullptr;
+    emit(g, {op, ga->id, out->id, bits, out->rows * out->cols});
+    return finish(g, out, v[3] == Py_True ? v[1] : nullptr);
+}
+// (opcode, a, output rows, output columns): an operation whose words end with the input's rows and columns
+PyObject *graph_shaped(Graph *g, PyObject *const *v, Py_ssize_t n) {
+    int64_t op, rows, cols;
+    if (!arity(n, 4) || !read_int(v[0], op) || !read_int(v[2], rows) || !read_int(v[3], cols)) return nullptr;
+    Tensor *a = as_tensor(v[1]);
+    Buffer *ga = a ? ensure(g, a) : nullptr, *out = ga ? new_output(g, rows, cols) : nullptr;
+    if (!out) return nullptr;
+    emit(g, {op, ga->id, out->id, a->rows, a->cols});
+    return finish(g, out, nullptr);
+}
+PyObject *two_shaped(Graph *g, int64_t op, Tensor *a, Tensor *b) {     // out like a; a's rows and columns
+    Buffer *ga = ensure(g, a), *gb = ga ? ensure(g, b) : nullptr, *out = gb ? new_output(g, a->rows, a->cols) : nullptr;
+    if (!out) return nullptr;
+    emit(g, {op, ga->id, gb->id, out->id, a->rows, a->cols});
+    return finish(g, out, nullptr);
+}
+// (opcode, a, b): words end with a's rows and columns (shapes checked by the caller)
+PyObject *graph_pair(Graph *g, PyObject *const *v, Py_ssize_t n) {
+    int64_t op;
+    if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
+    Tensor *a = as_tensor(v[1]), *b = a ? as_tensor(v[2]) : nullptr;
+    return b ? two_shaped(g, op, a, b) : nullptr;
+}
+// (opcode, a, row vector)
+PyObject *graph_rows(Graph *g, PyObject *const *v, Py_ssize_t n) {
+    int64_t op;
+    if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
+    Tensor *a = as_tensor(v[1]), *b = a ? as_tensor(v[2]) : nullptr;
+    if (!b) return nullptr;
+    if (b->rows != 1 || b->cols != a->cols) return PyErr_Format(PyExc_ValueError, "Expected row vector 1x%zd but got %zdx%zd", a->cols, b->rows, b->cols);
+    return two_shaped(g, op, a, b);
+}
+// (opcode, a, column vector)
+PyObject *graph_cols(Graph *g, PyObject *const *v, Py_ssize_t n) {
+    int64_t op;
+    if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
+    Tensor *a = as_tensor(v[1]), *b = a ? as_tensor(v[2]) : nullptr;
+    if (!b) return nullptr;
+    if (b->rows != a->rows || b->cols != 1) return PyErr_Format(PyExc_ValueError, "Expected col vector %zdx1 but got %zdx%zd", a->rows, b->rows, b->cols);
+    return two_shaped(g, op, a, b);
+}
+// (opcode, a, b)
+PyObject *graph_matmul(Graph *g, PyObject *const *v, Py_ssize_t n) {
+    int64_t op;
+    if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
+    Tensor *a = as_tensor(v[1]), *b = a ? as_tensor(v[2]) : nullptr;
+    if (!b) return nullptr;
+    if (a->cols != b->rows) return PyErr_Format(PyExc_ValueError, "Shape mismatch for matmul: %zdx%zd vs %zdx%zd", a->rows, a->cols, b->rows, b->cols);
+    Buffer *ga = ensure(g, a), *gb = ga ? ensure(g, b) : nullptr, *out = gb ? new_output(g, a->rows, b->cols) : nullptr;
+    if (!out) return nullptr;
+    emit(g, {op, ga->id, gb->id, out->id, a->rows, b->cols, a->cols});
+    return finish(g, out, nullptr);
+}
+// (opcode, w, g, m, v, lr, beta1, beta2, eps, weight decay, c1, c2): the first, third and fourth are updated where they are
+PyObject *graph_adamw(Graph *g, PyObject *const *v, Py_ssize_t n) {
+    int64_t op;
+    int32_t bits[7];
+    if (!arity(n, 12) || !read_int(v[0], op)) return nullptr;
+    Buffer *b[4];
+    Tensor *w = nullptr;
+    for (int i = 0; i < 4; i++) {
+        Tensor *t = as_tensor(v[1 + i]);
+        if (!t || !(b[i] = ensure(g, t))) return nullptr;
+        if (i == 0) w = t;
+    }
+    for (int i = 0; i < 7; i++)
+        if (!read_float_bits(v[5 + i], bits[i])) return nullptr;
+    emit(g, {op, b[0]->id, b[1]->id, b[2]->id, b[3]->id, bits[0], bits[1], bits[2], bits[3], bits[4], bits[5], bits[6], w->rows * w->cols});
+    for (int i : {0, 2, 3}) { b[i]->cpu_stale = 1; b[i]->needs_upload = 0; }
+    Py_RETURN_NONE;
+}
+
+// ── flush ───────────────────────────────────────────────────────────────────
+// The interpreter's lock is given up while a download waits for the device and held for the other calls, which only enqueue: a
+// flush is then one step to every other thread.
+PyObject *int_array(const std::vector<int32_t> &v) {       // array.array("i", v): what a runtime in Python is handed
+    static PyObject *type = nullptr;
+    if (!type) {
+        PyObject *m = PyImport_ImportModule("array");
+        type = m ? PyObject_GetAttrString(m, "array") : nullptr;
+        Py_XDECREF(m);
+        if (!type) return nullptr;
+    }
+    return PyObject_CallFunction(type, "sy#", "i", reinterpret_cast<const char *>(v.data()), (Py_ssize_t)(v.size() * 4));
+}
+bool call(PyObject *r) {
+    Py_XDECREF(r);
+    return r != nullptr;
+}
+bool allocate_pending(Graph *g) {
+    if (g->s->allocs.empty()) return true;
+    std::vector<int32_t> ids, sizes;
+    for (Buffer *b : g->s->allocs) { ids.push_back(b->id); sizes.push_back((int32_t)(b->rows * b->cols)); }
+    const size_t count = ids.size();
+    if (direct(g)) {
+        if (failed(g, g->native.alloc(ids.data(), sizes.data(), (int32_t)count))) return false;
+    } else {
+        PyObject *a = int_array(ids), *b = a ? int_array(sizes) : nullptr;
+        const bool ok = b && call(PyObject_CallMethod(g->runtime, "allocBuffers", "OOn", a, b, (Py_ssize_t)count));
+        Py_XDECREF(a);
+        Py_XDECREF(b);
+        if (!ok) return false;
+    }
+    std::vector<Buffer *> done(g->s->allocs.begin(), g->s->allocs.begin() + count);
+    g->s->allocs.erase(g->s->allocs.begin(), g->s->allocs.begin() + count);
+    for (Buffer *b : done) { b->allocated = 1; Py_DECREF(b); }
+    return true;
+}
+bool upload_pending(Graph *g) {
+    State *s = g->s;
+    if (s->uploads.empty()) return true;
+    const bool native = direct(g);
+    const size_t count = s->uploads.size();
+    std::vector<int32_t> fills;            // first: a buffer's zeros come before whatever else is sent to it
+    PyObject *zeros = nullptr;
+    for (size_t i = 0; i < count; i++) {
+        const Upload &u = s->uploads[i];
+        if (u.values) continue;
+        if (native) { for (int64_t w : {(int64_t)g_fill_op, (int64_t)u.id, (int64_t)0, u.count}) fills.push_back((int32_t)w); continue; }
+        if (!zeros && !(zeros = PyList_New(0))) return false;
+        PyObject *pair = Py_BuildValue("(iL)", u.id, (long long)u.count);
+        const bool ok = pair && PyList_Append(zeros, pair) == 0;
+        Py_XDECREF(pair);
+        if (!ok) { Py_DECREF(zeros); return false; }
+    }
+    if (!fills.empty()) {
+        if (failed(g, g->native.flush(fills.data(), (int32_t)fills.size()))) return false;
+    }
+    if (zeros) {
+        const bool ok = call(PyObject_CallFunctionObjArgs(g->zero_buffers, zeros, nullptr));
+        Py_DECREF(zeros);
+        if (!ok) return false;
+    }
+    for (size_t i = 0; i < count; i++) {
+        const Upload u = s->uploads[i];
+        if (!u.values) continue;
+        if (native) {
+            if (failed(g, g->native.upload(u.id, u.values, u.count))) return false;
+        } else {
+            PyObject *a = PyObject_CallFunction(g_empty, "nO", (Py_ssize_t)u.count, g_float32);
+            Py_buffer v;
+            if (!a || PyObject_GetBuffer(a, &v, PyBUF_CONTIG) != 0) { Py_XDECREF(a); return false; }
+            memcpy(v.buf, u.values, v.len);
+            PyBuffer_Release(&v);
+            const bool ok = call(PyObject_CallMethod(g->runtime, "uploadBuffer", "iO", u.id, a));
+            Py_DECREF(a);
+            if (!ok) return false;
+        }
+    }
+    for (size_t i = 0; i < count; i++) free(s->uploads[i].values);
+    s->uploads.erase(s->uploads.begin(), s->uploads.begin() + count);
+    return true;
+}
+bool execute_pending(Graph *g) {           // fails before its first launch: the ops stay recorded
+    State *s = g->s;
+    if (s->ops == 0) { s->cmd.clear(); return true; }
+    std::vector<int32_t> cmd;
+    cmd.swap(s->cmd);
+    const int64_t ops = s->ops;
+    s->ops = 0;
+    bool ok;
+    if (direct(g)) {
+        ok = !failed(g, g->native.flush(cmd.data(), (int32_t)cmd.size()));
+    } else {
+        PyObject *a = int_array(cmd);
+        ok = a && call(PyObject_CallMethod(g->runtime, "flushOps", "On", a, (Py_ssize_t)cmd.size()));
+        Py_XDECREF(a);
+    }
+    if (!ok) {
+        cmd.insert(cmd.end(), s->cmd.begin(), s->cmd.end());
+        s->cmd.swap(cmd);
+        s->ops += ops;
+    } else if (s->cmd.empty()) {           // keep the memory
+        cmd.clear();
+        s->cmd.swap(cmd);
+    }
+    return ok;
+}
+bool referenced_by_pending_ops(Graph *g, int id) {
+    const auto &c = g->s->cmd;
+    for (size_t pos = 0; pos < c.size();) {
+        auto m = g_op_meta.find(c[pos]);
+        if (m == g_op_meta.end()) return true;             // unknown op: be conservative
+        for (int slot : m->second.second)
+            if (pos + slot < c.size() && c[pos + slot] == id) return true;
+        pos += m->second.first;
+    }
+    return false;
+}
+bool release_ids(Graph *g, const std::vector<int32_t> &ids) {
+    if (direct(g)) {
+        return !failed(g, g->native.release(ids.data(), (int32_t)ids.size()));
+    }
+    PyObject *a = int_array(ids);
+    const bool ok = a && call(PyObject_CallMethod(g->runtime, "releaseBuffers", "On", a, (Py_ssize_t)ids.size()));
+    Py_XDECREF(a);
+    return ok;
+}
+bool release_orphans(Graph *g) {
+    State *s = g->s;
+    if (s->maybe_orphans.empty()) return true;
+    std::vector<int> candidates;
+    candidates.swap(s->maybe_orphans);
+    std::vector<int32_t> orphans;
+    for (int id : candidates) {
+        auto it = s->tensors.find(id);
+        if (it == s->tensors.end()) continue;              // unknown, or seen before
+        if (Tensor *t = it->second) {
+            Buffer *b = tag_of(t);
+            if (b && b->id == id) continue;
+        }
+        if (s->ops > 0 && referenced_by_pending_ops(g, id)) { s->maybe_orphans.push_back(id); continue; }
+        orphans.push_back(id);
+        forget(g, id);
+    }
+    if (orphans.empty()) return true;
+    if (!s->allocs.empty() || !s->uploads.empty()) {
+        auto gone = [&](int id) { return std::find(orphans.begin(), orphans.end(), id) != orphans.end(); };
+        std::vector<Buffer *> dropped;
+        auto keep = s->allocs.begin();
+        for (Buffer *b : s->allocs) if (gone(b->id)) dropped.push_back(b); else *keep++ = b;
+        s->allocs.erase(keep, s->allocs.end());
+        auto at = s->uploads.begin();
+        for (Upload &u : s->uploads) if (gone(u.id)) free(u.values); else *at++ = u;
+        s->uploads.erase(at, s->uploads.end());
+        for (Buffer *b : dropped) Py_DECREF(b);
+    }
+    return release_ids(g, orphans);
+}
+bool flush(Graph *g) {
+    if (g->s->ops == 0 && g->s->allocs.empty()) return release_orphans(g);
+    return allocate_pending(g) && upload_pending(g) && execute_pending(g) && release_orphans(g);
+}
+PyObject *graph_flush(Graph *g, PyObject *) {
+    if (!flush(g)) return nullptr;
+    Py_RETURN_NONE;
+}
+
+// The buffer's values in the tensor's host array: written there directly, and into an array of the runtime's own kind where
+// the tensor has none yet.
+bool fetch(Graph *g, Buffer *b, PyObject *flat) {          // flat: contiguous fp32 of the buffer's size
+    if (!direct(g)) return call(PyObject_CallMethod(g->runtime, "downloadBuffer", "iO", b->id, flat));
+    Py_buffer v;
+    if (PyObject_GetBuffer(flat, &v, PyBUF_CONTIG) != 0) return false;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = g->native.download(b->id, static_cast<float *>(v.buf), v.len / 4);
+    Py_END_ALLOW_THREADS
+    PyBuffer_Release(&v);
+    return !failed(g, rc);
+}
+bool download(Graph *g, Buffer *b, Tensor *t) {
+    const Py_ssize_t count = b->rows * b->cols;
+    bool plain = false;
+    if (has_data(t)) {
+        Py_buffer v;
+        plain = PyObject_GetBuffer(t->data, &v, PyBUF_CONTIG | PyBUF_FORMAT) == 0;
+        if (plain) {
+            plain = v.itemsize == 4 && v.format && strcmp(v.format, "f") == 0;
+            const Py_ssize_t have = v.len / 4;
+            PyBuffer_Release(&v);
+            if (plain && have != count) {
+                PyErr_Format(PyExc_ValueError, "Size mismatch: src has %zd floats but tensor is %zdx%zd", count, t->rows, t->cols);
+                return false;
+            }
+        } else {
+            PyErr_Clear();
+        }
+    }
+    if (plain) {
+        if (direct(g)) return fetch(g, b, t->data);
+        PyObject *flat = PyObject_CallMethod(t->data, "reshape", "i", -1);
+        const bool ok = flat && fetch(g, b, flat);
+        Py_XDECREF(flat);
+        return ok;
+    }
+    PyObject *flat = PyObject_CallFunction(g->host_array, "n", count);
+    bool ok = flat && fetch(g, b, flat);
+    if (ok && !has_data(t) && count == t->rows * t->cols) {
+        PyObject *shaped = PyObject_CallMethod(flat, "reshape", "nn", t->rows, t->cols);
+        ok = shaped != nullptr;
+        if (ok) Py_XSETREF(t->data, shaped);
+    } else if (ok) {
+        ok = call(PyObject_CallFunctionObjArgs(g_unpack, flat, t, nullptr));
+    }
+    Py_XDECREF(flat);
+    return ok;
+}
+PyObject *graph_materialize(Graph *g, PyObject *o) {
+    Tensor *t = as_tensor(o);
+    if (!t) return nullptr;
+    Buffer *b = tag_of(t);
+    if (!b || !b->cpu_stale) Py_RETURN_NONE;
+    Py_INCREF(b);
+    const bool ok = flush(g) && download(g, b, t);
+    if (ok) b->cpu_stale = 0;
+    Py_DECREF(b);
+    if (!ok) return nullptr;
+    Py_RETURN_NONE;
+}
+PyObject *graph_release_all(Graph *g, PyObject *) {
+    if (!flush(g)) return nullptr;
+    State *s = g->s;
+    std::vector<int32_t> ids;
+    for (auto &e : s->tensors) ids.push_back(e.first);
+    std::sort(ids.begin(), ids.end());
+    for (int id : ids) {
+        auto it = s->tensors.find(id);
+        Tensor *t = it == s->tensors.end() ? nullptr : it->second;
+        Buffer *b = t ? tag_of(t) : nullptr;
+        if (!b || !b->cpu_stale) continue;
+        Py_INCREF(t);
+        Py_INCREF(b);
+        const bool ok = download(g, b, t);
+        if (ok) b->cpu_stale = b->needs_upload = 0;
+        Py_DECREF(b);
+        Py_DECREF(t);
+        if (!ok) return nullptr;
+    }
+    for (int id : ids) {
+        auto it = s->tensors.find(id);
+        if (Tensor *t = it == s->tensors.end() ? nullptr : it->second) set_tag(t, Py_None);
+    }
+    if (!ids.empty() && !release_ids(g, ids)) return nullptr;
+    while (!s->tensors.empty()) forget(g, s->tensors.begin()->first);
+    s->maybe_orphans.clear();
+    drop_allocs(s);
+    drop_uploads(s);
+    s->cmd.clear();
+    s->ops = 0;
+    g->next_id = 0;
+    Py_RETURN_NONE;
+}
+PyObject *graph_is_empty(Graph *g, PyObject *) { return PyBool_FromLong(g->s->ops == 0); }
+
+#define FAST(name, f) {name, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
+PyMethodDef graph_methods[] = {
+    {"ensureGpuBuffer", (PyCFunction)graph_ensure, METH_O, nullptr},
+    FAST("newOutputBuffer", graph_new_output),
+    {"createOutputTensor", (PyCFunction)graph_output_tensor, METH_O, nullptr},
+    FAST("bindTensorToBuffer", graph_bind),
+    {"tensorLetGo", (PyCFunction)graph_let_go, METH_O, "Tensor.setGpuTag: the buffer is no longer the tag of a tensor that had it."},
+    FAST("_emit", graph_emit),
+    FAST("binary", graph_binary),
+    FAST("unary", graph_unary),
+    FAST("scalar", graph_scalar),
+    FAST("shaped", graph_shaped),
+    FAST("pair", graph_pair),
+    FAST("rowBroadcast", graph_rows),
+    FAST("colBroadcast", graph_cols),
+    FAST("matmul", graph_matmul),
+    FAST("adamW", graph_adamw),
+    {"isEmpty", (PyCFunction)graph_is_empty, METH_NOARGS, nullptr},
+    {"flush", (PyCFunction)graph_flush, METH_NOARGS, nullptr},
+    {"materialize", (PyCFunction)graph_materialize, METH_O, nullptr},
+    {"releaseAll", (PyCFunction)graph_release_all, METH_NOARGS, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyMemberDef graph_members[] = {
+    {"runtime", T_OBJECT_EX, offsetof(Graph, runtime), 0, nullptr},
+    {nullptr, 0, 0, 0, nullptr}};
+
+PyTypeObject BufferType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+PyTypeObject GraphType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+PyTypeObject TensorType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// set_helpers(numpy.empty, numpy.zeros, numpy.float32, pack_f32, unpack_f32_into, op meta {opcode: (stride, slots)}, fill opcode)
+PyObject *set_helpers(PyObject *, PyObject *args) {
+    PyObject *p[5], *meta;
+    if (!PyArg_ParseTuple(args, "OOOOOO!i", p, p + 1, p + 2, p + 3, p + 4, &PyDict_Type, &meta, &g_fill_op)) return nullptr;
+    PyObject **slot[5] = {&g_empty, &g_zeros, &g_float32, &g_pack, &g_unpack};
+    for (int i = 0; i < 5; i++) { Py_INCREF(p[i]); Py_XSETREF(*slot[i], p[i]); }
+    PyObject *key, *value;
+    for (Py_ssize_t pos = 0; PyDict_Next(meta, &pos, &key, &value);) {
+        int stride;
+        PyObject *slots;
+        if (!PyArg_ParseTuple(value, "iO!", &stride, &PyTuple_Type, &slots)) return nullptr;
+        std::vector<int> s;
+        for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(slots); i++) s.push_back((int)PyLong_AsLong(PyTuple_GET_ITEM(slots, i)));
+        if (PyErr_Occurred()) return nullptr;
+        g_op_meta[(int)PyLong_AsLong(key)] = {stride, s};
+    }
+    Py_RETURN_NONE;
+}
+PyObject *set_tensor_class(PyObject *, PyObject *o) {
+    if (!PyType_Check(o) || !PyType_IsSubtype(reinterpret_cast<PyTypeObject *>(o), &TensorType)) {
+        PyErr_SetString(PyExc_TypeError, "a class derived from TensorCore");
+        return nullptr;
+    }
+    Py_INCREF(o);
+    g_tensor_class = reinterpret_cast<PyTypeObject *>(o);
+    Py_RETURN_NONE;
+}
+PyMethodDef module_methods[] = {
+    {"set_helpers", set_helpers, METH_VARARGS, nullptr},
+    {"set_tensor_class", set_tensor_class, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_graph_core", nullptr, -1, module_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__graph_core() {
+    BufferType.tp_name = "deepj_amd.GpuBuffer";
+    BufferType.tp_doc = "GpuBuffer.java:9-32.";
+    BufferType.tp_basicsize = sizeof(Buffer);
+    BufferType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE | Py_TPFLAGS_HAVE_GC;
+    BufferType.tp_new = PyType_GenericNew;
+    BufferType.tp_init = (initproc)buffer_init;
+    BufferType.tp_traverse = (traverseproc)buffer_traverse;
+    BufferType.tp_clear = (inquiry)buffer_clear;
+    BufferType.tp_dealloc = (destructor)buffer_dealloc;
+    BufferType.tp_members = buffer_members;
+    BufferType.tp_methods = buffer_methods;
+
+    TensorType.tp_name = "deepj_amd._graph_core.TensorCore";
+    TensorType.tp_basicsize = sizeof(Tensor);
+    TensorType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE;
+    TensorType.tp_new = tensor_new;
+    TensorType.tp_init = (initproc)tensor_init;
+    TensorType.tp_dealloc = (destructor)tensor_dealloc;
+    TensorType.tp_members = tensor_members;
+    TensorType.tp_getset = tensor_getset;
+    TensorType.tp_methods = tensor_methods;
+
+    GraphType.tp_name = "deepj_amd._graph_core.GraphCore";
+    GraphType.tp_basicsize = sizeof(Graph);
+    GraphType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE | Py_TPFLAGS_HAVE_GC;
+    GraphType.tp_new = graph_new;
+    GraphType.tp_init = (initproc)graph_init;
+    GraphType.tp_traverse = (traverseproc)graph_traverse;
+    GraphType.tp_clear = (inquiry)graph_clear;
+    GraphType.tp_dealloc = (destructor)graph_dealloc;
+    GraphType.tp_members = graph_members;
+    GraphType.tp_methods = graph_methods;
+
+    if (PyType_Ready(&BufferType) < 0 || PyType_Ready(&TensorType) < 0 || PyType_Ready(&GraphType) < 0) return nullptr;
+    PyObject *m = PyModule_Create(&module_def);
+    if (!m) return nullptr;
+    Py_INCREF(&BufferType);
+    Py_INCREF(&TensorType);
+    Py_INCREF(&GraphType);
+    if (PyModule_AddObject(m, "GpuBuffer", reinterpret_cast<PyObject *>(&BufferType)) < 0 ||
+        PyModule_AddObject(m, "TensorCore", reinterpret_cast<PyObject *>(&TensorType)) < 0 ||
+        PyModule_AddObject(m, "GraphCore", reinterpret_cast<PyObject *>(&GraphType)) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -13,12 +13,16 @@ from __future__ import annotations
 import numpy as np
 
 from . import opcodes as op
-from ._native import HipNative, host_array
+from ._native import HipNative, call_addresses, host_array
 from .compute_graph import ComputeGraph, GpuBuffer
 from .tensor import Tensor
 
 
 class HipGpuRuntime:
+    """Five calls passed on to the native library; a graph over an object of exactly this class makes them itself."""
+
+    nativeCalls = staticmethod(call_addresses)
+
     def allocBuffers(self, ids, sizes, count): HipNative.nativeAllocBuffers(ids, sizes, count)
     def uploadBuffer(self, buf_id, data): HipNative.nativeUploadBuffer(buf_id, data)
     def downloadBuffer(self, buf_id, out): HipNative.nativeDownloadBuffer(buf_id, out)
@@ -29,16 +33,6 @@ class HipGpuRuntime:
     def zeroBuffers(self, buffers):
         cmd = [w for buf_id, n in buffers for w in (op.OP_FILL, buf_id, 0, n)]
         HipNative.nativeFlushOps(cmd, len(cmd))
-
-
-def _require_row_vector(v, target):
-    if v.rows != 1 or v.cols != target.cols:
-        raise ValueError(f"Expected row vector 1x{target.cols} but got {v.rows}x{v.cols}")
-
-
-def _require_col_vector(v, target):
-    if v.rows != target.rows or v.cols != 1:
-        raise ValueError(f"Expected col vector {target.rows}x1 but got {v.rows}x{v.cols}")
 
 
 class HipBackend:
@@ -68,101 +62,48 @@ class HipBackend:
         self._int_column_scratch.clear()
 
     # ── matmul / element-wise ───────────────────────────────────────────────
-    def matmul(self, a, b):
-        if a.cols != b.rows:
-            raise ValueError(f"Shape mismatch for matmul: {a.rows}x{a.cols} vs {b.rows}x{b.cols}")
-        ga, gb = self._in(a), self._in(b)
-        out = self.graph.newOutputBuffer(a.rows, b.cols)
-        self.graph.recordMatmul(ga, gb, out, a.rows, b.cols, a.cols)
-        return self._out(out)
-
-    def _binary(self, opcode, name, a, b):
-        Tensor.requireSameShape(a, b, name)
-        ga, gb = self._in(a), self._in(b)
-        out = self.graph.newOutputBuffer(a.rows, a.cols)
-        self.graph.recordBinary(opcode, ga, gb, out)
-        return out
-
-    def add(self, a, b): return self._out(self._binary(op.OP_ADD, "add", a, b))
-    def subtract(self, a, b): return self._out(self._binary(op.OP_SUBTRACT, "subtract", a, b))
-    def multiply(self, a, b): return self._out(self._binary(op.OP_MULTIPLY, "multiply", a, b))
-    def divide(self, a, b): return self._out(self._binary(op.OP_DIVIDE, "divide", a, b))
-    def reluBackward(self, x, g): return self._out(self._binary(op.OP_RELU_BACKWARD, "reluBackward", x, g))
-    def geluBackward(self, x, g): return self._out(self._binary(op.OP_GELU_BACKWARD, "geluBackward", x, g))
+    def matmul(self, a, b): return self.graph.matmul(op.OP_MATMUL, a, b)
+    def add(self, a, b): return self.graph.binary(op.OP_ADD, "add", a, b, False)
+    def subtract(self, a, b): return self.graph.binary(op.OP_SUBTRACT, "subtract", a, b, False)
+    def multiply(self, a, b): return self.graph.binary(op.OP_MULTIPLY, "multiply", a, b, False)
+    def divide(self, a, b): return self.graph.binary(op.OP_DIVIDE, "divide", a, b, False)
+    def reluBackward(self, x, g): return self.graph.binary(op.OP_RELU_BACKWARD, "reluBackward", x, g, False)
+    def geluBackward(self, x, g): return self.graph.binary(op.OP_GELU_BACKWARD, "geluBackward", x, g, False)
 
     # ── broadcasts ──────────────────────────────────────────────────────────
-    def _row_bcast(self, opcode, a, v):
-        _require_row_vector(v, a)
-        ga, gv = self._in(a), self._in(v)
-        out = self.graph.newOutputBuffer(a.rows, a.cols)
-        self.graph.recordRowBroadcast(opcode, ga, gv, out, a.rows, a.cols)
-        return self._out(out)
-
-    def _col_bcast(self, opcode, a, v):
-        _require_col_vector(v, a)
-        ga, gv = self._in(a), self._in(v)
-        out = self.graph.newOutputBuffer(a.rows, a.cols)
-        self.graph.recordColBroadcast(opcode, ga, gv, out, a.rows, a.cols)
-        return self._out(out)
-
-    def addRowVector(self, a, v): return self._row_bcast(op.OP_ADD_ROW_VECTOR, a, v)
+    def addRowVector(self, a, v): return self.graph.rowBroadcast(op.OP_ADD_ROW_VECTOR, a, v)
     def addBroadcastRows(self, a, v): return self.addRowVector(a, v)
-    def multiplyBroadcastRows(self, a, v): return self._row_bcast(op.OP_MULTIPLY_BROADCAST_ROWS, a, v)
-    def addBroadcastCols(self, a, v): return self._col_bcast(op.OP_ADD_BROADCAST_COLS, a, v)
-    def subtractBroadcastCols(self, a, v): return self._col_bcast(op.OP_SUBTRACT_BROADCAST_COLS, a, v)
-    def divideBroadcastCols(self, a, v): return self._col_bcast(op.OP_DIVIDE_BROADCAST_COLS, a, v)
-    def multiplyBroadcastCols(self, a, v): return self._col_bcast(op.OP_MULTIPLY_BROADCAST_COLS, a, v)
+    def multiplyBroadcastRows(self, a, v): return self.graph.rowBroadcast(op.OP_MULTIPLY_BROADCAST_ROWS, a, v)
+    def addBroadcastCols(self, a, v): return self.graph.colBroadcast(op.OP_ADD_BROADCAST_COLS, a, v)
+    def subtractBroadcastCols(self, a, v): return self.graph.colBroadcast(op.OP_SUBTRACT_BROADCAST_COLS, a, v)
+    def divideBroadcastCols(self, a, v): return self.graph.colBroadcast(op.OP_DIVIDE_BROADCAST_COLS, a, v)
+    def multiplyBroadcastCols(self, a, v): return self.graph.colBroadcast(op.OP_MULTIPLY_BROADCAST_COLS, a, v)
 
     # ── scalar ops ──────────────────────────────────────────────────────────
-    def _scalar(self, opcode, a, s):
-        ga = self._in(a)
-        out = self.graph.newOutputBuffer(a.rows, a.cols)
-        if opcode == op.OP_MULTIPLY_SCALAR:
-            self.graph.recordMultiplyScalar(ga, out, s)
-        else:
-            self.graph.recordScalarUnary(opcode, ga, out, s)
-        return out
-
-    def multiplyScalar(self, a, s): return self._out(self._scalar(op.OP_MULTIPLY_SCALAR, a, s))
-    def addScalar(self, a, s): return self._out(self._scalar(op.OP_ADD_SCALAR, a, s))
-    def divideScalar(self, a, s): return self._out(self._scalar(op.OP_DIVIDE_SCALAR, a, s))
+    def multiplyScalar(self, a, s): return self.graph.scalar(op.OP_MULTIPLY_SCALAR, a, s, False)
+    def addScalar(self, a, s): return self.graph.scalar(op.OP_ADD_SCALAR, a, s, False)
+    def divideScalar(self, a, s): return self.graph.scalar(op.OP_DIVIDE_SCALAR, a, s, False)
 
     # ── reductions ──────────────────────────────────────────────────────────
-    def _reduce(self, opcode, a, out_rows, out_cols):
-        ga = self._in(a)
-        out = self.graph.newOutputBuffer(out_rows, out_cols)
-        self.graph.recordReduction(opcode, ga, out, a.rows, a.cols)
-        return self._out(out)
-
-    def sumRows(self, a): return self._reduce(op.OP_SUM_ROWS, a, 1, a.cols)
+    def sumRows(self, a): return self.graph.shaped(op.OP_SUM_ROWS, a, 1, a.cols)
     def sumAlongCols(self, a): return self.sumRows(a)
-    def sumAlongRows(self, a): return self._reduce(op.OP_SUM_ALONG_ROWS, a, a.rows, 1)
-    def meanAlongRows(self, a): return self._reduce(op.OP_MEAN_ALONG_ROWS, a, a.rows, 1)
-    def varianceAlongRows(self, a): return self._reduce(op.OP_VARIANCE_ALONG_ROWS, a, a.rows, 1)
-    def maxAlongRows(self, a): return self._reduce(op.OP_MAX_ALONG_ROWS, a, a.rows, 1)
+    def sumAlongRows(self, a): return self.graph.shaped(op.OP_SUM_ALONG_ROWS, a, a.rows, 1)
+    def meanAlongRows(self, a): return self.graph.shaped(op.OP_MEAN_ALONG_ROWS, a, a.rows, 1)
+    def varianceAlongRows(self, a): return self.graph.shaped(op.OP_VARIANCE_ALONG_ROWS, a, a.rows, 1)
+    def maxAlongRows(self, a): return self.graph.shaped(op.OP_MAX_ALONG_ROWS, a, a.rows, 1)
 
     def sum(self, a) -> float:
-        ga = self._in(a)
-        out = self.graph.newOutputBuffer(1, 1)
-        self.graph.recordSumScalar(ga, out, a.rows, a.cols)
-        scalar = self._out(out)
+        scalar = self.graph.shaped(op.OP_SUM_SCALAR, a, 1, 1)
         scalar.materialize()
         return float(scalar.data[0, 0])
 
     def sumAbs(self, a) -> float:
-        ga = self._in(a)
-        rows = self.graph.newOutputBuffer(a.rows, 1)
-        self.graph.recordSumAbs(ga, rows, a.rows, a.cols)
-        scalar = self.sumRows(self._out(rows))
+        scalar = self.sumRows(self.graph.shaped(op.OP_SUM_ABS, a, a.rows, 1))
         scalar.materialize()
         return float(scalar.data[0, 0])
 
     # ── unary ───────────────────────────────────────────────────────────────
-    def transpose(self, a):
-        ga = self._in(a)
-        out = self.graph.newOutputBuffer(a.cols, a.rows)
-        self.graph.recordTranspose(ga, out, a.rows, a.cols)
-        return self._out(out)
+    def transpose(self, a): return self.graph.shaped(op.OP_TRANSPOSE, a, a.cols, a.rows)
 
     def clamp(self, a, lo, hi):
         ga = self._in(a)
@@ -170,66 +111,44 @@ class HipBackend:
         self.graph.recordClamp(ga, out, lo, hi)
         return self._out(out)
 
-    def pow(self, a, exponent):
-        ga = self._in(a)
-        out = self.graph.newOutputBuffer(a.rows, a.cols)
-        self.graph.recordPow(ga, out, exponent)
-        return self._out(out)
-
-    def _unary(self, opcode, a):
-        ga = self._in(a)
-        out = self.graph.newOutputBuffer(a.rows, a.cols)
-        self.graph.recordUnary(opcode, ga, out)
-        return out
-
-    def sqrt(self, a): return self._out(self._unary(op.OP_SQRT, a))
-    def neg(self, a): return self._out(self._unary(op.OP_NEG, a))
-    def exp(self, a): return self._out(self._unary(op.OP_EXP, a))
-    def log(self, a): return self._out(self._unary(op.OP_LOG, a))
-    def tanh(self, a): return self._out(self._unary(op.OP_TANH, a))
-    def sigmoid(self, a): return self._out(self._unary(op.OP_SIGMOID, a))
-    def relu(self, a): return self._out(self._unary(op.OP_RELU, a))
-    def gelu(self, a): return self._out(self._unary(op.OP_GELU, a))
+    def pow(self, a, exponent): return self.graph.scalar(op.OP_POW, a, exponent, False)
+    def sqrt(self, a): return self.graph.unary(op.OP_SQRT, a, False)
+    def neg(self, a): return self.graph.unary(op.OP_NEG, a, False)
+    def exp(self, a): return self.graph.unary(op.OP_EXP, a, False)
+    def log(self, a): return self.graph.unary(op.OP_LOG, a, False)
+    def tanh(self, a): return self.graph.unary(op.OP_TANH, a, False)
+    def sigmoid(self, a): return self.graph.unary(op.OP_SIGMOID, a, False)
+    def relu(self, a): return self.graph.unary(op.OP_RELU, a, False)
+    def gelu(self, a): return self.graph.unary(op.OP_GELU, a, False)
 
     # ── softmax ─────────────────────────────────────────────────────────────
-    def softmaxRows(self, logits):
-        ga = self._in(logits)
-        out = self.graph.newOutputBuffer(logits.rows, logits.cols)
-        self.graph.recordSoftmaxRows(ga, out, logits.rows, logits.cols)
-        return self._out(out)
+    def softmaxRows(self, logits): return self.graph.shaped(op.OP_SOFTMAX_ROWS, logits, logits.rows, logits.cols)
 
     def softmaxBackward(self, grad, softmax):
         Tensor.requireSameShape(grad, softmax, "softmaxBackward")
-        gg, gs = self._in(grad), self._in(softmax)
-        out = self.graph.newOutputBuffer(grad.rows, grad.cols)
-        self.graph.recordSoftmaxBackward(gg, gs, out, grad.rows, grad.cols)
-        return self._out(out)
+        return self.graph.pair(op.OP_SOFTMAX_BACKWARD, grad, softmax)
 
     # ── in-place: new buffer, rebind (MetalBackend.java:400-526) ────────────
-    def addInPlace(self, a, b): self.graph.bindTensorToBuffer(a, self._binary(op.OP_ADD, "addInPlace", a, b))
-    def subtractInPlace(self, a, b): self.graph.bindTensorToBuffer(a, self._binary(op.OP_SUBTRACT, "subtractInPlace", a, b))
-    def multiplyInPlace(self, a, b): self.graph.bindTensorToBuffer(a, self._binary(op.OP_MULTIPLY, "multiplyInPlace", a, b))
-    def divideInPlace(self, a, b): self.graph.bindTensorToBuffer(a, self._binary(op.OP_DIVIDE, "divideInPlace", a, b))
-    def multiplyScalarInPlace(self, a, s): self.graph.bindTensorToBuffer(a, self._scalar(op.OP_MULTIPLY_SCALAR, a, s))
-    def addScalarInPlace(self, a, s): self.graph.bindTensorToBuffer(a, self._scalar(op.OP_ADD_SCALAR, a, s))
-    def divideScalarInPlace(self, a, s): self.graph.bindTensorToBuffer(a, self._scalar(op.OP_DIVIDE_SCALAR, a, s))
-    def sqrtInPlace(self, a): self.graph.bindTensorToBuffer(a, self._unary(op.OP_SQRT, a))
-    def negInPlace(self, a): self.graph.bindTensorToBuffer(a, self._unary(op.OP_NEG, a))
-    def expInPlace(self, a): self.graph.bindTensorToBuffer(a, self._unary(op.OP_EXP, a))
-    def logInPlace(self, a): self.graph.bindTensorToBuffer(a, self._unary(op.OP_LOG, a))
-    def reluInPlace(self, a): self.graph.bindTensorToBuffer(a, self._unary(op.OP_RELU, a))
-    def geluInPlace(self, a): self.graph.bindTensorToBuffer(a, self._unary(op.OP_GELU, a))
-    def tanhInPlace(self, a): self.graph.bindTensorToBuffer(a, self._unary(op.OP_TANH, a))
-    def sigmoidInPlace(self, a): self.graph.bindTensorToBuffer(a, self._unary(op.OP_SIGMOID, a))
+    def addInPlace(self, a, b): self.graph.binary(op.OP_ADD, "addInPlace", a, b, True)
+    def subtractInPlace(self, a, b): self.graph.binary(op.OP_SUBTRACT, "subtractInPlace", a, b, True)
+    def multiplyInPlace(self, a, b): self.graph.binary(op.OP_MULTIPLY, "multiplyInPlace", a, b, True)
+    def divideInPlace(self, a, b): self.graph.binary(op.OP_DIVIDE, "divideInPlace", a, b, True)
+    def multiplyScalarInPlace(self, a, s): self.graph.scalar(op.OP_MULTIPLY_SCALAR, a, s, True)
+    def addScalarInPlace(self, a, s): self.graph.scalar(op.OP_ADD_SCALAR, a, s, True)
+    def divideScalarInPlace(self, a, s): self.graph.scalar(op.OP_DIVIDE_SCALAR, a, s, True)
+    def sqrtInPlace(self, a): self.graph.unary(op.OP_SQRT, a, True)
+    def negInPlace(self, a): self.graph.unary(op.OP_NEG, a, True)
+    def expInPlace(self, a): self.graph.unary(op.OP_EXP, a, True)
+    def logInPlace(self, a): self.graph.unary(op.OP_LOG, a, True)
+    def reluInPlace(self, a): self.graph.unary(op.OP_RELU, a, True)
+    def geluInPlace(self, a): self.graph.unary(op.OP_GELU, a, True)
+    def tanhInPlace(self, a): self.graph.unary(op.OP_TANH, a, True)
+    def sigmoidInPlace(self, a): self.graph.unary(op.OP_SIGMOID, a, True)
 
     # ── fused ops ───────────────────────────────────────────────────────────
     def crossEntropyGradient(self, logits, targets):
         Tensor.requireTargetsMatchRows(logits, targets)
-        tt = self._int_column(targets)
-        gl, gt = self._in(logits), self._in(tt)
-        out = self.graph.newOutputBuffer(logits.rows, logits.cols)
-        self.graph.recordCrossEntropyGradient(gl, gt, out, logits.rows, logits.cols)
-        return self._out(out)
+        return self.graph.pair(op.OP_CROSS_ENTROPY_GRADIENT, logits, self._int_column(targets))
 
     def crossEntropyLoss(self, logits, targets) -> float:
         Tensor.requireTargetsMatchRows(logits, targets)
@@ -244,12 +163,7 @@ class HipBackend:
     def adamWUpdate(self, w, g, mt, vt, lr, beta1, beta2, eps, weight_decay, bc1, bc2):
         for other in (g, mt, vt):
             Tensor.requireSameShape(w, other, "adamWUpdate")
-        gw, gg, gmt, gvt = self._in(w), self._in(g), self._in(mt), self._in(vt)
-        self.graph.recordAdamWUpdate(gw, gg, gmt, gvt, lr, beta1, beta2, eps, weight_decay, bc1, bc2,
-                                     w.rows * w.cols)
-        for b in (gw, gmt, gvt):
-            b.cpuStale = True
-            b.needsUpload = False
+        self.graph.adamW(op.OP_ADAMW_UPDATE, w, g, mt, vt, lr, beta1, beta2, eps, weight_decay, bc1, bc2)
 
     def layerNormBackward(self, dxhat, xhat, std, dim):
         Tensor.requireSameShape(dxhat, xhat, "layerNormBackward")

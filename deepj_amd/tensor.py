@@ -9,35 +9,20 @@ from __future__ import annotations
 
 import numpy as np
 
-from .compute_graph import GpuBuffer
+from .compute_graph import GpuBuffer, _graph_core
 
 
-class Tensor:
+class Tensor(_graph_core.TensorCore):
+    """Tensor(rows, cols), or a copy of another tensor (Tensor.java:50-59).  rows, cols, data (the host copy, made when it is
+    first asked for), getGpuTag and setGpuTag are csrc/graph_core.cpp."""
+
     _backend = None
 
-    def __init__(self, rows: int, cols: int | None = None):
-        self._gpu_tag = None
-        self._data = None                                 # the host copy: made when it is first asked for
-        if isinstance(rows, Tensor):                      # copy constructor (Tensor.java:50-59)
-            src = rows
-            src.materialize()
-            self.rows, self.cols = src.rows, src.cols
-            self._data = src.data.copy()
-        else:
-            self.rows, self.cols = int(rows), int(cols)
-            if self.rows < 0 or self.cols < 0:
-                raise ValueError("negative dimensions are not allowed")
+    def __getstate__(self): return self.rows, self.cols, self._data, self._gpu_tag, self.__dict__
 
-    @property
-    def data(self) -> np.ndarray:
-        """The host copy as it is (zeros before anything was put there); numpy() brings it up to date first."""
-        if self._data is None:
-            self._data = np.zeros((self.rows, self.cols), dtype=np.float32)
-        return self._data
-
-    @data.setter
-    def data(self, value) -> None:
-        self._data = value
+    def __setstate__(self, state):
+        self.rows, self.cols, self._data, self._gpu_tag, extra = state
+        self.__dict__.update(extra)
 
     # ── backend switch (Tensor.java:24-41) ──────────────────────────────────
     @staticmethod
@@ -51,13 +36,6 @@ class Tensor:
         if Tensor._backend is None:
             raise RuntimeError("no TensorBackend set: call Tensor.setBackend(HipBackend())")
         return Tensor._backend
-
-    def getGpuTag(self): return self._gpu_tag
-
-    def setGpuTag(self, tag):
-        old, self._gpu_tag = self._gpu_tag, tag
-        if old is not None and old is not tag and isinstance(old, GpuBuffer) and old.graph is not None:
-            old.graph.tensorLetGo(old)
 
     def materialize(self) -> "Tensor":
         if self._gpu_tag is not None:
@@ -222,3 +200,6 @@ class Tensor:
         """Materialised host copy."""
         self.materialize()
         return self.data
+
+
+_graph_core.set_tensor_class(Tensor)

@@ -314,3 +314,66 @@ def test_int_targets_travel_as_float_column(rt):                      # MetalBac
     assert len(cols) == 1 and list(cols[0]) == [4.0, 0.0, 2.0]
     s = list(rt.flushCalls[0][0])
     assert s[0] == op.OP_CROSS_ENTROPY_GRADIENT and s[4:6] == [3, 5]
+
+
+def test_tensors_graphs_and_copies_outlive_one_another():
+    """A tensor tells every graph that tracks it when it goes, and a graph that is gone is told nothing; host tensors copy."""
+    import copy
+    import pickle
+    first, second = RecordingRuntime(), RecordingRuntime()
+    g1, g2 = ComputeGraph(first), ComputeGraph(second)
+    t = Tensor.from2D([[1.0, 2.0]])
+    buf = g1.ensureGpuBuffer(t).id
+    assert g2.ensureGpuBuffer(t).id == buf and t.getGpuTag().graph is g2
+    kept = g1.createOutputTensor(g1.newOutputBuffer(2, 2))
+    g1.flush(), g2.flush()
+    del t
+    g1.flush(), g2.flush()
+    assert [list(r.releaseCalls[-1][0]) for r in (first, second)] == [[buf], [buf]]
+    del g1
+    gc.collect()
+    kept.setGpuTag(None)
+    del kept
+
+    # a buffer bound back to its tensor before the flush stays; one bound to another tensor belongs to that one
+    a, b = Tensor.from2D([[1.0]]), Tensor.from2D([[2.0]])
+    old = g2.ensureGpuBuffer(a)
+    g2.flush()
+    a.setGpuTag(None)
+    a.setGpuTag(old)
+    n = len(second.releaseCalls)
+    g2.flush()
+    assert len(second.releaseCalls) == n
+    g2.bindTensorToBuffer(b, old)
+    del a
+    g2.flush()
+    assert len(second.releaseCalls) == n
+    del b
+    g2.flush()
+    assert list(second.releaseCalls[-1][0]) == [old.id]
+
+    host = Tensor.from2D([[1.0, 2.0], [3.0, 4.0]])
+    host.note = "kept"
+    for c in (copy.copy(host), copy.deepcopy(host), pickle.loads(pickle.dumps(host))):
+        assert (c.rows, c.cols, c.note) == (2, 2, "kept") and np.array_equal(c.data, host.data)
+    assert copy.copy(host).data is host.data and copy.deepcopy(host).data is not host.data
+
+
+def test_values_of_other_layouts_travel_as_fp32_rows(graph, rt):
+    """Host arrays that are not contiguous fp32 are packed on the way out, filled on the way back; a size that does not fit is refused."""
+    t = Tensor(2, 3)
+    t.data = np.arange(6, dtype=np.float64).reshape(3, 2).T
+    buf = graph.ensureGpuBuffer(t)
+    graph.flush()
+    assert list(rt.uploads[0][1]) == [0, 2, 4, 1, 3, 5] and rt.uploads[0][1].dtype == np.float32
+    buf.cpuStale = True
+    rt.downloadResult = [5, 4, 3, 2, 1, 0]
+    graph.materialize(t)
+    assert t.data.dtype == np.float64 and t.data.tolist() == [[5, 4, 3], [2, 1, 0]]
+    small = Tensor(1, 2)
+    small.data.fill(1)
+    small.setGpuTag(graph.newOutputBuffer(3, 3))
+    with pytest.raises(ValueError, match="Size mismatch"):
+        graph.materialize(small)
+    with pytest.raises(TypeError):
+        graph.ensureGpuBuffer(np.zeros((2, 2)))
