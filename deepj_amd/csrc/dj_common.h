@@ -67,6 +67,14 @@ void launch_binary(hipStream_t s, int op, const float *a, const float *b, float 
 void launch_unary(hipStream_t s, int op, const float *a, float *out, int64_t n);
 void launch_scalar(hipStream_t s, int op, const float *a, float *out, float s0, float s1, int64_t n);
 void launch_broadcast(hipStream_t s, int op, const float *a, const float *v, float *out, int rows, int cols);
+// Consecutive element-wise operations over the same elements in one launch.  A slot holds a value per element: first those of
+// `ext` (the slot of the same number), then what the operations put there.
+constexpr int kChainOps = 8, kChainExt = 6, kChainSlots = 8;
+struct ChainExt { const float *p; int kind; };      // 0: an element each, 1: a row vector, 2: a column vector
+struct ChainOp { int op, a, b, dst; float *out; float s0, s1; };       // op: a binary, unary or scalar opcode
+struct Chain { ChainExt ext[kChainExt]; ChainOp ops[kChainOps]; int n_ext, n_ops; int64_t n; int cols; };
+bool chain_takes(int op);
+void launch_chain(hipStream_t s, const Chain &chain);
 void launch_transpose(hipStream_t s, const float *a, float *out, int rows, int cols);
 // AdamW on up to kAdamTensors tensors in one launch (none of them shares memory with another)
 constexpr int kAdamTensors = 16;

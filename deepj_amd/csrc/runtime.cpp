@@ -637,6 +637,130 @@ void need_positive(int op, const char *what, int64_t v) {
     if (v < 0) fail(std::string(op_name(op)) + ": negative " + what + " " + std::to_string(v));
 }
 
+// An element-wise op as a link of a chain: ids and what is done with them.  op 0: no such op.
+struct Link { int op = 0, kind = 0, words = 0; int32_t a = -1, b = -1, out = -1; int64_t n = 0, rows = 0, cols = 0; float s0 = 0.0f, s1 = 0.0f; };
+Link chain_link(const int32_t *w) {
+    Link l;
+    auto set = [&](int op, int kind, int words, int32_t a, int32_t b, int32_t out, int64_t n) { l.op = op; l.kind = kind; l.words = words; l.a = a; l.b = b; l.out = out; l.n = n; };
+    auto vec = [&](int op, int kind) { set(op, kind, 6, w[1], w[2], w[3], (int64_t)w[4] * w[5]); l.rows = w[4]; l.cols = w[5]; };
+    switch (w[0]) {
+        case DJ_OP_ADD: case DJ_OP_SUBTRACT: case DJ_OP_MULTIPLY: case DJ_OP_DIVIDE: case DJ_OP_RELU_BACKWARD: case DJ_OP_GELU_BACKWARD:
+            set(w[0], 0, 5, w[1], w[2], w[3], w[4]); break;
+        case DJ_OP_MULTIPLY_SCALAR: case DJ_OP_ADD_SCALAR: case DJ_OP_DIVIDE_SCALAR:
+            set(w[0], 0, 5, w[1], -1, w[2], w[4]); l.s0 = bits_to_float(w[3]); break;
+        case DJ_OP_CLAMP: set(w[0], 0, 6, w[1], -1, w[2], w[5]); l.s0 = bits_to_float(w[3]); l.s1 = bits_to_float(w[4]); break;
+        case DJ_OP_ADD_ROW_VECTOR: vec(DJ_OP_ADD, 1); break;
+        case DJ_OP_MULTIPLY_BROADCAST_ROWS: vec(DJ_OP_MULTIPLY, 1); break;
+        case DJ_OP_ADD_BROADCAST_COLS: vec(DJ_OP_ADD, 2); break;
+        case DJ_OP_SUBTRACT_BROADCAST_COLS: vec(DJ_OP_SUBTRACT, 2); break;
+        case DJ_OP_DIVIDE_BROADCAST_COLS: vec(DJ_OP_DIVIDE, 2); break;
+        case DJ_OP_MULTIPLY_BROADCAST_COLS: vec(DJ_OP_MULTIPLY, 2); break;
+        default:
+            if (chain_takes(w[0]) && stride_of(w[0]) == 4) set(w[0], 0, 4, w[1], -1, w[2], w[3]);
+    }
+    return l;
+}
+
+// The element-wise ops from here on that work on the same elements, as one launch (k_chain): one of a few between two products
+// costs little more than a launch, and each of them reads what the one before it wrote.  A product between two of them that
+// has nothing to do with those in front of it goes first.  False: too few.
+//
+// Every thread takes its elements through all the ops, so an op may read and write what others of them read and write at the
+// same elements - but a vector is read by all threads, and must be none of the results.
+void exec_one(Cursor &c);
+bool exec_chain(Cursor &c) {
+    Chain chain{};
+    int32_t ext_id[kChainExt], vectors[kChainOps], outs[kChainOps];
+    Link links[kChainOps];
+    int operand[kChainOps][2];                    // >= 0: an external value, < 0: the result of op -1 - operand
+    int n_vec = 0, count = 0;
+    int32_t at = c.pos, end = c.pos, products[2], planned[2];
+    int n_products = 0, n_planned = 0;
+    int64_t cols = 0;
+    auto among = [](const int32_t *ids, int n, int32_t id) { return std::find(ids, ids + n, id) != ids + n; };
+    while (at < c.len && count < kChainOps && at + stride_of(c.cmd[at]) <= c.len) {
+        const int32_t *w = c.cmd + at;
+        if (w[0] == DJ_OP_MATMUL && count > 0) {
+            if (n_planned == 2 || among(outs, count, w[1]) || among(outs, count, w[2]) || among(outs, count, w[3]) ||
+                among(ext_id, chain.n_ext, w[3])) break;
+            planned[n_planned++] = at;
+            at += 7;
+            continue;
+        }
+        const Link l = chain_link(w);
+        if (!l.op || l.n <= 0 || l.n > 0x7fffffffLL || (count && l.n != chain.n)) break;
+        if (l.kind) {
+            if ((cols && l.cols != cols) || l.cols <= 0 || among(outs, count, l.b) || l.out == l.b) break;
+        }
+        if (among(vectors, n_vec, l.out)) break;
+        int n_ext = chain.n_ext;
+        auto find = [&](int32_t id, int kind, int &to) {
+            if (kind == 0)
+                for (int k = count; k-- > 0;)
+                    if (outs[k] == id) { to = -1 - k; return true; }
+            for (int j = 0; j < n_ext; j++)
+                if (ext_id[j] == id && chain.ext[j].kind == kind) { to = j; return true; }
+            if (n_ext == kChainExt) return false;
+            ext_id[n_ext] = id;
+            chain.ext[n_ext].kind = kind;
+            to = n_ext++;
+            return true;
+        };
+        int a, b;
+        if (!find(l.a, 0, a)) break;
+        b = a;
+        if (l.b >= 0 && !find(l.b, l.kind, b)) break;
+        chain.n_ext = n_ext;
+        if (l.kind) { cols = l.cols; vectors[n_vec++] = l.b; }
+        operand[count][0] = a; operand[count][1] = b;
+        outs[count] = l.out;
+        links[count++] = l;
+        chain.n = l.n;
+        at += l.words;
+        end = at;
+        while (n_products < n_planned) { products[n_products] = planned[n_products]; n_products++; }
+    }
+    // What a launch costs against what k_chain's own code does (interpreting, LDS, half the memory rate of a kernel that does one
+    // thing), us together / one by one: 500 values, 2 ops 5.8 / 5.6 behind other kernels, 4 ops 5.4 / 10.2; 500 x 1024: 2 ops
+    // 4.8 .. 5.3 / 4.9 .. 5.2, behind a product 5.7 / 9.4, 4 ops 7.1 / 10.2; 500 x 2752: 2 ops 7.2 .. 9.2 / 5.4 .. 6.3, 4 ops 12.7 / 12.4,
+    // 5 behind products 16.5 / 27.6; 1024 x 7000: 2 ops 20 .. 27 / 18 .. 22, 4 ops 38 / 47; 2048 x 8192: 41 .. 52 / 38 .. 41, 91 / 106.
+    if (count < (chain.n < (1 << 17) ? 3 : chain.n <= (1 << 20) ? 2 : 4)) return false;
+
+    // A result takes the slot of an operand that nothing needs any more, or a free one: an op that would need a ninth ends the chain.
+    int last_use[kChainExt + kChainOps], slot_of[kChainExt + kChainOps];       // values: the external ones, then the results
+    auto value = [&](int x) { return x >= 0 ? x : kChainExt + (-1 - x); };
+    for (int &u : last_use) u = -1;
+    for (int k = 0; k < count; k++)
+        for (int x : operand[k]) last_use[value(x)] = k;
+    bool used[kChainSlots] = {};
+    for (int j = 0; j < chain.n_ext; j++) { slot_of[j] = j; used[j] = true; }
+    for (int k = 0; k < count; k++) {
+        const int va = value(operand[k][0]), vb = value(operand[k][1]);
+        for (int v : {va, vb})
+            if (last_use[v] == k) used[slot_of[v]] = false;
+        int dst = 0;
+        while (dst < kChainSlots && used[dst]) dst++;
+        if (dst == kChainSlots) return false;
+        slot_of[kChainExt + k] = dst;
+        used[dst] = last_use[kChainExt + k] > k;
+        const Link &l = links[k];
+        chain.ops[k] = {l.op, slot_of[va], slot_of[vb], dst, buf(l.out, l.n, l.op, "out"), l.s0, l.s1};
+    }
+    for (int j = 0; j < chain.n_ext; j++) {
+        const int kind = chain.ext[j].kind;
+        chain.ext[j].p = buf(ext_id[j], kind == 0 ? chain.n : kind == 1 ? cols : chain.n / cols, links[0].op, "in");
+    }
+    chain.n_ops = count;
+    chain.cols = cols ? (int)cols : (int)chain.n;
+    for (int i = 0; i < n_products; i++) {
+        Cursor m{c.cmd, c.len, products[i], false, {}};
+        exec_one(m);
+    }
+    launch_chain(g.stream, chain);
+    c.skip = end - c.pos - stride_of(c.cmd[c.pos]);
+    return true;
+}
+
 void exec_one(Cursor &c) {
     const int32_t *w = c.cmd + c.pos;
     const int op = w[0];
@@ -649,6 +773,7 @@ void exec_one(Cursor &c) {
         return run && was.valid && was.cmd == c.cmd && was.pos == c.pos && was.x_id == x_id && was.gamma_id == gamma_id && was.m == m &&
                was.k == k && (flags & DJ_LIN_RMSNORM) && !(flags & DJ_LIN_LAYERNORM);
     };
+    if (run && !c.alone && op < DJ_OP_Q8_QUANTIZE && exec_chain(c)) return;
     switch (op) {
         case DJ_OP_ADD: case DJ_OP_SUBTRACT: case DJ_OP_MULTIPLY: case DJ_OP_DIVIDE: case DJ_OP_RELU_BACKWARD:
         case DJ_OP_GELU_BACKWARD: {

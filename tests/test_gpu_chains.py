@@ -1,0 +1,104 @@
+"""Consecutive element-wise operations run as one launch: the same bits as each of them by itself, whatever they read and
+write in common."""
+import numpy as np
+import pytest
+
+from deepj_amd import opcodes as op
+from deepj_amd.fused import DeviceBuffers, Stream
+
+pytestmark = pytest.mark.gpu
+
+BINARY = [op.OP_ADD, op.OP_SUBTRACT, op.OP_MULTIPLY, op.OP_DIVIDE, op.OP_RELU_BACKWARD, op.OP_GELU_BACKWARD]
+UNARY = [op.OP_SQRT, op.OP_NEG, op.OP_EXP, op.OP_LOG, op.OP_TANH, op.OP_SIGMOID, op.OP_RELU, op.OP_GELU]
+SCALAR = [op.OP_MULTIPLY_SCALAR, op.OP_ADD_SCALAR, op.OP_DIVIDE_SCALAR, op.OP_POW]
+ROWS = [op.OP_ADD_ROW_VECTOR, op.OP_MULTIPLY_BROADCAST_ROWS]
+COLS = [op.OP_ADD_BROADCAST_COLS, op.OP_SUBTRACT_BROADCAST_COLS, op.OP_DIVIDE_BROADCAST_COLS, op.OP_MULTIPLY_BROADCAST_COLS]
+
+
+def _bits(x):
+    return int(np.float32(x).view(np.int32))
+
+
+def _program(rng, rows, cols, length):
+    """(ops, buffers): words with buffer indexes; 0 .. 5 hold rows x cols values, 6, 7 a row, 8, 9 a column, 10, 11 square operands."""
+    n, ops = rows * cols, []
+    full = lambda: int(rng.integers(0, 6))
+    for _ in range(length):
+        kind = int(rng.integers(0, 8))
+        a, b, out = full(), full(), full()
+        if kind <= 1:
+            ops.append([int(rng.choice(BINARY)), a, b, out, n])
+        elif kind == 2:
+            ops.append([int(rng.choice(UNARY)), a, out, n])
+        elif kind == 3:
+            ops.append([int(rng.choice(SCALAR)), a, out, _bits(rng.uniform(0.5, 1.5)), n])
+        elif kind == 4:
+            ops.append([op.OP_CLAMP, a, out, _bits(-1.5), _bits(2.0), n])
+        elif kind == 5:
+            ops.append([int(rng.choice(ROWS)), a, int(rng.integers(6, 8)), out, rows, cols])
+        elif kind == 6:
+            ops.append([int(rng.choice(COLS)), a, int(rng.integers(8, 10)), out, rows, cols])
+        else:
+            ops.append([op.OP_MATMUL, int(rng.integers(10, 12)), a, out, rows, cols, rows] if rng.random() < 0.7 and out != a
+                       else [op.OP_SUM_ALONG_ROWS, a, int(rng.integers(8, 10)), rows, cols])
+    return ops
+
+
+SLOTS = {5: (1, 2, 3), 4: (1, 2), 6: (1, 2, 3), 7: (1, 2, 3)}
+
+
+def _ids(word, ids):
+    code = word[0]
+    if code in UNARY or code in SCALAR or code in (op.OP_CLAMP, op.OP_SUM_ALONG_ROWS):
+        at = (1, 2)
+    else:
+        at = (1, 2, 3)
+    return [ids[w] if i in at else w for i, w in enumerate(word)]
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 3), (5, 1), (3, 5), (7, 64), (33, 130), (64, 257), (300, 41)])
+def test_a_chain_has_the_bits_of_its_operations(rows, cols):
+    rng = np.random.default_rng(rows * 1000 + cols)
+    for trial in range(40):
+        ops = _program(rng, rows, cols, int(rng.integers(2, 24)))
+        shapes = [rows * cols] * 6 + [cols] * 2 + [rows] * 2 + [rows * rows] * 2
+        values = [(rng.standard_normal(s) * (1.0 if i < 10 else rows ** -0.5)).astype(np.float32) for i, s in enumerate(shapes)]
+        if trial % 8 == 0:
+            values[0][0], values[1][-1], values[2][0] = np.inf, np.nan, -0.0
+        results = []
+        for together in (True, False):
+            dev = DeviceBuffers()
+            try:
+                ids = [dev.upload(v) for v in values]
+                if together:
+                    s = Stream()
+                    for o in ops:
+                        s.emit(*_ids(o, ids))
+                    s.run()
+                else:
+                    for o in ops:
+                        Stream().emit(*_ids(o, ids)).run()
+                results.append([dev.download(b, (n,)) for b, n in zip(ids, shapes)])
+            finally:
+                dev.release_all()
+        for k, (x, y) in enumerate(zip(*results)):
+            same = (x.view(np.uint32) == y.view(np.uint32)) | (np.isnan(x) & np.isnan(y))
+            assert same.all(), (trial, k, ops)
+
+
+def test_a_product_between_two_operations_that_depends_on_one_of_them_stays_there():
+    """x = a + b; y = m . x; z = y * x: the product reads a result in front of it, and overwrites an operand behind it."""
+    rng = np.random.default_rng(0)
+    a, b, m = (rng.standard_normal((32, 32)).astype(np.float32) for _ in range(3))
+    dev = DeviceBuffers()
+    try:
+        A, B, M, X, Z = dev.upload(a), dev.upload(b), dev.upload(m), dev.alloc(1024), dev.alloc(1024)
+        s = Stream().emit(op.OP_ADD, A, B, X, 1024).matmul(M, X, A, 32, 32, 32).emit(op.OP_MULTIPLY, A, X, Z, 1024).emit(op.OP_NEG, Z, B, 1024)
+        s.run()
+        got = dev.download(B, (32, 32))
+    finally:
+        dev.release_all()
+    x = (a + b).astype(np.float64)
+    exp = -(m.astype(np.float64) @ x) * x
+    bound = 2 * 33 * 2.0 ** -24 * (np.abs(m).astype(np.float64) @ np.abs(x)) * np.abs(x)
+    assert np.all(np.abs(got - exp) <= bound)
