@@ -126,13 +126,16 @@ void launch_argmax_rows(hipStream_t s, const float *a, int32_t *out, int rows, i
 void launch_matmul_f32(hipStream_t s, const float *a, const float *b, float *out, int m, int n, int k);
 
 // kernels_q8.hip
-// Two consecutive fp16 GEMMs of a stream, the second normalising (RMSNorm) and multiplying the first one's output: when
-// the first shares its tiles' K among workgroups, the kernel that adds their partial products also writes the second
-// one's activations in its layout, and the second skips its own split.
+// Two consecutive products of a stream, the second normalising and multiplying the first one's output: where the first shares its
+// tiles' K among workgroups, the kernel that adds their partial products also leaves the second one's activations in its
+// layout, and the second skips its own split.  Two fp16 GEMMs (RMSNorm), or k_gemm_q8 in front of k_gemm_q8_rows.
 struct GemmChain {
     const float *next_gamma = nullptr;   // to the first launch: the gain the next GEMM normalises this output with
-    bool left_planes = false;            // from the first launch: it left the next GEMM's activations in the workspace
+    bool left_planes = false;            // from the first launch: it left the next fp16 GEMM's activations in the workspace
     bool planes_ready = false;           // to the second launch: they are there
+    uint16_t *next_pieces = nullptr;     // to the first launch: the next product takes k_gemm_q8_rows, with its rows' pieces there
+    const float *next_beta = nullptr;    // (LayerNorm)
+    bool left_pieces = false, pieces_ready = false;
 };
 
 struct Q8Linear {
@@ -144,7 +147,7 @@ struct Q8Linear {
     const int32_t *m_dev = nullptr;   // GEMM path only: live row count = min(m, m_dev[0] + m_extra)
     int m_extra = 0;
     const float *prepared = nullptr;  // the weights in the fp16 GEMM's layout (launch_q8_prepare), or null: converted per call
-    GemmChain *chain = nullptr;       // fp16 GEMM only
+    GemmChain *chain = nullptr;
     RopeStore rope;                   // fp16 GEMM only: out = nullptr, the q | k | v row goes through RoPE to q and the caches
     bool small_workspace_only = false; // the caller's workspace cannot grow: stay on the kernels that need M * K floats at most
 };

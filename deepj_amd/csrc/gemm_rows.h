@@ -41,6 +41,10 @@ __device__ __forceinline__ void load_to_lds4(const void *base, uint32_t off, uin
 int q8_gemm_f16_forced();        // DEEPJ_HIP_GEMM_F16, -1 where it is not set; 0: every GEMM on k_gemm_q8
 // The rows, normalised if gamma (and beta) say so, in that order; rows [m, m_pad) as zeros
 void launch_split_operand(hipStream_t s, const float *x, const float *gamma, const float *beta, uint16_t *planes, int m, int m_pad, int k, int kp);
+// The same for rows that are still partial products [splits][m][k] and have to be stored as well: out = residual + (their sum + bias)
+bool split_operand_sum_ok(int k);
+void launch_split_operand_sum(hipStream_t s, const float *partial, int splits, const float *bias, const float *residual, float *out, const float *gamma,
+                              const float *beta, uint16_t *planes, int m, int k);
 
 // An estimate of a Q8 GEMM's time in us.  With x workgroups a compute unit, in `rounds` rounds, kk thousand k a workgroup and
 // `full` of its rows inside the matrix:
@@ -65,6 +69,6 @@ struct RowsPlan { int tmw, tnw, shares; double us; };      // a tile's rows and 
 bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared, bool may_share, RowsPlan *plan = nullptr);
 int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, const RowsPlan &plan);
 void launch_q8_gemm_rows(hipStream_t s, const float *x, const float *gamma, const float *beta, const int8_t *wq, const float *scales, float *out, int m, int k,
-                         int n_rows, const GemmEpilogue &ep, const RowsPlan &plan, float *workspace, int64_t workspace_floats);
+                         int n_rows, const GemmEpilogue &ep, const RowsPlan &plan, float *workspace, int64_t workspace_floats, bool pieces_ready);
 
 }  // namespace dj

@@ -350,14 +350,14 @@ int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, const RowsPlan &
 }
 
 void launch_q8_gemm_rows(hipStream_t s, const float *x, const float *gamma, const float *beta, const int8_t *wq, const float *scales, float *out, int m, int k,
-                         int n_rows, const GemmEpilogue &ep, const RowsPlan &p, float *workspace, int64_t workspace_floats) {
+                         int n_rows, const GemmEpilogue &ep, const RowsPlan &p, float *workspace, int64_t workspace_floats, bool pieces_ready) {
     if (workspace_floats < q8_gemm_rows_workspace_floats(m, n_rows, k, p)) fail("q8_gemm_rows: workspace too small");
     if (ep.swiglu && ((n_rows & 1) || ep.residual || ep.gelu)) fail("q8_gemm_rows: the SwiGLU epilogue needs an even row count and takes no residual or GELU");
     const int kp = q8_padded_k(k), ka = (int)round_up(kp, kOperandChunk), m_pad = (int)round_up(m, 32);
     const int m_tiles = (m + 32 * p.tmw - 1) / (32 * p.tmw), n_tiles = (n_rows + 32 * p.tnw - 1) / (32 * p.tnw);
     float *w = workspace;
     uint16_t *planes = reinterpret_cast<uint16_t *>(w); w += (int64_t)m_pad * ka / 2 * kOperandPieces;
-    launch_split_operand(s, x, gamma, beta, planes, m, m_pad, k, ka);
+    if (!pieces_ready) launch_split_operand(s, x, gamma, beta, planes, m, m_pad, k, ka);      // (the product in front has left them: GemmChain)
     GemmRowsArgs a{reinterpret_cast<const uintx4 *>(planes), wq, scales, out, m, n_rows, kp / kQ8Group, m_tiles, n_tiles, ep, 0, nullptr};
     dim3 grid((unsigned)((n_tiles + 7) / 8 * 8 * m_tiles));
     if (p.shares > 1) {

@@ -901,7 +901,7 @@ void launch_q8_sum_partials(hipStream_t s, const float *partial, float *out, int
 void launch_q8_gemm(hipStream_t s, const float *x, const int8_t *wq, const float *scales, float *out, int m,
                     int k, int n_rows, const float *bias, const float *bias2, const float *residual,
                     int interleaved_bias, const int32_t *m_dev, int m_extra, int gelu, int swiglu, float *workspace,
-                    int64_t workspace_floats) {
+                    int64_t workspace_floats, GemmChain *chain) {
     if (m <= 0 || n_rows <= 0) return;
     if (swiglu && ((n_rows & 1) || residual || gelu)) fail("q8_gemm: the SwiGLU epilogue needs an even row count and takes no residual or GELU");
     GemmEpilogue ep{bias, bias2, residual, interleaved_bias, m_dev, m_extra, gelu, swiglu};
@@ -923,7 +923,12 @@ void launch_q8_gemm(hipStream_t s, const float *x, const int8_t *wq, const float
         grid.z = shares;
         launch_kernel((k_gemm_q8<1, 1, kGroupsFew, kSetsFew>), grid, dim3(256 * kSetsFew), 0, s, x, wq, scales, out, m, n_rows, k, q8_padded_k(k), ep,
                       per * step, workspace);
-        launch_q8_sum_partials(s, workspace, out, shares, m, n_rows, ep);
+        if (chain && chain->next_pieces && !gelu && !swiglu && !interleaved_bias && split_operand_sum_ok(n_rows)) {
+            launch_split_operand_sum(s, workspace, shares, bias, residual, out, chain->next_gamma, chain->next_beta, chain->next_pieces, m, n_rows);
+            chain->left_pieces = true;
+        } else {
+            launch_q8_sum_partials(s, workspace, out, shares, m, n_rows, ep);
+        }
         return;
     }
     // few tiles (about one per CU): a workgroup brings its own second wavefront per SIMD

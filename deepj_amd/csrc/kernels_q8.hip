@@ -34,7 +34,7 @@ namespace dj {
 void launch_q8_gemm(hipStream_t s, const float *x, const int8_t *wq, const float *scales, float *out, int m,
                     int k, int n_rows, const float *bias, const float *bias2, const float *residual,
                     int interleaved_bias, const int32_t *m_dev, int m_extra, int gelu, int swiglu, float *workspace,
-                    int64_t workspace_floats);
+                    int64_t workspace_floats, GemmChain *chain = nullptr);
 int64_t q8_gemm_workspace_floats(int m, int n_rows, int k);
 
 namespace {
@@ -782,7 +782,8 @@ void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_
     if (!p.m_dev && !rope && !(p.chain && p.chain->planes_ready) && q8_gemm_rows_ok(p.m, n_rows, p.k, gamma != nullptr, p.prepared && may_share, may_share, &plan) &&
         pieces_floats >= q8_gemm_rows_workspace_floats(p.m, n_rows, p.k, plan)) {
         const GemmEpilogue ep{bias, swiglu ? bias2 : nullptr, residual, swiglu, nullptr, 0, swiglu ? 0 : gelu, swiglu, RopeStore{}};
-        launch_q8_gemm_rows(s, p.x, gamma, beta, p.wq, p.scales, p.out, p.m, p.k, n_rows, ep, plan, pieces, pieces_floats);
+        launch_q8_gemm_rows(s, p.x, gamma, beta, p.wq, p.scales, p.out, p.m, p.k, n_rows, ep, plan, pieces, pieces_floats,
+                            p.chain && p.chain->pieces_ready);
         return;
     }
     if (!p.m_dev && !p.small_workspace_only && q8_gemm_f16_shape_ok(p.m, n_rows, p.k, p.prepared != nullptr) && workspace_floats >= q8_gemm_f16_workspace_floats(p.m, n_rows, p.k, p.prepared != nullptr)) {
@@ -808,7 +809,8 @@ void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_
         // the GEMM's epilogue pairs the interleaved gate/up columns, so the 2N-wide product never reaches memory
         launch_q8_gemm(s, x, p.wq, p.scales, p.out, p.m, p.k, 2 * p.n, bias, bias2, nullptr, 1, nullptr, 0, 0, 1, part, part_floats);
     } else {
-        launch_q8_gemm(s, x, p.wq, p.scales, p.out, p.m, p.k, p.n, bias, nullptr, residual, 0, p.m_dev, p.m_extra, gelu, 0, part, part_floats);
+        launch_q8_gemm(s, x, p.wq, p.scales, p.out, p.m, p.k, p.n, bias, nullptr, residual, 0, p.m_dev, p.m_extra, gelu, 0, part, part_floats,
+                       p.chain);
     }
 }
 

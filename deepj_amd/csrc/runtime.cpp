@@ -101,7 +101,7 @@ struct Runtime {
     unsigned char *static_scratch = nullptr;       // device address of `scratch` below on g.device
     // Set by a K-sharing fp16 GEMM that also wrote the activations of the op right behind it in that op's layout
     // (GemmChain): which op of which stream, reading which buffer through which gain.  Good for that one op only.
-    struct ChainSlot { const int32_t *cmd = nullptr; int32_t pos = -1, x_id = -1, gamma_id = -1; int64_t m = 0, k = 0; bool valid = false; } chain;
+    struct ChainSlot { const int32_t *cmd = nullptr; int32_t pos = -1, x_id = -1, gamma_id = -1, beta_id = -1; int64_t m = 0, k = 0; bool pieces = false, valid = false; } chain;
     bool no_alloc = false;                         // inside deepj_hip_flush_ops_noalloc: nothing may allocate
     std::vector<std::pair<int32_t, void *>> *track = nullptr;   // graph capture: buffers the dry pass resolves
     Graph *capture_into = nullptr;                               // graph capture: the graph the run pass records for
@@ -770,8 +770,14 @@ void exec_one(Cursor &c) {
     if (run) g.chain.valid = false;
     // this op is the one a GemmChain's first launch prepared the activations of (x, gain, shape as it saw them)
     auto chained = [&](int32_t x_id, int32_t gamma_id, int flags, int64_t m, int64_t k) {
-        return run && was.valid && was.cmd == c.cmd && was.pos == c.pos && was.x_id == x_id && was.gamma_id == gamma_id && was.m == m &&
+        return run && was.valid && !was.pieces && was.cmd == c.cmd && was.pos == c.pos && was.x_id == x_id && was.gamma_id == gamma_id && was.m == m &&
                was.k == k && (flags & DJ_LIN_RMSNORM) && !(flags & DJ_LIN_LAYERNORM);
+    };
+    // the same for the rows' pieces that a product leaves to k_gemm_q8_rows
+    auto pieces_left = [&](int64_t m, int64_t k) {
+        const int flags = w[7];
+        return run && was.valid && was.pieces && was.cmd == c.cmd && was.pos == c.pos && was.x_id == w[1] && was.gamma_id == w[8] && was.m == m && was.k == k &&
+               (flags & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM)) && was.beta_id == (flags & DJ_LIN_LAYERNORM ? w[10] : -1);
     };
     if (run && !c.alone && op < DJ_OP_Q8_QUANTIZE && exec_chain(c)) return;
     switch (op) {
@@ -998,10 +1004,11 @@ void exec_one(Cursor &c) {
             // fp16 GEMM (whose operands live in a workspace sized by the shape) is never taken there.
             p.small_workspace_only = g.no_alloc;
             GemmChain chain;
-            int32_t next_gamma_id = -1;
+            int32_t next_gamma_id = -1, next_beta_id = -1;
             const int32_t next_pos = c.pos + stride_of(op);
             if (run && m > 1 && !g.no_alloc && !merge) {
                 chain.planes_ready = chained(w[1], w[8], flags, m, k);
+                chain.pieces_ready = pieces_left(m, k);
                 // the op right behind this one normalises this output (RMSNorm) and multiplies it on the fp16 GEMM: the
                 // launch may leave that op's activations ready (it does when this one shares its tiles' K)
                 if (next_pos < c.len && !sw) {
@@ -1015,13 +1022,28 @@ void exec_one(Cursor &c) {
                             chain.next_gamma = buf(next_gamma_id, n, op, "the next op's gamma");
                         }
                     }
+                    // ... or on the kernel that multiplies a batch of rows from the int8 weights
+                    const int norms = DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM;
+                    if (!chain.next_gamma && g.row_pieces && next_pos + 12 <= c.len && nw[0] == DJ_OP_Q8_LINEAR && nw[1] == w[3] && nw[4] == m && nw[5] == n &&
+                        nw[6] > 0 && nw[6] < (1 << 30) && (nw[7] & norms) && !(nw[7] & DJ_LIN_ATTN_MERGE)) {
+                        const int64_t n_rows = (nw[7] & DJ_LIN_SWIGLU) ? 2 * (int64_t)nw[6] : (int64_t)nw[6];
+                        auto it = g.prepared.find(nw[2]);
+                        const bool prepared = it != g.prepared.end() && it->second.k == n && it->second.rows == n_rows;
+                        const int64_t pieces = q8_linear_pieces_floats((int)m, (int)n, nw[6], nw[7], prepared);
+                        if (pieces > 0 && pieces <= g.row_pieces_floats) {
+                            next_gamma_id = nw[8];
+                            chain.next_gamma = buf(next_gamma_id, n, op, "the next op's gamma");
+                            if (nw[7] & DJ_LIN_LAYERNORM) { next_beta_id = nw[10]; chain.next_beta = buf(next_beta_id, n, op, "the next op's beta"); }
+                            chain.next_pieces = reinterpret_cast<uint16_t *>(g.row_pieces);
+                        }
+                    }
                 }
                 p.chain = &chain;
             }
             if (run) launch_q8_linear(s, p, g.workspace, g.workspace_floats, g.row_pieces, g.row_pieces_floats);
-            if (chain.left_planes) {
-                g.chain.cmd = c.cmd; g.chain.pos = next_pos; g.chain.x_id = w[3]; g.chain.gamma_id = next_gamma_id;
-                g.chain.m = m; g.chain.k = n; g.chain.valid = true;
+            if (chain.left_planes || chain.left_pieces) {
+                g.chain.cmd = c.cmd; g.chain.pos = next_pos; g.chain.x_id = w[3]; g.chain.gamma_id = next_gamma_id; g.chain.beta_id = next_beta_id;
+                g.chain.m = m; g.chain.k = n; g.chain.pieces = chain.left_pieces; g.chain.valid = true;
             }
             break;
         }

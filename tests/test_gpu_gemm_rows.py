@@ -208,3 +208,48 @@ def test_a_captured_product_outlives_a_larger_one(dev):
         replays(graphs[g])
         HipNative.graphDestroy(graphs[g])
     dev.release(src, wq, xb, ob, big_x, big_w, big_o)
+
+
+@pytest.mark.parametrize("m,k,n,n2,norm", [(90, 768, 768, 3072, "layer"), (75, 1024, 1024, 2304, "rms"), (33, 2752, 1000, 2000, "rms"), (64, 1024, 772, 3000, "layer"),
+                                           (2, 768, 516, 2048, "rms"), (200, 1100, 768, 2304, "layer"), (65, 4096, 1028, 3001, "rms")])
+def test_a_product_that_shares_k_leaves_the_next_ones_pieces_without_changing_a_bit(dev, m, k, n, n2, norm):
+    """The sum of k_gemm_q8's shares also normalises and splits the rows for the product behind it: the bits of the two ops by
+    themselves, with a ragged batch, widths past a whole chunk, both norms; another gain in between and the second splits its own."""
+    rng = np.random.default_rng(m + n)
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)
+    assert HipNative.q8GemmRowsTile(m, n, n2, norm=True)[0] and not HipNative.q8GemmRowsTile(m, k, n)[0]
+
+    def q8(r, c):
+        src, dst = dev.upload(f(r, c) * np.float32(r ** -0.5)), dev.alloc(HipNative.q8Floats(r, c))
+        Stream().q8_quantize(src, dst, r, c, 0, 1, c).run()
+        return dst
+    w1, w2 = q8(k, n), q8(n, n2)
+    x, res, bias, gamma, beta = dev.upload(f(m, k)), dev.upload(f(m, n)), dev.upload(f(1, n)), dev.upload(1 + 0.1 * f(1, n)), dev.upload(0.1 * f(1, n))
+    mid, out = dev.alloc(m * n), dev.alloc(m * n2)
+    norms = dict(gamma=gamma, beta=beta) if norm == "layer" else dict(gamma=gamma)
+    first = Stream().q8_linear(x, w1, mid, m, k, n, bias=bias, residual=res)
+    second = Stream().q8_linear(mid, w2, out, m, n, n2, **norms)
+    first.run(), second.run()
+    want = dev.download(mid, (m, n)), dev.download(out, (m, n2))
+    both = Stream()
+    both.words = first.words + second.words
+    for _ in range(2):
+        Stream().fill(mid, 0, m * n).fill(out, 0, m * n2).run()
+        both.run()
+        assert np.array_equal(dev.download(mid, (m, n)), want[0]) and np.array_equal(dev.download(out, (m, n2)), want[1])
+    alone = [int(HipNative.profileOps(s.array(), 2, detail=True)[2][0]) for s in (first, second)]
+    together = [int(c) for c in HipNative.profileOps(both.array(), 2, detail=True)[2]]
+    if alone[0] > 1:                                              # (it shares its K here)
+        assert together == [alone[0], alone[1] - 1], (alone, together)
+    handle = HipNative.graphCapture(both.array())
+    for _ in range(3):
+        Stream().fill(mid, 0, m * n).fill(out, 0, m * n2).run()
+        HipNative.graphLaunch(handle)
+        assert np.array_equal(dev.download(out, (m, n2)), want[1])
+    HipNative.graphDestroy(handle)
+    other = Stream().q8_linear(mid, w2, out, m, n, n2, **dict(norms, gamma=bias))
+    both.words = first.words + Stream().fill(out, 0, m * n2).words + other.words
+    both.run()
+    apart = dev.download(out, (m, n2))
+    other.run()
+    assert np.array_equal(dev.download(out, (m, n2)), apart)
