@@ -237,7 +237,8 @@ enum {
      *     one token's attention over latent rows (J/.../MultiHeadLatentAttention.java:98-123): ckv is appended to the layer's
      *     rows of `latent` [layers][maxSeq][rank] at position state[0]; out [H * hd] = attention of q (not rotated) over
      *     K = RoPE(rows . Wuk) and V = rows . Wuv, wukv a Q8 weight with the 2 * H * hd output rows Wuk, Wuv.  records: scratch
-     *     of H * deepj_hip_latent_decode_splits(H, hd, rank, maxSeq) * (hd + 4) floats; refused where that is 0.
+     *     of H * deepj_hip_latent_decode_splits(H, hd, rank, maxSeq) * (hd + 4) floats (its contents are not defined); refused where
+     *     that is 0.
      * Q8_LINEAR_PAIR [op, x, gamma, K, weightA, outA, nA, weightB, outB, nB]
      *     two Q8_LINEARs of one row with the same x and RMSNorm gain in one launch, the same bits; K a multiple of 4 up to 4096
      */

@@ -667,6 +667,45 @@ def test_decode_attention_over_latent_rows_matches_the_expanded_one(H, hd, rank,
     assert float(np.max(np.abs(got - exp))) <= 1e-5 * max(1.0, float(np.max(np.abs(exp))))
 
 
+@pytest.mark.parametrize("H,hd,rank,max_seq", [(4, 32, 32, 40), (3, 64, 288, 70), (2, 128, 512, 100), (300, 32, 260, 40)])
+def test_latent_decode_keeps_to_its_own_scratch(H, hd, rank, max_seq):
+    """What an earlier operation left in the scratch (NaN) reaches no result, splits without keys included; the allocation-free
+    entry point gives the same bits; a position behind the last appends nothing and reads the rows there are."""
+    rng = np.random.default_rng(H + rank)
+    d = H * hd
+    q, ckv, rows = (rng.standard_normal(n).astype(np.float32) for n in (d, rank, max_seq * rank))
+    w = (rng.standard_normal((rank, 2 * d)) * rank ** -0.5).astype(np.float32)
+    cos, sin = ref.rope_tables(hd, max_seq)
+    dev = DeviceBuffers()
+    try:
+        src, wq = dev.upload(w), dev.alloc(HipNative.q8Floats(rank, 2 * d))
+        Stream().q8_quantize(src, wq, rank, 2 * d, 0, 1, 2 * d).run()
+        n = HipNative.latentDecodeSplits(H, hd, rank, max_seq)
+        rec, out, lat, state = dev.alloc(H * n * (hd + 4)), dev.alloc(d), dev.alloc(max_seq * rank), dev.alloc(4)
+        nan_x, nan_out, gamma = dev.upload(np.full(600 * rank, np.nan, np.float32)), dev.alloc(600 * 2 * d), dev.upload(np.ones(rank, np.float32))
+        s = Stream().latent_decode(dev.upload(q), dev.upload(ckv), lat, wq, state, dev.upload(cos), dev.upload(sin), rec, out, H, hd, rank, max_seq, 0)
+        poison = Stream().q8_linear(nan_x, wq, nan_out, 600, rank, 2 * d, gamma=gamma)
+
+        def run(pos, how, before=None):
+            dev.write(lat, rows)
+            dev.write(state, np.array([pos, 0, 0, 0], np.int32))
+            if before:
+                before.run()
+            how()
+            return dev.download(out, (d,)), dev.download(lat, (max_seq, rank))
+        for pos in (3, max_seq - 1, max_seq):
+            want, cache = run(pos, s.run)
+            assert np.isfinite(want).all()
+            expect = rows.reshape(max_seq, rank).copy()
+            if pos < max_seq:
+                expect[pos] = ckv
+            assert np.array_equal(cache, expect)
+            assert np.array_equal(run(pos, s.run, poison)[0], want)
+            assert np.array_equal(run(pos, lambda: HipNative.flushOpsNoAlloc(s.array(), s.array().size))[0], want)
+    finally:
+        dev.release_all()
+
+
 def test_latent_decode_refuses_what_it_does_not_take():
     for shape in ((4, 48, 64, 64), (4, 64, 6, 64), (4, 64, 516, 64), (0, 64, 64, 64), (4, 64, 64, 0)):
         assert HipNative.latentDecodeSplits(*shape) == 0
