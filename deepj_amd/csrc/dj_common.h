@@ -128,9 +128,11 @@ void launch_matmul_f32(hipStream_t s, const float *a, const float *b, float *out
 // kernels_q8.hip
 // Two consecutive products of a stream, the second normalising and multiplying the first one's output: where the first shares its
 // tiles' K among workgroups, the kernel that adds their partial products also leaves the second one's activations in its
-// layout, and the second skips its own split.  Two fp16 GEMMs (RMSNorm), or k_gemm_q8 in front of k_gemm_q8_rows.
+// layout, and the second skips its own split.  Two fp16 GEMMs (RMSNorm), or any of them in front of k_gemm_q8_rows.  And two
+// products with no normalisation between them, the first on k_gemm_q8_rows with a tile's K in one workgroup: its epilogue leaves
+// the second one's pieces.
 struct GemmChain {
-    const float *next_gamma = nullptr;   // to the first launch: the gain the next GEMM normalises this output with
+    const float *next_gamma = nullptr;   // to the first launch: the gain the next GEMM normalises this output with, null: with none
     bool left_planes = false;            // from the first launch: it left the next fp16 GEMM's activations in the workspace
     bool planes_ready = false;           // to the second launch: they are there
     uint16_t *next_pieces = nullptr;     // to the first launch: the next product takes k_gemm_q8_rows, with its rows' pieces there
@@ -165,7 +167,7 @@ void launch_q8_linear_pair(hipStream_t s, const Q8LinearPair &p);
 // pieces: a block for the products that multiply a batch of rows straight from the int8 weights; others are taken where it is
 // smaller than q8_linear_pieces_floats
 void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_t workspace_floats, float *pieces, int64_t pieces_floats);
-int64_t q8_linear_pieces_floats(int m, int k, int n, int flags, bool prepared);
+int64_t q8_linear_pieces_floats(int m, int k, int n, int flags, bool prepared, bool ready = false, bool *unshared = nullptr);
 int64_t q8_linear_workspace_floats(int m, int k, int n, int flags);
 // The size at which launch_q8_linear takes its fastest path (>= the one above); callers that may grow their workspace
 // offer this much, callers that may not offer what they have.

@@ -6,6 +6,8 @@
 
 namespace dj {
 
+struct GemmChain;
+
 // Where the bf16 pieces of activation (row, c) lie for v_mfma_f32_32x32x16_bf16: blocks of 1 KB, one per 32 rows, 32 k, half of
 // those k and piece; in a block 8 consecutive k for each lane.  Lane l of step s of a group holds row l % 32 and
 // k = 16 (l / 32) + 8 s + j, as the weights' side does (a lane's 16 k of a weight row are 16 consecutive bytes).  The high
@@ -65,10 +67,10 @@ void launch_q8_sum_partials(hipStream_t s, const float *partial, float *out, int
 // kernels_gemm_rows.hip
 void q8_gemm_rows_configure();   // once per device, before the first launch
 struct RowsPlan { int tmw, tnw, shares; double us; };      // a tile's rows and columns in units of 32, the workgroups that share its K
-// false: not a product for this kernel.  may_share: a tile's K among several workgroups
-bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared, bool may_share, RowsPlan *plan = nullptr);
+// false: not a product for this kernel.  may_share: a tile's K among several workgroups; ready: its rows' pieces are there
+bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared, bool may_share, RowsPlan *plan = nullptr, bool ready = false);
 int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, const RowsPlan &plan);
 void launch_q8_gemm_rows(hipStream_t s, const float *x, const float *gamma, const float *beta, const int8_t *wq, const float *scales, float *out, int m, int k,
-                         int n_rows, const GemmEpilogue &ep, const RowsPlan &plan, float *workspace, int64_t workspace_floats, bool pieces_ready);
+                         int n_rows, const GemmEpilogue &ep, const RowsPlan &plan, float *workspace, int64_t workspace_floats, GemmChain *chain);
 
 }  // namespace dj

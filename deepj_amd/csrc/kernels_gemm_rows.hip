@@ -14,6 +14,9 @@
 // loads return in the order they were asked for, so waiting for activations that were asked for after a chunk is waiting for
 // the chunk.  The matrix cores' 32 cycles a product hide the group before's scaling and the next one's conversion.
 //
+// Where the next product takes this one's output as it is (a feed-forward layer's hidden rows), its pieces come out of this
+// epilogue (GemmRowsArgs::next), not out of a launch of their own; when that is worth it: rows_plan.
+//
 // What bounds it: up to 32 rows the weights' bytes (30 x 22016 over 4096: 94 MB in 34 us with the rows' normalisation and split, 42
 // where they come from HBM, 87 and 90 on k_gemm_q8), then the activations, which every tile reads anew from L2 (12 KB for every
 // 64 x 64 x 32: 64 x 22016 48 us, 53 from HBM, 86 and 92; 200 x 11264 over 2048 49 and 52, 66 and 67), and on small weights two
@@ -57,6 +60,8 @@ struct GemmRowsArgs {
     GemmEpilogue ep;
     int share_chunks;           // > 0: gridDim.z workgroups share a tile's K, this many chunks each
     float *partial;             // [gridDim.z][m][n] when they do
+    uint16_t *next;             // not null: where the next product takes this one's output as its rows, in operand order
+    int next_groups;            // ... their scale groups, padded to whole chunks
 };
 
 // four int8 of a word as bf16, exactly
@@ -262,13 +267,43 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             if (ep.swiglu) {
                 // (gate, up) pairs in neighbouring lanes (SiLU.java:20-24, SwiGLULayer.java:69)
                 const float other = __shfl_xor(v, 1, 64);
-                if (live && (col & 1) == 0) a.out[(int64_t)row * (a.n >> 1) + (col >> 1)] = v * (1.0f / (1.0f + expf(-v))) * other;
-                continue;
+                v = v * (1.0f / (1.0f + expf(-v))) * other;
+                if (live && (col & 1) == 0) a.out[(int64_t)row * (a.n >> 1) + (col >> 1)] = v;
+            } else if (live) {
+                if (ep.gelu) v = gemm_gelu(v);
+                if (ep.residual) v = ep.residual[(int64_t)row * a.n + col] + v;
+                a.out[(int64_t)row * a.n + col] = v;
             }
-            if (!live) continue;
-            if (ep.gelu) v = gemm_gelu(v);
-            if (ep.residual) v = ep.residual[(int64_t)row * a.n + col] + v;
-            a.out[(int64_t)row * a.n + col] = v;
+            s.w = v;                                   // (after four rows s holds the results)
+        }
+        if (a.next) red[q * 64 + lane] = s;            // (only this wavefront reads the place in the first wavefront's sums)
+    }
+    if (!a.next) return;
+    // The tile's results as the next product's rows: two columns of a row a thread at a time (a loop of few instructions: a
+    // launch fetches them anew).  What the tile has no result for - rows up to a multiple of 32, columns up to a whole chunk -
+    // is zero.
+    __syncthreads();
+    constexpr int R = 32 * TMW;
+    const int out_shift = ep.swiglu ? 1 : 0, n_out = a.n >> out_shift, c0 = n0 >> out_shift;
+    const int columns = n_tile == a.n_tiles - 1 ? a.next_groups * kQ8Group - c0 : TN >> out_shift;
+#pragma unroll 1
+    for (int i = t; i < R * columns / 2; i += 64 * kWaves) {
+        const int r32 = (i >> 2) % R, row = m0 + r32, at = i / (4 * R) * 8 + (i & 3) * 2, c = c0 + at;
+        if (row >= row_tiles * 32) continue;
+        const float *of_row = reinterpret_cast<const float *>(lds) + (((r32 >> 5) * TNW * 4 + ((r32 & 31) >> 3)) * 64 + ((r32 >> 2) & 1) * 32) * 4 + (r32 & 3);
+        float v[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int local = (at + e) << out_shift;
+            const float u = of_row[local < TN ? ((local >> 5) * 256 + (local & 31)) * 4 : 0];
+            v[e] = row < a.m && c + e < n_out && local < TN ? (operand_negated(c) ? -u : u) : 0.0f;
+        }
+        uint32_t *dst = reinterpret_cast<uint32_t *>(a.next + operand_at(row, c, a.next_groups));
+#pragma unroll
+        for (int p = 0; p < kOperandPieces; p++) {
+            const uint32_t w0 = __float_as_uint(v[0]) & 0xffff0000u, w1 = __float_as_uint(v[1]) & 0xffff0000u;
+            dst[p * (kOperandPiece / 2)] = (w0 >> 16) | w1;
+            v[0] -= __uint_as_float(w0); v[1] -= __uint_as_float(w1);
         }
     }
 }
@@ -295,7 +330,12 @@ int chunks_of(int k) { return (q8_padded_k(k) / kQ8Group + kChunk - 1) / kChunk;
 // No tile whose outputs would be worse than k_gemm_q8's: an output is `sums` sums of groups / sums terms each, and the squared error
 // against 64 bits, in units of 1e-14 of the result's squared rms, was 0.55 + 0.031 a term here (768 to 11008 k, every tile) and 1.07 +
 // 0.025 a term there.
-RowsPlan rows_plan(int m, int n_rows, int k, bool may_share, int sums_there) {
+//
+// ready: the product in front leaves the rows' pieces, which saves a launch and its pass over the rows and costs that product's
+// end up to 3 us a million values (64 x 11008 2.5, 400 x 3072 3.0).  Measured on that product and this one together, us: 64 x
+// 4096 over 11008 80.9 -> 76.2, 30 x 4096 over 11008 60.7 -> 54.7, 30 x 2048 over 5632 32.3 -> 28.5, 16 x 256 over 688 15.8 ->
+// 14.9; where k_gemm_q8 keeps the second one: 300 x 1024 over 2752 41.3, 43.2 with pieces, 400 x 768 over 3072 39.4, 42.7.
+RowsPlan rows_plan(int m, int n_rows, int k, bool may_share, int sums_there, bool ready) {
     struct Shape { int tmw, tnw, shares; GemmCost cost; };
     static constexpr Shape shapes[] = {
         {1, 1, 1, {5.65, 0.2, 2.52, 2.03, 0.3, 0.0, 7.0, 0.075}},  {1, 2, 1, {6.46, 0.83, 3.59, 3.04, 0.0, 0.0, 6.5, 0.08}},
@@ -315,7 +355,8 @@ RowsPlan rows_plan(int m, int n_rows, int k, bool may_share, int sums_there) {
         const int fit = h.tnw > 2 ? 1 : 2;
         const double rounds = x <= 2 * fit ? ceil(x) : fit * ceil(x / fit);
         const double kk = (((chunks + kWaves - 1) / kWaves + h.shares - 1) / h.shares) * kWaves * kChunk * kQ8Group * 1e-3;
-        const double us = h.cost.us(x, rounds, kk, 1.0, m, n_rows, k, h.shares);
+        double us = h.cost.us(x, rounds, kk, 1.0, m, n_rows, k, h.shares);
+        if (ready) us -= 2.5 + (h.cost.rows - 3.0) * m * k * 1e-6;
         if (!best.tmw || us < best.us) best = {h.tmw, h.tnw, h.shares, us};
     }
     return best;
@@ -335,30 +376,33 @@ void q8_gemm_rows_configure() {
 // is none (30 x 6144 over 2048 12.1, 16.0, but 8 x 768 over 256 6.7, 6.2 and 128 x 768 over 3072 15.0, 12.1).  Up to 768 rows: long
 // batches belong to k_gemm_q8's larger tiles (1500 x 50257 over 768 655 us, 504; 2048 rows 1058, 647; 1500 x 8001 over 1500 233, 158).  A
 // lane's offset into a column tile's weights is 32 bits.
-bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared, bool may_share, RowsPlan *plan) {
+bool q8_gemm_rows_ok(int m, int n_rows, int k, bool norm, bool prepared, bool may_share, RowsPlan *plan, bool ready) {
     if (m > 768 || k > (1 << 24) || q8_gemm_f16_forced() == 0 || q8_gemm_f16_shape_ok(m, n_rows, k, prepared)) return false;
     const Q8GemmEstimate there = q8_gemm_estimate(m, n_rows, k, norm, may_share);
-    const RowsPlan p = rows_plan(m, n_rows, k, may_share, there.sums);
+    const RowsPlan p = rows_plan(m, n_rows, k, may_share, there.sums, ready);
     if (plan) *plan = p;
-    return p.tmw && p.us < 0.98 * there.us - 0.2;
+    return p.tmw && (ready ? p.us < 1.01 * there.us : p.us < 0.98 * there.us - 0.2);
 }
 
+int64_t operand_floats(int m, int k) { return round_up(m, 32) * round_up(q8_padded_k(k), kOperandChunk) / 2 * kOperandPieces; }
 // floats of workspace: the activations' pieces, the partial products where K is shared
-int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, const RowsPlan &p) {
-    const int64_t m_pad = round_up(m, 32), ka = round_up(q8_padded_k(k), kOperandChunk);
-    return m_pad * ka / 2 * kOperandPieces + (p.shares > 1 ? (int64_t)p.shares * m * n_rows : 0);
-}
+int64_t q8_gemm_rows_workspace_floats(int m, int n_rows, int k, const RowsPlan &p) { return operand_floats(m, k) + (p.shares > 1 ? (int64_t)p.shares * m * n_rows : 0); }
 
 void launch_q8_gemm_rows(hipStream_t s, const float *x, const float *gamma, const float *beta, const int8_t *wq, const float *scales, float *out, int m, int k,
-                         int n_rows, const GemmEpilogue &ep, const RowsPlan &p, float *workspace, int64_t workspace_floats, bool pieces_ready) {
+                         int n_rows, const GemmEpilogue &ep, const RowsPlan &p, float *workspace, int64_t workspace_floats, GemmChain *chain) {
     if (workspace_floats < q8_gemm_rows_workspace_floats(m, n_rows, k, p)) fail("q8_gemm_rows: workspace too small");
     if (ep.swiglu && ((n_rows & 1) || ep.residual || ep.gelu)) fail("q8_gemm_rows: the SwiGLU epilogue needs an even row count and takes no residual or GELU");
-    const int kp = q8_padded_k(k), ka = (int)round_up(kp, kOperandChunk), m_pad = (int)round_up(m, 32);
+    const int kp = q8_padded_k(k), ka = (int)round_up(kp, kOperandChunk), m_pad = (int)round_up(m, 32), n_out = ep.swiglu ? n_rows / 2 : n_rows;
     const int m_tiles = (m + 32 * p.tmw - 1) / (32 * p.tmw), n_tiles = (n_rows + 32 * p.tnw - 1) / (32 * p.tnw);
-    float *w = workspace;
-    uint16_t *planes = reinterpret_cast<uint16_t *>(w); w += (int64_t)m_pad * ka / 2 * kOperandPieces;
-    if (!pieces_ready) launch_split_operand(s, x, gamma, beta, planes, m, m_pad, k, ka);      // (the product in front has left them: GemmChain)
-    GemmRowsArgs a{reinterpret_cast<const uintx4 *>(planes), wq, scales, out, m, n_rows, kp / kQ8Group, m_tiles, n_tiles, ep, 0, nullptr};
+    uint16_t *planes = reinterpret_cast<uint16_t *>(workspace);
+    float *w = workspace + operand_floats(m, k);
+    if (!(chain && chain->pieces_ready)) launch_split_operand(s, x, gamma, beta, planes, m, m_pad, k, ka);      // (the product in front has left them: GemmChain)
+    GemmRowsArgs a{reinterpret_cast<const uintx4 *>(planes), wq, scales, out, m, n_rows, kp / kQ8Group, m_tiles, n_tiles, ep, 0, nullptr, nullptr, 0};
+    if (p.shares == 1 && chain && chain->next_pieces && !chain->next_gamma) {
+        a.next = chain->next_pieces;
+        a.next_groups = (int)round_up(q8_padded_k(n_out), kOperandChunk) / kQ8Group;
+        chain->left_pieces = true;
+    }
     dim3 grid((unsigned)((n_tiles + 7) / 8 * 8 * m_tiles));
     if (p.shares > 1) {
         a.share_chunks = (chunks_of(k) + p.shares - 1) / p.shares;
@@ -368,7 +412,16 @@ void launch_q8_gemm_rows(hipStream_t s, const float *x, const float *gamma, cons
     each_kernel([&](auto kernel, int tmw, int tnw) {
         if (tmw == p.tmw && tnw == p.tnw) launch_kernel(kernel, grid, dim3(64 * kWaves), (size_t)lds_bytes(tmw, tnw), s, a);
     });
-    if (p.shares > 1) launch_q8_sum_partials(s, w, out, (int)grid.z, m, n_rows, ep);
+    if (p.shares == 1) return;
+    // (the next product's pieces may take the place of this one's, not of the partial products)
+    const float *next = chain ? reinterpret_cast<const float *>(chain->next_pieces) : nullptr;
+    if (next && chain->next_gamma && !ep.gelu && !ep.swiglu && !ep.interleaved_bias && split_operand_sum_ok(n_rows) &&
+        (next + operand_floats(m, n_rows) <= w || next >= w + (int64_t)p.shares * m * n_rows)) {
+        launch_split_operand_sum(s, w, (int)grid.z, ep.bias, ep.residual, out, chain->next_gamma, chain->next_beta, chain->next_pieces, m, n_rows);
+        chain->left_pieces = true;
+        return;
+    }
+    launch_q8_sum_partials(s, w, out, (int)grid.z, m, n_rows, ep);
 }
 
 }  // namespace dj

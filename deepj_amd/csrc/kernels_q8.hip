@@ -696,10 +696,11 @@ int64_t q8_linear_preferred_workspace_floats(int m, int k, int n, int flags, boo
     return ws;
 }
 
-int64_t q8_linear_pieces_floats(int m, int k, int n, int flags, bool prepared) {
+int64_t q8_linear_pieces_floats(int m, int k, int n, int flags, bool prepared, bool ready, bool *unshared) {
     const int n_rows = (flags & DJ_LIN_SWIGLU) ? 2 * n : n;
     RowsPlan plan;
-    if ((m == 1 && matvec_supported(k)) || !q8_gemm_rows_ok(m, n_rows, k, (flags & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM)) != 0, prepared, true, &plan)) return 0;
+    if ((m == 1 && matvec_supported(k)) || !q8_gemm_rows_ok(m, n_rows, k, (flags & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM)) != 0, prepared, true, &plan, ready)) return 0;
+    if (unshared) *unshared = plan.shares == 1;
     return q8_gemm_rows_workspace_floats(m, n_rows, k, plan);
 }
 
@@ -779,11 +780,11 @@ void launch_q8_linear(hipStream_t s, const Q8Linear &p, float *workspace, int64_
     // the weights exist, and without sharing K: one rule for the allocation-free entry point.
     const bool may_share = !p.small_workspace_only;
     RowsPlan plan;
-    if (!p.m_dev && !rope && !(p.chain && p.chain->planes_ready) && q8_gemm_rows_ok(p.m, n_rows, p.k, gamma != nullptr, p.prepared && may_share, may_share, &plan) &&
+    if (!p.m_dev && !rope && !(p.chain && p.chain->planes_ready) && q8_gemm_rows_ok(p.m, n_rows, p.k, gamma != nullptr, p.prepared && may_share, may_share, &plan,
+                                                                                            p.chain && p.chain->pieces_ready && !gamma) &&
         pieces_floats >= q8_gemm_rows_workspace_floats(p.m, n_rows, p.k, plan)) {
         const GemmEpilogue ep{bias, swiglu ? bias2 : nullptr, residual, swiglu, nullptr, 0, swiglu ? 0 : gelu, swiglu, RopeStore{}};
-        launch_q8_gemm_rows(s, p.x, gamma, beta, p.wq, p.scales, p.out, p.m, p.k, n_rows, ep, plan, pieces, pieces_floats,
-                            p.chain && p.chain->pieces_ready);
+        launch_q8_gemm_rows(s, p.x, gamma, beta, p.wq, p.scales, p.out, p.m, p.k, n_rows, ep, plan, pieces, pieces_floats, p.chain);
         return;
     }
     if (!p.m_dev && !p.small_workspace_only && q8_gemm_f16_shape_ok(p.m, n_rows, p.k, p.prepared != nullptr) && workspace_floats >= q8_gemm_f16_workspace_floats(p.m, n_rows, p.k, p.prepared != nullptr)) {

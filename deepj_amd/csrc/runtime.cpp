@@ -101,7 +101,7 @@ struct Runtime {
     unsigned char *static_scratch = nullptr;       // device address of `scratch` below on g.device
     // Set by a K-sharing fp16 GEMM that also wrote the activations of the op right behind it in that op's layout
     // (GemmChain): which op of which stream, reading which buffer through which gain.  Good for that one op only.
-    struct ChainSlot { const int32_t *cmd = nullptr; int32_t pos = -1, x_id = -1, gamma_id = -1, beta_id = -1; int64_t m = 0, k = 0; bool pieces = false, valid = false; } chain;
+    struct ChainSlot { const int32_t *cmd = nullptr; int32_t pos = -1, x_id = -1, gamma_id = -1, beta_id = -1; int64_t m = 0, k = 0, pieces_at = 0; bool pieces = false, plain = false, valid = false; } chain;
     bool no_alloc = false;                         // inside deepj_hip_flush_ops_noalloc: nothing may allocate
     std::vector<std::pair<int32_t, void *>> *track = nullptr;   // graph capture: buffers the dry pass resolves
     Graph *capture_into = nullptr;                               // graph capture: the graph the run pass records for
@@ -776,8 +776,9 @@ void exec_one(Cursor &c) {
     // the same for the rows' pieces that a product leaves to k_gemm_q8_rows
     auto pieces_left = [&](int64_t m, int64_t k) {
         const int flags = w[7];
-        return run && was.valid && was.pieces && was.cmd == c.cmd && was.pos == c.pos && was.x_id == w[1] && was.gamma_id == w[8] && was.m == m && was.k == k &&
-               (flags & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM)) && was.beta_id == (flags & DJ_LIN_LAYERNORM ? w[10] : -1);
+        return run && was.valid && was.pieces && was.cmd == c.cmd && was.pos == c.pos && was.x_id == w[1] && was.m == m && was.k == k &&
+               (was.plain ? !(flags & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM))
+                          : (flags & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM)) && was.gamma_id == w[8] && was.beta_id == (flags & DJ_LIN_LAYERNORM ? w[10] : -1));
     };
     if (run && !c.alone && op < DJ_OP_Q8_QUANTIZE && exec_chain(c)) return;
     switch (op) {
@@ -999,19 +1000,40 @@ void exec_one(Cursor &c) {
             }
             int64_t ws = g.no_alloc ? q8_linear_workspace_floats((int)m, (int)k, (int)n, flags)
                                     : q8_linear_preferred_workspace_floats((int)m, (int)k, (int)n, flags, p.prepared != nullptr);
-            need_scratch(c, ws, g.no_alloc ? 0 : q8_linear_pieces_floats((int)m, (int)k, (int)n, flags, p.prepared != nullptr));
+            bool unshared = false;
+            const int64_t own_pieces = g.no_alloc ? 0 : q8_linear_pieces_floats((int)m, (int)k, (int)n, flags, p.prepared != nullptr, false, &unshared);
+            // The op right behind this one multiplies this output as it is: where both are products for k_gemm_q8_rows, this one's
+            // epilogue leaves that one's pieces behind its own.
+            const int32_t *behind = c.pos + stride_of(op) + 12 <= c.len ? c.cmd + c.pos + stride_of(op) : nullptr;
+            const auto prepared_as = [&](int32_t weight, int64_t wk, int64_t wrows) {
+                auto it = g.prepared.find(weight);
+                return it != g.prepared.end() && it->second.k == wk && it->second.rows == wrows;
+            };
+            const auto rows_of = [](const int32_t *nw) { return (nw[7] & DJ_LIN_SWIGLU) ? 2 * (int64_t)nw[6] : (int64_t)nw[6]; };
+            const int64_t behind_own = (own_pieces + 63) / 64 * 64;
+            int64_t plain_pieces = 0;
+            if (m > 1 && own_pieces > 0 && unshared && behind && behind[0] == DJ_OP_Q8_LINEAR && behind[1] == w[3] && behind[4] == m && behind[5] == n && behind[6] > 0 &&
+                behind[6] < (1 << 30) && !(behind[7] & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM | DJ_LIN_ATTN_MERGE)))
+                plain_pieces = q8_linear_pieces_floats((int)m, (int)n, behind[6], behind[7], prepared_as(behind[2], n, rows_of(behind)), true);
+            need_scratch(c, ws, plain_pieces > 0 ? behind_own + plain_pieces : own_pieces);
             // One rule for the allocation-free entry point, whatever happens to fit its fixed array: the many-row
             // fp16 GEMM (whose operands live in a workspace sized by the shape) is never taken there.
             p.small_workspace_only = g.no_alloc;
             GemmChain chain;
             int32_t next_gamma_id = -1, next_beta_id = -1;
+            int64_t pieces_at = 0, next_at = 0;
             const int32_t next_pos = c.pos + stride_of(op);
             if (run && m > 1 && !g.no_alloc && !merge) {
                 chain.planes_ready = chained(w[1], w[8], flags, m, k);
                 chain.pieces_ready = pieces_left(m, k);
+                if (chain.pieces_ready) pieces_at = was.pieces_at;
+                if (plain_pieces > 0 && pieces_at + behind_own + plain_pieces <= g.row_pieces_floats) {
+                    next_at = pieces_at + behind_own;
+                    chain.next_pieces = reinterpret_cast<uint16_t *>(g.row_pieces + next_at);
+                }
                 // the op right behind this one normalises this output (RMSNorm) and multiplies it on the fp16 GEMM: the
                 // launch may leave that op's activations ready (it does when this one shares its tiles' K)
-                if (next_pos < c.len && !sw) {
+                if (next_pos < c.len && !sw && !chain.next_pieces) {
                     const int32_t *nw = c.cmd + next_pos;
                     const bool n_rope = nw[0] == DJ_OP_Q8_LINEAR_ROPE;
                     if ((nw[0] == DJ_OP_Q8_LINEAR || n_rope) && nw[1] == w[3] && nw[4] == m && nw[5] == n && (nw[7] & DJ_LIN_RMSNORM) &&
@@ -1026,10 +1048,7 @@ void exec_one(Cursor &c) {
                     const int norms = DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM;
                     if (!chain.next_gamma && g.row_pieces && next_pos + 12 <= c.len && nw[0] == DJ_OP_Q8_LINEAR && nw[1] == w[3] && nw[4] == m && nw[5] == n &&
                         nw[6] > 0 && nw[6] < (1 << 30) && (nw[7] & norms) && !(nw[7] & DJ_LIN_ATTN_MERGE)) {
-                        const int64_t n_rows = (nw[7] & DJ_LIN_SWIGLU) ? 2 * (int64_t)nw[6] : (int64_t)nw[6];
-                        auto it = g.prepared.find(nw[2]);
-                        const bool prepared = it != g.prepared.end() && it->second.k == n && it->second.rows == n_rows;
-                        const int64_t pieces = q8_linear_pieces_floats((int)m, (int)n, nw[6], nw[7], prepared);
+                        const int64_t pieces = q8_linear_pieces_floats((int)m, (int)n, nw[6], nw[7], prepared_as(nw[2], n, rows_of(nw)));
                         if (pieces > 0 && pieces <= g.row_pieces_floats) {
                             next_gamma_id = nw[8];
                             chain.next_gamma = buf(next_gamma_id, n, op, "the next op's gamma");
@@ -1040,8 +1059,9 @@ void exec_one(Cursor &c) {
                 }
                 p.chain = &chain;
             }
-            if (run) launch_q8_linear(s, p, g.workspace, g.workspace_floats, g.row_pieces, g.row_pieces_floats);
+            if (run) launch_q8_linear(s, p, g.workspace, g.workspace_floats, g.row_pieces + pieces_at, g.row_pieces_floats - pieces_at);
             if (chain.left_planes || chain.left_pieces) {
+                g.chain.pieces_at = next_at; g.chain.plain = chain.left_pieces && !chain.next_gamma;
                 g.chain.cmd = c.cmd; g.chain.pos = next_pos; g.chain.x_id = w[3]; g.chain.gamma_id = next_gamma_id; g.chain.beta_id = next_beta_id;
                 g.chain.m = m; g.chain.k = n; g.chain.pieces = chain.left_pieces; g.chain.valid = true;
             }

@@ -253,3 +253,57 @@ def test_a_product_that_shares_k_leaves_the_next_ones_pieces_without_changing_a_
     apart = dev.download(out, (m, n2))
     other.run()
     assert np.array_equal(dev.download(out, (m, n2)), apart)
+
+
+@pytest.mark.parametrize("m,d,dff,gated", [(64, 2048, 5632, True), (30, 2048, 5632, True), (90, 768, 3072, False), (75, 1024, 2752, True), (16, 256, 688, True),
+                                           (33, 512, 1001, False), (2, 768, 2050, True), (65, 512, 1100, True), (40, 768, 1003, True), (200, 1024, 4104, False)])
+def test_a_feed_forward_layer_hands_its_hidden_rows_on_in_pieces(dev, m, d, dff, gated):
+    """The hidden rows' product leaves them for the one behind it in operand order: both outputs against float64, the first one's bits
+    as by itself, in a captured graph too; ragged batches and widths (rows up to a multiple of 32 and columns up to a whole
+    chunk are zeros there, whatever the memory held), and the layer's next product, which takes its pieces from a third place."""
+    rng = np.random.default_rng(m + dff)
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)
+
+    def q8(*parts):
+        dst, r, c = dev.alloc(HipNative.q8Floats(parts[0].shape[0], parts[0].shape[1] * len(parts))), *parts[0].shape
+        for i, p in enumerate(parts):
+            src = dev.upload(p)
+            Stream().q8_quantize(src, dst, r, c, i, len(parts), c * len(parts)).run()
+            dev.release(src)
+        return dst
+    ups = [f(d, dff) * np.float32(d ** -0.5) for _ in range(2 if gated else 1)]
+    wd, wq = f(dff, d) * np.float32(dff ** -0.5), f(d, 3 * d) * np.float32(d ** -0.5)
+    x, gamma, bias = f(m, d), 1 + 0.1 * f(d), 0.1 * f(dff)
+    w1, w2, w3 = q8(*ups), q8(wd), q8(wq)
+    xb, gb, bb = dev.upload(x), dev.upload(gamma), dev.upload(bias)
+    hidden, out, last = dev.alloc(m * dff), dev.alloc(m * d), dev.alloc(m * 3 * d)
+    tiles = HipNative.q8GemmRowsTile(m, d, len(ups) * dff, norm=True)
+    assert tiles[0]
+    first = Stream().q8_linear(xb, w1, hidden, m, d, dff, gamma=gb, bias=bb, bias2=bb if gated else -1, swiglu=gated, gelu=not gated)
+    second = Stream().q8_linear(hidden, w2, out, m, dff, d, residual=xb)
+    third = Stream().q8_linear(out, w3, last, m, d, 3 * d, gamma=gb)
+    first.run()
+    hidden_alone = dev.download(hidden, (m, dff))
+    layer = Stream()
+    layer.words = first.words + second.words + third.words
+    poison, poison_out = dev.upload(np.full((700, dff), np.nan, np.float32)), dev.alloc(700 * d)
+
+    def results():
+        return dev.download(hidden, (m, dff)), dev.download(out, (m, d)), dev.download(last, (m, 3 * d))
+    layer.run()                                                   # (sizes the scratch)
+    Stream().q8_linear(poison, w2, poison_out, 700, dff, d).run()
+    Stream().fill(hidden, 0, m * dff).fill(out, 0, m * d).fill(last, 0, m * 3 * d).run()
+    Stream().fill(poison, 0, 700 * dff).fill(poison_out, 0, 700 * d).run()       # (a later buffer may get the memory)
+    layer.run()
+    got = results()
+    assert np.array_equal(got[0], hidden_alone)
+    deq = lambda w: ref.q8_roundtrip(w).astype(np.float64)
+    check(got[1], got[0].astype(np.float64) @ deq(wd) + x, dff, f"{m} x {d} over {dff}")
+    check(got[2], rms_normalised(got[1].astype(np.float64), gamma) @ deq(wq), d, f"{m} x {3 * d} over {d}", times=2)      # (and the normalisation's roundings)
+    graph = HipNative.graphCapture(layer.array())
+    for _ in range(3):
+        Stream().fill(hidden, 0, m * dff).fill(out, 0, m * d).fill(last, 0, m * 3 * d).run()
+        HipNative.graphLaunch(graph)
+        assert all(np.array_equal(a, b) for a, b in zip(results(), got))
+    HipNative.graphDestroy(graph)
+    dev.release(w1, w2, w3, xb, gb, bb, hidden, out, last, poison, poison_out)

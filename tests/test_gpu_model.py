@@ -702,6 +702,7 @@ def test_latent_decode_keeps_to_its_own_scratch(H, hd, rank, max_seq):
             assert np.array_equal(cache, expect)
             assert np.array_equal(run(pos, s.run, poison)[0], want)
             assert np.array_equal(run(pos, lambda: HipNative.flushOpsNoAlloc(s.array(), s.array().size))[0], want)
+        Stream().fill(nan_x, 0, 600 * rank).fill(nan_out, 0, 600 * 2 * d).run()      # (a later buffer may get the memory)
     finally:
         dev.release_all()
 
