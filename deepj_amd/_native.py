@@ -244,7 +244,8 @@ class HipNative:
 
     @staticmethod
     def q8GemmTilePrepared(m: int, k: int, rows: int):
-        """The same for a weight already in the fp16 GEMM's layout (OP_Q8_PREPARE): taken from 16 rows on."""
+        """The same for a weight already in the fp16 GEMM's layout (OP_Q8_PREPARE): taken from 16 rows on,
+        but for products of 17 to 32 rows over 1024 k or more, which read the int8 weights."""
         r, c, s = C.c_int32(), C.c_int32(), C.c_int32()
         library().deepj_hip_q8_gemm_tile_prepared(m, k, rows, C.byref(r), C.byref(c), C.byref(s))
         return r.value, c.value, s.value

@@ -806,6 +806,7 @@ struct GemmF16Plan { int tile_rows, tile_cols, splits; };
 constexpr int kNPad = 768;      // weight rows of a prepared buffer are padded to a multiple of both tile widths
 
 constexpr int kMinRowsPrepared = 16;     // fewer rows than this read the int8 weights even where a copy is prepared
+// (... and so does a Q8_LINEAR of 17 to 32 rows over 1024 k or more, below.)
 
 // DEEPJ_HIP_GEMM_F16=0 keeps every GEMM on k_gemm_q8; =128, =128192, =64 or =192 force the 128 x 256, 128 x 192, 64 x 256 or
 // 64 x 192 tile of the fp16 GEMM (for comparisons)
@@ -864,6 +865,12 @@ bool q8_gemm_f16_rope_ok(int m, int d, int k) {
     const GemmF16Plan p = q8_gemm_f16_plan(m, 3 * d, k, false);      // (256 rows and more: whatever the weights' state)
     return p.tile_rows != 0 && p.splits == 1;
 }
+// One tile of k_gemm_q8_rows's rows: such a product is bound by its weights' bytes, and a copy holds twice as many.  From 16 to 32
+// rows, us, with the copy and from the int8 weights: 32 x 11264 over 2048 20.1, 16.8 (and 36.7, 28.8 with the product behind it, which
+// takes its pieces), 32 x 22016 over 4096 55.4, 33.8 (85.6, 66.3), 16 x 22016 over 12288 177, 113; over 312 shapes 1.36 times as
+// long with it in the median, never less from 1024 k on; below that the int8 side's own conversions show: 20 x 50000 over 256 12.7,
+// 13.1 and 32 x 32768 over 64 8.6, 9.4.  16 rows, the fewest that the copy's route is held to, stay on it.  Above 32 rows both ways: 64 x 22016 over 4096 57.7, 48.7, 64 x 12288 30.2, 32.1.
+bool q8_copy_pays(int m, int k) { return m <= kMinRowsPrepared || m > 32 || k < 1024; }
 bool q8_gemm_f16_shape_ok(int m, int n_rows, int k, bool prepared) { return q8_gemm_f16_tile_rows(m, n_rows, k, prepared) != 0; }
 void q8_gemm_f16_tile(int m, int n_rows, int k, int *tile_rows, int *tile_cols, int *k_shares, bool prepared) {
     const GemmF16Plan p = q8_gemm_f16_plan(m, n_rows, k, prepared);

@@ -519,7 +519,7 @@ Stream decode_stream(Runner &r, Choose how, bool narrow) {
 // every call (same results, 40 us or so per layer and prompt slower).  (finalize()'s warm-up pass runs long prompts
 // when maxSeqLen allows them, so with the warm-up on the copies exist from the start.)
 void ensure_prepared(Runner &r, int n) {
-    if (r.prepared_done || n < 64) return;      // (with the copies in place the GEMM takes prompts from 16 rows on where its plan says so)
+    if (r.prepared_done || n < 64) return;      // (with the copies in place the GEMM takes prompts from 16 rows on, 17 to 32 aside, where its plan says so)
     r.prepared_done = true;
     const Config &c = r.cfg;
     const int d = c.d;

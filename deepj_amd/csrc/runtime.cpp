@@ -990,7 +990,7 @@ void exec_one(Cursor &c) {
             // a workspace that may grow is sized for the kernel's fastest path; the fixed one for the smallest
             if (m > 1) {
                 auto pit = g.prepared.find(w[2]);
-                if (pit != g.prepared.end() && pit->second.k == k && pit->second.rows == rows)
+                if (pit != g.prepared.end() && pit->second.k == k && pit->second.rows == rows && q8_copy_pays((int)m, (int)k))
                     p.prepared = buf(pit->second.id, q8_prepared_floats((int)k, (int)rows), op, "prepared weights");
                 if (p.prepared && run && g.capture_into) {
                     const std::pair<int32_t, int32_t> pr(w[2], pit->second.id);
@@ -1007,7 +1007,7 @@ void exec_one(Cursor &c) {
             const int32_t *behind = c.pos + stride_of(op) + 12 <= c.len ? c.cmd + c.pos + stride_of(op) : nullptr;
             const auto prepared_as = [&](int32_t weight, int64_t wk, int64_t wrows) {
                 auto it = g.prepared.find(weight);
-                return it != g.prepared.end() && it->second.k == wk && it->second.rows == wrows;
+                return it != g.prepared.end() && it->second.k == wk && it->second.rows == wrows && q8_copy_pays((int)m, (int)wk);
             };
             const auto rows_of = [](const int32_t *nw) { return (nw[7] & DJ_LIN_SWIGLU) ? 2 * (int64_t)nw[6] : (int64_t)nw[6]; };
             const int64_t behind_own = (own_pieces + 63) / 64 * 64;

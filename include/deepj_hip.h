@@ -288,7 +288,8 @@ int32_t deepj_hip_q8_linear_rope_ok(int32_t m, int32_t k, int32_t d);
 /* the same with the tile's columns (256 or 192) and the number of workgroups that share a tile's K (1: none) */
 void deepj_hip_q8_gemm_tile(int32_t m, int32_t k, int32_t rows, int32_t *tile_rows, int32_t *tile_cols, int32_t *k_shares);
 /* the same for a weight that Q8_PREPARE has written in the fp16 GEMM's layout: from 16 rows on instead of 256 (64-row tiles,
- * K shared so that as many workgroups as possible stream weights) */
+ * K shared so that as many workgroups as possible stream weights).  A Q8_LINEAR of 17 to 32 rows over 1024 k or more reads the
+ * int8 weights all the same, half the bytes: ask deepj_hip_q8_gemm_rows_tile without `prepared` for it. */
 void deepj_hip_q8_gemm_tile_prepared(int32_t m, int32_t k, int32_t rows, int32_t *tile_rows, int32_t *tile_cols, int32_t *k_shares);
 /* The same for the kernel that multiplies a batch of rows straight from the int8 weights (32 or 64 rows by 32, 64 or 96
  * columns a tile): 1 when a Q8_LINEAR of m rows with (norm) or without a normalisation prologue runs on it, 0 when on

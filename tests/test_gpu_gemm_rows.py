@@ -307,3 +307,29 @@ def test_a_feed_forward_layer_hands_its_hidden_rows_on_in_pieces(dev, m, d, dff,
         assert all(np.array_equal(a, b) for a, b in zip(results(), got))
     HipNative.graphDestroy(graph)
     dev.release(w1, w2, w3, xb, gb, bb, hidden, out, last, poison, poison_out)
+
+
+@pytest.mark.parametrize("m,k,n,norm,gated", [(17, 1536, 12288, True, False), (32, 1500, 32768, True, True), (20, 4096, 9216, False, False), (31, 2048, 11264, False, True)])
+def test_17_to_32_rows_read_the_int8_weights_whatever_copies_there_are(dev, m, k, n, norm, gated):
+    """Its bits with a copy in place are those without one; a captured stream then outlives the copy."""
+    rng = np.random.default_rng(m + n)
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)
+    assert HipNative.q8GemmTilePrepared(m, k, n)[0]
+    src, wq = dev.upload(f(k, n) * np.float32(k ** -0.5)), dev.alloc(HipNative.q8Floats(k, n))
+    Stream().q8_quantize(src, wq, k, n, 0, 1, n).run()
+    x, g, out, n_out = dev.upload(f(m, k)), dev.upload(1 + 0.1 * f(k)), dev.alloc(m * n), n // 2 if gated else n
+    s = Stream().q8_linear(x, wq, out, m, k, n_out, gamma=g if norm else -1, swiglu=gated)
+    s.run()
+    want = dev.download(out, (m, n_out))
+    copy = dev.alloc(HipNative.q8PreparedFloats(k, n))
+    Stream().q8_prepare(wq, copy, k, n).fill(out, 0, m * n_out).run()
+    s.run()
+    assert np.isfinite(want).all() and np.array_equal(dev.download(out, (m, n_out)), want)
+    graph = HipNative.graphCapture(s.array())
+    dev.release(copy)
+    for _ in range(3):
+        Stream().fill(out, 0, m * n_out).run()
+        HipNative.graphLaunch(graph)
+        assert np.array_equal(dev.download(out, (m, n_out)), want)
+    HipNative.graphDestroy(graph)
+    dev.release(src, wq, x, g, out)
