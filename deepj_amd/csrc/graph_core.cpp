@@ -361,6 +361,12 @@ Tensor *as_tensor(PyObject *o) {
     PyErr_Format(PyExc_TypeError, "expected a Tensor, not %.100s", Py_TYPE(o)->tp_name);
     return nullptr;
 }
+// Sizes, rows and columns travel as 32-bit words.
+bool fits_words(Py_ssize_t rows, Py_ssize_t cols) {
+    if (rows <= INT32_MAX && cols <= INT32_MAX && rows * cols <= INT32_MAX) return true;
+    PyErr_Format(PyExc_OverflowError, "a buffer of %zdx%zd: more than 32 bits count", rows, cols);
+    return false;
+}
 Buffer *ensure(Graph *g, Tensor *t) {      // borrowed
     if (Buffer *b = tag_of(t)) {
         auto it = g->s->tensors.find(b->id);
@@ -377,6 +383,7 @@ Buffer *ensure(Graph *g, Tensor *t) {      // borrowed
         }
         return b;
     }
+    if (!fits_words(t->rows, t->cols)) return nullptr;
     Buffer *b = new_buffer(g->next_id, t->rows, t->cols, true, false, reinterpret_cast<PyObject *>(g));
     if (!b) return nullptr;
     Py_INCREF(b);                          // until it is the tag
@@ -391,6 +398,7 @@ Buffer *ensure(Graph *g, Tensor *t) {      // borrowed
     return b;
 }
 Buffer *new_output(Graph *g, Py_ssize_t rows, Py_ssize_t cols) {       // a reference of the caller's
+    if (!fits_words(rows, cols)) return nullptr;
     Buffer *b = new_buffer(g->next_id, rows, cols, false, false, reinterpret_cast<PyObject *>(g));
     if (!b) return nullptr;
     g->next_id++;

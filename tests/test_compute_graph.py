@@ -305,6 +305,23 @@ def test_backend_shape_errors_before_recording(rt):                   # MetalBac
     assert be.graph.isEmpty()
 
 
+def test_what_32_bit_words_cannot_count_is_refused(rt):
+    class Clearing(RecordingRuntime):
+        def zeroBuffers(self, zeros): pass
+
+    runtime = Clearing()
+    backend = HipBackend(runtime)
+    big = Tensor(50000, 50000)                    # (its zeros are never made on the host)
+    for call in (lambda: backend.add(big, big), lambda: backend.matmul(Tensor(70000, 1), Tensor(1, 70000)),
+                 lambda: backend.transpose(Tensor(0, 1 << 31))):
+        with pytest.raises(OverflowError):
+            call()
+    out = backend.add(Tensor(2, 2), Tensor(2, 2))
+    backend.graph.flush()                         # what follows is recorded as ever
+    assert all((sizes <= 70000).all() for _, sizes, _ in runtime.allocCalls) and len(runtime.flushCalls) == 1
+    assert out.getGpuTag().allocatedOnGpu
+
+
 def test_int_targets_travel_as_float_column(rt):                      # MetalBackend.java:43-54,531-539
     be = HipBackend(rt)
     Tensor.setBackend(be)
