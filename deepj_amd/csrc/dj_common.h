@@ -281,13 +281,13 @@ struct LatentDecode {
     const int8_t *wq; const float *scales;      // [2 d] rows over rank: Wuk, then Wuv
     const int32_t *state;
     const float *cos_t, *sin_t;
-    float *records, *out;                       // scratch (latent_decode_workspace_floats), [d]
+    float *records, *out;                       // scratch (latent_decode_scratch_floats), [d]
     int heads, hd, rank, max_seq;
     float scale;                                // set by the launcher
 };
 int latent_decode_splits(int heads, int hd, int rank, int max_seq);
 void latent_decode_configure();                 // once per device, before the first launch
-int64_t latent_decode_workspace_floats(int heads, int hd, int rank, int max_seq);
+int64_t latent_decode_scratch_floats(int heads, int hd, int rank, int max_seq);
 void launch_latent_decode(hipStream_t s, LatentDecode a);
 
 }  // namespace dj

@@ -422,7 +422,7 @@ int latent_decode_splits(int heads, int hd, int rank, int max_seq) {
 }
 
 // Scratch: of every head of a launch and split the weighted latent row, the largest score and the sum of the weights
-int64_t latent_decode_workspace_floats(int heads, int hd, int rank, int max_seq) {
+int64_t latent_decode_scratch_floats(int heads, int hd, int rank, int max_seq) {
     const int64_t kmax = q8_padded_k(rank) > 256 ? 512 : 256;
     return (kmax + 2) * std::min(heads, kHeadsAtOnce) * latent_decode_splits(heads, hd, rank, max_seq);
 }

@@ -1356,11 +1356,12 @@ void exec_one(Cursor &c) {
             q8_weight(w[4], rank, 2 * d, op, "wukv", a.wq, a.scales);
             a.state = reinterpret_cast<const int32_t *>(buf(w[5], 4, op, "state"));
             a.cos_t = buf(w[6], max_seq * (hd / 2), op, "cos"); a.sin_t = buf(w[7], max_seq * (hd / 2), op, "sin");
-            buf(w[8], H * splits * (hd + 4), op, "records");       // (what the launches leave each other is larger, and goes to the workspace)
+            buf(w[8], H * splits * (hd + 4), op, "records");       // (what the launches leave each other is larger)
             a.out = buf(w[9], d, op, "out");
             a.heads = (int)H; a.hd = (int)hd; a.rank = (int)rank; a.max_seq = (int)max_seq;
-            need_scratch(c, latent_decode_workspace_floats((int)H, (int)hd, (int)rank, (int)max_seq), 0);
-            a.records = g.workspace;
+            // ... and goes to the block that stays for the graphs captured over it, where a graph of the workspace ends with a larger one
+            need_scratch(c, 0, latent_decode_scratch_floats((int)H, (int)hd, (int)rank, (int)max_seq));
+            a.records = g.row_pieces;
             if (run) launch_latent_decode(s, a);
             break;
         }

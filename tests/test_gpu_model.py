@@ -707,6 +707,39 @@ def test_latent_decode_keeps_to_its_own_scratch(H, hd, rank, max_seq):
         dev.release_all()
 
 
+def test_a_captured_latent_decode_outlives_a_larger_workspace():
+    """A graph of it stays launchable whatever workspace other streams need."""
+    H, hd, rank, max_seq, pos = 4, 64, 96, 100, 70
+    rng, d = np.random.default_rng(5), H * hd
+    q, ckv, rows = (rng.standard_normal(n).astype(np.float32) for n in (d, rank, max_seq * rank))
+    w = (rng.standard_normal((rank, 2 * d)) * rank ** -0.5).astype(np.float32)
+    cos, sin = ref.rope_tables(hd, max_seq)
+    dev, graph = DeviceBuffers(), 0
+    try:
+        src, wq = dev.upload(w), dev.alloc(HipNative.q8Floats(rank, 2 * d))
+        Stream().q8_quantize(src, wq, rank, 2 * d, 0, 1, 2 * d).run()
+        out, lat, state = dev.alloc(d), dev.upload(rows), dev.upload(np.array([pos, 0, 0, 0], np.int32))
+        rec = dev.alloc(H * HipNative.latentDecodeSplits(H, hd, rank, max_seq) * (hd + 4))
+        s = Stream().latent_decode(dev.upload(q), dev.upload(ckv), lat, wq, state, dev.upload(cos), dev.upload(sin), rec, out, H, hd, rank, max_seq, 0)
+        s.run()
+        want = dev.download(out, (d,)).copy()
+        graph = HipNative.graphCapture(s.array())
+        m, k, n = 1024, 32768, 8192                                    # 160 Mi floats of the fp16 GEMM's operands: more than any other test's
+        x, wide, gamma, y = dev.alloc(m * k), dev.alloc(HipNative.q8Floats(k, n)), dev.alloc(k), dev.alloc(m * n)
+        Stream().fill(x, 0, m * k).fill(wide, 0, HipNative.q8Floats(k, n)).fill(gamma, 0, k).run()
+        allocs = HipNative.poolStats()["driver_allocs"]
+        Stream().q8_linear(x, wide, y, m, k, n, gamma=gamma).run()
+        assert HipNative.poolStats()["driver_allocs"] > allocs
+        for _ in range(3):
+            dev.write(out, np.zeros(d, np.float32))
+            HipNative.graphLaunch(graph, 2)
+            assert np.array_equal(dev.download(out, (d,)), want)
+    finally:
+        if graph:
+            HipNative.graphDestroy(graph)
+        dev.release_all()
+
+
 def test_latent_decode_refuses_what_it_does_not_take():
     for shape in ((4, 48, 64, 64), (4, 64, 6, 64), (4, 64, 516, 64), (0, 64, 64, 64), (4, 64, 64, 0)):
         assert HipNative.latentDecodeSplits(*shape) == 0
