@@ -206,25 +206,27 @@ __global__ void __launch_bounds__(64 * KW) k_matmul(const float *__restrict__ A,
 // 2.2e-7 against 4.7e-7 at 2752; 6e-8 to 7e-8 against 1.1e-7 at 192.
 // Bound: the matrix cores at the clock they run the chip down to (about 27 products of 32 x 32 x 16 a ns over the whole chip; the
 // same rate at every depth of pipelining tried) once the tiles fill it, loads and splits in turn below.  k_matmul or
-// k_matmul_lds -> this: 500 x 2752 x 1024 31.4 -> 25.6 us, 1000 x 2752 x 1024 69 -> 43, 1000 x 7000 x 1024 153 -> 103.
+// k_matmul_lds -> this: 500 x 2752 x 1024 31.4 -> 24.5 us, 1000 x 2752 x 1024 69 -> 43, 1000 x 7000 x 1024 153 -> 103.
 struct Pieces { bf16x8 h, m, l; };
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
-// (a dot product of two with -1 and 0 takes the pieces off their values without unpacking them)
+// (Dot products of two with -1 and 0 would take the pieces off without unpacking them, half the instructions at more than twice the
+// time: 500 x 2752 x 1024 26.5 -> 25.3 us without them, 700 x 1024 x 2752 on 64 x 96 tiles 50.0 -> 45.3, 2000 x 4000 x 1024 on them
+// 153 -> 143.)
+__device__ __forceinline__ floatx2 less(floatx2 x, bf16x2 piece) {
+    const uint32_t p = __builtin_bit_cast(uint32_t, piece);
+    return {x[0] - __builtin_bit_cast(float, p << 16), x[1] - __builtin_bit_cast(float, p & 0xffff0000u)};
+}
 __device__ __forceinline__ Pieces split8(const float (&v)[8], float &most) {
     union U { bf16x2 p[4]; bf16x8 b; } h, m, l;
-    uint32_t lo = 0x0000bf80u, hi = 0xbf800000u;     // -1 in one half (in registers: as an inline constant -1.0 is the upper half's)
-    asm("" : "+s"(lo));
-    asm("" : "+s"(hi));
-    const bf16x2 first = __builtin_bit_cast(bf16x2, lo), second = __builtin_bit_cast(bf16x2, hi);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const floatx2 x = {v[2 * j], v[2 * j + 1]};
         asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(v[2 * j]), "v"(v[2 * j + 1]));   // (fmaxf: three instructions)
         h.p[j] = __builtin_convertvector(x, bf16x2);
-        const floatx2 r = {__builtin_amdgcn_fdot2_f32_bf16(h.p[j], first, x[0], false), __builtin_amdgcn_fdot2_f32_bf16(h.p[j], second, x[1], false)};
+        const floatx2 r = less(x, h.p[j]);
         m.p[j] = __builtin_convertvector(r, bf16x2);
-        const floatx2 t = {__builtin_amdgcn_fdot2_f32_bf16(m.p[j], first, r[0], false), __builtin_amdgcn_fdot2_f32_bf16(m.p[j], second, r[1], false)};
+        const floatx2 t = less(r, m.p[j]);
         l.p[j] = __builtin_convertvector(t, bf16x2);
     }
     return {h.b, m.b, l.b};
@@ -787,7 +789,10 @@ void launch_matmul_split(hipStream_t s, const float *a, const float *b, float *o
 // `odd`: the factor on per_k where words are loaded one by one (k, or for k_matmul_lds k or n, no multiple of 4).  k_matmul
 // and k_matmul_lds were fitted to 980 shapes of 1 to 12000 rows and columns over 4 to 6000 k, some of them odd, k_matmul_split
 // to 260 of 8 to 8000 over 32 to 6000; the choice takes 1.002 times the best one's time on average over the latter, 1.09 at
-// worst, where the choice without k_matmul_split takes 1.043 and 1.94.
+// worst, where the choice without k_matmul_split takes 1.043 and 1.94.  Its 32 x 96 tile is for outputs of half a million to
+// 800 thousand values, which leave half of the chip idle in tiles of 64 rows and are several rounds of k_matmul's: 700 x 1024 x
+// 2752 48 -> 41 us, 600 x 1100 x 512 14.0 -> 11.5, 148 x 4712 x 1396 28.8 -> 23.7; over 260 more shapes the choice with it is never
+// slower and 1.05 to 1.22 times as fast for 20.
 static int matmul_kernel(int m, int n, int k) {
     struct Shape { int rows, cols; double fixed, round, per_k, more; int fit; double odd; };
     static const Shape shapes[] = {{32, 32, 2.3, 0.15, 0.0061, 1.95, 0, 1.0},     // k_matmul
@@ -797,8 +802,9 @@ static int matmul_kernel(int m, int n, int k) {
                                    {64, 96, 0.9, 5.1, 0.0156, 0.81, 1, 1.02},
                                    {96, 128, 0.0, 7.2, 0.029, 0.8, 1, 1.03},
                                    {128, 128, 0.0, 9.6, 0.0348, 0.8, 1, 1.06},
+                                   {32, 96, 2.2, 3.7, 0.0119, 1.0, 2, 1.0},
                                    {64, 64, 1.8, 1.4, 0.032, 0.5, 4, 1.6}};       // k_matmul_lds
-    constexpr int kSplit = 3, kLds = 7;
+    constexpr int kSplit = 3, kLds = 8;
     // k_matmul and k_matmul_split address a tile's rows of A in 32 bits, k_matmul a stage's rows of B, k_matmul_split all of B
     const bool in_reach = (int64_t)k * 128 * 4 <= UINT32_MAX && (int64_t)n * 17 * 4 <= UINT32_MAX;
     const bool split_reach = in_reach && (int64_t)k * n * 4 <= INT32_MAX;
@@ -834,6 +840,7 @@ void launch_matmul_f32(hipStream_t s, const float *a, const float *b, float *out
         case 4: launch_matmul_split<2, 3, 4>(s, a, b, out, m, n, k); break;
         case 5: launch_matmul_split<3, 4, 2>(s, a, b, out, m, n, k); break;
         case 6: launch_matmul_split<4, 4, 2>(s, a, b, out, m, n, k); break;
+        case 7: launch_matmul_split<1, 3, 4>(s, a, b, out, m, n, k); break;
         default: {
             const int tn = (n + 63) / 64;
             launch_kernel(k_matmul_lds, dim3((m + 63) / 64 * tn), dim3(256), 0, s, a, b, out, m, n, k, tn);

@@ -53,7 +53,8 @@ def test_matmul_tiles_and_remainders(m, n, k):
 @pytest.mark.parametrize("m,n,k", [(551, 2878, 52), (743, 2462, 127), (1153, 3201, 321),                     # 64 x 64
                                    (2003, 515, 66), (500, 2752, 97), (449, 2785, 193), (846, 1233, 200),     # 64 x 96
                                    (1096, 1943, 39), (961, 2690, 131), (705, 2753, 97), (1000, 2752, 256),   # 96 x 128
-                                   (1000, 3083, 52), (1024, 3329, 129), (897, 3457, 159)])                   # 128 x 128
+                                   (1000, 3083, 52), (1024, 3329, 129), (897, 3457, 159),                    # 128 x 128
+                                   (513, 1345, 447), (481, 1441, 448), (1505, 385, 577), (129, 3361, 513)])  # 32 x 96
 def test_matmul_on_bf16_pieces(m, n, k):
     """The tiles that multiply exact bf16 pieces: an element past a tile in rows and columns, K at and past their steps (32 and
     64), under the same bound.  Then operands that have no pieces, or whose small ones are lost: infinities and NaN give what
