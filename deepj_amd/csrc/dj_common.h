@@ -76,6 +76,11 @@ struct Chain { ChainExt ext[kChainExt]; ChainOp ops[kChainOps]; int n_ext, n_ops
 bool chain_takes(int op);
 void launch_chain(hipStream_t s, const Chain &chain);
 void launch_transpose(hipStream_t s, const float *a, float *out, int rows, int cols);
+// Up to kTransposes of them in one launch, none of which reads or writes what another writes
+constexpr int kTransposes = 8;
+struct Transpose { const float *a; float *out; int rows, cols, first, across; };       // its first workgroup; tiles in a row of tiles
+struct Transposes { Transpose t[kTransposes]; int count = 0; };
+void launch_transposes(hipStream_t s, Transposes &all);
 // AdamW on up to kAdamTensors tensors in one launch (none of them shares memory with another)
 constexpr int kAdamTensors = 16;
 struct AdamTensor { float *w; const float *g; float *mt, *vt; int64_t n; float lr, beta1, beta2, eps, wd, bc1, bc2; };

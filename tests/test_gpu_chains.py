@@ -102,3 +102,49 @@ def test_a_product_between_two_operations_that_depends_on_one_of_them_stays_ther
     exp = -(m.astype(np.float64) @ x) * x
     bound = 2 * 33 * 2.0 ** -24 * (np.abs(m).astype(np.float64) @ np.abs(x)) * np.abs(x)
     assert np.all(np.abs(got - exp) <= bound)
+
+
+@pytest.mark.parametrize("n", [1, 5, 32, 33, 70, 200])
+def test_transposes_that_run_ahead_change_no_bit(n):
+    """Streams of transposes, products, sums and reductions over few square buffers, so that most transposes depend on what stands
+    in front of them: the bits of the operations one by one."""
+    rng = np.random.default_rng(n)
+    dev = DeviceBuffers()
+    try:
+        start = (rng.standard_normal((8, n, n)) * n ** -0.5).astype(np.float32)
+        ids = [dev.alloc(n * n) for _ in range(8)]
+        rows = [dev.alloc(n) for _ in range(2)]
+
+        def run(ops, together):
+            for i, a in zip(ids, start):
+                dev.write(i, a)
+            for r in rows:
+                dev.write(r, np.zeros(n, np.float32))
+            if together:
+                s = Stream()
+                for o in ops:
+                    s.emit(*o)
+                s.run()
+            else:
+                for o in ops:
+                    Stream().emit(*o).run()
+            return [dev.download(i, (n, n)).copy() for i in ids] + [dev.download(r, (n,)).copy() for r in rows]
+        for length in (2, 3, 9, 40, 80):
+            ops = []
+            for _ in range(length):
+                a, b, out = (int(x) for x in rng.choice(ids, 3, replace=False))
+                kind = int(rng.integers(0, 10))
+                if kind < 5:
+                    ops.append([op.OP_TRANSPOSE, a, out, n, n])
+                elif kind < 7:
+                    ops.append([op.OP_MATMUL, a, b, out, n, n, n])
+                elif kind == 7:
+                    ops.append([op.OP_SUBTRACT, a, b, out, n * n])
+                elif kind == 8:
+                    ops.append([op.OP_SUM_ROWS, a, int(rng.choice(rows)), n, n])
+                else:
+                    ops.append([op.OP_ADD_ROW_VECTOR, a, int(rng.choice(rows)), out, n, n] if rng.random() < 0.8 else [op.OP_EXP, a, a, n * n])
+            for got, want in zip(run(ops, True), run(ops, False)):
+                assert np.array_equal(got, want, equal_nan=True)
+    finally:
+        dev.release_all()
