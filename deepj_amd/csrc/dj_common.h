@@ -218,8 +218,6 @@ void launch_rope_rows(hipStream_t s, const float *x, float *out, const int32_t *
                       const float *sin_t, int rows, int H, int hd, int max_seq, int pos_from_row, int row_stride,
                       int live_extra);
 void launch_attention(hipStream_t s, const AttnArgs &a);
-// out [heads][hd] from base-2 records [heads][shares][hd + 4] = {max, sum, -, -, o[hd]} (max -inf: no keys)
-void launch_attention_merge(hipStream_t s, const float *records, float *out, int heads, int hd, int shares);
 void launch_attn_decode(hipStream_t s, const float *qkv, float *k_cache, float *v_cache, float *out,
                         const int32_t *state, float *scratch, const float *cos_t, const float *sin_t, int H, int hd,
                         int max_seq, unsigned *counters);

@@ -905,9 +905,6 @@ int64_t attention_scratch_floats(int S, int H, int hd, int max_seq) {
     return z > 1 ? (int64_t)S * H * z * (hd + 4) : 0;
 }
 
-void launch_attention_merge(hipStream_t s, const float *records, float *out, int heads, int hd, int shares) {
-    launch_kernel(k_attention_merge_shares, dim3(heads, 1), dim3(128), 0, s, records, out, heads, hd, shares);
-}
 
 int64_t attn_decode_scratch_floats(int H, int hd) { return (int64_t)H * fused_decode_splits(H) * (hd + 4); }
 
