@@ -197,6 +197,88 @@ __global__ void __launch_bounds__(64 * KW) k_matmul(const float *__restrict__ A,
         }
 }
 
+// Outputs of at most 512 tiles of 16 x 16, two a compute unit: tiles of 32 x 32 would leave half to all but a few of them idle, each
+// tile with four times the products behind one another.  As k_matmul: 16 wavefronts share K in stages of 16 k dealt in turn, operands straight into
+// registers, a stage ahead (two, three or five: 0 to 25 % slower); lane l has row or column l % 16 and the four k of a stage at 4 (l / 16), the x-th of which goes into
+// the x-th product (the four groups' k add up whatever their order).
+// Bound by a chain of a few trips to the caches and the launch.  k_matmul -> this, us: 256 x 192 x 768 7.4 -> 4.4, x 1003 9.3 -> 5.0;
+// 16 x 2048 x 2048 15.0 -> 7.6; 4 x 2752 x 1024 8.8 -> 4.8; 128 x 384 x 1500 12.0 -> 6.1; 17 x 17 x 4000 24.7 -> 11.0; 500 x 256 x 700 7.7 ->
+// 6.1; 256 x 512 x 2048 15.8 -> 13.5.  Error against float64 1.3e-7 of the result's rms at 1003 k, 1.6e-7 before.
+template <bool VEC>
+__global__ void __launch_bounds__(1024) k_matmul_16(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, const int M, const int N,
+                                                    const int K, const int tiles_m, const int tiles_n) {
+    constexpr int kWaves = 16, kStage = 16, kPitch = 17, D = 2;
+    typedef float floatx4 __attribute__((ext_vector_type(4)));
+    __shared__ float red[kWaves][16 * kPitch];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, quarter = lane >> 4;
+    const int total = tiles_m * tiles_n, xcd = blockIdx.x & 7, q = total >> 3, r = total & 7;      // (as k_matmul)
+    const int idx = xcd * q + (xcd < r ? xcd : r) + (int)(blockIdx.x >> 3);
+    const bool by_cols = N >= M;
+    const int tile_n = by_cols ? idx / tiles_m : idx % tiles_n, tile_m = by_cols ? idx % tiles_m : idx / tiles_n;
+    const int m0 = tile_m * 16, n0 = tile_n * 16;
+
+    // rows and columns past the matrix repeat its last one: their products are not stored
+    const float *Am = A + (int64_t)m0 * K;
+    const uint32_t a_off = ((uint32_t)(l16 < M - m0 ? l16 : M - 1 - m0) * (uint32_t)K + 4u * quarter) * 4u;
+    const uint32_t b_off = (4u * quarter * (uint32_t)N + (uint32_t)(n0 + l16 < N ? n0 + l16 : N - 1)) * 4u;
+    floatx4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};      // (two sums of half as many products: less error)
+    struct Stage { float a[4], b[4]; };
+    auto load = [&](Stage &st, int k0) {
+        const char *p = reinterpret_cast<const char *>(Am + k0) + a_off;
+        if constexpr (VEC) {
+            const float4 v = *reinterpret_cast<const float4 *>(p);
+            st.a[0] = v.x; st.a[1] = v.y; st.a[2] = v.z; st.a[3] = v.w;
+        } else {
+#pragma unroll
+            for (int x = 0; x < 4; x++) st.a[x] = reinterpret_cast<const float *>(p)[x];
+        }
+#pragma unroll
+        for (int x = 0; x < 4; x++) st.b[x] = at_bytes(B + (int64_t)(k0 + x) * N, b_off);
+    };
+    auto multiply = [&](const Stage &st) {
+#pragma unroll
+        for (int x = 0; x < 4; x++) acc[x & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.a[x], st.b[x], acc[x & 1], 0, 0, 0);
+    };
+    const int stages = K / kStage, mine = (stages - wave + kWaves - 1) / kWaves;
+    if (mine > 0) {
+        Stage st[D];
+        auto at = [&](int i) { return ((i < mine ? i : mine - 1) * kWaves + wave) * kStage; };
+#pragma unroll
+        for (int d = 0; d < D; d++) load(st[d], at(d));
+        int i = 0;
+        for (; i + D <= mine; i += D) {
+#pragma unroll
+            for (int d = 0; d < D; d++) {
+                multiply(st[d]);
+                load(st[d], at(i + d + D));
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D - 1; d++)
+            if (i + d < mine) multiply(st[d]);
+    }
+    if (stages * kStage < K && wave == (stages & (kWaves - 1))) {      // the rest of K, with zeros past its end
+        Stage st;
+        const int k0 = stages * kStage, k = k0 + 4 * quarter;
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            st.a[x] = k + x < K ? at_bytes(Am + k0 + x, a_off) : 0.0f;
+            st.b[x] = k + x < K ? at_bytes(B + (int64_t)(k0 + x) * N, b_off) : 0.0f;
+        }
+        multiply(st);
+    }
+    // acc[.][e] is C[4 quarter + e][l16]
+#pragma unroll
+    for (int e = 0; e < 4; e++) red[wave][(4 * quarter + e) * kPitch + l16] = acc[0][e] + acc[1][e];
+    __syncthreads();
+    if (threadIdx.x >= 256) return;
+    const int row = threadIdx.x >> 4, col = threadIdx.x & 15;
+    float v = red[0][row * kPitch + col];
+#pragma unroll
+    for (int w = 1; w < kWaves; w++) v += red[w][row * kPitch + col];
+    if (m0 + row < M && n0 + col < N) C[(int64_t)(m0 + row) * N + n0 + col] = v;
+}
+
 // ── fp32 x fp32 on the bf16 matrix cores ────────────────────────────────────
 // An fp32 value is the exact sum of three bf16 values (itself rounded to bf16, the remainder rounded, the rest), so
 //   a . b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh) + ...       what is left out is about 2^-26 of |a b|
@@ -775,6 +857,11 @@ void launch_matmul(hipStream_t s, const float *a, const float *b, float *out, in
     if ((k & 3) == 0) launch_kernel((k_matmul<TM, TN, KW, U, D, true>), dim3(tm * tn), dim3(64 * KW), 0, s, a, b, out, m, n, k, tm, tn);
     else launch_kernel((k_matmul<TM, TN, KW, U, D, false>), dim3(tm * tn), dim3(64 * KW), 0, s, a, b, out, m, n, k, tm, tn);
 }
+void launch_matmul_16(hipStream_t s, const float *a, const float *b, float *out, int m, int n, int k) {
+    const int tm = (m + 15) / 16, tn = (n + 15) / 16;
+    if ((k & 3) == 0) launch_kernel((k_matmul_16<true>), dim3(tm * tn), dim3(1024), 0, s, a, b, out, m, n, k, tm, tn);
+    else launch_kernel((k_matmul_16<false>), dim3(tm * tn), dim3(1024), 0, s, a, b, out, m, n, k, tm, tn);
+}
 template <int TM, int WC, int KS>
 void launch_matmul_split(hipStream_t s, const float *a, const float *b, float *out, int m, int n, int k) {
     const int tm = (m + 32 * TM - 1) / (32 * TM), tn = (n + 32 * WC - 1) / (32 * WC);
@@ -829,8 +916,10 @@ void launch_matmul_f32(hipStream_t s, const float *a, const float *b, float *out
     const int64_t blocks = (int64_t)((m + 31) / 32) * ((n + 31) / 32);
     switch (matmul_kernel(m, n, k)) {
         case 0:
-            // a tile per compute unit at most: more wavefronts share its K, with shorter stages so that their lines fit
-            if (blocks <= 256 && k > 256) launch_matmul<1, 1, 16, 1, 2>(s, a, b, out, m, n, k);
+            // a tile per compute unit at most: more wavefronts share its K, with shorter stages so that their lines fit; up to two
+            // tiles of 16 x 16, those (768 of them: 8.5 us where 32 x 32 take 8.1 at 768 k; at 256 k and less all take about 4)
+            if (k > 256 && (int64_t)((m + 15) / 16) * ((n + 15) / 16) <= 512) launch_matmul_16(s, a, b, out, m, n, k);
+            else if (blocks <= 256 && k > 256) launch_matmul<1, 1, 16, 1, 2>(s, a, b, out, m, n, k);
             else if (blocks <= 256) launch_matmul<1, 1, 8, 4, 2>(s, a, b, out, m, n, k);
             else launch_matmul<1, 1, 4, 4, 2>(s, a, b, out, m, n, k);
             break;

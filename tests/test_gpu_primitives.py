@@ -50,6 +50,22 @@ def test_matmul_tiles_and_remainders(m, n, k):
     assert np.all(np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= bound)
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 1, 257), (2, 17, 264), (16, 16, 260), (17, 33, 272), (33, 47, 511), (256, 192, 1003), (15, 4097, 271),
+                                   (512, 256, 304), (513, 256, 304), (4, 2752, 1024), (100, 300, 4001)])
+def test_matmul_of_small_outputs_over_a_long_k(m, n, k):
+    """Tiles of 16 x 16 that sixteen wavefronts share the K of: an element past a tile, a stage (16) and a round of them (256), the
+    most tiles there are and one row more, under the same bound; a NaN stays in its row."""
+    rng = np.random.default_rng(m + n * k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    bound = 2 * k * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
+    with backend() as be:
+        assert np.all(np.abs(be.matmul(tensor(a), tensor(b)).numpy() - exact) <= bound)
+        a[m - 1, k - 1] = np.nan
+        got = be.matmul(tensor(a), tensor(b)).numpy()
+    assert np.all(np.isnan(got[m - 1])) and np.all(np.abs(got[:m - 1] - exact[:m - 1]) <= bound[:m - 1])
+
+
 @pytest.mark.parametrize("m,n,k", [(551, 2878, 52), (743, 2462, 127), (1153, 3201, 321),                     # 64 x 64
                                    (2003, 515, 66), (500, 2752, 97), (449, 2785, 193), (846, 1233, 200),     # 64 x 96
                                    (1096, 1943, 39), (961, 2690, 131), (705, 2753, 97), (1000, 2752, 256),   # 96 x 128
