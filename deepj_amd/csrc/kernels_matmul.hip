@@ -280,7 +280,8 @@ __global__ void __launch_bounds__(1024) k_matmul_16(const float *__restrict__ A,
 }
 
 // ── fp32 x fp32 on the bf16 matrix cores ────────────────────────────────────
-// An fp32 value is the exact sum of three bf16 values (itself rounded to bf16, the remainder rounded, the rest), so
+// An fp32 value of at least 2^-103 is the exact sum of three bf16 values (itself rounded to bf16, the remainder rounded, the
+// rest), of a smaller one pieces below 2^-126 may be lost (k_matmul_split looks for results that this can be seen in); so
 //   a . b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh) + ...       what is left out is about 2^-26 of |a b|
 // and six bf16 products of 16 k take 0.375 of the time of eight fp32 products of 2.  The first product and the five small ones
 // have accumulators of their own, so that the large sum is cut off once per 16 k and set (fp32 instructions: eight times): its
@@ -327,8 +328,7 @@ __global__ void __launch_bounds__(64 * WC * KS) k_matmul_split(const float *__re
     constexpr int kStride = 36;                     // LDS row of a 32-column block (16-byte aligned, spreads the two halves)
     constexpr int kOperands = KS * TM * 3 * 64;     // 16-byte words of a step
     __shared__ uint32_t row_most[kRows], col_most[32 * WC];
-    __shared__ int any_tiny;
-    auto is_tiny = [](uint32_t most) { return most < (127u - 77u) << 23 && most > 0u; };       // 2^-77
+    __shared__ uint32_t again[kRows * WC], again_rows;          // the outputs to do again, a bit each; the blocks of 32 rows that hold some
     __shared__ __align__(16) uint4 lds[2 * kOperands * 16 > kWaves * 32 * kStride * 4 ? 2 * kOperands : kWaves * 32 * kStride / 4];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -452,38 +452,76 @@ __global__ void __launch_bounds__(64 * WC * KS) k_matmul_split(const float *__re
     // acc[i][e] is C[32 i + 8 (e / 4) + 4 half + e % 4][l32] of the wavefront's columns
     float *red = reinterpret_cast<float *>(lds);
     for (int o = threadIdx.x; o < kRows + 32 * WC; o += 64 * kWaves) (o < kRows ? row_most[o] : col_most[o - kRows]) = 0u;
+    for (int o = threadIdx.x; o < kRows * WC; o += 64 * kWaves) again[o] = 0u;
+    if (threadIdx.x == 0) again_rows = 0u;
     __syncthreads();
 #pragma unroll
     for (int g = 0; g < kStages; g++)
         if (wc + g * WC < TM) atomicMax(&row_most[32 * (wc + g * WC) + l32], __builtin_bit_cast(uint32_t, most_a[g]));
     atomicMax(&col_most[32 * wc + l32], __builtin_bit_cast(uint32_t, most_b));
-    if (threadIdx.x == 0) any_tiny = 0;
     __syncthreads();
-    for (int o = threadIdx.x; o < kRows + 32 * WC; o += 64 * kWaves)
-        if (is_tiny(o < kRows ? row_most[o] : col_most[o - kRows])) any_tiny = 1;
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
+    // What an output may have lost with pieces below 2^-126 is at most K 2^-126 (the row's largest + the column's); limit is 2^24
+    // times that (and as much for products below 2^-126), so that a larger result has lost less than one rounding.
+    const float scale = (float)K * 0x1p-42f;
+    auto limit = [&](uint32_t most) { return most ? (__builtin_bit_cast(float, most) + 0.5f) * 0x1p-60f * scale : -INFINITY; };    // (zeros lose nothing)
+    const int c = threadIdx.x % (32 * WC);
+    const float of_col = limit(col_most[c]);
+    auto store = [&](int i, auto &&of, auto &&wanted) {
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < 16; e++) red[(wave * 32 + 8 * (e >> 2) + 4 * half + (e & 3)) * kStride + l32] = acc[i][e] + low[i][e];
+        for (int e = 0; e < 16; e++) red[(wave * 32 + 8 * (e >> 2) + 4 * half + (e & 3)) * kStride + l32] = of(e);
         __syncthreads();
         for (int o = threadIdx.x; o < 1024 * WC; o += 64 * kWaves) {
-            const int row = o / (32 * WC), c = o % (32 * WC), at = ((c >> 5) * 32 + row) * kStride + (c & 31);
+            const int row = o / (32 * WC), at = ((c >> 5) * 32 + row) * kStride + (c & 31);
             float v = red[at];
 #pragma unroll
             for (int w = 1; w < KS; w++) v += red[w * WC * 32 * kStride + at];
             const int out_row = m0 + 32 * i + row, out_col = n0 + c;
-            if (out_row < M && out_col < N) {
-                // An operand that is no finite number has no such pieces, and a sum may leave the range in another order; and
-                // where a whole row or column is tiny, pieces below 2^-126 are lost that matter: there the products are
-                // added one by one.
-                if (!(fabsf(v) <= 3.40282347e38f) || (any_tiny && (is_tiny(row_most[32 * i + row]) || is_tiny(col_most[c])))) {
-                    v = 0.0f;
-                    for (int k = 0; k < K; k++) v = fmaf(A[(int64_t)out_row * K + k], B[(int64_t)k * N + out_col], v);
-                }
-                C[(int64_t)out_row * N + out_col] = v;
-            }
+            if (out_row < M && out_col < N && wanted(32 * i + row, v)) C[(int64_t)out_row * N + out_col] = v;
         }
+    };
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+        store(i, [&](int e) { return acc[i][e] + low[i][e]; }, [&](int row, float v) {
+            if (fabsf(v) <= 3.40282347e38f && !(fabsf(v) <= limit(row_most[row]) + of_col)) return true;
+            atomicOr(&again[row * WC + (c >> 5)], 1u << (c & 31));
+            atomicOr(&again_rows, 1u << (row >> 5));
+            return false;
+        });
+    __syncthreads();
+    const uint32_t rows_again = again_rows;
+    if (!rows_again) return;
+
+    // An operand that is no finite number has no such pieces, a sum may leave the range in another order, and small values may
+    // have lost theirs: those outputs come from the fp32 instructions, the 32 rows around one as in k_matmul.  1000 x 2752 x 1024:
+    // 46 us, 69 with a NaN in one row, 128 with nothing else in an operand, 95 with one of values near 1e-24 (whose sums cancel
+    // to below the limit here and there); a thread an output, product behind product, took 259 and 3070.
+    const uint32_t col_off = (uint32_t)col * 4u;
+#pragma unroll 1
+    for (int i = 0; i < TM; i++) {
+        if (!(rows_again >> i & 1)) continue;
+        const int row = 32 * i + l32;
+        const uint32_t row_off = (uint32_t)(row < M - m0 ? row : M - 1 - m0) * (uint32_t)K * 4u;
+        floatx16 sum[2];
+#pragma unroll
+        for (int e = 0; e < 16; e++) sum[0][e] = sum[1][e] = 0.0f;
+        auto products = [&](int k0, bool whole) __attribute__((always_inline)) {
+            float av[16], bv[16];
+#pragma unroll
+            for (int x = 0; x < 16; x++) {
+                const int k = k0 + 8 * (x >> 2) + 4 * half + (x & 3);
+                const bool in = whole || k < K;
+                av[x] = in ? at_bytes(Am + k, row_off) : 0.0f;
+                bv[x] = in ? at_bytes(B + (int64_t)k * N, col_off) : 0.0f;
+            }
+#pragma unroll
+            for (int x = 0; x < 16; x++) sum[x & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[x], bv[x], sum[x & 1], 0, 0, 0);
+        };
+        int k0 = 32 * set;
+#pragma unroll 1
+        for (; k0 + 32 <= K; k0 += 32 * KS) products(k0, true);
+        if (k0 < K) products(k0, false);
+        store(i, [&](int e) { return sum[0][e] + sum[1][e]; }, [&](int r, float) { return (again[r * WC + (c >> 5)] >> (c & 31) & 1) != 0; });
     }
 }
 

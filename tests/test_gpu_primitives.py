@@ -97,6 +97,33 @@ def test_matmul_on_bf16_pieces(m, n, k):
     assert np.all(np.abs(got[ok] - exact[ok]) <= bound[ok])
 
 
+@pytest.mark.parametrize("m,n,k", [(551, 2878, 52), (500, 2752, 97), (1000, 2752, 256), (1000, 3083, 52), (1024, 3329, 129), (513, 1345, 447)])
+def test_matmul_on_bf16_pieces_of_mixed_magnitudes(m, n, k):
+    """Values whose small pieces are lost (2^-104 and below, fp32 subnormals) beside ordinary ones in a row or a column, where the
+    other operand is zero at the ordinary ones and large at the small: the same bound; and no other output changes a bit."""
+    rng = np.random.default_rng(m + n * k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    with backend() as be:
+        plain = be.matmul(tensor(a), tensor(b)).numpy().copy()
+    rows, cols, ordinary = [2, 40, m - 1], [4, 70, n - 1], np.arange(k) % 5 == 0
+    small = np.exp2(-104.0 - np.arange(k) % 24)
+    for r, c, size in zip(rows, cols, (1.0, 1e-2, 2.0 ** -16)):            # (2^-144: subnormal)
+        a[r], b[:, c] = np.where(ordinary, a[r], a[r] * small * size), np.where(ordinary, 0.0, b[:, c] * np.float32(1e30))
+    a[9], b[:, 11] = np.where(ordinary, 0.0, a[9] * np.float32(1e30)), np.where(ordinary, b[:, 11], b[:, 11] * small)
+    a[12], b[:, 17] = np.eye(1, k, 3), np.where(np.arange(k) == 3, 0.0, b[:, 17] * small)       # one ordinary product, by zero
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    bound = 2 * k * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64)) + k * 2.0 ** -149
+    with backend() as be:
+        got = be.matmul(tensor(a), tensor(b)).numpy()
+    exact = a64 @ b64
+    wrong = np.argwhere((np.abs(got - exact) > bound) & (np.abs(exact) < 1e38))                  # (row 9 by a column of 1e30: beyond fp32)
+    assert not len(wrong), (wrong[:8], len(wrong))
+    assert got[12, 17] == 0.0
+    others = np.ones((m, n), bool)
+    others[[*rows, 9, 12]], others[:, [*cols, 11, 17]] = False, False
+    assert np.array_equal(got[others], plain[others])
+
+
 @pytest.mark.parametrize("m,n,k", [(128, 1, 8500000), (1, (1 << 26) + 5, 3)])
 def test_matmul_with_rows_beyond_32_bit_offsets(m, n, k):
     """A tile's rows of A, or a stage's rows of B, more than 4 GiB apart: what the last row and column hold is found there."""
