@@ -522,6 +522,8 @@ struct Cursor {
     bool alone = false; // every op by itself (per-op timing)
     int32_t done[kTransposes] = {};     // ops further on that have run already, in order: done[next_done] is the next one to pass
     int n_done = 0, next_done = 0;
+    int32_t pieces_pos = -1;            // the op that finds its rows' pieces made, and where in their block; the dry pass knows by shapes
+    int64_t pieces_at = 0;
 };
 
 const char *op_name(int op);
@@ -1052,7 +1054,8 @@ void exec_one(Cursor &c) {
             bool unshared = false;
             const int64_t own_pieces = g.no_alloc ? 0 : q8_linear_pieces_floats((int)m, (int)k, (int)n, flags, p.prepared != nullptr, false, &unshared);
             // The op right behind this one multiplies this output as it is: where both are products for k_gemm_q8_rows, this one's
-            // epilogue leaves that one's pieces behind its own.
+            // epilogue leaves that one's pieces behind its own, or in front of them where there is room.  Which products do so and where
+            // their pieces lie hangs on shapes alone, so that a stream has the same bits whatever size the block has grown to.
             const int32_t *behind = c.pos + stride_of(op) + 12 <= c.len ? c.cmd + c.pos + stride_of(op) : nullptr;
             const auto prepared_as = [&](int32_t weight, int64_t wk, int64_t wrows) {
                 auto it = g.prepared.find(weight);
@@ -1064,22 +1067,23 @@ void exec_one(Cursor &c) {
             if (m > 1 && own_pieces > 0 && unshared && behind && behind[0] == DJ_OP_Q8_LINEAR && behind[1] == w[3] && behind[4] == m && behind[5] == n && behind[6] > 0 &&
                 behind[6] < (1 << 30) && !(behind[7] & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM | DJ_LIN_ATTN_MERGE)))
                 plain_pieces = q8_linear_pieces_floats((int)m, (int)n, behind[6], behind[7], prepared_as(behind[2], n, rows_of(behind)), true);
-            need_scratch(c, ws, plain_pieces > 0 ? behind_own + plain_pieces : own_pieces);
+            const bool may_chain = run && m > 1 && !g.no_alloc && !merge;
+            const bool pieces_ready = may_chain && pieces_left(m, k);
+            const int64_t pieces_at = pieces_ready ? was.pieces_at : !run && c.pieces_pos == c.pos ? c.pieces_at : 0;
+            const int64_t next_at = plain_pieces <= 0 || pieces_at >= plain_pieces ? 0 : pieces_at + behind_own;
+            if (plain_pieces > 0) { c.pieces_pos = c.pos + stride_of(op); c.pieces_at = next_at; }
+            need_scratch(c, ws, plain_pieces > 0 ? std::max(pieces_at + behind_own, next_at + plain_pieces) : own_pieces > 0 ? pieces_at + own_pieces : 0);
             // One rule for the allocation-free entry point, whatever happens to fit its fixed array: the many-row
             // fp16 GEMM (whose operands live in a workspace sized by the shape) is never taken there.
             p.small_workspace_only = g.no_alloc;
             GemmChain chain;
             int32_t next_gamma_id = -1, next_beta_id = -1;
-            int64_t pieces_at = 0, next_at = 0;
             const int32_t next_pos = c.pos + stride_of(op);
-            if (run && m > 1 && !g.no_alloc && !merge) {
+            if (may_chain) {
                 chain.planes_ready = chained(w[1], w[8], flags, m, k);
-                chain.pieces_ready = pieces_left(m, k);
-                if (chain.pieces_ready) pieces_at = was.pieces_at;
-                if (plain_pieces > 0 && pieces_at + behind_own + plain_pieces <= g.row_pieces_floats) {
-                    next_at = pieces_at + behind_own;
+                chain.pieces_ready = pieces_ready;
+                if (plain_pieces > 0 && next_at + plain_pieces <= g.row_pieces_floats)      // (less only where the dry pass saw other prepared copies)
                     chain.next_pieces = reinterpret_cast<uint16_t *>(g.row_pieces + next_at);
-                }
                 // the op right behind this one normalises this output (RMSNorm) and multiplies it on the fp16 GEMM: the
                 // launch may leave that op's activations ready (it does when this one shares its tiles' K)
                 if (next_pos < c.len && !sw && !chain.next_pieces) {
@@ -1110,7 +1114,7 @@ void exec_one(Cursor &c) {
             }
             if (run) launch_q8_linear(s, p, g.workspace, g.workspace_floats, g.row_pieces + pieces_at, g.row_pieces_floats - pieces_at);
             if (chain.left_planes || chain.left_pieces) {
-                g.chain.pieces_at = next_at; g.chain.plain = chain.left_pieces && !chain.next_gamma;
+                g.chain.pieces_at = chain.next_gamma ? 0 : next_at; g.chain.plain = chain.left_pieces && !chain.next_gamma;
                 g.chain.cmd = c.cmd; g.chain.pos = next_pos; g.chain.x_id = w[3]; g.chain.gamma_id = next_gamma_id; g.chain.beta_id = next_beta_id;
                 g.chain.m = m; g.chain.k = n; g.chain.pieces = chain.left_pieces; g.chain.valid = true;
             }

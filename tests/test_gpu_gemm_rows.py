@@ -178,6 +178,43 @@ def test_a_row_that_is_not_finite_stays_alone(dev, m, k, n, taken):
     assert np.array_equal(got[keep], clean[keep])
 
 
+@pytest.mark.parametrize("widths,last_alone", [((64, 512, 50000, 64), False), ((1500, 512, 512, 64), True), ((2048, 1000, 2048, 64), False)])
+def test_products_in_a_row_have_the_same_bits_whatever_the_block_of_pieces_holds(dev, widths, last_alone):
+    """Three products behind one another, each multiplying the rows of the one in front as they are: the third takes the kernel that
+    it takes with its pieces made (also where it takes another by itself), in the first run, which makes the block, as after a
+    larger one; with its pieces behind the second one's and, where those lie far enough in, in front of them."""
+    m, makes_block = 100, widths[2] == 50000
+    rng = np.random.default_rng(3)
+    assert [HipNative.q8GemmRowsTile(m, k, n, norm=k == widths[0])[0] > 0 for k, n in zip(widths, widths[1:])] == [True, True, last_alone]
+    weights, rows = [], [dev.upload(rng.standard_normal((m, widths[0])).astype(np.float32)), *(dev.alloc(m * n) for n in widths[1:])]
+    gamma, big_m, big_k, big_n = dev.upload(np.ones(widths[0], np.float32)), 512, 16384, 1026
+    for k, n in (*zip(widths, widths[1:]), (big_k, big_n)):
+        last = rng.standard_normal((k, n), dtype=np.float32) * np.float32(k ** -0.5)
+        if len(weights) == 2:
+            third = last
+        src = dev.upload(last)
+        weights.append(dev.alloc(HipNative.q8Floats(k, n)))
+        Stream().q8_quantize(src, weights[-1], k, n).run()
+        dev.release(src)
+    big_x, big_o = dev.alloc(big_m * big_k), dev.alloc(big_m * big_n)
+    three, big = Stream(), Stream().fill(big_x, 0, big_m * big_k).q8_linear(big_x, weights[3], big_o, big_m, big_k, big_n)
+    for i, (k, n) in enumerate(zip(widths, widths[1:])):
+        three.q8_linear(rows[i], weights[i], rows[i + 1], m, k, n, gamma=-1 if i else gamma)
+    driver_allocs = lambda: HipNative.poolStats()["driver_allocs"]
+    before = driver_allocs()
+    three.run()
+    made = driver_allocs()
+    first = dev.download(rows[3], (m, widths[3])).copy()
+    check(first, dev.download(rows[2], (m, widths[2])).astype(np.float64) @ ref.q8_roundtrip(third).astype(np.float64), widths[2], widths)
+    big.run()
+    if makes_block:
+        assert before < made < driver_allocs()                           # a block of the size that the three need, then a larger one
+    Stream().fill(rows[3], 0, m * widths[3]).run()
+    three.run()
+    assert np.array_equal(dev.download(rows[3], (m, widths[3])), first)
+    dev.release(*weights, *rows, gamma, big_x, big_o)
+
+
 def test_a_captured_product_outlives_a_larger_one(dev):
     """A product without a normalisation needs no workspace: a graph of it stays launchable whatever other streams need, over the
     block of pieces that it was captured with, also beside graphs of other blocks and once one of its own block is gone."""
