@@ -60,6 +60,8 @@ def _bind(lib: C.CDLL) -> None:
     lib.deepj_hip_q8_gemm_tile_prepared.restype = None
     lib.deepj_hip_q8_gemm_rows_tile.argtypes = [C.c_int32] * 6 + [_i32p, _i32p, _i32p]
     lib.deepj_hip_q8_gemm_rows_tile.restype = C.c_int32
+    lib.deepj_hip_q8_gemm_rows_tile_behind.argtypes = [C.c_int32] * 4 + [_i32p, _i32p, _i32p]
+    lib.deepj_hip_q8_gemm_rows_tile_behind.restype = C.c_int32
     lib.deepj_hip_q8_linear_rope_ok.argtypes = [C.c_int32, C.c_int32, C.c_int32]
     lib.deepj_hip_q8_linear_rope_ok.restype = C.c_int32
     lib.deepj_hip_clock_probe.argtypes = [_i32p, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]
@@ -256,6 +258,13 @@ class HipNative:
         the int8 weights for this problem; rows 0: not taken."""
         r, c, s = C.c_int32(), C.c_int32(), C.c_int32()
         library().deepj_hip_q8_gemm_rows_tile(m, k, rows, norm, prepared, alloc_free, C.byref(r), C.byref(c), C.byref(s))
+        return r.value, c.value, s.value
+
+    @staticmethod
+    def q8GemmRowsTileBehind(m: int, k: int, rows: int, prepared: bool = False):
+        """The same right behind a product of this kernel that leaves it its rows ready (no normalisation in between)."""
+        r, c, s = C.c_int32(), C.c_int32(), C.c_int32()
+        library().deepj_hip_q8_gemm_rows_tile_behind(m, k, rows, prepared, C.byref(r), C.byref(c), C.byref(s))
         return r.value, c.value, s.value
 
     @staticmethod

@@ -1847,14 +1847,22 @@ void deepj_hip_q8_gemm_tile_prepared(int32_t m, int32_t k, int32_t rows, int32_t
     if (k_shares) *k_shares = ks;
 }
 
-int32_t deepj_hip_q8_gemm_rows_tile(int32_t m, int32_t k, int32_t rows, int32_t norm, int32_t prepared, int32_t alloc_free, int32_t *tile_rows, int32_t *tile_cols,
-                                    int32_t *k_shares) {
-    RowsPlan p{};
-    const bool taken = m > 0 && k > 0 && rows > 0 && q8_gemm_rows_ok(m, rows, k, norm != 0, prepared != 0 && !alloc_free, !alloc_free, &p);
+static int32_t rows_tile(bool taken, const RowsPlan &p, int32_t *tile_rows, int32_t *tile_cols, int32_t *k_shares) {
     if (tile_rows) *tile_rows = taken ? 32 * p.tmw : 0;
     if (tile_cols) *tile_cols = taken ? 32 * p.tnw : 0;
     if (k_shares) *k_shares = taken ? p.shares : 1;
     return taken;
+}
+int32_t deepj_hip_q8_gemm_rows_tile(int32_t m, int32_t k, int32_t rows, int32_t norm, int32_t prepared, int32_t alloc_free, int32_t *tile_rows, int32_t *tile_cols,
+                                    int32_t *k_shares) {
+    RowsPlan p{};
+    const bool taken = m > 0 && k > 0 && rows > 0 && q8_gemm_rows_ok(m, rows, k, norm != 0, prepared != 0 && !alloc_free, !alloc_free, &p);
+    return rows_tile(taken, p, tile_rows, tile_cols, k_shares);
+}
+int32_t deepj_hip_q8_gemm_rows_tile_behind(int32_t m, int32_t k, int32_t rows, int32_t prepared, int32_t *tile_rows, int32_t *tile_cols, int32_t *k_shares) {
+    RowsPlan p{};
+    const bool taken = m > 0 && k > 0 && rows > 0 && q8_gemm_rows_ok(m, rows, k, false, prepared != 0, true, &p, true);
+    return rows_tile(taken, p, tile_rows, tile_cols, k_shares);
 }
 
 int32_t deepj_hip_q8_linear_rope_ok(int32_t m, int32_t k, int32_t d) {

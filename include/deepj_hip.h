@@ -297,6 +297,10 @@ void deepj_hip_q8_gemm_tile_prepared(int32_t m, int32_t k, int32_t rows, int32_t
  * fixed workspace holds the rows. */
 int32_t deepj_hip_q8_gemm_rows_tile(int32_t m, int32_t k, int32_t rows, int32_t norm, int32_t prepared, int32_t alloc_free, int32_t *tile_rows,
                                     int32_t *tile_cols, int32_t *k_shares);
+/* The same for a Q8_LINEAR without a normalisation right behind the Q8_LINEAR whose output it multiplies, where that one runs on
+ * this kernel with a tile's K in one workgroup: it leaves the rows ready, and this one runs here also in cases where by itself
+ * it would take another kernel - the same accuracy, other last bits.  (deepj_hip_flush_ops_noalloc leaves nothing ready.) */
+int32_t deepj_hip_q8_gemm_rows_tile_behind(int32_t m, int32_t k, int32_t rows, int32_t prepared, int32_t *tile_rows, int32_t *tile_cols, int32_t *k_shares);
 /* Host arithmetic only (no GPU call): the last byte + 1 that the fp16 GEMM's direct global -> LDS loads reach in its three
  * operand buffers {activation planes, fp16 weights, transposed scales} for a tile of tile_rows x tile_cols (128 or 64 rows
  * by 256 or 192 columns; tile_rows 0: the tile the library would choose), and the bytes those buffers hold.  Returns 1

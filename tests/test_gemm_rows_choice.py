@@ -41,6 +41,19 @@ def test_every_choice_is_one_the_kernel_has():
     assert len(seen) == 12                               # eleven and none
 
 
+def test_a_product_whose_rows_are_ready_is_taken_in_more_cases():
+    """Right behind the product that leaves its rows ready it runs there wherever it does by itself without a normalisation."""
+    rng, more = random.Random(6), 0
+    for _ in range(5000):
+        m, k, n = (int(round(2 ** rng.uniform(a, b))) for a, b in ((1, 10), (3, 14), (3, 14)))
+        for prepared in (False, True):
+            alone, behind = HipNative.q8GemmRowsTile(m, k, n, prepared=prepared), HipNative.q8GemmRowsTileBehind(m, k, n, prepared)
+            assert behind[0] or not alone[0], (m, k, n, prepared)
+            more += behind[0] > 0 and not alone[0]
+    assert more > 100 and HipNative.q8GemmRowsTileBehind(0, 64, 64) == (0, 0, 1)
+    assert HipNative.q8GemmRowsTile(64, 11008, 4096) == (0, 0, 1) and HipNative.q8GemmRowsTileBehind(64, 11008, 4096) == (32, 64, 2)
+
+
 def test_the_switch_that_keeps_every_gemm_on_k_gemm_q8():
     shapes = [(30, 2048, 6144), (64, 4096, 22016), (200, 2048, 11264), (512, 2048, 6144), (200, 768, 2304)]
     program = f"""

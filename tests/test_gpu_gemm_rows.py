@@ -316,6 +316,7 @@ def test_a_feed_forward_layer_hands_its_hidden_rows_on_in_pieces(dev, m, d, dff,
     hidden, out, last = dev.alloc(m * dff), dev.alloc(m * d), dev.alloc(m * 3 * d)
     tiles = HipNative.q8GemmRowsTile(m, d, len(ups) * dff, norm=True)
     assert tiles[0]
+    behind, by_itself = HipNative.q8GemmRowsTileBehind(m, dff, d), HipNative.q8GemmRowsTile(m, dff, d)
     first = Stream().q8_linear(xb, w1, hidden, m, d, dff, gamma=gb, bias=bb, bias2=bb if gated else -1, swiglu=gated, gelu=not gated)
     second = Stream().q8_linear(hidden, w2, out, m, dff, d, residual=xb)
     third = Stream().q8_linear(out, w3, last, m, d, 3 * d, gamma=gb)
@@ -334,6 +335,13 @@ def test_a_feed_forward_layer_hands_its_hidden_rows_on_in_pieces(dev, m, d, dff,
     layer.run()
     got = results()
     assert np.array_equal(got[0], hidden_alone)
+    # the second one runs on the kernel that it is said to take, its rows ready, and has that kernel's bits
+    launches = [int(c) for c in HipNative.profileOps(layer.array(), 2, detail=True)[2]]
+    if tiles[2] == 1 and behind[0]:
+        assert launches[1] == (1 if behind[2] == 1 else 2), (launches, behind)
+    if tiles[2] > 1 or not behind[0] or behind == by_itself:
+        second.run()
+        assert np.array_equal(dev.download(out, (m, d)), got[1])
     deq = lambda w: ref.q8_roundtrip(w).astype(np.float64)
     check(got[1], got[0].astype(np.float64) @ deq(wd) + x, dff, f"{m} x {d} over {dff}")
     check(got[2], rms_normalised(got[1].astype(np.float64), gamma) @ deq(wq), d, f"{m} x {3 * d} over {d}", times=2)      # (and the normalisation's roundings)
