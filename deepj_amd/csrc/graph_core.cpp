@@ -152,7 +152,10 @@ PyObject *tensor_new(PyTypeObject *type, PyObject *, PyObject *) {
     if (t) new (&t->tracks) std::vector<Track>();
     return reinterpret_cast<PyObject *>(t);
 }
+int tensor_traverse(Tensor *t, visitproc visit, void *arg) { Py_VISIT(t->data); Py_VISIT(t->tag); return 0; }
+int tensor_clear(Tensor *t) { Py_CLEAR(t->data); Py_CLEAR(t->tag); return 0; }
 void tensor_dealloc(Tensor *t) {
+    PyObject_GC_UnTrack(t);
     for (const Track &k : t->tracks) {
         k.graph->s->tensors[k.id] = nullptr;
         k.graph->s->maybe_orphans.push_back(k.id);
@@ -954,9 +957,11 @@ PyMODINIT_FUNC PyInit__graph_core() {
 
     TensorType.tp_name = "deepj_amd._graph_core.TensorCore";
     TensorType.tp_basicsize = sizeof(Tensor);
-    TensorType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE;
+    TensorType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE | Py_TPFLAGS_HAVE_GC;
     TensorType.tp_new = tensor_new;
     TensorType.tp_init = (initproc)tensor_init;
+    TensorType.tp_traverse = (traverseproc)tensor_traverse;
+    TensorType.tp_clear = (inquiry)tensor_clear;
     TensorType.tp_dealloc = (destructor)tensor_dealloc;
     TensorType.tp_members = tensor_members;
     TensorType.tp_getset = tensor_getset;

@@ -3,6 +3,7 @@ reference's own src/test/java/io/github/kirstenali/deepj/tensor/ComputeGraphTest
 does.  Each test cites the reference test it mirrors."""
 import gc
 import struct
+import weakref
 
 import numpy as np
 import pytest
@@ -374,6 +375,22 @@ def test_tensors_graphs_and_copies_outlive_one_another():
     for c in (copy.copy(host), copy.deepcopy(host), pickle.loads(pickle.dumps(host))):
         assert (c.rows, c.cols, c.note) == (2, 2, "kept") and np.array_equal(c.data, host.data)
     assert copy.copy(host).data is host.data and copy.deepcopy(host).data is not host.data
+
+
+@pytest.mark.parametrize("holder", ["graph", "runtime", "tensor"])
+def test_cycles_through_tensors_are_collected(holder):
+    """A graph, a runtime or a tensor that keeps a tensor of the graph's (or itself): all of it goes when the program lets go."""
+    runtime = RecordingRuntime()
+    graph = ComputeGraph(runtime)
+    t = Tensor.from2D([[1.0, 2.0]])
+    graph.ensureGpuBuffer(t)
+    graph.flush()
+    out = graph.createOutputTensor(graph.newOutputBuffer(2, 2))         # (its buffer is still to be made)
+    {"graph": graph, "runtime": runtime, "tensor": t}[holder].kept = [t, out]
+    gone = [weakref.ref(o) for o in (graph, t, out)]
+    del graph, runtime, t, out
+    gc.collect()
+    assert [r() for r in gone] == [None] * 3
 
 
 def test_values_of_other_layouts_travel_as_fp32_rows(graph, rt):
