@@ -352,7 +352,14 @@ int send_now(Graph *g, Buffer *b, Tensor *t) {
     int r = 0;
     if (v.itemsize == 4 && v.format && strcmp(v.format, "f") == 0 && v.len == t->rows * t->cols * 4) {
         const int32_t id = b->id, size = (int32_t)(t->rows * t->cols);
-        r = failed(g, g->native.alloc(&id, &size, 1)) || failed(g, g->native.upload(id, static_cast<const float *>(v.buf), size)) ? -1 : 1;
+        r = failed(g, g->native.alloc(&id, &size, 1)) ? -1 : 1;
+        if (r > 0 && failed(g, g->native.upload(id, static_cast<const float *>(v.buf), size))) {
+            PyObject *type, *value, *trace;
+            PyErr_Fetch(&type, &value, &trace);
+            (void)g->native.release(&id, 1);       // the next buffer gets this id, and may have another size
+            PyErr_Restore(type, value, trace);
+            r = -1;
+        }
         if (r > 0) b->allocated = 1;
     }
     PyBuffer_Release(&v);

@@ -1,6 +1,7 @@
 """The lazy-graph protocol without a GPU: a recording GpuRuntime logs the five calls, as the
 reference's own src/test/java/io/github/kirstenali/deepj/tensor/ComputeGraphTest.java:546-591
 does.  Each test cites the reference test it mirrors."""
+import ctypes as C
 import gc
 import struct
 import weakref
@@ -33,6 +34,60 @@ class RecordingRuntime:
 
     def flushOps(self, cmd, length):
         self.flushCalls.append((np.array(cmd[:length]).copy(), length))
+
+
+class NativeLibrary:
+    """The five calls and the error text as C functions, which a graph calls by address: what a library does with ids and sizes, the
+    calls in order, and one upload that fails when told to."""
+
+    def __init__(self):
+        ids, values = C.POINTER(C.c_int32), C.POINTER(C.c_float)
+        self.calls, self.sizes, self.held, self.fail_upload, self.during = [], {}, {}, False, None
+        self.message = C.create_string_buffer(b"the library says so")
+        self.functions = [C.CFUNCTYPE(C.c_int, ids, ids, C.c_int32)(self.alloc), C.CFUNCTYPE(C.c_int, C.c_int32, values, C.c_int64)(self.upload),
+                          C.CFUNCTYPE(C.c_int, C.c_int32, values, C.c_int64)(self.download), C.CFUNCTYPE(C.c_int, ids, C.c_int32)(self.release),
+                          C.CFUNCTYPE(C.c_int, ids, C.c_int32)(self.flush), C.CFUNCTYPE(C.c_void_p)(lambda: C.addressof(self.message))]
+
+    def graph(self):
+        class Runtime:
+            nativeCalls = staticmethod(lambda: tuple(C.cast(f, C.c_void_p).value for f in self.functions))
+            def zeroBuffers(self, buffers): raise AssertionError("not called where the library is")
+            def hostArray(self, n): return np.empty(n, np.float32)
+        return ComputeGraph(Runtime())
+
+    def log(self, name, *args):
+        self.calls.append((name, *args))
+        if self.during:
+            self.during(name)
+
+    def alloc(self, ids, sizes, n):
+        self.log("alloc", ids[:n])
+        for i, size in zip(ids[:n], sizes[:n]):
+            self.sizes.setdefault(i, size)                            # (an id that exists stays as it is)
+        return 0
+
+    def upload(self, i, values, n):
+        self.log("upload", i, n)
+        if self.fail_upload or n > self.sizes.get(i, -1):
+            return 1
+        self.held[i] = values[:n]
+        return 0
+
+    def download(self, i, out, n):
+        self.log("download", i, n)
+        for k, v in enumerate(self.held.get(i, [0.0] * n)):
+            out[k] = v
+        return 0
+
+    def release(self, ids, n):
+        self.log("release", ids[:n])
+        for i in ids[:n]:
+            self.sizes.pop(i, None)
+        return 0
+
+    def flush(self, words, n):
+        self.log("flush", words[:n])
+        return 0
 
 
 @pytest.fixture
@@ -375,6 +430,21 @@ def test_tensors_graphs_and_copies_outlive_one_another():
     for c in (copy.copy(host), copy.deepcopy(host), pickle.loads(pickle.dumps(host))):
         assert (c.rows, c.cols, c.note) == (2, 2, "kept") and np.array_equal(c.data, host.data)
     assert copy.copy(host).data is host.data and copy.deepcopy(host).data is not host.data
+
+
+def test_an_upload_that_fails_leaves_its_id_to_the_next_buffer():
+    """A large tensor's values are sent when it is first used; one that cannot be sent leaves no buffer of its size behind."""
+    lib = NativeLibrary()
+    graph = lib.graph()
+    lib.fail_upload = True
+    with pytest.raises(RuntimeError, match="the library says so"):
+        graph.ensureGpuBuffer(Tensor.from2D(np.ones((512, 512), np.float32)))
+    assert not lib.sizes
+    lib.fail_upload = False
+    t = Tensor.from2D(np.full((1024, 512), 2.0, np.float32))
+    buf = graph.ensureGpuBuffer(t)
+    graph.flush()
+    assert lib.sizes == {buf.id: t.rows * t.cols} and lib.held[buf.id][-1] == 2.0
 
 
 @pytest.mark.parametrize("holder", ["graph", "runtime", "tensor"])
