@@ -18,7 +18,9 @@
 #include <cstdlib>
 #include <cstring>
 #include <initializer_list>
+#include <mutex>
 #include <new>
+#include <string>
 #include <unordered_map>
 #include <utility>
 #include <vector>
@@ -300,11 +302,37 @@ bool direct(Graph *g) {
     PyObject **d = _PyObject_GetDictPtr(g->runtime);
     return !d || !*d || PyDict_GET_SIZE(*d) == 0;
 }
-bool failed(Graph *g, int rc) {
-    if (rc == 0) return false;
-    PyObject *text = PyUnicode_DecodeUTF8(g->native.error(), (Py_ssize_t)strlen(g->native.error()), "replace");
-    if (text) { PyErr_SetObject(PyExc_RuntimeError, text); Py_DECREF(text); }
-    return true;
+// The library's calls run one at a time, as it asks of its callers, and without the interpreter's lock, as through ctypes: an upload
+// copies its values and may wait for a full ring, a flush may grow the workspace, a download waits for the device.  Whoever is
+// about to make one holds this from before it takes out of a graph what it sends until it has noted what became of that (in the
+// same thread again where a finaliser makes another); other threads record on meanwhile.
+std::recursive_mutex g_calls;
+struct Calls {
+    Calls() {
+        if (g_calls.try_lock()) return;
+        Py_BEGIN_ALLOW_THREADS
+        g_calls.lock();
+        Py_END_ALLOW_THREADS
+    }
+    ~Calls() { g_calls.unlock(); }
+    Calls(const Calls &) = delete;
+    // Runs f, which makes calls and returns the first code that is not 0; false, with the library's text raised, if there is one.
+    template <class F> bool operator()(Graph *g, F &&f) const {
+        const Native n = g->native;
+        std::string text;
+        int rc;
+        Py_BEGIN_ALLOW_THREADS
+        rc = f(n, text);
+        Py_END_ALLOW_THREADS
+        if (rc == 0) return true;
+        PyObject *message = PyUnicode_DecodeUTF8(text.data(), (Py_ssize_t)text.size(), "replace");
+        if (message) { PyErr_SetObject(PyExc_RuntimeError, message); Py_DECREF(message); }
+        return false;
+    }
+};
+int noted(int rc, const Native &n, std::string &text) {
+    if (rc != 0) text = n.error();
+    return rc;
 }
 
 // A copy of the tensor's host values as fp32 in row order: straight where they are that already, through pack_f32 otherwise.
@@ -340,7 +368,6 @@ bool add_upload(Graph *g, int id, Tensor *t) {
     return true;
 }
 
-bool failed(Graph *g, int rc);
 // The values of a new buffer from 1 MiB on are sent as they are instead of being copied for the flush (three weights of 11 MB:
 // 7.8 ms to their first result with the copies, 1.8 without): nothing recorded refers to the buffer yet, so it does not matter when they arrive.
 // 1: sent, 0: not of that kind, -1: an error.
@@ -352,14 +379,12 @@ int send_now(Graph *g, Buffer *b, Tensor *t) {
     int r = 0;
     if (v.itemsize == 4 && v.format && strcmp(v.format, "f") == 0 && v.len == t->rows * t->cols * 4) {
         const int32_t id = b->id, size = (int32_t)(t->rows * t->cols);
-        r = failed(g, g->native.alloc(&id, &size, 1)) ? -1 : 1;
-        if (r > 0 && failed(g, g->native.upload(id, static_cast<const float *>(v.buf), size))) {
-            PyObject *type, *value, *trace;
-            PyErr_Fetch(&type, &value, &trace);
-            (void)g->native.release(&id, 1);       // the next buffer gets this id, and may have another size
-            PyErr_Restore(type, value, trace);
-            r = -1;
-        }
+        const Calls calls;
+        r = calls(g, [&](const Native &n, std::string &text) {
+            int rc = noted(n.alloc(&id, &size, 1), n, text);
+            if (rc == 0 && (rc = noted(n.upload(id, static_cast<const float *>(v.buf), size), n, text)) != 0) (void)n.release(&id, 1);
+            return rc;
+        }) ? 1 : -1;
         if (r > 0) b->allocated = 1;
     }
     PyBuffer_Release(&v);
@@ -396,10 +421,10 @@ Buffer *ensure(Graph *g, Tensor *t) {      // borrowed
     if (!fits_words(t->rows, t->cols)) return nullptr;
     Buffer *b = new_buffer(g->next_id, t->rows, t->cols, true, false, reinterpret_cast<PyObject *>(g));
     if (!b) return nullptr;
+    g->next_id++;
     Py_INCREF(b);                          // until it is the tag
     const int sent = send_now(g, b, t);
     if (sent < 0 || (sent == 0 && !add_upload(g, b->id, t))) { Py_DECREF(b); Py_DECREF(b); return nullptr; }
-    g->next_id++;
     if (sent) Py_DECREF(b);
     else g->s->allocs.push_back(b);        // (takes the reference)
     set_tag(t, reinterpret_cast<PyObject *>(b));
@@ -622,8 +647,7 @@ PyObject *graph_adamw(Graph *g, PyObject *const *v, Py_ssize_t n) {
 }
 
 // ── flush ───────────────────────────────────────────────────────────────────
-// The interpreter's lock is given up while a download waits for the device and held for the other calls, which only enqueue: a
-// flush is then one step to every other thread.
+// A runtime in Python is handed one thing after the other; the library all of it in one go (flush_native).
 PyObject *int_array(const std::vector<int32_t> &v) {       // array.array("i", v): what a runtime in Python is handed
     static PyObject *type = nullptr;
     if (!type) {
@@ -643,15 +667,11 @@ bool allocate_pending(Graph *g) {
     std::vector<int32_t> ids, sizes;
     for (Buffer *b : g->s->allocs) { ids.push_back(b->id); sizes.push_back((int32_t)(b->rows * b->cols)); }
     const size_t count = ids.size();
-    if (direct(g)) {
-        if (failed(g, g->native.alloc(ids.data(), sizes.data(), (int32_t)count))) return false;
-    } else {
-        PyObject *a = int_array(ids), *b = a ? int_array(sizes) : nullptr;
-        const bool ok = b && call(PyObject_CallMethod(g->runtime, "allocBuffers", "OOn", a, b, (Py_ssize_t)count));
-        Py_XDECREF(a);
-        Py_XDECREF(b);
-        if (!ok) return false;
-    }
+    PyObject *a = int_array(ids), *b = a ? int_array(sizes) : nullptr;
+    const bool ok = b && call(PyObject_CallMethod(g->runtime, "allocBuffers", "OOn", a, b, (Py_ssize_t)count));
+    Py_XDECREF(a);
+    Py_XDECREF(b);
+    if (!ok) return false;
     std::vector<Buffer *> done(g->s->allocs.begin(), g->s->allocs.begin() + count);
     g->s->allocs.erase(g->s->allocs.begin(), g->s->allocs.begin() + count);
     for (Buffer *b : done) { b->allocated = 1; Py_DECREF(b); }
@@ -660,22 +680,16 @@ bool allocate_pending(Graph *g) {
 bool upload_pending(Graph *g) {
     State *s = g->s;
     if (s->uploads.empty()) return true;
-    const bool native = direct(g);
     const size_t count = s->uploads.size();
-    std::vector<int32_t> fills;            // first: a buffer's zeros come before whatever else is sent to it
-    PyObject *zeros = nullptr;
+    PyObject *zeros = nullptr;             // first: a buffer's zeros come before whatever else is sent to it
     for (size_t i = 0; i < count; i++) {
         const Upload &u = s->uploads[i];
         if (u.values) continue;
-        if (native) { for (int64_t w : {(int64_t)g_fill_op, (int64_t)u.id, (int64_t)0, u.count}) fills.push_back((int32_t)w); continue; }
         if (!zeros && !(zeros = PyList_New(0))) return false;
         PyObject *pair = Py_BuildValue("(iL)", u.id, (long long)u.count);
         const bool ok = pair && PyList_Append(zeros, pair) == 0;
         Py_XDECREF(pair);
         if (!ok) { Py_DECREF(zeros); return false; }
-    }
-    if (!fills.empty()) {
-        if (failed(g, g->native.flush(fills.data(), (int32_t)fills.size()))) return false;
     }
     if (zeros) {
         const bool ok = call(PyObject_CallFunctionObjArgs(g->zero_buffers, zeros, nullptr));
@@ -685,18 +699,14 @@ bool upload_pending(Graph *g) {
     for (size_t i = 0; i < count; i++) {
         const Upload u = s->uploads[i];
         if (!u.values) continue;
-        if (native) {
-            if (failed(g, g->native.upload(u.id, u.values, u.count))) return false;
-        } else {
-            PyObject *a = PyObject_CallFunction(g_empty, "nO", (Py_ssize_t)u.count, g_float32);
-            Py_buffer v;
-            if (!a || PyObject_GetBuffer(a, &v, PyBUF_CONTIG) != 0) { Py_XDECREF(a); return false; }
-            memcpy(v.buf, u.values, v.len);
-            PyBuffer_Release(&v);
-            const bool ok = call(PyObject_CallMethod(g->runtime, "uploadBuffer", "iO", u.id, a));
-            Py_DECREF(a);
-            if (!ok) return false;
-        }
+        PyObject *a = PyObject_CallFunction(g_empty, "nO", (Py_ssize_t)u.count, g_float32);
+        Py_buffer v;
+        if (!a || PyObject_GetBuffer(a, &v, PyBUF_CONTIG) != 0) { Py_XDECREF(a); return false; }
+        memcpy(v.buf, u.values, v.len);
+        PyBuffer_Release(&v);
+        const bool ok = call(PyObject_CallMethod(g->runtime, "uploadBuffer", "iO", u.id, a));
+        Py_DECREF(a);
+        if (!ok) return false;
     }
     for (size_t i = 0; i < count; i++) free(s->uploads[i].values);
     s->uploads.erase(s->uploads.begin(), s->uploads.begin() + count);
@@ -709,14 +719,9 @@ bool execute_pending(Graph *g) {           // fails before its first launch: the
     cmd.swap(s->cmd);
     const int64_t ops = s->ops;
     s->ops = 0;
-    bool ok;
-    if (direct(g)) {
-        ok = !failed(g, g->native.flush(cmd.data(), (int32_t)cmd.size()));
-    } else {
-        PyObject *a = int_array(cmd);
-        ok = a && call(PyObject_CallMethod(g->runtime, "flushOps", "On", a, (Py_ssize_t)cmd.size()));
-        Py_XDECREF(a);
-    }
+    PyObject *a = int_array(cmd);
+    const bool ok = a && call(PyObject_CallMethod(g->runtime, "flushOps", "On", a, (Py_ssize_t)cmd.size()));
+    Py_XDECREF(a);
     if (!ok) {
         cmd.insert(cmd.end(), s->cmd.begin(), s->cmd.end());
         s->cmd.swap(cmd);
@@ -740,7 +745,8 @@ bool referenced_by_pending_ops(Graph *g, int id) {
 }
 bool release_ids(Graph *g, const std::vector<int32_t> &ids) {
     if (direct(g)) {
-        return !failed(g, g->native.release(ids.data(), (int32_t)ids.size()));
+        const Calls calls;
+        return calls(g, [&](const Native &n, std::string &text) { return noted(n.release(ids.data(), (int32_t)ids.size()), n, text); });
     }
     PyObject *a = int_array(ids);
     const bool ok = a && call(PyObject_CallMethod(g->runtime, "releaseBuffers", "On", a, (Py_ssize_t)ids.size()));
@@ -778,7 +784,60 @@ bool release_orphans(Graph *g) {
     }
     return release_ids(g, orphans);
 }
+// Taken out of the graph first, so that what other threads record meanwhile is the next flush's; what was not done goes back in front
+// of it (all uploads, where one of them failed).
+bool flush_native(Graph *g) {
+    State *s = g->s;
+    std::vector<Buffer *> allocs;
+    std::vector<Upload> uploads;
+    std::vector<int32_t> cmd, ids, sizes, fills;
+    allocs.swap(s->allocs); uploads.swap(s->uploads); cmd.swap(s->cmd);
+    const int64_t ops = s->ops;
+    s->ops = 0;
+    for (Buffer *b : allocs) { ids.push_back(b->id); sizes.push_back((int32_t)(b->rows * b->cols)); }
+    for (const Upload &u : uploads)        // (a buffer's zeros come before whatever else is sent to it)
+        if (!u.values)
+            for (int64_t w : {(int64_t)g_fill_op, (int64_t)u.id, (int64_t)0, u.count}) fills.push_back((int32_t)w);
+    bool made = false, sent = false;
+    const Calls calls;                     // (held by flush already)
+    const bool ok = calls(g, [&](const Native &n, std::string &text) {
+        int rc = 0;
+        if (!ids.empty() && (rc = noted(n.alloc(ids.data(), sizes.data(), (int32_t)ids.size()), n, text)) != 0) return rc;
+        made = true;
+        if (!fills.empty() && (rc = noted(n.flush(fills.data(), (int32_t)fills.size()), n, text)) != 0) return rc;
+        for (const Upload &u : uploads)
+            if (u.values && (rc = noted(n.upload(u.id, u.values, u.count), n, text)) != 0) return rc;
+        sent = true;
+        return ops > 0 ? noted(n.flush(cmd.data(), (int32_t)cmd.size()), n, text) : 0;
+    });
+    if (sent) {
+        for (Upload &u : uploads) free(u.values);
+    } else {
+        uploads.insert(uploads.end(), s->uploads.begin(), s->uploads.end());
+        s->uploads.swap(uploads);
+    }
+    if (!ok) {                             // fails before its first launch: the ops stay recorded
+        cmd.insert(cmd.end(), s->cmd.begin(), s->cmd.end());
+        s->cmd.swap(cmd);
+        s->ops += ops;
+    } else if (s->cmd.empty()) {           // keep the memory
+        cmd.clear();
+        s->cmd.swap(cmd);
+    }
+    if (made) {
+        for (Buffer *b : allocs) { b->allocated = 1; Py_DECREF(b); }
+    } else {
+        allocs.insert(allocs.end(), s->allocs.begin(), s->allocs.end());
+        s->allocs.swap(allocs);
+    }
+    return ok;
+}
 bool flush(Graph *g) {
+    if (direct(g)) {
+        const Calls calls;
+        if ((g->s->ops != 0 || !g->s->allocs.empty()) && !flush_native(g)) return false;
+        return release_orphans(g);
+    }
     if (g->s->ops == 0 && g->s->allocs.empty()) return release_orphans(g);
     return allocate_pending(g) && upload_pending(g) && execute_pending(g) && release_orphans(g);
 }
@@ -793,12 +852,10 @@ bool fetch(Graph *g, Buffer *b, PyObject *flat) {          // flat: contiguous f
     if (!direct(g)) return call(PyObject_CallMethod(g->runtime, "downloadBuffer", "iO", b->id, flat));
     Py_buffer v;
     if (PyObject_GetBuffer(flat, &v, PyBUF_CONTIG) != 0) return false;
-    int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = g->native.download(b->id, static_cast<float *>(v.buf), v.len / 4);
-    Py_END_ALLOW_THREADS
+    const Calls calls;
+    const bool ok = calls(g, [&](const Native &n, std::string &text) { return noted(n.download(b->id, static_cast<float *>(v.buf), v.len / 4), n, text); });
     PyBuffer_Release(&v);
-    return !failed(g, rc);
+    return ok;
 }
 bool download(Graph *g, Buffer *b, Tensor *t) {
     const Py_ssize_t count = b->rows * b->cols;

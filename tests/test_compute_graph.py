@@ -4,6 +4,9 @@ does.  Each test cites the reference test it mirrors."""
 import ctypes as C
 import gc
 import struct
+import subprocess
+import threading
+import time
 import weakref
 
 import numpy as np
@@ -445,6 +448,88 @@ def test_an_upload_that_fails_leaves_its_id_to_the_next_buffer():
     buf = graph.ensureGpuBuffer(t)
     graph.flush()
     assert lib.sizes == {buf.id: t.rows * t.cols} and lib.held[buf.id][-1] == 2.0
+
+
+BLOCKING = """
+#include <stdint.h>
+#include <unistd.h>
+volatile int block, inside, go, late, together;
+static int active;
+static int enter(int which) {
+    if (__sync_fetch_and_add(&active, 1)) together = 1;
+    if (block == which) {
+        inside = 1;
+        for (int i = 0; i < 50000 && !go; i++) usleep(100);
+        if (!go) late = 1;
+    } else usleep(block ? 0 : 20);
+    __sync_fetch_and_sub(&active, 1);
+    return 0;
+}
+int alloc(const int32_t *ids, const int32_t *sizes, int32_t n) { return enter(1); }
+int upload(int32_t id, const float *v, int64_t n) { return enter(2); }
+int flush(const int32_t *words, int32_t n) { return enter(3); }
+int release(const int32_t *ids, int32_t n) { return enter(4); }
+int download(int32_t id, float *v, int64_t n) { return enter(5); }
+const char *error(void) { return "none"; }
+"""
+CALLS = ("alloc", "upload", "flush", "release", "download", "error")
+
+
+@pytest.fixture
+def blocking(tmp_path):
+    """A library in C: no call of it needs the interpreter, and one of them waits until it is let go (5 s at most)."""
+    (tmp_path / "blocking.c").write_text(BLOCKING)
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", str(tmp_path / "blocking.so"), str(tmp_path / "blocking.c")], check=True)
+    lib = C.CDLL(str(tmp_path / "blocking.so"))
+    lib.value = {n: C.c_int.in_dll(lib, n) for n in ("block", "inside", "go", "late", "together")}
+
+    class Runtime:
+        nativeCalls = staticmethod(lambda: tuple(C.cast(getattr(lib, n), C.c_void_p).value for n in ("alloc", "upload", "download", "release", "flush", "error")))
+        def zeroBuffers(self, buffers): raise AssertionError("not called where the library is")
+        def hostArray(self, n): return np.empty(n, np.float32)
+    lib.runtime = Runtime
+    return lib
+
+
+@pytest.mark.parametrize("call", range(1, 7), ids=(*CALLS[:5], "large upload"))
+def test_other_threads_run_and_record_while_a_call_of_the_library_waits(blocking, call):
+    state, backend = blocking.value, HipBackend(blocking.runtime())
+    graph, a, b = backend.graph, Tensor.from2D([[1.0, 2.0]]), Tensor.from2D([[3.0, 4.0]])
+    backend.add(a, b)                                                  # a result nobody keeps: the flush releases it
+    kept = backend.multiply(a, b)
+    large = Tensor.from2D(np.ones((512, 1024), np.float32))
+    state["block"].value = min(call, 5) if call < 6 else 2
+    worker = threading.Thread(target=lambda: kept.materialize() if call < 6 else graph.ensureGpuBuffer(large), daemon=True)
+    Tensor.setBackend(backend)
+    worker.start()
+    until = time.monotonic() + 4
+    while not state["inside"].value and time.monotonic() < until:
+        time.sleep(0.001)
+    more = backend.subtract(a, Tensor.from2D([[5.0, 6.0]]))            # recorded meanwhile: the next flush's
+    state["go"].value = 1
+    worker.join()
+    assert state["inside"].value and not state["late"].value and not state["together"].value
+    assert not graph.isEmpty() and not more.getGpuTag().allocatedOnGpu
+    graph.flush()
+    assert graph.isEmpty() and more.getGpuTag().allocatedOnGpu
+    if call == 6:
+        assert large.getGpuTag().allocatedOnGpu
+
+
+def test_the_librarys_calls_run_one_at_a_time(blocking):
+    """It asks that of its callers; graphs of several threads keep to it."""
+    def work(backend):
+        for _ in range(30):
+            x = Tensor.from2D(np.ones((512, 512), np.float32))
+            y = backend.add(x, Tensor.from2D(np.ones((512, 512), np.float32)))
+            backend.materializeTensor(y)
+            del x, y
+    threads = [threading.Thread(target=work, args=(HipBackend(blocking.runtime()),)) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not blocking.value["together"].value
 
 
 @pytest.mark.parametrize("holder", ["graph", "runtime", "tensor"])
