@@ -22,6 +22,7 @@
 #include <new>
 #include <string>
 #include <unordered_map>
+#include <unordered_set>
 #include <utility>
 #include <vector>
 
@@ -119,6 +120,7 @@ struct State {
     int64_t ops = 0;
     std::vector<Buffer *> allocs;          // strong
     std::vector<Upload> uploads;
+    int64_t uploads_taken_out = 0;         // how often some of them were
     std::unordered_map<int, Tensor *> tensors;     // null: it has died
     std::vector<int> maybe_orphans;
 };
@@ -251,6 +253,7 @@ PyObject *graph_new(PyTypeObject *type, PyObject *, PyObject *) {
 void drop_uploads(State *s) {
     for (Upload &u : s->uploads) free(u.values);
     s->uploads.clear();
+    s->uploads_taken_out++;
 }
 void drop_allocs(State *s) {
     std::vector<Buffer *> gone;
@@ -662,54 +665,68 @@ bool call(PyObject *r) {
     Py_XDECREF(r);
     return r != nullptr;
 }
+// (A call may record and flush itself: what it has handed over then is no longer the first of what waits.)
 bool allocate_pending(Graph *g) {
-    if (g->s->allocs.empty()) return true;
-    std::vector<int32_t> ids, sizes;
-    for (Buffer *b : g->s->allocs) { ids.push_back(b->id); sizes.push_back((int32_t)(b->rows * b->cols)); }
-    const size_t count = ids.size();
-    PyObject *a = int_array(ids), *b = a ? int_array(sizes) : nullptr;
-    const bool ok = b && call(PyObject_CallMethod(g->runtime, "allocBuffers", "OOn", a, b, (Py_ssize_t)count));
-    Py_XDECREF(a);
-    Py_XDECREF(b);
-    if (!ok) return false;
-    std::vector<Buffer *> done(g->s->allocs.begin(), g->s->allocs.begin() + count);
-    g->s->allocs.erase(g->s->allocs.begin(), g->s->allocs.begin() + count);
-    for (Buffer *b : done) { b->allocated = 1; Py_DECREF(b); }
+    State *s = g->s;
+    while (!s->allocs.empty()) {
+        const std::vector<Buffer *> taken = s->allocs;
+        std::vector<int32_t> ids, sizes;
+        for (Buffer *b : taken) { Py_INCREF(b); ids.push_back(b->id); sizes.push_back((int32_t)(b->rows * b->cols)); }
+        PyObject *a = int_array(ids), *b = a ? int_array(sizes) : nullptr;
+        const bool ok = b && call(PyObject_CallMethod(g->runtime, "allocBuffers", "OOn", a, b, (Py_ssize_t)taken.size()));
+        Py_XDECREF(a);
+        Py_XDECREF(b);
+        std::vector<Buffer *> done;
+        if (ok) {
+            const std::unordered_set<Buffer *> made(taken.begin(), taken.end());
+            auto at = std::stable_partition(s->allocs.begin(), s->allocs.end(), [&](Buffer *w) { return !made.count(w); });
+            done.assign(at, s->allocs.end());
+            s->allocs.erase(at, s->allocs.end());
+            for (Buffer *w : taken) w->allocated = 1;
+        }
+        for (Buffer *w : done) Py_DECREF(w);
+        for (Buffer *w : taken) Py_DECREF(w);
+        if (!ok) return false;
+    }
     return true;
 }
 bool upload_pending(Graph *g) {
     State *s = g->s;
-    if (s->uploads.empty()) return true;
-    const size_t count = s->uploads.size();
-    PyObject *zeros = nullptr;             // first: a buffer's zeros come before whatever else is sent to it
-    for (size_t i = 0; i < count; i++) {
-        const Upload &u = s->uploads[i];
-        if (u.values) continue;
-        if (!zeros && !(zeros = PyList_New(0))) return false;
-        PyObject *pair = Py_BuildValue("(iL)", u.id, (long long)u.count);
-        const bool ok = pair && PyList_Append(zeros, pair) == 0;
-        Py_XDECREF(pair);
-        if (!ok) { Py_DECREF(zeros); return false; }
+    while (!s->uploads.empty()) {
+        const size_t count = s->uploads.size();
+        const int64_t taken_out = s->uploads_taken_out;        // (other: an inner flush has sent them)
+        PyObject *zeros = nullptr;                             // first: a buffer's zeros come before whatever else is sent to it
+        for (size_t i = 0; i < count && s->uploads_taken_out == taken_out; i++) {
+            const Upload u = s->uploads[i];
+            if (u.values) continue;
+            if (!zeros && !(zeros = PyList_New(0))) return false;
+            PyObject *pair = Py_BuildValue("(iL)", u.id, (long long)u.count);
+            const bool ok = pair && PyList_Append(zeros, pair) == 0;
+            Py_XDECREF(pair);
+            if (!ok) { Py_DECREF(zeros); return false; }
+        }
+        if (zeros) {
+            const bool ok = call(PyObject_CallFunctionObjArgs(g->zero_buffers, zeros, nullptr));
+            Py_DECREF(zeros);
+            if (!ok) return false;
+        }
+        for (size_t i = 0; i < count && s->uploads_taken_out == taken_out; i++) {
+            const Upload u = s->uploads[i];
+            if (!u.values) continue;
+            PyObject *a = PyObject_CallFunction(g_empty, "nO", (Py_ssize_t)u.count, g_float32);
+            Py_buffer v;
+            if (!a || PyObject_GetBuffer(a, &v, PyBUF_CONTIG) != 0) { Py_XDECREF(a); return false; }
+            if (s->uploads_taken_out == taken_out) memcpy(v.buf, u.values, v.len);
+            PyBuffer_Release(&v);
+            const bool ok = s->uploads_taken_out != taken_out || call(PyObject_CallMethod(g->runtime, "uploadBuffer", "iO", u.id, a));
+            Py_DECREF(a);
+            if (!ok) return false;
+        }
+        if (s->uploads_taken_out != taken_out) continue;
+        for (size_t i = 0; i < count; i++) free(s->uploads[i].values);
+        s->uploads.erase(s->uploads.begin(), s->uploads.begin() + count);
+        s->uploads_taken_out++;
     }
-    if (zeros) {
-        const bool ok = call(PyObject_CallFunctionObjArgs(g->zero_buffers, zeros, nullptr));
-        Py_DECREF(zeros);
-        if (!ok) return false;
-    }
-    for (size_t i = 0; i < count; i++) {
-        const Upload u = s->uploads[i];
-        if (!u.values) continue;
-        PyObject *a = PyObject_CallFunction(g_empty, "nO", (Py_ssize_t)u.count, g_float32);
-        Py_buffer v;
-        if (!a || PyObject_GetBuffer(a, &v, PyBUF_CONTIG) != 0) { Py_XDECREF(a); return false; }
-        memcpy(v.buf, u.values, v.len);
-        PyBuffer_Release(&v);
-        const bool ok = call(PyObject_CallMethod(g->runtime, "uploadBuffer", "iO", u.id, a));
-        Py_DECREF(a);
-        if (!ok) return false;
-    }
-    for (size_t i = 0; i < count; i++) free(s->uploads[i].values);
-    s->uploads.erase(s->uploads.begin(), s->uploads.begin() + count);
     return true;
 }
 bool execute_pending(Graph *g) {           // fails before its first launch: the ops stay recorded
@@ -780,6 +797,7 @@ bool release_orphans(Graph *g) {
         auto at = s->uploads.begin();
         for (Upload &u : s->uploads) if (gone(u.id)) free(u.values); else *at++ = u;
         s->uploads.erase(at, s->uploads.end());
+        s->uploads_taken_out++;
         for (Buffer *b : dropped) Py_DECREF(b);
     }
     return release_ids(g, orphans);

@@ -435,6 +435,37 @@ def test_tensors_graphs_and_copies_outlive_one_another():
     assert copy.copy(host).data is host.data and copy.deepcopy(host).data is not host.data
 
 
+@pytest.mark.parametrize("call", ["allocBuffers", "uploadBuffer", "flushOps", "releaseBuffers", "zeroBuffers"])
+def test_a_runtime_may_flush_from_inside_a_call(call):
+    """A runtime in Python that reads a tensor (and so flushes) while it is handed things: each thing is handed over, and nothing twice
+    beside what the inner flush was handed again."""
+    class Clearing(RecordingRuntime):
+        def __init__(self):
+            super().__init__()
+            self.zeros = []
+
+        def zeroBuffers(self, buffers):
+            self.zeros.append(list(buffers))
+
+    rt = Clearing()
+    backend, depth = HipBackend(rt), [0]
+    plain = getattr(rt, call)
+
+    def again(*args):
+        plain(*args)
+        if depth[0] < 2:
+            depth[0] += 1
+            for k in range(20):                                        # (more of everything than the outer call holds)
+                backend.add(Tensor.from2D([[1.0 + k]]), Tensor(1, 1))
+            backend.graph.flush()
+    setattr(rt, call, again)
+    for round in range(3):
+        kept = [backend.add(Tensor.from2D([[1.0, float(k)]]), Tensor(1, 2)) for k in range(30)]
+        backend.graph.flush()
+    assert backend.graph.isEmpty() and all(t.getGpuTag().allocatedOnGpu for t in kept)
+    backend.releaseResources()
+
+
 def test_an_upload_that_fails_leaves_its_id_to_the_next_buffer():
     """A large tensor's values are sent when it is first used; one that cannot be sent leaves no buffer of its size behind."""
     lib = NativeLibrary()
