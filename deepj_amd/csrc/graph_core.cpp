@@ -405,8 +405,18 @@ bool fits_words(Py_ssize_t rows, Py_ssize_t cols) {
     PyErr_Format(PyExc_OverflowError, "a buffer of %zdx%zd: more than 32 bits count", rows, cols);
     return false;
 }
-Buffer *ensure(Graph *g, Tensor *t) {      // borrowed
+// A buffer held through what may run meanwhile: another thread while values are sent, a host array of some other class.
+struct Held {
+    Buffer *b;
+    explicit Held(Buffer *taken) : b(taken) {}             // takes the caller's reference
+    ~Held() { Py_XDECREF(b); }
+    Held(const Held &) = delete;
+    Buffer *operator->() const { return b; }
+    explicit operator bool() const { return b != nullptr; }
+};
+Buffer *ensure(Graph *g, Tensor *t) {      // a reference of the caller's
     if (Buffer *b = tag_of(t)) {
+        Py_INCREF(b);
         auto it = g->s->tensors.find(b->id);
         if (it == g->s->tensors.end() || it->second != t) {
             track(g, b->id, t);
@@ -414,8 +424,9 @@ Buffer *ensure(Graph *g, Tensor *t) {      // borrowed
             Py_XSETREF(b->graph, reinterpret_cast<PyObject *>(g));
         }
         if (b->needs_upload) {
-            if (!has_data(t)) { PyObject *d = tensor_data(t, nullptr); if (!d) return nullptr; Py_DECREF(d); }
-            if (!add_upload(g, b->id, t)) return nullptr;
+            PyObject *d = has_data(t) ? nullptr : tensor_data(t, nullptr);
+            Py_XDECREF(d);
+            if (!has_data(t) || !add_upload(g, b->id, t)) { Py_DECREF(b); return nullptr; }
             b->needs_upload = 0;
             b->cpu_stale = 0;
         }
@@ -425,14 +436,13 @@ Buffer *ensure(Graph *g, Tensor *t) {      // borrowed
     Buffer *b = new_buffer(g->next_id, t->rows, t->cols, true, false, reinterpret_cast<PyObject *>(g));
     if (!b) return nullptr;
     g->next_id++;
-    Py_INCREF(b);                          // until it is the tag
+    Py_INCREF(b);                          // (two: the caller's, and the list's of what is to be made)
     const int sent = send_now(g, b, t);
     if (sent < 0 || (sent == 0 && !add_upload(g, b->id, t))) { Py_DECREF(b); Py_DECREF(b); return nullptr; }
     if (sent) Py_DECREF(b);
     else g->s->allocs.push_back(b);        // (takes the reference)
     set_tag(t, reinterpret_cast<PyObject *>(b));
     track(g, b->id, t);
-    Py_DECREF(b);
     return b;
 }
 Buffer *new_output(Graph *g, Py_ssize_t rows, Py_ssize_t cols) {       // a reference of the caller's
@@ -494,9 +504,7 @@ bool arity(Py_ssize_t n, Py_ssize_t want) {
 
 PyObject *graph_ensure(Graph *g, PyObject *o) {
     Tensor *t = as_tensor(o);
-    Buffer *b = t ? ensure(g, t) : nullptr;
-    Py_XINCREF(b);
-    return reinterpret_cast<PyObject *>(b);
+    return reinterpret_cast<PyObject *>(t ? ensure(g, t) : nullptr);
 }
 PyObject *graph_new_output(Graph *g, PyObject *const *a, Py_ssize_t n) {
     int64_t r, c;
@@ -551,7 +559,8 @@ PyObject *graph_binary(Graph *g, PyObject *const *v, Py_ssize_t n) {
     if (!arity(n, 5) || !read_int(v[0], op)) return nullptr;
     Tensor *a = as_tensor(v[2]), *b = a ? as_tensor(v[3]) : nullptr;
     if (!b || !same_shape(a, b, v[1])) return nullptr;
-    Buffer *ga = ensure(g, a), *gb = ga ? ensure(g, b) : nullptr, *out = gb ? new_output(g, a->rows, a->cols) : nullptr;
+    const Held ga(ensure(g, a)), gb(ga ? ensure(g, b) : nullptr);
+    Buffer *out = gb ? new_output(g, a->rows, a->cols) : nullptr;
     if (!out) return nullptr;
     emit(g, {op, ga->id, gb->id, out->id, out->rows * out->cols});
     return finish(g, out, v[4] == Py_True ? v[2] : nullptr);
@@ -561,7 +570,8 @@ PyObject *graph_unary(Graph *g, PyObject *const *v, Py_ssize_t n) {
     int64_t op;
     if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
     Tensor *a = as_tensor(v[1]);
-    Buffer *ga = a ? ensure(g, a) : nullptr, *out = ga ? new_output(g, a->rows, a->cols) : nullptr;
+    const Held ga(a ? ensure(g, a) : nullptr);
+    Buffer *out = ga ? new_output(g, a->rows, a->cols) : nullptr;
     if (!out) return nullptr;
     emit(g, {op, ga->id, out->id, out->rows * out->cols});
     return finish(g, out, v[2] == Py_True ? v[1] : nullptr);
@@ -572,7 +582,8 @@ PyObject *graph_scalar(Graph *g, PyObject *const *v, Py_ssize_t n) {
     int32_t bits;
     if (!arity(n, 4) || !read_int(v[0], op) || !read_float_bits(v[2], bits)) return nullptr;
     Tensor *a = as_tensor(v[1]);
-    Buffer *ga = a ? ensure(g, a) : nullptr, *out = ga ? new_output(g, a->rows, a->cols) : nullptr;
+    const Held ga(a ? ensure(g, a) : nullptr);
+    Buffer *out = ga ? new_output(g, a->rows, a->cols) : nullptr;
     if (!out) return nullptr;
     emit(g, {op, ga->id, out->id, bits, out->rows * out->cols});
     return finish(g, out, v[3] == Py_True ? v[1] : nullptr);
@@ -582,13 +593,15 @@ PyObject *graph_shaped(Graph *g, PyObject *const *v, Py_ssize_t n) {
     int64_t op, rows, cols;
     if (!arity(n, 4) || !read_int(v[0], op) || !read_int(v[2], rows) || !read_int(v[3], cols)) return nullptr;
     Tensor *a = as_tensor(v[1]);
-    Buffer *ga = a ? ensure(g, a) : nullptr, *out = ga ? new_output(g, rows, cols) : nullptr;
+    const Held ga(a ? ensure(g, a) : nullptr);
+    Buffer *out = ga ? new_output(g, rows, cols) : nullptr;
     if (!out) return nullptr;
     emit(g, {op, ga->id, out->id, a->rows, a->cols});
     return finish(g, out, nullptr);
 }
 PyObject *two_shaped(Graph *g, int64_t op, Tensor *a, Tensor *b) {     // out like a; a's rows and columns
-    Buffer *ga = ensure(g, a), *gb = ga ? ensure(g, b) : nullptr, *out = gb ? new_output(g, a->rows, a->cols) : nullptr;
+    const Held ga(ensure(g, a)), gb(ga ? ensure(g, b) : nullptr);
+    Buffer *out = gb ? new_output(g, a->rows, a->cols) : nullptr;
     if (!out) return nullptr;
     emit(g, {op, ga->id, gb->id, out->id, a->rows, a->cols});
     return finish(g, out, nullptr);
@@ -625,7 +638,8 @@ PyObject *graph_matmul(Graph *g, PyObject *const *v, Py_ssize_t n) {
     Tensor *a = as_tensor(v[1]), *b = a ? as_tensor(v[2]) : nullptr;
     if (!b) return nullptr;
     if (a->cols != b->rows) return PyErr_Format(PyExc_ValueError, "Shape mismatch for matmul: %zdx%zd vs %zdx%zd", a->rows, a->cols, b->rows, b->cols);
-    Buffer *ga = ensure(g, a), *gb = ga ? ensure(g, b) : nullptr, *out = gb ? new_output(g, a->rows, b->cols) : nullptr;
+    const Held ga(ensure(g, a)), gb(ga ? ensure(g, b) : nullptr);
+    Buffer *out = gb ? new_output(g, a->rows, b->cols) : nullptr;
     if (!out) return nullptr;
     emit(g, {op, ga->id, gb->id, out->id, a->rows, b->cols, a->cols});
     return finish(g, out, nullptr);
@@ -635,17 +649,15 @@ PyObject *graph_adamw(Graph *g, PyObject *const *v, Py_ssize_t n) {
     int64_t op;
     int32_t bits[7];
     if (!arity(n, 12) || !read_int(v[0], op)) return nullptr;
-    Buffer *b[4];
-    Tensor *w = nullptr;
-    for (int i = 0; i < 4; i++) {
-        Tensor *t = as_tensor(v[1 + i]);
-        if (!t || !(b[i] = ensure(g, t))) return nullptr;
-        if (i == 0) w = t;
-    }
+    Tensor *t[4];
+    for (int i = 0; i < 4; i++)
+        if (!(t[i] = as_tensor(v[1 + i]))) return nullptr;
+    const Held w(ensure(g, t[0])), gw(w ? ensure(g, t[1]) : nullptr), mt(gw ? ensure(g, t[2]) : nullptr), vt(mt ? ensure(g, t[3]) : nullptr);
+    if (!vt) return nullptr;
     for (int i = 0; i < 7; i++)
         if (!read_float_bits(v[5 + i], bits[i])) return nullptr;
-    emit(g, {op, b[0]->id, b[1]->id, b[2]->id, b[3]->id, bits[0], bits[1], bits[2], bits[3], bits[4], bits[5], bits[6], w->rows * w->cols});
-    for (int i : {0, 2, 3}) { b[i]->cpu_stale = 1; b[i]->needs_upload = 0; }
+    emit(g, {op, w->id, gw->id, mt->id, vt->id, bits[0], bits[1], bits[2], bits[3], bits[4], bits[5], bits[6], t[0]->rows * t[0]->cols});
+    for (Buffer *b : {w.b, mt.b, vt.b}) { b->cpu_stale = 1; b->needs_upload = 0; }
     Py_RETURN_NONE;
 }
 

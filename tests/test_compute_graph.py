@@ -547,6 +547,27 @@ def test_other_threads_run_and_record_while_a_call_of_the_library_waits(blocking
         assert large.getGpuTag().allocatedOnGpu
 
 
+def test_an_operand_may_get_another_buffer_while_the_other_ones_values_are_sent():
+    """A host array of some other class runs code of its own when it is packed; here it takes the other operand's buffer away."""
+    runtime = RecordingRuntime()
+    backend = HipBackend(runtime)
+    a, b = Tensor.from2D([[1.0, 2.0]]), Tensor(1, 2)
+
+    class Taking:
+        def astype(self, dtype, order):
+            a.setGpuTag(None)
+            gc.collect()
+            [GpuBuffer(100 + k, 7, 7, False) for k in range(64)]       # (what may get the memory)
+            return np.array([[3.0, 4.0]], np.float32)
+    b._data = Taking()
+    first = backend.graph.ensureGpuBuffer(a).id
+    backend.graph.flush()                                              # (what waits to be made would hold it)
+    out = backend.add(a, b)
+    backend.graph.flush()
+    words = [list(c[0]) for c in runtime.flushCalls]
+    assert words == [[op.OP_ADD, first, b.getGpuTag().id, out.getGpuTag().id, 2]]
+
+
 def test_the_librarys_calls_run_one_at_a_time(blocking):
     """It asks that of its callers; graphs of several threads keep to it."""
     def work(backend):
