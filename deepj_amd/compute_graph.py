@@ -141,6 +141,105 @@ class ComputeGraph(_graph_core.GraphCore):
                    float_bits(beta2), float_bits(eps), float_bits(weight_decay), float_bits(bc1), float_bits(bc2), n)
 
 
+# What the operations of HipBackend record, through the graph's methods: csrc/graph_core.cpp does the same for tensors on a graph
+# whose methods are ComputeGraph's, and calls these for everything else.
+def _result(graph, out, into=None):
+    return graph.createOutputTensor(out) if into is None else graph.bindTensorToBuffer(into, out)
+
+
+def _binary(graph, opcode, name, a, b, in_place):
+    if a.rows != b.rows or a.cols != b.cols:
+        raise ValueError(f"Shape mismatch for {name}: {a.rows}x{a.cols} vs {b.rows}x{b.cols}")
+    ga, gb = graph.ensureGpuBuffer(a), graph.ensureGpuBuffer(b)
+    out = graph.newOutputBuffer(a.rows, a.cols)
+    graph.recordBinary(opcode, ga, gb, out)
+    return _result(graph, out, a if in_place else None)
+
+
+def _unary(graph, opcode, a, in_place):
+    ga = graph.ensureGpuBuffer(a)
+    out = graph.newOutputBuffer(a.rows, a.cols)
+    graph.recordUnary(opcode, ga, out)
+    return _result(graph, out, a if in_place else None)
+
+
+def _scalar(graph, opcode, a, value, in_place):
+    ga = graph.ensureGpuBuffer(a)
+    out = graph.newOutputBuffer(a.rows, a.cols)
+    if opcode == op.OP_MULTIPLY_SCALAR:
+        graph.recordMultiplyScalar(ga, out, value)
+    elif opcode == op.OP_POW:
+        graph.recordPow(ga, out, value)
+    else:
+        graph.recordScalarUnary(opcode, ga, out, value)
+    return _result(graph, out, a if in_place else None)
+
+
+_SHAPED = {op.OP_TRANSPOSE: "recordTranspose", op.OP_SOFTMAX_ROWS: "recordSoftmaxRows", op.OP_SUM_SCALAR: "recordSumScalar",
+           op.OP_SUM_ABS: "recordSumAbs"}
+_PAIRS = {op.OP_SOFTMAX_BACKWARD: "recordSoftmaxBackward", op.OP_CROSS_ENTROPY_GRADIENT: "recordCrossEntropyGradient"}
+
+
+def _shaped(graph, opcode, a, rows, cols):
+    ga = graph.ensureGpuBuffer(a)
+    out = graph.newOutputBuffer(rows, cols)
+    if opcode in _SHAPED:
+        getattr(graph, _SHAPED[opcode])(ga, out, a.rows, a.cols)
+    else:
+        graph.recordReduction(opcode, ga, out, a.rows, a.cols)
+    return _result(graph, out)
+
+
+def _pair(graph, opcode, a, b):
+    ga, gb = graph.ensureGpuBuffer(a), graph.ensureGpuBuffer(b)
+    out = graph.newOutputBuffer(a.rows, a.cols)
+    getattr(graph, _PAIRS[opcode])(ga, gb, out, a.rows, a.cols)
+    return _result(graph, out)
+
+
+def _row_broadcast(graph, opcode, a, v):
+    if v.rows != 1 or v.cols != a.cols:
+        raise ValueError(f"Expected row vector 1x{a.cols} but got {v.rows}x{v.cols}")
+    ga, gv = graph.ensureGpuBuffer(a), graph.ensureGpuBuffer(v)
+    out = graph.newOutputBuffer(a.rows, a.cols)
+    graph.recordRowBroadcast(opcode, ga, gv, out, a.rows, a.cols)
+    return _result(graph, out)
+
+
+def _col_broadcast(graph, opcode, a, v):
+    if v.rows != a.rows or v.cols != 1:
+        raise ValueError(f"Expected col vector {a.rows}x1 but got {v.rows}x{v.cols}")
+    ga, gv = graph.ensureGpuBuffer(a), graph.ensureGpuBuffer(v)
+    out = graph.newOutputBuffer(a.rows, a.cols)
+    graph.recordColBroadcast(opcode, ga, gv, out, a.rows, a.cols)
+    return _result(graph, out)
+
+
+def _matmul(graph, opcode, a, b):
+    if a.cols != b.rows:
+        raise ValueError(f"Shape mismatch for matmul: {a.rows}x{a.cols} vs {b.rows}x{b.cols}")
+    ga, gb = graph.ensureGpuBuffer(a), graph.ensureGpuBuffer(b)
+    out = graph.newOutputBuffer(a.rows, b.cols)
+    graph.recordMatmul(ga, gb, out, a.rows, b.cols, a.cols)
+    return _result(graph, out)
+
+
+def _adamw(graph, opcode, w, g, mt, vt, lr, beta1, beta2, eps, weight_decay, bc1, bc2):
+    gw, gg, gm, gv = (graph.ensureGpuBuffer(t) for t in (w, g, mt, vt))
+    graph.recordAdamWUpdate(gw, gg, gm, gv, lr, beta1, beta2, eps, weight_decay, bc1, bc2, w.rows * w.cols)
+    for b in (gw, gm, gv):
+        b.cpuStale = True
+        b.needsUpload = False
+
+
+_graph_core.set_methods(
+    {"binary": _binary, "unary": _unary, "scalar": _scalar, "shaped": _shaped, "pair": _pair, "rowBroadcast": _row_broadcast,
+     "colBroadcast": _col_broadcast, "matmul": _matmul, "adamW": _adamw}, ComputeGraph,
+    ["ensureGpuBuffer", "newOutputBuffer", "createOutputTensor", "bindTensorToBuffer", "flush", "_emit", "recordBinary", "recordUnary",
+     "recordMultiplyScalar", "recordPow", "recordScalarUnary", "recordReduction", "recordRowBroadcast", "recordColBroadcast", "recordMatmul",
+     "recordAdamWUpdate", *_SHAPED.values(), *_PAIRS.values()])
+
+
 # TensorAdapters.java:9-47
 def pack_f32(t) -> np.ndarray:
     return t.data.astype(np.float32, order="C").reshape(-1)          # a copy: the tensor may change before the flush

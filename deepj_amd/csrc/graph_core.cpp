@@ -300,8 +300,42 @@ int graph_init(Graph *g, PyObject *args, PyObject *) {
     }
     return 0;
 }
+struct Methods {                           // attributes of a class as they were, and whether some class still has them
+    std::vector<std::pair<PyObject *, PyObject *>> of;
+    PyTypeObject *seen = nullptr;
+    unsigned seen_tag = 0;
+    bool seen_same = false;
+    bool take(PyTypeObject *type, PyObject *names) {
+        PyObject *list = PySequence_Tuple(names);
+        if (!list) return false;
+        for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(list); i++) {
+            PyObject *name = PyTuple_GET_ITEM(list, i), *value = _PyType_Lookup(type, name);
+            if (!value) { PyErr_SetObject(PyExc_AttributeError, name); Py_DECREF(list); return false; }
+            Py_INCREF(name);
+            Py_INCREF(value);
+            of.emplace_back(name, value);
+        }
+        Py_DECREF(list);
+        return true;
+    }
+    bool same(PyTypeObject *type) {        // (a class's version changes with it and with its bases)
+        if (type == seen && PyType_HasFeature(type, Py_TPFLAGS_VALID_VERSION_TAG) && type->tp_version_tag == seen_tag) return seen_same;
+        bool all = !of.empty();
+        for (const auto &m : of) all = all && _PyType_Lookup(type, m.first) == m.second;
+        seen = type;
+        seen_tag = type->tp_version_tag;
+        seen_same = all;
+        return all;
+    }
+};
+Methods g_graph_methods, g_runtime_methods, g_native_methods;
+PyTypeObject *g_runtime_class, *g_native_class;                    // deepj_amd.HipGpuRuntime, HipNative
+PyObject *g_general;                       // compute_graph.py's {name: function of the graph}
+
+// Whether the graph makes the library's calls itself: not where something was put in place of a method that would make them.
 bool direct(Graph *g) {
     if (!g->native_type || Py_TYPE(g->runtime) != g->native_type) return false;
+    if (g->native_type == g_runtime_class && !(g_runtime_methods.same(g_runtime_class) && g_native_methods.same(g_native_class))) return false;
     PyObject **d = _PyObject_GetDictPtr(g->runtime);
     return !d || !*d || PyDict_GET_SIZE(*d) == 0;
 }
@@ -405,6 +439,14 @@ bool fits_words(Py_ssize_t rows, Py_ssize_t cols) {
     PyErr_Format(PyExc_OverflowError, "a buffer of %zdx%zd: more than 32 bits count", rows, cols);
     return false;
 }
+// setGpuTag, the class's own where it has one
+bool retag(Tensor *t, PyObject *tag) {
+    static PyObject *name = PyUnicode_InternFromString("setGpuTag"), *own = PyDict_GetItem(TensorType.tp_dict, name);
+    if (_PyType_Lookup(Py_TYPE(t), name) == own) { set_tag(t, tag); return true; }
+    PyObject *r = PyObject_CallMethodObjArgs(reinterpret_cast<PyObject *>(t), name, tag, nullptr);
+    Py_XDECREF(r);
+    return r != nullptr;
+}
 // A buffer held through what may run meanwhile: another thread while values are sent, a host array of some other class.
 struct Held {
     Buffer *b;
@@ -441,7 +483,7 @@ Buffer *ensure(Graph *g, Tensor *t) {      // a reference of the caller's
     if (sent < 0 || (sent == 0 && !add_upload(g, b->id, t))) { Py_DECREF(b); Py_DECREF(b); return nullptr; }
     if (sent) Py_DECREF(b);
     else g->s->allocs.push_back(b);        // (takes the reference)
-    set_tag(t, reinterpret_cast<PyObject *>(b));
+    if (!retag(t, reinterpret_cast<PyObject *>(b))) { Py_DECREF(b); return nullptr; }
     track(g, b->id, t);
     return b;
 }
@@ -467,17 +509,18 @@ PyObject *output_tensor(Graph *g, Buffer *b) {
     Py_XSETREF(b->graph, reinterpret_cast<PyObject *>(g));
     return o;
 }
-void bind(Graph *g, Tensor *t, Buffer *b) {
-    set_tag(t, reinterpret_cast<PyObject *>(b));
+bool bind(Graph *g, Tensor *t, Buffer *b) {
+    if (!retag(t, reinterpret_cast<PyObject *>(b))) return false;
     track(g, b->id, t);
     Py_INCREF(g);
     Py_XSETREF(b->graph, reinterpret_cast<PyObject *>(g));
+    return true;
 }
 // The result of a recorded operation: a new tensor, or `into` on its new buffer.  Takes the caller's reference to out.
-PyObject *finish(Graph *g, Buffer *out, PyObject *into) {
+PyObject *finish(Graph *g, Buffer *out, Tensor *into) {
     PyObject *r;
-    if (into) { bind(g, reinterpret_cast<Tensor *>(into), out); r = Py_None; Py_INCREF(r); }
-    else r = output_tensor(g, out);
+    if (!into) r = output_tensor(g, out);
+    else if ((r = bind(g, into, out) ? Py_None : nullptr)) Py_INCREF(r);
     Py_DECREF(out);
     return r;
 }
@@ -525,7 +568,7 @@ PyObject *graph_bind(Graph *g, PyObject *const *a, Py_ssize_t n) {
     Tensor *t = as_tensor(a[0]);
     Buffer *b = t ? as_buffer(a[1]) : nullptr;
     if (!b) return nullptr;
-    bind(g, t, b);
+    if (!bind(g, t, b)) return nullptr;
     Py_RETURN_NONE;
 }
 PyObject *graph_let_go(Graph *g, PyObject *o) {
@@ -548,52 +591,73 @@ PyObject *graph_emit(Graph *g, PyObject *const *a, Py_ssize_t n) {     // one op
 }
 
 // ── operations of the backend: check, inputs, output, words ─────────────────
-bool same_shape(Tensor *a, Tensor *b, PyObject *name) {
-    if (a->rows == b->rows && a->cols == b->cols) return true;
-    PyErr_Format(PyExc_ValueError, "Shape mismatch for %U: %zdx%zd vs %zdx%zd", name, a->rows, a->cols, b->rows, b->cols);
-    return false;
+// They go past the graph's own methods, so only where those are ComputeGraph's and the operands tensors; everything else - a class
+// derived from it, a method replaced, an object that stands in for a graph or a tensor - takes the way through the methods
+// (compute_graph.py).
+Graph *plain_graph(PyObject *o) {
+    if (!PyObject_TypeCheck(o, &GraphType) || !g_graph_methods.same(Py_TYPE(o))) return nullptr;
+    PyObject **d = _PyObject_GetDictPtr(o);
+    if (d && *d && PyDict_GET_SIZE(*d) > 0)
+        for (const auto &m : g_graph_methods.of)
+            if (PyDict_Contains(*d, m.first) != 0) { PyErr_Clear(); return nullptr; }
+    return reinterpret_cast<Graph *>(o);
 }
-// (opcode, name, a, b, in place)
-PyObject *graph_binary(Graph *g, PyObject *const *v, Py_ssize_t n) {
+Tensor *tensor(PyObject *o) { return PyObject_TypeCheck(o, &TensorType) ? reinterpret_cast<Tensor *>(o) : nullptr; }
+PyObject *general(const char *name, PyObject *const *v, Py_ssize_t n) {
+    PyObject *f = g_general ? PyDict_GetItemString(g_general, name) : nullptr;
+    if (!f) return PyErr_Format(PyExc_RuntimeError, "no function for %s", name);
+    return PyObject_Vectorcall(f, v, (size_t)n, nullptr);
+}
+
+// (graph, opcode, name, a, b, in place)
+PyObject *record_binary(PyObject *, PyObject *const *v, Py_ssize_t n) {
     int64_t op;
-    if (!arity(n, 5) || !read_int(v[0], op)) return nullptr;
-    Tensor *a = as_tensor(v[2]), *b = a ? as_tensor(v[3]) : nullptr;
-    if (!b || !same_shape(a, b, v[1])) return nullptr;
+    Graph *g = n == 6 ? plain_graph(v[0]) : nullptr;
+    Tensor *a = g ? tensor(v[3]) : nullptr, *b = a ? tensor(v[4]) : nullptr;
+    if (!b) return general("binary", v, n);
+    if (!read_int(v[1], op)) return nullptr;
+    if (a->rows != b->rows || a->cols != b->cols) return PyErr_Format(PyExc_ValueError, "Shape mismatch for %U: %zdx%zd vs %zdx%zd", v[2], a->rows, a->cols, b->rows, b->cols);
     const Held ga(ensure(g, a)), gb(ga ? ensure(g, b) : nullptr);
     Buffer *out = gb ? new_output(g, a->rows, a->cols) : nullptr;
     if (!out) return nullptr;
     emit(g, {op, ga->id, gb->id, out->id, out->rows * out->cols});
-    return finish(g, out, v[4] == Py_True ? v[2] : nullptr);
+    return finish(g, out, v[5] == Py_True ? a : nullptr);
 }
-// (opcode, a, in place)
-PyObject *graph_unary(Graph *g, PyObject *const *v, Py_ssize_t n) {
+// (graph, opcode, a, in place)
+PyObject *record_unary(PyObject *, PyObject *const *v, Py_ssize_t n) {
     int64_t op;
-    if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
-    Tensor *a = as_tensor(v[1]);
-    const Held ga(a ? ensure(g, a) : nullptr);
+    Graph *g = n == 4 ? plain_graph(v[0]) : nullptr;
+    Tensor *a = g ? tensor(v[2]) : nullptr;
+    if (!a) return general("unary", v, n);
+    if (!read_int(v[1], op)) return nullptr;
+    const Held ga(ensure(g, a));
     Buffer *out = ga ? new_output(g, a->rows, a->cols) : nullptr;
     if (!out) return nullptr;
     emit(g, {op, ga->id, out->id, out->rows * out->cols});
-    return finish(g, out, v[2] == Py_True ? v[1] : nullptr);
+    return finish(g, out, v[3] == Py_True ? a : nullptr);
 }
-// (opcode, a, scalar, in place)
-PyObject *graph_scalar(Graph *g, PyObject *const *v, Py_ssize_t n) {
+// (graph, opcode, a, scalar, in place)
+PyObject *record_scalar(PyObject *, PyObject *const *v, Py_ssize_t n) {
     int64_t op;
     int32_t bits;
-    if (!arity(n, 4) || !read_int(v[0], op) || !read_float_bits(v[2], bits)) return nullptr;
-    Tensor *a = as_tensor(v[1]);
-    const Held ga(a ? ensure(g, a) : nullptr);
+    Graph *g = n == 5 ? plain_graph(v[0]) : nullptr;
+    Tensor *a = g ? tensor(v[2]) : nullptr;
+    if (!a) return general("scalar", v, n);
+    if (!read_int(v[1], op) || !read_float_bits(v[3], bits)) return nullptr;
+    const Held ga(ensure(g, a));
     Buffer *out = ga ? new_output(g, a->rows, a->cols) : nullptr;
     if (!out) return nullptr;
     emit(g, {op, ga->id, out->id, bits, out->rows * out->cols});
-    return finish(g, out, v[3] == Py_True ? v[1] : nullptr);
+    return finish(g, out, v[4] == Py_True ? a : nullptr);
 }
-// (opcode, a, output rows, output columns): an operation whose words end with the input's rows and columns
-PyObject *graph_shaped(Graph *g, PyObject *const *v, Py_ssize_t n) {
+// (graph, opcode, a, output rows, output columns): an operation whose words end with the input's rows and columns
+PyObject *record_shaped(PyObject *, PyObject *const *v, Py_ssize_t n) {
     int64_t op, rows, cols;
-    if (!arity(n, 4) || !read_int(v[0], op) || !read_int(v[2], rows) || !read_int(v[3], cols)) return nullptr;
-    Tensor *a = as_tensor(v[1]);
-    const Held ga(a ? ensure(g, a) : nullptr);
+    Graph *g = n == 5 ? plain_graph(v[0]) : nullptr;
+    Tensor *a = g ? tensor(v[2]) : nullptr;
+    if (!a) return general("shaped", v, n);
+    if (!read_int(v[1], op) || !read_int(v[3], rows) || !read_int(v[4], cols)) return nullptr;
+    const Held ga(ensure(g, a));
     Buffer *out = ga ? new_output(g, rows, cols) : nullptr;
     if (!out) return nullptr;
     emit(g, {op, ga->id, out->id, a->rows, a->cols});
@@ -606,37 +670,39 @@ PyObject *two_shaped(Graph *g, int64_t op, Tensor *a, Tensor *b) {     // out li
     emit(g, {op, ga->id, gb->id, out->id, a->rows, a->cols});
     return finish(g, out, nullptr);
 }
-// (opcode, a, b): words end with a's rows and columns (shapes checked by the caller)
-PyObject *graph_pair(Graph *g, PyObject *const *v, Py_ssize_t n) {
+// (graph, opcode, a, b): words end with a's rows and columns (shapes checked by the caller)
+PyObject *record_pair(PyObject *, PyObject *const *v, Py_ssize_t n) {
     int64_t op;
-    if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
-    Tensor *a = as_tensor(v[1]), *b = a ? as_tensor(v[2]) : nullptr;
-    return b ? two_shaped(g, op, a, b) : nullptr;
+    Graph *g = n == 4 ? plain_graph(v[0]) : nullptr;
+    Tensor *a = g ? tensor(v[2]) : nullptr, *b = a ? tensor(v[3]) : nullptr;
+    if (!b) return general("pair", v, n);
+    return read_int(v[1], op) ? two_shaped(g, op, a, b) : nullptr;
 }
-// (opcode, a, row vector)
-PyObject *graph_rows(Graph *g, PyObject *const *v, Py_ssize_t n) {
+// (graph, opcode, a, row vector)
+PyObject *record_rows(PyObject *, PyObject *const *v, Py_ssize_t n) {
     int64_t op;
-    if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
-    Tensor *a = as_tensor(v[1]), *b = a ? as_tensor(v[2]) : nullptr;
-    if (!b) return nullptr;
+    Graph *g = n == 4 ? plain_graph(v[0]) : nullptr;
+    Tensor *a = g ? tensor(v[2]) : nullptr, *b = a ? tensor(v[3]) : nullptr;
+    if (!b) return general("rowBroadcast", v, n);
     if (b->rows != 1 || b->cols != a->cols) return PyErr_Format(PyExc_ValueError, "Expected row vector 1x%zd but got %zdx%zd", a->cols, b->rows, b->cols);
-    return two_shaped(g, op, a, b);
+    return read_int(v[1], op) ? two_shaped(g, op, a, b) : nullptr;
 }
-// (opcode, a, column vector)
-PyObject *graph_cols(Graph *g, PyObject *const *v, Py_ssize_t n) {
+// (graph, opcode, a, column vector)
+PyObject *record_cols(PyObject *, PyObject *const *v, Py_ssize_t n) {
     int64_t op;
-    if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
-    Tensor *a = as_tensor(v[1]), *b = a ? as_tensor(v[2]) : nullptr;
-    if (!b) return nullptr;
+    Graph *g = n == 4 ? plain_graph(v[0]) : nullptr;
+    Tensor *a = g ? tensor(v[2]) : nullptr, *b = a ? tensor(v[3]) : nullptr;
+    if (!b) return general("colBroadcast", v, n);
     if (b->rows != a->rows || b->cols != 1) return PyErr_Format(PyExc_ValueError, "Expected col vector %zdx1 but got %zdx%zd", a->rows, b->rows, b->cols);
-    return two_shaped(g, op, a, b);
+    return read_int(v[1], op) ? two_shaped(g, op, a, b) : nullptr;
 }
-// (opcode, a, b)
-PyObject *graph_matmul(Graph *g, PyObject *const *v, Py_ssize_t n) {
+// (graph, opcode, a, b)
+PyObject *record_matmul(PyObject *, PyObject *const *v, Py_ssize_t n) {
     int64_t op;
-    if (!arity(n, 3) || !read_int(v[0], op)) return nullptr;
-    Tensor *a = as_tensor(v[1]), *b = a ? as_tensor(v[2]) : nullptr;
-    if (!b) return nullptr;
+    Graph *g = n == 4 ? plain_graph(v[0]) : nullptr;
+    Tensor *a = g ? tensor(v[2]) : nullptr, *b = a ? tensor(v[3]) : nullptr;
+    if (!b) return general("matmul", v, n);
+    if (!read_int(v[1], op)) return nullptr;
     if (a->cols != b->rows) return PyErr_Format(PyExc_ValueError, "Shape mismatch for matmul: %zdx%zd vs %zdx%zd", a->rows, a->cols, b->rows, b->cols);
     const Held ga(ensure(g, a)), gb(ga ? ensure(g, b) : nullptr);
     Buffer *out = gb ? new_output(g, a->rows, b->cols) : nullptr;
@@ -644,18 +710,20 @@ PyObject *graph_matmul(Graph *g, PyObject *const *v, Py_ssize_t n) {
     emit(g, {op, ga->id, gb->id, out->id, a->rows, b->cols, a->cols});
     return finish(g, out, nullptr);
 }
-// (opcode, w, g, m, v, lr, beta1, beta2, eps, weight decay, c1, c2): the first, third and fourth are updated where they are
-PyObject *graph_adamw(Graph *g, PyObject *const *v, Py_ssize_t n) {
+// (graph, opcode, w, g, m, v, lr, beta1, beta2, eps, weight decay, c1, c2): the first, third and fourth are updated where they are
+PyObject *record_adamw(PyObject *, PyObject *const *v, Py_ssize_t n) {
     int64_t op;
     int32_t bits[7];
-    if (!arity(n, 12) || !read_int(v[0], op)) return nullptr;
-    Tensor *t[4];
-    for (int i = 0; i < 4; i++)
-        if (!(t[i] = as_tensor(v[1 + i]))) return nullptr;
+    Graph *g = n == 13 ? plain_graph(v[0]) : nullptr;
+    Tensor *t[4] = {};
+    for (int i = 0; g && i < 4; i++)
+        if (!(t[i] = tensor(v[2 + i]))) g = nullptr;
+    if (!g) return general("adamW", v, n);
+    if (!read_int(v[1], op)) return nullptr;
     const Held w(ensure(g, t[0])), gw(w ? ensure(g, t[1]) : nullptr), mt(gw ? ensure(g, t[2]) : nullptr), vt(mt ? ensure(g, t[3]) : nullptr);
     if (!vt) return nullptr;
     for (int i = 0; i < 7; i++)
-        if (!read_float_bits(v[5 + i], bits[i])) return nullptr;
+        if (!read_float_bits(v[6 + i], bits[i])) return nullptr;
     emit(g, {op, w->id, gw->id, mt->id, vt->id, bits[0], bits[1], bits[2], bits[3], bits[4], bits[5], bits[6], t[0]->rows * t[0]->cols});
     for (Buffer *b : {w.b, mt.b, vt.b}) { b->cpu_stale = 1; b->needs_upload = 0; }
     Py_RETURN_NONE;
@@ -871,6 +939,7 @@ bool flush(Graph *g) {
     if (g->s->ops == 0 && g->s->allocs.empty()) return release_orphans(g);
     return allocate_pending(g) && upload_pending(g) && execute_pending(g) && release_orphans(g);
 }
+bool flush_method(Graph *g) { return plain_graph(reinterpret_cast<PyObject *>(g)) ? flush(g) : call(PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "flush", nullptr)); }
 PyObject *graph_flush(Graph *g, PyObject *) {
     if (!flush(g)) return nullptr;
     Py_RETURN_NONE;
@@ -930,14 +999,14 @@ PyObject *graph_materialize(Graph *g, PyObject *o) {
     Buffer *b = tag_of(t);
     if (!b || !b->cpu_stale) Py_RETURN_NONE;
     Py_INCREF(b);
-    const bool ok = flush(g) && download(g, b, t);
+    const bool ok = flush_method(g) && download(g, b, t);
     if (ok) b->cpu_stale = 0;
     Py_DECREF(b);
     if (!ok) return nullptr;
     Py_RETURN_NONE;
 }
 PyObject *graph_release_all(Graph *g, PyObject *) {
-    if (!flush(g)) return nullptr;
+    if (!flush_method(g)) return nullptr;
     State *s = g->s;
     std::vector<int32_t> ids;
     for (auto &e : s->tensors) ids.push_back(e.first);
@@ -957,7 +1026,12 @@ PyObject *graph_release_all(Graph *g, PyObject *) {
     }
     for (int id : ids) {
         auto it = s->tensors.find(id);
-        if (Tensor *t = it == s->tensors.end() ? nullptr : it->second) set_tag(t, Py_None);
+        Tensor *t = it == s->tensors.end() ? nullptr : it->second;
+        if (!t) continue;
+        Py_INCREF(t);
+        const bool ok = retag(t, Py_None);
+        Py_DECREF(t);
+        if (!ok) return nullptr;
     }
     if (!ids.empty() && !release_ids(g, ids)) return nullptr;
     while (!s->tensors.empty()) forget(g, s->tensors.begin()->first);
@@ -979,15 +1053,6 @@ PyMethodDef graph_methods[] = {
     FAST("bindTensorToBuffer", graph_bind),
     {"tensorLetGo", (PyCFunction)graph_let_go, METH_O, "Tensor.setGpuTag: the buffer is no longer the tag of a tensor that had it."},
     FAST("_emit", graph_emit),
-    FAST("binary", graph_binary),
-    FAST("unary", graph_unary),
-    FAST("scalar", graph_scalar),
-    FAST("shaped", graph_shaped),
-    FAST("pair", graph_pair),
-    FAST("rowBroadcast", graph_rows),
-    FAST("colBroadcast", graph_cols),
-    FAST("matmul", graph_matmul),
-    FAST("adamW", graph_adamw),
     {"isEmpty", (PyCFunction)graph_is_empty, METH_NOARGS, nullptr},
     {"flush", (PyCFunction)graph_flush, METH_NOARGS, nullptr},
     {"materialize", (PyCFunction)graph_materialize, METH_O, nullptr},
@@ -1028,7 +1093,39 @@ PyObject *set_tensor_class(PyObject *, PyObject *o) {
     g_tensor_class = reinterpret_cast<PyTypeObject *>(o);
     Py_RETURN_NONE;
 }
+// set_methods({name: function}, ComputeGraph, names): the way through a graph's methods, and which those are
+PyObject *set_methods(PyObject *, PyObject *args) {
+    PyObject *functions, *graph, *names;
+    if (!PyArg_ParseTuple(args, "O!O!O", &PyDict_Type, &functions, &PyType_Type, &graph, &names)) return nullptr;
+    if (!g_graph_methods.take(reinterpret_cast<PyTypeObject *>(graph), names)) return nullptr;
+    Py_INCREF(functions);
+    Py_XSETREF(g_general, functions);
+    Py_RETURN_NONE;
+}
+// set_native(HipGpuRuntime, names, HipNative, names): the methods that calls by address stand for
+PyObject *set_native(PyObject *, PyObject *args) {
+    PyObject *runtime, *names, *native, *native_names;
+    if (!PyArg_ParseTuple(args, "O!OO!O", &PyType_Type, &runtime, &names, &PyType_Type, &native, &native_names)) return nullptr;
+    if (!g_runtime_methods.take(reinterpret_cast<PyTypeObject *>(runtime), names)) return nullptr;
+    if (!g_native_methods.take(reinterpret_cast<PyTypeObject *>(native), native_names)) return nullptr;
+    Py_INCREF(runtime);
+    Py_INCREF(native);
+    g_runtime_class = reinterpret_cast<PyTypeObject *>(runtime);
+    g_native_class = reinterpret_cast<PyTypeObject *>(native);
+    Py_RETURN_NONE;
+}
 PyMethodDef module_methods[] = {
+    FAST("binary", record_binary),
+    FAST("unary", record_unary),
+    FAST("scalar", record_scalar),
+    FAST("shaped", record_shaped),
+    FAST("pair", record_pair),
+    FAST("rowBroadcast", record_rows),
+    FAST("colBroadcast", record_cols),
+    FAST("matmul", record_matmul),
+    FAST("adamW", record_adamw),
+    {"set_methods", set_methods, METH_VARARGS, nullptr},
+    {"set_native", set_native, METH_VARARGS, nullptr},
     {"set_helpers", set_helpers, METH_VARARGS, nullptr},
     {"set_tensor_class", set_tensor_class, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};

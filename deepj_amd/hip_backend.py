@@ -14,12 +14,13 @@ import numpy as np
 
 from . import opcodes as op
 from ._native import HipNative, call_addresses, host_array
-from .compute_graph import ComputeGraph, GpuBuffer
+from .compute_graph import ComputeGraph, GpuBuffer, _graph_core as record
 from .tensor import Tensor
 
 
 class HipGpuRuntime:
-    """Five calls passed on to the native library; a graph over an object of exactly this class makes them itself."""
+    """Five calls passed on to the native library; a graph over an object of exactly this class makes them itself, as long as
+    nothing is put in place of them or of HipNative's."""
 
     nativeCalls = staticmethod(call_addresses)
 
@@ -33,6 +34,10 @@ class HipGpuRuntime:
     def zeroBuffers(self, buffers):
         cmd = [w for buf_id, n in buffers for w in (op.OP_FILL, buf_id, 0, n)]
         HipNative.nativeFlushOps(cmd, len(cmd))
+
+
+record.set_native(HipGpuRuntime, ("allocBuffers", "uploadBuffer", "downloadBuffer", "releaseBuffers", "flushOps", "zeroBuffers"),
+                  HipNative, ("nativeAllocBuffers", "nativeUploadBuffer", "nativeDownloadBuffer", "nativeReleaseBuffers", "nativeFlushOps"))
 
 
 class HipBackend:
@@ -62,48 +67,48 @@ class HipBackend:
         self._int_column_scratch.clear()
 
     # ── matmul / element-wise ───────────────────────────────────────────────
-    def matmul(self, a, b): return self.graph.matmul(op.OP_MATMUL, a, b)
-    def add(self, a, b): return self.graph.binary(op.OP_ADD, "add", a, b, False)
-    def subtract(self, a, b): return self.graph.binary(op.OP_SUBTRACT, "subtract", a, b, False)
-    def multiply(self, a, b): return self.graph.binary(op.OP_MULTIPLY, "multiply", a, b, False)
-    def divide(self, a, b): return self.graph.binary(op.OP_DIVIDE, "divide", a, b, False)
-    def reluBackward(self, x, g): return self.graph.binary(op.OP_RELU_BACKWARD, "reluBackward", x, g, False)
-    def geluBackward(self, x, g): return self.graph.binary(op.OP_GELU_BACKWARD, "geluBackward", x, g, False)
+    def matmul(self, a, b): return record.matmul(self.graph, op.OP_MATMUL, a, b)
+    def add(self, a, b): return record.binary(self.graph, op.OP_ADD, "add", a, b, False)
+    def subtract(self, a, b): return record.binary(self.graph, op.OP_SUBTRACT, "subtract", a, b, False)
+    def multiply(self, a, b): return record.binary(self.graph, op.OP_MULTIPLY, "multiply", a, b, False)
+    def divide(self, a, b): return record.binary(self.graph, op.OP_DIVIDE, "divide", a, b, False)
+    def reluBackward(self, x, g): return record.binary(self.graph, op.OP_RELU_BACKWARD, "reluBackward", x, g, False)
+    def geluBackward(self, x, g): return record.binary(self.graph, op.OP_GELU_BACKWARD, "geluBackward", x, g, False)
 
     # ── broadcasts ──────────────────────────────────────────────────────────
-    def addRowVector(self, a, v): return self.graph.rowBroadcast(op.OP_ADD_ROW_VECTOR, a, v)
+    def addRowVector(self, a, v): return record.rowBroadcast(self.graph, op.OP_ADD_ROW_VECTOR, a, v)
     def addBroadcastRows(self, a, v): return self.addRowVector(a, v)
-    def multiplyBroadcastRows(self, a, v): return self.graph.rowBroadcast(op.OP_MULTIPLY_BROADCAST_ROWS, a, v)
-    def addBroadcastCols(self, a, v): return self.graph.colBroadcast(op.OP_ADD_BROADCAST_COLS, a, v)
-    def subtractBroadcastCols(self, a, v): return self.graph.colBroadcast(op.OP_SUBTRACT_BROADCAST_COLS, a, v)
-    def divideBroadcastCols(self, a, v): return self.graph.colBroadcast(op.OP_DIVIDE_BROADCAST_COLS, a, v)
-    def multiplyBroadcastCols(self, a, v): return self.graph.colBroadcast(op.OP_MULTIPLY_BROADCAST_COLS, a, v)
+    def multiplyBroadcastRows(self, a, v): return record.rowBroadcast(self.graph, op.OP_MULTIPLY_BROADCAST_ROWS, a, v)
+    def addBroadcastCols(self, a, v): return record.colBroadcast(self.graph, op.OP_ADD_BROADCAST_COLS, a, v)
+    def subtractBroadcastCols(self, a, v): return record.colBroadcast(self.graph, op.OP_SUBTRACT_BROADCAST_COLS, a, v)
+    def divideBroadcastCols(self, a, v): return record.colBroadcast(self.graph, op.OP_DIVIDE_BROADCAST_COLS, a, v)
+    def multiplyBroadcastCols(self, a, v): return record.colBroadcast(self.graph, op.OP_MULTIPLY_BROADCAST_COLS, a, v)
 
     # ── scalar ops ──────────────────────────────────────────────────────────
-    def multiplyScalar(self, a, s): return self.graph.scalar(op.OP_MULTIPLY_SCALAR, a, s, False)
-    def addScalar(self, a, s): return self.graph.scalar(op.OP_ADD_SCALAR, a, s, False)
-    def divideScalar(self, a, s): return self.graph.scalar(op.OP_DIVIDE_SCALAR, a, s, False)
+    def multiplyScalar(self, a, s): return record.scalar(self.graph, op.OP_MULTIPLY_SCALAR, a, s, False)
+    def addScalar(self, a, s): return record.scalar(self.graph, op.OP_ADD_SCALAR, a, s, False)
+    def divideScalar(self, a, s): return record.scalar(self.graph, op.OP_DIVIDE_SCALAR, a, s, False)
 
     # ── reductions ──────────────────────────────────────────────────────────
-    def sumRows(self, a): return self.graph.shaped(op.OP_SUM_ROWS, a, 1, a.cols)
+    def sumRows(self, a): return record.shaped(self.graph, op.OP_SUM_ROWS, a, 1, a.cols)
     def sumAlongCols(self, a): return self.sumRows(a)
-    def sumAlongRows(self, a): return self.graph.shaped(op.OP_SUM_ALONG_ROWS, a, a.rows, 1)
-    def meanAlongRows(self, a): return self.graph.shaped(op.OP_MEAN_ALONG_ROWS, a, a.rows, 1)
-    def varianceAlongRows(self, a): return self.graph.shaped(op.OP_VARIANCE_ALONG_ROWS, a, a.rows, 1)
-    def maxAlongRows(self, a): return self.graph.shaped(op.OP_MAX_ALONG_ROWS, a, a.rows, 1)
+    def sumAlongRows(self, a): return record.shaped(self.graph, op.OP_SUM_ALONG_ROWS, a, a.rows, 1)
+    def meanAlongRows(self, a): return record.shaped(self.graph, op.OP_MEAN_ALONG_ROWS, a, a.rows, 1)
+    def varianceAlongRows(self, a): return record.shaped(self.graph, op.OP_VARIANCE_ALONG_ROWS, a, a.rows, 1)
+    def maxAlongRows(self, a): return record.shaped(self.graph, op.OP_MAX_ALONG_ROWS, a, a.rows, 1)
 
     def sum(self, a) -> float:
-        scalar = self.graph.shaped(op.OP_SUM_SCALAR, a, 1, 1)
+        scalar = record.shaped(self.graph, op.OP_SUM_SCALAR, a, 1, 1)
         scalar.materialize()
         return float(scalar.data[0, 0])
 
     def sumAbs(self, a) -> float:
-        scalar = self.sumRows(self.graph.shaped(op.OP_SUM_ABS, a, a.rows, 1))
+        scalar = self.sumRows(record.shaped(self.graph, op.OP_SUM_ABS, a, a.rows, 1))
         scalar.materialize()
         return float(scalar.data[0, 0])
 
     # ── unary ───────────────────────────────────────────────────────────────
-    def transpose(self, a): return self.graph.shaped(op.OP_TRANSPOSE, a, a.cols, a.rows)
+    def transpose(self, a): return record.shaped(self.graph, op.OP_TRANSPOSE, a, a.cols, a.rows)
 
     def clamp(self, a, lo, hi):
         ga = self._in(a)
@@ -111,44 +116,44 @@ class HipBackend:
         self.graph.recordClamp(ga, out, lo, hi)
         return self._out(out)
 
-    def pow(self, a, exponent): return self.graph.scalar(op.OP_POW, a, exponent, False)
-    def sqrt(self, a): return self.graph.unary(op.OP_SQRT, a, False)
-    def neg(self, a): return self.graph.unary(op.OP_NEG, a, False)
-    def exp(self, a): return self.graph.unary(op.OP_EXP, a, False)
-    def log(self, a): return self.graph.unary(op.OP_LOG, a, False)
-    def tanh(self, a): return self.graph.unary(op.OP_TANH, a, False)
-    def sigmoid(self, a): return self.graph.unary(op.OP_SIGMOID, a, False)
-    def relu(self, a): return self.graph.unary(op.OP_RELU, a, False)
-    def gelu(self, a): return self.graph.unary(op.OP_GELU, a, False)
+    def pow(self, a, exponent): return record.scalar(self.graph, op.OP_POW, a, exponent, False)
+    def sqrt(self, a): return record.unary(self.graph, op.OP_SQRT, a, False)
+    def neg(self, a): return record.unary(self.graph, op.OP_NEG, a, False)
+    def exp(self, a): return record.unary(self.graph, op.OP_EXP, a, False)
+    def log(self, a): return record.unary(self.graph, op.OP_LOG, a, False)
+    def tanh(self, a): return record.unary(self.graph, op.OP_TANH, a, False)
+    def sigmoid(self, a): return record.unary(self.graph, op.OP_SIGMOID, a, False)
+    def relu(self, a): return record.unary(self.graph, op.OP_RELU, a, False)
+    def gelu(self, a): return record.unary(self.graph, op.OP_GELU, a, False)
 
     # ── softmax ─────────────────────────────────────────────────────────────
-    def softmaxRows(self, logits): return self.graph.shaped(op.OP_SOFTMAX_ROWS, logits, logits.rows, logits.cols)
+    def softmaxRows(self, logits): return record.shaped(self.graph, op.OP_SOFTMAX_ROWS, logits, logits.rows, logits.cols)
 
     def softmaxBackward(self, grad, softmax):
         Tensor.requireSameShape(grad, softmax, "softmaxBackward")
-        return self.graph.pair(op.OP_SOFTMAX_BACKWARD, grad, softmax)
+        return record.pair(self.graph, op.OP_SOFTMAX_BACKWARD, grad, softmax)
 
     # ── in-place: new buffer, rebind (MetalBackend.java:400-526) ────────────
-    def addInPlace(self, a, b): self.graph.binary(op.OP_ADD, "addInPlace", a, b, True)
-    def subtractInPlace(self, a, b): self.graph.binary(op.OP_SUBTRACT, "subtractInPlace", a, b, True)
-    def multiplyInPlace(self, a, b): self.graph.binary(op.OP_MULTIPLY, "multiplyInPlace", a, b, True)
-    def divideInPlace(self, a, b): self.graph.binary(op.OP_DIVIDE, "divideInPlace", a, b, True)
-    def multiplyScalarInPlace(self, a, s): self.graph.scalar(op.OP_MULTIPLY_SCALAR, a, s, True)
-    def addScalarInPlace(self, a, s): self.graph.scalar(op.OP_ADD_SCALAR, a, s, True)
-    def divideScalarInPlace(self, a, s): self.graph.scalar(op.OP_DIVIDE_SCALAR, a, s, True)
-    def sqrtInPlace(self, a): self.graph.unary(op.OP_SQRT, a, True)
-    def negInPlace(self, a): self.graph.unary(op.OP_NEG, a, True)
-    def expInPlace(self, a): self.graph.unary(op.OP_EXP, a, True)
-    def logInPlace(self, a): self.graph.unary(op.OP_LOG, a, True)
-    def reluInPlace(self, a): self.graph.unary(op.OP_RELU, a, True)
-    def geluInPlace(self, a): self.graph.unary(op.OP_GELU, a, True)
-    def tanhInPlace(self, a): self.graph.unary(op.OP_TANH, a, True)
-    def sigmoidInPlace(self, a): self.graph.unary(op.OP_SIGMOID, a, True)
+    def addInPlace(self, a, b): record.binary(self.graph, op.OP_ADD, "addInPlace", a, b, True)
+    def subtractInPlace(self, a, b): record.binary(self.graph, op.OP_SUBTRACT, "subtractInPlace", a, b, True)
+    def multiplyInPlace(self, a, b): record.binary(self.graph, op.OP_MULTIPLY, "multiplyInPlace", a, b, True)
+    def divideInPlace(self, a, b): record.binary(self.graph, op.OP_DIVIDE, "divideInPlace", a, b, True)
+    def multiplyScalarInPlace(self, a, s): record.scalar(self.graph, op.OP_MULTIPLY_SCALAR, a, s, True)
+    def addScalarInPlace(self, a, s): record.scalar(self.graph, op.OP_ADD_SCALAR, a, s, True)
+    def divideScalarInPlace(self, a, s): record.scalar(self.graph, op.OP_DIVIDE_SCALAR, a, s, True)
+    def sqrtInPlace(self, a): record.unary(self.graph, op.OP_SQRT, a, True)
+    def negInPlace(self, a): record.unary(self.graph, op.OP_NEG, a, True)
+    def expInPlace(self, a): record.unary(self.graph, op.OP_EXP, a, True)
+    def logInPlace(self, a): record.unary(self.graph, op.OP_LOG, a, True)
+    def reluInPlace(self, a): record.unary(self.graph, op.OP_RELU, a, True)
+    def geluInPlace(self, a): record.unary(self.graph, op.OP_GELU, a, True)
+    def tanhInPlace(self, a): record.unary(self.graph, op.OP_TANH, a, True)
+    def sigmoidInPlace(self, a): record.unary(self.graph, op.OP_SIGMOID, a, True)
 
     # ── fused ops ───────────────────────────────────────────────────────────
     def crossEntropyGradient(self, logits, targets):
         Tensor.requireTargetsMatchRows(logits, targets)
-        return self.graph.pair(op.OP_CROSS_ENTROPY_GRADIENT, logits, self._int_column(targets))
+        return record.pair(self.graph, op.OP_CROSS_ENTROPY_GRADIENT, logits, self._int_column(targets))
 
     def crossEntropyLoss(self, logits, targets) -> float:
         Tensor.requireTargetsMatchRows(logits, targets)
@@ -163,7 +168,7 @@ class HipBackend:
     def adamWUpdate(self, w, g, mt, vt, lr, beta1, beta2, eps, weight_decay, bc1, bc2):
         for other in (g, mt, vt):
             Tensor.requireSameShape(w, other, "adamWUpdate")
-        self.graph.adamW(op.OP_ADAMW_UPDATE, w, g, mt, vt, lr, beta1, beta2, eps, weight_decay, bc1, bc2)
+        record.adamW(self.graph, op.OP_ADAMW_UPDATE, w, g, mt, vt, lr, beta1, beta2, eps, weight_decay, bc1, bc2)
 
     def layerNormBackward(self, dxhat, xhat, std, dim):
         Tensor.requireSameShape(dxhat, xhat, "layerNormBackward")

@@ -12,7 +12,7 @@ import weakref
 import numpy as np
 import pytest
 
-from deepj_amd import ComputeGraph, GpuBuffer, HipBackend, Tensor, opcodes as op
+from deepj_amd import ComputeGraph, GpuBuffer, HipBackend, HipGpuRuntime, HipNative, Tensor, opcodes as op
 
 
 class RecordingRuntime:
@@ -582,6 +582,134 @@ def test_the_librarys_calls_run_one_at_a_time(blocking):
     for t in threads:
         t.join()
     assert not blocking.value["together"].value
+
+
+class CountingGraph(ComputeGraph):
+    """Every method an operation goes through, counted."""
+
+    def __init__(self, runtime):
+        super().__init__(runtime)
+        self.seen = []
+
+
+for _name in ("ensureGpuBuffer", "newOutputBuffer", "createOutputTensor", "bindTensorToBuffer", "flush", *(n for n in dir(ComputeGraph) if n.startswith("record"))):
+    def _counting(self, *args, _name=_name):
+        self.seen.append(_name)
+        return getattr(ComputeGraph, _name)(self, *args)
+    setattr(CountingGraph, _name, _counting)
+
+
+def _every_operation(be):
+    """Each operation of the backend once, over operands of its own; what it hands back."""
+    t = lambda r, c, first=1.0: Tensor.from2D(np.arange(first, first + r * c, dtype=np.float32).reshape(r, c))
+    m, row, col, results = t(2, 3), t(1, 3), t(2, 1), []
+    for name in ("add", "subtract", "multiply", "divide", "reluBackward", "geluBackward", "softmaxBackward"):
+        results.append(getattr(be, name)(m, t(2, 3, 4.0)))
+    for name in ("addInPlace", "subtractInPlace", "multiplyInPlace", "divideInPlace"):
+        x = t(2, 3, 2.0)
+        results += [getattr(be, name)(x, m), x]
+    for name in ("sqrt", "neg", "exp", "log", "tanh", "sigmoid", "relu", "gelu", "transpose", "softmaxRows", "sumRows", "sumAlongRows", "meanAlongRows",
+                 "varianceAlongRows", "maxAlongRows"):
+        results.append(getattr(be, name)(m))
+    for name in ("sqrtInPlace", "negInPlace", "expInPlace", "logInPlace", "reluInPlace", "geluInPlace", "tanhInPlace", "sigmoidInPlace"):
+        x = t(2, 3, 3.0)
+        results += [getattr(be, name)(x), x]
+    for name in ("multiplyScalar", "addScalar", "divideScalar", "pow"):
+        results.append(getattr(be, name)(m, 1.5))
+    for name in ("multiplyScalarInPlace", "addScalarInPlace", "divideScalarInPlace"):
+        x = t(2, 3, 5.0)
+        results += [getattr(be, name)(x, 2.5), x]
+    results += [be.addRowVector(m, row), be.multiplyBroadcastRows(m, row)]
+    results += [getattr(be, name)(m, col) for name in ("addBroadcastCols", "subtractBroadcastCols", "divideBroadcastCols", "multiplyBroadcastCols")]
+    results += [be.matmul(m, t(3, 4)), be.clamp(m, 0.0, 1.0), be.sum(m), be.sumAbs(m), be.crossEntropyLoss(m, [0, 1]), be.crossEntropyGradient(m, [2, 0])]
+    w, mt, vt = t(2, 3), t(2, 3), t(2, 3)
+    results += [be.adamWUpdate(w, m, mt, vt, 1e-3, 0.9, 0.99, 1e-8, 0.0, 1.0, 1.0), w, mt, vt, be.layerNormBackward(m, t(2, 3), col, 3)]
+    for call, bad in ((be.add, (m, row)), (be.matmul, (m, m)), (be.addRowVector, (m, col)), (be.addBroadcastCols, (m, row)), (be.multiplyInPlace, (m, col))):
+        with pytest.raises(ValueError) as e:
+            call(*bad)
+        results.append(str(e.value))
+    be.graph.flush()
+    return [r.getGpuTag().id if isinstance(r, Tensor) else r for r in results]
+
+
+def _calls(runtime):
+    return [[(list(a), list(b)) for a, b, _ in runtime.allocCalls], [(i, list(v)) for i, v in runtime.uploads], runtime.downloads,
+            [list(c) for c, _ in runtime.flushCalls], [list(a) for a, _ in runtime.releaseCalls]]
+
+
+class Forwarding:
+    """An object that is no ComputeGraph and passes everything on to one."""
+
+    def __init__(self, runtime): self.inner = ComputeGraph(runtime)
+    def __getattr__(self, name): return getattr(self.inner, name)
+
+
+@pytest.mark.parametrize("way", ["subclass", "instance", "class", "other object"])
+def test_methods_of_a_graph_that_are_replaced_are_called(way, monkeypatch):
+    """By a class derived from ComputeGraph, on one graph, on ComputeGraph itself, or by an object in its place: the operations go
+    through the methods, and record and hand back what they do otherwise."""
+    plain_rt, rt = RecordingRuntime(), RecordingRuntime()
+    plain = HipBackend(plain_rt)
+    Tensor.setBackend(plain)
+    want = _every_operation(plain)
+    be, seen = HipBackend(rt), []
+    if way == "subclass":
+        be.graph = CountingGraph(rt)
+        seen = be.graph.seen
+    elif way == "instance":
+        record = be.graph.recordBinary
+        be.graph.recordBinary = lambda *a: (seen.append("recordBinary"), record(*a))
+    elif way == "class":
+        record = ComputeGraph.recordBinary
+        monkeypatch.setattr(ComputeGraph, "recordBinary", lambda self, *a: (seen.append("recordBinary"), record(self, *a))[1])
+    else:
+        be.graph = Forwarding(rt)
+        seen.append("recordBinary")
+    Tensor.setBackend(be)
+    assert _every_operation(be) == want
+    assert _calls(rt) == _calls(plain_rt)
+    assert "recordBinary" in seen
+    if way == "subclass":
+        assert set(seen) == {n for n in dir(CountingGraph) if not n.startswith("_")} - {
+            "recordScatterAddRows", "recordScatterAddRowsAtomic", "runtime", "isEmpty", "materialize", "releaseAll", "tensorLetGo", "seen"}
+    monkeypatch.undo()
+    n = len(seen)
+    if way == "class":
+        be.add(Tensor(1, 1), Tensor(1, 1))
+        assert len(seen) == n                                          # and the short way is back
+
+
+@pytest.mark.parametrize("owner,names", [(HipGpuRuntime, ("allocBuffers", "uploadBuffer", "downloadBuffer", "releaseBuffers", "flushOps", "zeroBuffers")),
+                                         (HipNative, ("nativeAllocBuffers", "nativeUploadBuffer", "nativeDownloadBuffer", "nativeReleaseBuffers", "nativeFlushOps"))])
+def test_calls_of_the_runtime_that_are_replaced_are_called(owner, names, monkeypatch):
+    """On the classes that pass them on to the library; a large tensor's values too, and back."""
+    seen = []
+    for name in names:
+        if owner is HipNative:
+            monkeypatch.setattr(owner, name, staticmethod(lambda *a, name=name: seen.append(name)))
+        else:
+            monkeypatch.setattr(owner, name, lambda self, *a, name=name: seen.append(name))
+    be = HipBackend()
+    out = be.add(be.add(Tensor.from2D(np.ones((512, 512), np.float32)), Tensor(512, 512)), Tensor(512, 512))
+    be.graph.flush()
+    be.materializeTensor(out)
+    del out
+    be.graph.flush()
+    assert set(seen) == set(names)
+    be.releaseResources()
+
+
+def test_a_tensor_class_with_a_set_gpu_tag_of_its_own_has_it_called():
+    class Watching(Tensor):
+        def setGpuTag(self, tag):
+            self.__dict__.setdefault("tags", []).append(tag)
+            super().setGpuTag(tag)
+    be = HipBackend(RecordingRuntime())
+    t = Watching(1, 2)
+    t.data[:] = 1.0
+    be.negInPlace(t)
+    be.releaseResources()
+    assert [type(x) for x in t.tags] == [GpuBuffer, GpuBuffer, type(None)] and t.tags[0] is not t.tags[1]
 
 
 @pytest.mark.parametrize("holder", ["graph", "runtime", "tensor"])
