@@ -11,6 +11,7 @@ protocol the Java class speaks (same encodings, same call order).
 from __future__ import annotations
 
 import struct
+import weakref
 from typing import Protocol
 
 import numpy as np
@@ -70,6 +71,11 @@ _OP_META[op.OP_LAYERNORM_BACKWARD] = (7, (1, 2, 3, 4))
 _OP_META[op.OP_ADAMW_UPDATE] = (13, (1, 2, 3, 4))
 
 
+class _OtherRef(weakref.ref):
+    """A weak reference that remembers which buffer its object stood for."""
+    __slots__ = ("id",)
+
+
 class ComputeGraph(_graph_core.GraphCore):
     """ComputeGraph.java.  Buffer management (:172-234), flush (:528-671), materialize and release (:676-740) are
     csrc/graph_core.cpp, and so are the operations HipBackend records most; nothing walks all tracked tensors: buffers that may
@@ -86,6 +92,76 @@ class ComputeGraph(_graph_core.GraphCore):
             native = None
         super().__init__(runtime, getattr(runtime, "zeroBuffers", None),
                          getattr(runtime, "hostArray", None) or (lambda n: np.zeros(n, dtype=np.float32)), native, calls)
+
+    # ── objects that stand in for a tensor: rows, cols, data, _data, _gpu_tag and setGpuTag are all that is asked of one ──
+    def _ensureOther(self, o):
+        if not hasattr(o, "_gpu_tag"):
+            raise TypeError(f"expected a Tensor, not {type(o).__name__}")
+        buf = o._gpu_tag
+        if isinstance(buf, GpuBuffer):
+            ref = (self._others or {}).get(buf.id)
+            if ref is None or ref() is not o:
+                self._trackOther(buf, o)
+            if buf.needsUpload:
+                self._uploadOther(buf, o, pack_f32(o))
+                buf.needsUpload = buf.cpuStale = False
+            return buf
+        buf = _graph_core.GraphCore.newOutputBuffer(self, o.rows, o.cols)
+        buf.cpuStale, buf.needsUpload = False, True
+        self._uploadOther(buf, o, None if o._data is None else pack_f32(o))
+        o.setGpuTag(buf)
+        self._trackOther(buf, o)
+        return buf
+
+    def _trackOther(self, buf, o):
+        self._forget(buf.id)
+        if self._others is None:
+            self._others = {}
+        self._others[buf.id] = ref = _OtherRef(o, self._otherDied)
+        ref.id = buf.id
+        buf.graph = self
+
+    def _otherDied(self, ref): self._lost(ref.id)
+
+    def _uploadOther(self, buf, o, values):
+        carrier = _tensor_class()(o.rows, o.cols)
+        carrier._data = values
+        self._upload(buf.id, carrier)
+
+    def _downloadOther(self, buf, o):
+        carrier = _tensor_class()(o.rows, o.cols)
+        carrier._data = o._data
+        self._download(buf, carrier)
+        if o._data is None:
+            o._data = carrier._data
+
+    def _bindOther(self, o, buf):
+        o.setGpuTag(buf)
+        self._trackOther(buf, o)
+
+    def _materializeOther(self, o):
+        if not hasattr(o, "_gpu_tag"):
+            raise TypeError(f"expected a Tensor, not {type(o).__name__}")
+        buf = o._gpu_tag
+        if isinstance(buf, GpuBuffer) and buf.cpuStale:
+            self.flush()
+            self._downloadOther(buf, o)
+            buf.cpuStale = False
+
+    def _otherHolds(self, buf_id):
+        o = self._others[buf_id]()
+        return o is not None and isinstance(o._gpu_tag, GpuBuffer) and o._gpu_tag.id == buf_id
+
+    def _releaseOthers(self):
+        held = [o for o in (ref() for ref in self._others.values()) if o is not None]
+        for o in held:
+            buf = o._gpu_tag
+            if isinstance(buf, GpuBuffer) and buf.cpuStale:
+                self._downloadOther(buf, o)
+                buf.cpuStale = buf.needsUpload = False
+        for o in held:
+            o.setGpuTag(None)
+        return list(self._others)
 
     # ── op recording (ComputeGraph.java:238-518) ────────────────────────────
     def recordBinary(self, opcode, a, b, out): self._emit(opcode, a.id, b.id, out.id, out.floatCount())
@@ -240,6 +316,11 @@ _graph_core.set_methods(
      "recordAdamWUpdate", *_SHAPED.values(), *_PAIRS.values()])
 
 
+def _tensor_class():
+    from .tensor import Tensor
+    return Tensor
+
+
 # TensorAdapters.java:9-47
 def pack_f32(t) -> np.ndarray:
     return t.data.astype(np.float32, order="C").reshape(-1)          # a copy: the tensor may change before the flush
@@ -252,8 +333,7 @@ def unpack_f32_into(src: np.ndarray, dst) -> None:
 
 
 def from_int_column(values) -> "object":
-    from .tensor import Tensor
-    t = Tensor(len(values), 1)
+    t = _tensor_class()(len(values), 1)
     t.data[:, 0] = np.asarray(values, dtype=np.float32)
     return t
 

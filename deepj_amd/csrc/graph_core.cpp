@@ -129,11 +129,26 @@ struct Graph {
     PyObject *runtime, *zero_buffers, *host_array;
     int next_id;
     Native native;
+    PyObject *others;                      // null, None, or what else it tracks: {id: weak reference} (ComputeGraph, compute_graph.py)
     PyTypeObject *native_type;             // a runtime of exactly this class, with nothing set on it, is spoken to directly
     State *s;
 };
 
+bool has_other(Graph *g, int id) {
+    if (!g->others || !PyDict_Check(g->others)) return false;
+    PyObject *key = PyLong_FromLong(id);
+    const bool r = key && PyDict_Contains(g->others, key) == 1;
+    Py_XDECREF(key);
+    PyErr_Clear();
+    return r;
+}
+void drop_other(Graph *g, int id) {
+    PyObject *key = PyLong_FromLong(id);
+    if (!key || PyDict_DelItem(g->others, key) != 0) PyErr_Clear();
+    Py_XDECREF(key);
+}
 void track(Graph *g, int id, Tensor *t) {
+    if (has_other(g, id)) drop_other(g, id);
     Tensor *&slot = g->s->tensors[id];
     if (slot == t) return;
     if (slot)
@@ -261,12 +276,12 @@ void drop_allocs(State *s) {
     for (Buffer *b : gone) Py_DECREF(b);
 }
 int graph_traverse(Graph *g, visitproc visit, void *arg) {
-    Py_VISIT(g->runtime); Py_VISIT(g->zero_buffers); Py_VISIT(g->host_array); Py_VISIT(g->native_type);
+    Py_VISIT(g->runtime); Py_VISIT(g->zero_buffers); Py_VISIT(g->host_array); Py_VISIT(g->native_type); Py_VISIT(g->others);
     for (Buffer *b : g->s->allocs) Py_VISIT(b);
     return 0;
 }
 int graph_clear(Graph *g) {
-    Py_CLEAR(g->runtime); Py_CLEAR(g->zero_buffers); Py_CLEAR(g->host_array); Py_CLEAR(g->native_type);
+    Py_CLEAR(g->runtime); Py_CLEAR(g->zero_buffers); Py_CLEAR(g->host_array); Py_CLEAR(g->native_type); Py_CLEAR(g->others);
     drop_allocs(g->s);
     return 0;
 }
@@ -428,8 +443,9 @@ int send_now(Graph *g, Buffer *b, Tensor *t) {
     return r;
 }
 
+Tensor *tensor(PyObject *o) { return PyObject_TypeCheck(o, &TensorType) ? reinterpret_cast<Tensor *>(o) : nullptr; }
 Tensor *as_tensor(PyObject *o) {
-    if (PyObject_TypeCheck(o, &TensorType)) return reinterpret_cast<Tensor *>(o);
+    if (Tensor *t = tensor(o)) return t;
     PyErr_Format(PyExc_TypeError, "expected a Tensor, not %.100s", Py_TYPE(o)->tp_name);
     return nullptr;
 }
@@ -545,9 +561,10 @@ bool arity(Py_ssize_t n, Py_ssize_t want) {
     return false;
 }
 
+// An object that stands in for a tensor is looked after by methods of ComputeGraph.
 PyObject *graph_ensure(Graph *g, PyObject *o) {
-    Tensor *t = as_tensor(o);
-    return reinterpret_cast<PyObject *>(t ? ensure(g, t) : nullptr);
+    if (Tensor *t = tensor(o)) return reinterpret_cast<PyObject *>(ensure(g, t));
+    return PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "_ensureOther", "O", o);
 }
 PyObject *graph_new_output(Graph *g, PyObject *const *a, Py_ssize_t n) {
     int64_t r, c;
@@ -565,9 +582,10 @@ PyObject *graph_output_tensor(Graph *g, PyObject *o) {
 }
 PyObject *graph_bind(Graph *g, PyObject *const *a, Py_ssize_t n) {
     if (!arity(n, 2)) return nullptr;
-    Tensor *t = as_tensor(a[0]);
-    Buffer *b = t ? as_buffer(a[1]) : nullptr;
+    Buffer *b = as_buffer(a[1]);
     if (!b) return nullptr;
+    Tensor *t = tensor(a[0]);
+    if (!t) return PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "_bindOther", "OO", a[0], a[1]);
     if (!bind(g, t, b)) return nullptr;
     Py_RETURN_NONE;
 }
@@ -602,7 +620,6 @@ Graph *plain_graph(PyObject *o) {
             if (PyDict_Contains(*d, m.first) != 0) { PyErr_Clear(); return nullptr; }
     return reinterpret_cast<Graph *>(o);
 }
-Tensor *tensor(PyObject *o) { return PyObject_TypeCheck(o, &TensorType) ? reinterpret_cast<Tensor *>(o) : nullptr; }
 PyObject *general(const char *name, PyObject *const *v, Py_ssize_t n) {
     PyObject *f = g_general ? PyDict_GetItemString(g_general, name) : nullptr;
     if (!f) return PyErr_Format(PyExc_RuntimeError, "no function for %s", name);
@@ -858,14 +875,22 @@ bool release_orphans(Graph *g) {
     std::vector<int32_t> orphans;
     for (int id : candidates) {
         auto it = s->tensors.find(id);
-        if (it == s->tensors.end()) continue;              // unknown, or seen before
-        if (Tensor *t = it->second) {
+        const bool other = it == s->tensors.end();
+        if (other) {
+            if (!has_other(g, id)) continue;               // unknown, or seen before
+            PyObject *held = PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "_otherHolds", "i", id);
+            const bool stays = held != Py_False;
+            Py_XDECREF(held);
+            if (!held) { s->maybe_orphans.insert(s->maybe_orphans.end(), candidates.begin(), candidates.end()); return false; }
+            if (stays) continue;
+        } else if (Tensor *t = it->second) {
             Buffer *b = tag_of(t);
             if (b && b->id == id) continue;
         }
         if (s->ops > 0 && referenced_by_pending_ops(g, id)) { s->maybe_orphans.push_back(id); continue; }
         orphans.push_back(id);
-        forget(g, id);
+        if (other) drop_other(g, id);
+        else forget(g, id);
     }
     if (orphans.empty()) return true;
     if (!s->allocs.empty() || !s->uploads.empty()) {
@@ -994,8 +1019,8 @@ bool download(Graph *g, Buffer *b, Tensor *t) {
     return ok;
 }
 PyObject *graph_materialize(Graph *g, PyObject *o) {
-    Tensor *t = as_tensor(o);
-    if (!t) return nullptr;
+    Tensor *t = tensor(o);
+    if (!t) return PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "_materializeOther", "O", o);
     Buffer *b = tag_of(t);
     if (!b || !b->cpu_stale) Py_RETURN_NONE;
     Py_INCREF(b);
@@ -1009,6 +1034,14 @@ PyObject *graph_release_all(Graph *g, PyObject *) {
     if (!flush_method(g)) return nullptr;
     State *s = g->s;
     std::vector<int32_t> ids;
+    if (g->others && PyDict_Check(g->others)) {
+        PyObject *more = PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "_releaseOthers", nullptr), *list = more ? PySequence_Tuple(more) : nullptr;
+        Py_XDECREF(more);
+        if (!list) return nullptr;
+        for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(list); i++) ids.push_back((int32_t)PyLong_AsLong(PyTuple_GET_ITEM(list, i)));
+        Py_DECREF(list);
+        if (PyErr_Occurred()) return nullptr;
+    }
     for (auto &e : s->tensors) ids.push_back(e.first);
     std::sort(ids.begin(), ids.end());
     for (int id : ids) {
@@ -1035,12 +1068,41 @@ PyObject *graph_release_all(Graph *g, PyObject *) {
     }
     if (!ids.empty() && !release_ids(g, ids)) return nullptr;
     while (!s->tensors.empty()) forget(g, s->tensors.begin()->first);
+    Py_CLEAR(g->others);
     s->maybe_orphans.clear();
     drop_allocs(s);
     drop_uploads(s);
     s->cmd.clear();
     s->ops = 0;
     g->next_id = 0;
+    Py_RETURN_NONE;
+}
+// (id, tensor): its host values are sent there; (buffer, tensor): the buffer's values come into its host array; (id): no tensor of
+// its own has it; (id): whatever had it is gone
+PyObject *graph_upload(Graph *g, PyObject *const *a, Py_ssize_t n) {
+    int64_t id;
+    if (!arity(n, 2) || !read_int(a[0], id)) return nullptr;
+    Tensor *t = as_tensor(a[1]);
+    if (!t || !add_upload(g, (int)id, t)) return nullptr;
+    Py_RETURN_NONE;
+}
+PyObject *graph_download(Graph *g, PyObject *const *a, Py_ssize_t n) {
+    if (!arity(n, 2)) return nullptr;
+    Buffer *b = as_buffer(a[0]);
+    Tensor *t = b ? as_tensor(a[1]) : nullptr;
+    if (!t || !download(g, b, t)) return nullptr;
+    Py_RETURN_NONE;
+}
+PyObject *graph_forget(Graph *g, PyObject *o) {
+    int64_t id;
+    if (!read_int(o, id)) return nullptr;
+    forget(g, (int)id);
+    Py_RETURN_NONE;
+}
+PyObject *graph_lost(Graph *g, PyObject *o) {
+    int64_t id;
+    if (!read_int(o, id)) return nullptr;
+    g->s->maybe_orphans.push_back((int)id);
     Py_RETURN_NONE;
 }
 PyObject *graph_is_empty(Graph *g, PyObject *) { return PyBool_FromLong(g->s->ops == 0); }
@@ -1053,6 +1115,10 @@ PyMethodDef graph_methods[] = {
     FAST("bindTensorToBuffer", graph_bind),
     {"tensorLetGo", (PyCFunction)graph_let_go, METH_O, "Tensor.setGpuTag: the buffer is no longer the tag of a tensor that had it."},
     FAST("_emit", graph_emit),
+    FAST("_upload", graph_upload),
+    FAST("_download", graph_download),
+    {"_forget", (PyCFunction)graph_forget, METH_O, nullptr},
+    {"_lost", (PyCFunction)graph_lost, METH_O, nullptr},
     {"isEmpty", (PyCFunction)graph_is_empty, METH_NOARGS, nullptr},
     {"flush", (PyCFunction)graph_flush, METH_NOARGS, nullptr},
     {"materialize", (PyCFunction)graph_materialize, METH_O, nullptr},
@@ -1060,6 +1126,7 @@ PyMethodDef graph_methods[] = {
     {nullptr, nullptr, 0, nullptr}};
 PyMemberDef graph_members[] = {
     {"runtime", T_OBJECT_EX, offsetof(Graph, runtime), 0, nullptr},
+    {"_others", T_OBJECT, offsetof(Graph, others), 0, nullptr},
     {nullptr, 0, 0, 0, nullptr}};
 
 PyTypeObject BufferType = {PyVarObject_HEAD_INIT(nullptr, 0)};

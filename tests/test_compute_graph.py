@@ -699,6 +699,80 @@ def test_calls_of_the_runtime_that_are_replaced_are_called(owner, names, monkeyp
     be.releaseResources()
 
 
+class Matrix:
+    """No Tensor, but all that a graph asks of one."""
+
+    def __init__(self, rows, cols, values=None):
+        self.rows, self.cols, self._gpu_tag, self._data = rows, cols, None, values
+
+    @property
+    def data(self):
+        if self._data is None:
+            self._data = np.zeros((self.rows, self.cols), np.float32)
+        return self._data
+
+    def setGpuTag(self, tag):
+        old, self._gpu_tag = self._gpu_tag, tag
+        if old is not None and old is not tag:
+            old.graph.tensorLetGo(old)
+
+
+def _host_tensor(values):
+    t = Tensor(*values.shape)
+    t._data = values
+    return t
+
+
+def test_objects_that_stand_in_for_a_tensor_are_taken():
+    """An object with a tensor's attributes as operand, in place, read back, dropped and released: the calls that tensors make."""
+    calls = []
+    for make in (_host_tensor, lambda v: Matrix(*v.shape, v)):
+        rt = RecordingRuntime()
+        rt.downloadResult = [9.0, 8.0, 7.0, 6.0]
+        be = HipBackend(rt)
+        Tensor.setBackend(be)
+        a, b = make(np.array([[1, 2], [3, 4]], np.float32)), make(np.array([[5, 6], [7, 8]], np.float64).T)
+        blank = make(np.zeros((2, 2), np.float32)) if make is _host_tensor else Matrix(2, 2)
+        dropped = be.add(a, b)
+        be.multiplyInPlace(a, blank)
+        be.materializeTensor(a)
+        assert a._data.tolist() == [[9, 8], [7, 6]] and not a._gpu_tag.cpuStale
+        out = be.matmul(b, a)
+        b._gpu_tag.needsUpload = True
+        be.addScalarInPlace(b, 1.0)
+        be.reluInPlace(b)
+        del dropped
+        be.materializeTensor(out)
+        held = blank._gpu_tag.id
+        del blank
+        be.graph.flush()
+        assert list(rt.releaseCalls[-1][0]) == [held]
+        be.subtract(a, out)
+        be.releaseResources()
+        assert a._gpu_tag is None and b._gpu_tag is None and b._data.tolist() == [[9, 8], [7, 6]]
+        calls.append(_calls(rt))
+    plain, other = calls
+    assert other == plain
+    graph = ComputeGraph(RecordingRuntime())
+    with pytest.raises(TypeError):
+        graph.materialize(np.zeros((1, 1)))
+    m, t = Matrix(1, 1), Tensor(1, 1)
+    buf = graph.ensureGpuBuffer(m)                                     # from one kind to the other and back
+    graph.bindTensorToBuffer(t, buf)
+    m.setGpuTag(None)
+    graph.flush()
+    assert not graph.runtime.releaseCalls
+    graph.bindTensorToBuffer(m, buf)
+    t.setGpuTag(None)
+    graph.flush()
+    assert not graph.runtime.releaseCalls
+    gone = weakref.ref(graph)
+    del graph, buf
+    m.setGpuTag(None)
+    gc.collect()
+    assert gone() is None
+
+
 def test_a_tensor_class_with_a_set_gpu_tag_of_its_own_has_it_called():
     class Watching(Tensor):
         def setGpuTag(self, tag):
