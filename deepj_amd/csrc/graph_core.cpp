@@ -36,6 +36,32 @@ PyTypeObject *g_tensor_class;                                      // deepj_amd.
 std::unordered_map<int, std::pair<int, std::vector<int>>> g_op_meta;     // opcode -> stride, buffer slots
 int g_fill_op;
 
+// Attributes as a class in Python has them: a size is whatever counts (numpy's integers too), a flag whatever is true or not.
+template <class T> T &at_offset(PyObject *o, void *offset) { return *reinterpret_cast<T *>(reinterpret_cast<char *>(o) + reinterpret_cast<size_t>(offset)); }
+bool deleted(PyObject *v) {
+    if (v) return false;
+    PyErr_SetString(PyExc_AttributeError, "can't delete attribute");
+    return true;
+}
+PyObject *get_size(PyObject *o, void *offset) { return PyLong_FromSsize_t(at_offset<Py_ssize_t>(o, offset)); }
+int set_size(PyObject *o, PyObject *v, void *offset) {
+    if (deleted(v)) return -1;
+    PyObject *number = PyNumber_Long(v);
+    const Py_ssize_t n = number ? PyLong_AsSsize_t(number) : -1;
+    Py_XDECREF(number);
+    if (n == -1 && PyErr_Occurred()) return -1;
+    at_offset<Py_ssize_t>(o, offset) = n;
+    return 0;
+}
+PyObject *get_flag(PyObject *o, void *offset) { return PyBool_FromLong(at_offset<char>(o, offset)); }
+int set_flag(PyObject *o, PyObject *v, void *offset) {
+    const int is = deleted(v) ? -1 : PyObject_IsTrue(v);
+    if (is < 0) return -1;
+    at_offset<char>(o, offset) = (char)is;
+    return 0;
+}
+#define ATTRIBUTE(name, kind, type, field) {name, get_##kind, set_##kind, nullptr, reinterpret_cast<void *>(offsetof(type, field))}
+
 // ── GpuBuffer ───────────────────────────────────────────────────────────────
 struct Buffer {
     PyObject_HEAD
@@ -78,13 +104,15 @@ void buffer_dealloc(Buffer *self) {
 PyObject *buffer_float_count(Buffer *self, PyObject *) { return PyLong_FromSsize_t(self->rows * self->cols); }
 PyMemberDef buffer_members[] = {
     {"id", T_INT, offsetof(Buffer, id), 0, nullptr},
-    {"rows", T_PYSSIZET, offsetof(Buffer, rows), 0, nullptr},
-    {"cols", T_PYSSIZET, offsetof(Buffer, cols), 0, nullptr},
-    {"needsUpload", T_BOOL, offsetof(Buffer, needs_upload), 0, nullptr},
-    {"cpuStale", T_BOOL, offsetof(Buffer, cpu_stale), 0, nullptr},
-    {"allocatedOnGpu", T_BOOL, offsetof(Buffer, allocated), 0, nullptr},
     {"graph", T_OBJECT, offsetof(Buffer, graph), 0, nullptr},
     {nullptr, 0, 0, 0, nullptr}};
+PyGetSetDef buffer_getset[] = {
+    ATTRIBUTE("rows", size, Buffer, rows),
+    ATTRIBUTE("cols", size, Buffer, cols),
+    ATTRIBUTE("needsUpload", flag, Buffer, needs_upload),
+    ATTRIBUTE("cpuStale", flag, Buffer, cpu_stale),
+    ATTRIBUTE("allocatedOnGpu", flag, Buffer, allocated),
+    {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyMethodDef buffer_methods[] = {{"floatCount", (PyCFunction)buffer_float_count, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 
 // ── tensors ─────────────────────────────────────────────────────────────────
@@ -246,12 +274,12 @@ PyObject *tensor_set_tag(Tensor *t, PyObject *tag) {
     Py_RETURN_NONE;
 }
 PyMemberDef tensor_members[] = {
-    {"rows", T_PYSSIZET, offsetof(Tensor, rows), 0, nullptr},
-    {"cols", T_PYSSIZET, offsetof(Tensor, cols), 0, nullptr},
     {"_data", T_OBJECT, offsetof(Tensor, data), 0, nullptr},
     {"_gpu_tag", T_OBJECT, offsetof(Tensor, tag), 0, nullptr},
     {nullptr, 0, 0, 0, nullptr}};
 PyGetSetDef tensor_getset[] = {
+    ATTRIBUTE("rows", size, Tensor, rows),
+    ATTRIBUTE("cols", size, Tensor, cols),
     {"data", (getter)tensor_data, (setter)tensor_set_data, "The host copy as it is (zeros before anything was put there); numpy() brings it up to date first.", nullptr},
     {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyMethodDef tensor_methods[] = {
@@ -1211,6 +1239,7 @@ PyMODINIT_FUNC PyInit__graph_core() {
     BufferType.tp_clear = (inquiry)buffer_clear;
     BufferType.tp_dealloc = (destructor)buffer_dealloc;
     BufferType.tp_members = buffer_members;
+    BufferType.tp_getset = buffer_getset;
     BufferType.tp_methods = buffer_methods;
 
     TensorType.tp_name = "deepj_amd._graph_core.TensorCore";

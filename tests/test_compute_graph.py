@@ -773,6 +773,25 @@ def test_objects_that_stand_in_for_a_tensor_are_taken():
     assert gone() is None
 
 
+def test_sizes_and_flags_take_what_counts():
+    """numpy's integers and truth values, as attributes of a class in Python do."""
+    t, b = Tensor(2, 3), GpuBuffer(1, 2, 3, False)
+    for o in (t, b):
+        for name, value in (("rows", np.int64(4)), ("cols", np.int32(5)), ("rows", True), ("cols", 6)):
+            setattr(o, name, value)
+            assert getattr(o, name) == value and type(getattr(o, name)) is int
+        for wrong in ("a", None):
+            with pytest.raises((TypeError, ValueError)):
+                o.rows = wrong
+        assert (o.rows, o.cols) == (1, 6)
+    for name in ("needsUpload", "cpuStale", "allocatedOnGpu"):
+        for value in (np.bool_(True), 0, 1, False):
+            setattr(b, name, value)
+            assert getattr(b, name) is bool(value)
+    b.id = np.int64(7)
+    assert b.id == 7 and b.floatCount() == 6
+
+
 def test_a_tensor_class_with_a_set_gpu_tag_of_its_own_has_it_called():
     class Watching(Tensor):
         def setGpuTag(self, tag):
