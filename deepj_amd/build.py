@@ -4,9 +4,12 @@
 """
 from __future__ import annotations
 
+import glob
+import hashlib
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -103,16 +106,29 @@ def _compile(item):
     return obj, out
 
 
+def graph_core_path() -> str:
+    """The recording half's file for this Python and this source: one built for another version or from other source is none."""
+    with open(os.path.join(CSRC, "graph_core.cpp"), "rb") as f:
+        source = hashlib.sha256(f.read()).hexdigest()[:12]
+    return os.path.join(HERE, f"_graph_core-{source}{sysconfig.get_config_var('EXT_SUFFIX')}")
+
+
 def build_graph_core() -> str:
     """The recording half of the tensor backend, a CPython extension (host code only)."""
-    import sysconfig
-    lib = os.path.join(HERE, "_graph_core.so")
+    lib = graph_core_path()
     cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-fvisibility=hidden", "-I", sysconfig.get_paths()["include"],
            os.path.join(CSRC, "graph_core.cpp"), "-o", lib + f".{os.getpid()}"]
-    r = subprocess.run(cmd, capture_output=True, text=True)
+    try:
+        r = subprocess.run(cmd, capture_output=True, text=True)
+    except FileNotFoundError:
+        raise RuntimeError(f"{lib} is not built, and there is no g++ to build it with (run: python -m deepj_amd.build)") from None
     if r.returncode != 0:
         raise RuntimeError("g++ failed on graph_core.cpp:\n" + r.stdout + r.stderr)
     os.replace(lib + f".{os.getpid()}", lib)        # (this process may have the present one loaded)
+    for old in glob.glob(os.path.join(HERE, "_graph_core*.so")):
+        suffix = sysconfig.get_config_var("EXT_SUFFIX")
+        if old != lib and (old.endswith(suffix) or os.path.basename(old) == "_graph_core.so"):
+            os.remove(old)
     return lib
 
 

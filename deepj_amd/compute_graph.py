@@ -10,21 +10,34 @@ protocol the Java class speaks (same encodings, same call order).
 """
 from __future__ import annotations
 
+import importlib.util
+import os
 import struct
+import sys
 import weakref
 from typing import Protocol
 
 import numpy as np
 
 from . import opcodes as op
+from .build import build_graph_core, graph_core_path
 
-try:
-    from . import _graph_core
-except ImportError:                             # not built yet
-    from .build import build_graph_core
-    build_graph_core()
-    from . import _graph_core
 
+
+def _load_graph_core():
+    name = __package__ + "._graph_core"
+    if name not in sys.modules:
+        path = graph_core_path()
+        if not os.path.exists(path):            # not built yet
+            build_graph_core()
+        spec = importlib.util.spec_from_file_location(name, path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        sys.modules[name] = module
+    return sys.modules[name]
+
+
+_graph_core = _load_graph_core()
 GpuBuffer = _graph_core.GpuBuffer               # GpuBuffer.java:9-32
 
 
