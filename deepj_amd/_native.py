@@ -296,7 +296,8 @@ class HipNative:
     @staticmethod
     def profileOps(cmd_stream, iters: int, max_ops: int = 4096, detail: bool = False):
         """Mean kernel time (microseconds) of every op of the stream: a start and a stop event on each of the op's
-        dispatches, summed per op.  detail=True also returns the op's longest dispatch (its main kernel) and its
+        dispatches, summed per op; -1 for one that launched nothing, as those a launch of an op in front takes along.
+        detail=True also returns the op's longest dispatch (its main kernel) and its
         number of dispatches."""
         cmd = _ids(cmd_stream)
         out = np.empty(max_ops, dtype=np.float32)

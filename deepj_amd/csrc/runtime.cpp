@@ -519,7 +519,6 @@ struct Cursor {
     bool dry;          // validate only
     Scratch need;      // collected in the dry pass
     int32_t skip = 0;  // words behind this op whose ops its launch has taken along
-    bool alone = false; // every op by itself (per-op timing)
     int32_t done[kTransposes] = {};     // ops further on that have run already, in order: done[next_done] is the next one to pass
     int n_done = 0, next_done = 0;
     int32_t pieces_pos = -1;            // the op that finds its rows' pieces made, and where in their block; the dry pass knows by shapes
@@ -830,7 +829,7 @@ void exec_one(Cursor &c) {
                (was.plain ? !(flags & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM))
                           : (flags & (DJ_LIN_RMSNORM | DJ_LIN_LAYERNORM)) && was.gamma_id == w[8] && was.beta_id == (flags & DJ_LIN_LAYERNORM ? w[10] : -1));
     };
-    if (run && !c.alone && op < DJ_OP_Q8_QUANTIZE && exec_chain(c)) return;
+    if (run && op < DJ_OP_Q8_QUANTIZE && exec_chain(c)) return;
     switch (op) {
         case DJ_OP_ADD: case DJ_OP_SUBTRACT: case DJ_OP_MULTIPLY: case DJ_OP_DIVIDE: case DJ_OP_RELU_BACKWARD:
         case DJ_OP_GELU_BACKWARD: {
@@ -874,7 +873,7 @@ void exec_one(Cursor &c) {
             int64_t rows = w[3], cols = w[4]; need_positive(op, "rows", rows); need_positive(op, "cols", cols);
             const float *a = buf(w[1], rows * cols, op, "in");
             float *o = buf(w[2], rows * cols, op, "out");
-            if (run && !c.alone && c.next_done == c.n_done && exec_transposes(c)) break;
+            if (run && c.next_done == c.n_done && exec_transposes(c)) break;
             if (run) launch_transpose(s, a, o, (int)rows, (int)cols);
             break;
         }
@@ -953,7 +952,7 @@ void exec_one(Cursor &c) {
                 t.lr = bits_to_float(v[5]); t.beta1 = bits_to_float(v[6]); t.beta2 = bits_to_float(v[7]); t.eps = bits_to_float(v[8]);
                 t.wd = bits_to_float(v[9]); t.bc1 = bits_to_float(v[10]); t.bc2 = bits_to_float(v[11]);
                 v += 13;
-            } while (run && !c.alone && count < kAdamTensors && v + 13 <= c.cmd + c.len && v[0] == DJ_OP_ADAMW_UPDATE && !shares(v));
+            } while (run && count < kAdamTensors && v + 13 <= c.cmd + c.len && v[0] == DJ_OP_ADAMW_UPDATE && !shares(v));
             if (run) {
                 launch_adamw(s, batch, count);
                 c.skip = (int32_t)(v - w) - 13;
@@ -1938,8 +1937,9 @@ int deepj_hip_clock_probe(const int32_t *cmd, int32_t len, int32_t iters, int32_
 }
 
 // Per-op kernel durations: every kernel dispatch of every op of the stream carries a start and a stop event, the
-// stream runs `iters` times in order, and us_per_op[i] receives the mean over the passes of the summed begin-to-end
-// times of op i's dispatches in microseconds (-1 for an op that launched nothing).  Optional outputs of the same
+// stream runs `iters` times in order with the launches of a flush, and us_per_op[i] receives the mean over the passes of the
+// summed begin-to-end times of op i's dispatches in microseconds (-1 for an op that launched nothing: also one that a launch of
+// an op in front of it has taken along, with all of that launch's time there).  Optional outputs of the same
 // length: us_longest[i], the longest single dispatch of the op (its main kernel), and dispatches[i], how many
 // dispatches the op made (at most kMaxTimedLaunches of them are timed).
 int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float *us_per_op, int32_t capacity,
@@ -1968,15 +1968,20 @@ int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float 
             for (auto &e : ev) DJ_HIP(hipEventCreate(&e));
             for (int it = 0; it < iters; it++) {
                 g.chain.valid = false;
+                Cursor c{cmd, len, 0, false, 0};                     // (as walk)
                 for (int i = 0; i < n; i++) {
-                    Cursor c{cmd, len, starts[(size_t)i], false, 0};
-                    c.alone = true;
+                    launches[(size_t)i] = 0;
+                    if (c.pos > starts[(size_t)i]) continue;         // an op in front has taken it along
+                    const int32_t stride = stride_of(cmd[c.pos]);
+                    if (c.next_done < c.n_done && c.done[c.next_done] == c.pos) { c.next_done++; c.pos += stride; continue; }
                     g_launch_timing.pairs = ev.data() + (size_t)per_op * i;
                     g_launch_timing.used = 0;
                     g_launch_timing.armed = true;
                     exec_one(c);
                     launches[(size_t)i] = g_launch_timing.used;
                     g_launch_timing.armed = false;
+                    c.pos += stride + c.skip;
+                    c.skip = 0;
                 }
                 DJ_HIP(hipStreamSynchronize(g.stream));
                 for (int i = 0; i < n; i++) {

@@ -5,7 +5,7 @@ leave results alone and end by themselves."""
 import numpy as np
 import pytest
 
-from deepj_amd import HipNative
+from deepj_amd import HipNative, opcodes as op
 from deepj_amd.fused import DeviceBuffers, Stream
 
 pytestmark = pytest.mark.gpu
@@ -65,6 +65,30 @@ def test_profile_ops_counts_every_dispatch_of_an_op_and_changes_no_result(dev):
     assert abs(total[1] - longest[1]) < 1e-3 and abs(total[2] - longest[2]) < 1e-3
     assert np.array_equal(dev.download(out, (m, n)), ref_out) and np.array_equal(dev.download(out1, (1, n)), ref_out1)
     assert np.allclose(st.profile(2), total, rtol=0.5)
+
+
+def test_profile_ops_makes_the_launches_of_a_flush(dev):
+    """Element-wise ops, transposes and AdamW updates that run as one launch: its time at the first of them, nothing at the others."""
+    n = 1 << 16
+    ids = [dev.alloc(n) for _ in range(8)]
+    st = Stream()
+    for i in ids:
+        st.fill(i, 0x3f800000, n)
+    a, b, c, d, e, f, g, h = ids
+    st.emit(op.OP_ADD, a, b, c, n).emit(op.OP_MULTIPLY, c, b, d, n).matmul(a, b, e, 256, 256, 256).emit(op.OP_SUBTRACT, e, d, c, n)
+    st.emit(op.OP_TRANSPOSE, a, f, 256, 256).emit(op.OP_SUM_ROWS, c, g, 256, 256).emit(op.OP_TRANSPOSE, b, h, 128, 512)
+    for w, grad, mt, vt in ((c, a, e, f), (d, b, g, h)):
+        st.emit(op.OP_ADAMW_UPDATE, w, grad, mt, vt, 0, 0, 0, 0x3f800000, 0, 0x3f800000, 0x3f800000, n // 2)
+    st.run()
+    before = [dev.download(i, (n,)).copy() for i in ids]
+    us, longest, count = HipNative.profileOps(st.array(), 3, detail=True)
+    # the chain takes its product along; the second transpose goes with the first; the second update too
+    assert list(count[:13]) == [1] * 8 + [2, 0, 0, 0, 1] and count[13] >= 1 and list(count[14:]) == [0, 1, 0], list(count)
+    assert all((t > 0) == (k > 0) and (t == -1.0 or k > 0) for t, k in zip(us, count)) and all((t > 0) == (k > 0) for t, k in zip(longest, count))
+    alone = HipNative.profileOps(Stream().emit(op.OP_MULTIPLY, c, b, d, n).array(), 3, detail=True)[2]
+    assert list(alone) == [1]
+    st.run()
+    assert all(np.array_equal(dev.download(i, (n,)), x) for i, x in zip(ids, before))
 
 
 def test_clock_probe_samples_a_plausible_clock_and_ends_by_itself(dev):
