@@ -869,7 +869,8 @@ bool q8_gemm_f16_rope_ok(int m, int d, int k) {
 // rows, us, with the copy and from the int8 weights: 32 x 11264 over 2048 20.1, 16.8 (and 36.7, 28.8 with the product behind it, which
 // takes its pieces), 32 x 22016 over 4096 55.4, 33.8 (85.6, 66.3), 16 x 22016 over 12288 177, 113; over 312 shapes 1.36 times as
 // long with it in the median, never less from 1024 k on; below that the int8 side's own conversions show: 20 x 50000 over 256 12.7,
-// 13.1 and 32 x 32768 over 64 8.6, 9.4.  16 rows, the fewest that the copy's route is held to, stay on it.  Above 32 rows both ways: 64 x 22016 over 4096 57.7, 48.7, 64 x 12288 30.2, 32.1.
+// 13.1 and 32 x 32768 over 64 8.6, 9.4.  (16 rows stay on the copy, which is the slower way for them too: that a copy is read from
+// 16 rows on is what the interface says.)  Above 32 rows both ways: 64 x 22016 over 4096 57.7, 48.7, 64 x 12288 30.2, 32.1.
 bool q8_copy_pays(int m, int k) { return m <= kMinRowsPrepared || m > 32 || k < 1024; }
 bool q8_gemm_f16_shape_ok(int m, int n_rows, int k, bool prepared) { return q8_gemm_f16_tile_rows(m, n_rows, k, prepared) != 0; }
 void q8_gemm_f16_tile(int m, int n_rows, int k, int *tile_rows, int *tile_cols, int *k_shares, bool prepared) {

@@ -729,7 +729,8 @@ bool exec_chain(Cursor &c) {
     // 5 behind products 16.5 / 27.6; 1024 x 7000: 2 ops 20 .. 27 / 18 .. 22, 4 ops 38 / 47; 2048 x 8192: 41 .. 52 / 38 .. 41, 91 / 106.
     if (count < (chain.n < (1 << 17) ? 3 : chain.n <= (1 << 20) ? 2 : 4)) return false;
 
-    // A result takes the slot of an operand that nothing needs any more, or a free one: an op that would need a ninth ends the chain.
+    // A result takes the slot of an operand that nothing needs any more, or a free one.  A chain that would need a ninth is not
+    // taken: its first op runs by itself, and the chain from the second on is looked at anew.
     int last_use[kChainExt + kChainOps], slot_of[kChainExt + kChainOps];       // values: the external ones, then the results
     auto value = [&](int x) { return x >= 0 ? x : kChainExt + (-1 - x); };
     for (int &u : last_use) u = -1;

@@ -3,7 +3,7 @@ write in common."""
 import numpy as np
 import pytest
 
-from deepj_amd import opcodes as op
+from deepj_amd import HipNative, opcodes as op
 from deepj_amd.fused import DeviceBuffers, Stream
 
 pytestmark = pytest.mark.gpu
@@ -84,6 +84,83 @@ def test_a_chain_has_the_bits_of_its_operations(rows, cols):
         for k, (x, y) in enumerate(zip(*results)):
             same = (x.view(np.uint32) == y.view(np.uint32)) | (np.isnan(x) & np.isnan(y))
             assert same.all(), (trial, k, ops)
+
+
+@pytest.mark.parametrize("rows,cols,least", [(255, 513, 3), (257, 511, 2), (1021, 1027, 2), (1025, 1031, 4), (2051, 4111, 4)])
+def test_the_operations_that_make_a_chain(rows, cols, least):
+    """From how many operations on they run as one launch, at sizes on either side of each rule (2^17 and 2^20 values) and past what
+    one pass of a launch covers (2^23), none a multiple of four, vectors of both kinds among the operands: one launch, and the bits
+    of the operations one by one."""
+    rng, n = np.random.default_rng(rows), rows * cols
+    a, b, row, col = (rng.standard_normal(s).astype(np.float32) for s in (n, n, cols, rows))
+    dev = DeviceBuffers()
+    try:
+        A, B, R, C = (dev.upload(v) for v in (a, b, row, col))
+        outs = [dev.alloc(n) for _ in range(4)]
+        words = [[op.OP_MULTIPLY_BROADCAST_COLS, A, C, outs[0], rows, cols], [op.OP_ADD_ROW_VECTOR, outs[0], R, outs[1], rows, cols],
+                 [op.OP_SIGMOID, outs[1], outs[2], n], [op.OP_SUBTRACT, outs[2], B, outs[3], n]]
+        for length in (2, 3, 4):
+            stream = Stream()
+            for w in words[:length]:
+                stream.emit(*w)
+                Stream().emit(*w).run()
+            want = [dev.download(o, (n,)).copy() for o in outs[:length]]
+            for o in outs:
+                Stream().fill(o, 0, n).run()
+            stream.run()
+            for o, x in zip(outs, want):
+                assert np.array_equal(dev.download(o, (n,)).view(np.uint32), x.view(np.uint32))
+            launches = [int(c) for c in HipNative.profileOps(stream.array(), 1, detail=True)[2]]
+            assert launches == ([1] + [0] * (length - 1) if length >= least else [1] * length), (length, launches)
+    finally:
+        dev.release_all()
+
+
+def test_values_that_need_a_ninth_slot_run_in_shorter_chains():
+    """Six operands and three results needed to the end are more than a chain holds: the same bits all the same."""
+    rng, n = np.random.default_rng(1), 1000
+    dev = DeviceBuffers()
+    try:
+        e = [dev.upload(rng.standard_normal(n).astype(np.float32)) for _ in range(6)]
+        r = [dev.alloc(n) for _ in range(8)]
+        words = [[op.OP_ADD, e[0], e[1], r[0], n], [op.OP_SUBTRACT, e[2], e[3], r[1], n], [op.OP_MULTIPLY, e[4], e[5], r[2], n], [op.OP_ADD, e[0], r[0], r[3], n],
+                 [op.OP_MULTIPLY, e[1], e[2], r[4], n], [op.OP_SUBTRACT, r[3], r[1], r[5], n], [op.OP_ADD, e[3], e[4], r[6], n], [op.OP_DIVIDE, r[2], e[5], r[7], n]]
+        for w in words:
+            Stream().emit(*w).run()
+        want = [dev.download(o, (n,)).copy() for o in r]
+        stream = Stream()
+        for w in words:
+            stream.emit(*w)
+        for o in r:
+            Stream().fill(o, 0, n).run()
+        stream.run()
+        assert all(np.array_equal(dev.download(o, (n,)), x) for o, x in zip(r, want))
+        launches = [int(c) for c in HipNative.profileOps(stream.array(), 1, detail=True)[2]]
+        assert launches[0] == 1 and launches[1] == 1 and sum(launches) < len(words), launches
+    finally:
+        dev.release_all()
+
+
+def test_transposes_of_any_shape_in_one_launch():
+    """Eight that depend on nothing, of different rows and columns (one tile, a tile's edge on either side, rows, columns), between
+    operations that they go past: all in the first one's launch."""
+    rng = np.random.default_rng(2)
+    shapes = [(1, 70), (70, 1), (32, 32), (33, 31), (5, 257), (300, 40), (64, 1003), (31, 97)]
+    dev = DeviceBuffers()
+    try:
+        values = [rng.standard_normal(s).astype(np.float32) for s in shapes]
+        ins, outs = [dev.upload(v) for v in values], [dev.alloc(v.size) for v in values]
+        x = dev.upload(rng.standard_normal((20, 30)).astype(np.float32))
+        stream = Stream()
+        for (rows, cols), i, o in zip(shapes, ins, outs):
+            stream.emit(op.OP_TRANSPOSE, i, o, rows, cols).emit(op.OP_EXP, x, x, 600)
+        stream.run()
+        for v, o in zip(values, outs):
+            assert np.array_equal(dev.download(o, v.T.shape), v.T)
+        launches = [int(c) for c in HipNative.profileOps(stream.array(), 1, detail=True)[2]]
+        assert launches == [1, 1] + [0, 1] * 7, launches
+    finally:
+        dev.release_all()
 
 
 def test_a_product_between_two_operations_that_depends_on_one_of_them_stays_there():
