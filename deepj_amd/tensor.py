@@ -21,6 +21,10 @@ class Tensor(_graph_core.TensorCore):
     def __getstate__(self): return self.rows, self.cols, self._data, self._gpu_tag, self.__dict__
 
     def __setstate__(self, state):
+        if isinstance(state, dict):             # attributes by name
+            for name, value in state.items():
+                setattr(self, name, value)
+            return
         self.rows, self.cols, self._data, self._gpu_tag, extra = state
         self.__dict__.update(extra)
 

@@ -821,6 +821,14 @@ def test_cycles_through_tensors_are_collected(holder):
     assert [r() for r in gone] == [None] * 3
 
 
+def test_a_tensor_saved_as_its_attributes_loads():
+    """As tensors were pickled while all they held was in their dictionary, and as a derived class may save itself."""
+    state = {"_gpu_tag": None, "_data": np.array([[1.0, 2.0]], np.float32), "rows": 1, "cols": 2, "note": "kept"}
+    t = Tensor.__new__(Tensor)
+    t.__setstate__(state)
+    assert (t.rows, t.cols, t.note, t.getGpuTag()) == (1, 2, "kept", None) and t.numpy().tolist() == [[1.0, 2.0]]
+
+
 def test_values_of_other_layouts_travel_as_fp32_rows(graph, rt):
     """Host arrays that are not contiguous fp32 are packed on the way out, filled on the way back; a size that does not fit is refused."""
     t = Tensor(2, 3)
