@@ -145,7 +145,7 @@ class ComputeGraph(_graph_core.GraphCore):
         carrier = _tensor_class()(o.rows, o.cols)
         carrier._data = o._data
         self._download(buf, carrier)
-        if o._data is None:
+        if o._data is not carrier._data:
             o._data = carrier._data
 
     def _bindOther(self, o, buf):
@@ -342,7 +342,10 @@ def pack_f32(t) -> np.ndarray:
 def unpack_f32_into(src: np.ndarray, dst) -> None:
     if src.size != dst.rows * dst.cols:
         raise ValueError(f"Size mismatch: src has {src.size} floats but tensor is {dst.rows}x{dst.cols}")
-    dst.data[...] = np.reshape(src, (dst.rows, dst.cols))
+    if dst.data.flags.writeable:
+        dst.data[...] = np.reshape(src, (dst.rows, dst.cols))
+    else:
+        dst._data = np.reshape(src, (dst.rows, dst.cols)).astype(np.float32, copy=False)
 
 
 def from_int_column(values) -> "object":

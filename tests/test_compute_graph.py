@@ -821,6 +821,22 @@ def test_cycles_through_tensors_are_collected(holder):
     assert [r() for r in gone] == [None] * 3
 
 
+@pytest.mark.parametrize("make", [_host_tensor, lambda v: Matrix(*v.shape, v)])
+def test_results_reach_a_tensor_whose_host_array_cannot_be_written(graph, rt, make):
+    """A view of bytes, of a file mapped to be read: the tensor gets an array of its own, and what it was made from stays as it is."""
+    raw = np.array([1.0, 2.0], np.float32).tobytes()
+    t = make(np.frombuffer(raw, np.float32).reshape(1, 2))
+    buf = graph.ensureGpuBuffer(t)
+    graph.flush()
+    rt.downloadResult = [5.0, 6.0]
+    for release in (lambda: graph.materialize(t), graph.releaseAll):
+        buf.cpuStale = True
+        release()
+        assert t.data.tolist() == [[5.0, 6.0]] and t.data.flags.writeable
+        assert raw == np.array([1.0, 2.0], np.float32).tobytes()
+        rt.downloadResult = [5.0, 6.0]
+
+
 def test_a_tensor_saved_as_its_attributes_loads():
     """As tensors were pickled while all they held was in their dictionary, and as a derived class may save itself."""
     state = {"_gpu_tag": None, "_data": np.array([[1.0, 2.0]], np.float32), "rows": 1, "cols": 2, "note": "kept"}
