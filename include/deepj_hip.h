@@ -238,9 +238,9 @@ enum {
      * LATENT_DECODE [op, q, ckv, latent, wukv, state, cosT, sinT, records, out, H, hd, rank, maxSeq, layer]
      *     one token's attention over latent rows (J/.../MultiHeadLatentAttention.java:98-123): ckv is appended to the layer's
      *     rows of `latent` [layers][maxSeq][rank] at position state[0]; out [H * hd] = attention of q (not rotated) over
-     *     K = RoPE(rows . Wuk) and V = rows . Wuv, wukv a Q8 weight with the 2 * H * hd output rows Wuk, Wuv.  records: scratch
-     *     of H * deepj_hip_latent_decode_splits(H, hd, rank, maxSeq) * (hd + 4) floats (its contents are not defined); refused where
-     *     that is 0.
+     *     K = RoPE(rows . Wuk) and V = rows . Wuv, wukv a Q8 weight with the 2 * H * hd output rows Wuk, Wuv.  records: a
+     *     buffer of H * deepj_hip_latent_decode_splits(H, hd, rank, maxSeq) * (hd + 4) floats, checked but left as it is (the
+     *     launches leave each other more than it holds, in a block of the library's); refused where that is 0.
      * Q8_LINEAR_PAIR [op, x, gamma, K, weightA, outA, nA, weightB, outB, nB]
      *     two Q8_LINEARs of one row with the same x and RMSNorm gain in one launch, the same bits; K a multiple of 4 up to 4096
      */
