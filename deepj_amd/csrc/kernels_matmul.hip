@@ -466,6 +466,7 @@ __global__ void __launch_bounds__(64 * WC * KS) k_matmul_split(const float *__re
     auto limit = [&](uint32_t most) { return most ? (__builtin_bit_cast(float, most) + 0.5f) * 0x1p-60f * scale : -INFINITY; };    // (zeros lose nothing)
     const int c = threadIdx.x % (32 * WC);
     const float of_col = limit(col_most[c]);
+    for (int o = threadIdx.x; o < kRows; o += 64 * kWaves) row_most[o] = __builtin_bit_cast(uint32_t, limit(row_most[o]));    // (read behind a barrier)
     auto store = [&](int i, auto &&of, auto &&wanted) {
         __syncthreads();
 #pragma unroll
@@ -483,7 +484,7 @@ __global__ void __launch_bounds__(64 * WC * KS) k_matmul_split(const float *__re
 #pragma unroll
     for (int i = 0; i < TM; i++)
         store(i, [&](int e) { return acc[i][e] + low[i][e]; }, [&](int row, float v) {
-            if (fabsf(v) <= 3.40282347e38f && !(fabsf(v) <= limit(row_most[row]) + of_col)) return true;
+            if (fabsf(v) <= 3.40282347e38f && !(fabsf(v) <= __builtin_bit_cast(float, row_most[row]) + of_col)) return true;
             atomicOr(&again[row * WC + (c >> 5)], 1u << (c & 31));
             atomicOr(&again_rows, 1u << (row >> 5));
             return false;
@@ -496,30 +497,37 @@ __global__ void __launch_bounds__(64 * WC * KS) k_matmul_split(const float *__re
     // have lost theirs: those outputs come from the fp32 instructions, the 32 rows around one as in k_matmul.  1000 x 2752 x 1024:
     // 46 us, 69 with a NaN in one row, 128 with nothing else in an operand, 95 with one of values near 1e-24 (whose sums cancel
     // to below the limit here and there); a thread an output, product behind product, took 259 and 3070.
-    const uint32_t col_off = (uint32_t)col * 4u;
+    // Lane and offsets are worked out anew, and few values are in flight: what this part keeps through the loops above, or holds
+    // beyond their registers, changes how those are scheduled (500 x 2752 x 1024 23.3 -> 24.2 us with 32 k a round).
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    const int lane_of = t & 63, wave_of = __builtin_amdgcn_readfirstlane(t >> 6), half_of = lane_of >> 5, l32_of = lane_of & 31;
+    const int col_of = n0 + 32 * (wave_of % WC) + l32_of;
+    const uint32_t col_off = (uint32_t)(col_of < N ? col_of : N - 1) * 4u;
+    const float *rows_of_tile = A + (int64_t)m0 * K;
 #pragma unroll 1
     for (int i = 0; i < TM; i++) {
         if (!(rows_again >> i & 1)) continue;
-        const int row = 32 * i + l32;
+        const int row = 32 * i + l32_of;
         const uint32_t row_off = (uint32_t)(row < M - m0 ? row : M - 1 - m0) * (uint32_t)K * 4u;
         floatx16 sum[2];
 #pragma unroll
         for (int e = 0; e < 16; e++) sum[0][e] = sum[1][e] = 0.0f;
         auto products = [&](int k0, bool whole) __attribute__((always_inline)) {
-            float av[16], bv[16];
+            float av[8], bv[8];
 #pragma unroll
-            for (int x = 0; x < 16; x++) {
-                const int k = k0 + 8 * (x >> 2) + 4 * half + (x & 3);
+            for (int x = 0; x < 8; x++) {
+                const int k = k0 + 8 * (x >> 2) + 4 * half_of + (x & 3);
                 const bool in = whole || k < K;
-                av[x] = in ? at_bytes(Am + k, row_off) : 0.0f;
+                av[x] = in ? at_bytes(rows_of_tile + k, row_off) : 0.0f;
                 bv[x] = in ? at_bytes(B + (int64_t)k * N, col_off) : 0.0f;
             }
 #pragma unroll
-            for (int x = 0; x < 16; x++) sum[x & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[x], bv[x], sum[x & 1], 0, 0, 0);
+            for (int x = 0; x < 8; x++) sum[x & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[x], bv[x], sum[x & 1], 0, 0, 0);
         };
-        int k0 = 32 * set;
+        int k0 = 16 * (wave_of / WC);
 #pragma unroll 1
-        for (; k0 + 32 <= K; k0 += 32 * KS) products(k0, true);
+        for (; k0 + 16 <= K; k0 += 16 * KS) products(k0, true);
         if (k0 < K) products(k0, false);
         store(i, [&](int e) { return sum[0][e] + sum[1][e]; }, [&](int r, float) { return (again[r * WC + (c >> 5)] >> (c & 31) & 1) != 0; });
     }
@@ -955,7 +963,8 @@ void launch_matmul_f32(hipStream_t s, const float *a, const float *b, float *out
     switch (matmul_kernel(m, n, k)) {
         case 0:
             // a tile per compute unit at most: more wavefronts share its K, with shorter stages so that their lines fit; up to two
-            // tiles of 16 x 16, those (768 of them: 8.5 us where 32 x 32 take 8.1 at 768 k; at 256 k and less all take about 4)
+            // tiles of 16 x 16, those (768 of them: 8.5 us where 32 x 32 take 8.1 at 768 k; at 256 k and less all take about 4).  They
+            // have no estimate of their own: where another tile's is below that of 32 x 32, it stays with that one.
             if (k > 256 && (int64_t)((m + 15) / 16) * ((n + 15) / 16) <= 512) launch_matmul_16(s, a, b, out, m, n, k);
             else if (blocks <= 256 && k > 256) launch_matmul<1, 1, 16, 1, 2>(s, a, b, out, m, n, k);
             else if (blocks <= 256) launch_matmul<1, 1, 8, 4, 2>(s, a, b, out, m, n, k);
