@@ -371,7 +371,7 @@ struct Methods {                           // attributes of a class as they were
         return all;
     }
 };
-Methods g_graph_methods, g_runtime_methods, g_native_methods;
+Methods g_tensor_methods, g_graph_methods, g_runtime_methods, g_native_methods;
 PyTypeObject *g_runtime_class, *g_native_class;                    // deepj_amd.HipGpuRuntime, HipNative
 PyObject *g_general;                       // compute_graph.py's {name: function of the graph}
 
@@ -471,9 +471,11 @@ int send_now(Graph *g, Buffer *b, Tensor *t) {
     return r;
 }
 
-Tensor *tensor(PyObject *o) { return PyObject_TypeCheck(o, &TensorType) ? reinterpret_cast<Tensor *>(o) : nullptr; }
+// What is looked into here: a tensor whose class leaves its sizes, values and buffer as Tensor has them.  One that does not is an
+// object that stands in for a tensor (ComputeGraph, compute_graph.py).
+Tensor *tensor(PyObject *o) { return PyObject_TypeCheck(o, &TensorType) && g_tensor_methods.same(Py_TYPE(o)) ? reinterpret_cast<Tensor *>(o) : nullptr; }
 Tensor *as_tensor(PyObject *o) {
-    if (Tensor *t = tensor(o)) return t;
+    if (PyObject_TypeCheck(o, &TensorType)) return reinterpret_cast<Tensor *>(o);
     PyErr_Format(PyExc_TypeError, "expected a Tensor, not %.100s", Py_TYPE(o)->tp_name);
     return nullptr;
 }
@@ -482,14 +484,6 @@ bool fits_words(Py_ssize_t rows, Py_ssize_t cols) {
     if (rows <= INT32_MAX && cols <= INT32_MAX && rows * cols <= INT32_MAX) return true;
     PyErr_Format(PyExc_OverflowError, "a buffer of %zdx%zd: more than 32 bits count", rows, cols);
     return false;
-}
-// setGpuTag, the class's own where it has one
-bool retag(Tensor *t, PyObject *tag) {
-    static PyObject *name = PyUnicode_InternFromString("setGpuTag"), *own = PyDict_GetItem(TensorType.tp_dict, name);
-    if (_PyType_Lookup(Py_TYPE(t), name) == own) { set_tag(t, tag); return true; }
-    PyObject *r = PyObject_CallMethodObjArgs(reinterpret_cast<PyObject *>(t), name, tag, nullptr);
-    Py_XDECREF(r);
-    return r != nullptr;
 }
 // A buffer held through what may run meanwhile: another thread while values are sent, a host array of some other class.
 struct Held {
@@ -527,7 +521,7 @@ Buffer *ensure(Graph *g, Tensor *t) {      // a reference of the caller's
     if (sent < 0 || (sent == 0 && !add_upload(g, b->id, t))) { Py_DECREF(b); Py_DECREF(b); return nullptr; }
     if (sent) Py_DECREF(b);
     else g->s->allocs.push_back(b);        // (takes the reference)
-    if (!retag(t, reinterpret_cast<PyObject *>(b))) { Py_DECREF(b); return nullptr; }
+    set_tag(t, reinterpret_cast<PyObject *>(b));
     track(g, b->id, t);
     return b;
 }
@@ -553,18 +547,17 @@ PyObject *output_tensor(Graph *g, Buffer *b) {
     Py_XSETREF(b->graph, reinterpret_cast<PyObject *>(g));
     return o;
 }
-bool bind(Graph *g, Tensor *t, Buffer *b) {
-    if (!retag(t, reinterpret_cast<PyObject *>(b))) return false;
+void bind(Graph *g, Tensor *t, Buffer *b) {
+    set_tag(t, reinterpret_cast<PyObject *>(b));
     track(g, b->id, t);
     Py_INCREF(g);
     Py_XSETREF(b->graph, reinterpret_cast<PyObject *>(g));
-    return true;
 }
 // The result of a recorded operation: a new tensor, or `into` on its new buffer.  Takes the caller's reference to out.
 PyObject *finish(Graph *g, Buffer *out, Tensor *into) {
     PyObject *r;
     if (!into) r = output_tensor(g, out);
-    else if ((r = bind(g, into, out) ? Py_None : nullptr)) Py_INCREF(r);
+    else { bind(g, into, out); r = Py_None; Py_INCREF(r); }
     Py_DECREF(out);
     return r;
 }
@@ -614,7 +607,7 @@ PyObject *graph_bind(Graph *g, PyObject *const *a, Py_ssize_t n) {
     if (!b) return nullptr;
     Tensor *t = tensor(a[0]);
     if (!t) return PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "_bindOther", "OO", a[0], a[1]);
-    if (!bind(g, t, b)) return nullptr;
+    bind(g, t, b);
     Py_RETURN_NONE;
 }
 PyObject *graph_let_go(Graph *g, PyObject *o) {
@@ -1088,11 +1081,7 @@ PyObject *graph_release_all(Graph *g, PyObject *) {
     for (int id : ids) {
         auto it = s->tensors.find(id);
         Tensor *t = it == s->tensors.end() ? nullptr : it->second;
-        if (!t) continue;
-        Py_INCREF(t);
-        const bool ok = retag(t, Py_None);
-        Py_DECREF(t);
-        if (!ok) return nullptr;
+        if (t) set_tag(t, Py_None);
     }
     if (!ids.empty() && !release_ids(g, ids)) return nullptr;
     while (!s->tensors.empty()) forget(g, s->tensors.begin()->first);
@@ -1184,6 +1173,10 @@ PyObject *set_tensor_class(PyObject *, PyObject *o) {
         PyErr_SetString(PyExc_TypeError, "a class derived from TensorCore");
         return nullptr;
     }
+    PyObject *names = Py_BuildValue("(sssssss)", "rows", "cols", "data", "_data", "_gpu_tag", "getGpuTag", "setGpuTag");
+    const bool ok = names && g_tensor_methods.take(reinterpret_cast<PyTypeObject *>(o), names);
+    Py_XDECREF(names);
+    if (!ok) return nullptr;
     Py_INCREF(o);
     g_tensor_class = reinterpret_cast<PyTypeObject *>(o);
     Py_RETURN_NONE;

@@ -699,6 +699,24 @@ def test_calls_of_the_runtime_that_are_replaced_are_called(owner, names, monkeyp
     be.releaseResources()
 
 
+def test_a_tensor_class_with_values_of_its_own_has_them_sent():
+    class Doubled(Tensor):
+        @property
+        def data(self):
+            return 2 * super().data
+    rt = RecordingRuntime()
+    be = HipBackend(rt)
+    t = Doubled(1, 2)
+    t._data = np.array([[1.0, 2.0]], np.float32)
+    out = be.add(t, Tensor.from2D([[0.0, 0.0]]))
+    be.graph.flush()
+    assert [list(v) for _, v in rt.uploads] == [[2.0, 4.0], [0.0, 0.0]] and out.getGpuTag().allocatedOnGpu
+    held = t.getGpuTag().id
+    del t
+    be.graph.flush()
+    assert list(rt.releaseCalls[-1][0]) == [held]
+
+
 class Matrix:
     """No Tensor, but all that a graph asks of one."""
 
