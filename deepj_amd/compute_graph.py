@@ -324,7 +324,7 @@ def _adamw(graph, opcode, w, g, mt, vt, lr, beta1, beta2, eps, weight_decay, bc1
 _graph_core.set_methods(
     {"binary": _binary, "unary": _unary, "scalar": _scalar, "shaped": _shaped, "pair": _pair, "rowBroadcast": _row_broadcast,
      "colBroadcast": _col_broadcast, "matmul": _matmul, "adamW": _adamw}, ComputeGraph,
-    ["ensureGpuBuffer", "newOutputBuffer", "createOutputTensor", "bindTensorToBuffer", "flush", "_emit", "recordBinary", "recordUnary",
+    ["ensureGpuBuffer", "newOutputBuffer", "createOutputTensor", "bindTensorToBuffer", "tensorLetGo", "flush", "_emit", "recordBinary", "recordUnary",
      "recordMultiplyScalar", "recordPow", "recordScalarUnary", "recordReduction", "recordRowBroadcast", "recordColBroadcast", "recordMatmul",
      "recordAdamWUpdate", *_SHAPED.values(), *_PAIRS.values()])
 

@@ -259,18 +259,28 @@ PyObject *tensor_get_tag(Tensor *t, PyObject *) {
     Py_INCREF(o);
     return o;
 }
-void set_tag(Tensor *t, PyObject *tag) {   // tag: borrowed
+Graph *plain_graph(PyObject *o);
+// tag: borrowed.  The graph that tracks the buffer it had is told; false: it raised something (the tag is in place all the same).
+bool set_tag(Tensor *t, PyObject *tag) {
     PyObject *old = t->tag;
     Py_INCREF(tag);
     t->tag = tag;
+    bool ok = true;
     if (old && old != tag && is_buffer(old)) {
         PyObject *g = reinterpret_cast<Buffer *>(old)->graph;
-        if (g && PyObject_TypeCheck(g, &GraphType)) reinterpret_cast<Graph *>(g)->s->maybe_orphans.push_back(reinterpret_cast<Buffer *>(old)->id);
+        if (Graph *plain = g ? plain_graph(g) : nullptr) {
+            plain->s->maybe_orphans.push_back(reinterpret_cast<Buffer *>(old)->id);
+        } else if (g && g != Py_None) {
+            PyObject *r = PyObject_CallMethod(g, "tensorLetGo", "O", old);
+            ok = r != nullptr;
+            Py_XDECREF(r);
+        }
     }
     Py_XDECREF(old);
+    return ok;
 }
 PyObject *tensor_set_tag(Tensor *t, PyObject *tag) {
-    set_tag(t, tag);
+    if (!set_tag(t, tag)) return nullptr;
     Py_RETURN_NONE;
 }
 PyMemberDef tensor_members[] = {
@@ -521,7 +531,7 @@ Buffer *ensure(Graph *g, Tensor *t) {      // a reference of the caller's
     if (sent < 0 || (sent == 0 && !add_upload(g, b->id, t))) { Py_DECREF(b); Py_DECREF(b); return nullptr; }
     if (sent) Py_DECREF(b);
     else g->s->allocs.push_back(b);        // (takes the reference)
-    set_tag(t, reinterpret_cast<PyObject *>(b));
+    if (!set_tag(t, reinterpret_cast<PyObject *>(b))) { Py_DECREF(b); return nullptr; }
     track(g, b->id, t);
     return b;
 }
@@ -547,17 +557,18 @@ PyObject *output_tensor(Graph *g, Buffer *b) {
     Py_XSETREF(b->graph, reinterpret_cast<PyObject *>(g));
     return o;
 }
-void bind(Graph *g, Tensor *t, Buffer *b) {
-    set_tag(t, reinterpret_cast<PyObject *>(b));
+bool bind(Graph *g, Tensor *t, Buffer *b) {
+    if (!set_tag(t, reinterpret_cast<PyObject *>(b))) return false;
     track(g, b->id, t);
     Py_INCREF(g);
     Py_XSETREF(b->graph, reinterpret_cast<PyObject *>(g));
+    return true;
 }
 // The result of a recorded operation: a new tensor, or `into` on its new buffer.  Takes the caller's reference to out.
 PyObject *finish(Graph *g, Buffer *out, Tensor *into) {
     PyObject *r;
     if (!into) r = output_tensor(g, out);
-    else { bind(g, into, out); r = Py_None; Py_INCREF(r); }
+    else if ((r = bind(g, into, out) ? Py_None : nullptr)) Py_INCREF(r);
     Py_DECREF(out);
     return r;
 }
@@ -607,7 +618,7 @@ PyObject *graph_bind(Graph *g, PyObject *const *a, Py_ssize_t n) {
     if (!b) return nullptr;
     Tensor *t = tensor(a[0]);
     if (!t) return PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "_bindOther", "OO", a[0], a[1]);
-    bind(g, t, b);
+    if (!bind(g, t, b)) return nullptr;
     Py_RETURN_NONE;
 }
 PyObject *graph_let_go(Graph *g, PyObject *o) {
@@ -1081,7 +1092,11 @@ PyObject *graph_release_all(Graph *g, PyObject *) {
     for (int id : ids) {
         auto it = s->tensors.find(id);
         Tensor *t = it == s->tensors.end() ? nullptr : it->second;
-        if (t) set_tag(t, Py_None);
+        if (!t) continue;
+        Py_INCREF(t);
+        const bool ok = set_tag(t, Py_None);
+        Py_DECREF(t);
+        if (!ok) return nullptr;
     }
     if (!ids.empty() && !release_ids(g, ids)) return nullptr;
     while (!s->tensors.empty()) forget(g, s->tensors.begin()->first);
