@@ -460,25 +460,26 @@ bool add_upload(Graph *g, int id, Tensor *t) {
 
 // The values of a new buffer from 1 MiB on are sent as they are instead of being copied for the flush (three weights of 11 MB:
 // 7.8 ms to their first result with the copies, 1.8 without): nothing recorded refers to the buffer yet, so it does not matter when they arrive.
-// 1: sent, 0: not of that kind, -1: an error.
-int send_now(Graph *g, Buffer *b, Tensor *t) {
+// false: not of that kind, or it could not be sent: the flush sends it, and says why it cannot.
+bool send_now(Graph *g, Buffer *b, Tensor *t) {
     constexpr Py_ssize_t kLarge = 1 << 20;
-    if (!has_data(t) || t->rows * t->cols * 4 < kLarge || !direct(g)) return 0;
+    if (!has_data(t) || t->rows * t->cols * 4 < kLarge || !direct(g)) return false;
     Py_buffer v;
-    if (PyObject_GetBuffer(t->data, &v, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) != 0) { PyErr_Clear(); return 0; }
-    int r = 0;
+    if (PyObject_GetBuffer(t->data, &v, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) != 0) { PyErr_Clear(); return false; }
+    bool sent = false;
     if (v.itemsize == 4 && v.format && strcmp(v.format, "f") == 0 && v.len == t->rows * t->cols * 4) {
         const int32_t id = b->id, size = (int32_t)(t->rows * t->cols);
         const Calls calls;
-        r = calls(g, [&](const Native &n, std::string &text) {
+        sent = calls(g, [&](const Native &n, std::string &text) {
             int rc = noted(n.alloc(&id, &size, 1), n, text);
             if (rc == 0 && (rc = noted(n.upload(id, static_cast<const float *>(v.buf), size), n, text)) != 0) (void)n.release(&id, 1);
             return rc;
-        }) ? 1 : -1;
-        if (r > 0) b->allocated = 1;
+        });
+        if (sent) b->allocated = 1;
+        else PyErr_Clear();
     }
     PyBuffer_Release(&v);
-    return r;
+    return sent;
 }
 
 // What is looked into here: a tensor whose class leaves its sizes, values and buffer as Tensor has them.  One that does not is an
@@ -527,8 +528,8 @@ Buffer *ensure(Graph *g, Tensor *t) {      // a reference of the caller's
     if (!b) return nullptr;
     g->next_id++;
     Py_INCREF(b);                          // (two: the caller's, and the list's of what is to be made)
-    const int sent = send_now(g, b, t);
-    if (sent < 0 || (sent == 0 && !add_upload(g, b->id, t))) { Py_DECREF(b); Py_DECREF(b); return nullptr; }
+    const bool sent = send_now(g, b, t);
+    if (!sent && !add_upload(g, b->id, t)) { Py_DECREF(b); Py_DECREF(b); return nullptr; }
     if (sent) Py_DECREF(b);
     else g->s->allocs.push_back(b);        // (takes the reference)
     if (!set_tag(t, reinterpret_cast<PyObject *>(b))) { Py_DECREF(b); return nullptr; }

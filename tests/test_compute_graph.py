@@ -466,19 +466,23 @@ def test_a_runtime_may_flush_from_inside_a_call(call):
     backend.releaseResources()
 
 
-def test_an_upload_that_fails_leaves_its_id_to_the_next_buffer():
-    """A large tensor's values are sent when it is first used; one that cannot be sent leaves no buffer of its size behind."""
+def test_values_that_cannot_be_sent_are_the_flushs_to_report():
+    """A large tensor's values are sent when it is first used.  One that cannot be sent then is recorded all the same, as a small one
+    is, and leaves no buffer of its size to the next one; the flush says what is wrong, and sends it once that is over."""
     lib = NativeLibrary()
     graph = lib.graph()
     lib.fail_upload = True
+    first = Tensor.from2D(np.ones((512, 512), np.float32))
+    buf = graph.ensureGpuBuffer(first)
+    assert not lib.sizes and not buf.allocatedOnGpu
     with pytest.raises(RuntimeError, match="the library says so"):
-        graph.ensureGpuBuffer(Tensor.from2D(np.ones((512, 512), np.float32)))
-    assert not lib.sizes
+        graph.flush()
     lib.fail_upload = False
-    t = Tensor.from2D(np.full((1024, 512), 2.0, np.float32))
-    buf = graph.ensureGpuBuffer(t)
+    second = Tensor.from2D(np.full((1024, 512), 2.0, np.float32))
+    other = graph.ensureGpuBuffer(second)
+    graph._emit(op.OP_NEG, buf.id, other.id, 512 * 512)
     graph.flush()
-    assert lib.sizes == {buf.id: t.rows * t.cols} and lib.held[buf.id][-1] == 2.0
+    assert lib.sizes == {buf.id: 512 * 512, other.id: 1024 * 512} and lib.held[other.id][-1] == 2.0 and lib.held[buf.id][-1] == 1.0
 
 
 BLOCKING = """
