@@ -151,6 +151,7 @@ struct State {
     int64_t uploads_taken_out = 0;         // how often some of them were
     std::unordered_map<int, Tensor *> tensors;     // null: it has died
     std::vector<int> maybe_orphans;
+    std::vector<int32_t> gone;             // no longer tracked, and still to be released
 };
 struct Graph {
     PyObject_HEAD
@@ -900,9 +901,9 @@ bool release_ids(Graph *g, const std::vector<int32_t> &ids) {
     Py_XDECREF(a);
     return ok;
 }
-bool release_orphans(Graph *g) {
+void collect_orphans(Graph *g) {           // into gone
     State *s = g->s;
-    if (s->maybe_orphans.empty()) return true;
+    if (s->maybe_orphans.empty()) return;
     std::vector<int> candidates;
     candidates.swap(s->maybe_orphans);
     std::vector<int32_t> orphans;
@@ -913,8 +914,8 @@ bool release_orphans(Graph *g) {
             if (!has_other(g, id)) continue;               // unknown, or seen before
             PyObject *held = PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "_otherHolds", "i", id);
             const bool stays = held != Py_False;
+            if (!held) PyErr_WriteUnraisable(reinterpret_cast<PyObject *>(g));
             Py_XDECREF(held);
-            if (!held) { s->maybe_orphans.insert(s->maybe_orphans.end(), candidates.begin(), candidates.end()); return false; }
             if (stays) continue;
         } else if (Tensor *t = it->second) {
             Buffer *b = tag_of(t);
@@ -925,7 +926,7 @@ bool release_orphans(Graph *g) {
         if (other) drop_other(g, id);
         else forget(g, id);
     }
-    if (orphans.empty()) return true;
+    if (orphans.empty()) return;
     if (!s->allocs.empty() || !s->uploads.empty()) {
         auto gone = [&](int id) { return std::find(orphans.begin(), orphans.end(), id) != orphans.end(); };
         std::vector<Buffer *> dropped;
@@ -938,7 +939,16 @@ bool release_orphans(Graph *g) {
         s->uploads_taken_out++;
         for (Buffer *b : dropped) Py_DECREF(b);
     }
-    return release_ids(g, orphans);
+    s->gone.insert(s->gone.end(), orphans.begin(), orphans.end());
+}
+bool release_gone(Graph *g) {
+    std::vector<int32_t> ids;
+    ids.swap(g->s->gone);
+    return ids.empty() || release_ids(g, ids);
+}
+bool release_orphans(Graph *g) {
+    collect_orphans(g);
+    return release_gone(g);
 }
 // Taken out of the graph first, so that what other threads record meanwhile is the next flush's; what was not done goes back in front
 // of it (all uploads, where one of them failed).
@@ -988,16 +998,18 @@ bool flush_native(Graph *g) {
     }
     return ok;
 }
-bool flush(Graph *g) {
+// A download behind it takes along what is to be released: one time less that the interpreter's lock is given up and taken.
+bool flush(Graph *g, bool download_follows = false) {
     if (direct(g)) {
         const Calls calls;
         if ((g->s->ops != 0 || !g->s->allocs.empty()) && !flush_native(g)) return false;
-        return release_orphans(g);
+        collect_orphans(g);
+        return download_follows || release_gone(g);
     }
     if (g->s->ops == 0 && g->s->allocs.empty()) return release_orphans(g);
     return allocate_pending(g) && upload_pending(g) && execute_pending(g) && release_orphans(g);
 }
-bool flush_method(Graph *g) { return plain_graph(reinterpret_cast<PyObject *>(g)) ? flush(g) : call(PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "flush", nullptr)); }
+bool flush_method(Graph *g, bool download_follows = false) { return plain_graph(reinterpret_cast<PyObject *>(g)) ? flush(g, download_follows) : call(PyObject_CallMethod(reinterpret_cast<PyObject *>(g), "flush", nullptr)); }
 PyObject *graph_flush(Graph *g, PyObject *) {
     if (!flush(g)) return nullptr;
     Py_RETURN_NONE;
@@ -1010,7 +1022,12 @@ bool fetch(Graph *g, Buffer *b, PyObject *flat) {          // flat: contiguous f
     Py_buffer v;
     if (PyObject_GetBuffer(flat, &v, PyBUF_CONTIG) != 0) return false;
     const Calls calls;
-    const bool ok = calls(g, [&](const Native &n, std::string &text) { return noted(n.download(b->id, static_cast<float *>(v.buf), v.len / 4), n, text); });
+    std::vector<int32_t> gone;
+    gone.swap(g->s->gone);
+    const bool ok = calls(g, [&](const Native &n, std::string &text) {
+        const int rc = gone.empty() ? 0 : noted(n.release(gone.data(), (int32_t)gone.size()), n, text);
+        return rc ? rc : noted(n.download(b->id, static_cast<float *>(v.buf), v.len / 4), n, text);
+    });
     PyBuffer_Release(&v);
     return ok;
 }
@@ -1057,9 +1074,15 @@ PyObject *graph_materialize(Graph *g, PyObject *o) {
     Buffer *b = tag_of(t);
     if (!b || !b->cpu_stale) Py_RETURN_NONE;
     Py_INCREF(b);
-    const bool ok = flush_method(g) && download(g, b, t);
+    bool ok = flush_method(g, true) && download(g, b, t);
     if (ok) b->cpu_stale = 0;
     Py_DECREF(b);
+    if (!g->s->gone.empty()) {             // (the download was not made)
+        PyObject *type, *value, *trace;
+        PyErr_Fetch(&type, &value, &trace);
+        ok = release_gone(g) && ok;
+        if (type) { PyErr_Clear(); PyErr_Restore(type, value, trace); }
+    }
     if (!ok) return nullptr;
     Py_RETURN_NONE;
 }

@@ -466,6 +466,28 @@ def test_a_runtime_may_flush_from_inside_a_call(call):
     backend.releaseResources()
 
 
+@pytest.mark.parametrize("fails", [False, True])
+def test_a_read_releases_what_the_flush_in_front_of_it_has_orphaned(fails):
+    """Behind the flush and in front of the download; and all the same where the download cannot be made."""
+    lib = NativeLibrary()
+    backend = HipBackend(lib.graph().runtime)
+    a = Tensor.from2D([[1.0, 2.0]])
+    for _ in range(2):
+        dropped = backend.neg(a)
+        kept = backend.exp(dropped)
+        gone = dropped.getGpuTag().id
+        del dropped
+        if fails:
+            kept._data = np.zeros((3, 3), np.float32)
+            with pytest.raises(ValueError, match="Size mismatch"):
+                backend.materializeTensor(kept)
+        else:
+            backend.materializeTensor(kept)
+        names = [c[0] for c in lib.calls]
+        assert names[-3:] == (["upload", "flush", "release"] if fails else ["flush", "release", "download"])
+        assert gone in lib.calls[-1 if fails else -2][1] and gone not in lib.sizes and kept.getGpuTag().id in lib.sizes
+
+
 def test_values_that_cannot_be_sent_are_the_flushs_to_report():
     """A large tensor's values are sent when it is first used.  One that cannot be sent then is recorded all the same, as a small one
     is, and leaves no buffer of its size to the next one; the flush says what is wrong, and sends it once that is over."""
