@@ -50,6 +50,7 @@ SOURCES = {
     "kernels_decode.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kernels_latent.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "kernels_token.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "runner.cpp": [],
     "host_random.cpp": [],
 }

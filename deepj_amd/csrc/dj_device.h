@@ -60,5 +60,52 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+// Digit planes in LDS: plane p holds one byte per k (k padded with zeros to a multiple of 64), `pitch` bytes apart (16 more
+// than they hold: the four planes' reads of one k fall on different banks); unit[g]
+// the power of two of group g (NaN where the group holds an infinity or a NaN).
+// Thread with four values of k = 4 i .. 4 i + 3 (eight consecutive lanes share a group).
+__device__ __forceinline__ void stage_digits4(uint8_t *planes, int pitch, float *unit, int i, float4 v) {
+    uint32_t m = max(max(__float_as_uint(v.x) & 0x7fffffffu, __float_as_uint(v.y) & 0x7fffffffu),
+                     max(__float_as_uint(v.z) & 0x7fffffffu, __float_as_uint(v.w) & 0x7fffffffu));
+    m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xf, 0xf, false));      // quad_perm [1,0,3,2]
+    m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xf, 0xf, false));      // quad_perm [2,3,0,1]
+    m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, false));     // row_half_mirror
+    // m = f 2^e, f in [0.5, 1): values times 2^(29 - e) are at most 2^29.  The shift stays where 2^shift and 2^-shift are
+    // normal numbers.
+    const int e = __builtin_amdgcn_frexp_expf(__uint_as_float(m));
+    const int shift = min(29 - e, 120);
+    const float up = ldexpf(1.0f, shift);
+    // t = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3 with signed bytes: add 128 to each of the three low bytes, then flip their top bits
+    auto digits = [&](float x) { return ((uint32_t)(int)rintf(x * up) + 0x00808080u) ^ 0x00808080u; };
+    const uint32_t w0 = digits(v.x), w1 = digits(v.y), w2 = digits(v.z), w3 = digits(v.w);
+    const uint32_t a = __builtin_amdgcn_perm(w1, w0, 0x05010400u), b = __builtin_amdgcn_perm(w3, w2, 0x05010400u);
+    const uint32_t c = __builtin_amdgcn_perm(w1, w0, 0x07030602u), d = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
+    uint32_t *p = reinterpret_cast<uint32_t *>(planes) + i;
+    p[0] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+    p[pitch / 4] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    p[2 * (pitch / 4)] = __builtin_amdgcn_perm(d, c, 0x05040100u);
+    p[3 * (pitch / 4)] = __builtin_amdgcn_perm(d, c, 0x07060302u);
+    if ((i & 7) == 0) unit[i >> 3] = m >= 0x7f800000u ? __uint_as_float(0x7fc00000u) : ldexpf(1.0f, -shift);
+}
+
+// The value of the lanes `OFF` apart: a of one, b of the other (the same pair for both)
+template <int OFF> __device__ __forceinline__ void lane_pair(float v, float &a, float &b) {
+    if constexpr (OFF == 8) {
+        a = v;
+        b = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false));   // row_ror:8
+    } else {
+        const unsigned u = __builtin_bit_cast(unsigned, v);
+        const auto r = OFF == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false) : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        a = __builtin_bit_cast(float, (unsigned)r[0]);
+        b = __builtin_bit_cast(float, (unsigned)r[1]);
+    }
+}
+__device__ __forceinline__ float quarters_sum(float v) {
+    float a, b;
+    lane_pair<16>(v, a, b);
+    lane_pair<32>(a + b, a, b);
+    return a + b;
+}
+
 }  // namespace dev
 }  // namespace dj

@@ -93,6 +93,11 @@ struct Runner {
     int32_t sampler = -1;                                  // DECODE_SAMPLE's parameters
     // Captured per-token streams by how the token is chosen (Choose), whether the blocks are narrow, and kReplayTokens.
     int32_t graph[3][2][3] = {};
+    // The model's tokens as one launch (deepj_hip_token_plan_*); 0: replayed graphs.  Between such a run and the first sight of
+    // what it left, `pending` says what it was (a step: of which token), should it have to be done again by launches.
+    int32_t plan = 0, token_groups = 0;
+    enum Pending { kSettled, kRun, kStep } pending = kSettled;
+    int32_t pending_token = 0;
     bool finalized = false;
     int32_t pos = 0;          // host mirror of state[0]
     int32_t generated = 0;    // host mirror of state[2]
@@ -326,6 +331,17 @@ void alloc_acts(Runner &r, Acts &a, int rows) {
 
 void warm_up(Runner &r);
 
+// Tokens of a run as one launch (Llama and GPT; DeepSeek's stay launches).
+void make_plan(Runner &r) {
+    const Config &c = r.cfg;
+    if (c.kind == 1 || r.token_groups < 0) return;
+    std::vector<int32_t> w{c.kind, c.vocab, c.max_seq, c.d, c.heads, c.layers, c.dff, r.token_groups, r.emb, r.pos_table, r.gf, r.bf, r.wlm, r.blm,
+                           r.cos_t, r.sin_t, r.kc, r.vc, r.state, r.tokens, r.logits, r.dec.x};
+    for (const Layer &L : r.layers)
+        for (int32_t id : {L.g1, L.be1, L.g2, L.be2, L.wqkv, L.wo, L.wgu, L.bg, L.bu, L.wd, L.bd}) w.push_back(id);
+    hip(deepj_hip_token_plan_create(w.data(), (int32_t)w.size(), &r.plan));
+}
+
 void finalize(Runner &r) {
     const Config &c = r.cfg;
     if (r.finalized) return;
@@ -381,6 +397,7 @@ void finalize(Runner &r) {
     }
     // the prompt-sized buffers for the longest prompt the cache can take, so that no request pays for allocation
     alloc_acts(r, r.pre, c.max_seq);
+    make_plan(r);
     r.finalized = true;
     warm_up(r);
 }
@@ -578,12 +595,50 @@ void upload_state(Runner &r, int32_t token) {
     hip(deepj_hip_upload(r.state, reinterpret_cast<const float *>(st), 4));
 }
 
+int token_launches(const Config &c, bool narrow);
+void decode_steps(Runner &r, int steps, int mode, Choose how, bool narrow);
+
+void drop_plan(Runner &r) {
+    if (r.plan) hip(deepj_hip_token_plan_destroy(r.plan));
+    r.plan = 0;
+    r.pending = Runner::kSettled;
+}
+
+// What a run of the plan left, now that the stream has got there (`arrived`: something behind it has been downloaded).  A run
+// that could not have the whole device (its state is that behind the last whole token) is finished by launches, and so is
+// everything after it.  True: results read before this call have to be read again.
+bool settle(Runner &r, bool arrived = false) {
+    if (r.pending == Runner::kSettled) return false;
+    if (!arrived) hip(deepj_hip_synchronize());
+    const Runner::Pending was = r.pending;
+    r.pending = Runner::kSettled;
+    if (!deepj_hip_token_plan_failed(r.plan)) return false;
+    drop_plan(r);
+    int32_t st[4];
+    hip(deepj_hip_download(r.state, reinterpret_cast<float *>(st), 4));
+    const int at = was == Runner::kStep ? r.pos - 1 : st[0], steps = r.pos - at;
+    if (was == Runner::kStep) {
+        st[0] = at;
+        st[1] = r.pending_token;
+        hip(deepj_hip_upload(r.state, reinterpret_cast<const float *>(st), 4));
+        r.run(decode_stream(r, kNone, false));
+        upload_state(r, r.pending_token);
+        return true;
+    }
+    Stream s;                                                // (the embedding that the launches start from)
+    emit(s, DJ_OP_EMBED_GATHER, r.emb, r.state, r.dec.x, 1, r.cfg.d, r.cfg.vocab, 1);
+    r.run(s);
+    decode_steps(r, steps, 0, kGreedy, false);
+    return true;
+}
+
 // Runs the prompt rows through the model, filling the cache.  Leaves the last row's
 // logits in r.logits; unless `how` is kNone the next token is chosen on the device as well.
 void prefill(Runner &r, const int32_t *ids, int n, float *all_logits, Choose how) {
     const Config &c = r.cfg;
     if (!r.finalized) finalize(r);
     if (n <= 0) throw Error("prefill: empty prompt");
+    settle(r);
     check_ids(c, ids, n);
     if (r.pos + n > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + n) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
@@ -606,6 +661,8 @@ void prefill(Runner &r, const int32_t *ids, int n, float *all_logits, Choose how
 
 void reset(Runner &r) {
     if (!r.finalized) finalize(r);
+    // (what a run left is not asked for any more; one that could not finish shows in the next)
+    r.pending = Runner::kSettled;
     r.pos = 0;
     r.generated = 0;
     upload_state(r, 0);
@@ -626,8 +683,6 @@ void capture(Runner &r, Choose how, bool narrow, int size) {
 // 1.3 ms once) and, for a narrow model, those of the blocks in five launches, which it takes late in a long context or never
 // (1.1 ms once, where loading a 4-layer model of width 256 paid 3.3).  The 16-token graph is captured and not run: its first
 // replay costs what every other does.
-int token_launches(const Config &c, bool narrow);
-void decode_steps(Runner &r, int steps, int mode, Choose how, bool narrow);
 void warm_up(Runner &r) {
     const Config &c = r.cfg;
     const char *env = getenv("DEEPJ_HIP_WARMUP");           // "0": skip (profiling runs that want only the request's launches)
@@ -688,6 +743,22 @@ void decode(Runner &r, int steps, int mode, Choose how) {
     if (steps <= 0) return;
     if (r.pos + steps > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + steps) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
+    settle(r);
+    if (r.plan && mode == 1 && how != kNone) {
+        if (how == kGreedy) hip(deepj_hip_token_plan_run(r.plan, steps, 1));
+        else {
+            Stream s;
+            choose_next(r, s, how, 1);
+            for (int i = 0; i < steps; i++) {
+                hip(deepj_hip_token_plan_run(r.plan, 1, 0));
+                r.run(s);
+            }
+        }
+        r.pending = Runner::kRun;
+        r.pos += steps;
+        r.generated += steps;
+        return;
+    }
     const int narrow = std::min(steps, std::max(0, r.narrow_positions() - r.pos));
     if (narrow) decode_steps(r, narrow, mode, how, true);
     if (steps > narrow) decode_steps(r, steps - narrow, mode, how, false);
@@ -703,7 +774,16 @@ void step_token(Runner &r, int32_t token, int mode) {
     check_ids(c, &token, 1);
     if (r.pos + 1 > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + 1) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
+    settle(r);
     upload_state(r, token);
+    if (r.plan && mode == 1) {
+        hip(deepj_hip_token_plan_run(r.plan, 1, 0));
+        r.pos += 1;
+        upload_state(r, token);
+        r.pending = Runner::kStep;
+        r.pending_token = token;
+        return;
+    }
     // Replayed like a greedy token: the launches of a token one by one cost the host 2.4 us each (43 of them: 190 us a
     // step of 8 layers, 130 as a graph).
     const bool narrow = r.pos < r.narrow_positions();
@@ -770,8 +850,8 @@ int32_t sample_from_logits(const std::vector<float> &logits, float temperature, 
 // 172-175).  While the whole sequence fits the window its rows keep their positions, so the KV cache serves them;
 // once it is longer the window slides by one per token and every row's position changes, so each further token is
 // a fresh forward of the maxSeqLen-row window - what the reference does for every token.
-void generate(Runner &r, const int32_t *prompt, int n_prompt, int max_new, float temperature, int top_k,
-              int64_t seed, int32_t *out, int mode) {
+void generate_once(Runner &r, const int32_t *prompt, int n_prompt, int max_new, float temperature, int top_k,
+                   int64_t seed, int32_t *out, int mode) {
     const Config &c = r.cfg;
     if (max_new < 0) throw Error("maxNewTokens must be >= 0");
     if (!(temperature > 0.0f)) throw Error("temperature must be > 0");
@@ -790,6 +870,7 @@ void generate(Runner &r, const int32_t *prompt, int n_prompt, int max_new, float
         std::vector<float> logits(how == kNone ? (size_t)c.vocab : 0);
         auto sample = [&](int t) {
             hip(deepj_hip_download(r.logits, logits.data(), c.vocab));
+            if (settle(r, true)) hip(deepj_hip_download(r.logits, logits.data(), c.vocab));
             out[n_prompt + t] = sample_from_logits(logits, temperature, top_k, rng);
         };
         reset(r);
@@ -804,6 +885,8 @@ void generate(Runner &r, const int32_t *prompt, int n_prompt, int max_new, float
             prefill(r, prompt, n_prompt, nullptr, how);
             decode(r, cached - 1, mode, how);
             hip(deepj_hip_download(r.tokens, reinterpret_cast<float *>(out + n_prompt), cached));
+            if (r.plan && deepj_hip_token_plan_failed(r.plan)) return;          // (once more, by launches)
+            r.pending = Runner::kSettled;
         } else if (cached > 0) {
             prefill(r, prompt, n_prompt, nullptr, kNone);
             for (int t = 0; t < cached; t++) {
@@ -824,6 +907,14 @@ void generate(Runner &r, const int32_t *prompt, int n_prompt, int max_new, float
         throw;
     }
     if (rng) deepj_host_random_destroy(rng);
+}
+
+void generate(Runner &r, const int32_t *prompt, int n_prompt, int max_new, float temperature, int top_k,
+              int64_t seed, int32_t *out, int mode) {
+    generate_once(r, prompt, n_prompt, max_new, temperature, top_k, seed, out, mode);
+    if (!r.plan || !deepj_hip_token_plan_failed(r.plan)) return;       // (its tokens have been downloaded)
+    drop_plan(r);
+    generate_once(r, prompt, n_prompt, max_new, temperature, top_k, seed, out, mode);
 }
 
 template <class F> int guarded(Runner *r, F &&f) {
@@ -867,6 +958,7 @@ void deepj_runner_destroy(void *h) {
         for (auto &sizes : r->graph[how])
             for (int32_t g : sizes)
                 if (g) deepj_hip_graph_destroy(g);
+    if (r->plan) deepj_hip_token_plan_destroy(r->plan);
     deepj_hip_synchronize();
     // every id in [id_base, next_id) that is still live belongs to this runner
     std::vector<int32_t> ids;
@@ -923,6 +1015,18 @@ int deepj_runner_set_prepared_budget(void *h, int64_t bytes) {
     });
 }
 
+// XCDs that token runs take: 0 the library's choice, -1 none (tokens are replayed graphs).  Before finalize.
+int deepj_runner_set_token_groups(void *h, int32_t groups) {
+    auto *r = static_cast<Runner *>(h);
+    return guarded(r, [&] {
+        if (r->finalized) throw Error("set_token_groups after finalize");
+        if (groups < -1 || groups > 8) throw Error("token groups must be -1 (no token runs), 0 (the library's choice) or 1 to 8");
+        r->token_groups = groups;
+    });
+}
+
+int32_t deepj_runner_token_plan(void *h) { return h ? static_cast<Runner *>(h)->plan : 0; }
+
 int64_t deepj_runner_prepared_bytes(void *h) { return h ? static_cast<Runner *>(h)->prepared_bytes : 0; }
 
 int deepj_runner_finalize(void *h) {
@@ -958,6 +1062,7 @@ int deepj_runner_last_logits(void *h, float *out) {
     auto *r = static_cast<Runner *>(h);
     return guarded(r, [&] {
         hip(deepj_hip_download(r->logits, out, r->cfg.vocab));
+        if (settle(*r, true)) hip(deepj_hip_download(r->logits, out, r->cfg.vocab));
     });
 }
 
@@ -968,6 +1073,7 @@ int deepj_runner_tokens(void *h, int32_t *out, int32_t capacity, int32_t *n) {
         int32_t count = std::min(r->generated, capacity);
         if (count > 0) hip(deepj_hip_download(r->tokens, reinterpret_cast<float *>(out), count));
         else hip(deepj_hip_synchronize());
+        if (settle(*r, true) && count > 0) hip(deepj_hip_download(r->tokens, reinterpret_cast<float *>(out), count));
         if (n) *n = count;
     });
 }
@@ -987,6 +1093,7 @@ int deepj_runner_prefill_stream(void *h, int32_t n, int32_t *out, int32_t capaci
     auto *r = static_cast<Runner *>(h);
     return guarded(r, [&] {
         if (!r->finalized) finalize(*r);
+        settle(*r);
         if (n <= 0 || r->pos + n > r->cfg.max_seq) throw Error("prefill_stream: row count outside the context window");
         Stream s = prompt_stream(*r, n, kNone);
         if (len) *len = (int32_t)s.size();
@@ -999,6 +1106,7 @@ int deepj_runner_decode_stream(void *h, int32_t *out, int32_t capacity, int32_t 
     auto *r = static_cast<Runner *>(h);
     return guarded(r, [&] {
         if (!r->finalized) finalize(*r);
+        settle(*r);
         Stream s = decode_stream(*r, kGreedy, r->pos < r->narrow_positions());
         if (len) *len = (int32_t)s.size();
         if (out && capacity >= (int32_t)s.size()) std::memcpy(out, s.data(), s.size() * sizeof(int32_t));

@@ -29,6 +29,7 @@
 #include <sys/mman.h>
 
 #include "dj_common.h"
+#include "token_run.h"
 #include "gemm_rows.h"
 
 namespace dj {
@@ -61,12 +62,26 @@ struct Graph {
     std::vector<std::pair<int32_t, int32_t>> prepared, self_prepared;
 };
 
+// A model's tokens in one launch (kernels_token.hip).  The plan holds the weights in that kernel's order, the block its
+// workgroups exchange words in, and the buffers it was made over (id, address); a run is refused once one of them is gone.
+struct TokenPlan {
+    TokenRun run{};
+    std::vector<std::pair<int32_t, void *>> refs;
+    struct Block { void *p; size_t bytes; };
+    std::vector<Block> blocks;        // device memory it owns
+    int64_t exchange_words = 0;
+    uint32_t next_tag = 1;            // (the exchange block starts as zeros)
+    int slot = -1;                    // its word of the pinned block: set by a run that could not finish
+};
+constexpr int kPlanSlots = 1024;
+
 constexpr int kRingSegments = 4;
 constexpr size_t kRingSegmentBytes = (size_t)1 << 20;
 constexpr size_t kStageBytes = (size_t)4 << 20;
 constexpr int64_t kMaxFlags = 16384;
 constexpr size_t kStageAt = kRingSegments * kRingSegmentBytes, kFlagsAt = kStageAt + kStageBytes;
-constexpr size_t kPinnedBytes = kFlagsAt + (size_t)kMaxFlags * sizeof(uint32_t);
+constexpr size_t kPlansAt = kFlagsAt + (size_t)kMaxFlags * sizeof(uint32_t);
+constexpr size_t kPinnedBytes = kPlansAt + (size_t)kPlanSlots * sizeof(uint32_t);
 
 // Host memory that kernels and the host read and write while either runs (the ring, the stage, flags, results whose chunks are
 // announced by flags) has to be coherent; the default is so only as long as the environment (HIP_HOST_COHERENT) leaves it.
@@ -97,6 +112,8 @@ struct Runtime {
     bool capturing = false;
     std::unordered_map<int32_t, Graph> graphs;
     int32_t next_graph = 1;
+    std::map<int32_t, TokenPlan> plans;
+    int32_t next_plan = 1;
     unsigned *attn_counters = nullptr;             // kAttnCounterHeads zeroed words: decode attention's split arrivals
     unsigned char *static_scratch = nullptr;       // device address of `scratch` below on g.device
     // Set by a K-sharing fp16 GEMM that also wrote the activations of the op right behind it in that op's layout
@@ -1753,6 +1770,9 @@ int deepj_hip_shutdown(void) {
             if (b) (void)hipFree(b);
         g.row_pieces = nullptr; g.row_pieces_floats = 0;
         g.graphs.clear();
+        for (auto &kv : g.plans)
+            for (const TokenPlan::Block &b : kv.second.blocks) (void)hipFree(b.p);
+        g.plans.clear();
         for (auto &kv : g.live) (void)hipFree(kv.second.ptr);
         g.live.clear();
         for (auto &kv : g.cache)
@@ -2110,6 +2130,192 @@ int deepj_hip_graph_destroy(int32_t handle) {
         float *pieces = it->second.row_pieces;
         g.graphs.erase(it);
         if (pieces && pieces != g.row_pieces && !graph_holds_pieces(pieces)) DJ_HIP(hipFree(pieces));
+    });
+}
+
+// ── runs of tokens ──────────────────────────────────────────────────────────
+static void plan_release(TokenPlan &p) {
+    for (const TokenPlan::Block &b : p.blocks) { g.live_bytes -= (int64_t)b.bytes; pool_free(b.p, b.bytes); }
+    p.blocks.clear();
+}
+
+int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
+    return guarded([&] {
+        ensure_init();
+        if (!handle) fail("token_plan_create: null handle");
+        *handle = 0;
+        if (!w || n < DEEPJ_HIP_TOKEN_PLAN_WORDS) fail("token_plan_create: truncated description");
+        const int layers = w[5];
+        if (layers < 1 || (int64_t)n != DEEPJ_HIP_TOKEN_PLAN_WORDS + (int64_t)layers * DEEPJ_HIP_TOKEN_PLAN_LAYER_WORDS)
+            fail("token_plan_create: the description does not hold its layers");
+        if (w[0] != 0 && w[0] != 2) fail("token_plan_create: kind must be 0 (Llama) or 2 (GPT)");
+        for (int i : {1, 2, 3, 4, 6})
+            if (w[i] <= 0) fail("token_plan_create: sizes must be positive");
+        if (w[3] % w[4] != 0) fail("token_plan_create: d must be a multiple of the heads");
+        if (w[7] < 0) fail("token_plan_create: bad group count");
+        const bool gpt = w[0] == 2;
+        TokenShape s{w[3], w[4], w[3] / w[4], layers, w[6], w[1], w[2], w[7], gpt ? 1 : 0};
+        if (s.groups == 0) s.groups = token_run_groups(s);
+        if (!token_run_ok(s) || (int)g.plans.size() >= kPlanSlots || !token_run_resident(s)) return;      // handle 0: not a model for it
+        TokenPlan p;
+        const int op = DJ_OP_Q8_LINEAR;
+        g.track = &p.refs;
+        std::vector<TokenLayer> table((size_t)layers);
+        struct Weight { const int8_t *q = nullptr; const float *s = nullptr; int k = 0; };
+        std::vector<Weight> weights;
+        Weight head;
+        try {
+            TokenRun &r = p.run;
+            const int64_t d = s.d, half = s.hd / 2;
+            r.shape = s;
+            r.emb = buf(w[8], (int64_t)s.vocab * d, op, "emb");
+            r.pos = gpt ? buf(w[9], (int64_t)s.max_seq * d, op, "pos") : nullptr;
+            r.gf = buf(w[10], d, op, "gf");
+            r.bf = gpt ? buf(w[11], d, op, "bf") : nullptr;
+            q8_weight(w[12], d, s.vocab, op, "wlm", head.q, head.s);
+            head.k = s.d;
+            r.blm = buf(w[13], s.vocab, op, "blm");
+            r.cos_t = buf(w[14], s.max_seq * half, op, "cos");
+            r.sin_t = buf(w[15], s.max_seq * half, op, "sin");
+            r.kc = buf(w[16], (int64_t)layers * s.max_seq * d, op, "kCache");
+            r.vc = buf(w[17], (int64_t)layers * s.max_seq * d, op, "vCache");
+            r.state = reinterpret_cast<int32_t *>(buf(w[18], 4, op, "state"));
+            r.tokens = reinterpret_cast<int32_t *>(buf(w[19], s.max_seq, op, "tokens"));
+            r.logits = buf(w[20], s.vocab, op, "logits");
+            r.x = buf(w[21], d, op, "x");
+            r.scale = (float)(1.0 / std::sqrt((double)s.hd));
+            r.polls = kTokenPolls;
+            for (int l = 0; l < layers; l++) {
+                const int32_t *v = w + DEEPJ_HIP_TOKEN_PLAN_WORDS + l * DEEPJ_HIP_TOKEN_PLAN_LAYER_WORDS;
+                TokenLayer &L = table[(size_t)l];
+                L = TokenLayer{};
+                L.g1 = buf(v[0], d, op, "g1");
+                if (gpt) L.be1 = buf(v[1], d, op, "be1");
+                L.g2 = buf(v[2], d, op, "g2");
+                if (gpt) L.be2 = buf(v[3], d, op, "be2");
+                Weight qkv, wo, up, down;
+                q8_weight(v[4], d, 3 * d, op, "wqkv", qkv.q, qkv.s);
+                q8_weight(v[5], d, d, op, "wo", wo.q, wo.s);
+                q8_weight(v[6], d, (gpt ? 1 : 2) * (int64_t)s.dff, op, "wgu", up.q, up.s);
+                q8_weight(v[9], s.dff, d, op, "wd", down.q, down.s);
+                qkv.k = wo.k = up.k = s.d;
+                down.k = s.dff;
+                L.bg = buf(v[7], s.dff, op, "bg");
+                if (!gpt) L.bu = buf(v[8], s.dff, op, "bu");
+                L.bd = buf(v[10], d, op, "bd");
+                for (const Weight &x : {qkv, wo, up, down}) weights.push_back(x);
+            }
+        } catch (...) {
+            g.track = nullptr;
+            throw;
+        }
+        g.track = nullptr;
+        std::sort(p.refs.begin(), p.refs.end());
+        p.refs.erase(std::unique(p.refs.begin(), p.refs.end()), p.refs.end());
+        try {
+            std::vector<uint32_t> offsets((size_t)s.groups * kTokenMembers * kTokenWaves);
+            const int64_t items = token_run_items(s, offsets.data());
+            auto take = [&](int64_t bytes) {
+                const size_t cls = size_class((size_t)bytes);
+                void *m = pool_alloc(cls);
+                p.blocks.push_back({m, cls});
+                g.live_bytes += (int64_t)cls;
+                return m;
+            };
+            p.exchange_words = token_exchange(s).total;
+            auto *packed = (unsigned char *)take(items * kTokenItemBytes);
+            auto *at = (uint32_t *)take((int64_t)offsets.size() * 4);
+            auto *dev_table = (TokenLayer *)take((int64_t)table.size() * (int64_t)sizeof(TokenLayer));
+            p.run.exchange = (unsigned long long *)take(p.exchange_words * 8);
+            p.run.items = packed;
+            p.run.offsets = at;
+            p.run.layers = dev_table;
+            launch_uploads();
+            stage_upload((float *)at, (const float *)offsets.data(), (int64_t)offsets.size());
+            stage_upload((float *)dev_table, (const float *)table.data(), (int64_t)(table.size() * sizeof(TokenLayer) / 4));
+            launch_uploads();
+            launch_fill(g.stream, (uint32_t *)p.run.exchange, 0, p.exchange_words * 2);
+            for (int l = 0; l < layers; l++)
+                for (int phase = kTokenQkv; phase <= kTokenDown; phase++) {
+                    const Weight &x = weights[(size_t)l * 4 + phase];
+                    launch_token_pack(g.stream, s, phase, l, x.q, x.s, x.k, packed, at);
+                }
+            launch_token_pack(g.stream, s, kTokenHead, 0, head.q, head.s, head.k, packed, at);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) fail(std::string("kernel launch failed: ") + hipGetErrorString(e));
+        } catch (...) {
+            plan_release(p);
+            throw;
+        }
+        std::vector<bool> used(kPlanSlots, false);
+        for (const auto &kv : g.plans) used[(size_t)kv.second.slot] = true;
+        p.slot = (int)(std::find(used.begin(), used.end(), false) - used.begin());
+        p.run.failed = (uint32_t *)(g.pinned + kPlansAt) + p.slot;
+        *p.run.failed = 0;
+        *handle = g.next_plan++;
+        g.plans.emplace(*handle, std::move(p));
+    });
+}
+
+int deepj_hip_token_plan_run(int32_t handle, int32_t steps, int32_t choose) {
+    return guarded([&] {
+        auto it = g.plans.find(handle);
+        if (it == g.plans.end()) fail("token_plan_run: unknown plan " + std::to_string(handle));
+        TokenPlan &p = it->second;
+        if (choose != kTokenLogits && choose != kTokenGreedy) fail("token_plan_run: choose must be 0 (logits only) or 1 (greedy)");
+        if (steps < 1 || (choose == kTokenLogits && steps != 1)) fail("token_plan_run: bad step count " + std::to_string(steps));
+        for (const auto &ref : p.refs) {
+            auto b = g.live.find(ref.first);
+            if (b == g.live.end() || b->second.ptr != ref.second)
+                fail("token_plan_run: buffer id=" + std::to_string(ref.first) + " was released or reallocated after plan " + std::to_string(handle) + " was made");
+        }
+        launch_uploads();
+        // (launches of a moderate length: a run of thousands of tokens does not hold the device in one piece)
+        constexpr int kMost = 256;
+        for (int done = 0; done < steps; done += kMost) {
+            const int n = std::min(kMost, steps - done);
+            const uint64_t need = 1 + (uint64_t)n * token_tags(p.run.shape);
+            if (p.next_tag + need > 0xffffffffull) {             // tags start over: nothing of them may be left
+                launch_fill(g.stream, (uint32_t *)p.run.exchange, 0, p.exchange_words * 2);
+                p.next_tag = 1;
+            }
+            TokenRun r = p.run;
+            r.tag = p.next_tag;
+            r.steps = n;
+            r.choose = choose;
+            launch_token_run(g.stream, r);
+            p.next_tag += (uint32_t)need;
+        }
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) fail(std::string("kernel launch failed: ") + hipGetErrorString(e));
+    });
+}
+
+int32_t deepj_hip_token_plan_failed(int32_t handle) {
+    auto it = g.plans.find(handle);
+    return it == g.plans.end() ? 0 : (int32_t)*(volatile uint32_t *)it->second.run.failed;
+}
+
+int32_t deepj_hip_token_plan_groups(int32_t handle) {
+    auto it = g.plans.find(handle);
+    return it == g.plans.end() ? 0 : it->second.run.shape.groups;
+}
+
+int deepj_hip_token_plan_set_polls(int32_t handle, int32_t polls) {
+    return guarded([&] {
+        auto it = g.plans.find(handle);
+        if (it == g.plans.end()) fail("token_plan_set_polls: unknown plan " + std::to_string(handle));
+        if (polls < 0 || polls > kTokenPolls) fail("token_plan_set_polls: 0 to " + std::to_string(kTokenPolls));
+        it->second.run.polls = polls;
+    });
+}
+
+int deepj_hip_token_plan_destroy(int32_t handle) {
+    return guarded([&] {
+        auto it = g.plans.find(handle);
+        if (it == g.plans.end()) return;
+        plan_release(it->second);                                // (blocks are reused behind the stream's work)
+        g.plans.erase(it);
     });
 }
 

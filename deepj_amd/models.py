@@ -38,6 +38,8 @@ def _lib():
         lib.deepj_runner_set_prepared_budget.argtypes = [C.c_void_p, C.c_int64]
         lib.deepj_runner_prepared_bytes.argtypes = [C.c_void_p]
         lib.deepj_runner_prepared_bytes.restype = C.c_int64
+        lib.deepj_runner_set_token_groups.argtypes = [C.c_void_p, C.c_int32]
+        lib.deepj_runner_token_plan.argtypes = [C.c_void_p]
         lib.deepj_runner_reset.argtypes = [C.c_void_p]
         lib.deepj_runner_prefill.argtypes = [C.c_void_p, _i32p, C.c_int32, C.c_void_p, C.c_int32]
         lib.deepj_runner_decode.argtypes = [C.c_void_p, C.c_int32, C.c_int32]
@@ -216,6 +218,11 @@ class _DecoderOnlyModel:
     def preparedBytes(self) -> int:
         return int(_lib().deepj_runner_prepared_bytes(self._h))
 
+    def setTokenGroups(self, groups: int) -> None:
+        """XCDs that runs of tokens take as one launch: 0 = the library's choice (default), 1 to 8, -1 = none: every token is a
+        replayed graph of launches.  Before finalize()."""
+        self._check(_lib().deepj_runner_set_token_groups(self._h, int(groups)))
+
     # inference ----------------------------------------------------------------
     def reset(self) -> None:
         self._check(_lib().deepj_runner_reset(self._h))
@@ -234,7 +241,7 @@ class _DecoderOnlyModel:
                                                 1 if choose_next else 0))
 
     def _mode(self, use_graph) -> int:
-        """0 eager per-token stream, 1 the stream as a replayed HIP graph (default)."""
+        """0 eager per-token stream, 1 tokens as one launch, or the stream as a replayed HIP graph (default)."""
         return 0 if use_graph is False else 1
 
     def decode(self, steps: int, use_graph: bool | None = None) -> None:

@@ -310,6 +310,31 @@ int32_t deepj_hip_q8_gemm_rows_tile_behind(int32_t m, int32_t k, int32_t rows, i
  * one of these kernels'.  Every launch runs the same check. */
 int32_t deepj_hip_q8_gemm_f16_extents(int32_t m, int32_t k, int32_t rows, int32_t tile_rows, int32_t tile_cols, int64_t *reach3, int64_t *size3);
 
+/* ── runs of tokens ───────────────────────────────────────────────────────
+ * All of a decoder model's token - blocks, head, the greedy choice of the next one - as one launch of many tokens: the
+ * workgroups stay on the device and hand the row to one another.  A plan is made over the buffers of a model as the ops above
+ * lay them out, and holds the weights once more in its kernel's order (1.125 bytes a weight; as they are when it is made).
+ *   create: words = {kind (0 Llama: RMSNorm, RoPE tables, SwiGLU; 2 GPT: LayerNorm, learned positions, GELU), vocab, maxSeq, d,
+ *     heads, layers, dff, groups (0: the library's choice, else 1 to 8 XCDs), emb, pos (GPT), gf, bf (GPT), wlm, blm, cosT, sinT,
+ *     kCache, vCache [layers][heads][maxSeq][hd], state, tokens, logits, x}, then per layer {g1, be1 (GPT), g2, be2 (GPT), wqkv [3 d]
+ *     rows, wo, wgu (Llama: rows 2 n gate, 2 n + 1 up), bg, bu (Llama), wd, bd}.  *plan = 0, without an error, where the
+ *     shape or the device is not one for it: DECODE_ATTN ... DECODE_NEXT are the way.
+ *   run: `steps` tokens from state {position, token, generated}.  choose 1: each like the ops of a token with DECODE_NEXT behind
+ *     them (logits hold the last one's, x its successor's embedding); choose 0: one token up to its logits, state as it was.
+ *     Enqueues only.  Buffers that were released or made again since are refused.
+ *   failed: 1 once a run could not have all of its workgroups on the device at the same time within about a second (another
+ *     process's run of this kind may hold a part of it): state is then that behind the last whole token.  Valid after a
+ *     synchronisation or a download behind the run. */
+#define DEEPJ_HIP_TOKEN_PLAN_WORDS 22
+#define DEEPJ_HIP_TOKEN_PLAN_LAYER_WORDS 11
+int deepj_hip_token_plan_create(const int32_t *words, int32_t n, int32_t *plan);
+int deepj_hip_token_plan_run(int32_t plan, int32_t steps, int32_t choose);
+int32_t deepj_hip_token_plan_failed(int32_t plan);
+int32_t deepj_hip_token_plan_groups(int32_t plan);       /* its groups (XCDs); 0: no such plan */
+/* Loads after which a workgroup gives a word up that it waits for (2^21, the most, to begin with; 0: at once) */
+int deepj_hip_token_plan_set_polls(int32_t plan, int32_t polls);
+int deepj_hip_token_plan_destroy(int32_t plan);
+
 /* ── host side: java.util.Random twin ─────────────────────────────────────
  * Tensor.random(rows, cols, Random) of the reference (J/tensor/cpu/CpuBackend.java:148-152)
  * reproduced bit for bit (JDK-specified LCG + polar nextGaussian with StrictMath.log),
@@ -349,6 +374,10 @@ int deepj_runner_init_seeded_gpt(void *runner, int64_t seed, float init_scale, i
  * Prompts of 256 rows and more give the same bits whatever the budget; shorter ones take the fp16 GEMM only where a
  * copy exists (others otherwise: same tolerance, other last bits).  deepj_runner_prepared_bytes: what the copies take now. */
 int deepj_runner_set_prepared_budget(void *runner, int64_t bytes);
+/* XCDs that this model's runs of tokens take as one launch (deepj_hip_token_plan_*): 0 the library's choice (the default), 1 to 8;
+ * -1: none, every token is a replayed graph.  Before finalize.  deepj_runner_token_plan: the plan, 0 if there is none. */
+int deepj_runner_set_token_groups(void *runner, int32_t groups);
+int32_t deepj_runner_token_plan(void *runner);
 int64_t deepj_runner_prepared_bytes(void *runner);
 int deepj_runner_finalize(void *runner);
 int deepj_runner_reset(void *runner);

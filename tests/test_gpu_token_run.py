@@ -1,0 +1,176 @@
+"""Runs of tokens as one launch (deepj_hip_token_plan_*) against the launches of a token and the prompt's rows: every way the
+work is dealt to groups and workgroups, at the edges of its tiles, slices, key splits and item slots."""
+import numpy as np
+import pytest
+
+from deepj_amd import GPTConfig, GPTModel, LlamaConfig, LlamaModel, TextGenerator, parameter_names, parameter_shapes
+from deepj_amd._native import library
+from oracle import cpu_ref as ref
+
+pytestmark = pytest.mark.gpu
+
+
+def model(gpt, vocab, max_seq, d, heads, layers, dff, groups, seed=7):
+    cfg = (GPTConfig if gpt else LlamaConfig)(vocab, max_seq, d, heads, layers, dff)
+    m = (GPTModel if gpt else LlamaModel)(cfg, None)
+    m.setTokenGroups(groups)
+    rng = np.random.default_rng(seed)
+    for name, (r, c) in zip(parameter_names(cfg), parameter_shapes(cfg)):
+        a = rng.standard_normal((r, c), dtype=np.float32) * np.float32(d ** -0.5)
+        m.setWeight(name, 1.0 + a if name.split(".")[-1] in ("g1", "g2", "gf") else a)
+    m.finalize()
+    return m
+
+
+def plan_of(m):
+    return library().deepj_runner_token_plan(m._h)
+
+
+# (gpt, vocab, d, heads, dff, groups, prompt): one to eight groups with even and uneven heads and hidden units; widths that leave
+# workgroups without a tile (64, 96), a last tile of one word, hidden widths no multiple of 64, 8 or 4; all head widths; one key to
+# several rounds of key tiles; wavefronts with more items than slots (2048 over 8192 on four groups, 4096); rows of two sets
+SHAPES = [(False, 251, 64, 2, 50, 1, 3), (False, 97, 96, 3, 130, 2, 60), (True, 253, 64, 2, 173, 2, 5), (False, 4097, 256, 8, 697, 1, 30),
+          (False, 300, 256, 8, 697, 8, 30), (True, 1003, 320, 10, 1000, 4, 70), (True, 300, 384, 6, 1537, 4, 200), (False, 64, 128, 4, 260, 4, 1),
+          (False, 500, 640, 5, 1000, 4, 900), (True, 1000, 768, 12, 3072, 8, 130), (False, 300, 512, 16, 1376, 1, 1500),
+          (False, 8193, 1024, 16, 2752, 8, 1100), (False, 300, 2048, 16, 8192, 4, 40), (False, 2000, 2112, 33, 5000, 8, 40),
+          (False, 500, 4096, 32, 11008, 8, 20)]
+
+
+@pytest.mark.parametrize("gpt,vocab,d,heads,dff,groups,prompt", SHAPES)
+def test_tokens_of_a_run_equal_those_of_launches(gpt, vocab, d, heads, dff, groups, prompt):
+    """Stepped logits against the prompt's rows (the tolerance of the other such tests, of logits of order 1 to 5), a greedy run
+    against the launches' and the prompt's largest logit, a sampled one, and one that takes turns with launches."""
+    new = 12
+    m = model(gpt, vocab, prompt + 40, d, heads, 2, dff, groups)
+    try:
+        assert plan_of(m) and library().deepj_hip_token_plan_groups(plan_of(m)) == groups
+        ids = ref.JavaRandom(5).ints(prompt + new, vocab)
+        full = m.forward(ids)
+        scale = max(1.0, float(np.abs(full).max()) / 5)
+        m.reset()
+        m.prefill(ids[:prompt], choose_next=False)
+        for t in range(prompt, prompt + new):
+            m.step(int(ids[t]))
+            assert float(np.max(np.abs(m.lastLogits() - full[t]))) <= 2e-4 * scale, t
+        greedy = TextGenerator.generate(m, ids[:prompt], 30, top_k=1)
+        logits = m.forward(greedy)
+        for t in range(prompt, len(greedy)):
+            assert logits[t - 1].max() - logits[t - 1, greedy[t]] <= 4e-4 * scale, t
+        assert np.array_equal(greedy, TextGenerator.generate(m, ids[:prompt], 30, top_k=1))
+        assert np.array_equal(greedy, TextGenerator.generate(m, ids[:prompt], 30, top_k=1, use_graph=False))
+        sampled = [TextGenerator.generate(m, ids[:prompt], 20, 0.9, 5, 3, use_graph=g) for g in (True, False)]
+        assert np.array_equal(*sampled)
+        m.reset()
+        m.prefill(ids[:prompt])
+        for n, graph in ((5, True), (3, False), (1, True), (7, True), (2, False), (11, True)):
+            m.decode(n, use_graph=graph)
+        assert np.array_equal(m.tokens(), greedy[prompt:])
+        assert not library().deepj_hip_token_plan_failed(plan_of(m))
+    finally:
+        m.close()
+
+
+def test_ties_and_no_numbers_are_chosen_as_by_the_launches():
+    """Equal logits: the lowest index, across tiles and workgroups; a NaN logit above everything; the two zeros are equal."""
+    m = model(False, 1500, 40, 256, 8, 1, 300, 1)
+    try:
+        ids = ref.JavaRandom(1).ints(6, 1500)
+        for blm in (np.zeros(1500), np.where(np.arange(1500) % 700 == 699, 3.0, 0.0), np.where(np.arange(1500) == 1234, np.nan, 0.0)):
+            tied = LlamaModel(m.cfg, None)
+            tied.setTokenGroups(1)
+            for name, (r, c) in zip(parameter_names(m.cfg), parameter_shapes(m.cfg)):
+                w = np.zeros((r, c), np.float32) if name == "wlm" else np.full((r, c), 0.01, np.float32)
+                tied.setWeight(name, blm.astype(np.float32).reshape(1, -1) if name == "blm" else w)
+            tied.finalize()
+            assert plan_of(tied)
+            a = TextGenerator.generate(tied, ids, 8, top_k=1)
+            b = TextGenerator.generate(tied, ids, 8, top_k=1, use_graph=False)
+            assert np.array_equal(a, b)
+            assert np.all(a[6:] == (1234 if np.isnan(blm).any() else int(np.argmax(blm))))
+            tied.close()
+    finally:
+        m.close()
+
+
+@pytest.mark.parametrize("groups", [1, 8])
+def test_a_run_that_cannot_finish_is_done_by_launches(groups):
+    """A wait that is given up at once: the run leaves without a token, and tokens, logits, prompts and samples behind it are those
+    of the launches."""
+    lib = library()
+    ids = ref.JavaRandom(9).ints(40, 300)
+    good = model(False, 300, 80, 256, 8, 2, 300, -1)
+    assert plan_of(good) == 0
+
+    def fresh():
+        m = model(False, 300, 80, 256, 8, 2, 300, groups)
+        lib.deepj_hip_token_plan_set_polls(plan_of(m), 0)
+        return m
+    try:
+        full = good.forward(ids)
+        m = fresh()
+        assert np.array_equal(TextGenerator.generate(m, ids[:20], 20, top_k=1), TextGenerator.generate(good, ids[:20], 20, top_k=1))
+        assert plan_of(m) == 0                                       # (dropped)
+        m.close()
+        m = fresh()
+        assert np.array_equal(TextGenerator.generate(m, ids[:20], 20, 0.8, 6, 4), TextGenerator.generate(good, ids[:20], 20, 0.8, 6, 4))
+        m.close()
+        m = fresh()
+        assert np.array_equal(TextGenerator.generate(m, ids[:20], 6, 0.8, 0, 4), TextGenerator.generate(good, ids[:20], 6, 0.8, 0, 4))
+        m.close()
+        m = fresh()
+        m.reset()
+        m.prefill(ids[:20], choose_next=False)
+        for t in range(20, 24):
+            m.step(int(ids[t]))
+            assert float(np.max(np.abs(m.lastLogits() - full[t]))) <= 2e-4, t
+        m.close()
+        m = fresh()                                                  # a step and a run whose results nobody reads before the next
+        for x in (m, good):
+            x.reset()
+            x.prefill(ids[:20], choose_next=False)
+            x.step(int(ids[20]))
+            x.prefill(ids[21:30])
+        lib.deepj_hip_token_plan_set_polls(plan_of(m), 0) if plan_of(m) else None
+        for x in (m, good):
+            x.decode(9)
+            x.decode(4)
+            x.prefill(ids[30:36])
+            x.decode(3)
+        assert np.array_equal(m.tokens(), good.tokens())
+        assert float(np.max(np.abs(m.lastLogits() - good.lastLogits()))) <= 2e-4
+        m.close()
+    finally:
+        good.close()
+
+
+def test_plans_are_refused_with_a_reason_or_not_made():
+    lib = library()
+    m = model(False, 300, 40, 256, 8, 1, 300, 1)
+    try:
+        plan = plan_of(m)
+        assert lib.deepj_hip_token_plan_run(plan, 0, 1) != 0 and b"step count" in lib.deepj_hip_last_error()
+        assert lib.deepj_hip_token_plan_run(plan, 2, 0) != 0
+        assert lib.deepj_hip_token_plan_run(plan, 1, 2) != 0 and b"choose" in lib.deepj_hip_last_error()
+        assert lib.deepj_hip_token_plan_run(plan + 1000, 1, 1) != 0 and b"unknown plan" in lib.deepj_hip_last_error()
+        assert lib.deepj_hip_token_plan_set_polls(plan, -1) != 0
+    finally:
+        m.close()
+    assert lib.deepj_hip_token_plan_run(plan, 1, 1) != 0             # gone with its model
+    for args in ((300, 40, 256, 2, 1, 300, 8),):                     # two heads for eight groups: launches, not an error
+        m = model(False, *args)
+        try:
+            assert plan_of(m) == 0
+            ids = ref.JavaRandom(2).ints(9, 300)
+            assert np.array_equal(TextGenerator.generate(m, ids, 9, top_k=1), TextGenerator.generate(m, ids, 9, top_k=1, use_graph=False))
+        finally:
+            m.close()
+    m = LlamaModel(LlamaConfig(64, 16, 64, 2, 1, 96), 1)
+    try:
+        with pytest.raises(RuntimeError, match="after finalize"):
+            m.setTokenGroups(1)
+    finally:
+        m.close()
+    m = LlamaModel(LlamaConfig(64, 16, 64, 2, 1, 96), None)
+    with pytest.raises(ValueError, match="token groups must be"):
+        m.setTokenGroups(9)
+    m.close()
