@@ -18,25 +18,30 @@
 // member a tile, the members say so with a word each (`beat`).  Waits are bounded (kTokenPolls loads, about a second): if the
 // device did not hold all workgroups at once, each leaves, the state stays behind the last whole token, and *failed tells the host.
 //
-// A workgroup is eight wavefronts that speak - make, send and fetch rows, attend - and eight that multiply, for two reasons: a
-// compute unit's loads return in order and a wavefront's wait for one is a wait for all before it, so weights on their way would
-// hold up the words that everybody waits for; and 128 registers each are then enough.  The two meet at barriers, the same ones in
-// the same order on both sides (named in the code).
+// A workgroup is eight wavefronts that speak - make, send and fetch rows, attend - and eight that multiply.  The two meet at
+// barriers, the same ones in the same order on both sides (named in the code).
 // Weights come in the order in which a wavefront takes them (k_token_pack lays them out once): items of 16 outputs x 64 k, 1 KB in
-// the lanes' order and 32 scales.  A phase's first items are asked for while the phase before it multiplies.
+// the lanes' order and 32 scales.  They go straight to LDS, kRing of them a wavefront, asked for ahead of the phase that is on and by a
+// count of their own: the compiler, which sees branches between registers' loads and their uses, waits for all of them at each (16
+// blocks of d 2048: 410 us a token with items loaded to registers, where launches take 404).  A phase's first twelve move on to
+// registers before its row is there.
 // Products run on v_mfma_i32_16x16x64_i8 as in kernels_decode.hip: the activations of 32 k in four signed-byte digits of one
 // power of two, the two scale groups of the 64 k in rows of their own.
+// The speakers' way has no load that waits for another (norm weights and biases stand at computed places, no table of pointers) and
+// nothing kept in memory between phases: each such wait is one for the weights in front of it (GPT 177 us a token, 155 without).
 //
-// Bound by the serial chain: instructions on the way from a row's arrival to the next one's departure (a phase of one item a
-// wavefront takes 1500 to 2000 clocks, of which the exchange is 1000), and by memory where a block has more than some 20 MB.  Us a
-// token, launches and this: 4 blocks of d 256, 4096 words 50.9, 36.9; d 1024, 8192 words 67.2, 51.6; d 2048, 32000 words 117, 107;
-// GPT, 4 blocks of 768, 50257 words 79.3, 58.6.
+// Bound by the serial chain: instructions on the way from a row's arrival to the next one's departure, one every four clocks of a
+// wavefront at best (a phase of one item a wavefront takes 1200 clocks, an exchange 1000 inside a group and 5000 between groups), and by
+// memory where a block has more than some 20 MB.  Us a token, launches and this: 4 blocks of d 256, 256 words 48.0, 37.3; 8 of d 1024,
+// 8192 words 126, 98; d 2048, 32000 words, 4 blocks 120, 102, 16 blocks 404, 343; GPT, 12 blocks of 768, 50257 words 200, 152.
 // Taken back: one set of wavefronts for everything (256 registers: 51.6 us where this takes 36.5); the heads' records merged
-// through LDS; next phase's weights asked for behind the products (every wait for a row then waits for them too).
+// through LDS; all slots filled behind every phase (372 us at 16 blocks of d 2048); items asked for by the clock while the
+// multiplying wavefronts wait (122 us at 4 blocks, where the same by counts took 114).
 #include <type_traits>
 
 #include "dj_common.h"
 #include "dj_device.h"
+#include "gemm_rows.h"
 #include "token_run.h"
 
 namespace dj {
@@ -44,13 +49,15 @@ namespace {
 using namespace dev;
 
 typedef int intx4 __attribute__((ext_vector_type(4)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef unsigned long long word;
 
 constexpr int kWaves = kTokenWaves, kMembers = kTokenMembers;
 constexpr int kSpeakers = 64 * kWaves;           // threads that make, send and receive rows; as many multiply
 constexpr int kThreads = 2 * kSpeakers;
-constexpr int kEven = 12, kOdd = 6;              // items a wavefront holds of a phase: q | k | v and up (and the head), Wo and down
+constexpr int kRing = 12;                        // items of a wavefront in LDS or on their way there (108 KB in all)
+constexpr int kTogether = 3;                     // items whose products are made side by side
 constexpr int kCrossSleep = 16;                  // of 64 clocks
 constexpr int kRed = 12;                         // floats between two outputs' sums (the wavefronts' eight; 16-byte steps over all banks)
 constexpr float kLog2e = 1.44269504088896340736f;
@@ -89,14 +96,15 @@ __device__ __forceinline__ void fetch(Words<8> &w, const word *b, const uint32_t
 template <int N> __device__ __forceinline__ bool receive(Words<N> &w, const word *base, uint32_t (&p)[N], uint32_t tag, int polls) {
 #pragma unroll
     for (int i = 0; i < N; i++) p[i] *= 8;
-    for (int n = 0; n < polls; n++) {
+    for (int n = polls;;) {                                              // (once at least: w is written on every way out)
         fetch(w, base, p);
         uint32_t off = 0;
 #pragma unroll
         for (int i = 0; i < N; i++) off |= (w.v[i].y ^ tag) | (w.v[i].w ^ tag);
+        if (n <= 0) return false;
         if (off == 0) return true;
+        n--;
     }
-    return false;
 }
 __device__ __forceinline__ float first(uintx4 v) { return __uint_as_float(v.x); }
 __device__ __forceinline__ float second(uintx4 v) { return __uint_as_float(v.z); }
@@ -146,13 +154,12 @@ __device__ unsigned long long g_token_trace[256 * 64];
 #define DJ_STAMP2(i) do {} while (0)
 #endif
 
-template <int N> struct Hold { static constexpr int slots = N; intx4 w[N]; float s[N]; };
-
 // kSets: of four values of the row a speaking thread (1: rows of up to 2048)
 template <int HD, bool GPT, int kSets>
 __global__ void __launch_bounds__(kThreads)
 k_token_run(TokenRun r) {
     constexpr uint32_t kZeros = 4 * (kSets * 4 * kSpeakers + 64 + 16);   // (16 bytes of them behind the digit planes)
+    constexpr bool kKeysAhead = kSets == 1 && !GPT;                              // a block's first keys and values asked for beside the down projection before it
     constexpr int LPK = HD / 4, KPW = 64 / LPK, TILE = kWaves * KPW, U = 4;
     __shared__ __align__(16) uint8_t planes[kZeros + 16];
     __shared__ __align__(16) float unit[kTokenMostD / 32 + 2];
@@ -163,6 +170,8 @@ k_token_run(TokenRun r) {
     __shared__ uint64_t most[kWaves];
     __shared__ int s_fail, s_far;
     __shared__ int4 s_part[kTokenHead + 1], s_item[(kTokenHead + 1) * kWaves];
+
+    extern __shared__ __align__(16) unsigned char ring[];               // the multiplying wavefronts' items
 
     const TokenShape &s = r.shape;
     const int g = blockIdx.x & 7, m = blockIdx.x >> 3, lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6) & (kWaves - 1);
@@ -188,6 +197,7 @@ k_token_run(TokenRun r) {
     }
     if (threadIdx.x == 0) { s_fail = 0; s_far = 0; }
     if (threadIdx.x < 4) reinterpret_cast<uint32_t *>(planes + kZeros)[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < kTokenTiles * 16 * kRed; i += kThreads) red[i] = 0.0f;
     lds_barrier();
 
     struct Part { int t0, tiles, steps; };
@@ -201,36 +211,14 @@ k_token_run(TokenRun r) {
     // splits with keys at position p, and whether this workgroup has some
     auto active_at = [&](int p) { return min(splits, p / TILE + 1); };
     int pos = uniform(r.state[0]);
-    pos = min(max(pos, 0), s.max_seq - 1);                               // (the host never lets it be another; stay in bounds)
+    pos = uniform(min(max(pos, 0), s.max_seq - 1));                      // (the host never lets it be another; stay in bounds)
 
     if (!speaks) {
         // ── the multiplying wavefronts ──
-        // Weights: a phase's first items are asked for as the phase before begins to multiply, so that they are there when that
-        // one's results have been handed on - and are not in front of the words that the speakers wait for: a compute unit's
-        // loads return in order.
+        // A wavefront's items are one stream, the same for every token.  It keeps the next kRing of them in LDS or on their way there.
         const uint32_t lane16 = lane * 16, lane_scale = 1024 + ((lane & 15) * 2 + (lane >> 5)) * 4;
-        const uint32_t start = uniform((int)r.offsets[(g * kMembers + m) * kWaves + wave]);
-        uint32_t at = start;                                             // the phase's first item
-        Hold<kEven> even;
-        Hold<kOdd> odd;
-        auto load = [&](auto &hold, int j, uint32_t item) {
-            const unsigned char *const p = r.items + (uint64_t)(uint32_t)uniform((int)item) * kTokenItemBytes;
-            hold.w[j] = *reinterpret_cast<const intx4 *>(p + lane16);
-            hold.s[j] = *reinterpret_cast<const float *>(p + lane_scale);
-        };
-        // slots [j0, j1) of the n first items from item `from` on
-        auto load_some = [&](auto &hold, uint32_t from, int n, auto j0, auto j1) {
-#pragma unroll
-            for (int j = 0; j < std::remove_reference_t<decltype(hold)>::slots; j++)
-                if (j >= j0 && j < j1 && j < n) load(hold, j, from + j);
-        };
-        constexpr std::integral_constant<int, 0> none{};
-        constexpr std::integral_constant<int, kEven> all_even{};
-        // (the items are here before the next phase's are asked for: waits behind that could not tell them apart)
-        auto arrived = [&](auto &hold) {
-#pragma unroll
-            for (int j = 0; j < hold.slots; j++) asm volatile("" : "+v"(hold.w[j]), "+v"(hold.s[j]));
-        };
+        const unsigned char *const slots = ring + wave * (kRing * kTokenItemBytes);
+        const uint32_t slots_at = uniform((int)(uint32_t)(uintptr_t)(const __attribute__((address_space(3))) unsigned char *)slots);
         struct Work { int tile, st, n, steps; };
         auto work_of = [&](int phase) {
             const int4 q = s_item[phase * kWaves + wave];
@@ -240,127 +228,167 @@ k_token_run(TokenRun r) {
             const TokenItems it = token_items(min(ph.t0 + ph.tiles - t0, kTokenTiles), ph.steps, wave);
             return Work{it.first / ph.steps, it.first % ph.steps, it.end - it.first, ph.steps};
         };
+        const uint32_t start = uniform((int)r.offsets[(g * kMembers + m) * kWaves + wave]);
+        uint32_t end = start;
+        for (int p = kTokenQkv; p <= kTokenDown; p++) end += (uint32_t)(s.layers * work_of(p).n);
+        end += (uint32_t)token_head_items(TokenPart{ph.t0, ph.t0 + ph.tiles, ph.steps}, wave);
+        // When items are asked for.  A compute unit's loads return in order, so what is asked for in front of the words that everybody
+        // waits for delays them by its way from memory; behind a row that has just been sent to the other groups, beside products and
+        // beside the attention there is time for some.  A block of more items than slots needs all of these, a smaller one the few
+        // that delay nothing (us a token, one and the other: 16 blocks of d 2048 343 and 353, 8 of d 1024 100.7 and 97.4).
+        const bool heavy = work_of(kTokenQkv).n + work_of(kTokenWo).n + work_of(kTokenUp).n + work_of(kTokenDown).n > kRing;
+        uint32_t next = start, left = (end - start) * (uint32_t)r.steps; // to be asked for: the next item, and how many in all
+        int held = 0, put = 0, take = 0;                                 // asked for and not multiplied yet; the slots of the next ones
+        auto ask = [&]() {
+            const unsigned char *const p = r.items + (uint64_t)next * kTokenItemBytes;
+            const uint32_t to = slots_at + (uint32_t)put * kTokenItemBytes;
+            load_to_lds16(p, lane16, to);
+            if (lane < 8) load_to_lds16(p + 1024, lane16, to + 1024);    // (lane i's 16 bytes go to 16 i)
+            next = next + 1 == end ? start : next + 1;
+            put = put + 1 == kRing ? 0 : put + 1;
+            held++; left--;
+        };
+        // All but the last `behind` items asked for are here (two loads each; this wavefront makes no others in its loop)
+        auto wait_but = [&](int behind) {
+            if (behind <= 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            else if (behind == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+            else if (behind == 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+            else if (behind == 3) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+            else if (behind == 4) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+            else if (behind == 5) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+            else if (behind == 6) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+            else if (behind == 7) asm volatile("s_waitcnt vmcnt(14)" ::: "memory");
+            else if (behind == 8) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(18)" ::: "memory");
+        };
+        // Up to n more items asked for (the slots' last reads have been answered)
+        auto refill = [&](int n) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            for (; n > 0 && held < kRing && left > 0; n--) ask();
+        };
+        auto leave = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };         // (nothing may be on its way to LDS that is given back)
         // this lane's row of the activations: digit plane (r & 1) | (r & 4) / 2 of scale group r / 8; in the other group's k zeros
         const int quarter = lane >> 4, ar = lane & 15;
         const bool in_group = (ar >> 3) == (quarter >> 1);
         const uint32_t a_plane = (ar & 1) | ((ar >> 1) & 2), a_steps = in_group ? ~0u : 0u;
         const float high = (quarter & 1) ? 65536.0f : 1.0f;
-        // This wavefront's items of `tiles` tiles with the staged row; their sums to red.  Between them, unless they still load some
-        // themselves, the n_after items of `after` are asked for.
-        auto products = [&](auto &hold, const Work &k, int tiles, int pitch, auto &after, int n_after) {
+        const uint32_t unit_at = (quarter >> 1) * 4, red_lane = (lane & 15) * (kRed * 4) + wave * 4;
+        // The next c (1 to 3) items, out of their slots: whatever else of the batch is there is anything
+        constexpr int Q = kTogether;
+        struct Batch { intx4 w[Q]; float s[Q]; };
+        auto take_batch = [&](Batch &b, int c) {
+            wait_but(held - c);
+#pragma unroll
+            for (int q = 0, slot = take; q < Q; q++, slot = slot + 1 == kRing ? 0 : slot + 1) {
+                const unsigned char *const p = slots + slot * kTokenItemBytes;
+                b.w[q] = *reinterpret_cast<const intx4 *>(p + lane16);
+                b.s[q] = *reinterpret_cast<const float *>(p + lane_scale);
+            }
+            held -= c;
+            take = take + c >= kRing ? take + c - kRing : take + c;
+        };
+        Batch b0, b1, b2, b3;                                            // of a phase: its first items, taken before its row is there
+        constexpr int kFirst = 4 * Q;
+        auto take_first = [&](const Work &k) {
+            if (k.n > 0) take_batch(b0, min(Q, k.n));
+            if (k.n > Q) take_batch(b1, min(Q, k.n - Q));
+            if (k.n > 2 * Q) take_batch(b2, min(Q, k.n - 2 * Q));
+            if (k.n > 3 * Q) take_batch(b3, min(Q, k.n - 3 * Q));
+        };
+        // This wavefront's items with the staged row; their sums to red.
+        auto products = [&](const Work &k, int pitch) {
             const uint32_t a_at = in_group ? a_plane * pitch + quarter * 16 : kZeros;
-            int tile = k.tile, st = k.st;
+            int st = k.st;
+            uint32_t to = red_lane + k.tile * (16 * kRed * 4);
             float acc = 0.0f;
-            for (int q = lane; q < tiles * 16; q += 64) red[q * kRed + wave] = 0.0f;
-            // Q items from item i on, in slots j ..: their operands and products together, then their sums one by one
-            auto some = [&](auto count, int j, int i) {
-                constexpr int Q = decltype(count)::value;
+            // The batch with items i, i + 1, ..: operands and products together, then the sums one by one; then it takes the second next
+            auto some = [&](Batch &b, int i) {
+                const int c = min(Q, k.n - i);
                 int sq[Q];
-                intx4 v[Q], c[Q];
+                intx4 v[Q], p[Q];
                 float u[Q];
                 sq[0] = st;
 #pragma unroll
                 for (int q = 1; q < Q; q++) sq[q] = sq[q - 1] + 1 == k.steps ? 0 : sq[q - 1] + 1;
 #pragma unroll
                 for (int q = 0; q < Q; q++) {
-                    v[q] = *reinterpret_cast<const intx4 *>(planes + a_at + (a_steps & (uint32_t)(sq[q] * 64)));
-                    u[q] = unit[sq[q] * 2 + (quarter >> 1)];
+                    v[q] = *reinterpret_cast<const intx4 *>(planes + (a_at + (a_steps & (uint32_t)(sq[q] * 64))));
+                    u[q] = *reinterpret_cast<const float *>(reinterpret_cast<const unsigned char *>(unit) + (unit_at + (uint32_t)sq[q] * 8));
                 }
 #pragma unroll
-                for (int q = 0; q < Q; q++) c[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v[q], hold.w[j + q], (intx4){0, 0, 0, 0}, 0, 0, 0);
+                for (int q = 0; q < Q; q++) p[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v[q], b.w[q], (intx4){0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
                 for (int q = 0; q < Q; q++) {
-                    // C rows 4 quarter + e: digits 2 (quarter & 1) + e of group quarter / 2
-                    const float f = u[q] * high, p = fmaf((float)c[q][1], f * 256.0f, (float)c[q][0] * f);
-                    if (i + q < k.n) {
-                        acc = fmaf(p, hold.s[j + q], acc);
+                    // C rows 4 quarter + e: digits 2 (quarter & 1) + e of group quarter / 2 (up to 2^20 each: their sum is exact)
+                    const float t = (float)((p[q][1] << 8) + p[q][0]) * u[q];
+                    if (q < c) {
+                        acc = fmaf(t, b.s[q], acc);
                         if (sq[q] + 1 == k.steps || i + q == k.n - 1) {
-                            const float v16 = quarters_sum(acc);
-                            if (lane < 16) red[(tile * 16 + lane) * kRed + wave] = v16;
+                            const float v16 = quarters_sum(acc * high);
+                            if (lane < 16) *reinterpret_cast<float *>(reinterpret_cast<unsigned char *>(red) + to) = v16;
                             acc = 0.0f;
-                            tile++;
+                            to += 16 * kRed * 4;
                         }
                     }
                 }
-                st = sq[Q - 1] + 1 == k.steps ? 0 : sq[Q - 1] + 1;
-            };
-            constexpr int kSlots = std::remove_reference_t<decltype(hold)>::slots;
-            constexpr std::integral_constant<int, 3> three{};
-            constexpr std::integral_constant<int, 1> one{};
-            int b = 0;
-            for (; b + kSlots < k.n; b += kSlots)                        // (the last round's slots past n repeat its last item)
-#pragma unroll
-                for (int j = 0; j < kSlots; j += 3) {
-                    some(three, j, b + j);
-#pragma unroll
-                    for (int q = 0; q < 3; q++) load(hold, j + q, at + min(b + kSlots + j + q, k.n - 1));
+                st = sq[c - 1] + 1 == k.steps ? 0 : sq[c - 1] + 1;
+                const int more = k.n - i - kFirst;
+                if (more > 0) {
+                    take_batch(b, min(Q, more));
+                    // (what follows a product is asked for behind its sums)
+                    if (more - Q > held) refill(more - Q - held);
                 }
-            constexpr int kGroups = kSlots / 3, kAfter = std::remove_reference_t<decltype(after)>::slots;
-            auto group = [&](auto q) {
-                constexpr int j = 3 * q;
-                if (b + j + 1 < k.n) some(three, j, b + j);
-                else if (b + j < k.n) some(one, j, b + j);
-                load_some(after, at + k.n, n_after, std::integral_constant<int, kAfter * q / kGroups>{}, std::integral_constant<int, kAfter * (q + 1) / kGroups>{});
             };
-            group(std::integral_constant<int, 0>{});
-            group(std::integral_constant<int, 1>{});
-            if constexpr (kGroups > 2) { group(std::integral_constant<int, 2>{}); group(std::integral_constant<int, 3>{}); }
-            static_assert(kGroups == 2 || kGroups == 4);
+            for (int i = 0; i < k.n; i += kFirst) {
+                some(b0, i);
+                if (i + Q < k.n) some(b1, i + Q);
+                if (i + 2 * Q < k.n) some(b2, i + 2 * Q);
+                if (i + 3 * Q < k.n) some(b3, i + 3 * Q);
+            }
         };
-        // A phase: [staged], the products and what is asked for beside them, [sums]
-        auto phase = [&](auto &hold, auto &after, const Work &k, int tiles, int pitch, int n_after) {
-            arrived(hold);
-            lds_barrier();                                               // [staged]
-            const bool beside = k.n <= hold.slots;
-            products(hold, k, tiles, pitch, after, beside ? n_after : 0);
-            lds_barrier();                                               // [sums]
-            if (!beside) load_some(after, at + k.n, n_after, none, std::integral_constant<int, std::remove_reference_t<decltype(after)>::slots>{});
-            at += k.n;
-        };
-        load_some(even, at, work_of(kTokenQkv).n, none, all_even);
+        refill(kRing);
         lds_barrier();                                                   // [place]
+        Work k = work_of(kTokenQkv);
+        take_first(k);
         for (int step = 0; step < r.steps; step++) {
-            const bool attends = split < active_at(pos) && hl < heads, ends_run = step + 1 == r.steps;
-            for (int i = 0; i < 2 * s.layers; i++) {                     // q | k | v and Wo, up and down
-                const int p0 = 2 * (i & 1), p1 = p0 + 1;
-                const Work k0 = work_of(p0), k1 = work_of(p1), k2 = work_of(i + 1 == 2 * s.layers ? (int)kTokenHead : p0 ^ 2);
-                if (GPT) lds_barrier();                                  // [moments]
-                if (uniform(s_fail) != 0) return;
-                DJ_STAMP2(2 * p0);
-                phase(even, odd, k0, part_of(p0).tiles, pitch_d, k1.n);
-                DJ_STAMP2(2 * p0 + 1);
-                if (p0 == 0) {
-                    // the up projection's weights: the most of a block's, on their way while the speakers attend
-                    const uint32_t up = at + k1.n;
-                    if (attends) lds_barrier();                          // [q k v]
-                    load_some(even, up, k2.n, none, std::integral_constant<int, kEven / 2>{});
-                    if (attends) lds_barrier();                          // [heads]
-                    load_some(even, up, k2.n, std::integral_constant<int, kEven / 2>{}, all_even);
+            const bool attends = split < active_at(pos) && hl < heads;
+            for (int i = 0; i <= 4 * s.layers; i++) {
+                const int p = i == 4 * s.layers ? (int)kTokenHead : i & 3, p_next = i + 1 == 4 * s.layers ? (int)kTokenHead : (p + 1) & 3;
+                const int beside = !heavy ? 0 : p == kTokenWo ? 1 : p == kTokenDown ? 0 : 2;
+                const int after = p == kTokenQkv ? (heavy ? 2 : 0) : p == kTokenWo ? 6 : p == kTokenUp ? 0 : p == kTokenDown ? 1 : kRing;
+                if (GPT && (p & 1) == 0) lds_barrier();                  // [moments]
+                if ((p & 1) == 0 && uniform(s_fail) != 0) return leave();
+                for (int t0 = ph.t0;;) {                                 // (the head's passes; one of any other product)
+                    lds_barrier();                                       // [staged]; of a pass that is not the first, [read]
+                    DJ_STAMP2(2 * p);
+                    refill(max(beside, k.n - kFirst - held));
+                    if (p != kTokenHead || ph.tiles > 0) {               // (without a tile of the head: no pass)
+                        products(k, p == kTokenWo ? pitch_o : p == kTokenDown ? pitch_h : pitch_d);
+                        lds_barrier();                                   // [sums]
+                    }
+                    DJ_STAMP2(2 * p + 1);
+                    t0 += kTokenTiles;
+                    const bool again = p == kTokenHead && t0 < ph.t0 + ph.tiles;
+                    k = again ? head_pass(t0) : work_of(p == kTokenHead ? (int)kTokenQkv : p_next);
+                    refill(max(after, min(k.n, kFirst) - held));
+                    if (!again && p == kTokenHead && step + 1 == r.steps) break;
+                    if (p != kTokenQkv) take_first(k);
+                    if (!again) break;
                 }
-                phase(odd, even, k1, part_of(p1).tiles, p0 == 0 ? pitch_o : pitch_h, p0 == 0 ? 0 : k2.n);
+                if (p == kTokenQkv) {
+                    if (attends) lds_barrier();                          // [q k v]
+                    refill(2);   
+                    if (attends) lds_barrier();                          // [heads]
+                    refill(max(5, k.n - held));
+                    take_first(k);
+                }
             }
-            if (GPT) lds_barrier();                                      // [moments]
-            if (uniform(s_fail) != 0) return;
-            Work k = work_of(kTokenHead);
-            arrived(even);
-            lds_barrier();                                               // [staged]
-            for (int t0 = ph.t0; t0 < ph.t0 + ph.tiles; t0 += kTokenTiles) {
-                const int tiles = min(ph.t0 + ph.tiles - t0, kTokenTiles);
-                const bool last = t0 + tiles == ph.t0 + ph.tiles;
-                if (t0 > ph.t0) lds_barrier();                           // [read]
-                products(even, k, tiles, pitch_d, odd, 0);
-                lds_barrier();                                           // [sums]
-                at += k.n;
-                if (!last) { k = head_pass(t0 + kTokenTiles); load_some(even, at, k.n, none, all_even); }
-            }
-            if (r.choose != kTokenGreedy) return;
-            at = start;
-            if (!ends_run) load_some(even, at, work_of(kTokenQkv).n, none, all_even);
+            if (r.choose != kTokenGreedy) return leave();
             lds_barrier();                                               // [most]
             lds_barrier();                                               // [all]
-            pos = min(pos + 1, s.max_seq - 1);
+            pos = uniform(min(pos + 1, s.max_seq - 1));
         }
-        return;
+        return leave();
     }
 
     // ── the speaking wavefronts ──
@@ -372,11 +400,17 @@ k_token_run(TokenRun r) {
     };
     word *const ex = r.exchange;
     const TokenExchange e = token_exchange(s);
+    const TokenVectors at_vec = token_vectors(s);
     const uint32_t mine = (uint32_t)(g * e.group);                       // the group's words
     // output i of the pass: what the wavefronts left
     auto sum_of = [&](int i) {
         const float4 a = *reinterpret_cast<const float4 *>(red + i * kRed), b = *reinterpret_cast<const float4 *>(red + i * kRed + 4);
         return ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
+    };
+    // .. and zeros again, as they have to be for the wavefronts without items of its tile
+    auto clear = [&](int i) {
+        float4 *const p = reinterpret_cast<float4 *>(red + i * kRed);
+        p[0] = p[1] = make_float4(0.f, 0.f, 0.f, 0.f);
     };
     // A wait that ends without its words says so; behind the next barrier the whole workgroup leaves.
     auto check = [&](bool ok) { if (!ok) s_fail = 1; };
@@ -415,7 +449,7 @@ k_token_run(TokenRun r) {
 #pragma unroll
         for (int q = 0; q < kSets; q++) {
             const int i = t + q * kSpeakers;
-            v[q] = 4 * i < d ? reinterpret_cast<const float4 *>(p)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[q] = 4 * i < d ? *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(p) + (uint32_t)i * 16) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     };
     auto wave_part = [&](int t, float v, float *to) {
@@ -484,6 +518,7 @@ k_token_run(TokenRun r) {
             lds_barrier();                                               // [staged]
             divisor = sqrtf(all_waves(sums) * inv_d + kRmsEps);
             inverse = 1.0f / divisor;
+            asm volatile("" : "+v"(divisor), "+v"(inverse));             // (now, beside the products, and not where they are used)
         }
     };
     // What the workgroup's tiles p of a product leave of the row, added to x.  Between groups: the member's slice of all groups' sums
@@ -494,6 +529,7 @@ k_token_run(TokenRun r) {
             const float v = sum_of(t);
             if (crossing) send(ex, part + g * d + p.t0 * 16 + t, v, tag, true);
             else send(ex, to + p.t0 * 16 + t, v, tag + 1, far);
+            clear(t);
         }
         DJ_STAMP(24);
         // (by wavefronts that have, as a rule, not sent: a wait for loads waits for the stores in front of them too)
@@ -550,14 +586,31 @@ k_token_run(TokenRun r) {
         }
         const int active = active_at(pos);
         const bool attends = hl < heads && split < active;
-        const float2 cs = *reinterpret_cast<const float2 *>(r.cos_t + (int64_t)pos * (HD / 2) + lane % LPK * 2);
-        const float2 sn = *reinterpret_cast<const float2 *>(r.sin_t + (int64_t)pos * (HD / 2) + lane % LPK * 2);
+        const uint32_t angle = (uint32_t)(lane % LPK) * 8;
+        const float2 cs = *reinterpret_cast<const float2 *>(reinterpret_cast<const char *>(r.cos_t + (int64_t)pos * (HD / 2)) + angle);
+        const float2 sn = *reinterpret_cast<const float2 *>(reinterpret_cast<const char *>(r.sin_t + (int64_t)pos * (HD / 2)) + angle);
         // (a phase's small operands are asked for while the products in front of it run)
         float4 gamma[kSets], beta[kSets];
-        row_operand(me(), gamma, r.layers[0].g1);
-        if constexpr (GPT) row_operand(me(), beta, r.layers[0].be1);
+        row_operand(me(), gamma, r.vectors + at_vec.g1);
+        if constexpr (GPT) row_operand(me(), beta, r.vectors + at_vec.be1);
+        // The head's keys and values; a row is HD floats, of which a lane has four.  A round of them: keys of tile
+        // `split + (r0 + u) splits` of TILE (past the cached ones: the first key's, again)
+        floatx4 K[U], V[U];
+        auto keys_at = [&](int l) { return ((int64_t)(l * s.heads + h0 + (hl < heads ? hl : 0)) * s.max_seq) * HD; };
+        auto load_round = [&](int l, int r0) {
+            const char *const kb = reinterpret_cast<const char *>(r.kc + keys_at(l)), *const vb = reinterpret_cast<const char *>(r.vc + keys_at(l));
+            const int t = me(), dl = (t & 63) % LPK, key0 = (t >> 6) * KPW + (t & 63) / LPK;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int key = (split + (r0 + u) * splits) * TILE + key0;
+                const uint32_t from = (key < pos ? key : 0) * (HD * 4) + dl * 16;
+                K[u] = *reinterpret_cast<const floatx4 *>(kb + from);
+                V[u] = *reinterpret_cast<const floatx4 *>(vb + from);
+            }
+        };
+        if (kKeysAhead && attends) load_round(0, 0);
         for (int l = 0; l < s.layers; l++) {
-            const TokenLayer &L = r.layers[l];
+            const float *const vec = r.vectors + (int64_t)l * at_vec.stride;
             const uint32_t tag = tag0 + (uint32_t)l * 8;
             int at_pos = pos, t = me();
             asm volatile("" : "+v"(at_pos));
@@ -570,32 +623,21 @@ k_token_run(TokenRun r) {
             if (give_up()) return;
             t = me();
             const int sub = (t & 63) / LPK, dl = (t & 63) % LPK, key0 = (t >> 6) * KPW + sub;
-            // the head's keys and values; a row is HD floats, of which this lane has four
-            const int64_t base = ((int64_t)(l * s.heads + h0 + (attends ? hl : 0)) * s.max_seq) * HD;
-            char *const kb = reinterpret_cast<char *>(r.kc + base), *const vb = reinterpret_cast<char *>(r.vc + base);
-            float4 K[U], V[U];
-            // keys of tile `split + (r0 + u) splits` of TILE (past the cached ones: the first key's, again)
-            auto load_round = [&](int r0) {
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const int key = (split + (r0 + u) * splits) * TILE + key0;
-                    const uint32_t from = (key < at_pos ? key : 0) * (HD * 4) + dl * 16;
-                    K[u] = *reinterpret_cast<const float4 *>(kb + from);
-                    V[u] = *reinterpret_cast<const float4 *>(vb + from);
-                }
-            };
-            load_round(0);                                               // (whoever attends to none: a row it may read)
+            if (!kKeysAhead && attends) load_round(l, 0);
             const Part pa = part_of(kTokenQkv), pc = part_of(kTokenWo);
             lds_barrier();                                               // [sums]
             DJ_STAMP(3);
-            if (t < pa.tiles * 16) send(ex, mine + e.qkv + pa.t0 * 16 + t, divide(sum_of(t)), tag, far);
+            if (t < pa.tiles * 16) {
+                send(ex, mine + e.qkv + pa.t0 * 16 + t, divide(sum_of(t)), tag, far);
+                clear(t);
+            }
             DJ_STAMP(4);
 
             // ── attention of this workgroup's share of a head's keys ──
             // (they are here; a wait where the ways meet again would also wait for what has been sent)
 #pragma unroll
             for (int u = 0; u < U; u++)
-                asm volatile("" : "+v"(K[u].x), "+v"(K[u].y), "+v"(K[u].z), "+v"(K[u].w), "+v"(V[u].x), "+v"(V[u].y), "+v"(V[u].z), "+v"(V[u].w));
+                asm volatile("" : "+v"(K[u]), "+v"(V[u]));
             if (attends) {
                 if (t < 3 * HD / 2) {
                     const int part = t / (HD / 2), c = 2 * (t - part * (HD / 2));
@@ -620,7 +662,8 @@ k_token_run(TokenRun r) {
                         const int tile = (split + (r0 + u) * splits) * TILE, key = tile + key0;
                         if (tile > at_pos) continue;                     // (uniform; like lanes past the last key it weighs nothing)
                         if (tile + TILE > at_pos && key == at_pos) {     // the new row: used from registers, and appended
-                            K[u] = nk; V[u] = nv;
+                            K[u] = floatx4{nk.x, nk.y, nk.z, nk.w}; V[u] = floatx4{nv.x, nv.y, nv.z, nv.w};
+                            char *const kb = reinterpret_cast<char *>(r.kc + keys_at(l)), *const vb = reinterpret_cast<char *>(r.vc + keys_at(l));
                             const uint32_t to = (uint32_t)key * (HD * 4) + dl * 16;
                             *reinterpret_cast<float4 *>(kb + to) = nk;
                             *reinterpret_cast<float4 *>(vb + to) = nv;
@@ -646,7 +689,7 @@ k_token_run(TokenRun r) {
                 };
                 round(0);
                 for (int r0 = U; (split + r0 * splits) * TILE <= at_pos; r0 += U) {      // workgroup-uniform
-                    load_round(r0);
+                    load_round(l, r0);
                     round(r0);
                 }
                 // the lane groups of a wavefront, then the wavefronts (LDS)
@@ -733,12 +776,12 @@ k_token_run(TokenRun r) {
             if (give_up()) return;
             DJ_STAMP(8);
             t = me();
-            row_operand(t, gamma, L.g2);
-            if constexpr (GPT) row_operand(t, beta, L.be2);
+            row_operand(t, gamma, vec + at_vec.g2);
+            if constexpr (GPT) row_operand(t, beta, vec + at_vec.be2);
             const Part pd = part_of(kTokenUp), pe = part_of(kTokenDown);
             const int unit_n = pd.t0 * (GPT ? 16 : 8) + t;               // this thread's unit of the group's
             const bool has_unit = t < pd.tiles * (GPT ? 16 : 8) && unit_n < units;
-            const float bg = has_unit ? L.bg[u0 + unit_n] : 0.0f, bu = !GPT && has_unit ? L.bu[u0 + unit_n] : 0.0f;
+            const float bg = has_unit ? vec[at_vec.bg + u0 + unit_n] : 0.0f, bu = !GPT && has_unit ? vec[at_vec.bu + u0 + unit_n] : 0.0f;
             lds_barrier();                                               // [sums]
             DJ_STAMP(10);
             exchange_row(t, e.part, e.row, beats, pc, tag + 2);
@@ -751,10 +794,9 @@ k_token_run(TokenRun r) {
             t = me();
             if (give_up()) return;
             float4 bd[kSets];
-            row_operand(t, bd, L.bd);
-            const bool ends = l + 1 == s.layers;
-            row_operand(t, gamma, ends ? r.gf : r.layers[l + 1].g1);
-            if constexpr (GPT) row_operand(t, beta, ends ? r.bf : r.layers[l + 1].be1);
+            row_operand(t, bd, vec + at_vec.bd);
+            row_operand(t, gamma, vec + at_vec.stride + at_vec.g1);
+            if constexpr (GPT) row_operand(t, beta, vec + at_vec.stride + at_vec.be1);
             lds_barrier();                                               // [sums]
             DJ_STAMP(16);
             t = me();
@@ -766,6 +808,10 @@ k_token_run(TokenRun r) {
                     v = gate * (1.0f / (1.0f + expf(-gate))) * up;               // SiLU.java:20-24, SwiGLULayer.java:69
                 }
                 send(ex, mine + e.hid + unit_n, v, tag + 4, far);
+            }
+            if (t < pd.tiles * (GPT ? 16 : 8)) {
+                clear(GPT ? t : 2 * t);
+                if (!GPT) clear(2 * t + 1);
             }
             if (beats_up && t == 0) send(ex, mine + e.beat2 + m, 0.0f, tag + 4, far);
             DJ_STAMP(17);
@@ -801,6 +847,7 @@ k_token_run(TokenRun r) {
                 DJ_STAMP(18);
                 if (give_up()) return;
             }
+            if (kKeysAhead && attends && l + 1 < s.layers) load_round(l + 1, 0);
 #pragma unroll
             for (int q = 0; q < kSets; q++) { x[q].x += bd[q].x; x[q].y += bd[q].y; x[q].z += bd[q].z; x[q].w += bd[q].w; }
             lds_barrier();                                               // [sums]
@@ -821,8 +868,10 @@ k_token_run(TokenRun r) {
             const float bias = has_logit ? r.blm[c] : 0.0f;
             if (t0 > ph.t0) lds_barrier();                               // [read]
             lds_barrier();                                               // [sums]
+            const float sum = has_logit ? sum_of(t) : 0.0f;
+            if (t < tiles * 16) clear(t);
             if (has_logit) {
-                const float v = divide(sum_of(t)) + bias;
+                const float v = divide(sum) + bias;
                 r.logits[c] = v;
                 const uint64_t k = logit_key(v, c);
                 key = k > key ? k : key;
@@ -842,9 +891,11 @@ k_token_run(TokenRun r) {
             send(ex, e.best + kTokenBestWords * (g * kMembers + m) + t, __uint_as_float(t ? (uint32_t)(key >> 32) : (uint32_t)key), tag, crossing || far);
         }
         key = 0;
-        if (t < X * kMembers) {
+        // (by wavefronts that have, as a rule, stored no logits: a wait for loads waits for the stores in front of them too)
+        const int from = t - (kSpeakers - kMembers * kTokenGroupsMost);
+        if (from >= 0 && from < X * kMembers) {
             Words<1> w;
-            uint32_t p[1] = {(uint32_t)(e.best + kTokenBestWords * t)};
+            uint32_t p[1] = {(uint32_t)(e.best + kTokenBestWords * from)};
             check(receive(w, ex, p, tag, r.polls));
             key = (uint64_t)w.v[0].z << 32 | w.v[0].x;
         }
@@ -863,7 +914,7 @@ k_token_run(TokenRun r) {
             r.state[2] = generated + 1;
         }
         generated++;
-        pos = min(pos + 1, s.max_seq - 1);
+        pos = uniform(min(pos + 1, s.max_seq - 1));
     }
     // the next token's embedding, where the launches of a token expect it
     if (g == 0 && m == 0)
@@ -915,6 +966,11 @@ k_token_pack(TokenShape s, int phase, int layer, const int8_t *wq, const float *
     }
 }
 
+__global__ void __launch_bounds__(256) k_token_copy(const float *from, float *to, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) to[i] = from[i];
+}
+
 template <int HD, bool GPT> auto kernel_of(const TokenShape &s) { return s.d <= 4 * kSpeakers ? &k_token_run<HD, GPT, 1> : &k_token_run<HD, GPT, 2>; }
 void (*kernel_for(const TokenShape &s))(TokenRun) {
     if (s.hd == 32) return s.gpt ? kernel_of<32, true>(s) : kernel_of<32, false>(s);
@@ -922,7 +978,7 @@ void (*kernel_for(const TokenShape &s))(TokenRun) {
     return s.gpt ? kernel_of<128, true>(s) : kernel_of<128, false>(s);
 }
 constexpr int kBlocks = kMembers * kTokenGroupsMost;
-constexpr size_t kPadLds = (size_t)24 << 10;             // with the kernel's own more than half of a compute unit's LDS: one workgroup each
+constexpr int kRingBytes = kWaves * kRing * kTokenItemBytes;             // (more than half of a compute unit's LDS: one workgroup each)
 
 }  // namespace
 
@@ -966,7 +1022,8 @@ bool token_run_resident(const TokenShape &s) {
     int device = 0, blocks = 0, units = 0;
     DJ_HIP(hipGetDevice(&device));
     DJ_HIP(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device));
-    DJ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void *>(kernel_for(s)), kThreads, kPadLds));
+    DJ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel_for(s)), hipFuncAttributeMaxDynamicSharedMemorySize, kRingBytes));
+    DJ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void *>(kernel_for(s)), kThreads, kRingBytes));
     return (int64_t)blocks * units >= kBlocks;
 }
 
@@ -991,7 +1048,20 @@ void launch_token_pack(hipStream_t st, const TokenShape &s, int phase, int layer
     launch_kernel(k_token_pack, dim3(s.groups * kMembers * kWaves), dim3(256), 0, st, s, phase, layer, wq, scales, k_total, items, offsets);
 }
 
-void launch_token_run(hipStream_t st, const TokenRun &r) { launch_kernel(kernel_for(r.shape), dim3(kBlocks), dim3(kThreads), kPadLds, st, r); }
+void launch_token_vectors(hipStream_t st, const TokenShape &s, int layer, const TokenLayer &from, float *vectors) {
+    const TokenVectors v = token_vectors(s);
+    float *const to = vectors + (int64_t)layer * v.stride;
+    auto copy = [&](const float *f, int at, int n) { if (f) launch_kernel(k_token_copy, dim3((n + 255) / 256), dim3(256), 0, st, f, to + at, n); };
+    copy(from.g1, v.g1, s.d);
+    copy(from.be1, v.be1, s.d);
+    copy(from.g2, v.g2, s.d);
+    copy(from.be2, v.be2, s.d);
+    copy(from.bd, v.bd, s.d);
+    copy(from.bg, v.bg, s.dff);
+    copy(from.bu, v.bu, s.dff);
+}
+
+void launch_token_run(hipStream_t st, const TokenRun &r) { launch_kernel(kernel_for(r.shape), dim3(kBlocks), dim3(kThreads), kRingBytes, st, r); }
 
 }  // namespace dj
 

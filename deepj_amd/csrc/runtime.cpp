@@ -2160,7 +2160,7 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
         TokenPlan p;
         const int op = DJ_OP_Q8_LINEAR;
         g.track = &p.refs;
-        std::vector<TokenLayer> table((size_t)layers);
+        std::vector<TokenLayer> table((size_t)layers + 1);                       // (the last: the final norm)
         struct Weight { const int8_t *q = nullptr; const float *s = nullptr; int k = 0; };
         std::vector<Weight> weights;
         Weight head;
@@ -2170,8 +2170,8 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
             r.shape = s;
             r.emb = buf(w[8], (int64_t)s.vocab * d, op, "emb");
             r.pos = gpt ? buf(w[9], (int64_t)s.max_seq * d, op, "pos") : nullptr;
-            r.gf = buf(w[10], d, op, "gf");
-            r.bf = gpt ? buf(w[11], d, op, "bf") : nullptr;
+            table.back().g1 = buf(w[10], d, op, "gf");
+            if (gpt) table.back().be1 = buf(w[11], d, op, "bf");
             q8_weight(w[12], d, s.vocab, op, "wlm", head.q, head.s);
             head.k = s.d;
             r.blm = buf(w[13], s.vocab, op, "blm");
@@ -2188,7 +2188,6 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
             for (int l = 0; l < layers; l++) {
                 const int32_t *v = w + DEEPJ_HIP_TOKEN_PLAN_WORDS + l * DEEPJ_HIP_TOKEN_PLAN_LAYER_WORDS;
                 TokenLayer &L = table[(size_t)l];
-                L = TokenLayer{};
                 L.g1 = buf(v[0], d, op, "g1");
                 if (gpt) L.be1 = buf(v[1], d, op, "be1");
                 L.g2 = buf(v[2], d, op, "g2");
@@ -2225,16 +2224,16 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
             p.exchange_words = token_exchange(s).total;
             auto *packed = (unsigned char *)take(items * kTokenItemBytes);
             auto *at = (uint32_t *)take((int64_t)offsets.size() * 4);
-            auto *dev_table = (TokenLayer *)take((int64_t)table.size() * (int64_t)sizeof(TokenLayer));
+            auto *vectors = (float *)take((int64_t)table.size() * token_vectors(s).stride * 4);
             p.run.exchange = (unsigned long long *)take(p.exchange_words * 8);
             p.run.items = packed;
             p.run.offsets = at;
-            p.run.layers = dev_table;
+            p.run.vectors = vectors;
             launch_uploads();
             stage_upload((float *)at, (const float *)offsets.data(), (int64_t)offsets.size());
-            stage_upload((float *)dev_table, (const float *)table.data(), (int64_t)(table.size() * sizeof(TokenLayer) / 4));
             launch_uploads();
             launch_fill(g.stream, (uint32_t *)p.run.exchange, 0, p.exchange_words * 2);
+            for (int l = 0; l <= layers; l++) launch_token_vectors(g.stream, s, l, table[(size_t)l], vectors);
             for (int l = 0; l < layers; l++)
                 for (int phase = kTokenQkv; phase <= kTokenDown; phase++) {
                     const Weight &x = weights[(size_t)l * 4 + phase];

@@ -79,13 +79,20 @@ __host__ __device__ inline TokenExchange token_exchange(const TokenShape &s) {
 }
 
 struct TokenLayer { const float *g1, *be1, *g2, *be2, *bg, *bu, *bd; };
+// A block's norm weights and biases in the plan, one behind the other in floats (the last place is the final norm's, as g1 and
+// be1): addresses the kernel computes, where a table of pointers would be a load in front of every load.
+struct TokenVectors { int g1, be1, g2, be2, bd, bg, bu, stride; };
+__host__ __device__ inline TokenVectors token_vectors(const TokenShape &s) {
+    const int d = s.d, f = (s.dff + 3) & ~3;
+    return TokenVectors{0, d, 2 * d, 3 * d, 4 * d, 5 * d, 5 * d + f, 5 * d + 2 * f};
+}
 enum { kTokenLogits = 0, kTokenGreedy = 1 };
 struct TokenRun {
     TokenShape shape;
     const unsigned char *items;           // every wavefront's items in the order it takes them
     const uint32_t *offsets;              // [groups * members * waves]: a wavefront's first item
-    const TokenLayer *layers;
-    const float *emb, *pos, *gf, *bf, *blm, *cos_t, *sin_t;
+    const float *vectors;                 // [layers + 1] of TokenVectors
+    const float *emb, *pos, *blm, *cos_t, *sin_t;
     float *kc, *vc, *logits, *x;
     int32_t *state, *tokens;
     unsigned long long *exchange;
@@ -102,6 +109,7 @@ int token_run_groups(const TokenShape &s);
 bool token_run_resident(const TokenShape &s);     // whether all of a run's workgroups fit on the device at once
 int64_t token_run_items(const TokenShape &s, uint32_t *offsets);      // their number; offsets[groups * members * waves]
 void launch_token_pack(hipStream_t st, const TokenShape &s, int phase, int layer, const int8_t *wq, const float *scales, int k_total, unsigned char *items, const uint32_t *offsets);
+void launch_token_vectors(hipStream_t st, const TokenShape &s, int layer, const TokenLayer &from, float *vectors);     // (null: left as it is)
 void launch_token_run(hipStream_t st, const TokenRun &r);
 
 }  // namespace dj
