@@ -33,6 +33,10 @@ __host__ __device__ inline bool operand_negated(int c) { return (c / kOperandChu
 __device__ __forceinline__ void load_to_lds16(const void *base, uint32_t off, uint32_t dst) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
 }
+// .. of bytes that pass by: they take no place in the caches from what is read again
+__device__ __forceinline__ void load_passing_to_lds16(const void *base, uint32_t off, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
+}
 __device__ __forceinline__ void load_to_lds4(const void *base, uint32_t off, uint32_t dst) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
 }

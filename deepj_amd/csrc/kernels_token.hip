@@ -33,7 +33,7 @@
 // Bound by the serial chain: instructions on the way from a row's arrival to the next one's departure, one every four clocks of a
 // wavefront at best (a phase of one item a wavefront takes 1200 clocks, an exchange 1000 inside a group and 5000 between groups), and by
 // memory where a block has more than some 20 MB.  Us a token, launches and this: 4 blocks of d 256, 256 words 48.0, 37.3; 8 of d 1024,
-// 8192 words 126, 98; d 2048, 32000 words, 4 blocks 120, 102, 16 blocks 404, 343; GPT, 12 blocks of 768, 50257 words 200, 152.
+// 8192 words 126, 98; d 2048, 32000 words, 4 blocks 120, 97, 16 blocks 404, 331; GPT, 12 blocks of 768, 50257 words 200, 152.
 // Taken back: one set of wavefronts for everything (256 registers: 51.6 us where this takes 36.5); the heads' records merged
 // through LDS; all slots filled behind every phase (372 us at 16 blocks of d 2048); items asked for by the clock while the
 // multiplying wavefronts wait (122 us at 4 blocks, where the same by counts took 114).
@@ -237,13 +237,19 @@ k_token_run(TokenRun r) {
         // beside the attention there is time for some.  A block of more items than slots needs all of these, a smaller one the few
         // that delay nothing (us a token, one and the other: 16 blocks of d 2048 343 and 353, 8 of d 1024 100.7 and 97.4).
         const bool heavy = work_of(kTokenQkv).n + work_of(kTokenWo).n + work_of(kTokenUp).n + work_of(kTokenDown).n > kRing;
+        const bool passing = r.passing != 0;
         uint32_t next = start, left = (end - start) * (uint32_t)r.steps; // to be asked for: the next item, and how many in all
         int held = 0, put = 0, take = 0;                                 // asked for and not multiplied yet; the slots of the next ones
         auto ask = [&]() {
             const unsigned char *const p = r.items + (uint64_t)next * kTokenItemBytes;
             const uint32_t to = slots_at + (uint32_t)put * kTokenItemBytes;
-            load_to_lds16(p, lane16, to);
-            if (lane < 8) load_to_lds16(p + 1024, lane16, to + 1024);    // (lane i's 16 bytes go to 16 i)
+            if (passing) {
+                load_passing_to_lds16(p, lane16, to);
+                if (lane < 8) load_passing_to_lds16(p + 1024, lane16, to + 1024);        // (lane i's 16 bytes go to 16 i)
+            } else {
+                load_to_lds16(p, lane16, to);
+                if (lane < 8) load_to_lds16(p + 1024, lane16, to + 1024);
+            }
             next = next + 1 == end ? start : next + 1;
             put = put + 1 == kRing ? 0 : put + 1;
             held++; left--;

@@ -2227,6 +2227,7 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
             auto *vectors = (float *)take((int64_t)table.size() * token_vectors(s).stride * 4);
             p.run.exchange = (unsigned long long *)take(p.exchange_words * 8);
             p.run.items = packed;
+            p.run.passing = items * kTokenItemBytes > kTokenPassingBytes;
             p.run.offsets = at;
             p.run.vectors = vectors;
             launch_uploads();

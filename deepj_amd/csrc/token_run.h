@@ -13,6 +13,10 @@ constexpr int kTokenTiles = 32;                 // tiles of 16 outputs that a wo
 constexpr int kTokenItemBytes = 1024 + 128;     // 16 outputs x 64 k: the int8 weights in the lanes' order, then their 32 scales
 constexpr int kTokenBestWords = 16;             // a line each: writers of one line wait for one another
 constexpr int kTokenMostD = 4096, kTokenMostSlice = 2048;
+// Items of more bytes than this are loaded as passing by: the memory-side cache (256 MB) does not hold them until the next token, and
+// with them on their way through the caches it does not hold the rows and keys either.  Us a token without and with: 195 MB 88.2
+// and 95.1, 256 MB 121.3 and 124.4, 291 MB 102.8 and 96.6, 326 MB 152.0 and 146.4, 1 GB 344 and 331.
+constexpr int64_t kTokenPassingBytes = 272LL << 20;
 constexpr int kTokenPolls = 1 << 21;            // about a second
 enum TokenPhase { kTokenQkv = 0, kTokenWo = 1, kTokenUp = 2, kTokenDown = 3, kTokenHead = 4 };
 
@@ -99,6 +103,7 @@ struct TokenRun {
     uint32_t *failed;                     // (pinned host memory)
     uint32_t tag;                         // of the run's first exchange
     int steps, choose;
+    int passing;                          // the items are more than kTokenPassingBytes
     int polls;                            // loads of a word until a wait is given up
     float scale;
 };

@@ -29,12 +29,12 @@ def plan_of(m):
 # (gpt, vocab, d, heads, dff, groups, prompt): one to eight groups with even and uneven heads and hidden units; widths that leave
 # workgroups without a tile (64, 96), a last tile of one word, hidden widths no multiple of 64, 8 or 4; all head widths; one key to
 # several rounds of key tiles; wavefronts with more items than slots (2048 over 8192 on four groups, 4096); rows of two sets; heads of
-# several passes, and of none in most workgroups
+# several passes, and of none in most workgroups; more weights than the memory-side cache holds (4096 over 11008 with 60000 words)
 SHAPES = [(False, 251, 64, 2, 50, 1, 3), (False, 17001, 64, 2, 50, 1, 20), (True, 33000, 128, 2, 300, 2, 9), (False, 97, 96, 3, 130, 2, 60), (True, 253, 64, 2, 173, 2, 5), (False, 4097, 256, 8, 697, 1, 30),
           (False, 300, 256, 8, 697, 8, 30), (True, 1003, 320, 10, 1000, 4, 70), (True, 300, 384, 6, 1537, 4, 200), (False, 64, 128, 4, 260, 4, 1),
           (False, 500, 640, 5, 1000, 4, 900), (True, 1000, 768, 12, 3072, 8, 130), (False, 300, 512, 16, 1376, 1, 1500),
           (False, 8193, 1024, 16, 2752, 8, 1100), (False, 300, 2048, 16, 8192, 4, 40), (False, 2000, 2112, 33, 5000, 8, 40),
-          (False, 500, 4096, 32, 11008, 8, 20)]
+          (False, 500, 4096, 32, 11008, 8, 20), (False, 60000, 4096, 32, 11008, 8, 20)]
 
 
 @pytest.mark.parametrize("gpt,vocab,d,heads,dff,groups,prompt", SHAPES)
