@@ -31,9 +31,9 @@
 // nothing kept in memory between phases: each such wait is one for the weights in front of it (GPT 177 us a token, 155 without).
 //
 // Bound by the serial chain: instructions on the way from a row's arrival to the next one's departure, one every four clocks of a
-// wavefront at best (a phase of one item a wavefront takes 1200 clocks, an exchange 1000 inside a group and 5000 between groups), and by
-// memory where a block has more than some 20 MB.  Us a token, launches and this: 4 blocks of d 256, 256 words 48.0, 37.3; 8 of d 1024,
-// 8192 words 126, 98; d 2048, 32000 words, 4 blocks 120, 97, 16 blocks 404, 331; GPT, 12 blocks of 768, 50257 words 200, 152.
+// wavefront at best (a phase of one item a wavefront takes 1100 clocks, an exchange 1000 inside a group and 5000 between groups), and by
+// memory where a block has more than some 20 MB.  Us a token, launches and this: 4 blocks of d 256, 256 words 48.0, 36.2; 8 of d 1024,
+// 8192 words 126, 95.8; d 2048, 32000 words, 4 blocks 120, 92, 16 blocks 404, 314; GPT, 12 blocks of 768, 50257 words 200, 148.
 // Taken back: one set of wavefronts for everything (256 registers: 51.6 us where this takes 36.5); the heads' records merged
 // through LDS; all slots filled behind every phase (372 us at 16 blocks of d 2048); items asked for by the clock while the
 // multiplying wavefronts wait (122 us at 4 blocks, where the same by counts took 114).
@@ -235,7 +235,7 @@ k_token_run(TokenRun r) {
         // When items are asked for.  A compute unit's loads return in order, so what is asked for in front of the words that everybody
         // waits for delays them by its way from memory; behind a row that has just been sent to the other groups, beside products and
         // beside the attention there is time for some.  A block of more items than slots needs all of these, a smaller one the few
-        // that delay nothing (us a token, one and the other: 16 blocks of d 2048 343 and 353, 8 of d 1024 100.7 and 97.4).
+        // that delay nothing (us a token, one and the other: 16 blocks of d 2048 314 and 330, 8 of d 1024 99 and 96).
         const bool heavy = work_of(kTokenQkv).n + work_of(kTokenWo).n + work_of(kTokenUp).n + work_of(kTokenDown).n > kRing;
         const bool passing = r.passing != 0;
         uint32_t next = start, left = (end - start) * (uint32_t)r.steps; // to be asked for: the next item, and how many in all
@@ -307,9 +307,9 @@ k_token_run(TokenRun r) {
             int st = k.st;
             uint32_t to = red_lane + k.tile * (16 * kRed * 4);
             float acc = 0.0f;
-            // The batch with items i, i + 1, ..: operands and products together, then the sums one by one; then it takes the second next
-            auto some = [&](Batch &b, int i) {
-                const int c = min(Q, k.n - i);
+            // A batch of the `rem` items that are left: operands and products together, then the sums one by one; then it takes others
+            auto some = [&](Batch &b, int rem) {
+                const int c = min(Q, rem);
                 int sq[Q];
                 intx4 v[Q], p[Q];
                 float u[Q];
@@ -321,15 +321,16 @@ k_token_run(TokenRun r) {
                     v[q] = *reinterpret_cast<const intx4 *>(planes + (a_at + (a_steps & (uint32_t)(sq[q] * 64))));
                     u[q] = *reinterpret_cast<const float *>(reinterpret_cast<const unsigned char *>(unit) + (unit_at + (uint32_t)sq[q] * 8));
                 }
+                __builtin_amdgcn_sched_barrier(0);                       // (all of them on their way at once)
 #pragma unroll
                 for (int q = 0; q < Q; q++) p[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v[q], b.w[q], (intx4){0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
                 for (int q = 0; q < Q; q++) {
                     // C rows 4 quarter + e: digits 2 (quarter & 1) + e of group quarter / 2 (up to 2^20 each: their sum is exact)
                     const float t = (float)((p[q][1] << 8) + p[q][0]) * u[q];
-                    if (q < c) {
+                    if (q < rem) {
                         acc = fmaf(t, b.s[q], acc);
-                        if (sq[q] + 1 == k.steps || i + q == k.n - 1) {
+                        if (sq[q] + 1 == k.steps || rem == q + 1) {
                             const float v16 = quarters_sum(acc * high);
                             if (lane < 16) *reinterpret_cast<float *>(reinterpret_cast<unsigned char *>(red) + to) = v16;
                             acc = 0.0f;
@@ -338,18 +339,18 @@ k_token_run(TokenRun r) {
                     }
                 }
                 st = sq[c - 1] + 1 == k.steps ? 0 : sq[c - 1] + 1;
-                const int more = k.n - i - kFirst;
+                const int more = rem - kFirst;
                 if (more > 0) {
                     take_batch(b, min(Q, more));
                     // (what follows a product is asked for behind its sums)
                     if (more - Q > held) refill(more - Q - held);
                 }
             };
-            for (int i = 0; i < k.n; i += kFirst) {
-                some(b0, i);
-                if (i + Q < k.n) some(b1, i + Q);
-                if (i + 2 * Q < k.n) some(b2, i + 2 * Q);
-                if (i + 3 * Q < k.n) some(b3, i + 3 * Q);
+            for (int rem = k.n; rem > 0; rem -= kFirst) {
+                some(b0, rem);
+                if (rem > Q) some(b1, rem - Q);
+                if (rem > 2 * Q) some(b2, rem - 2 * Q);
+                if (rem > 3 * Q) some(b3, rem - 3 * Q);
             }
         };
         refill(kRing);
@@ -360,14 +361,14 @@ k_token_run(TokenRun r) {
             const bool attends = split < active_at(pos) && hl < heads;
             for (int i = 0; i <= 4 * s.layers; i++) {
                 const int p = i == 4 * s.layers ? (int)kTokenHead : i & 3, p_next = i + 1 == 4 * s.layers ? (int)kTokenHead : (p + 1) & 3;
-                const int beside = !heavy ? 0 : p == kTokenWo ? 1 : p == kTokenDown ? 0 : 2;
-                const int after = p == kTokenQkv ? (heavy ? 2 : 0) : p == kTokenWo ? 6 : p == kTokenUp ? 0 : p == kTokenDown ? 1 : kRing;
+                const int beside = !heavy ? 0 : p == kTokenQkv ? 2 : p == kTokenWo ? 1 : p == kTokenUp ? 3 : 0;
+                const int after = p == kTokenQkv ? (heavy ? 2 : 0) : p == kTokenWo ? 6 : p == kTokenUp ? (heavy ? 8 : 0) : p == kTokenDown ? 1 : kRing;
                 if (GPT && (p & 1) == 0) lds_barrier();                  // [moments]
                 if ((p & 1) == 0 && uniform(s_fail) != 0) return leave();
                 for (int t0 = ph.t0;;) {                                 // (the head's passes; one of any other product)
                     lds_barrier();                                       // [staged]; of a pass that is not the first, [read]
                     DJ_STAMP2(2 * p);
-                    refill(max(beside, k.n - kFirst - held));
+                    if (max(beside, k.n - kFirst - held) > 0) refill(max(beside, k.n - kFirst - held));
                     if (p != kTokenHead || ph.tiles > 0) {               // (without a tile of the head: no pass)
                         products(k, p == kTokenWo ? pitch_o : p == kTokenDown ? pitch_h : pitch_d);
                         lds_barrier();                                   // [sums]
@@ -383,7 +384,7 @@ k_token_run(TokenRun r) {
                 }
                 if (p == kTokenQkv) {
                     if (attends) lds_barrier();                          // [q k v]
-                    refill(2);   
+                    refill(heavy ? 3 : 2);
                     if (attends) lds_barrier();                          // [heads]
                     refill(max(5, k.n - held));
                     take_first(k);
