@@ -72,7 +72,8 @@ __device__ __forceinline__ void send(word *base, uint32_t at, float v, uint32_t 
     if (far) __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-// N times two words, loaded together past the L1 until all carry the tag.  False: they did not in time.
+// N times two words, loaded together past the L1 until all of them carry the tag, those of all the wavefront's lanes that are here: one
+// count and one branch a try, where lanes that end by themselves cost some forty instructions of masks.  False: they did not in time.
 template <int N> struct Words { uintx4 v[N]; };
 #define DJ_LD(i, at, base) "global_load_dwordx4 %" #i ", %" #at ", %" #base " sc1\n\t"
 __device__ __forceinline__ void fetch(Words<1> &w, const word *b, const uint32_t (&p)[1]) {
@@ -80,6 +81,10 @@ __device__ __forceinline__ void fetch(Words<1> &w, const word *b, const uint32_t
 }
 __device__ __forceinline__ void fetch(Words<2> &w, const word *b, const uint32_t (&p)[2]) {
     asm volatile(DJ_LD(0, 2, 4) DJ_LD(1, 3, 4) "s_waitcnt vmcnt(0)" : "=&v"(w.v[0]), "=&v"(w.v[1]) : "v"(p[0]), "v"(p[1]), "s"(b) : "memory");
+}
+__device__ __forceinline__ void fetch(Words<3> &w, const word *b, const uint32_t (&p)[3]) {
+    asm volatile(DJ_LD(0, 3, 6) DJ_LD(1, 4, 6) DJ_LD(2, 5, 6) "s_waitcnt vmcnt(0)"
+                 : "=&v"(w.v[0]), "=&v"(w.v[1]), "=&v"(w.v[2]) : "v"(p[0]), "v"(p[1]), "v"(p[2]), "s"(b) : "memory");
 }
 __device__ __forceinline__ void fetch(Words<6> &w, const word *b, const uint32_t (&p)[6]) {
     asm volatile(DJ_LD(0, 6, 12) DJ_LD(1, 7, 12) DJ_LD(2, 8, 12) DJ_LD(3, 9, 12) DJ_LD(4, 10, 12) DJ_LD(5, 11, 12) "s_waitcnt vmcnt(0)"
@@ -96,15 +101,16 @@ __device__ __forceinline__ void fetch(Words<8> &w, const word *b, const uint32_t
 template <int N> __device__ __forceinline__ bool receive(Words<N> &w, const word *base, uint32_t (&p)[N], uint32_t tag, int polls) {
 #pragma unroll
     for (int i = 0; i < N; i++) p[i] *= 8;
-    for (int n = polls;;) {                                              // (once at least: w is written on every way out)
+    bool missing;
+    int n = polls;
+    do {                                                                 // (once at least: w is written on every way out)
         fetch(w, base, p);
         uint32_t off = 0;
 #pragma unroll
         for (int i = 0; i < N; i++) off |= (w.v[i].y ^ tag) | (w.v[i].w ^ tag);
-        if (n <= 0) return false;
-        if (off == 0) return true;
-        n--;
-    }
+        missing = __builtin_amdgcn_ballot_w64(off != 0) != 0;
+    } while (missing && --n > 0);
+    return !missing && polls > 0;
 }
 __device__ __forceinline__ float first(uintx4 v) { return __uint_as_float(v.x); }
 __device__ __forceinline__ float second(uintx4 v) { return __uint_as_float(v.z); }
@@ -735,21 +741,22 @@ k_token_run(TokenRun r) {
             t = me();
             if (wo_tiles) {
                 const int p8 = (t & 63) >> 3, q8 = t & 7;
-                for (int v0 = (t >> 6) * 32; v0 < pc.steps * 64; v0 += kWaves * 32) {
+                for (int v0 = wave * 32; v0 < pc.steps * 64; v0 += kWaves * 32) {
                     const int head = min(v0 / HD, heads - 1), c = v0 % HD + 4 * q8;      // (past the heads' values: zeros)
                     float M = -INFINITY, sum = 0.0f;
                     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-                    for (int i = 0; i < active; i += 16) {
-                        uint32_t p[6];
+                    auto records = [&](int i, auto count) {              // of splits i + p8 and, for two, i + 8 + p8
+                        constexpr int J = decltype(count)::value;
+                        uint32_t p[3 * J];
 #pragma unroll
-                        for (int j = 0; j < 2; j++) {
+                        for (int j = 0; j < J; j++) {
                             const uint32_t from = mine + e.rec + (head * splits + min(i + 8 * j + p8, active - 1)) * (HD + 2);
                             p[3 * j] = from + c; p[3 * j + 1] = from + c + 2; p[3 * j + 2] = from + HD;
                         }
-                        Words<6> w;
+                        Words<3 * J> w;
                         check(receive(w, ex, p, tag + 1, r.polls));
 #pragma unroll
-                        for (int j = 0; j < 2; j++) {
+                        for (int j = 0; j < J; j++) {
                             const bool on = i + 8 * j + p8 < active;
                             const float m2 = on ? first(w.v[3 * j + 2]) : -INFINITY, top = fmaxf(M, m2);
                             const float a = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - top), b = on ? __builtin_amdgcn_exp2f(m2 - top) : 0.0f;
@@ -758,7 +765,10 @@ k_token_run(TokenRun r) {
                             o.z = o.z * a + (on ? first(w.v[3 * j + 1]) : 0.0f) * b; o.w = o.w * a + (on ? second(w.v[3 * j + 1]) : 0.0f) * b;
                             M = top;
                         }
-                    }
+                    };
+                    if (active <= 8) records(0, std::integral_constant<int, 1>{});
+                    else
+                        for (int i = 0; i < active; i += 16) records(i, std::integral_constant<int, 2>{});
                     auto parts = [&](float v, auto op) {
                         float a, b;
                         lane_pair<8>(v, a, b);
