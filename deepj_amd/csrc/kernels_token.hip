@@ -58,7 +58,7 @@ constexpr int kSpeakers = 64 * kWaves;           // threads that make, send and 
 constexpr int kThreads = 2 * kSpeakers;
 constexpr int kRing = 12;                        // items of a wavefront in LDS or on their way there (108 KB in all)
 constexpr int kTogether = 3;                     // items whose products are made side by side
-constexpr int kCrossSleep = 16;                  // of 64 clocks
+constexpr int kCrossSleep = 18;                  // of 64 clocks
 constexpr int kRed = 12;                         // floats between two outputs' sums (the wavefronts' eight; 16-byte steps over all banks)
 constexpr float kLog2e = 1.44269504088896340736f;
 
@@ -484,7 +484,7 @@ k_token_run(TokenRun r) {
 #pragma unroll
             for (int q = 0; q < kSets; q++) sm += (x[q].x + x[q].y) + (x[q].z + x[q].w);          // (zeros past the row's end)
             sm = wave_sum_dpp(sm);
-            const float here = n > 0.0f ? sm / n : 0.0f;
+            const float here = n > 0.0f ? sm * __builtin_amdgcn_rcpf(n) : 0.0f;      // (near the mean is enough: what it is off by goes in as a square)
 #pragma unroll
             for (int q = 0; q < kSets; q++) {
                 const bool on = 4 * (t + q * kSpeakers) < d;
@@ -509,7 +509,7 @@ k_token_run(TokenRun r) {
                 const bool on = 4 * (t + q * kSpeakers) < d;
                 c[q] = on ? make_float4(x[q].x - mean, x[q].y - mean, x[q].z - mean, x[q].w - mean) : make_float4(0.f, 0.f, 0.f, 0.f);
             }
-            const float sd = sqrtf(squares * inv_d + kLayerNormEps), isd = 1.0f / sd;
+            const float sd = sqrtf(squares * inv_d + kLayerNormEps), isd = __builtin_amdgcn_rcpf(sd);        // (each quotient is corrected by its residual)
             auto over = [&](float v) { const float y = v * isd; return fmaf(fmaf(-y, sd, v), isd, y); };
 #pragma unroll
             for (int q = 0; q < kSets; q++)
@@ -545,6 +545,9 @@ k_token_run(TokenRun r) {
             clear(t);
         }
         DJ_STAMP(24);
+        // Nothing can be here yet.  Words of the row would only be in the way, and a first try for the other groups' sums that comes too early costs
+        // its whole way before the next (us a token at GPT 12 blocks of 768 and 16 of d 2048: without 5 and 5 more, 12 139.0 and 314.0, this 138.2 and 313.4, 32 5 and 1 more).
+        if (crossing) __builtin_amdgcn_s_sleep(kCrossSleep);
         // (by wavefronts that have, as a rule, not sent: a wait for loads waits for the stores in front of them too)
         if (crossing && t >= kSpeakers / 2 && t - kSpeakers / 2 < p.tiles * 8) {         // two outputs a thread
             const int o = p.t0 * 16 + 2 * (t - kSpeakers / 2);
@@ -560,7 +563,6 @@ k_token_run(TokenRun r) {
             send(ex, to + o, a, tag + 1, far);
             send(ex, to + o + 1, b, tag + 1, far);
         }
-        else if (crossing) __builtin_amdgcn_s_sleep(kCrossSleep);        // (nothing of the row can be here yet: its first words would only be in the way)
         DJ_STAMP(25);
         if (beat && t == kSpeakers - 1) send(ex, mine + e.beat + m, 0.0f, tag + 1, far);
         if (beat && t >= kSpeakers - kMembers / 2) {
@@ -782,7 +784,7 @@ k_token_run(TokenRun r) {
                     const float top = parts(M, [](float a, float b) { return fmaxf(a, b); }), w = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - top);
                     sum = parts(sum * w, add);
                     o = make_float4(parts(o.x * w, add), parts(o.y * w, add), parts(o.z * w, add), parts(o.w * w, add));
-                    const float inv = 1.0f / sum;
+                    const float inv = __builtin_amdgcn_rcpf(sum);
                     auto over = [&](float v) { const float y = v * inv; return fmaf(fmaf(-y, sum, v), inv, y); };
                     o = v0 < slice ? make_float4(over(o.x), over(o.y), over(o.z), over(o.w)) : make_float4(0.f, 0.f, 0.f, 0.f);
                     if (p8 == 0) stage_digits4(planes, pitch_o, unit, v0 / 4 + q8, o);
