@@ -216,7 +216,7 @@ k_token_run(TokenRun r) {
     const bool wo_tiles = part_of(kTokenWo).tiles > 0;
     // splits with keys at position p, and whether this workgroup has some
     auto active_at = [&](int p) { return min(splits, p / TILE + 1); };
-    int pos = uniform(r.state[0]);
+    int pos = uniform(r.given ? r.pos_given : r.state[0]);
     pos = uniform(min(max(pos, 0), s.max_seq - 1));                      // (the host never lets it be another; stay in bounds)
 
     if (!speaks) {
@@ -432,7 +432,7 @@ k_token_run(TokenRun r) {
         if (threadIdx.x == 0) __hip_atomic_store(r.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         return true;
     };
-    int token = uniform(r.state[1]), generated = uniform(r.state[2]);
+    int token = uniform(r.given ? r.token_given : r.state[1]), generated = uniform(r.given ? r.generated_given : r.state[2]);
     // A group's words stay in its L2 only if its workgroups all run on one XCD; else they go through memory.
     {
         const int t = threadIdx.x;
@@ -897,7 +897,10 @@ k_token_run(TokenRun r) {
             }
         }
         DJ_STAMP(26);
-        if (r.choose != kTokenGreedy) return;
+        if (r.choose != kTokenGreedy) {
+            if (r.given && g == 0 && m == 0 && threadIdx.x == 0) { r.state[0] = pos + 1; r.state[1] = token; r.state[2] = generated; }
+            return;
+        }
 
         // ── the largest one ──
         const uint32_t tag = tag0 + (uint32_t)s.layers * 8;

@@ -614,17 +614,17 @@ bool settle(Runner &r, bool arrived = false) {
     r.pending = Runner::kSettled;
     if (!deepj_hip_token_plan_failed(r.plan)) return false;
     drop_plan(r);
-    int32_t st[4];
-    hip(deepj_hip_download(r.state, reinterpret_cast<float *>(st), 4));
-    const int at = was == Runner::kStep ? r.pos - 1 : st[0], steps = r.pos - at;
     if (was == Runner::kStep) {
-        st[0] = at;
-        st[1] = r.pending_token;
-        hip(deepj_hip_upload(r.state, reinterpret_cast<const float *>(st), 4));
+        r.pos -= 1;
+        upload_state(r, r.pending_token);
         r.run(decode_stream(r, kNone, false));
+        r.pos += 1;
         upload_state(r, r.pending_token);
         return true;
     }
+    int32_t st[4];
+    hip(deepj_hip_download(r.state, reinterpret_cast<float *>(st), 4));
+    const int steps = r.pos - st[0];
     Stream s;                                                // (the embedding that the launches start from)
     emit(s, DJ_OP_EMBED_GATHER, r.emb, r.state, r.dec.x, 1, r.cfg.d, r.cfg.vocab, 1);
     r.run(s);
@@ -775,15 +775,14 @@ void step_token(Runner &r, int32_t token, int mode) {
     if (r.pos + 1 > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + 1) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
     settle(r);
-    upload_state(r, token);
     if (r.plan && mode == 1) {
-        hip(deepj_hip_token_plan_run(r.plan, 1, 0));
+        hip(deepj_hip_token_plan_step(r.plan, r.pos, token, r.generated));
         r.pos += 1;
-        upload_state(r, token);
         r.pending = Runner::kStep;
         r.pending_token = token;
         return;
     }
+    upload_state(r, token);
     // Replayed like a greedy token: the launches of a token one by one cost the host 2.4 us each (43 of them: 190 us a
     // step of 8 layers, 130 as a graph).
     const bool narrow = r.pos < r.narrow_positions();

@@ -71,6 +71,7 @@ struct TokenPlan {
     std::vector<Block> blocks;        // device memory it owns
     int64_t exchange_words = 0;
     uint32_t next_tag = 1;            // (the exchange block starts as zeros)
+    uint64_t releases_seen = 0;       // g.releases when refs were last found to be there
     int slot = -1;                    // its word of the pinned block: set by a run that could not finish
 };
 constexpr int kPlanSlots = 1024;
@@ -113,6 +114,7 @@ struct Runtime {
     std::unordered_map<int32_t, Graph> graphs;
     int32_t next_graph = 1;
     std::map<int32_t, TokenPlan> plans;
+    uint64_t releases = 0;                         // buffers that have gone so far
     int32_t next_plan = 1;
     unsigned *attn_counters = nullptr;             // kAttnCounterHeads zeroed words: decode attention's split arrivals
     unsigned char *static_scratch = nullptr;       // device address of `scratch` below on g.device
@@ -1689,6 +1691,7 @@ int deepj_hip_release(const int32_t *ids, int32_t count) {
             g.live_bytes -= (int64_t)it->second.capacity;
             pool_free(it->second.ptr, it->second.capacity);
             g.live.erase(it);
+            g.releases++;
             forget_prepared(ids[i]);
         }
     });
@@ -1775,6 +1778,7 @@ int deepj_hip_shutdown(void) {
         g.plans.clear();
         for (auto &kv : g.live) (void)hipFree(kv.second.ptr);
         g.live.clear();
+        g.releases++;
         for (auto &kv : g.cache)
             for (void *p : kv.second) (void)hipFree(p);
         g.cache.clear();
@@ -2252,40 +2256,70 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
         p.slot = (int)(std::find(used.begin(), used.end(), false) - used.begin());
         p.run.failed = (uint32_t *)(g.pinned + kPlansAt) + p.slot;
         *p.run.failed = 0;
+        p.releases_seen = g.releases;
         *handle = g.next_plan++;
         g.plans.emplace(*handle, std::move(p));
     });
 }
 
+// The plan, if the buffers it was made over are still there: looked up again only once some buffer has been released.
+static TokenPlan &plan_of(int32_t handle, const char *call) {
+    auto it = g.plans.find(handle);
+    if (it == g.plans.end()) fail(std::string(call) + ": unknown plan " + std::to_string(handle));
+    TokenPlan &p = it->second;
+    if (p.releases_seen == g.releases) return p;
+    for (const auto &ref : p.refs) {
+        auto b = g.live.find(ref.first);
+        if (b == g.live.end() || b->second.ptr != ref.second)
+            fail(std::string(call) + ": buffer id=" + std::to_string(ref.first) + " was released or reallocated after plan " + std::to_string(handle) + " was made");
+    }
+    p.releases_seen = g.releases;
+    return p;
+}
+
+static void plan_launch(TokenPlan &p, TokenRun r) {
+    const uint64_t need = 1 + (uint64_t)r.steps * token_tags(r.shape);
+    if (p.next_tag + need > 0xffffffffull) {                     // tags start over: nothing of them may be left
+        launch_fill(g.stream, (uint32_t *)r.exchange, 0, p.exchange_words * 2);
+        p.next_tag = 1;
+    }
+    r.tag = p.next_tag;
+    launch_token_run(g.stream, r);
+    p.next_tag += (uint32_t)need;
+}
+
 int deepj_hip_token_plan_run(int32_t handle, int32_t steps, int32_t choose) {
     return guarded([&] {
-        auto it = g.plans.find(handle);
-        if (it == g.plans.end()) fail("token_plan_run: unknown plan " + std::to_string(handle));
-        TokenPlan &p = it->second;
         if (choose != kTokenLogits && choose != kTokenGreedy) fail("token_plan_run: choose must be 0 (logits only) or 1 (greedy)");
         if (steps < 1 || (choose == kTokenLogits && steps != 1)) fail("token_plan_run: bad step count " + std::to_string(steps));
-        for (const auto &ref : p.refs) {
-            auto b = g.live.find(ref.first);
-            if (b == g.live.end() || b->second.ptr != ref.second)
-                fail("token_plan_run: buffer id=" + std::to_string(ref.first) + " was released or reallocated after plan " + std::to_string(handle) + " was made");
-        }
+        TokenPlan &p = plan_of(handle, "token_plan_run");
         launch_uploads();
         // (launches of a moderate length: a run of thousands of tokens does not hold the device in one piece)
         constexpr int kMost = 256;
         for (int done = 0; done < steps; done += kMost) {
-            const int n = std::min(kMost, steps - done);
-            const uint64_t need = 1 + (uint64_t)n * token_tags(p.run.shape);
-            if (p.next_tag + need > 0xffffffffull) {             // tags start over: nothing of them may be left
-                launch_fill(g.stream, (uint32_t *)p.run.exchange, 0, p.exchange_words * 2);
-                p.next_tag = 1;
-            }
             TokenRun r = p.run;
-            r.tag = p.next_tag;
-            r.steps = n;
+            r.steps = std::min(kMost, steps - done);
             r.choose = choose;
-            launch_token_run(g.stream, r);
-            p.next_tag += (uint32_t)need;
+            plan_launch(p, r);
         }
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) fail(std::string("kernel launch failed: ") + hipGetErrorString(e));
+    });
+}
+
+int deepj_hip_token_plan_step(int32_t handle, int32_t pos, int32_t token, int32_t generated) {
+    return guarded([&] {
+        TokenPlan &p = plan_of(handle, "token_plan_step");
+        if (pos < 0 || pos >= p.run.shape.max_seq) fail("token_plan_step: position " + std::to_string(pos) + " outside the context window");
+        launch_uploads();
+        TokenRun r = p.run;
+        r.steps = 1;
+        r.choose = kTokenLogits;
+        r.given = 1;
+        r.pos_given = pos;
+        r.token_given = token;
+        r.generated_given = generated;
+        plan_launch(p, r);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) fail(std::string("kernel launch failed: ") + hipGetErrorString(e));
     });

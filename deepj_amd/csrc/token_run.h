@@ -103,6 +103,7 @@ struct TokenRun {
     uint32_t *failed;                     // (pinned host memory)
     uint32_t tag;                         // of the run's first exchange
     int steps, choose;
+    int given, pos_given, token_given, generated_given;       // given: the state by value, for one token without a choice; the run leaves it one position on
     int passing;                          // the items are more than kTokenPassingBytes
     int polls;                            // loads of a word until a wait is given up
     float scale;

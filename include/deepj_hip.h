@@ -329,6 +329,9 @@ int32_t deepj_hip_q8_gemm_f16_extents(int32_t m, int32_t k, int32_t rows, int32_
 #define DEEPJ_HIP_TOKEN_PLAN_LAYER_WORDS 11
 int deepj_hip_token_plan_create(const int32_t *words, int32_t n, int32_t *plan);
 int deepj_hip_token_plan_run(int32_t plan, int32_t steps, int32_t choose);
+/* One token that the caller chose, at a position of the caller's (the buffers' state words are not read): logits, and the state
+ * {pos + 1, token, generated}. */
+int deepj_hip_token_plan_step(int32_t plan, int32_t pos, int32_t token, int32_t generated);
 int32_t deepj_hip_token_plan_failed(int32_t plan);
 int32_t deepj_hip_token_plan_groups(int32_t plan);       /* its groups (XCDs); 0: no such plan */
 /* Loads after which a workgroup gives a word up that it waits for (2^21, the most, to begin with; 0: at once) */

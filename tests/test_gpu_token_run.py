@@ -3,7 +3,7 @@ work is dealt to groups and workgroups, at the edges of its tiles, slices, key s
 import numpy as np
 import pytest
 
-from deepj_amd import GPTConfig, GPTModel, LlamaConfig, LlamaModel, TextGenerator, parameter_names, parameter_shapes
+from deepj_amd import models, GPTConfig, GPTModel, LlamaConfig, LlamaModel, TextGenerator, parameter_names, parameter_shapes
 from deepj_amd._native import library
 from oracle import cpu_ref as ref
 
@@ -144,6 +144,55 @@ def test_a_run_that_cannot_finish_is_done_by_launches(groups):
         good.close()
 
 
+@pytest.mark.parametrize("gpt,groups", [(False, 1), (True, 8)])
+def test_a_step_leaves_the_state_that_launches_leave(gpt, groups):
+    """Steps in front of prompts whose tokens go on as runs and as launches, with and without tokens generated before them."""
+    ids = ref.JavaRandom(3).ints(30, 500)
+    got = []
+    for g in (groups, -1):
+        m = model(gpt, 500, 90, 256, 8, 2, 300, g)
+        try:
+            m.prefill(ids[:5], choose_next=False)
+            for t in range(5, 8):
+                m.step(int(ids[t]))
+            m.prefill(ids[8:10])
+            m.decode(6)
+            m.step(int(ids[10]))
+            m.step(int(ids[11]))
+            m.prefill(ids[12:13])
+            m.decode(3, use_graph=False)
+            m.step(int(ids[13]))
+            m.prefill(ids[14:20])
+            m.decode(4)
+            m.step(int(ids[20]))
+            got.append((m.tokens(), m.lastLogits()))
+        finally:
+            m.close()
+    assert np.array_equal(got[0][0], got[1][0]) and len(got[0][0]) == 16
+    assert float(np.max(np.abs(got[0][1] - got[1][1]))) <= 2e-4
+
+
+def test_a_plan_whose_buffer_has_gone_is_refused():
+    """Its buffers are looked up again once some buffer has been released: runs go on where another model's have gone, and end where the
+    plan's own first one (the embedding) has."""
+    lib = library()
+    other = model(False, 300, 40, 64, 2, 1, 50, 1)
+    base = models._next_id_base[0]
+    m = model(False, 300, 40, 256, 8, 1, 300, 1)
+    try:
+        assert parameter_names(m.cfg)[0] == "emb"
+        m.prefill(ref.JavaRandom(1).ints(4, 300))
+        other.close()
+        m.decode(2)
+        m.step(7)
+        assert len(m.tokens()) == 3
+        lib.deepj_hip_release(np.array([base], dtype=np.int32).ctypes.data, 1)
+        assert lib.deepj_hip_token_plan_run(plan_of(m), 1, 1) != 0 and b"released" in lib.deepj_hip_last_error()
+        assert lib.deepj_hip_token_plan_step(plan_of(m), 7, 1, 3) != 0 and b"released" in lib.deepj_hip_last_error()
+    finally:
+        m.close()
+
+
 def test_plans_are_refused_with_a_reason_or_not_made():
     lib = library()
     m = model(False, 300, 40, 256, 8, 1, 300, 1)
@@ -154,6 +203,9 @@ def test_plans_are_refused_with_a_reason_or_not_made():
         assert lib.deepj_hip_token_plan_run(plan, 1, 2) != 0 and b"choose" in lib.deepj_hip_last_error()
         assert lib.deepj_hip_token_plan_run(plan + 1000, 1, 1) != 0 and b"unknown plan" in lib.deepj_hip_last_error()
         assert lib.deepj_hip_token_plan_set_polls(plan, -1) != 0
+        assert lib.deepj_hip_token_plan_step(plan, 40, 1, 0) != 0 and b"context window" in lib.deepj_hip_last_error()
+        assert lib.deepj_hip_token_plan_step(plan, -1, 1, 0) != 0
+        assert lib.deepj_hip_token_plan_step(plan + 1000, 0, 1, 0) != 0 and b"unknown plan" in lib.deepj_hip_last_error()
     finally:
         m.close()
     assert lib.deepj_hip_token_plan_run(plan, 1, 1) != 0             # gone with its model
