@@ -32,11 +32,12 @@
 //
 // Bound by the serial chain: instructions on the way from a row's arrival to the next one's departure, one every four clocks of a
 // wavefront at best (a phase of one item a wavefront takes 1100 clocks, an exchange 1000 inside a group and 5000 between groups), and by
-// memory where a block has more than some 20 MB.  Us a token, launches and this: 4 blocks of d 256, 256 words 48.0, 36.2; 8 of d 1024,
-// 8192 words 126, 95.8; d 2048, 32000 words, 4 blocks 120, 92, 16 blocks 404, 314; GPT, 12 blocks of 768, 50257 words 200, 148.
+// memory where a block has more than some 20 MB.  Us a token, launches and this: 4 blocks of d 256, 256 words 48.0, 33.0; 8 of d 1024,
+// 8192 words 126, 87.7; d 2048, 32000 words, 4 blocks 120, 92, 16 blocks 404, 310; GPT, 12 blocks of 768, 50257 words 200, 137.
 // Taken back: one set of wavefronts for everything (256 registers: 51.6 us where this takes 36.5); the heads' records merged
-// through LDS; all slots filled behind every phase (372 us at 16 blocks of d 2048); items asked for by the clock while the
-// multiplying wavefronts wait (122 us at 4 blocks, where the same by counts took 114).
+// through LDS; all slots filled behind every phase (372 us at 16 blocks of d 2048 where this took 343); items asked for by the clock
+// while the multiplying wavefronts wait (122 us at 4 blocks, where the same by counts took 114); the other groups' sums awaited by several
+// wavefronts by turns (GPT 153 where one takes 152); a key tile alone without the other three's weights (registers to memory: 146).
 #include <type_traits>
 
 #include "dj_common.h"
@@ -374,12 +375,14 @@ k_token_run(TokenRun r) {
                 for (int t0 = ph.t0;;) {                                 // (the head's passes; one of any other product)
                     lds_barrier();                                       // [staged]; of a pass that is not the first, [read]
                     DJ_STAMP2(2 * p);
+                    __builtin_amdgcn_s_setprio(2);                       // (in front of what the speakers do beside them: 0.8 % of a token)
                     if (max(beside, k.n - kFirst - held) > 0) refill(max(beside, k.n - kFirst - held));
                     if (p != kTokenHead || ph.tiles > 0) {               // (without a tile of the head: no pass)
                         products(k, p == kTokenWo ? pitch_o : p == kTokenDown ? pitch_h : pitch_d);
                         lds_barrier();                                   // [sums]
                     }
                     DJ_STAMP2(2 * p + 1);
+                    __builtin_amdgcn_s_setprio(0);
                     t0 += kTokenTiles;
                     const bool again = p == kTokenHead && t0 < ph.t0 + ph.tiles;
                     k = again ? head_pass(t0) : work_of(p == kTokenHead ? (int)kTokenQkv : p_next);
@@ -1020,10 +1023,10 @@ bool token_run_ok(const TokenShape &s) {
     return (int64_t)s.layers * s.heads * s.max_seq < (int64_t)1 << 31;
 }
 
-// Groups for a model.  One alone crosses nothing, and gets its weights at what one XCD's share of the memory gives: a token of a
-// 4-layer Llama takes 30.5 us and 1.13 more per MB of weights on one, 43.5 and 0.12 on eight (42 and 0.21 on four), so one is
-// the better choice up to some 3 MB a layer (d 256 over 4096 words: 36.9 us, 44 on eight; d 384: 43.4, 44.4 on four; d 512: 49.3,
-// 45.3 on eight).  Else as many as there are heads for (d 1024: 51.6 us on eight, 56.0 on four, 73.9 on two).
+// Groups for a model.  One alone crosses nothing, and gets its weights at what one XCD's share of the memory gives; it is the better choice
+// up to some 3 MB a layer (us a token on one group and on the most: 0.2 MB a layer 41.0 and 52.2, 0.8 MB 102.6 and 123.3, 1.5 MB 31.1 and
+// 33.9, 2.2 MB 66.1 and 68.4, 2.6 MB 34.5 and 34.4, 3.0 MB 59.8 and 61.2, 4.5 MB 29.3 and 26.6, 5.0 MB 76.0 and 63.6, 5.4 MB 96.0 and 71.5).  Else as
+// many as there are heads for (d 896: 93.2 us on eight, 97.5 on four, 119 on two).
 int token_run_groups(const TokenShape &s) {
     constexpr int64_t kOneGroup = (int64_t)3 << 20;
     const int64_t bytes = ((int64_t)s.layers * (4LL * s.d * s.d + (s.gpt ? 2LL : 3LL) * s.d * s.dff) + (int64_t)s.d * s.vocab) * 9 / 8;
