@@ -104,7 +104,7 @@ int deepj_hip_time_ops(const int32_t *cmd, int32_t len, int32_t iters, float *ms
  * launch takes along ops behind (element-wise ones, transposes, AdamW updates) its time stands at the first of them and
  * the others have launched nothing; an op by itself is measured in a stream of its own.  us_longest (optional, same length): the op's longest single dispatch, its
  * main kernel; dispatches (optional): how many the op made.  *n_ops = ops in the stream; fails when capacity is
- * smaller. */
+ * smaller.  The stream runs two more times in front, uncounted. */
 int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float *us_per_op, int32_t capacity,
                           int32_t *n_ops, float *us_longest, int32_t *dispatches);
 /* Measurement aid, no counterpart in the reference: the shader clock while a stream runs.  A one-wavefront kernel on a
