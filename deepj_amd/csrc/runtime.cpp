@@ -2228,10 +2228,18 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
                 return m;
             };
             p.exchange_words = token_exchange(s).total;
-            auto *packed = (unsigned char *)take(items * kTokenItemBytes);
-            auto *at = (uint32_t *)take((int64_t)offsets.size() * 4);
-            auto *vectors = (float *)take((int64_t)table.size() * token_vectors(s).stride * 4);
-            p.run.exchange = (unsigned long long *)take(p.exchange_words * 8);
+            unsigned char *packed;
+            uint32_t *at;
+            float *vectors;
+            try {
+                packed = (unsigned char *)take(items * kTokenItemBytes);
+                at = (uint32_t *)take((int64_t)offsets.size() * 4);
+                vectors = (float *)take((int64_t)table.size() * token_vectors(s).stride * 4);
+                p.run.exchange = (unsigned long long *)take(p.exchange_words * 8);
+            } catch (const std::exception &) {                               // a model that fits without a plan goes on without one
+                plan_release(p);
+                return;
+            }
             p.run.items = packed;
             p.run.passing = items * kTokenItemBytes > kTokenPassingBytes;
             p.run.offsets = at;

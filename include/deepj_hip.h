@@ -318,7 +318,7 @@ int32_t deepj_hip_q8_gemm_f16_extents(int32_t m, int32_t k, int32_t rows, int32_
  *     heads, layers, dff, groups (0: the library's choice, else 1 to 8 XCDs), emb, pos (GPT), gf, bf (GPT), wlm, blm, cosT, sinT,
  *     kCache, vCache [layers][heads][maxSeq][hd], state, tokens, logits, x}, then per layer {g1, be1 (GPT), g2, be2 (GPT), wqkv [3 d]
  *     rows, wo, wgu (Llama: rows 2 n gate, 2 n + 1 up), bg, bu (Llama), wd, bd}.  *plan = 0, without an error, where the
- *     shape or the device is not one for it: DECODE_ATTN ... DECODE_NEXT are the way.
+ *     shape or the device is not one for it, or the memory does not suffice: DECODE_ATTN ... DECODE_NEXT are the way.
  *   run: `steps` tokens from state {position, token, generated}.  choose 1: each like the ops of a token with DECODE_NEXT behind
  *     them (logits hold the last one's, x its successor's embedding); choose 0: one token up to its logits, state as it was.
  *     Enqueues only.  Buffers that were released or made again since are refused.
