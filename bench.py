@@ -7,11 +7,14 @@ Workload (the configuration the headline metric is quoted on):
 Llama decode, dModel 2048, 16 layers, 32 heads (head dim 64), SwiGLU hidden 5632, vocab
 32000, maxSeq 2048; weights = new LlamaModel(cfg, 42) (java.util.Random Gaussians x 0.1),
 all matmul weights Q8; prompt = 512 ids from Random(3).nextInt(32000); batch-1 greedy decode
-with a device-resident fp32 KV cache.  A step = one decoded token (one replay of the
-per-token HIP graph).  Prints ONE JSON line.
+with a device-resident fp32 KV cache.  A step = one decoded token (of a run of tokens
+in one launch).  Prints ONE JSON line.
 
 Besides tok/s the line carries
-  roofline     - the Q8 matvec kernel (the dominant kernel): algorithmic bytes per launch /
+  end_to_end   - bytes a decoded token cannot do without over its time (`frac_of_hbm_peak`): what the
+                 run of tokens reaches of the memory
+  roofline     - the Q8 matvec kernel, which tokens run on that are launches (`--eager`, models and
+                 devices without such runs): algorithmic bytes per launch /
                  mean kernel duration, measured live with a start and a stop HIP event on every
                  dispatch of the per-token stream run in order on the model's own weights (1 GB of
                  distinct weights per token, so nothing is served from the 256 MB Infinity Cache) -
@@ -587,7 +590,7 @@ def main() -> int:
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--prompt", type=int, default=512)
     ap.add_argument("--eager", action="store_true",
-                    help="decode without the HIP graph (same kernels, launched one by one): for runs under a tracer")
+                    help="decode by launches, one by one (the kernels of `roofline`): for runs under a tracer")
     ap.add_argument("--prefill-only", action="store_true",
                     help="stop after the prompt: prints the prefill object alone (short runs under a counter-collecting profiler)")
     ap.add_argument("--sweep", action="store_true",
@@ -646,7 +649,7 @@ def main() -> int:
         return 0
 
     graph = False if args.eager else None
-    model.decode(args.warmup, use_graph=graph)      # captures the graph on first use
+    model.decode(args.warmup, use_graph=graph)
     HipNative.synchronize()
     t0 = time.perf_counter()
     model.decode(args.steps, use_graph=graph)
