@@ -705,6 +705,10 @@ k_token_run(TokenRun r) {
                         mx = mn;
                     }
                 };
+                // Row 0 stands in for keys past the cached ones; at the first position it holds anything, and weighs nothing as zeros only
+                if (at_pos == 0)
+#pragma unroll
+                    for (int u = 0; u < U; u++) V[u] = floatx4{0.f, 0.f, 0.f, 0.f};
                 round(0);
                 for (int r0 = U; (split + r0 * splits) * TILE <= at_pos; r0 += U) {      // workgroup-uniform
                     load_round(l, r0);

@@ -227,3 +227,45 @@ def test_plans_are_refused_with_a_reason_or_not_made():
     with pytest.raises(ValueError, match="token groups must be"):
         m.setTokenGroups(9)
     m.close()
+
+
+def bare(gpt, groups, d=256, heads=8, dff=600, vocab=300, max_seq=40, layers=2, seed=7, **changed):
+    """A small model; `changed` maps a weight's name (dots as __) to what makes its values from the drawn ones."""
+    cfg = (GPTConfig if gpt else LlamaConfig)(vocab, max_seq, d, heads, layers, dff)
+    m = (GPTModel if gpt else LlamaModel)(cfg, None)
+    m.setTokenGroups(groups)
+    rng = np.random.default_rng(seed)
+    for name, (r, c) in zip(parameter_names(cfg), parameter_shapes(cfg)):
+        a = rng.standard_normal((r, c), dtype=np.float32) * np.float32(d ** -0.5)
+        a = 1.0 + a if name.split(".")[-1] in ("g1", "g2", "gf") else a
+        key = name.replace(".", "__")
+        m.setWeight(name, changed[key](a) if key in changed else a)
+    m.finalize()
+    return m
+
+
+@pytest.mark.parametrize("gpt", [False, True])
+@pytest.mark.parametrize("d,heads,groups", [(256, 8, 1), (512, 4, 4), (2112, 33, 8)])
+def test_a_first_position_takes_nothing_from_the_rows_an_earlier_sequence_left(gpt, d, heads, groups):
+    """A step at position 0 over cache rows that hold no numbers (a sequence with a NaN embedding left them in every block): the
+    logits are those of the token alone.  Rows of one and of two sets of values a thread."""
+    def with_nan(a):
+        a = a.copy()
+        a[5] = np.nan
+        return a
+    m = bare(gpt, groups, d, heads, emb=with_nan)
+    try:
+        assert plan_of(m)
+        alone = m.forward([7, 11])
+        assert np.isfinite(alone).all()
+        for _ in range(2):
+            m.reset()
+            m.step(5)
+            m.step(5)
+            assert np.isnan(m.lastLogits()).all()
+            m.reset()
+            for t, token in enumerate((7, 11)):
+                m.step(token)
+                assert float(np.max(np.abs(m.lastLogits() - alone[t]))) <= 2e-4, t
+    finally:
+        m.close()
