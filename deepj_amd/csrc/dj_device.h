@@ -107,5 +107,13 @@ __device__ __forceinline__ float quarters_sum(float v) {
     return a + b;
 }
 
+// v / by for many v: the product with 1 / by, corrected by its residual.  An infinite divisor or product has no residual: the
+// first takes part as the largest float beside its reciprocal of 0, the second stands.
+__device__ __forceinline__ float residual_divisor(float by) { return fminf(by, 3.402823466e38f); }
+__device__ __forceinline__ float quotient(float v, float residual_by, float inverse) {
+    const float y = v * inverse, q = fmaf(fmaf(-y, residual_by, v), inverse, y);
+    return fabsf(y) == INFINITY ? y : q;
+}
+
 }  // namespace dev
 }  // namespace dj

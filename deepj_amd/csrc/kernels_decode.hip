@@ -275,11 +275,8 @@ k_decode_attn(const float *x, const float *part, const int8_t *wqkv, const float
         k.x += a1.x; k.y += a1.y; k.z += a1.z; k.w += a1.w;
         nv.x += a2.x; nv.y += a2.y; nv.z += a2.z; nv.w += a2.w;
     }
-    const float by = divisor, inverse = 1.0f / by;
-    auto divide = [&](float &v) {                              // v / by: the quotient by the reciprocal, corrected by its residual
-        const float y = v * inverse;
-        v = fmaf(fmaf(-y, by, v), inverse, y);
-    };
+    const float inverse = 1.0f / divisor, by = residual_divisor(divisor);
+    auto divide = [&](float &v) { v = quotient(v, by, inverse); };
     divide(q.x); divide(q.y); divide(q.z); divide(q.w);
     divide(k.x); divide(k.y); divide(k.z); divide(k.w);
     divide(nv.x); divide(nv.y); divide(nv.z); divide(nv.w);

@@ -456,10 +456,9 @@ k_token_run(TokenRun r) {
     float4 x[kSets];
     float divisor = 1.0f, inverse = 1.0f;
     const float inv_d = 1.0f / (float)d;
-    auto divide = [&](float v) {                                         // v / divisor: by the reciprocal, corrected by its residual
+    auto divide = [&](float v) {                                         // by the root mean square of the row
         if constexpr (GPT) return v;
-        const float y = v * inverse;
-        return fmaf(fmaf(-y, divisor, v), inverse, y);
+        else return quotient(v, divisor, inverse);
     };
     auto row_operand = [&](int t, float4 (&v)[kSets], const float *p) {
 #pragma unroll
@@ -512,8 +511,8 @@ k_token_run(TokenRun r) {
                 const bool on = 4 * (t + q * kSpeakers) < d;
                 c[q] = on ? make_float4(x[q].x - mean, x[q].y - mean, x[q].z - mean, x[q].w - mean) : make_float4(0.f, 0.f, 0.f, 0.f);
             }
-            const float sd = sqrtf(squares * inv_d + kLayerNormEps), isd = __builtin_amdgcn_rcpf(sd);        // (each quotient is corrected by its residual)
-            auto over = [&](float v) { const float y = v * isd; return fmaf(fmaf(-y, sd, v), isd, y); };
+            const float deviation = sqrtf(squares * inv_d + kLayerNormEps), isd = __builtin_amdgcn_rcpf(deviation), sd = residual_divisor(deviation);
+            auto over = [&](float v) { const float y = v * isd; return fmaf(fmaf(-y, sd, v), isd, y); };     // (as quotient: at most sqrt(d))
 #pragma unroll
             for (int q = 0; q < kSets; q++)
                 if (t + q * kSpeakers < steps_d * 16)
@@ -534,6 +533,7 @@ k_token_run(TokenRun r) {
             lds_barrier();                                               // [staged]
             divisor = sqrtf(all_waves(sums) * inv_d + kRmsEps);
             inverse = 1.0f / divisor;
+            divisor = residual_divisor(divisor);
             asm volatile("" : "+v"(divisor), "+v"(inverse));             // (now, beside the products, and not where they are used)
         }
     };

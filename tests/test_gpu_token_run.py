@@ -10,14 +10,16 @@ from oracle import cpu_ref as ref
 pytestmark = pytest.mark.gpu
 
 
-def model(gpt, vocab, max_seq, d, heads, layers, dff, groups, seed=7):
+def model(gpt, vocab, max_seq, d, heads, layers, dff, groups, seed=7, **changed):
+    """Drawn weights; `changed`: a weight's name (with __ for its dot) and what makes its values from the drawn ones."""
     cfg = (GPTConfig if gpt else LlamaConfig)(vocab, max_seq, d, heads, layers, dff)
     m = (GPTModel if gpt else LlamaModel)(cfg, None)
     m.setTokenGroups(groups)
     rng = np.random.default_rng(seed)
     for name, (r, c) in zip(parameter_names(cfg), parameter_shapes(cfg)):
         a = rng.standard_normal((r, c), dtype=np.float32) * np.float32(d ** -0.5)
-        m.setWeight(name, 1.0 + a if name.split(".")[-1] in ("g1", "g2", "gf") else a)
+        a = 1.0 + a if name.split(".")[-1] in ("g1", "g2", "gf") else a
+        m.setWeight(name, changed.get(name.replace(".", "__"), lambda v: v)(a))
     m.finalize()
     return m
 
@@ -229,21 +231,6 @@ def test_plans_are_refused_with_a_reason_or_not_made():
     m.close()
 
 
-def bare(gpt, groups, d=256, heads=8, dff=600, vocab=300, max_seq=40, layers=2, seed=7, **changed):
-    """A small model; `changed` maps a weight's name (dots as __) to what makes its values from the drawn ones."""
-    cfg = (GPTConfig if gpt else LlamaConfig)(vocab, max_seq, d, heads, layers, dff)
-    m = (GPTModel if gpt else LlamaModel)(cfg, None)
-    m.setTokenGroups(groups)
-    rng = np.random.default_rng(seed)
-    for name, (r, c) in zip(parameter_names(cfg), parameter_shapes(cfg)):
-        a = rng.standard_normal((r, c), dtype=np.float32) * np.float32(d ** -0.5)
-        a = 1.0 + a if name.split(".")[-1] in ("g1", "g2", "gf") else a
-        key = name.replace(".", "__")
-        m.setWeight(name, changed[key](a) if key in changed else a)
-    m.finalize()
-    return m
-
-
 @pytest.mark.parametrize("gpt", [False, True])
 @pytest.mark.parametrize("d,heads,groups", [(256, 8, 1), (512, 4, 4), (2112, 33, 8)])
 def test_a_first_position_takes_nothing_from_the_rows_an_earlier_sequence_left(gpt, d, heads, groups):
@@ -253,7 +240,7 @@ def test_a_first_position_takes_nothing_from_the_rows_an_earlier_sequence_left(g
         a = a.copy()
         a[5] = np.nan
         return a
-    m = bare(gpt, groups, d, heads, emb=with_nan)
+    m = model(gpt, 300, 40, d, heads, 2, 600, groups, emb=with_nan)
     try:
         assert plan_of(m)
         alone = m.forward([7, 11])
@@ -269,3 +256,45 @@ def test_a_first_position_takes_nothing_from_the_rows_an_earlier_sequence_left(g
                 assert float(np.max(np.abs(m.lastLogits() - alone[t]))) <= 2e-4, t
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("gpt,d,heads,groups", [(False, 256, 8, 1), (False, 2112, 33, 8), (True, 256, 8, 1), (True, 768, 12, 8), (True, 2112, 33, 8)])
+def test_rows_whose_squares_overflow_are_divided_as_by_the_launches(gpt, d, heads, groups):
+    """Finite rows of 1e25: their root mean square (deviation) is infinite, the quotients zero, in every norm of every block."""
+    def huge(a):
+        a = a.copy()
+        a[5] = np.where(np.arange(a.shape[1]) % 2, np.float32(1e25), np.float32(-1e25))
+        return a
+    got = []
+    for g in (groups, -1):
+        m = model(gpt, 300, 40, d, heads, 2, 600, g, emb=huge)
+        try:
+            assert bool(plan_of(m)) == (g > 0)
+            m.prefill([3, 4], choose_next=False)
+            m.step(5)
+            got.append(m.lastLogits())
+        finally:
+            m.close()
+    assert np.isfinite(got[1]).all()
+    assert float(np.max(np.abs(got[0] - got[1]))) <= 2e-4
+
+
+@pytest.mark.parametrize("d,heads,groups", [(256, 8, 1), (2048, 16, 8)])
+def test_sums_that_overflow_stay_infinite_behind_the_division(d, heads, groups):
+    """Logits whose sums pass the largest float, each of one sign throughout: infinite ones of that sign, as the launches give."""
+    def signs(a):
+        return np.where(np.arange(a.shape[1]) % 2, np.float32(1), np.float32(-1)) * np.where(np.arange(a.shape[1]) % 3, np.float32(1e4), np.float32(1)) * np.ones_like(a)
+    got = []
+    for g in (groups, -1):
+        m = model(False, 300, 40, d, heads, 2, 600, g, emb=lambda a: 1.0 + np.abs(a), gf=lambda a: np.full_like(a, 1e34), wlm=signs,
+                 L1__wd=lambda a: 0 * a, L1__bd=lambda a: 0 * a, L0__wd=lambda a: 0 * a, L0__bd=lambda a: 0 * a, L0__wo=lambda a: 0 * a, L1__wo=lambda a: 0 * a)
+        try:
+            m.prefill([3, 4], choose_next=False)
+            m.step(5)
+            got.append(m.lastLogits())
+        finally:
+            m.close()
+    assert np.isinf(got[1]).any() and np.isfinite(got[1]).any()
+    assert np.array_equal(np.isinf(got[0]), np.isinf(got[1])) and np.array_equal(np.sign(got[0]), np.sign(got[1]))
+    both = np.isfinite(got[1])
+    assert float(np.max(np.abs(got[0][both] / got[1][both] - 1))) <= 1e-5
