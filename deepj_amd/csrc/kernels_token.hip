@@ -1014,7 +1014,11 @@ constexpr int kRingBytes = kWaves * kRing * kTokenItemBytes;             // (mor
 // Shapes that the kernel's arrays hold: the row, a group's heads and hidden units, a workgroup's tiles.
 bool token_run_ok(const TokenShape &s) {
     if (s.groups < 1 || s.groups > kTokenGroupsMost || (s.hd != 32 && s.hd != 64 && s.hd != 128)) return false;
-    if (s.d != s.heads * s.hd || s.d > kTokenMostD || s.layers < 1 || s.vocab < 1 || s.dff < 1 || s.max_seq < 1) return false;
+    if (s.heads < 1 || s.heads > kTokenMostD / s.hd || s.d != s.heads * s.hd || s.layers < 1 || s.vocab < 1 || s.dff < 1 || s.max_seq < 1) return false;
+    if (s.dff > s.groups * kTokenMostSlice) return false;
+    // what the kernel counts in 32 bits: a head's rows in bytes, the head's tiles times the workgroups they are dealt to, a run's tags
+    if ((int64_t)s.max_seq * s.hd * 4 > (int64_t)1 << 32) return false;
+    if (s.vocab > (1 << 28) - 16 || s.layers >= 1 << 21) return false;
     for (int g = 0; g < s.groups; g++) {
         const int heads = token_head0(s, g + 1) - token_head0(s, g), units = token_unit0(s, g + 1) - token_unit0(s, g);
         if (heads < 1 || heads > kMembers || heads * s.hd > kTokenMostSlice || units < 1 || units > kTokenMostSlice) return false;

@@ -2145,6 +2145,17 @@ static void plan_release(TokenPlan &p) {
     p.blocks.clear();
 }
 
+// The groups that a plan of this shape takes; 0: it is none for one
+static int shape_groups(TokenShape s) {
+    if (s.groups == 0) s.groups = token_run_groups(s);
+    return token_run_ok(s) ? s.groups : 0;
+}
+
+int32_t deepj_hip_token_plan_shape_groups(int32_t kind, int32_t vocab, int32_t max_seq, int32_t d, int32_t heads, int32_t layers, int32_t dff, int32_t groups) {
+    if ((kind != 0 && kind != 2) || vocab <= 0 || max_seq <= 0 || d <= 0 || heads <= 0 || layers <= 0 || dff <= 0 || d % heads != 0 || groups < 0) return 0;
+    return shape_groups(TokenShape{d, heads, d / heads, layers, dff, vocab, max_seq, groups, kind == 2 ? 1 : 0});
+}
+
 int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
     return guarded([&] {
         ensure_init();
@@ -2161,8 +2172,8 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
         if (w[7] < 0) fail("token_plan_create: bad group count");
         const bool gpt = w[0] == 2;
         TokenShape s{w[3], w[4], w[3] / w[4], layers, w[6], w[1], w[2], w[7], gpt ? 1 : 0};
-        if (s.groups == 0) s.groups = token_run_groups(s);
-        if (!token_run_ok(s) || (int)g.plans.size() >= kPlanSlots || !token_run_resident(s)) return;      // handle 0: not a model for it
+        s.groups = shape_groups(s);
+        if (!s.groups || (int)g.plans.size() >= kPlanSlots || !token_run_resident(s)) return;      // handle 0: not a model for it
         TokenPlan p;
         const int op = DJ_OP_Q8_LINEAR;
         g.track = &p.refs;
@@ -2304,11 +2315,9 @@ int deepj_hip_token_plan_run(int32_t handle, int32_t steps, int32_t choose) {
         if (steps < 1 || (choose == kTokenLogits && steps != 1)) fail("token_plan_run: bad step count " + std::to_string(steps));
         TokenPlan &p = plan_of(handle, "token_plan_run");
         launch_uploads();
-        // (launches of a moderate length: a run of thousands of tokens does not hold the device in one piece)
-        constexpr int kMost = 256;
-        for (int done = 0; done < steps; done += kMost) {
+        for (int done = 0; done < steps; done += kTokenMostSteps) {
             TokenRun r = p.run;
-            r.steps = std::min(kMost, steps - done);
+            r.steps = std::min(kTokenMostSteps, steps - done);
             r.choose = choose;
             plan_launch(p, r);
         }

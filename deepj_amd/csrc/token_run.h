@@ -108,9 +108,10 @@ struct TokenRun {
     int polls;                            // loads of a word until a wait is given up
     float scale;
 };
+constexpr int kTokenMostSteps = 256;         // tokens of a launch: a run of thousands does not hold the device in one piece
 __host__ __device__ inline uint32_t token_tags(const TokenShape &s) { return (uint32_t)s.layers * 8 + 8; }   // a token's tags
 
-bool token_run_ok(const TokenShape &s);
+bool token_run_ok(const TokenShape &s);           // (host arithmetic, like the next)
 int token_run_groups(const TokenShape &s);
 bool token_run_resident(const TokenShape &s);     // whether all of a run's workgroups fit on the device at once
 int64_t token_run_items(const TokenShape &s, uint32_t *offsets);      // their number; offsets[groups * members * waves]

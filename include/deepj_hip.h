@@ -328,6 +328,8 @@ int32_t deepj_hip_q8_gemm_f16_extents(int32_t m, int32_t k, int32_t rows, int32_
 #define DEEPJ_HIP_TOKEN_PLAN_WORDS 22
 #define DEEPJ_HIP_TOKEN_PLAN_LAYER_WORDS 11
 int deepj_hip_token_plan_create(const int32_t *words, int32_t n, int32_t *plan);
+/* The groups that a plan of these words takes (host arithmetic, no GPU call); 0: the shape is none for a plan. */
+int32_t deepj_hip_token_plan_shape_groups(int32_t kind, int32_t vocab, int32_t max_seq, int32_t d, int32_t heads, int32_t layers, int32_t dff, int32_t groups);
 int deepj_hip_token_plan_run(int32_t plan, int32_t steps, int32_t choose);
 /* One token that the caller chose, at a position of the caller's (the buffers' state words are not read): logits, and the state
  * {pos + 1, token, generated}. */
