@@ -15,8 +15,9 @@
 // Exchange.  A value travels with a tag of its own in one aligned 8-byte word (float, tag), so no flag has to follow the data and
 // nothing is cleared: the tag names token, block and phase, and a reader loads until it sees it.  A region is written again one
 // block later; before that every reader has sent something the writer waits for - where a product is too narrow to give every
-// member a tile, the members say so with a word each (`beat`).  Waits are bounded (kTokenPolls loads, about a second): if the
-// device did not hold all workgroups at once, each leaves, the state stays behind the last whole token, and *failed tells the host.
+// member a tile, the members say so with a word each (`beat`).  Waits are bounded (kTokenPolls loads, seconds): if the
+// device did not hold all workgroups at once, each leaves, the state stays behind the last whole token, *failed tells the host, and the
+// plan's launches behind this one leave at their start.
 //
 // A workgroup is eight wavefronts that speak - make, send and fetch rows, attend - and eight that multiply.  The two meet at
 // barriers, the same ones in the same order on both sides (named in the code).
@@ -432,7 +433,10 @@ k_token_run(TokenRun r) {
     auto check = [&](bool ok) { if (!ok) s_fail = 1; };
     auto give_up = [&]() {
         if (uniform(s_fail) == 0) return false;
-        if (threadIdx.x == 0) __hip_atomic_store(r.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (threadIdx.x == 0) {
+            __hip_atomic_store(r.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(ex + e.failed, (word)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         return true;
     };
     int token = uniform(r.given ? r.token_given : r.state[1]), generated = uniform(r.given ? r.generated_given : r.state[2]);
@@ -448,6 +452,8 @@ k_token_run(TokenRun r) {
             check(receive(w, ex, p, r.tag, r.polls));
             if (w.v[0].x != xcc || w.v[0].z != xcc) s_far = 1;
         }
+        // a run in front that gave up: this one would wait as long, for words that may never come
+        if (t == 64) check(__hip_atomic_load(ex + e.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0);
     }
     lds_barrier();                                                       // [place]
     if (give_up()) return;

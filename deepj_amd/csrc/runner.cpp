@@ -749,7 +749,7 @@ void decode(Runner &r, int steps, int mode, Choose how) {
         else {
             Stream s;
             choose_next(r, s, how, 1);
-            for (int i = 0; i < steps; i++) {
+            for (int i = 0; i < steps && !deepj_hip_token_plan_failed(r.plan); i++) {
                 hip(deepj_hip_token_plan_run(r.plan, 1, 0));
                 r.run(s);
             }

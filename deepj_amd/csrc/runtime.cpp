@@ -69,7 +69,6 @@ struct TokenPlan {
     std::vector<std::pair<int32_t, void *>> refs;
     struct Block { void *p; size_t bytes; };
     std::vector<Block> blocks;        // device memory it owns
-    int64_t exchange_words = 0;
     uint32_t next_tag = 1;            // (the exchange block starts as zeros)
     uint64_t releases_seen = 0;       // g.releases when refs were last found to be there
     int slot = -1;                    // its word of the pinned block: set by a run that could not finish
@@ -2238,7 +2237,7 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
                 g.live_bytes += (int64_t)cls;
                 return m;
             };
-            p.exchange_words = token_exchange(s).total;
+            const int64_t exchange_words = token_exchange(s).total;
             unsigned char *packed;
             uint32_t *at;
             float *vectors;
@@ -2246,7 +2245,7 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
                 packed = (unsigned char *)take(items * kTokenItemBytes);
                 at = (uint32_t *)take((int64_t)offsets.size() * 4);
                 vectors = (float *)take((int64_t)table.size() * token_vectors(s).stride * 4);
-                p.run.exchange = (unsigned long long *)take(p.exchange_words * 8);
+                p.run.exchange = (unsigned long long *)take(exchange_words * 8);
             } catch (const std::exception &) {                               // a model that fits without a plan goes on without one
                 plan_release(p);
                 return;
@@ -2258,7 +2257,7 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
             launch_uploads();
             stage_upload((float *)at, (const float *)offsets.data(), (int64_t)offsets.size());
             launch_uploads();
-            launch_fill(g.stream, (uint32_t *)p.run.exchange, 0, p.exchange_words * 2);
+            launch_fill(g.stream, (uint32_t *)p.run.exchange, 0, exchange_words * 2);
             for (int l = 0; l <= layers; l++) launch_token_vectors(g.stream, s, l, table[(size_t)l], vectors);
             for (int l = 0; l < layers; l++)
                 for (int phase = kTokenQkv; phase <= kTokenDown; phase++) {
@@ -2298,10 +2297,13 @@ static TokenPlan &plan_of(int32_t handle, const char *call) {
     return p;
 }
 
+static bool plan_failed(const TokenPlan &p) { return *(volatile uint32_t *)p.run.failed != 0; }
+
 static void plan_launch(TokenPlan &p, TokenRun r) {
+    if (plan_failed(p)) return;                                  // (it would leave at once)
     const uint64_t need = 1 + (uint64_t)r.steps * token_tags(r.shape);
     if (p.next_tag + need > 0xffffffffull) {                     // tags start over: nothing of them may be left
-        launch_fill(g.stream, (uint32_t *)r.exchange, 0, p.exchange_words * 2);
+        launch_fill(g.stream, (uint32_t *)r.exchange, 0, (int64_t)token_exchange(r.shape).failed * 2);
         p.next_tag = 1;
     }
     r.tag = p.next_tag;
@@ -2346,7 +2348,7 @@ int deepj_hip_token_plan_step(int32_t handle, int32_t pos, int32_t token, int32_
 
 int32_t deepj_hip_token_plan_failed(int32_t handle) {
     auto it = g.plans.find(handle);
-    return it == g.plans.end() ? 0 : (int32_t)*(volatile uint32_t *)it->second.run.failed;
+    return it == g.plans.end() ? 0 : (int32_t)plan_failed(it->second);
 }
 
 int32_t deepj_hip_token_plan_groups(int32_t handle) {

@@ -17,7 +17,7 @@ constexpr int kTokenMostD = 4096, kTokenMostSlice = 2048;
 // with them on their way through the caches it does not hold the rows and keys either.  Us a token without and with: 195 MB 88.2
 // and 95.1, 256 MB 121.3 and 124.4, 291 MB 102.8 and 96.6, 326 MB 152.0 and 146.4, 1 GB 344 and 331.
 constexpr int64_t kTokenPassingBytes = 272LL << 20;
-constexpr int kTokenPolls = 1 << 21;            // about a second
+constexpr int kTokenPolls = 1 << 21;            // loads of a word that is waited for: 1 s inside an XCD, 2 to 4 between XCDs
 enum TokenPhase { kTokenQkv = 0, kTokenWo = 1, kTokenUp = 2, kTokenDown = 3, kTokenHead = 4 };
 
 struct TokenShape { int d, heads, hd, layers, dff, vocab, max_seq, groups, gpt; };
@@ -59,7 +59,7 @@ __host__ __device__ inline int token_head_items(const TokenPart &p, int w) {
 }
 
 // Where the exchanged words of a group, and those that groups share, lie in the exchange block (in 8-byte words)
-struct TokenExchange { int qkv, rec, row, row2, hid, beat, beat2, group; int part, part2, best, place, total; };
+struct TokenExchange { int qkv, rec, row, row2, hid, beat, beat2, group; int part, part2, best, place, failed, total; };
 __host__ __device__ inline TokenExchange token_exchange(const TokenShape &s) {
     TokenExchange e;
     const int heads = (s.heads + s.groups - 1) / s.groups, units = ((s.dff + 63) / 64 + s.groups - 1) / s.groups * 64;
@@ -78,6 +78,7 @@ __host__ __device__ inline TokenExchange token_exchange(const TokenShape &s) {
     e.part2 = take(s.groups * s.d);
     e.best = take(kTokenBestWords * kTokenMembers * s.groups);
     e.place = take(kTokenMembers * s.groups);
+    e.failed = take(1);                  // (the last: tags that start over clear the words in front of it)
     e.total = at;
     return e;
 }
@@ -100,7 +101,7 @@ struct TokenRun {
     float *kc, *vc, *logits, *x;
     int32_t *state, *tokens;
     unsigned long long *exchange;
-    uint32_t *failed;                     // (pinned host memory)
+    uint32_t *failed;                     // (pinned host memory; the exchange block's word says the same to launches behind)
     uint32_t tag;                         // of the run's first exchange
     int steps, choose;
     int given, pos_given, token_given, generated_given;       // given: the state by value, for one token without a choice; the run leaves it one position on

@@ -322,9 +322,9 @@ int32_t deepj_hip_q8_gemm_f16_extents(int32_t m, int32_t k, int32_t rows, int32_
  *   run: `steps` tokens from state {position, token, generated}.  choose 1: each like the ops of a token with DECODE_NEXT behind
  *     them (logits hold the last one's, x its successor's embedding); choose 0: one token up to its logits, state as it was.
  *     Enqueues only.  Buffers that were released or made again since are refused.
- *   failed: 1 once a run could not have all of its workgroups on the device at the same time within about a second (another
- *     process's run of this kind may hold a part of it): state is then that behind the last whole token.  Valid after a
- *     synchronisation or a download behind the run. */
+ *   failed: 1 once a run could not have all of its workgroups on the device at the same time within some seconds (another
+ *     process's run of this kind may hold a part of it): state is then that behind the last whole token, and the plan's later runs
+ *     do nothing.  Valid after a synchronisation or a download behind the run. */
 #define DEEPJ_HIP_TOKEN_PLAN_WORDS 22
 #define DEEPJ_HIP_TOKEN_PLAN_LAYER_WORDS 11
 int deepj_hip_token_plan_create(const int32_t *words, int32_t n, int32_t *plan);

@@ -1,10 +1,14 @@
 """Runs of tokens as one launch (deepj_hip_token_plan_*) against the launches of a token and the prompt's rows: every way the
 work is dealt to groups and workgroups, at the edges of its tiles, slices, key splits and item slots."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from deepj_amd import models, GPTConfig, GPTModel, LlamaConfig, LlamaModel, TextGenerator, parameter_names, parameter_shapes
+from deepj_amd import models, GPTConfig, GPTModel, HipNative, LlamaConfig, LlamaModel, TextGenerator, parameter_names, parameter_shapes
+from deepj_amd import opcodes as op
 from deepj_amd._native import library
+from deepj_amd.fused import Stream
 from oracle import cpu_ref as ref
 
 pytestmark = pytest.mark.gpu
@@ -298,3 +302,68 @@ def test_sums_that_overflow_stay_infinite_behind_the_division(d, heads, groups):
     assert np.array_equal(np.isinf(got[0]), np.isinf(got[1])) and np.array_equal(np.sign(got[0]), np.sign(got[1]))
     both = np.isfinite(got[1])
     assert float(np.max(np.abs(got[0][both] / got[1][both] - 1))) <= 1e-5
+
+
+class RawPlan:
+    """A plan over zeroed buffers of the test's own: one Llama block of d 64."""
+    SHAPE = dict(vocab=64, max_seq=40, d=64, heads=2, dff=64)
+
+    def __init__(self, base):
+        lib, s = library(), self.SHAPE
+        d, f, v, n = s["d"], s["dff"], s["vocab"], s["max_seq"]
+        q8 = lib.deepj_hip_q8_floats
+        sizes = dict(emb=v * d, gf=d, wlm=q8(d, v), blm=v, cos=n * 16, sin=n * 16, kc=n * d, vc=n * d, state=4, tokens=n, logits=v, x=d,
+                     g1=d, g2=d, wqkv=q8(d, 3 * d), wo=q8(d, d), wgu=q8(d, 2 * f), bg=f, bu=f, wd=q8(f, d), bd=d)
+        self.id = {name: base + i for i, name in enumerate(sizes)}
+        self.sizes = sizes
+        ids, counts = (np.array(list(a), dtype=np.int32) for a in (self.id.values(), sizes.values()))
+        assert lib.deepj_hip_alloc_buffers(ids.ctypes.data, counts.ctypes.data, len(ids)) == 0
+        fills = Stream()
+        for name in sizes:
+            fills.emit(op.OP_FILL, self.id[name], 0, sizes[name])
+        HipNative.nativeFlushOps(fills.array(), len(fills.array()))
+        self.plan = 0
+        self.make()
+
+    def make(self):
+        b, s = self.id, self.SHAPE
+        words = np.array([0, s["vocab"], s["max_seq"], s["d"], s["heads"], 1, s["dff"], 1, b["emb"], -1, b["gf"], -1, b["wlm"], b["blm"], b["cos"], b["sin"],
+                          b["kc"], b["vc"], b["state"], b["tokens"], b["logits"], b["x"],
+                          b["g1"], -1, b["g2"], -1, b["wqkv"], b["wo"], b["wgu"], b["bg"], b["bu"], b["wd"], b["bd"]], dtype=np.int32)
+        plan = C.c_int32()
+        assert library().deepj_hip_token_plan_create(words.ctypes.data_as(C.c_void_p), len(words), C.byref(plan)) == 0 and plan.value
+        self.plan = plan.value
+
+    def state(self):
+        out = np.empty(4, dtype=np.int32)
+        assert library().deepj_hip_download(self.id["state"], out.ctypes.data, 4) == 0
+        return out.tolist()
+
+    def close(self):
+        lib = library()
+        if self.plan:
+            lib.deepj_hip_token_plan_destroy(self.plan)
+        ids = np.array(list(self.id.values()), dtype=np.int32)
+        lib.deepj_hip_release(ids.ctypes.data, len(ids))
+
+
+@pytest.fixture
+def raw():
+    HipNative.init(0)
+    p = RawPlan(1 << 28)
+    yield p
+    p.close()
+
+
+def test_runs_behind_one_that_gave_up_do_nothing(raw):
+    """Each would wait as long for the same workgroups.  The state stays behind the last whole token."""
+    lib = library()
+    assert lib.deepj_hip_token_plan_run(raw.plan, 2, 1) == 0
+    lib.deepj_hip_token_plan_set_polls(raw.plan, 0)
+    assert lib.deepj_hip_token_plan_run(raw.plan, 3, 1) == 0
+    lib.deepj_hip_token_plan_set_polls(raw.plan, 1 << 21)
+    assert lib.deepj_hip_token_plan_run(raw.plan, 3, 1) == 0          # (on its way before the host can know)
+    assert raw.state() == [2, 0, 2, 0] and lib.deepj_hip_token_plan_failed(raw.plan)
+    assert lib.deepj_hip_token_plan_run(raw.plan, 3, 1) == 0
+    assert lib.deepj_hip_token_plan_step(raw.plan, 7, 1, 3) == 0
+    assert raw.state() == [2, 0, 2, 0]
