@@ -93,11 +93,12 @@ struct Runner {
     int32_t sampler = -1;                                  // DECODE_SAMPLE's parameters
     // Captured per-token streams by how the token is chosen (Choose), whether the blocks are narrow, and kReplayTokens.
     int32_t graph[3][2][3] = {};
-    // The model's tokens as one launch (deepj_hip_token_plan_*); 0: replayed graphs.  Between such a run and the first sight of
-    // what it left, `pending` says what it was (a step: of which token), should it have to be done again by launches.
+    // The model's tokens as one launch (deepj_hip_token_plan_*); 0: replayed graphs.  `pending`: the calls since the first run whose
+    // outcome nobody has looked at, should they have to be done again by launches: greedy tokens, a step's token or a prompt.
     int32_t plan = 0, token_groups = 0;
-    enum Pending { kSettled, kRun, kStep } pending = kSettled;
-    int32_t pending_token = 0;
+    struct Pending { int32_t pos, generated, steps, token; std::vector<int32_t> prompt; bool chooses; };
+    std::vector<Pending> pending;
+    int32_t fed = 0, pending_fed = 0;                      // state[1] (now, in front of `pending`); -1: the token that was chosen last
     bool finalized = false;
     int32_t pos = 0;          // host mirror of state[0]
     int32_t generated = 0;    // host mirror of state[2]
@@ -597,38 +598,84 @@ void upload_state(Runner &r, int32_t token) {
 
 int token_launches(const Config &c, bool narrow);
 void decode_steps(Runner &r, int steps, int mode, Choose how, bool narrow);
+void replay(Runner &r, Choose how, bool narrow, int size, int times);
 
 void drop_plan(Runner &r) {
     if (r.plan) hip(deepj_hip_token_plan_destroy(r.plan));
     r.plan = 0;
-    r.pending = Runner::kSettled;
+    r.pending.clear();
 }
 
-// What a run of the plan left, now that the stream has got there (`arrived`: something behind it has been downloaded).  A run
-// that could not have the whole device (its state is that behind the last whole token) is finished by launches, and so is
-// everything after it.  True: results read before this call have to be read again.
+// A token of the caller's by launches, its logits and the state behind it
+void step_by_launches(Runner &r, int32_t token, int mode) {
+    upload_state(r, token);
+    // Replayed like a greedy token: the launches of a token one by one cost the host 2.4 us each (43 of them: 190 us a
+    // step of 8 layers, 130 as a graph).
+    const bool narrow = r.pos < r.narrow_positions();
+    if (mode == 1) replay(r, kNone, narrow, 2, 1);
+    else r.run(decode_stream(r, kNone, narrow));
+    r.pos += 1;
+    r.fed = token;
+    upload_state(r, token);             // the next launch takes it along, or the next step's overwrites it where it is staged
+}
+
+// DecoderOnlyModel.forward returns logits for every row; only parity tests ask for them.
+void prompt_logits(Runner &r, int n, float *out) {
+    const int64_t count = (int64_t)n * r.cfg.vocab;
+    int32_t full = r.alloc(count);
+    Stream s;
+    head_rows(r, s, r.pre.x, full, n);
+    r.run(s);
+    hip(deepj_hip_download(full, out, count));
+    r.release(full);
+}
+
+// The prompt's rows, and the state behind them
+void run_prompt(Runner &r, const int32_t *ids, int n, float *all_logits, Choose how) {
+    Stream s = prompt_stream(r, n, how);
+    hip(deepj_hip_upload(r.pre.ids, reinterpret_cast<const float *>(ids), n));   // (prompt_stream sized r.pre for n rows)
+    r.run(s);
+    if (all_logits) prompt_logits(r, n, all_logits);
+    r.pos += n;
+    r.fed = how != kNone ? -1 : 0;
+    if (how != kNone) r.generated += 1;
+    else upload_state(r, 0);            // advance the position without choosing a token
+}
+
+// Whether the runs since the last look had the whole device, now that the stream has got there (`arrived`: something behind them
+// has been downloaded).  Nobody waits for that before results are read, or launches follow that read them: behind a run that
+// gave up none does anything, prompts work at positions that are written again, and launches do all of it once more.  True:
+// results read before this call have to be read again.
 bool settle(Runner &r, bool arrived = false) {
-    if (r.pending == Runner::kSettled) return false;
+    if (r.pending.empty()) return false;
     if (!arrived) hip(deepj_hip_synchronize());
-    const Runner::Pending was = r.pending;
-    r.pending = Runner::kSettled;
+    std::vector<Runner::Pending> work;
+    work.swap(r.pending);
     if (!deepj_hip_token_plan_failed(r.plan)) return false;
     drop_plan(r);
-    if (was == Runner::kStep) {
-        r.pos -= 1;
-        upload_state(r, r.pending_token);
-        r.run(decode_stream(r, kNone, false));
-        r.pos += 1;
-        upload_state(r, r.pending_token);
-        return true;
+    const int32_t generated = r.generated;
+    r.pos = work[0].pos;
+    r.generated = work[0].generated;
+    int32_t token = r.pending_fed;
+    if (token < 0) {
+        std::vector<int32_t> tokens((size_t)r.generated);
+        hip(deepj_hip_download(r.tokens, reinterpret_cast<float *>(tokens.data()), r.generated));
+        token = tokens.back();
     }
-    int32_t st[4];
-    hip(deepj_hip_download(r.state, reinterpret_cast<float *>(st), 4));
-    const int steps = r.pos - st[0];
-    Stream s;                                                // (the embedding that the launches start from)
-    emit(s, DJ_OP_EMBED_GATHER, r.emb, r.state, r.dec.x, 1, r.cfg.d, r.cfg.vocab, 1);
-    r.run(s);
-    decode_steps(r, steps, 0, kGreedy, false);
+    upload_state(r, token);
+    for (const Runner::Pending &w : work) {
+        r.generated = w.generated;
+        if (!w.prompt.empty()) run_prompt(r, w.prompt.data(), (int)w.prompt.size(), nullptr, w.chooses ? kGreedy : kNone);
+        else if (!w.steps) step_by_launches(r, w.token, 0);
+        else {
+            Stream s;                                        // (the embedding that the launches start from)
+            emit(s, DJ_OP_EMBED_GATHER, r.emb, r.state, r.dec.x, 1, r.cfg.d, r.cfg.vocab, 1);
+            r.run(s);
+            decode_steps(r, w.steps, 0, kGreedy, false);
+            r.pos += w.steps;
+        }
+    }
+    r.generated = generated;
     return true;
 }
 
@@ -638,33 +685,22 @@ void prefill(Runner &r, const int32_t *ids, int n, float *all_logits, Choose how
     const Config &c = r.cfg;
     if (!r.finalized) finalize(r);
     if (n <= 0) throw Error("prefill: empty prompt");
-    settle(r);
     check_ids(c, ids, n);
     if (r.pos + n > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + n) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
-    Stream s = prompt_stream(r, n, how);
-    hip(deepj_hip_upload(r.pre.ids, reinterpret_cast<const float *>(ids), n));   // (prompt_stream sized r.pre for n rows)
-    r.run(s);
-    if (all_logits) {
-        // DecoderOnlyModel.forward returns logits for every row; only parity tests ask for them.
-        int32_t full = r.alloc((int64_t)n * c.vocab);
-        Stream t;
-        head_rows(r, t, r.pre.x, full, n);
-        r.run(t);
-        hip(deepj_hip_download(full, all_logits, (int64_t)n * c.vocab));
-        r.release(full);
-    }
-    r.pos += n;
-    if (how != kNone) r.generated += 1;
-    else upload_state(r, 0);            // advance the position without choosing a token
+    const int32_t pos = r.pos, generated = r.generated;
+    run_prompt(r, ids, n, all_logits, how);
+    if (!r.pending.empty()) r.pending.push_back({pos, generated, 0, 0, {ids, ids + n}, how != kNone});
+    if (all_logits && settle(r, true)) prompt_logits(r, n, all_logits);
 }
 
 void reset(Runner &r) {
     if (!r.finalized) finalize(r);
     // (what a run left is not asked for any more; one that could not finish shows in the next)
-    r.pending = Runner::kSettled;
+    r.pending.clear();
     r.pos = 0;
     r.generated = 0;
+    r.fed = 0;
     upload_state(r, 0);
 }
 
@@ -743,10 +779,14 @@ void decode(Runner &r, int steps, int mode, Choose how) {
     if (steps <= 0) return;
     if (r.pos + steps > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + steps) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
-    settle(r);
+    if (!r.plan || mode != 1) settle(r);
     if (r.plan && mode == 1 && how != kNone) {
-        if (how == kGreedy) hip(deepj_hip_token_plan_run(r.plan, steps, 1));
-        else {
+        if (how == kGreedy) {
+            hip(deepj_hip_token_plan_run(r.plan, steps, 1));
+            if (r.pending.empty()) r.pending_fed = r.fed;
+            if (!r.pending.empty() && r.pending.back().steps) r.pending.back().steps += steps;
+            else r.pending.push_back({r.pos, r.generated, steps, 0, {}, true});
+        } else {                                             // (generate, which has its tokens itself, asks what became of them)
             Stream s;
             choose_next(r, s, how, 1);
             for (int i = 0; i < steps && !deepj_hip_token_plan_failed(r.plan); i++) {
@@ -754,9 +794,9 @@ void decode(Runner &r, int steps, int mode, Choose how) {
                 r.run(s);
             }
         }
-        r.pending = Runner::kRun;
         r.pos += steps;
         r.generated += steps;
+        r.fed = -1;
         return;
     }
     const int narrow = std::min(steps, std::max(0, r.narrow_positions() - r.pos));
@@ -764,6 +804,7 @@ void decode(Runner &r, int steps, int mode, Choose how) {
     if (steps > narrow) decode_steps(r, steps - narrow, mode, how, false);
     r.pos += steps;
     r.generated += steps;
+    r.fed = -1;
 }
 
 // One token through the single-row path with the token chosen by the caller: logits of the
@@ -774,22 +815,16 @@ void step_token(Runner &r, int32_t token, int mode) {
     check_ids(c, &token, 1);
     if (r.pos + 1 > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + 1) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
-    settle(r);
     if (r.plan && mode == 1) {
         hip(deepj_hip_token_plan_step(r.plan, r.pos, token, r.generated));
+        if (r.pending.empty()) r.pending_fed = r.fed;
+        r.pending.push_back({r.pos, r.generated, 0, token, {}, false});
         r.pos += 1;
-        r.pending = Runner::kStep;
-        r.pending_token = token;
+        r.fed = token;
         return;
     }
-    upload_state(r, token);
-    // Replayed like a greedy token: the launches of a token one by one cost the host 2.4 us each (43 of them: 190 us a
-    // step of 8 layers, 130 as a graph).
-    const bool narrow = r.pos < r.narrow_positions();
-    if (mode == 1) replay(r, kNone, narrow, 2, 1);
-    else r.run(decode_stream(r, kNone, narrow));
-    r.pos += 1;
-    upload_state(r, token);             // the next launch takes it along, or the next step's overwrites it where it is staged
+    settle(r);
+    step_by_launches(r, token, mode);
 }
 
 // ── TextGenerator.sampleFromLogits on the host (temperature / top-k > 1) ────
@@ -885,7 +920,7 @@ void generate_once(Runner &r, const int32_t *prompt, int n_prompt, int max_new, 
             decode(r, cached - 1, mode, how);
             hip(deepj_hip_download(r.tokens, reinterpret_cast<float *>(out + n_prompt), cached));
             if (r.plan && deepj_hip_token_plan_failed(r.plan)) return;          // (once more, by launches)
-            r.pending = Runner::kSettled;
+            r.pending.clear();
         } else if (cached > 0) {
             prefill(r, prompt, n_prompt, nullptr, kNone);
             for (int t = 0; t < cached; t++) {
@@ -893,7 +928,8 @@ void generate_once(Runner &r, const int32_t *prompt, int n_prompt, int max_new, 
                 sample(t);
                 r.generated = t + 1;
             }
-            upload_state(r, out[n_prompt + cached - 1]);
+            r.fed = out[n_prompt + cached - 1];
+            upload_state(r, r.fed);
         }
         for (int t = cached; t < max_new; t++) {
             reset(r);

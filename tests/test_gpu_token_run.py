@@ -1,6 +1,7 @@
 """Runs of tokens as one launch (deepj_hip_token_plan_*) against the launches of a token and the prompt's rows: every way the
 work is dealt to groups and workgroups, at the edges of its tiles, slices, key splits and item slots."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -367,3 +368,95 @@ def test_runs_behind_one_that_gave_up_do_nothing(raw):
     assert lib.deepj_hip_token_plan_run(raw.plan, 3, 1) == 0
     assert lib.deepj_hip_token_plan_step(raw.plan, 7, 1, 3) == 0
     assert raw.state() == [2, 0, 2, 0]
+
+
+def test_calls_behind_a_run_wait_for_nothing():
+    """Tokens one at a time, forced ones and a prompt, behind work that takes the device far longer than their calls the host."""
+    lib = library()
+    m = model(False, 300, 80, 256, 8, 2, 300, 1)
+    big, size = np.array([1 << 28], dtype=np.int32), np.array([1 << 28], dtype=np.int32)
+    assert lib.deepj_hip_alloc_buffers(big.ctypes.data, size.ctypes.data, 1) == 0
+    try:
+        ids = ref.JavaRandom(3).ints(40, 300)
+        fills = Stream()
+        for _ in range(400):
+            fills.emit(op.OP_FILL, int(big[0]), 0, int(size[0]))
+        fills = fills.array()
+
+        def calls():
+            m.reset()
+            m.prefill(ids[:20])
+            for _ in range(4):
+                m.decode(1)
+            m.step(int(ids[20]))
+            m.step(int(ids[21]))
+            m.prefill(ids[22:30])
+            m.decode(2)
+        calls()
+        tokens = m.tokens()
+        start = time.perf_counter()
+        HipNative.nativeFlushOps(fills, len(fills))
+        calls()
+        called = time.perf_counter() - start
+        assert np.array_equal(m.tokens(), tokens) and len(tokens) == 8
+        assert called < 0.5 * (time.perf_counter() - start), called
+    finally:
+        lib.deepj_hip_release(big.ctypes.data, 1)
+        m.close()
+
+
+@pytest.mark.parametrize("gpt,groups", [(False, 1), (True, 8), (False, 4)])
+def test_everything_behind_a_run_that_gave_up_is_done_again(gpt, groups):
+    """Runs, steps and prompts whose results nobody reads in between, with the wait that is given up at each of them: tokens and
+    logits are those of the launches."""
+    lib = library()
+    ids = ref.JavaRandom(9).ints(40, 300)
+    calls = [lambda m: m.decode(3), lambda m: m.decode(1), lambda m: m.step(int(ids[5])), lambda m: m.step(int(ids[6])),
+             lambda m: m.prefill(ids[7:9]), lambda m: m.decode(4), lambda m: m.prefill(ids[9:14], choose_next=False),
+             lambda m: m.step(int(ids[14])), lambda m: m.prefill(ids[15:33]), lambda m: m.decode(2), lambda m: m.decode(5)]
+
+    def results(m, ends, at=None):
+        m.reset()
+        m.prefill(ids[:5])
+        for i, call in enumerate(calls[:ends]):
+            if i == at:
+                lib.deepj_hip_token_plan_set_polls(plan_of(m), 0)
+            call(m)
+        return (m.lastLogits(), m.tokens()) if ends % 2 else (m.tokens(), m.lastLogits())[::-1]
+    good = model(gpt, 300, 90, 256, 8, 2, 600, -1)
+    try:
+        for ends in (1, 4, 8, 11):
+            logits, tokens = results(good, ends)
+            for at in range(ends):
+                m = model(gpt, 300, 90, 256, 8, 2, 600, groups)
+                try:
+                    got = results(m, ends, at)
+                    late = all(i in (4, 6, 8) for i in range(at, ends))       # (no run behind it)
+                    assert bool(plan_of(m)) == late, (ends, at)
+                    assert np.array_equal(got[1], tokens), (ends, at)
+                    assert float(np.max(np.abs(got[0] - logits))) <= 2e-4, (ends, at)
+                finally:
+                    m.close()
+    finally:
+        good.close()
+
+
+def test_rows_of_a_prompt_behind_a_run_that_gave_up():
+    """Every row's logits of a prompt whose cache the run left short."""
+    m, good = (model(False, 300, 90, 256, 8, 2, 300, g) for g in (1, -1))
+    try:
+        ids = ref.JavaRandom(4).ints(30, 300)
+        library().deepj_hip_token_plan_set_polls(plan_of(m), 0)
+        got = []
+        for x in (m, good):
+            x.prefill(ids[:9])
+            x.decode(4)
+            out = np.empty((17, 300), dtype=np.float32)
+            chunk = np.ascontiguousarray(ids[9:26])
+            assert library().deepj_runner_prefill(x._h, chunk.ctypes.data_as(C.POINTER(C.c_int32)), 17, out.ctypes.data, 1) == 0
+            x.decode(3)
+            got.append((out, x.tokens()))
+        assert float(np.max(np.abs(got[0][0] - got[1][0]))) <= 2e-4 and np.array_equal(got[0][1], got[1][1])
+    finally:
+        m.close()
+        good.close()
