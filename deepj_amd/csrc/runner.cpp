@@ -398,9 +398,9 @@ void finalize(Runner &r) {
     }
     // the prompt-sized buffers for the longest prompt the cache can take, so that no request pays for allocation
     alloc_acts(r, r.pre, c.max_seq);
-    make_plan(r);
     r.finalized = true;
     warm_up(r);
+    make_plan(r);       // (behind the weights' fp16 copies and the workspace: a second copy for tokens takes what is left)
 }
 
 // ── command streams ────────────────────────────────────────────────────────
@@ -679,6 +679,14 @@ bool settle(Runner &r, bool arrived = false) {
     return true;
 }
 
+// Whether tokens are runs.  A plan whose memory was given back goes, once it is known what its last runs left.
+bool has_plan(Runner &r) {
+    if (!r.plan || deepj_hip_token_plan_groups(r.plan)) return r.plan != 0;
+    settle(r);
+    drop_plan(r);
+    return false;
+}
+
 // Runs the prompt rows through the model, filling the cache.  Leaves the last row's
 // logits in r.logits; unless `how` is kNone the next token is chosen on the device as well.
 void prefill(Runner &r, const int32_t *ids, int n, float *all_logits, Choose how) {
@@ -779,8 +787,7 @@ void decode(Runner &r, int steps, int mode, Choose how) {
     if (steps <= 0) return;
     if (r.pos + steps > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + steps) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
-    if (!r.plan || mode != 1) settle(r);
-    if (r.plan && mode == 1 && how != kNone) {
+    if (mode == 1 && how != kNone && has_plan(r)) {
         if (how == kGreedy) {
             hip(deepj_hip_token_plan_run(r.plan, steps, 1));
             if (r.pending.empty()) r.pending_fed = r.fed;
@@ -799,6 +806,7 @@ void decode(Runner &r, int steps, int mode, Choose how) {
         r.fed = -1;
         return;
     }
+    settle(r);
     const int narrow = std::min(steps, std::max(0, r.narrow_positions() - r.pos));
     if (narrow) decode_steps(r, narrow, mode, how, true);
     if (steps > narrow) decode_steps(r, steps - narrow, mode, how, false);
@@ -815,7 +823,7 @@ void step_token(Runner &r, int32_t token, int mode) {
     check_ids(c, &token, 1);
     if (r.pos + 1 > c.max_seq)
         throw Error("context of " + std::to_string(r.pos + 1) + " tokens exceeds maxSeqLen " + std::to_string(c.max_seq));
-    if (r.plan && mode == 1) {
+    if (mode == 1 && has_plan(r)) {
         hip(deepj_hip_token_plan_step(r.plan, r.pos, token, r.generated));
         if (r.pending.empty()) r.pending_fed = r.fed;
         r.pending.push_back({r.pos, r.generated, 0, token, {}, false});
@@ -1060,7 +1068,10 @@ int deepj_runner_set_token_groups(void *h, int32_t groups) {
     });
 }
 
-int32_t deepj_runner_token_plan(void *h) { return h ? static_cast<Runner *>(h)->plan : 0; }
+int32_t deepj_runner_token_plan(void *h) {
+    const int32_t plan = h ? static_cast<Runner *>(h)->plan : 0;
+    return plan && deepj_hip_token_plan_groups(plan) ? plan : 0;
+}
 
 int64_t deepj_runner_prepared_bytes(void *h) { return h ? static_cast<Runner *>(h)->prepared_bytes : 0; }
 

@@ -68,7 +68,7 @@ struct TokenPlan {
     TokenRun run{};
     std::vector<std::pair<int32_t, void *>> refs;
     struct Block { void *p; size_t bytes; };
-    std::vector<Block> blocks;        // device memory it owns
+    std::vector<Block> blocks;        // device memory it owns; none: given back where other memory was short
     uint32_t next_tag = 1;            // (the exchange block starts as zeros)
     uint64_t releases_seen = 0;       // g.releases when refs were last found to be there
     int slot = -1;                    // its word of the pinned block: set by a run that could not finish
@@ -95,6 +95,7 @@ struct Runtime {
     std::map<size_t, std::vector<void *>> cache;   // size class -> free blocks
     int64_t live_bytes = 0, cached_bytes = 0, driver_allocs = 0;
     size_t cache_limit = (size_t)16 << 30;
+    int64_t memory_limit = -1;                     // bytes that may be held (device_held); -1: what the device has
     float *workspace = nullptr;
     int64_t workspace_floats = 0;
     float *row_pieces = nullptr;
@@ -449,7 +450,51 @@ size_t size_class(size_t bytes) {
     return (bytes + step - 1) / step * step;
 }
 
-void *pool_alloc(size_t cls) {
+// The memory of token plans, weights that their models hold a second time: back to the driver.  Their models' tokens go on as launches.
+bool give_plans_back() {
+    bool some = false;
+    for (auto &kv : g.plans) {
+        for (const TokenPlan::Block &b : kv.second.blocks) {
+            (void)hipFree(b.p);
+            g.live_bytes -= (int64_t)b.bytes;
+            some = true;
+        }
+        kv.second.blocks.clear();
+    }
+    return some;
+}
+
+int64_t device_held() { return g.live_bytes + g.cached_bytes + 4 * (g.workspace_floats + g.row_pieces_floats); }
+
+// Device memory from the driver.  Where that has none left, what the pool keeps goes back to it first, then what token plans hold
+// (not for the sake of another plan).
+void *device_memory(size_t bytes, bool for_plan = false) {
+    void *p = nullptr;
+    auto ask = [&] { return g.memory_limit >= 0 && device_held() + (int64_t)bytes > g.memory_limit ? hipErrorOutOfMemory : hipMalloc(&p, bytes); };
+    hipError_t e = ask();
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        DJ_HIP(hipStreamSynchronize(g.stream));
+        for (auto &kv : g.cache) {
+            for (void *q : kv.second) (void)hipFree(q);
+            kv.second.clear();
+        }
+        g.cached_bytes = 0;
+        e = ask();
+        if (e != hipSuccess && !for_plan && give_plans_back()) {
+            (void)hipGetLastError();
+            e = ask();
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            fail("Failed to allocate HIP buffer of " + std::to_string(bytes) + " bytes: " + hipGetErrorString(e));
+        }
+    }
+    g.driver_allocs++;
+    return p;
+}
+
+void *pool_alloc(size_t cls, bool for_plan = false) {
     auto it = g.cache.find(cls);
     if (it != g.cache.end() && !it->second.empty()) {
         void *p = it->second.back();
@@ -459,25 +504,7 @@ void *pool_alloc(size_t cls) {
     }
     if (g.capturing) fail("deepj_hip: device allocation requested while a graph is being captured");
     if (g.no_alloc) fail("deepj_hip: device allocation requested inside the allocation-free entry point");
-    void *p = nullptr;
-    hipError_t e = hipMalloc(&p, cls);
-    if (e != hipSuccess) {
-        // give cached blocks back to the driver and retry once
-        (void)hipGetLastError();
-        DJ_HIP(hipStreamSynchronize(g.stream));
-        for (auto &kv : g.cache) {
-            for (void *q : kv.second) (void)hipFree(q);
-            kv.second.clear();
-        }
-        g.cached_bytes = 0;
-        e = hipMalloc(&p, cls);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            fail("Failed to allocate HIP buffer of " + std::to_string(cls) + " bytes: " + hipGetErrorString(e));
-        }
-    }
-    g.driver_allocs++;
-    return p;
+    return device_memory(cls, for_plan);
 }
 
 void pool_free(void *p, size_t cls) {
@@ -506,8 +533,7 @@ void ensure_workspace(int64_t floats) {
     g.workspace = nullptr;
     g.workspace_floats = 0;
     int64_t want = std::max<int64_t>(floats, (int64_t)1 << 20);
-    DJ_HIP(hipMalloc((void **)&g.workspace, (size_t)want * 4));
-    g.driver_allocs++;
+    g.workspace = static_cast<float *>(device_memory((size_t)want * 4));
     g.workspace_floats = want;
 }
 
@@ -523,8 +549,7 @@ void ensure_scratch(const Scratch &need) {
     g.row_pieces = nullptr;
     g.row_pieces_floats = 0;
     const int64_t want = std::max<int64_t>(need.row_pieces, (int64_t)1 << 20);
-    DJ_HIP(hipMalloc((void **)&g.row_pieces, (size_t)want * 4));
-    g.driver_allocs++;
+    g.row_pieces = static_cast<float *>(device_memory((size_t)want * 4));
     g.row_pieces_floats = want;
 }
 
@@ -1808,6 +1833,13 @@ int deepj_hip_pool_stats(int64_t out[4]) {
     });
 }
 
+int deepj_hip_limit_memory(int64_t more) {
+    return guarded([&] {
+        if (more < -1) fail("limit_memory: a byte count, or -1 for no limit");
+        g.memory_limit = more < 0 ? -1 : device_held() + more;
+    });
+}
+
 void *deepj_hip_host_alloc(int64_t bytes) {
     void *p = nullptr;
     guarded([&] {
@@ -2232,7 +2264,7 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
             const int64_t items = token_run_items(s, offsets.data());
             auto take = [&](int64_t bytes) {
                 const size_t cls = size_class((size_t)bytes);
-                void *m = pool_alloc(cls);
+                void *m = pool_alloc(cls, true);
                 p.blocks.push_back({m, cls});
                 g.live_bytes += (int64_t)cls;
                 return m;
@@ -2287,6 +2319,7 @@ static TokenPlan &plan_of(int32_t handle, const char *call) {
     auto it = g.plans.find(handle);
     if (it == g.plans.end()) fail(std::string(call) + ": unknown plan " + std::to_string(handle));
     TokenPlan &p = it->second;
+    if (p.blocks.empty()) fail(std::string(call) + ": the memory of plan " + std::to_string(handle) + " was given back");
     if (p.releases_seen == g.releases) return p;
     for (const auto &ref : p.refs) {
         auto b = g.live.find(ref.first);
@@ -2353,7 +2386,7 @@ int32_t deepj_hip_token_plan_failed(int32_t handle) {
 
 int32_t deepj_hip_token_plan_groups(int32_t handle) {
     auto it = g.plans.find(handle);
-    return it == g.plans.end() ? 0 : it->second.run.shape.groups;
+    return it == g.plans.end() || it->second.blocks.empty() ? 0 : it->second.run.shape.groups;
 }
 
 int deepj_hip_token_plan_set_polls(int32_t handle, int32_t polls) {

@@ -82,6 +82,9 @@ int deepj_hip_shutdown(void);              /* frees every buffer and the cache *
 int deepj_hip_trim(void);                  /* returns cached (released) memory to the driver */
 /* out[0]=live buffers, out[1]=live bytes, out[2]=cached bytes, out[3]=driver allocations so far */
 int deepj_hip_pool_stats(int64_t out[4]);
+/* Device memory that buffers (those released and kept too), plans and workspaces may take beyond what they hold at this call, in
+ * bytes; -1 (at first): what the device has.  What does not fit fails as where the device has no more. */
+int deepj_hip_limit_memory(int64_t more);
 /* Host memory that deepj_hip_download fills without a copy in between (pinned; blocks given back are handed out again).
  * NULL where ordinary memory is the better choice: below 64 KiB, for the first requests of about a size (making a block costs
  * more than several downloads), where the blocks made so far are kept rather than given back, and when the bound on such
@@ -318,7 +321,8 @@ int32_t deepj_hip_q8_gemm_f16_extents(int32_t m, int32_t k, int32_t rows, int32_
  *     heads, layers, dff, groups (0: the library's choice, else 1 to 8 XCDs), emb, pos (GPT), gf, bf (GPT), wlm, blm, cosT, sinT,
  *     kCache, vCache [layers][heads][maxSeq][hd], state, tokens, logits, x}, then per layer {g1, be1 (GPT), g2, be2 (GPT), wqkv [3 d]
  *     rows, wo, wgu (Llama: rows 2 n gate, 2 n + 1 up), bg, bu (Llama), wd, bd}.  *plan = 0, without an error, where the
- *     shape or the device is not one for it, or the memory does not suffice: DECODE_ATTN ... DECODE_NEXT are the way.
+ *     shape or the device is not one for it, or the memory does not suffice: DECODE_ATTN ... DECODE_NEXT are the way.  Where memory
+ *     is short for anything else later on, plans give theirs back first: their runs are refused from then on.
  *   run: `steps` tokens from state {position, token, generated}.  choose 1: each like the ops of a token with DECODE_NEXT behind
  *     them (logits hold the last one's, x its successor's embedding); choose 0: one token up to its logits, state as it was.
  *     Enqueues only.  Buffers that were released or made again since are refused.
@@ -335,7 +339,7 @@ int deepj_hip_token_plan_run(int32_t plan, int32_t steps, int32_t choose);
  * {pos + 1, token, generated}. */
 int deepj_hip_token_plan_step(int32_t plan, int32_t pos, int32_t token, int32_t generated);
 int32_t deepj_hip_token_plan_failed(int32_t plan);
-int32_t deepj_hip_token_plan_groups(int32_t plan);       /* its groups (XCDs); 0: no such plan */
+int32_t deepj_hip_token_plan_groups(int32_t plan);       /* its groups (XCDs); 0: no such plan, or its memory was given back */
 /* Loads after which a workgroup gives a word up that it waits for (2^21, the most, to begin with; 0: at once) */
 int deepj_hip_token_plan_set_polls(int32_t plan, int32_t polls);
 int deepj_hip_token_plan_destroy(int32_t plan);

@@ -309,7 +309,7 @@ class RawPlan:
     """A plan over zeroed buffers of the test's own: one Llama block of d 64."""
     SHAPE = dict(vocab=64, max_seq=40, d=64, heads=2, dff=64)
 
-    def __init__(self, base):
+    def __init__(self, base, room=True):
         lib, s = library(), self.SHAPE
         d, f, v, n = s["d"], s["dff"], s["vocab"], s["max_seq"]
         q8 = lib.deepj_hip_q8_floats
@@ -324,15 +324,15 @@ class RawPlan:
             fills.emit(op.OP_FILL, self.id[name], 0, sizes[name])
         HipNative.nativeFlushOps(fills.array(), len(fills.array()))
         self.plan = 0
-        self.make()
+        self.make(room)
 
-    def make(self):
+    def make(self, room=True):
         b, s = self.id, self.SHAPE
         words = np.array([0, s["vocab"], s["max_seq"], s["d"], s["heads"], 1, s["dff"], 1, b["emb"], -1, b["gf"], -1, b["wlm"], b["blm"], b["cos"], b["sin"],
                           b["kc"], b["vc"], b["state"], b["tokens"], b["logits"], b["x"],
                           b["g1"], -1, b["g2"], -1, b["wqkv"], b["wo"], b["wgu"], b["bg"], b["bu"], b["wd"], b["bd"]], dtype=np.int32)
         plan = C.c_int32()
-        assert library().deepj_hip_token_plan_create(words.ctypes.data_as(C.c_void_p), len(words), C.byref(plan)) == 0 and plan.value
+        assert library().deepj_hip_token_plan_create(words.ctypes.data_as(C.c_void_p), len(words), C.byref(plan)) == 0 and bool(plan.value) == room
         self.plan = plan.value
 
     def state(self):
@@ -460,3 +460,77 @@ def test_rows_of_a_prompt_behind_a_run_that_gave_up():
     finally:
         m.close()
         good.close()
+
+
+class limited:
+    """Device memory that the library may take beyond what its buffers hold now, in bytes."""
+
+    def __init__(self, more):
+        self.more = more
+
+    def __enter__(self):
+        library().deepj_hip_trim()
+        assert library().deepj_hip_limit_memory(C.c_int64(self.more)) == 0
+
+    def __exit__(self, *exc):
+        library().deepj_hip_limit_memory(C.c_int64(-1))
+
+
+def test_a_model_that_fits_without_a_plan_loads_without_one():
+    """Memory for the weights, their fp16 copies and the prompt's buffers, and not for the plan."""
+    shape = (False, 3000, 512, 1024, 16, 2, 2816)
+    before = HipNative.poolStats()["live_bytes"]
+    plain = model(*shape, -1)                                        # (the workspaces are at their sizes behind it)
+    need, copies = HipNative.poolStats()["live_bytes"] - before, plain.preparedBytes()
+    plain.close()
+    assert copies > 0
+    with limited(need):
+        m = model(*shape, 8)
+        try:
+            assert plan_of(m) == 0 and m.preparedBytes() == copies
+            ids = ref.JavaRandom(2).ints(30, 3000)
+            assert np.array_equal(TextGenerator.generate(m, ids, 9, top_k=1), TextGenerator.generate(m, ids, 9, top_k=1, use_graph=False))
+        finally:
+            m.close()
+    m = model(*shape, 8)
+    assert plan_of(m) and m.preparedBytes() == copies
+    m.close()
+
+
+def test_a_plan_gives_its_memory_back_where_other_memory_is_short():
+    """For a buffer that would not fit beside it; tokens behind it, and those of runs that nobody had looked at, are right.  Another
+    plan is no reason."""
+    lib = library()
+    shape = (False, 3000, 200, 1024, 16, 2, 2816)
+    ids = ref.JavaRandom(2).ints(30, 3000)
+    m = model(*shape, 8)
+    one, size = np.array([1 << 28], dtype=np.int32), np.array([1 << 18], dtype=np.int32)
+    try:
+        exp = TextGenerator.generate(m, ids, 12, top_k=1, use_graph=False)[30:]
+        m.reset()
+        m.prefill(ids)
+        m.decode(5)
+        plan = plan_of(m)
+        before = HipNative.poolStats()["live_bytes"]
+        raw = RawPlan(1 << 27)
+        raw_bytes = HipNative.poolStats()["live_bytes"] - before
+        raw.close()
+        with limited(raw_bytes - 1024):                               # (all of it but its plan)
+            raw = RawPlan(1 << 27, room=False)
+            assert plan_of(m) == plan
+            raw.close()
+        with limited(0):
+            assert lib.deepj_hip_alloc_buffers(one.ctypes.data, size.ctypes.data, 1) == 0
+        assert plan_of(m) == 0
+        assert lib.deepj_hip_token_plan_run(plan, 1, 1) != 0 and b"given back" in lib.deepj_hip_last_error()
+        m.decode(4)
+        m.decode(2)
+        assert np.array_equal(m.tokens(), exp)
+        assert np.array_equal(TextGenerator.generate(m, ids, 12, top_k=1)[30:], exp)
+        with limited(0):                                              # with nothing left to give back
+            size[0] = 1 << 28
+            one[0] += 1
+            assert lib.deepj_hip_alloc_buffers(one.ctypes.data, size.ctypes.data, 1) != 0 and b"Failed to allocate" in lib.deepj_hip_last_error()
+    finally:
+        lib.deepj_hip_release(np.array([1 << 28], dtype=np.int32).ctypes.data, 1)
+        m.close()
