@@ -72,6 +72,7 @@ struct TokenPlan {
     uint32_t next_tag = 1;            // (the exchange block starts as zeros)
     uint64_t releases_seen = 0;       // g.releases when refs were last found to be there
     int slot = -1;                    // its word of the pinned block: set by a run that could not finish
+    bool launched = false;            // some run was
 };
 constexpr int kPlanSlots = 1024;
 
@@ -2340,6 +2341,7 @@ static void plan_launch(TokenPlan &p, TokenRun r) {
         p.next_tag = 1;
     }
     r.tag = p.next_tag;
+    p.launched = true;
     launch_token_run(g.stream, r);
     p.next_tag += (uint32_t)need;
 }
@@ -2402,7 +2404,9 @@ int deepj_hip_token_plan_destroy(int32_t handle) {
     return guarded([&] {
         auto it = g.plans.find(handle);
         if (it == g.plans.end()) return;
-        plan_release(it->second);                                // (blocks are reused behind the stream's work)
+        // Blocks are reused behind the stream's work; its word of the pinned block, which the host writes for the next plan, is not
+        if (it->second.launched) DJ_HIP(hipStreamSynchronize(g.stream));
+        plan_release(it->second);
         g.plans.erase(it);
     });
 }

@@ -534,3 +534,23 @@ def test_a_plan_gives_its_memory_back_where_other_memory_is_short():
     finally:
         lib.deepj_hip_release(np.array([1 << 28], dtype=np.int32).ctypes.data, 1)
         m.close()
+
+def test_a_run_of_a_plan_that_has_gone_marks_no_other(raw):
+    """A run that gives up behind its plan's end, with another plan made meanwhile: the other one has not failed."""
+    lib = library()
+    big, size = np.array([(1 << 28) + 1000], dtype=np.int32), np.array([1 << 26], dtype=np.int32)
+    assert lib.deepj_hip_alloc_buffers(big.ctypes.data, size.ctypes.data, 1) == 0
+    try:
+        fills = Stream()
+        for _ in range(400):
+            fills.emit(op.OP_FILL, int(big[0]), 0, int(size[0]))
+        HipNative.nativeFlushOps(fills.array(), len(fills.array()))       # (some 20 ms that the run stands behind)
+        lib.deepj_hip_token_plan_set_polls(raw.plan, 0)
+        assert lib.deepj_hip_token_plan_run(raw.plan, 3, 1) == 0
+        lib.deepj_hip_token_plan_destroy(raw.plan)
+        raw.make()
+        assert lib.deepj_hip_synchronize() == 0
+        assert not lib.deepj_hip_token_plan_failed(raw.plan)
+        assert lib.deepj_hip_token_plan_run(raw.plan, 3, 1) == 0 and raw.state()[0] == 3
+    finally:
+        lib.deepj_hip_release(big.ctypes.data, 1)
