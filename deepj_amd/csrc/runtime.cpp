@@ -42,6 +42,7 @@ struct Buffer {
     void *ptr = nullptr;
     size_t capacity = 0;      // bytes actually owned (size class)
     int64_t floats = 0;       // size the caller asked for
+    uint64_t made = 0;        // a number of its own
 };
 
 // Floats of device scratch that a stream needs: the workspace, and the block for the Q8 GEMM that multiplies a batch of rows
@@ -63,10 +64,11 @@ struct Graph {
 };
 
 // A model's tokens in one launch (kernels_token.hip).  The plan holds the weights in that kernel's order, the block its
-// workgroups exchange words in, and the buffers it was made over (id, address); a run is refused once one of them is gone.
+// workgroups exchange words in, and the buffers it was made over (id, number); a run is refused once one of them is gone, also where
+// another of its id lies in its place: the plan's weights are those of the first.
 struct TokenPlan {
     TokenRun run{};
-    std::vector<std::pair<int32_t, void *>> refs;
+    std::vector<std::pair<int32_t, uint64_t>> refs;
     struct Block { void *p; size_t bytes; };
     std::vector<Block> blocks;        // device memory it owns; none: given back where other memory was short
     uint32_t next_tag = 1;            // (the exchange block starts as zeros)
@@ -115,7 +117,7 @@ struct Runtime {
     std::unordered_map<int32_t, Graph> graphs;
     int32_t next_graph = 1;
     std::map<int32_t, TokenPlan> plans;
-    uint64_t releases = 0;                         // buffers that have gone so far
+    uint64_t releases = 0, made = 0;               // buffers that have gone, and been made, so far
     int32_t next_plan = 1;
     unsigned *attn_counters = nullptr;             // kAttnCounterHeads zeroed words: decode attention's split arrivals
     unsigned char *static_scratch = nullptr;       // device address of `scratch` below on g.device
@@ -1668,6 +1670,7 @@ int deepj_hip_alloc_buffers(const int32_t *ids, const int32_t *sizes, int32_t co
             b.ptr = pool_alloc(cls);
             b.capacity = cls;
             b.floats = sizes[i];
+            b.made = ++g.made;
             g.live.emplace(ids[i], b);
             g.live_bytes += (int64_t)cls;
         }
@@ -2208,7 +2211,8 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
         if (!s.groups || (int)g.plans.size() >= kPlanSlots || !token_run_resident(s)) return;      // handle 0: not a model for it
         TokenPlan p;
         const int op = DJ_OP_Q8_LINEAR;
-        g.track = &p.refs;
+        std::vector<std::pair<int32_t, void *>> named;
+        g.track = &named;
         std::vector<TokenLayer> table((size_t)layers + 1);                       // (the last: the final norm)
         struct Weight { const int8_t *q = nullptr; const float *s = nullptr; int k = 0; };
         std::vector<Weight> weights;
@@ -2258,6 +2262,7 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
             throw;
         }
         g.track = nullptr;
+        for (const auto &ref : named) p.refs.emplace_back(ref.first, g.live.at(ref.first).made);
         std::sort(p.refs.begin(), p.refs.end());
         p.refs.erase(std::unique(p.refs.begin(), p.refs.end()), p.refs.end());
         try {
@@ -2324,7 +2329,7 @@ static TokenPlan &plan_of(int32_t handle, const char *call) {
     if (p.releases_seen == g.releases) return p;
     for (const auto &ref : p.refs) {
         auto b = g.live.find(ref.first);
-        if (b == g.live.end() || b->second.ptr != ref.second)
+        if (b == g.live.end() || b->second.made != ref.second)
             fail(std::string(call) + ": buffer id=" + std::to_string(ref.first) + " was released or reallocated after plan " + std::to_string(handle) + " was made");
     }
     p.releases_seen = g.releases;

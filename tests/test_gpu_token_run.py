@@ -554,3 +554,12 @@ def test_a_run_of_a_plan_that_has_gone_marks_no_other(raw):
         assert lib.deepj_hip_token_plan_run(raw.plan, 3, 1) == 0 and raw.state()[0] == 3
     finally:
         lib.deepj_hip_release(big.ctypes.data, 1)
+
+def test_a_plan_over_a_buffer_that_was_made_again_is_refused(raw):
+    """Also where the new buffer of that id lies where the old one did: the plan's copies are of what the old one held."""
+    lib = library()
+    assert lib.deepj_hip_token_plan_run(raw.plan, 2, 1) == 0 and raw.state()[0] == 2
+    one, size = np.array([raw.id["wo"]], dtype=np.int32), np.array([raw.sizes["wo"]], dtype=np.int32)
+    assert lib.deepj_hip_release(one.ctypes.data, 1) == 0
+    assert lib.deepj_hip_alloc_buffers(one.ctypes.data, size.ctypes.data, 1) == 0
+    assert lib.deepj_hip_token_plan_run(raw.plan, 1, 1) != 0 and b"released" in lib.deepj_hip_last_error()
