@@ -203,7 +203,7 @@ k_token_run(TokenRun r) {
         const TokenItems it = token_items(min(q.t1 - q.t0, kTokenTiles), q.steps, w);
         s_item[phase * kWaves + w] = make_int4(it.first / q.steps, it.first % q.steps, it.end - it.first, q.steps);
     }
-    if (threadIdx.x == 0) { s_fail = 0; s_far = 0; }
+    if (threadIdx.x == 0) { s_fail = 0; s_far = r.far; }
     if (threadIdx.x < 4) reinterpret_cast<uint32_t *>(planes + kZeros)[threadIdx.x] = 0;
     for (int i = threadIdx.x; i < kTokenTiles * 16 * kRed; i += kThreads) red[i] = 0.0f;
     lds_barrier();

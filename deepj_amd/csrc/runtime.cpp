@@ -2396,12 +2396,29 @@ int32_t deepj_hip_token_plan_groups(int32_t handle) {
     return it == g.plans.end() || it->second.blocks.empty() ? 0 : it->second.run.shape.groups;
 }
 
+static TokenPlan &plan_to_set(int32_t handle, const char *call) {
+    auto it = g.plans.find(handle);
+    if (it == g.plans.end()) fail(std::string(call) + ": unknown plan " + std::to_string(handle));
+    return it->second;
+}
+
 int deepj_hip_token_plan_set_polls(int32_t handle, int32_t polls) {
     return guarded([&] {
-        auto it = g.plans.find(handle);
-        if (it == g.plans.end()) fail("token_plan_set_polls: unknown plan " + std::to_string(handle));
+        TokenPlan &p = plan_to_set(handle, "token_plan_set_polls");
         if (polls < 0 || polls > kTokenPolls) fail("token_plan_set_polls: 0 to " + std::to_string(kTokenPolls));
-        it->second.run.polls = polls;
+        p.run.polls = polls;
+    });
+}
+
+int deepj_hip_token_plan_set_far(int32_t handle, int32_t far) {
+    return guarded([&] { plan_to_set(handle, "token_plan_set_far").run.far = far != 0; });
+}
+
+int deepj_hip_token_plan_set_tag(int32_t handle, uint32_t tag) {
+    return guarded([&] {
+        TokenPlan &p = plan_to_set(handle, "token_plan_set_tag");
+        if (tag < p.next_tag) fail("token_plan_set_tag: words with tags up to " + std::to_string(p.next_tag - 1) + " may lie in the exchange block");
+        p.next_tag = tag;
     });
 }
 

@@ -107,6 +107,7 @@ struct TokenRun {
     int given, pos_given, token_given, generated_given;       // given: the state by value, for one token without a choice; the run leaves it one position on
     int passing;                          // the items are more than kTokenPassingBytes
     int polls;                            // loads of a word until a wait is given up
+    int far;                              // a group's words go through memory, also where its workgroups share an L2
     float scale;
 };
 constexpr int kTokenMostSteps = 256;         // tokens of a launch: a run of thousands does not hold the device in one piece

@@ -342,6 +342,11 @@ int32_t deepj_hip_token_plan_failed(int32_t plan);
 int32_t deepj_hip_token_plan_groups(int32_t plan);       /* its groups (XCDs); 0: no such plan, or its memory was given back */
 /* Loads after which a workgroup gives a word up that it waits for (2^21, the most, to begin with; 0: at once) */
 int deepj_hip_token_plan_set_polls(int32_t plan, int32_t polls);
+/* 1: words travel through memory inside a group too, as where its workgroups do not share an XCD (0 to begin with: as they do) */
+int deepj_hip_token_plan_set_far(int32_t plan, int32_t far);
+/* The number that the next run's words begin with; refused where an earlier run's may be as large.  Runs count on, and clear the words
+ * where 32 bits end. */
+int deepj_hip_token_plan_set_tag(int32_t plan, uint32_t tag);
 int deepj_hip_token_plan_destroy(int32_t plan);
 
 /* ── host side: java.util.Random twin ─────────────────────────────────────

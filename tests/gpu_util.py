@@ -1,7 +1,8 @@
 """Helpers shared by the GPU parity tests."""
 import numpy as np
 
-from deepj_amd import HipBackend, Tensor
+from deepj_amd import GPTModel, HipBackend, Tensor
+from deepj_amd._native import library
 from oracle import cpu_ref as ref
 
 
@@ -39,3 +40,16 @@ class backend:
     def __exit__(self, *exc):
         self.be.releaseResources()
         return False
+
+
+def seeded(cls, cfg, seed, groups):
+    """cls(cfg, seed) whose tokens run on so many XCDs (0: the library's choice), or with -1 as replayed graphs."""
+    m = cls(cfg, None)
+    m.setTokenGroups(groups)
+    if cls is GPTModel:
+        m._check(library().deepj_runner_init_seeded_gpt(m._h, seed, cfg.initScale, 0))
+    else:
+        m._check(library().deepj_runner_init_seeded(m._h, seed, 0))
+    m.finalize()
+    assert bool(library().deepj_runner_token_plan(m._h)) == (groups >= 0)
+    return m

@@ -9,7 +9,7 @@ import pytest
 from deepj_amd import GPTConfig, GPTModel, HipNative, ModelSerializer, TextGenerator, parameter_names
 from deepj_amd.fused import DeviceBuffers, Stream
 from oracle import cpu_ref as ref
-from gpu_util import assert_close
+from gpu_util import assert_close, seeded
 
 pytestmark = pytest.mark.gpu
 
@@ -125,13 +125,13 @@ def oracle_gpt(cfg, seed):
     return m
 
 
-@pytest.fixture(scope="module")
-def g1():
+@pytest.fixture(scope="module", params=[0, -1], ids=["runs", "graphs"])
+def g1(request):
     ref.set_threads(ref.default_threads())
     # initScale 1: with the default 0.2 every gain is 0.2 and the logits of a random model shrink to ~1e-3,
     # which would make the absolute logit gate vacuous (the default scale has its own test below)
     cfg = GPTConfig(G1.vocabSize, G1.maxSeqLen, G1.dModel, G1.nHeads, G1.nLayers, G1.dFF, initScale=1.0)
-    gpu, cpu = GPTModel(cfg, 42), oracle_gpt(cfg, 42)
+    gpu, cpu = seeded(GPTModel, cfg, 42, request.param), oracle_gpt(cfg, 42)
     yield gpu, cpu
     gpu.close()
     ref.set_threads(1)

@@ -13,6 +13,7 @@ from deepj_amd import opcodes as op
 from deepj_amd._native import library
 from deepj_amd.fused import DeviceBuffers, Stream
 from deepj_amd.models import _DecoderOnlyModel
+from gpu_util import seeded
 from oracle import cpu_ref as ref
 
 pytestmark = pytest.mark.gpu
@@ -27,10 +28,10 @@ def oracle_model(cfg, seed, **extra):
     return m
 
 
-@pytest.fixture(scope="module")
-def c1():
+@pytest.fixture(scope="module", params=[0, -1], ids=["runs", "graphs"])
+def c1(request):
     ref.set_threads(ref.default_threads())
-    gpu = LlamaModel(C1, 42)
+    gpu = seeded(LlamaModel, C1, 42, request.param)
     cpu = oracle_model(C1, 42)
     yield gpu, cpu
     gpu.close()
@@ -574,14 +575,15 @@ def test_a_narrow_block_in_two_launches_matches_the_layers(d, hd, dff, max_seq, 
     assert float(np.max(np.abs(keys - K))) <= 2e-5 and float(np.max(np.abs(values - V))) <= 2e-5
 
 
+@pytest.mark.parametrize("groups", [0, -1], ids=["runs", "graphs"])
 @pytest.mark.parametrize("d,hd,dff,gpt", [(256, 64, 300, False), (128, 64, 130, True), (256, 32, 257, True), (64, 64, 512, False), (192, 32, 384, False)])
-def test_one_generation_goes_from_two_launches_a_block_to_five(d, hd, dff, gpt):
+def test_one_generation_goes_from_two_launches_a_block_to_five(d, hd, dff, gpt, groups):
     """Around the position where a narrow model's blocks change: rows of the cached path equal the prompt's on both sides (within
     the tolerance of the other such tests), and a greedy, a sampled and an eager run that pass it agree with one another and
     with the prompt's logits."""
     at = library().deepj_hip_decode_block_positions(d, hd, dff)
     cls, config = (GPTModel, GPTConfig) if gpt else (LlamaModel, LlamaConfig)
-    gpu = cls(config(vocabSize=97, maxSeqLen=at + 60, dModel=d, nHeads=d // hd, nLayers=2, dFF=dff), 11)
+    gpu = seeded(cls, config(vocabSize=97, maxSeqLen=at + 60, dModel=d, nHeads=d // hd, nLayers=2, dFF=dff), 11, groups)
     try:
         before = len(gpu.decodeStream())
         ids = ref.JavaRandom(5).ints(at + 5, 97)

@@ -563,3 +563,109 @@ def test_a_plan_over_a_buffer_that_was_made_again_is_refused(raw):
     assert lib.deepj_hip_release(one.ctypes.data, 1) == 0
     assert lib.deepj_hip_alloc_buffers(one.ctypes.data, size.ctypes.data, 1) == 0
     assert lib.deepj_hip_token_plan_run(raw.plan, 1, 1) != 0 and b"released" in lib.deepj_hip_last_error()
+
+
+@pytest.mark.parametrize("gpt,groups", [(False, 1), (True, 8)])
+def test_a_run_of_more_tokens_than_a_launch_takes(gpt, groups):
+    """300 and 600 tokens, in launches of 256, against the launches of a token."""
+    m = model(gpt, 300, 700, 256, 8, 2, 600, groups)
+    try:
+        ids = ref.JavaRandom(6).ints(20, 300)
+        exp = TextGenerator.generate(m, ids, 601, top_k=1, use_graph=False)
+        assert np.array_equal(TextGenerator.generate(m, ids, 301, top_k=1), exp[:321])
+        assert np.array_equal(TextGenerator.generate(m, ids, 601, top_k=1), exp)
+        assert plan_of(m)
+    finally:
+        m.close()
+
+
+@pytest.mark.parametrize("gpt,groups", [(False, 1), (True, 8)])
+def test_tags_start_over(gpt, groups):
+    """The words' numbers at the end of 32 bits: a token has 24 here, a run one more.  Runs that just fit, just do not, and steps."""
+    lib = library()
+    ids = ref.JavaRandom(6).ints(20, 300)
+    m = model(gpt, 300, 90, 256, 8, 2, 600, groups)
+    try:
+        exp = TextGenerator.generate(m, ids, 14, top_k=1, use_graph=False)[20:]
+    finally:
+        m.close()
+    for left in (0, 1, 24, 25, 26, 48, 49, 50, 73, 74, 200):
+        m = model(gpt, 300, 90, 256, 8, 2, 600, groups)
+        try:
+            plan = plan_of(m)
+            m.prefill(ids)
+            m.decode(3)
+            assert lib.deepj_hip_token_plan_set_tag(plan, C.c_uint32(0xffffffff - left)) == 0
+            m.decode(2)
+            m.decode(1)
+            m.decode(3)
+            assert lib.deepj_hip_token_plan_set_tag(plan, C.c_uint32(1)) != 0 and b"exchange block" in lib.deepj_hip_last_error()
+            m.decode(4)
+            assert np.array_equal(m.tokens(), exp) and plan_of(m), left
+            m.step(5)
+            logits = m.lastLogits()
+            m.reset()
+            m.prefill(np.concatenate([ids, exp[:13]]), choose_next=False)
+            m.step(5)
+            assert np.array_equal(m.lastLogits().view(np.int32), logits.view(np.int32)) or np.max(np.abs(m.lastLogits() - logits)) <= 2e-4
+        finally:
+            m.close()
+
+
+@pytest.mark.parametrize("gpt,d,heads,dff,groups", [(False, 64, 2, 50, 1), (False, 256, 8, 600, 1), (True, 256, 8, 600, 1), (False, 320, 10, 1000, 4), (True, 768, 12, 3072, 8), (False, 2112, 33, 5000, 8)])
+def test_words_through_memory_are_the_words_of_a_shared_l2(gpt, d, heads, dff, groups):
+    """Groups whose workgroups do not share an XCD: the same bits."""
+    m = model(gpt, 1003, 200, d, heads, 2, dff, groups)
+    try:
+        ids = ref.JavaRandom(6).ints(100, 1003)
+        got = []
+        for far in (0, 1, 0):
+            assert library().deepj_hip_token_plan_set_far(plan_of(m), far) == 0
+            tokens = TextGenerator.generate(m, ids, 40, top_k=1)
+            m.step(7)
+            got.append((tokens, m.lastLogits()))
+        for tokens, logits in got[1:]:
+            assert np.array_equal(tokens, got[0][0]) and np.array_equal(logits.view(np.int32), got[0][1].view(np.int32))
+        assert plan_of(m)
+    finally:
+        m.close()
+
+
+@pytest.mark.parametrize("gpt,groups", [(False, 1), (True, 8)])
+def test_a_run_that_gives_up_somewhere_is_done_again(gpt, groups):
+    """Waits of a few loads: which of them ends a run, in front of, behind or inside some of its tokens, is the device's choice, and what
+    comes out is not."""
+    ids = ref.JavaRandom(9).ints(20, 300)
+    good = model(gpt, 300, 90, 256, 8, 2, 600, -1)
+    try:
+        exp = TextGenerator.generate(good, ids, 40, top_k=1)[20:]
+        good.step(3)
+        logits = good.lastLogits()
+    finally:
+        good.close()
+    for polls in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 64):
+        m = model(gpt, 300, 90, 256, 8, 2, 600, groups)
+        try:
+            library().deepj_hip_token_plan_set_polls(plan_of(m), polls)
+            m.prefill(ids)
+            m.decode(30)
+            m.decode(9)
+            m.step(3)
+            assert float(np.max(np.abs(m.lastLogits() - logits))) <= 2e-4, polls
+            assert np.array_equal(m.tokens(), exp), polls
+        finally:
+            m.close()
+
+
+def test_a_run_that_gives_up_leaves_the_state_behind_a_whole_token(raw):
+    """What the plan's caller finds: as many tokens generated as positions passed, and never more than were asked for."""
+    lib = library()
+    for polls in (1, 2, 4, 8, 16, 32, 64):
+        lib.deepj_hip_token_plan_destroy(raw.plan)
+        raw.make()
+        lib.deepj_hip_token_plan_set_polls(raw.plan, polls)
+        lib.deepj_hip_upload(raw.id["state"], np.zeros(4, dtype=np.int32).ctypes.data, 4)
+        assert lib.deepj_hip_token_plan_run(raw.plan, 30, 1) == 0
+        pos, token, generated, _ = raw.state()
+        assert 0 <= pos == generated <= 30 and token == 0
+        assert pos == 30 or lib.deepj_hip_token_plan_failed(raw.plan)
