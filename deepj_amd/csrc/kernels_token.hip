@@ -203,7 +203,7 @@ k_token_run(TokenRun r) {
         const TokenItems it = token_items(min(q.t1 - q.t0, kTokenTiles), q.steps, w);
         s_item[phase * kWaves + w] = make_int4(it.first / q.steps, it.first % q.steps, it.end - it.first, q.steps);
     }
-    if (threadIdx.x == 0) { s_fail = 0; s_far = r.far; }
+    if (threadIdx.x == 0) { s_fail = 0; s_far = 0; }
     if (threadIdx.x < 4) reinterpret_cast<uint32_t *>(planes + kZeros)[threadIdx.x] = 0;
     for (int i = threadIdx.x; i < kTokenTiles * 16 * kRed; i += kThreads) red[i] = 0.0f;
     lds_barrier();
@@ -416,6 +416,7 @@ k_token_run(TokenRun r) {
         return t;
     };
     word *const ex = r.exchange;
+    word *const front = ex - kTokenFront;
     const TokenExchange e = token_exchange(s);
     const TokenVectors at_vec = token_vectors(s);
     const uint32_t mine = (uint32_t)(g * e.group);                       // the group's words
@@ -435,7 +436,7 @@ k_token_run(TokenRun r) {
         if (uniform(s_fail) == 0) return false;
         if (threadIdx.x == 0) {
             __hip_atomic_store(r.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            __hip_atomic_store(ex + e.failed, (word)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(reinterpret_cast<uint32_t *>(front), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         return true;
     };
@@ -453,7 +454,11 @@ k_token_run(TokenRun r) {
             if (w.v[0].x != xcc || w.v[0].z != xcc) s_far = 1;
         }
         // a run in front that gave up: this one would wait as long, for words that may never come
-        if (t == 64) check(__hip_atomic_load(ex + e.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0);
+        if (t == 64) {
+            const word w = __hip_atomic_load(front, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            check((uint32_t)w == 0);
+            if (w >> 32) s_far = 1;
+        }
     }
     lds_barrier();                                                       // [place]
     if (give_up()) return;

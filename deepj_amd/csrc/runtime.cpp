@@ -2275,7 +2275,8 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
                 g.live_bytes += (int64_t)cls;
                 return m;
             };
-            const int64_t exchange_words = token_exchange(s).total;
+            const int64_t exchange_words = kTokenFront + token_exchange(s).total;
+            unsigned long long *exchange;
             unsigned char *packed;
             uint32_t *at;
             float *vectors;
@@ -2283,19 +2284,20 @@ int deepj_hip_token_plan_create(const int32_t *w, int32_t n, int32_t *handle) {
                 packed = (unsigned char *)take(items * kTokenItemBytes);
                 at = (uint32_t *)take((int64_t)offsets.size() * 4);
                 vectors = (float *)take((int64_t)table.size() * token_vectors(s).stride * 4);
-                p.run.exchange = (unsigned long long *)take(exchange_words * 8);
+                exchange = (unsigned long long *)take(exchange_words * 8);
             } catch (const std::exception &) {                               // a model that fits without a plan goes on without one
                 plan_release(p);
                 return;
             }
             p.run.items = packed;
+            p.run.exchange = exchange + kTokenFront;
             p.run.passing = items * kTokenItemBytes > kTokenPassingBytes;
             p.run.offsets = at;
             p.run.vectors = vectors;
             launch_uploads();
             stage_upload((float *)at, (const float *)offsets.data(), (int64_t)offsets.size());
             launch_uploads();
-            launch_fill(g.stream, (uint32_t *)p.run.exchange, 0, exchange_words * 2);
+            launch_fill(g.stream, (uint32_t *)exchange, 0, exchange_words * 2);
             for (int l = 0; l <= layers; l++) launch_token_vectors(g.stream, s, l, table[(size_t)l], vectors);
             for (int l = 0; l < layers; l++)
                 for (int phase = kTokenQkv; phase <= kTokenDown; phase++) {
@@ -2342,7 +2344,7 @@ static void plan_launch(TokenPlan &p, TokenRun r) {
     if (plan_failed(p)) return;                                  // (it would leave at once)
     const uint64_t need = 1 + (uint64_t)r.steps * token_tags(r.shape);
     if (p.next_tag + need > 0xffffffffull) {                     // tags start over: nothing of them may be left
-        launch_fill(g.stream, (uint32_t *)r.exchange, 0, (int64_t)token_exchange(r.shape).failed * 2);
+        launch_fill(g.stream, (uint32_t *)r.exchange, 0, (int64_t)token_exchange(r.shape).total * 2);
         p.next_tag = 1;
     }
     r.tag = p.next_tag;
@@ -2411,7 +2413,11 @@ int deepj_hip_token_plan_set_polls(int32_t handle, int32_t polls) {
 }
 
 int deepj_hip_token_plan_set_far(int32_t handle, int32_t far) {
-    return guarded([&] { plan_to_set(handle, "token_plan_set_far").run.far = far != 0; });
+    return guarded([&] {
+        const TokenPlan &p = plan_to_set(handle, "token_plan_set_far");
+        if (p.blocks.empty()) return;
+        launch_fill(g.stream, (uint32_t *)(p.run.exchange - kTokenFront) + 1, far != 0, 1);
+    });
 }
 
 int deepj_hip_token_plan_set_tag(int32_t handle, uint32_t tag) {

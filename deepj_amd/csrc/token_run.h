@@ -11,6 +11,9 @@ namespace dj {
 constexpr int kTokenMembers = 32, kTokenGroupsMost = 8, kTokenWaves = 8, kTokenThreads = 64 * kTokenWaves;
 constexpr int kTokenTiles = 32;                 // tiles of 16 outputs that a workgroup takes in one pass
 constexpr int kTokenItemBytes = 1024 + 128;     // 16 outputs x 64 k: the int8 weights in the lanes' order, then their 32 scales
+// In front of the exchanged words, a page (so that they lie as in a block of their own), of which a run reads the first word: its low half
+// is set by a run that gave up, its high half sends a group's words through memory also where its workgroups share an L2.
+constexpr int kTokenFront = 512;
 constexpr int kTokenBestWords = 16;             // a line each: writers of one line wait for one another
 constexpr int kTokenMostD = 4096, kTokenMostSlice = 2048;
 // Items of more bytes than this are loaded as passing by: the memory-side cache (256 MB) does not hold them until the next token, and
@@ -59,7 +62,7 @@ __host__ __device__ inline int token_head_items(const TokenPart &p, int w) {
 }
 
 // Where the exchanged words of a group, and those that groups share, lie in the exchange block (in 8-byte words)
-struct TokenExchange { int qkv, rec, row, row2, hid, beat, beat2, group; int part, part2, best, place, failed, total; };
+struct TokenExchange { int qkv, rec, row, row2, hid, beat, beat2, group; int part, part2, best, place, total; };
 __host__ __device__ inline TokenExchange token_exchange(const TokenShape &s) {
     TokenExchange e;
     const int heads = (s.heads + s.groups - 1) / s.groups, units = ((s.dff + 63) / 64 + s.groups - 1) / s.groups * 64;
@@ -78,7 +81,6 @@ __host__ __device__ inline TokenExchange token_exchange(const TokenShape &s) {
     e.part2 = take(s.groups * s.d);
     e.best = take(kTokenBestWords * kTokenMembers * s.groups);
     e.place = take(kTokenMembers * s.groups);
-    e.failed = take(1);                  // (the last: tags that start over clear the words in front of it)
     e.total = at;
     return e;
 }
@@ -100,14 +102,13 @@ struct TokenRun {
     const float *emb, *pos, *blm, *cos_t, *sin_t;
     float *kc, *vc, *logits, *x;
     int32_t *state, *tokens;
-    unsigned long long *exchange;
-    uint32_t *failed;                     // (pinned host memory; the exchange block's word says the same to launches behind)
+    unsigned long long *exchange;         // (kTokenFront words behind the block's start)
+    uint32_t *failed;                     // (pinned host memory)
     uint32_t tag;                         // of the run's first exchange
     int steps, choose;
     int given, pos_given, token_given, generated_given;       // given: the state by value, for one token without a choice; the run leaves it one position on
     int passing;                          // the items are more than kTokenPassingBytes
     int polls;                            // loads of a word until a wait is given up
-    int far;                              // a group's words go through memory, also where its workgroups share an L2
     float scale;
 };
 constexpr int kTokenMostSteps = 256;         // tokens of a launch: a run of thousands does not hold the device in one piece
