@@ -624,14 +624,12 @@ k_token_run(TokenRun r) {
         if constexpr (GPT) row_operand(me(), beta, r.vectors + at_vec.be1);
         // The head's keys and values; a row is HD floats, of which a lane has four.  A round of them: keys of tile
         // `split + (r0 + u) splits` of TILE (past the cached ones: the first key's, again).  At the first position row 0 holds anything,
-        // and a masked value that is no number would not weigh nothing: there numbers stand in for it, the items' offsets (zeroing the
-        // values instead costs 1.5 % of a GPT token, this nothing beyond what runs differ by).
-        static_assert(kMembers * kWaves >= HD, "the offsets of one group hold a row");
+        // and a masked value weighs nothing only where it is a number: there norm weights stand in for it, which make every row NaN by
+        // themselves where they are none.
         floatx4 K[U], V[U];
         auto keys_at = [&](int l) { return ((int64_t)(l * s.heads + h0 + (hl < heads ? hl : 0)) * s.max_seq) * HD; };
         auto load_round = [&](int l, int r0) {
-            const char *const kb = reinterpret_cast<const char *>(r.kc + keys_at(l));
-            const char *const vb = pos == 0 ? reinterpret_cast<const char *>(r.offsets) : reinterpret_cast<const char *>(r.vc + keys_at(l));
+            const char *const kb = reinterpret_cast<const char *>(r.kc + keys_at(l)), *const vb = reinterpret_cast<const char *>(pos == 0 ? r.vectors : r.vc + keys_at(l));
             const int t = me(), dl = (t & 63) % LPK, key0 = (t >> 6) * KPW + (t & 63) / LPK;
 #pragma unroll
             for (int u = 0; u < U; u++) {
