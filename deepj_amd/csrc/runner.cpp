@@ -330,7 +330,10 @@ void alloc_acts(Runner &r, Acts &a, int rows) {
     a.rows = rows;
 }
 
+bool warms_up();
 void warm_up(Runner &r);
+void decode(Runner &r, int steps, int mode, Choose how);
+void reset(Runner &r);
 
 // Tokens of a run as one launch (Llama and GPT; DeepSeek's stay launches).
 void make_plan(Runner &r) {
@@ -401,6 +404,10 @@ void finalize(Runner &r) {
     r.finalized = true;
     warm_up(r);
     make_plan(r);       // (behind the weights' fp16 copies and the workspace: a second copy for tokens takes what is left)
+    if (r.plan && warms_up()) {
+        decode(r, 1, 1, kGreedy);
+        reset(r);
+    }
 }
 
 // ── command streams ────────────────────────────────────────────────────────
@@ -719,6 +726,11 @@ void capture(Runner &r, Choose how, bool narrow, int size) {
     hip(deepj_hip_graph_capture(s.data(), (int32_t)s.size(), &r.graph[how][narrow][size]));
 }
 
+bool warms_up() {
+    const char *env = getenv("DEEPJ_HIP_WARMUP");           // "0": skip (profiling runs that want only the request's launches)
+    return !(env && env[0] == '0');
+}
+
 // The runtime builds a kernel's function object on its first launch (a few hundred microseconds each).  One pass over
 // prompts of the lengths that select the different GEMM and attention variants, and a few tokens, move that from the first
 // request to finalize(), and with it the capture of the graphs that greedy decoding replays first; the sequence state is
@@ -726,11 +738,11 @@ void capture(Runner &r, Choose how, bool narrow, int size) {
 // it).  What a program may never use is left to the request that does: graphs of sampled and of caller-chosen tokens (0.5 to
 // 1.3 ms once) and, for a narrow model, those of the blocks in five launches, which it takes late in a long context or never
 // (1.1 ms once, where loading a 4-layer model of width 256 paid 3.3).  The 16-token graph is captured and not run: its first
-// replay costs what every other does.
+// replay costs what every other does.  A model whose tokens are runs has one of a token too, behind this (finalize); the graphs
+// serve what runs do not, and everything once memory or the device is shared.
 void warm_up(Runner &r) {
     const Config &c = r.cfg;
-    const char *env = getenv("DEEPJ_HIP_WARMUP");           // "0": skip (profiling runs that want only the request's launches)
-    if (env && env[0] == '0') return;
+    if (!warms_up()) return;
     std::vector<int32_t> ids((size_t)std::min(c.max_seq, 2048), 0);
     for (int n : {2048, 1024, 512, 256, 128, 64, 32, 16, 4}) {
         if (n > (int)ids.size()) continue;

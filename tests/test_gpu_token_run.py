@@ -669,3 +669,19 @@ def test_a_run_that_gives_up_leaves_the_state_behind_a_whole_token(raw):
         pos, token, generated, _ = raw.state()
         assert 0 <= pos == generated <= 30 and token == 0
         assert pos == 30 or lib.deepj_hip_token_plan_failed(raw.plan)
+
+
+@pytest.mark.parametrize("warms_up", [True, False])
+def test_loading_a_model_runs_a_token_of_its_plan(warms_up, monkeypatch):
+    """The first launch of the kernel is the loading's, not the first request's, unless warming up is switched off.  (A plan no run
+    has been launched of takes any number for its first words.)"""
+    if not warms_up:
+        monkeypatch.setenv("DEEPJ_HIP_WARMUP", "0")
+    m = model(False, 300, 40, 256, 8, 2, 600, 1)
+    try:
+        assert (library().deepj_hip_token_plan_set_tag(plan_of(m), C.c_uint32(1)) != 0) == warms_up
+        assert len(m.tokens()) == 0
+        ids = ref.JavaRandom(6).ints(5, 300)
+        assert np.array_equal(TextGenerator.generate(m, ids, 9, top_k=1), TextGenerator.generate(m, ids, 9, top_k=1, use_graph=False))
+    finally:
+        m.close()
