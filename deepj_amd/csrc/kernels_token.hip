@@ -624,12 +624,16 @@ k_token_run(TokenRun r) {
         if constexpr (GPT) row_operand(me(), beta, r.vectors + at_vec.be1);
         // The head's keys and values; a row is HD floats, of which a lane has four.  A round of them: keys of tile
         // `split + (r0 + u) splits` of TILE (past the cached ones: the first key's, again).  At the first position row 0 holds anything,
-        // and a masked value weighs nothing only where it is a number: there norm weights stand in for it, which make every row NaN by
-        // themselves where they are none.
+        // and a masked value weighs nothing only where it is a number: there numbers stand in for it, the items' offsets (whole numbers) or,
+        // which a GPT's tokens are the faster by, norm weights (where they are no numbers every row is none).  Us for the greedy, sampled and
+        // stepped workloads of a narrow Llama, a GPT and a Llama: offsets in both families 1722, 6843 and 3825, norm weights in both
+        // 1728, 6799 and 3873, as here 1707, 6801 and 3836; without a stand-in 1716, 6806 and 3838, and zeros behind the loads a GPT's 6870.
+        static_assert(kMembers * kWaves >= HD, "the offsets of one group hold a row");
         floatx4 K[U], V[U];
         auto keys_at = [&](int l) { return ((int64_t)(l * s.heads + h0 + (hl < heads ? hl : 0)) * s.max_seq) * HD; };
         auto load_round = [&](int l, int r0) {
-            const char *const kb = reinterpret_cast<const char *>(r.kc + keys_at(l)), *const vb = reinterpret_cast<const char *>(pos == 0 ? r.vectors : r.vc + keys_at(l));
+            const float *const stand_in = GPT ? r.vectors : reinterpret_cast<const float *>(r.offsets);
+            const char *const kb = reinterpret_cast<const char *>(r.kc + keys_at(l)), *const vb = reinterpret_cast<const char *>(pos == 0 ? stand_in : r.vc + keys_at(l));
             const int t = me(), dl = (t & 63) % LPK, key0 = (t >> 6) * KPW + (t & 63) / LPK;
 #pragma unroll
             for (int u = 0; u < U; u++) {
