@@ -32,7 +32,8 @@
 // nothing kept in memory between phases: each such wait is one for the weights in front of it (GPT 177 us a token, 155 without).
 //
 // Bound by the serial chain: instructions on the way from a row's arrival to the next one's departure, one every four clocks of a
-// wavefront at best (a phase of one item a wavefront takes 1100 clocks, an exchange 1000 inside a group and 5000 between groups), and by
+// wavefront at best (clocks, with the stamps of a DJ_TRACE build in them: a product of one item a wavefront 700 to 1200 from the staged row to
+// its sums, an exchange 1300 inside a group and 4700 to 8700 between groups, from the sums to the row), and by
 // memory where a block has more than some 20 MB.  Us a token, launches and this: 4 blocks of d 256, 256 words 48.0, 33.0; 8 of d 1024,
 // 8192 words 126, 87.7; d 2048, 32000 words, 4 blocks 120, 92, 16 blocks 404, 310; GPT, 12 blocks of 768, 50257 words 200, 137.
 // Taken back: one set of wavefronts for everything (256 registers: 51.6 us where this takes 36.5); the heads' records merged
@@ -559,8 +560,9 @@ k_token_run(TokenRun r) {
             clear(t);
         }
         DJ_STAMP(24);
-        // Nothing can be here yet.  Words of the row would only be in the way, and a first try for the other groups' sums that comes too early costs
-        // its whole way before the next (us a token at GPT 12 blocks of 768 and 16 of d 2048: without 5 and 5 more, 12 139.0 and 314.0, this 138.2 and 313.4, 32 5 and 1 more).
+        // Nothing can be here yet.  Words of the row would only be in the way, and a first try for the other groups' sums that comes too early
+        // costs its whole way before the next.  Us a token at GPT 12 blocks of 768 and 16 of d 2048, by the length of the sleep: none 140.6 and
+        // 302.8, 5 137.9 and 297.1, 12 136.4 and 293.4, this 135.4 and 292.6, 32 142.8 and 297.2.
         if (crossing) __builtin_amdgcn_s_sleep(kCrossSleep);
         // (by wavefronts that have, as a rule, not sent: a wait for loads waits for the stores in front of them too)
         if (crossing && t >= kSpeakers / 2 && t - kSpeakers / 2 < p.tiles * 8) {         // two outputs a thread

@@ -6,9 +6,9 @@
 
 namespace dj {
 
-// A group is the kMembers workgroups of one XCD (one per compute unit, kWavesPerBlock wavefronts each).  What a group shares
-// travels through its L2, what groups share through memory.
-constexpr int kTokenMembers = 32, kTokenGroupsMost = 8, kTokenWaves = 8, kTokenThreads = 64 * kTokenWaves;
+// A group is the kTokenMembers workgroups of one XCD, one per compute unit, of kTokenWaves wavefronts that speak and as many that multiply.
+// What a group shares travels through its L2, what groups share through memory.
+constexpr int kTokenMembers = 32, kTokenGroupsMost = 8, kTokenWaves = 8;
 constexpr int kTokenTiles = 32;                 // tiles of 16 outputs that a workgroup takes in one pass
 constexpr int kTokenItemBytes = 1024 + 128;     // 16 outputs x 64 k: the int8 weights in the lanes' order, then their 32 scales
 // In front of the exchanged words, a page (so that they lie as in a block of their own), of which a run reads the first word: its low half
