@@ -159,7 +159,7 @@ def matvec_roofline(model, position: int, iters: int = 12):
                               "bench.py --sweep, scaled by k_copy)",
             "kernel": "k_q8_matvec", "launches_per_token": launches, "bytes_per_launch": lin_bytes // launches,
             "avg_launch_us": round(lin_us / launches, 3),
-            "timing": "mean kernel duration (start/stop events on each dispatch, whole token in order, HBM-cold); "
+            "timing": "mean kernel duration, of each launch the median of its passes (start/stop events on each dispatch, whole token in order, HBM-cold); "
                       "rocprofv3 --kernel-trace reports the same quantity",
             "back_to_back_avg_launch_us": round(b2b_us, 3), "cache_warm_avg_launch_us": round(warm_us, 3),
             "per_kernel": table,

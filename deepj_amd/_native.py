@@ -295,7 +295,7 @@ class HipNative:
 
     @staticmethod
     def profileOps(cmd_stream, iters: int, max_ops: int = 4096, detail: bool = False):
-        """Mean kernel time (microseconds) of every op of the stream: a start and a stop event on each of the op's
+        """Kernel time (microseconds, the median of the passes) of every op of the stream: a start and a stop event on each of the op's
         dispatches, summed per op; -1 for one that launched nothing, as those a launch of an op in front takes along.
         detail=True also returns the op's longest dispatch (its main kernel) and its
         number of dispatches."""

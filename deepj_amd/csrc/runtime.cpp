@@ -2018,16 +2018,16 @@ int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float 
         if (n > capacity) fail("profile_ops: the stream holds " + std::to_string(n) + " ops, the output only " + std::to_string(capacity));
         constexpr int per_op = 2 * kMaxTimedLaunches;
         std::vector<hipEvent_t> ev((size_t)per_op * n, nullptr);
-        std::vector<double> sum((size_t)n, 0.0), longest((size_t)n, 0.0);
-        std::vector<int> count((size_t)n, 0), launches((size_t)n, 0);
+        std::vector<std::vector<float>> sums((size_t)n), longest((size_t)n);
+        std::vector<int> launches((size_t)n, 0);
         auto cleanup = [&] {
             g_launch_timing = LaunchTiming{};
             for (hipEvent_t e : ev) if (e) (void)hipEventDestroy(e);
         };
         try {
             for (auto &e : ev) DJ_HIP(hipEventCreate(&e));
-            // Two passes in front are not counted: what the runtime sets up for events it has not used yet, or uses again for the first
-            // time, shows in their times (20 us on one of 4 were seen, in the first call of a process and in no later one).
+            // An op's time is the median of its passes, two more than asked for: one pass in some 400 shows a dispatch 5 to 75 us longer than
+            // all others (in 1800 passes over three ops: 5), and no few passes' mean is near the kernel's time with one of them in it.
             for (int it = -2; it < iters; it++) {
                 g.chain.valid = false;
                 Cursor c{cmd, len, 0, false, 0};                     // (as walk)
@@ -2047,7 +2047,7 @@ int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float 
                 }
                 DJ_HIP(hipStreamSynchronize(g.stream));
                 for (int i = 0; i < n; i++) {
-                    if (!launches[(size_t)i] || it < 0) continue;
+                    if (!launches[(size_t)i]) continue;
                     double total = 0.0, top = 0.0;
                     for (int j = 0; j < launches[(size_t)i]; j++) {
                         float ms = 0.0f;
@@ -2055,9 +2055,8 @@ int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float 
                         total += (double)ms * 1e3;
                         top = std::max(top, (double)ms * 1e3);
                     }
-                    sum[(size_t)i] += total;
-                    longest[(size_t)i] += top;
-                    count[(size_t)i]++;
+                    sums[(size_t)i].push_back((float)total);
+                    longest[(size_t)i].push_back((float)top);
                 }
             }
         } catch (...) {
@@ -2065,10 +2064,14 @@ int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float 
             throw;
         }
         cleanup();
+        auto median = [](std::vector<float> &v) {
+            if (v.empty()) return -1.0f;
+            std::sort(v.begin(), v.end());
+            return 0.5f * (v[(v.size() - 1) / 2] + v[v.size() / 2]);
+        };
         for (int i = 0; i < n; i++) {
-            const bool ok = count[(size_t)i] > 0;
-            us_per_op[i] = ok ? (float)(sum[(size_t)i] / count[(size_t)i]) : -1.0f;
-            if (us_longest) us_longest[i] = ok ? (float)(longest[(size_t)i] / count[(size_t)i]) : -1.0f;
+            us_per_op[i] = median(sums[(size_t)i]);
+            if (us_longest) us_longest[i] = median(longest[(size_t)i]);
             if (dispatches) dispatches[i] = launches[(size_t)i];
         }
         hipError_t e = hipGetLastError();

@@ -184,7 +184,7 @@ class Stream:
         HipNative.nativeFlushOps(self.words, len(self.words))
 
     def profile(self, iters: int) -> np.ndarray:
-        """Mean kernel duration of every op in microseconds (events on each op's own dispatch)."""
+        """Kernel duration of every op in microseconds (the median of the passes; events on each op's own dispatch)."""
         return HipNative.profileOps(self.array(), iters)
 
     def time(self, iters: int) -> float:

@@ -101,13 +101,13 @@ void *deepj_hip_stream(void);
 int deepj_hip_time_ops(const int32_t *cmd, int32_t len, int32_t iters, float *ms_total);
 
 /* Runs a validated stream `iters` times in order with a start and a stop event attached to every kernel dispatch
- * of every op: us_per_op[i] receives the mean over the passes of the summed begin-to-end times of op i's
+ * of every op: us_per_op[i] receives the median over the passes of the summed begin-to-end times of op i's
  * dispatches on the device, in microseconds - the durations a kernel trace reports, helpers of the op included
  * (-1 for an op that launched nothing).  The launches are those of a flush, so their sum is its kernel time: where one
  * launch takes along ops behind (element-wise ones, transposes, AdamW updates) its time stands at the first of them and
  * the others have launched nothing; an op by itself is measured in a stream of its own.  us_longest (optional, same length): the op's longest single dispatch, its
  * main kernel; dispatches (optional): how many the op made.  *n_ops = ops in the stream; fails when capacity is
- * smaller.  The stream runs two more times in front, uncounted. */
+ * smaller.  The stream runs two more times than that. */
 int deepj_hip_profile_ops(const int32_t *cmd, int32_t len, int32_t iters, float *us_per_op, int32_t capacity,
                           int32_t *n_ops, float *us_longest, int32_t *dispatches);
 /* Measurement aid, no counterpart in the reference: the shader clock while a stream runs.  A one-wavefront kernel on a
